@@ -1,18 +1,20 @@
-"""Build libfdb_hip.so (gfx950) in-tree with hipcc.
+"""Build libfdb_hip.so (gfx950) with hipcc and the host extension _native.so with the C++ compiler, in-tree.
 
     python -m flashdeberta_amd.csrc.build
 
-The shared object lands next to the package (flashdeberta_amd/libfdb_hip.so) so that it
-travels with the source tree; nothing is installed outside it.
+The shared objects land next to the package (flashdeberta_amd/libfdb_hip.so, flashdeberta_amd/_native.so) so that
+they travel with the source tree; nothing is installed outside it.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libfdb_hip.so")
+NATIVE = os.path.join(PKG, "_native.so")
 SOURCES = ["fdb_api.cpp", "fdb_attn.hip", "fdb_near.hip", "fdb_fp8.hip", "fdb_aux.hip", "fdb_bwd.hip", "fdb_chain.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -33,9 +35,37 @@ def _compile(src):
     return obj, err
 
 
+def _compile_native():
+    """csrc/fdb_torch.cpp: host code only, against torch's headers; it finds libfdb_hip.so beside itself."""
+    import torch
+
+    base = os.path.dirname(torch.__file__)
+    obj = os.path.join(HERE, "fdb_torch.o")
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-c", os.path.join(HERE, "fdb_torch.cpp"), "-o", obj,
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           "-isystem", os.path.join(base, "include"), "-isystem", os.path.join(base, "include", "torch", "csrc", "api", "include"),
+           "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"]]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("the C++ compiler failed for fdb_torch.cpp:\n" + r.stderr)
+    return obj, os.path.join(base, "lib")
+
+
+def _link_native(obj, torch_lib):
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", NATIVE, obj, "-L" + PKG, "-l:libfdb_hip.so", "-Wl,-rpath,$ORIGIN",
+           "-L" + torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    os.remove(obj)
+    if r.returncode != 0:
+        raise RuntimeError("link failed:\n" + r.stderr)
+
+
 def build(verbose=True):
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as ex:
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as ex:
+        native = ex.submit(_compile_native)
         results = list(ex.map(_compile, SOURCES))
+        native_obj, torch_lib = native.result()
     objs = [o for o, _ in results]
     for _, err in results:
         if verbose and err.strip():
@@ -46,8 +76,9 @@ def build(verbose=True):
         raise RuntimeError("link failed:\n" + r.stderr)
     for o in objs:
         os.remove(o)
+    _link_native(native_obj, torch_lib)
     if verbose:
-        print("built", LIB)
+        print("built", LIB, NATIVE)
     return LIB
 
 

@@ -560,6 +560,14 @@ int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_t
   return fdb_launch_worklist(cu_seqlens, batch, worklist, fdb_worklist_max_tiles(total_tokens, batch), stream);
 }
 
+int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64_t stride_b, int64_t stride_l, int32_t batch,
+                    int32_t length, int32_t* seq_start, int32_t* seq_len, void* stream) {
+  if (!mask || !seq_start || !seq_len) return FDB_ERR_NULL;
+  if (elem_size != 1 && elem_size != 2 && elem_size != 4 && elem_size != 8) return FDB_ERR_DTYPE;
+  if (batch < 1 || length < 1) return FDB_ERR_SHAPE;
+  return fdb_launch_mask_bounds(mask, elem_size, is_float != 0, stride_b, stride_l, batch, length, seq_start, seq_len, stream);
+}
+
 int32_t fdb_delta_lut_radius(int32_t position_buckets, int32_t max_position) {
   if (!lut_config_ok(position_buckets, max_position)) return FDB_ERR_LUT_ARGS;
   const int32_t span = position_buckets > 0 ? position_buckets : max_position;

@@ -75,6 +75,42 @@ __global__ __launch_bounds__(kWlThreads) void fdb_worklist_kernel(const int32_t*
   }
 }
 
+// Bounds of a padded batch's real tokens, one workgroup per row: first and last non-zero mask element and their count.
+// One pass over the mask in one launch; the same as a chain of torch reductions is ten launches of 3 us each.
+template <class T>
+__global__ __launch_bounds__(256) void fdb_mask_bounds_kernel(const T* __restrict__ mask, T ignore, int64_t stride_b, int64_t stride_l,
+                                                              int32_t length, int32_t* __restrict__ start, int32_t* __restrict__ len) {
+  const T* row = mask + (int64_t)blockIdx.x * stride_b;
+  int32_t first = length, last = -1, count = 0;
+  for (int32_t l = threadIdx.x; l < length; l += 256)
+    if ((row[(int64_t)l * stride_l] & (T)~ignore) != 0) {
+      first = min(first, l);
+      last = l;
+      ++count;
+    }
+  __shared__ int32_t part[3][4];
+  for (int off = 32; off > 0; off >>= 1) {
+    first = min(first, __shfl_xor(first, off));
+    last = max(last, __shfl_xor(last, off));
+    count += __shfl_xor(count, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    part[0][threadIdx.x >> 6] = first;
+    part[1][threadIdx.x >> 6] = last;
+    part[2][threadIdx.x >> 6] = count;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) {
+      first = min(first, part[0][w]);
+      last = max(last, part[1][w]);
+      count += part[2][w];
+    }
+    start[blockIdx.x] = count > 0 ? first : 0;
+    len[blockIdx.x] = count > 0 && last - first + 1 != count ? -1 : count;
+  }
+}
+
 __global__ void fdb_fill_u32(uint32_t* p, int n, uint32_t v) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -203,6 +239,22 @@ int fdb_launch_dequant(const void* y, int64_t y_st, int64_t y_sh, const float* s
     default: return -3;
   }
 #undef FDB_DQ
+  return (int)hipGetLastError();
+}
+
+int fdb_launch_mask_bounds(const void* mask, int elem_size, bool is_float, int64_t stride_b, int64_t stride_l, int32_t batch, int32_t length,
+                           int32_t* start, int32_t* len, void* stream) {
+#define FDB_MB(T)                                                                                                     \
+  hipLaunchKernelGGL(fdb_mask_bounds_kernel<T>, dim3(batch), dim3(256), 0, (hipStream_t)stream, (const T*)mask,      \
+                     is_float ? (T)((T)1 << (8 * sizeof(T) - 1)) : (T)0, stride_b, stride_l, length, start, len);
+  switch (elem_size) {
+    case 1: FDB_MB(uint8_t) break;
+    case 2: FDB_MB(uint16_t) break;
+    case 4: FDB_MB(uint32_t) break;
+    case 8: FDB_MB(uint64_t) break;
+    default: return FDB_ERR_DTYPE;
+  }
+#undef FDB_MB
   return (int)hipGetLastError();
 }
 

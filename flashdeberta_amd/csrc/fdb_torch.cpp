@@ -1,0 +1,546 @@
+// Host path of the operators in native code: what stands between a Python call and the launches of libfdb_hip.so.
+//
+// A short sequence's attention takes the GPU about ten microseconds, so the time of such a call is what the host spends
+// on it.  Building the argument block through ctypes, attribute by attribute, and the views and allocations around it took
+// 22 us per forward call (57 us for a module layer with its remembered projections); the same work here -- tensor
+// metadata read in place, one scratch allocation for everything that does not leave the call -- takes a fifth of that.
+//
+// This file is glue on torch's C++ interface (ATen tensors, the caching allocator, the current stream); everything that
+// runs on the GPU is behind include/fdb.h.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <map>
+#include <optional>
+#include <tuple>
+#include <utility>
+#include <vector>
+
+#include "../../include/fdb.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+// ---- Python arguments -------------------------------------------------------------------------------------------
+const Tensor& tensor_arg(PyObject* o, const char* name) {
+  TORCH_CHECK_TYPE(THPVariable_Check(o), name, " must be a tensor");
+  return THPVariable_Unpack(o);
+}
+OptTensor opt_tensor_arg(PyObject* o, const char* name) {
+  if (o == Py_None) return std::nullopt;
+  return tensor_arg(o, name);
+}
+int64_t int_arg(PyObject* o) {
+  if (!PyLong_CheckExact(o)) {  // numpy integers, bools, zero-dimensional tensors
+    PyObject* n = PyNumber_Long(o);
+    if (!n) throw python_error();
+    const int64_t v = PyLong_AsLongLong(n);
+    Py_DECREF(n);
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return v;
+  }
+  const int64_t v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+double float_arg(PyObject* o) {
+  const double v = PyFloat_AsDouble(o);
+  if (v == -1.0 && PyErr_Occurred()) throw python_error();
+  return v;
+}
+bool bool_arg(PyObject* o) {
+  const int v = PyObject_IsTrue(o);
+  if (v < 0) throw python_error();
+  return v != 0;
+}
+
+// Negative codes are argument errors (ValueError), positive ones HIP errors (RuntimeError).
+void check(int code, const char* what) {
+  if (code == 0) return;
+  TORCH_CHECK_VALUE(code > 0, what, " failed: ", fdb_strerror(code), " (code ", code, ")");
+  TORCH_CHECK(false, what, " failed: ", fdb_strerror(code), " (code ", code, ")");
+}
+
+int fdb_dtype_of(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return FDB_F32;
+    case at::kBFloat16: return FDB_BF16;
+    case at::kHalf: return FDB_F16;
+    default: return -1;
+  }
+}
+
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+
+int64_t att_span(int64_t buckets, int64_t max_relative) { return buckets > 0 ? buckets : max_relative; }
+
+// ---- the delta table on the device ---------------------------------------------------------------------------------
+// One per (buckets, positions, device), built by the Python callable registered below and kept for the life of the
+// process like the host table it comes from.  Reached with the GIL held.
+struct Lut {
+  Tensor table;
+  int32_t radius;
+};
+PyObject* g_lut_source = nullptr;
+std::map<std::tuple<int64_t, int64_t, int>, Lut> g_luts;
+
+const Lut& lut_for(int64_t buckets, int64_t max_relative, const Tensor& on) {
+  const auto key = std::make_tuple(buckets, max_relative, (int)on.get_device());
+  const auto hit = g_luts.find(key);
+  if (hit != g_luts.end()) return hit->second;
+  PyObject* dev = THPDevice_New(on.device());
+  if (!dev) throw python_error();
+  PyObject* r = PyObject_CallFunction(g_lut_source, "LLN", (long long)buckets, (long long)max_relative, dev);
+  if (!r) throw python_error();
+  Lut lut{THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(r, 1))};
+  Py_DECREF(r);
+  return g_luts.emplace(key, std::move(lut)).first->second;
+}
+
+// ---- forward -----------------------------------------------------------------------------------------------------
+// K_r / Q_r as [H, 2S, D] with a unit last stride (a leading singleton batch dimension, as the module produces it, is dropped).
+Tensor pos_arg(const Tensor& x, int64_t H, int64_t D, int64_t span, const char* name) {
+  Tensor t = x.dim() == 4 && x.size(0) == 1 ? x.select(0, 0) : x;
+  TORCH_CHECK_VALUE(t.dim() == 3 && t.size(0) == H && t.size(2) == D && t.size(1) >= 2 * span, name,
+                    " must be the projected relative embeddings [H=", H, ", >=2S=", 2 * span, ", D=", D, "], got ", x.sizes(),
+                    ". (The pre-multiplied [B,H,L,2S] bias tensors of the reference op are not an input here: the product is fused "
+                    "into the kernel.)");
+  return t.stride(2) == 1 ? t : t.contiguous();
+}
+
+Tensor unit_last(const Tensor& x) { return x.stride(-1) == 1 ? x : x.contiguous(); }
+
+// Per-row bounds of a padded batch / per-head scales: a contiguous GPU vector of n entries, kept alive by the caller's `keep`.
+const void* vector_arg(const Tensor& x, at::ScalarType type, int64_t n, const char* name, const char* what, std::vector<Tensor>& keep) {
+  TORCH_CHECK_VALUE(x.scalar_type() == type && x.is_cuda() && x.numel() == n, name, " must be ", what);
+  keep.push_back(x.contiguous());
+  return keep.back().data_ptr();
+}
+
+struct Fwd {
+  OptTensor pos_key, pos_query, cu, seq_start, seq_len, q_scale, k_scale, pk_scale, pq_scale, out, workspace;
+  int64_t max_seqlen = -1, buckets = 0, max_relative = 0, far_splits = 0, near_splits = 0, part = 0;
+  double sm_scale = NAN;  // NaN: 1 / sqrt(D * terms)
+  bool causal = false, return_lse = false, single_kernel = false, no_alloc = false;
+  PyObject* ask = nullptr;  // packed calls: asks the library for the workspace size (address of the argument block -> bytes)
+};
+
+constexpr int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }
+
+// The scratch of a call (log-sum-exp hand-over, work-list, partial results) is one allocation, cut up here; the caching
+// allocator hands it to the next call on this stream, whose launches queue up behind this call's.
+void launch_forward(fdb_attn_args& a, const Tensor& on, bool need_lse, const Fwd& o) {
+  void* stream = stream_of(on);
+  const int64_t lse_bytes = need_lse && !a.lse ? up256((int64_t)a.total_tokens * a.heads * 4) : 0;
+  const int64_t wl_bytes = a.cu_seqlens ? up256(fdb_worklist_ints(a.total_tokens, a.batch) * 4) : 0;
+  // the size depends on whether these buffers are there, not on where
+  if (lse_bytes) a.lse = (float*)16;
+  if (wl_bytes) a.worklist = (int32_t*)16;
+  int64_t ws_bytes = 0;
+  if (o.workspace) {
+    const Tensor& w = *o.workspace;
+    TORCH_CHECK_VALUE(w.scalar_type() == at::kByte && w.is_cuda() && w.is_contiguous(), "workspace must be a contiguous uint8 GPU tensor");
+    if (w.numel() > 0) {
+      a.workspace = w.data_ptr();
+      a.workspace_bytes = w.numel();
+    }
+  } else if (o.ask && a.cu_seqlens) {
+    PyObject* r = PyObject_CallFunction(o.ask, "K", (unsigned long long)(uintptr_t)&a);
+    if (!r) throw python_error();
+    ws_bytes = int_arg(r);
+    Py_DECREF(r);
+  } else {
+    ws_bytes = fdb_attn_workspace_bytes(&a);
+  }
+  Tensor scratch;
+  if (lse_bytes + wl_bytes + ws_bytes > 0) {
+    scratch = at::empty({lse_bytes + wl_bytes + ws_bytes}, on.options().dtype(at::kByte));
+    char* p = (char*)scratch.data_ptr();
+    if (lse_bytes) a.lse = (float*)p;
+    if (wl_bytes) a.worklist = (int32_t*)(p + lse_bytes);
+    if (ws_bytes) {
+      a.workspace = p + lse_bytes + wl_bytes;
+      a.workspace_bytes = ws_bytes;
+    }
+  }
+  if (wl_bytes) check(fdb_build_worklist(a.cu_seqlens, a.batch, a.total_tokens, a.worklist, stream), "fdb_build_worklist");
+  if (o.part) check(fdb_attn_fwd_part(&a, (int32_t)o.part, stream), "fdb_attn_fwd_part");
+  else check(fdb_attn_fwd(&a, stream), "fdb_attn_fwd");
+}
+
+std::pair<Tensor, Tensor> forward(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Fwd& o) {
+  TORCH_CHECK(q_in.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", q_in.device());
+  const bool varlen = o.cu.has_value();
+  int64_t B, L, H, D, T;
+  if (varlen) {
+    TORCH_CHECK_VALUE(q_in.dim() == 3, "with cu_seqlens, q/k/v must be [T, H, D]");
+    T = q_in.size(0), H = q_in.size(1), D = q_in.size(2);
+    B = o.cu->numel() - 1;
+    L = o.max_seqlen >= 0 ? o.max_seqlen : T;
+    TORCH_CHECK_VALUE(o.cu->scalar_type() == at::kInt && o.cu->is_cuda(), "cu_seqlens must be an int32 tensor on the GPU");
+  } else {
+    TORCH_CHECK_VALUE(q_in.dim() == 4, "q/k/v must be [B, L, H, D] (or [T, H, D] with cu_seqlens)");
+    B = q_in.size(0), L = q_in.size(1), H = q_in.size(2), D = q_in.size(3);
+    T = B * L;
+  }
+  TORCH_CHECK_VALUE(k_in.sizes() == q_in.sizes() && v_in.sizes() == q_in.sizes(), "q, k, v must have the same shape (self-attention): ",
+                    q_in.sizes(), " ", k_in.sizes(), " ", v_in.sizes());
+  const auto qt = q_in.scalar_type();
+  const bool fp8 = qt == at::kFloat8_e4m3fn;
+  fdb_attn_args a = {};
+  if (fp8) {
+    TORCH_CHECK_VALUE(k_in.scalar_type() == qt && v_in.scalar_type() == at::kBFloat16, "fp8 path: q and k float8_e4m3fn, v bfloat16");
+    TORCH_CHECK_VALUE(o.q_scale && o.k_scale && (!o.pos_key || o.pk_scale) && (!o.pos_query || o.pq_scale),
+                      "fp8 path: q_scale, k_scale and a scale for each position tensor are required");
+    a.dtype = FDB_FP8_E4M3;
+  } else {
+    TORCH_CHECK_VALUE(fdb_dtype_of(qt) >= 0 && k_in.scalar_type() == qt && v_in.scalar_type() == qt, "unsupported dtypes ", qt, " ",
+                      k_in.scalar_type(), " ", v_in.scalar_type());
+    a.dtype = fdb_dtype_of(qt);
+  }
+  const Tensor q = unit_last(q_in), k = unit_last(k_in), v = unit_last(v_in);
+  const int64_t span = att_span(o.buckets, o.max_relative);
+  Tensor pk, pq;
+  if (o.pos_key) pk = pos_arg(*o.pos_key, H, D, span, "pos_key");
+  if (o.pos_query) pq = pos_arg(*o.pos_query, H, D, span, "pos_query");
+  TORCH_CHECK_VALUE(!pk.defined() || pk.scalar_type() == qt, "pos_key dtype ", pk.scalar_type(), " does not match q dtype ", qt);
+  TORCH_CHECK_VALUE(!pq.defined() || pq.scalar_type() == qt, "pos_query dtype ", pq.scalar_type(), " does not match q dtype ", qt);
+  const bool has_pos = pk.defined() || pq.defined();
+  const int terms = 1 + (pk.defined() ? 1 : 0) + (pq.defined() ? 1 : 0);
+  if (has_pos) {
+    const Lut& lut = lut_for(o.buckets, o.max_relative, q);
+    a.delta_lut = (const int16_t*)lut.table.data_ptr();
+    a.lut_radius = lut.radius;
+    a.att_span = (int32_t)span;
+  }
+  const c10::hip::HIPGuard guard(q.get_device());
+  Tensor out;
+  if (o.out) {
+    out = *o.out;
+    TORCH_CHECK_VALUE(out.sizes() == q.sizes() && out.scalar_type() == v.scalar_type() && out.stride(-1) == 1,
+                      "out must have q's shape, v's dtype and a unit stride on D");
+  } else {
+    out = at::empty(q.sizes(), v.options());
+  }
+  TORCH_CHECK_VALUE(!o.no_alloc || (!o.single_kernel && !o.workspace), "no_alloc excludes single_kernel and a caller-owned workspace");
+  // The log-sum-exp buffer is also the hand-over between the far-tile and near-tile launches, so it is always provided
+  // when a position term is present (T*H floats), unless the caller wants one kernel.
+  Tensor lse;
+  if (o.return_lse) {
+    lse = at::empty({T, H}, q.options().dtype(at::kFloat));
+    a.lse = (float*)lse.data_ptr();
+  }
+  a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.out = out.data_ptr();
+  const int64_t t_ax = varlen ? 0 : 1;
+  a.q_stride_b = varlen ? 0 : q.stride(0), a.q_stride_t = q.stride(t_ax), a.q_stride_h = q.stride(t_ax + 1);
+  a.k_stride_b = varlen ? 0 : k.stride(0), a.k_stride_t = k.stride(t_ax), a.k_stride_h = k.stride(t_ax + 1);
+  a.v_stride_b = varlen ? 0 : v.stride(0), a.v_stride_t = v.stride(t_ax), a.v_stride_h = v.stride(t_ax + 1);
+  a.o_stride_b = varlen ? 0 : out.stride(0), a.o_stride_t = out.stride(t_ax), a.o_stride_h = out.stride(t_ax + 1);
+  std::vector<Tensor> keep;
+  if (varlen) {
+    a.cu_seqlens = (const int32_t*)o.cu->data_ptr();
+  } else {
+    const char* what = "an int32 GPU tensor with one entry per batch row";
+    if (o.seq_start) a.seq_start = (const int32_t*)vector_arg(*o.seq_start, at::kInt, B, "seq_start", what, keep);
+    if (o.seq_len) a.seq_len = (const int32_t*)vector_arg(*o.seq_len, at::kInt, B, "seq_len", what, keep);
+  }
+  if (pk.defined()) a.pos_key = pk.data_ptr(), a.pk_stride_h = pk.stride(0), a.pk_stride_r = pk.stride(1);
+  if (pq.defined()) a.pos_query = pq.data_ptr(), a.pq_stride_h = pq.stride(0), a.pq_stride_r = pq.stride(1);
+  if (fp8) {
+    const char* what = "a float32 GPU tensor with one entry per head";
+    if (o.q_scale) a.q_scale = (const float*)vector_arg(*o.q_scale, at::kFloat, H, "q_scale", what, keep);
+    if (o.k_scale) a.k_scale = (const float*)vector_arg(*o.k_scale, at::kFloat, H, "k_scale", what, keep);
+    if (o.pk_scale) a.pk_scale = (const float*)vector_arg(*o.pk_scale, at::kFloat, H, "pk_scale", what, keep);
+    if (o.pq_scale) a.pq_scale = (const float*)vector_arg(*o.pq_scale, at::kFloat, H, "pq_scale", what, keep);
+  }
+  a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)T;
+  a.causal = o.causal ? 1 : 0;
+  a.sm_scale = (float)(std::isnan(o.sm_scale) ? 1.0 / std::sqrt((double)(D * terms)) : o.sm_scale);
+  a.far_splits = (int32_t)o.far_splits, a.near_splits = (int32_t)o.near_splits;
+  if (o.no_alloc) check(fdb_attn_fwd_noalloc(&a, stream_of(q)), "fdb_attn_fwd_noalloc");
+  else launch_forward(a, q, has_pos && !o.single_kernel, o);
+  return {out, lse};
+}
+
+// attention_fwd(q, k, v, pos_key, pos_query, cu_seqlens, max_seqlen, sm_scale, position_buckets, max_relative_positions, causal,
+//               return_lse, seq_start, seq_len, q_scale, k_scale, pos_key_scale, pos_query_scale, out, single_kernel, far_splits,
+//               near_splits, workspace, no_alloc, part, ask) -> out or (out, lse)
+PyObject* py_attention_fwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 26, "attention_fwd takes 26 arguments");
+  Fwd o;
+  o.pos_key = opt_tensor_arg(x[3], "pos_key");
+  o.pos_query = opt_tensor_arg(x[4], "pos_query");
+  o.cu = opt_tensor_arg(x[5], "cu_seqlens");
+  if (x[6] != Py_None) o.max_seqlen = int_arg(x[6]);
+  if (x[7] != Py_None) o.sm_scale = float_arg(x[7]);
+  o.buckets = int_arg(x[8]);
+  o.max_relative = int_arg(x[9]);
+  o.causal = bool_arg(x[10]);
+  o.return_lse = bool_arg(x[11]);
+  o.seq_start = opt_tensor_arg(x[12], "seq_start");
+  o.seq_len = opt_tensor_arg(x[13], "seq_len");
+  o.q_scale = opt_tensor_arg(x[14], "q_scale");
+  o.k_scale = opt_tensor_arg(x[15], "k_scale");
+  o.pk_scale = opt_tensor_arg(x[16], "pos_key_scale");
+  o.pq_scale = opt_tensor_arg(x[17], "pos_query_scale");
+  o.out = opt_tensor_arg(x[18], "out");
+  o.single_kernel = bool_arg(x[19]);
+  o.far_splits = int_arg(x[20]);
+  o.near_splits = int_arg(x[21]);
+  o.workspace = opt_tensor_arg(x[22], "workspace");
+  o.no_alloc = bool_arg(x[23]);
+  o.part = int_arg(x[24]);
+  o.ask = x[25];
+  auto r = forward(tensor_arg(x[0], "q"), tensor_arg(x[1], "k"), tensor_arg(x[2], "v"), o);
+  PyObject* out = nullptr;
+  if (x[18] != Py_None) {
+    out = x[18];
+    Py_INCREF(out);
+  } else {
+    out = THPVariable_Wrap(std::move(r.first));
+  }
+  if (!o.return_lse) return out;
+  return Py_BuildValue("NN", out, THPVariable_Wrap(std::move(r.second)));
+  END_HANDLE_TH_ERRORS
+}
+
+// layer_attention(hidden, weight, bias, pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start,
+//                 seq_len) -> context [B, L, H*D]
+// The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
+PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 11, "layer_attention takes 11 arguments");
+  const Tensor& hidden = tensor_arg(x[0], "hidden");
+  const int64_t H = int_arg(x[5]);
+  const Tensor qkv = at::linear(hidden, tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"));
+  const int64_t B = qkv.size(0), L = qkv.size(1), D = qkv.size(2) / (3 * H), width = H * D;
+  const std::array<int64_t, 4> size{B, L, H, D}, stride{L * 3 * width, 3 * width, D, 1};
+  const Tensor all = unit_last(qkv).contiguous();
+  Fwd o;
+  o.pos_key = opt_tensor_arg(x[3], "pos_key");
+  o.pos_query = opt_tensor_arg(x[4], "pos_query");
+  o.sm_scale = float_arg(x[6]);
+  o.buckets = int_arg(x[7]);
+  o.max_relative = int_arg(x[8]);
+  o.seq_start = opt_tensor_arg(x[9], "seq_start");
+  o.seq_len = opt_tensor_arg(x[10], "seq_len");
+  const int64_t at0 = all.storage_offset();
+  const Tensor out = forward(all.as_strided(size, stride, at0), all.as_strided(size, stride, at0 + width), all.as_strided(size, stride, at0 + 2 * width), o).first;
+  return THPVariable_Wrap(out.view({B, L, width}));
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- e4m3 quantisation ---------------------------------------------------------------------------------------------
+// quantize_e4m3(x0, x1 or None) -> (y0, scale0[, y1, scale1]); shapes and layouts are checked by the callers' contract below
+PyObject* py_quantize(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 2, "quantize_e4m3 takes 2 arguments");
+  const bool pair = x[1] != Py_None;
+  const Tensor& a0 = tensor_arg(x[0], "x0");
+  const Tensor a1 = pair ? tensor_arg(x[1], "x1") : a0;
+  const char* name = pair ? "quantize_e4m3_per_head_pair" : "quantize_e4m3_per_head";
+  for (const Tensor* t : {&a0, &a1})
+    TORCH_CHECK_VALUE(t->is_cuda() && t->scalar_type() == at::kBFloat16, name, pair ? " expects bfloat16 GPU tensors" : " expects a bfloat16 GPU tensor");
+  TORCH_CHECK_VALUE(a0.sizes() == a1.sizes(), name, ": shapes differ: ", a0.sizes(), " ", a1.sizes());
+  const int64_t H = a0.size(-2), D = a0.size(-1);
+  Tensor r0 = a0.reshape({-1, H, D}), r1 = pair ? a1.reshape({-1, H, D}) : r0;
+  if (r0.strides() != r1.strides() || r0.stride(2) != 1) r0 = r0.contiguous(), r1 = r1.contiguous();
+  const c10::hip::HIPGuard guard(r0.get_device());
+  const int64_t tokens = r0.size(0), count = pair ? 2 : 1;
+  const Tensor y = at::empty({count, tokens, H, D}, r0.options().dtype(at::kFloat8_e4m3fn));
+  const Tensor scale = at::empty({count, H}, r0.options().dtype(at::kFloat));
+  const Tensor ws = at::empty({count * H}, r0.options().dtype(at::kInt));
+  char* y0 = (char*)y.data_ptr();
+  float* s0 = (float*)scale.data_ptr();
+  if (pair)
+    check(fdb_quant_e4m3_per_head_pair(r0.data_ptr(), r1.data_ptr(), r0.stride(0), r0.stride(1), y0, y0 + tokens * H * D, H * D, D, s0, s0 + H,
+                                       (uint32_t*)ws.data_ptr(), (int32_t)tokens, (int32_t)H, (int32_t)D, stream_of(r0)),
+          "fdb_quant_e4m3_per_head_pair");
+  else
+    check(fdb_quant_e4m3_per_head(r0.data_ptr(), r0.stride(0), r0.stride(1), y0, H * D, D, s0, (uint32_t*)ws.data_ptr(), (int32_t)tokens,
+                                  (int32_t)H, (int32_t)D, stream_of(r0)),
+          "fdb_quant_e4m3_per_head");
+  if (!pair) return Py_BuildValue("NN", THPVariable_Wrap(y.select(0, 0).reshape(a0.sizes())), THPVariable_Wrap(scale.select(0, 0)));
+  return Py_BuildValue("NNNN", THPVariable_Wrap(y.select(0, 0).reshape(a0.sizes())), THPVariable_Wrap(scale.select(0, 0)),
+                       THPVariable_Wrap(y.select(0, 1).reshape(a1.sizes())), THPVariable_Wrap(scale.select(0, 1)));
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- bounds of a padding mask -----------------------------------------------------------------------------------------
+// mask_bounds(mask [B, L], [B, L, L] or [B, 1, L, L] on the GPU) -> (seq_start, seq_len) int32 [B]; None for an element type it
+// does not read.
+PyObject* py_mask_bounds(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 1, "mask_bounds takes 1 argument");
+  const Tensor& m = tensor_arg(x[0], "mask");
+  const bool real = m.is_floating_point();
+  if (!m.is_cuda() || m.is_complex() || m.dim() < 2 || m.dim() > 4 || (real && m.element_size() == 1)) Py_RETURN_NONE;
+  const int64_t B = m.size(0), L = m.size(-1);
+  if (B < 1 || L < 1 || (m.dim() > 2 && m.size(-2) != L)) Py_RETURN_NONE;
+  const int64_t step = m.stride(-1) + (m.dim() > 2 ? m.stride(-2) : 0);  // a square mask's diagonal says which tokens are real
+  const c10::hip::HIPGuard guard(m.get_device());
+  const Tensor out = at::empty({2, B}, m.options().dtype(at::kInt));
+  int32_t* p = (int32_t*)out.data_ptr();
+  check(fdb_mask_bounds(m.data_ptr(), (int32_t)m.element_size(), real ? 1 : 0, m.stride(0), step, (int32_t)B, (int32_t)L, p, p + B, stream_of(m)),
+        "fdb_mask_bounds");
+  return Py_BuildValue("NN", THPVariable_Wrap(out.select(0, 0)), THPVariable_Wrap(out.select(0, 1)));
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_register_lut_source(PyObject*, PyObject* fn) {
+  Py_INCREF(fn);
+  Py_XDECREF(g_lut_source);
+  g_lut_source = fn;
+  Py_RETURN_NONE;
+}
+
+// ---- Memo ---------------------------------------------------------------------------------------------------------
+// One remembered value, valid while the tensors it was computed from are the same objects, have not been written in place
+// (version counter), still sit in the same storage with the same dtype on the same device (`p.data = x` and `module.to(dtype)`
+// swap those under an unchanged object), and `extra` compares equal.  The tensors are held weakly.
+struct Stamp {
+  c10::weak_intrusive_ptr<c10::TensorImpl> impl;
+  const void* data;
+  int64_t version;
+  at::ScalarType dtype;
+  at::Device device;
+};
+struct MemoState {
+  std::vector<Stamp> stamps;
+  PyObject* extra = nullptr;
+  PyObject* value = nullptr;
+};
+struct MemoObject {
+  PyObject_HEAD
+  MemoState* state;
+};
+
+bool tracked(const Tensor& t) { return t.defined() && !t.is_inference(); }  // inference tensors count no versions
+bool plain(const Tensor& t) { return t.has_storage(); }
+const void* address(const Tensor& t) { return plain(t) ? t.data_ptr() : nullptr; }
+
+void memo_clear(MemoState* s) {
+  s->stamps.clear();
+  Py_CLEAR(s->extra);
+  Py_CLEAR(s->value);
+}
+PyObject* memo_get(PyObject* self, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  MemoState* s = ((MemoObject*)self)->state;
+  TORCH_CHECK_TYPE(n >= 1 && n <= 2 && PyTuple_Check(x[0]), "get(tensors, extra=None) takes a tuple of tensors");
+  const Py_ssize_t count = PyTuple_GET_SIZE(x[0]);
+  if (!s->value || (size_t)count != s->stamps.size()) Py_RETURN_NONE;
+  PyObject* extra = n > 1 ? x[1] : Py_None;
+  if (extra != s->extra) {
+    const int same = PyObject_RichCompareBool(extra, s->extra, Py_EQ);
+    if (same < 0) throw python_error();
+    if (!same) Py_RETURN_NONE;
+  }
+  for (Py_ssize_t i = 0; i < count; ++i) {
+    const Tensor& t = tensor_arg(PyTuple_GET_ITEM(x[0], i), "tensors");
+    const Stamp& st = s->stamps[i];
+    if (st.impl._unsafe_get_target() != t.unsafeGetTensorImpl() || !tracked(t) || (int64_t)t._version() != st.version || address(t) != st.data ||
+        t.scalar_type() != st.dtype || t.device() != st.device)
+      Py_RETURN_NONE;
+  }
+  Py_INCREF(s->value);
+  return s->value;
+  END_HANDLE_TH_ERRORS
+}
+PyObject* memo_put(PyObject* self, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  MemoState* s = ((MemoObject*)self)->state;
+  TORCH_CHECK_TYPE(n >= 2 && n <= 3 && PyTuple_Check(x[0]), "put(tensors, value, extra=None) takes a tuple of tensors");
+  const Py_ssize_t count = PyTuple_GET_SIZE(x[0]);
+  std::vector<Stamp> stamps;
+  bool all = true;
+  for (Py_ssize_t i = 0; i < count && all; ++i) {
+    const Tensor& t = tensor_arg(PyTuple_GET_ITEM(x[0], i), "tensors");
+    all = tracked(t);
+    if (all) stamps.push_back(Stamp{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), address(t), (int64_t)t._version(), t.scalar_type(), t.device()});
+  }
+  memo_clear(s);
+  if (all) {
+    s->stamps = std::move(stamps);
+    s->extra = n > 2 ? x[2] : Py_None;
+    Py_INCREF(s->extra);
+    s->value = x[1];
+    Py_INCREF(s->value);
+  }
+  Py_INCREF(x[1]);
+  return x[1];
+  END_HANDLE_TH_ERRORS
+}
+PyObject* memo_reduce(PyObject* self, PyObject*) {  // copies and pickles of a module start with nothing remembered
+  return Py_BuildValue("O()", (PyObject*)Py_TYPE(self));
+}
+PyObject* memo_new(PyTypeObject* type, PyObject*, PyObject*) {
+  MemoObject* m = (MemoObject*)type->tp_alloc(type, 0);
+  if (m) m->state = new MemoState();
+  return (PyObject*)m;
+}
+int memo_traverse(PyObject* self, visitproc visit, void* arg) {
+  MemoState* s = ((MemoObject*)self)->state;
+  if (s) {
+    Py_VISIT(s->extra);
+    Py_VISIT(s->value);
+  }
+  return 0;
+}
+int memo_gc_clear(PyObject* self) {
+  MemoState* s = ((MemoObject*)self)->state;
+  if (s) memo_clear(s);
+  return 0;
+}
+void memo_dealloc(PyObject* self) {
+  PyObject_GC_UnTrack(self);
+  memo_gc_clear(self);
+  delete ((MemoObject*)self)->state;
+  Py_TYPE(self)->tp_free(self);
+}
+PyMethodDef memo_methods[] = {
+    {"get", (PyCFunction)(void*)memo_get, METH_FASTCALL, "get(tensors, extra=None): the value remembered for these tensors, or None"},
+    {"put", (PyCFunction)(void*)memo_put, METH_FASTCALL, "put(tensors, value, extra=None): remembers the value and returns it"},
+    {"__reduce__", memo_reduce, METH_NOARGS, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyTypeObject MemoType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+PyMethodDef module_methods[] = {
+    {"attention_fwd", (PyCFunction)(void*)py_attention_fwd, METH_FASTCALL, nullptr},
+    {"layer_attention", (PyCFunction)(void*)py_layer_attention, METH_FASTCALL, nullptr},
+    {"quantize_e4m3", (PyCFunction)(void*)py_quantize, METH_FASTCALL, nullptr},
+    {"mask_bounds", (PyCFunction)(void*)py_mask_bounds, METH_FASTCALL, nullptr},
+    {"register_lut_source", py_register_lut_source, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", "Native host path of the operators.", -1, module_methods};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  MemoType.tp_name = "flashdeberta_amd._native.Memo";
+  MemoType.tp_basicsize = sizeof(MemoObject);
+  MemoType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
+  MemoType.tp_doc = "One remembered value, valid while the tensors it was computed from are unchanged.";
+  MemoType.tp_new = memo_new;
+  MemoType.tp_traverse = memo_traverse;
+  MemoType.tp_clear = memo_gc_clear;
+  MemoType.tp_dealloc = memo_dealloc;
+  MemoType.tp_methods = memo_methods;
+  if (PyType_Ready(&MemoType) < 0) return nullptr;
+  PyObject* m = PyModule_Create(&module_def);
+  if (!m) return nullptr;
+  Py_INCREF(&MemoType);
+  PyModule_AddObject(m, "Memo", (PyObject*)&MemoType);
+  return m;
+}

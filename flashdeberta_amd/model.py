@@ -10,7 +10,6 @@ here); attention-probability dropout is not applied (nor is it on the reference'
 on the relative embeddings remains, model.py:159-160).
 """
 import math
-import weakref
 
 import torch
 import torch.nn.functional as F
@@ -22,39 +21,14 @@ from transformers.models.deberta_v2.modeling_deberta_v2 import (
 )
 
 from . import ops
+from ._lib import native
 from .padding import key_padding_mask, seq_bounds
 
 
-def _stamp(t):
-    """What a remembered value depends on besides the tensor object: its in-place version counter, and the
-    storage, dtype and device behind it (`p.data = x`, `module.to(dtype)` and `.half()` swap those under
-    an unchanged object and version)."""
-    return (t._version, t.data_ptr(), t.dtype, t.device)
-
-
-class _Memo:
-    """One remembered value, valid while the tensors it was computed from are the same objects, have not
-    been written in place, still sit in the same storage with the same dtype on the same device, and
-    `extra` compares equal.  The tensors are held weakly."""
-
-    def __init__(self):
-        self._state = ((), (), None, None)  # (weak references, stamps, extra, value): replaced as a whole, read once
-
-    def get(self, tensors, extra=None):
-        refs, stamps, old_extra, value = self._state
-        if len(refs) != len(tensors) or extra != old_extra:
-            return None
-        for ref, stamp, t in zip(refs, stamps, tensors):
-            if ref() is not t or _stamp(t) != stamp:
-                return None
-        return value
-
-    def put(self, tensors, value, extra=None):
-        self._state = (tuple(weakref.ref(t) for t in tensors), tuple(_stamp(t) for t in tensors), extra, value)
-        return value
-
-    def __reduce__(self):  # copies and pickles of a module start with nothing remembered
-        return (_Memo, ())
+# One remembered value, valid while the tensors it was computed from are the same objects, have not been written in
+# place, still sit in the same storage with the same dtype on the same device, and `extra` compares equal; the tensors
+# are held weakly: get(tensors, extra=None), put(tensors, value, extra=None).
+_Memo = native.Memo
 
 
 def _seq_bounds_of(attention_mask, memo):
@@ -64,9 +38,18 @@ def _seq_bounds_of(attention_mask, memo):
     in place.  Nothing is stored on the caller's tensor and nothing is process-global."""
     hit = memo.get((attention_mask,))
     if hit is None:
-        start, length, _ = seq_bounds(key_padding_mask(attention_mask))
-        hit = memo.put((attention_mask,), (start, length))
+        hit = native.mask_bounds(attention_mask)  # one launch; None where it does not read the mask (CPU, odd forms)
+        if hit is None:
+            hit = seq_bounds(key_padding_mask(attention_mask))[:2]
+        memo.put((attention_mask,), hit)
     return hit
+
+
+def _weight_and_bias(module):
+    """A projection's parameters; a plain Linear's without nn.Module's attribute machinery (a quarter of a microsecond each)."""
+    if type(module) is torch.nn.Linear:
+        return module._parameters["weight"], module._parameters["bias"]
+    return module.weight, module.bias
 
 
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
@@ -88,15 +71,17 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
 
     def _fused_qkv(self):
         """Concatenated [3*H*D, hidden] weight and bias of the query, key and value projections."""
-        projs = (self.query_proj, self.key_proj, self.value_proj)
-        params = tuple(p.weight for p in projs) + tuple(p.bias for p in projs if p.bias is not None)
-        if len(params) not in (3, 6):
+        modules = self._modules
+        (qw, qb), (kw, kb), (vw, vb) = [_weight_and_bias(modules[n]) for n in ("query_proj", "key_proj", "value_proj")]
+        with_bias = qb is not None and kb is not None and vb is not None
+        if not with_bias and not (qb is None and kb is None and vb is None):
             return None
+        params = (qw, kw, vw, qb, kb, vb) if with_bias else (qw, kw, vw)
         hit = self._qkv_memo.get(params)
         if hit is None:
             with torch.no_grad():
-                w = torch.cat([p.weight for p in projs], dim=0)
-                b = torch.cat([p.bias for p in projs], dim=0) if len(params) == 6 else None
+                w = torch.cat([qw, kw, vw], dim=0)
+                b = torch.cat([qb, kb, vb], dim=0) if with_bias else None
             hit = self._qkv_memo.put(params, (w, b))
         return hit
 
@@ -120,15 +105,15 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             return None, None
         # the position projections exist only for the terms the module has (transformers :170-178)
         kproj = qproj = None
+        modules = self._modules
         if "c2p" in self.pos_att_type:
-            kproj = self.key_proj if self.share_att_key else self.pos_key_proj
+            kproj = modules["key_proj" if self.share_att_key else "pos_key_proj"]
         if "p2c" in self.pos_att_type:
-            qproj = self.query_proj if self.share_att_key else self.pos_query_proj
+            qproj = modules["query_proj" if self.share_att_key else "pos_query_proj"]
         key = None
         recording = torch.is_grad_enabled() and (rel_embeddings.requires_grad or self.query_proj.weight.requires_grad)
         if not self.training and not recording:  # a remembered K_r / Q_r must not carry an autograd graph
-            key = (rel_embeddings,) + tuple(p for m in (kproj, qproj) if m is not None for p in (m.weight, m.bias)
-                                            if p is not None)
+            key = (rel_embeddings,) + tuple(p for m in (kproj, qproj) if m is not None for p in _weight_and_bias(m) if p is not None)
             hit = self._pos_memo.get(key, tuple(self.pos_att_type))
             if hit is not None:
                 return hit
@@ -156,8 +141,9 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             query_states = hidden_states
         B, L, _ = hidden_states.shape
         H, D = self.num_attention_heads, self.attention_head_size
-
-        q, k, v = self._qkv(hidden_states, query_states)
+        # nothing recorded: the projections run as one product over the concatenated weights
+        recording = torch.is_grad_enabled() and (hidden_states.requires_grad or self.query_proj.weight.requires_grad)
+        fused = None if (self.training or recording or query_states is not hidden_states) else self._fused_qkv()
         pos_key, pos_query = self._pos_layers(rel_embeddings)
 
         scale_factor = 1 + ("c2p" in self.pos_att_type and pos_key is not None) + \
@@ -174,6 +160,14 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             # arbitrary masks).
             seq_start, seq_len = _seq_bounds_of(attention_mask, self._mask_memo)
 
+        buckets = self.position_buckets if self.relative_attention else 0
+        max_distance = self.max_relative_positions if self.relative_attention else 0
+        if fused is not None and not self.fp8_qk and not (
+                torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (pos_key, pos_query))):
+            return (native.layer_attention(hidden_states, fused[0], fused[1], pos_key, pos_query, H, sm_scale, buckets, max_distance,
+                                           seq_start, seq_len), None)
+
+        q, k, v = self._qkv(hidden_states, query_states)
         kw = {}
         if self.fp8_qk:
             if q.dtype != torch.bfloat16:
@@ -201,9 +195,7 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
 
         ctx = ops.disentangled_attention(
             q, k, v, pos_key, pos_query, sm_scale=sm_scale,
-            position_buckets=self.position_buckets if self.relative_attention else 0,
-            max_relative_positions=self.max_relative_positions if self.relative_attention else 0,
-            seq_start=seq_start, seq_len=seq_len, **kw)
+            position_buckets=buckets, max_relative_positions=max_distance, seq_start=seq_start, seq_len=seq_len, **kw)
         return (ctx.view(B, L, H * D), None)
 
 

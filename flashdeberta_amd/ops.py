@@ -14,7 +14,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import FdbAttnArgs, check, lib
+from ._lib import FdbAttnArgs, check, lib, native
 
 _DTYPES = {torch.float32: _lib.FDB_F32, torch.bfloat16: _lib.FDB_BF16, torch.float16: _lib.FDB_F16}
 _FP8 = torch.float8_e4m3fn
@@ -61,6 +61,9 @@ def delta_lut_device(position_buckets, max_relative_positions, device):
         hit = (torch.from_numpy(host).to(device), radius)
         _lut_dev_cache[key] = hit
     return hit
+
+
+native.register_lut_source(delta_lut_device)
 
 
 def _stream_ptr(device):
@@ -115,125 +118,14 @@ def disentangled_attention_fwd(q, k, v, pos_key=None, pos_query=None, *, cu_seql
        GPU must not overlap), so with `out` given nothing is allocated on the way; single_kernel is not
        available there.
     """
-    if not q.is_cuda:
-        raise RuntimeError("disentangled_attention_fwd runs on the GPU only; got device %s" % q.device)
-    varlen = cu_seqlens is not None
-    if varlen:
-        if q.dim() != 3:
-            raise ValueError("with cu_seqlens, q/k/v must be [T, H, D]")
-        T, H, D = q.shape
-        B = cu_seqlens.numel() - 1
-        L = int(max_seqlen) if max_seqlen is not None else T
-        if cu_seqlens.dtype != torch.int32 or not cu_seqlens.is_cuda:
-            raise ValueError("cu_seqlens must be an int32 tensor on the GPU")
-    else:
-        if q.dim() != 4:
-            raise ValueError("q/k/v must be [B, L, H, D] (or [T, H, D] with cu_seqlens)")
-        B, L, H, D = q.shape
-        T = B * L
-    if k.shape != q.shape or v.shape != q.shape:
-        raise ValueError("q, k, v must have the same shape (self-attention): %s %s %s"
-                         % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
-    fp8 = q.dtype == _FP8
-    if fp8:
-        if k.dtype != _FP8 or v.dtype != torch.bfloat16:
-            raise ValueError("fp8 path: q and k float8_e4m3fn, v bfloat16")
-        if q_scale is None or k_scale is None or (pos_key is not None and pos_key_scale is None) or (
-                pos_query is not None and pos_query_scale is None):
-            raise ValueError("fp8 path: q_scale, k_scale and a scale for each position tensor are required")
-        dt = _lib.FDB_FP8_E4M3
-    else:
-        if q.dtype not in _DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
-            raise ValueError("unsupported dtypes %s %s %s" % (q.dtype, k.dtype, v.dtype))
-        dt = _DTYPES[q.dtype]
-    q, k, v = [x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v)]
-    span = att_span(position_buckets, max_relative_positions)
-    pos_key = _pos_arg(pos_key, H, D, span, "pos_key")
-    pos_query = _pos_arg(pos_query, H, D, span, "pos_query")
-    for pname, x in (("pos_key", pos_key), ("pos_query", pos_query)):
-        if x is not None and x.dtype != q.dtype:
-            raise ValueError("%s dtype %s does not match q dtype %s" % (pname, x.dtype, q.dtype))
-    n_terms = 1 + (pos_key is not None) + (pos_query is not None)
-    if sm_scale is None:
-        sm_scale = 1.0 / math.sqrt(D * n_terms)
+    return native.attention_fwd(q, k, v, pos_key, pos_query, cu_seqlens, max_seqlen, sm_scale, position_buckets, max_relative_positions,
+                                causal, return_lse, seq_start, seq_len, q_scale, k_scale, pos_key_scale, pos_query_scale, out,
+                                single_kernel, far_splits, near_splits, workspace, no_alloc, _part, _packed_workspace_bytes)
 
-    a = FdbAttnArgs()
-    keep = []
-    if pos_key is not None or pos_query is not None:
-        lut, radius = delta_lut_device(position_buckets, max_relative_positions, q.device)
-        a.delta_lut, a.lut_radius, a.att_span = lut.data_ptr(), radius, span
-    if out is None:
-        out = torch.empty(q.shape, dtype=v.dtype, device=q.device)
-    elif out.shape != q.shape or out.dtype != v.dtype or out.stride(-1) != 1:
-        raise ValueError("out must have q's shape, v's dtype and a unit stride on D")
-    # the log-sum-exp buffer is also the hand-over between the far-tile and near-tile launches, so it is
-    # always provided when a position term is present (T*H floats)
-    if no_alloc and (single_kernel or workspace is not None):
-        raise ValueError("no_alloc excludes single_kernel and a caller-owned workspace")
-    want_lse = return_lse or ((pos_key is not None or pos_query is not None) and not single_kernel and not no_alloc)
-    lse = torch.empty((T, H), dtype=torch.float32, device=q.device) if want_lse else None
-    a.q, a.k, a.v, a.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    a.pos_key, a.pos_query = (_ptr(pos_key) or ctypes.c_void_p()).value, (_ptr(pos_query) or ctypes.c_void_p()).value
-    a.lse = lse.data_ptr() if lse is not None else None
-    if varlen:
-        for n, x in (("q", q), ("k", k), ("v", v), ("o", out)):
-            setattr(a, n + "_stride_b", 0)
-            setattr(a, n + "_stride_t", x.stride(0))
-            setattr(a, n + "_stride_h", x.stride(1))
-        a.cu_seqlens = cu_seqlens.data_ptr()
-        if not no_alloc:
-            wl = torch.empty(int(lib.fdb_worklist_ints(T, B)), dtype=torch.int32, device=q.device)
-            keep.append(wl)
-            check(lib.fdb_build_worklist(_ptr(cu_seqlens), B, T, _ptr(wl), _stream_ptr(q.device)), "fdb_build_worklist")
-            a.worklist = wl.data_ptr()
-    else:
-        for n, x in (("q", q), ("k", k), ("v", v), ("o", out)):
-            setattr(a, n + "_stride_b", x.stride(0))
-            setattr(a, n + "_stride_t", x.stride(1))
-            setattr(a, n + "_stride_h", x.stride(2))
-        for n, x in (("seq_start", seq_start), ("seq_len", seq_len)):
-            if x is not None:
-                if x.dtype != torch.int32 or not x.is_cuda or x.numel() != B:
-                    raise ValueError("%s must be an int32 GPU tensor with one entry per batch row" % n)
-                x = x.contiguous()
-                keep.append(x)
-                setattr(a, n, x.data_ptr())
-    if pos_key is not None:
-        a.pk_stride_h, a.pk_stride_r = pos_key.stride(0), pos_key.stride(1)
-    if pos_query is not None:
-        a.pq_stride_h, a.pq_stride_r = pos_query.stride(0), pos_query.stride(1)
-    if fp8:
-        scales = {"q_scale": q_scale, "k_scale": k_scale, "pk_scale": pos_key_scale, "pq_scale": pos_query_scale}
-        for n, s in scales.items():
-            if s is not None:
-                if s.dtype != torch.float32 or s.numel() != H or not s.is_cuda:
-                    raise ValueError("%s must be a float32 GPU tensor with one entry per head" % n)
-                s = s.contiguous()
-                keep.append(s)
-                setattr(a, n, s.data_ptr())
-    a.batch, a.heads, a.head_dim, a.max_seqlen, a.total_tokens = B, H, D, L, T
-    a.dtype, a.causal, a.sm_scale, a.far_splits = dt, int(bool(causal)), float(sm_scale), int(far_splits)
-    a.near_splits = int(near_splits)
-    with torch.cuda.device(q.device):
-        if no_alloc:
-            check(lib.fdb_attn_fwd_noalloc(ctypes.byref(a), _stream_ptr(q.device)), "fdb_attn_fwd_noalloc")
-            return (out, lse) if return_lse else out
-        if workspace is not None:
-            if workspace.dtype != torch.uint8 or not workspace.is_cuda or not workspace.is_contiguous():
-                raise ValueError("workspace must be a contiguous uint8 GPU tensor")
-            if workspace.numel() > 0:
-                a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
-        else:
-            ws_bytes = lib.fdb_attn_workspace_bytes(ctypes.byref(a))
-            if ws_bytes > 0:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-                keep.append(ws)
-                a.workspace, a.workspace_bytes = ws.data_ptr(), ws_bytes
-        if _part:  # measurement only (bench.py): 1 = the far launch alone, 2 = the near launch alone; `out` is then no result
-            check(lib.fdb_attn_fwd_part(ctypes.byref(a), int(_part), _stream_ptr(q.device)), "fdb_attn_fwd_part")
-        else:
-            check(lib.fdb_attn_fwd(ctypes.byref(a), _stream_ptr(q.device)), "fdb_attn_fwd")
-    return (out, lse) if return_lse else out
+
+def _packed_workspace_bytes(args_address):
+    """What the library asks for a packed call: its shares follow from the mean length (see fdb_attn_workspace_bytes)."""
+    return lib.fdb_attn_workspace_bytes(ctypes.byref(FdbAttnArgs.from_address(args_address)))
 
 
 def _scores_f32(x, pos_t):
@@ -553,42 +445,13 @@ def flash_attention_with_disentangled_varlen(q, k, v, q_pos, k_pos, cu_seqlens_q
 def quantize_e4m3_per_head(x):
     """x: bf16 [..., H, D] on the GPU -> (float8_e4m3fn tensor of the same shape, float32 scales [H]);
     scale[h] = max(absmax over everything but h, 1e-12) / 448, y = e4m3_rne(x / scale[h])."""
-    if not x.is_cuda or x.dtype != torch.bfloat16:
-        raise ValueError("quantize_e4m3_per_head expects a bfloat16 GPU tensor")
-    H, D = x.shape[-2], x.shape[-1]
-    x3 = x.reshape(-1, H, D)
-    if x3.stride(2) != 1:
-        x3 = x3.contiguous()
-    y = torch.empty(x3.shape, dtype=torch.uint8, device=x.device)
-    scale = torch.empty(H, dtype=torch.float32, device=x.device)
-    ws = torch.empty(H, dtype=torch.int32, device=x.device)
-    with torch.cuda.device(x.device):
-        check(lib.fdb_quant_e4m3_per_head(_ptr(x3), x3.stride(0), x3.stride(1), _ptr(y), y.stride(0), y.stride(1),
-                                          _ptr(scale), _ptr(ws), x3.shape[0], H, D, _stream_ptr(x.device)),
-              "fdb_quant_e4m3_per_head")
-    return y.view(_FP8).reshape(x.shape), scale
+    return native.quantize_e4m3(x, None)
 
 
 def quantize_e4m3_per_head_pair(x0, x1):
     """quantize_e4m3_per_head for two bf16 tensors of one shape and one set of strides (q and k of a layer, K_r and
     Q_r) in the same three launches -> (y0, scale0, y1, scale1).  Tensors whose layouts differ are made contiguous."""
-    for x in (x0, x1):
-        if not x.is_cuda or x.dtype != torch.bfloat16:
-            raise ValueError("quantize_e4m3_per_head_pair expects bfloat16 GPU tensors")
-    if x0.shape != x1.shape:
-        raise ValueError("quantize_e4m3_per_head_pair: shapes differ: %s %s" % (tuple(x0.shape), tuple(x1.shape)))
-    H, D = x0.shape[-2], x0.shape[-1]
-    a, b = x0.reshape(-1, H, D), x1.reshape(-1, H, D)
-    if a.stride() != b.stride() or a.stride(2) != 1:
-        a, b = a.contiguous(), b.contiguous()
-    y = torch.empty((2,) + tuple(a.shape), dtype=torch.uint8, device=a.device)
-    scale = torch.empty((2, H), dtype=torch.float32, device=a.device)
-    ws = torch.empty(2 * H, dtype=torch.int32, device=a.device)
-    with torch.cuda.device(a.device):
-        check(lib.fdb_quant_e4m3_per_head_pair(_ptr(a), _ptr(b), a.stride(0), a.stride(1), _ptr(y[0]), _ptr(y[1]), y.stride(1), y.stride(2),
-                                               _ptr(scale[0]), _ptr(scale[1]), _ptr(ws), a.shape[0], H, D, _stream_ptr(a.device)),
-              "fdb_quant_e4m3_per_head_pair")
-    return y[0].view(_FP8).reshape(x0.shape), scale[0], y[1].view(_FP8).reshape(x1.shape), scale[1]
+    return native.quantize_e4m3(x0, x1)
 
 
 def dequantize_e4m3_per_head(y, scale):

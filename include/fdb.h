@@ -294,6 +294,16 @@ int32_t fdb_worklist_max_tiles(int32_t total_tokens, int32_t batch);
 /* Rows of one q-tile (the work-list granularity). */
 int32_t fdb_tile_rows(void);
 
+/*
+ * The bounds of a padded batch from its mask, on the device: token l of row b is real where the element at
+ * mask + (b * stride_b + l * stride_l) elements is not zero.  seq_start[b] = the first real token (0 if there is none),
+ * seq_len[b] = the number of real tokens, or -1 where masked tokens lie between real ones (fdb_attn_args.seq_len's mark for
+ * a row the kernels cannot honour).  elem_size: 1, 2, 4 or 8 bytes; is_float: the element's sign bit alone (-0.0) counts as
+ * zero.  Replaces the host syncs of the reference's unpadding (src/flashdeberta/padding.py:79-88).
+ */
+int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64_t stride_b, int64_t stride_l, int32_t batch,
+                    int32_t length, int32_t* seq_start, int32_t* seq_len, void* stream);
+
 /* Enqueue the device-side work-list construction from cu_seqlens. */
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens,
                        int32_t* worklist, void* stream);
