@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libfdb_hip.so")
 NATIVE = os.path.join(PKG, "_native.so")
-SOURCES = ["fdb_api.cpp", "fdb_attn.hip", "fdb_near.hip", "fdb_fp8.hip", "fdb_aux.hip", "fdb_bwd.hip", "fdb_chain.hip"]
+SOURCES = ["fdb_api.cpp", "fdb_attn.hip", "fdb_near.hip", "fdb_fp8.hip", "fdb_aux.hip", "fdb_bwd.hip", "fdb_chain.hip", "fdb_linear.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-x", "hip",
@@ -54,7 +54,7 @@ def _compile_native():
 
 def _link_native(obj, torch_lib):
     cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", NATIVE, obj, "-L" + PKG, "-l:libfdb_hip.so", "-Wl,-rpath,$ORIGIN",
-           "-L" + torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+           "-L" + torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lhipblaslt"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     os.remove(obj)
     if r.returncode != 0:

@@ -568,6 +568,17 @@ int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64
   return fdb_launch_mask_bounds(mask, elem_size, is_float != 0, stride_b, stride_l, batch, length, seq_start, seq_len, stream);
 }
 
+int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_t rows, int32_t cols, int32_t depth, int64_t ldx,
+               int64_t ldw, int64_t ldo, int32_t dtype, void* stream) {
+  if (!x || !w || !out) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  if (rows < 1 || cols < 2 || depth < 32 || cols % 2 || depth % 32 || ldx < depth || ldw < depth || ldo < cols || ldo % 2 ||
+      (rows + 15) / 16 > 65535)
+    return FDB_ERR_SHAPE;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || (reinterpret_cast<uintptr_t>(bias) & 1u)) return FDB_ERR_ALIGN;
+  return fdb_launch_linear(x, w, bias, out, rows, cols, depth, ldx, ldw, ldo, dtype, stream);
+}
+
 int32_t fdb_delta_lut_radius(int32_t position_buckets, int32_t max_position) {
   if (!lut_config_ok(position_buckets, max_position)) return FDB_ERR_LUT_ARGS;
   const int32_t span = position_buckets > 0 ? position_buckets : max_position;

@@ -166,6 +166,8 @@ int fdb_launch_merge(const FdbKParams& p, int dtype, void* stream);
 // fdb_launch_merge_parts: after a one-kernel launch with key_parts > 1: out (and lse, when given) from the key_parts
 // partial results in the workspace (any element type and head_dim).
 int fdb_launch_merge_parts(const FdbKParams& p, int dtype, int head_dim, void* stream);
+int fdb_launch_linear(const void* x, const void* w, const void* bias, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldw,
+                      int64_t ldo, int dtype, void* stream);  // fdb_linear.hip
 int fdb_launch_mask_bounds(const void* mask, int elem_size, bool is_float, int64_t stride_b, int64_t stride_l, int32_t batch, int32_t length,
                            int32_t* start, int32_t* len, void* stream);
 int fdb_launch_worklist(const int32_t* cu, int32_t batch, int32_t* wl, int32_t max_tiles, void* stream);

@@ -10,8 +10,10 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/HIPContextLight.h>
 #include <c10/hip/HIPGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <hipblaslt/hipblaslt.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -81,6 +83,152 @@ int fdb_dtype_of(at::ScalarType t) {
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
 int64_t att_span(int64_t buckets, int64_t max_relative) { return buckets > 0 ? buckets : max_relative; }
+
+// ---- matrix products -----------------------------------------------------------------------------------------------
+// The projections around the attention are plain products, which hipBLASLt does; torch's own call of it costs the host
+// 17 us (it builds descriptors and asks for the heuristic's choice each time), more than the GPU needs for the product of a
+// short batch.  Here both are kept per (shape, strides, type, epilogue) and the call is the launch alone.
+//   D [M, N] (row stride ldd) = op(A) op(B) (+ bias over N) (+ D): row-major matrices, A [M, K] or its transpose, B [K, N] or its transpose.
+struct GemmKey {
+  int64_t m, n, k, lda, ldb, ldd, batch, sa, sb, sd;
+  int32_t device, type, out_type, flags;  // flags: 1 A transposed, 2 B transposed, 4 bias, 8 accumulate onto D
+  bool operator<(const GemmKey& o) const {
+    return std::tie(m, n, k, lda, ldb, ldd, batch, sa, sb, sd, device, type, out_type, flags) <
+           std::tie(o.m, o.n, o.k, o.lda, o.ldb, o.ldd, o.batch, o.sa, o.sb, o.sd, o.device, o.type, o.out_type, o.flags);
+  }
+};
+struct GemmPlan {
+  hipblasLtMatmulDesc_t desc = nullptr;
+  hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
+  hipblasLtMatmulAlgo_t algo;
+  int64_t workspace = 0;
+  ~GemmPlan() {
+    if (a) hipblasLtMatrixLayoutDestroy(a);
+    if (b) hipblasLtMatrixLayoutDestroy(b);
+    if (d) hipblasLtMatrixLayoutDestroy(d);
+    if (desc) hipblasLtMatmulDescDestroy(desc);
+  }
+};
+constexpr size_t kMostPlans = 512;  // a plan is a few hundred bytes; a program with more shapes than this starts over
+
+void blas(hipblasStatus_t s, const char* what) { TORCH_CHECK(s == HIPBLAS_STATUS_SUCCESS, what, " failed: hipBLASLt status ", (int)s); }
+
+hipDataType blas_type(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return HIP_R_32F;
+    case at::kBFloat16: return HIP_R_16BF;
+    case at::kHalf: return HIP_R_16F;
+    default: TORCH_CHECK_VALUE(false, "unsupported dtype ", t);
+  }
+}
+
+hipblasLtHandle_t blas_handle(int device) {
+  static hipblasLtHandle_t handles[64] = {};
+  if (!handles[device]) blas(hipblasLtCreate(&handles[device]), "hipblasLtCreate");
+  return handles[device];
+}
+
+// The library is column-major: D^T [N, M] = op(B)^T op(A)^T, so B's memory is its first operand and A's the second.
+std::map<GemmKey, GemmPlan> g_plans;  // reached with the GIL held
+GemmPlan& gemm_plan(const GemmKey& key) {
+  const auto hit = g_plans.find(key);
+  if (hit != g_plans.end()) return hit->second;
+  if (g_plans.size() >= kMostPlans) g_plans.clear();
+  GemmPlan& p = g_plans[key];
+  try {
+    blas(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F), "hipblasLtMatmulDescCreate");
+    const auto set = [&](hipblasLtMatmulDescAttributes_t what, const void* v, size_t n) { blas(hipblasLtMatmulDescSetAttribute(p.desc, what, v, n), "hipblasLtMatmulDescSetAttribute"); };
+    const hipblasOperation_t op_first = key.flags & 2 ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_second = key.flags & 1 ? HIPBLAS_OP_T : HIPBLAS_OP_N;
+    set(HIPBLASLT_MATMUL_DESC_TRANSA, &op_first, sizeof(op_first));
+    set(HIPBLASLT_MATMUL_DESC_TRANSB, &op_second, sizeof(op_second));
+    const auto in = (hipDataType)key.type, out = (hipDataType)key.out_type;
+    if (key.flags & 4) {
+      const hipblasLtEpilogue_t e = HIPBLASLT_EPILOGUE_BIAS;
+      set(HIPBLASLT_MATMUL_DESC_EPILOGUE, &e, sizeof(e));
+      set(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &in, sizeof(in));
+    }
+    // row-major [M, K] with row stride lda is column-major [K, M]
+    blas(hipblasLtMatrixLayoutCreate(&p.a, in, key.flags & 2 ? key.k : key.n, key.flags & 2 ? key.n : key.k, key.ldb), "hipblasLtMatrixLayoutCreate");
+    blas(hipblasLtMatrixLayoutCreate(&p.b, in, key.flags & 1 ? key.m : key.k, key.flags & 1 ? key.k : key.m, key.lda), "hipblasLtMatrixLayoutCreate");
+    blas(hipblasLtMatrixLayoutCreate(&p.d, out, key.n, key.m, key.ldd), "hipblasLtMatrixLayoutCreate");
+    if (key.batch > 1) {
+      const int32_t count = (int32_t)key.batch;
+      const std::pair<hipblasLtMatrixLayout_t, int64_t> ls[] = {{p.a, key.sb}, {p.b, key.sa}, {p.d, key.sd}};
+      for (const auto& l : ls) {
+        blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &count, sizeof(count)), "hipblasLtMatrixLayoutSetAttribute");
+        blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &l.second, sizeof(l.second)), "hipblasLtMatrixLayoutSetAttribute");
+      }
+    }
+    hipblasLtMatmulPreference_t pref = nullptr;
+    blas(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
+    const size_t most = at::cuda::getCUDABlasLtWorkspaceSize();  // torch's own bound, so that the choice is torch's own
+    hipblasLtMatmulHeuristicResult_t found = {};
+    int n = 0;
+    hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most, sizeof(most));
+    const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(blas_handle(key.device), p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
+    hipblasLtMatmulPreferenceDestroy(pref);
+    blas(rc, "hipblasLtMatmulAlgoGetHeuristic");
+    TORCH_CHECK(n > 0, "hipBLASLt has no kernel for this product");
+    p.algo = found.algo;
+    p.workspace = (int64_t)found.workspaceSize;
+  } catch (...) {
+    g_plans.erase(key);
+    throw;
+  }
+  return p;
+}
+
+struct Mat {  // `batch` row-major matrices, `ld` elements between rows, `stride` elements between matrices
+  const void* p;
+  int64_t ld, stride = 0;
+};
+void gemm(const Tensor& on, at::ScalarType type, at::ScalarType out_type, bool trans_a, bool trans_b, int64_t batch, int64_t m, int64_t n, int64_t k,
+          Mat a, Mat b, Mat d, const void* bias = nullptr, bool accumulate = false) {
+  const int device = on.get_device();
+  GemmPlan& p = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, batch, a.stride, b.stride, d.stride, device, (int32_t)blas_type(type), (int32_t)blas_type(out_type),
+                                  (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
+  if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias, sizeof(bias)), "hipblasLtMatmulDescSetAttribute");
+  Tensor ws;
+  if (p.workspace > 0) ws = at::empty({p.workspace}, on.options().dtype(at::kByte));
+  const float one = 1.f, beta = accumulate ? 1.f : 0.f;
+  blas(hipblasLtMatmul(blas_handle(device), p.desc, &one, b.p, p.a, a.p, p.b, &beta, d.p, p.d, const_cast<void*>(d.p), p.d, &p.algo,
+                       p.workspace > 0 ? ws.data_ptr() : nullptr, p.workspace, (hipStream_t)stream_of(on)),
+       "hipblasLtMatmul");
+}
+
+// x [..., K] . w [N, K]^T + bias -> [..., N], as torch's linear computes it, bit for bit (the heuristic's choice is the same).
+// With `own`, a product of few rows takes the library's kernels instead: up to 32 rows, or while 64 x 64 tiles make one round
+// of workgroups and the contraction is short; beyond that hipBLASLt's larger tiles and its split contraction are faster by more
+// than its call costs the host.
+Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool own) {
+  const auto type = x_in.scalar_type();
+  const bool half = type == at::kBFloat16 || type == at::kHalf;
+  const int64_t k = x_in.size(-1), m = k > 0 ? x_in.numel() / k : 0;
+  if (!x_in.is_cuda() || !half || w.scalar_type() != type || (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 ||
+      w.stride(1) != 1 || k != w.size(1) || !bias || !bias->is_contiguous())
+    return at::linear(x_in, w, bias);
+  const Tensor x = x_in.contiguous();
+  const int64_t n = w.size(0);
+  auto size = x.sizes().vec();
+  size.back() = n;
+  const Tensor out = at::empty(size, x.options());
+  const void* b = bias->data_ptr();
+  if (own && (m <= 32 || (k <= 1536 && ((m + 63) / 64) * ((n + 63) / 64) <= 256))) {
+    const int rc = fdb_linear(x.data_ptr(), w.data_ptr(), b, out.data_ptr(), (int32_t)m, (int32_t)n, (int32_t)k, k, w.stride(0), n, fdb_dtype_of(type), stream_of(x));
+    if (rc == 0) return out;
+    if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
+  }
+  gemm(x, type, type, false, true, 1, m, n, k, {x.data_ptr(), k}, {w.data_ptr(), w.stride(0)}, {out.data_ptr(), n}, b);
+  return out;
+}
+
+// linear(x, weight, bias, own) -> x . weight^T + bias
+PyObject* py_linear(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 4, "linear takes 4 arguments");
+  return THPVariable_Wrap(project(tensor_arg(x[0], "x"), tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), bool_arg(x[3])));
+  END_HANDLE_TH_ERRORS
+}
 
 // ---- the delta table on the device ---------------------------------------------------------------------------------
 // One per (buckets, positions, device), built by the Python callable registered below and kept for the life of the
@@ -176,6 +324,56 @@ void launch_forward(fdb_attn_args& a, const Tensor& on, bool need_lse, const Fwd
   else check(fdb_attn_fwd(&a, stream), "fdb_attn_fwd");
 }
 
+// The rest of a call whose q, k, v, out, sizes and dtype are in `a`: position tensors, row bounds, scales, scratch, launches.
+// `on`: a tensor of the device; returns the log-sum-exp tensor where the caller asked for it.
+Tensor run_forward(fdb_attn_args& a, const Tensor& on, at::ScalarType qt, const Fwd& o) {
+  const int64_t B = a.batch, H = a.heads, D = a.head_dim, span = att_span(o.buckets, o.max_relative);
+  Tensor pk, pq;
+  if (o.pos_key) pk = pos_arg(*o.pos_key, H, D, span, "pos_key");
+  if (o.pos_query) pq = pos_arg(*o.pos_query, H, D, span, "pos_query");
+  TORCH_CHECK_VALUE(!pk.defined() || pk.scalar_type() == qt, "pos_key dtype ", pk.scalar_type(), " does not match q dtype ", qt);
+  TORCH_CHECK_VALUE(!pq.defined() || pq.scalar_type() == qt, "pos_query dtype ", pq.scalar_type(), " does not match q dtype ", qt);
+  const bool has_pos = pk.defined() || pq.defined();
+  const int terms = 1 + (pk.defined() ? 1 : 0) + (pq.defined() ? 1 : 0);
+  if (has_pos) {
+    const Lut& lut = lut_for(o.buckets, o.max_relative, on);
+    a.delta_lut = (const int16_t*)lut.table.data_ptr();
+    a.lut_radius = lut.radius;
+    a.att_span = (int32_t)span;
+  }
+  TORCH_CHECK_VALUE(!o.no_alloc || (!o.single_kernel && !o.workspace), "no_alloc excludes single_kernel and a caller-owned workspace");
+  // The log-sum-exp buffer is also the hand-over between the far-tile and near-tile launches, so it is always provided
+  // when a position term is present (T*H floats), unless the caller wants one kernel.
+  Tensor lse;
+  if (o.return_lse) {
+    lse = at::empty({a.total_tokens, H}, on.options().dtype(at::kFloat));
+    a.lse = (float*)lse.data_ptr();
+  }
+  std::vector<Tensor> keep;
+  if (o.cu) {
+    a.cu_seqlens = (const int32_t*)o.cu->data_ptr();
+  } else {
+    const char* what = "an int32 GPU tensor with one entry per batch row";
+    if (o.seq_start) a.seq_start = (const int32_t*)vector_arg(*o.seq_start, at::kInt, B, "seq_start", what, keep);
+    if (o.seq_len) a.seq_len = (const int32_t*)vector_arg(*o.seq_len, at::kInt, B, "seq_len", what, keep);
+  }
+  if (pk.defined()) a.pos_key = pk.data_ptr(), a.pk_stride_h = pk.stride(0), a.pk_stride_r = pk.stride(1);
+  if (pq.defined()) a.pos_query = pq.data_ptr(), a.pq_stride_h = pq.stride(0), a.pq_stride_r = pq.stride(1);
+  if (a.dtype == FDB_FP8_E4M3) {
+    const char* what = "a float32 GPU tensor with one entry per head";
+    if (o.q_scale) a.q_scale = (const float*)vector_arg(*o.q_scale, at::kFloat, H, "q_scale", what, keep);
+    if (o.k_scale) a.k_scale = (const float*)vector_arg(*o.k_scale, at::kFloat, H, "k_scale", what, keep);
+    if (o.pk_scale) a.pk_scale = (const float*)vector_arg(*o.pk_scale, at::kFloat, H, "pk_scale", what, keep);
+    if (o.pq_scale) a.pq_scale = (const float*)vector_arg(*o.pq_scale, at::kFloat, H, "pq_scale", what, keep);
+  }
+  a.causal = o.causal ? 1 : 0;
+  a.sm_scale = (float)(std::isnan(o.sm_scale) ? 1.0 / std::sqrt((double)(D * terms)) : o.sm_scale);
+  a.far_splits = (int32_t)o.far_splits, a.near_splits = (int32_t)o.near_splits;
+  if (o.no_alloc) check(fdb_attn_fwd_noalloc(&a, stream_of(on)), "fdb_attn_fwd_noalloc");
+  else launch_forward(a, on, has_pos && !o.single_kernel, o);
+  return lse;
+}
+
 std::pair<Tensor, Tensor> forward(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Fwd& o) {
   TORCH_CHECK(q_in.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", q_in.device());
   const bool varlen = o.cu.has_value();
@@ -207,20 +405,6 @@ std::pair<Tensor, Tensor> forward(const Tensor& q_in, const Tensor& k_in, const 
     a.dtype = fdb_dtype_of(qt);
   }
   const Tensor q = unit_last(q_in), k = unit_last(k_in), v = unit_last(v_in);
-  const int64_t span = att_span(o.buckets, o.max_relative);
-  Tensor pk, pq;
-  if (o.pos_key) pk = pos_arg(*o.pos_key, H, D, span, "pos_key");
-  if (o.pos_query) pq = pos_arg(*o.pos_query, H, D, span, "pos_query");
-  TORCH_CHECK_VALUE(!pk.defined() || pk.scalar_type() == qt, "pos_key dtype ", pk.scalar_type(), " does not match q dtype ", qt);
-  TORCH_CHECK_VALUE(!pq.defined() || pq.scalar_type() == qt, "pos_query dtype ", pq.scalar_type(), " does not match q dtype ", qt);
-  const bool has_pos = pk.defined() || pq.defined();
-  const int terms = 1 + (pk.defined() ? 1 : 0) + (pq.defined() ? 1 : 0);
-  if (has_pos) {
-    const Lut& lut = lut_for(o.buckets, o.max_relative, q);
-    a.delta_lut = (const int16_t*)lut.table.data_ptr();
-    a.lut_radius = lut.radius;
-    a.att_span = (int32_t)span;
-  }
   const c10::hip::HIPGuard guard(q.get_device());
   Tensor out;
   if (o.out) {
@@ -230,43 +414,14 @@ std::pair<Tensor, Tensor> forward(const Tensor& q_in, const Tensor& k_in, const 
   } else {
     out = at::empty(q.sizes(), v.options());
   }
-  TORCH_CHECK_VALUE(!o.no_alloc || (!o.single_kernel && !o.workspace), "no_alloc excludes single_kernel and a caller-owned workspace");
-  // The log-sum-exp buffer is also the hand-over between the far-tile and near-tile launches, so it is always provided
-  // when a position term is present (T*H floats), unless the caller wants one kernel.
-  Tensor lse;
-  if (o.return_lse) {
-    lse = at::empty({T, H}, q.options().dtype(at::kFloat));
-    a.lse = (float*)lse.data_ptr();
-  }
   a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr(), a.out = out.data_ptr();
   const int64_t t_ax = varlen ? 0 : 1;
   a.q_stride_b = varlen ? 0 : q.stride(0), a.q_stride_t = q.stride(t_ax), a.q_stride_h = q.stride(t_ax + 1);
   a.k_stride_b = varlen ? 0 : k.stride(0), a.k_stride_t = k.stride(t_ax), a.k_stride_h = k.stride(t_ax + 1);
   a.v_stride_b = varlen ? 0 : v.stride(0), a.v_stride_t = v.stride(t_ax), a.v_stride_h = v.stride(t_ax + 1);
   a.o_stride_b = varlen ? 0 : out.stride(0), a.o_stride_t = out.stride(t_ax), a.o_stride_h = out.stride(t_ax + 1);
-  std::vector<Tensor> keep;
-  if (varlen) {
-    a.cu_seqlens = (const int32_t*)o.cu->data_ptr();
-  } else {
-    const char* what = "an int32 GPU tensor with one entry per batch row";
-    if (o.seq_start) a.seq_start = (const int32_t*)vector_arg(*o.seq_start, at::kInt, B, "seq_start", what, keep);
-    if (o.seq_len) a.seq_len = (const int32_t*)vector_arg(*o.seq_len, at::kInt, B, "seq_len", what, keep);
-  }
-  if (pk.defined()) a.pos_key = pk.data_ptr(), a.pk_stride_h = pk.stride(0), a.pk_stride_r = pk.stride(1);
-  if (pq.defined()) a.pos_query = pq.data_ptr(), a.pq_stride_h = pq.stride(0), a.pq_stride_r = pq.stride(1);
-  if (fp8) {
-    const char* what = "a float32 GPU tensor with one entry per head";
-    if (o.q_scale) a.q_scale = (const float*)vector_arg(*o.q_scale, at::kFloat, H, "q_scale", what, keep);
-    if (o.k_scale) a.k_scale = (const float*)vector_arg(*o.k_scale, at::kFloat, H, "k_scale", what, keep);
-    if (o.pk_scale) a.pk_scale = (const float*)vector_arg(*o.pk_scale, at::kFloat, H, "pk_scale", what, keep);
-    if (o.pq_scale) a.pq_scale = (const float*)vector_arg(*o.pq_scale, at::kFloat, H, "pq_scale", what, keep);
-  }
   a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)T;
-  a.causal = o.causal ? 1 : 0;
-  a.sm_scale = (float)(std::isnan(o.sm_scale) ? 1.0 / std::sqrt((double)(D * terms)) : o.sm_scale);
-  a.far_splits = (int32_t)o.far_splits, a.near_splits = (int32_t)o.near_splits;
-  if (o.no_alloc) check(fdb_attn_fwd_noalloc(&a, stream_of(q)), "fdb_attn_fwd_noalloc");
-  else launch_forward(a, q, has_pos && !o.single_kernel, o);
+  const Tensor lse = run_forward(a, q, qt, o);
   return {out, lse};
 }
 
@@ -313,29 +468,66 @@ PyObject* py_attention_fwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// layer_attention(hidden, weight, bias, pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start,
-//                 seq_len) -> context [B, L, H*D]
 // The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
+// x: pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start, seq_len
+Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, PyObject* const* x, bool own) {
+  TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be [B, L, hidden]");
+  const Tensor qkv = project(hidden, weight, bias, own);
+  TORCH_CHECK(qkv.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", qkv.device());
+  const auto type = qkv.scalar_type();
+  TORCH_CHECK_VALUE(fdb_dtype_of(type) >= 0, "unsupported dtype ", type);
+  const int64_t B = qkv.size(0), L = qkv.size(1), H = int_arg(x[2]), D = qkv.size(2) / (3 * H), width = H * D;
+  Fwd o;
+  o.pos_key = opt_tensor_arg(x[0], "pos_key");
+  o.pos_query = opt_tensor_arg(x[1], "pos_query");
+  o.sm_scale = float_arg(x[3]);
+  o.buckets = int_arg(x[4]);
+  o.max_relative = int_arg(x[5]);
+  o.seq_start = opt_tensor_arg(x[6], "seq_start");
+  o.seq_len = opt_tensor_arg(x[7], "seq_len");
+  const c10::hip::HIPGuard guard(qkv.get_device());
+  const Tensor out = at::empty({B, L, width}, qkv.options());
+  fdb_attn_args a = {};
+  const char* p = (const char*)qkv.data_ptr();
+  const int64_t bytes = width * qkv.element_size();
+  a.dtype = fdb_dtype_of(type);
+  a.q = p, a.k = p + bytes, a.v = p + 2 * bytes, a.out = out.data_ptr();
+  a.q_stride_b = a.k_stride_b = a.v_stride_b = L * 3 * width;
+  a.q_stride_t = a.k_stride_t = a.v_stride_t = 3 * width;
+  a.q_stride_h = a.k_stride_h = a.v_stride_h = a.o_stride_h = D;
+  a.o_stride_b = L * width, a.o_stride_t = width;
+  a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)(B * L);
+  run_forward(a, qkv, type, o);
+  return out;
+}
+
+// layer_attention(hidden, weight, bias, pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start,
+//                 seq_len, own) -> context [B, L, H*D]
 PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK_TYPE(n == 11, "layer_attention takes 11 arguments");
+  TORCH_CHECK_TYPE(n == 12, "layer_attention takes 12 arguments");
+  return THPVariable_Wrap(layer_attention(tensor_arg(x[0], "hidden"), tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), x + 3, bool_arg(x[11])));
+  END_HANDLE_TH_ERRORS
+}
+
+// encoder_layer(hidden, weight, bias, pos_key, ..., seq_len [as layer_attention], out_weight, out_bias, norm1_weight, norm1_bias, eps1,
+//               up_weight, up_bias, down_weight, down_bias, norm2_weight, norm2_bias, eps2) -> hidden states of the next layer
+// A whole post-norm encoder layer with GELU; the caller has checked that the layer is one.  Every product, sum, norm and GELU is
+// the one its modules would run, in the same order, so the result has the same bits: in a 16-bit type twelve layers turn one
+// differing rounding into a percent.
+PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 23, "encoder_layer takes 23 arguments");
   const Tensor& hidden = tensor_arg(x[0], "hidden");
-  const int64_t H = int_arg(x[5]);
-  const Tensor qkv = at::linear(hidden, tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"));
-  const int64_t B = qkv.size(0), L = qkv.size(1), D = qkv.size(2) / (3 * H), width = H * D;
-  const std::array<int64_t, 4> size{B, L, H, D}, stride{L * 3 * width, 3 * width, D, 1};
-  const Tensor all = unit_last(qkv).contiguous();
-  Fwd o;
-  o.pos_key = opt_tensor_arg(x[3], "pos_key");
-  o.pos_query = opt_tensor_arg(x[4], "pos_query");
-  o.sm_scale = float_arg(x[6]);
-  o.buckets = int_arg(x[7]);
-  o.max_relative = int_arg(x[8]);
-  o.seq_start = opt_tensor_arg(x[9], "seq_start");
-  o.seq_len = opt_tensor_arg(x[10], "seq_len");
-  const int64_t at0 = all.storage_offset();
-  const Tensor out = forward(all.as_strided(size, stride, at0), all.as_strided(size, stride, at0 + width), all.as_strided(size, stride, at0 + 2 * width), o).first;
-  return THPVariable_Wrap(out.view({B, L, width}));
+  const auto norm = [](Tensor y, const Tensor& residual, PyObject* const* p) {
+    return at::layer_norm(y.add_(residual), {y.size(-1)}, tensor_arg(p[0], "norm_weight"), tensor_arg(p[1], "norm_bias"), float_arg(p[2]));
+  };
+  const Tensor context = layer_attention(hidden, tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), x + 3, false);
+  const c10::hip::HIPGuard guard(hidden.get_device());
+  const Tensor attended = norm(project(context, tensor_arg(x[11], "out_weight"), opt_tensor_arg(x[12], "out_bias"), false), hidden, x + 13);
+  const Tensor up = project(attended, tensor_arg(x[16], "up_weight"), opt_tensor_arg(x[17], "up_bias"), false);
+  at::gelu_(const_cast<Tensor&>(up));
+  return THPVariable_Wrap(norm(project(up, tensor_arg(x[18], "down_weight"), opt_tensor_arg(x[19], "down_bias"), false), attended, x + 20));
   END_HANDLE_TH_ERRORS
 }
 
@@ -518,6 +710,8 @@ PyTypeObject MemoType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 PyMethodDef module_methods[] = {
     {"attention_fwd", (PyCFunction)(void*)py_attention_fwd, METH_FASTCALL, nullptr},
     {"layer_attention", (PyCFunction)(void*)py_layer_attention, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, nullptr},
+    {"encoder_layer", (PyCFunction)(void*)py_encoder_layer, METH_FASTCALL, nullptr},
     {"quantize_e4m3", (PyCFunction)(void*)py_quantize, METH_FASTCALL, nullptr},
     {"mask_bounds", (PyCFunction)(void*)py_mask_bounds, METH_FASTCALL, nullptr},
     {"register_lut_source", py_register_lut_source, METH_O, nullptr},

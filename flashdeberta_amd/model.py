@@ -13,10 +13,16 @@ import math
 
 import torch
 import torch.nn.functional as F
+from torch.nn.modules import module as nn_module
 from transformers.models.deberta_v2.modeling_deberta_v2 import (
+    DebertaV2Attention,
     DebertaV2Config,
     DebertaV2Encoder,
+    DebertaV2Intermediate,
+    DebertaV2Layer,
     DebertaV2Model,
+    DebertaV2Output,
+    DebertaV2SelfOutput,
     DisentangledSelfAttention,
 )
 
@@ -63,6 +69,10 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     (a copy kept per module, rebuilt when a parameter is replaced or written in place), and K_r / Q_r
     are remembered for as long as the relative embeddings handed in are the same tensor (an encoder
     patched by `patch_model` hands in the same tensor until its embedding table changes)."""
+
+    # Projections of a few rows by the library's own kernels, which start sooner than hipBLASLt's but add up in another order;
+    # off in a patched encoder, whose twelve layers turn one differing rounding of a 16-bit type into a percent.
+    _own_products = True
 
     def __init__(self, config, fp8_qk=None):
         super().__init__(config)
@@ -130,6 +140,36 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             self._pos_memo.put(key, (pos_key, pos_query), tuple(self.pos_att_type))
         return pos_key, pos_query
 
+    def _score_settings(self, pos_key, pos_query):
+        """(sm_scale, position_buckets, max_relative_positions) of the operator (reference model.py:151-157)."""
+        present = not self.relative_attention
+        terms = 1 + ("c2p" in self.pos_att_type and (present or pos_key is not None)) + \
+            ("p2c" in self.pos_att_type and (present or pos_query is not None))
+        sm_scale = 1.0 / math.sqrt(self.attention_head_size * terms)
+        return (sm_scale, self.position_buckets, self.max_relative_positions) if self.relative_attention else (sm_scale, 0, 0)
+
+    def _bounds(self, attention_mask):
+        """(seq_start, seq_len) of the batch.  The kernels take the real tokens of a row as one contiguous run and write
+        zeros into the padded rows themselves; a row whose mask has a hole inside that run carries seq_len -1 and comes
+        back as NaN in every position, so the unsupported mask cannot pass for a result (the eager module honours
+        arbitrary masks)."""
+        return (None, None) if attention_mask is None else _seq_bounds_of(attention_mask, self._mask_memo)
+
+    def _native_args(self, attention_mask, rel_embeddings, hidden_requires_grad):
+        """What follows the hidden states in a call of native.layer_attention, or None where that path does not serve:
+        in training or while anything is recorded (the concatenated weights are a copy made outside autograd), under
+        autocast, with FP8 operands, or with projections that have no weights to concatenate."""
+        if self.training or self.fp8_qk or torch.is_autocast_enabled():
+            return None
+        if torch.is_grad_enabled() and (hidden_requires_grad or (rel_embeddings is not None and rel_embeddings.requires_grad)
+                                        or any(p.requires_grad for p in self.parameters())):
+            return None
+        fused = self._fused_qkv()
+        if fused is None:
+            return None
+        pos_key, pos_query = self._pos_layers(rel_embeddings)
+        return (*fused, pos_key, pos_query, self.num_attention_heads, *self._score_settings(pos_key, pos_query), *self._bounds(attention_mask))
+
     def forward(self, hidden_states, attention_mask, output_attentions=False, query_states=None,
                 relative_pos=None, rel_embeddings=None):
         """-> (context [B, L, H*D], None).  `relative_pos` is ignored: the bucketed relative
@@ -141,31 +181,12 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             query_states = hidden_states
         B, L, _ = hidden_states.shape
         H, D = self.num_attention_heads, self.attention_head_size
-        # nothing recorded: the projections run as one product over the concatenated weights
-        recording = torch.is_grad_enabled() and (hidden_states.requires_grad or self.query_proj.weight.requires_grad)
-        fused = None if (self.training or recording or query_states is not hidden_states) else self._fused_qkv()
+        args = self._native_args(attention_mask, rel_embeddings, hidden_states.requires_grad) if query_states is hidden_states else None
+        if args is not None:
+            return native.layer_attention(hidden_states, *args, self._own_products), None
         pos_key, pos_query = self._pos_layers(rel_embeddings)
-
-        scale_factor = 1 + ("c2p" in self.pos_att_type and pos_key is not None) + \
-            ("p2c" in self.pos_att_type and pos_query is not None)
-        if not self.relative_attention:
-            scale_factor = 1 + ("c2p" in self.pos_att_type) + ("p2c" in self.pos_att_type)  # model.py:151-157
-        sm_scale = 1.0 / math.sqrt(D * scale_factor)
-
-        seq_start = seq_len = None
-        if attention_mask is not None:
-            # The kernels take the real tokens of a row as one contiguous run and write zeros into the padded
-            # rows themselves; a row whose mask has a hole inside that run carries seq_len -1 and comes back as
-            # NaN in every position, so the unsupported mask cannot pass for a result (the eager module honours
-            # arbitrary masks).
-            seq_start, seq_len = _seq_bounds_of(attention_mask, self._mask_memo)
-
-        buckets = self.position_buckets if self.relative_attention else 0
-        max_distance = self.max_relative_positions if self.relative_attention else 0
-        if fused is not None and not self.fp8_qk and not (
-                torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (pos_key, pos_query))):
-            return (native.layer_attention(hidden_states, fused[0], fused[1], pos_key, pos_query, H, sm_scale, buckets, max_distance,
-                                           seq_start, seq_len), None)
+        sm_scale, buckets, max_distance = self._score_settings(pos_key, pos_query)
+        seq_start, seq_len = self._bounds(attention_mask)
 
         q, k, v = self._qkv(hidden_states, query_states)
         kw = {}
@@ -203,6 +224,60 @@ DEBERTA_SELF_ATTENTION_CLASSES = {
     "eager": DisentangledSelfAttention,
     "flash_attention_2": FlashDisentangledSelfAttention,
 }
+
+
+def _hooked(module):
+    return module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+
+
+class FlashDebertaV2Layer(DebertaV2Layer):
+    """transformers' encoder layer whose inference in a 16-bit type is one native call (native.encoder_layer): the same
+    projections, attention, GELU and post-norms, with the same bits, without a module call per step.
+    Anything else -- training, recording, autocast, hooks on any part, a part of another class (adapters, quantised
+    projections, another activation) -- takes transformers' own forward.  Instances are made by `patch_model`."""
+
+    def _native_args(self, hidden_states, attention_mask, rel_embeddings):
+        if self.training or torch.is_grad_enabled() or hidden_states.dtype not in (torch.bfloat16, torch.float16) or not hidden_states.is_cuda \
+                or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or torch.compiler.is_compiling():
+            return None
+        own = self._modules
+        attention, intermediate, output = own["attention"], own["intermediate"], own["output"]
+        if type(attention) is not DebertaV2Attention or type(intermediate) is not DebertaV2Intermediate or type(output) is not DebertaV2Output:
+            return None
+        att, att_out = attention._modules["self"], attention._modules["output"]
+        if type(att) is not FlashDisentangledSelfAttention or type(att_out) is not DebertaV2SelfOutput:
+            return None
+        act = intermediate._modules.get("intermediate_act_fn")
+        linears = att_out._modules["dense"], intermediate._modules["dense"], output._modules["dense"]
+        norms = att_out._modules["LayerNorm"], output._modules["LayerNorm"]
+        if getattr(act, "act", None) is not F.gelu:
+            return None
+        shape = hidden_states.shape[-1:]
+        for m in linears:
+            if type(m) is not torch.nn.Linear or m._parameters["weight"].dtype != hidden_states.dtype:
+                return None
+        for m in norms:
+            if type(m) is not torch.nn.LayerNorm or m.normalized_shape != shape or m._parameters["bias"] is None \
+                    or m._parameters["weight"].dtype != hidden_states.dtype:
+                return None
+        if any(_hooked(m) for m in (attention, intermediate, output, att, att_out, act, *linears, *norms,
+                                      *att._modules.values())):
+            return None
+        args = att._native_args(attention_mask, rel_embeddings, False)
+        if args is None:
+            return None
+        (ow, ob), (uw, ub), (dw, db) = [_weight_and_bias(m) for m in linears]
+        n1, n2 = norms
+        return (*args, ow, ob, n1._parameters["weight"], n1._parameters["bias"], n1.eps, uw, ub, dw, db,
+                n2._parameters["weight"], n2._parameters["bias"], n2.eps)
+
+    def forward(self, hidden_states, attention_mask, query_states=None, relative_pos=None, rel_embeddings=None, output_attentions=False):
+        if query_states is None or query_states is hidden_states:
+            args = self._native_args(hidden_states, attention_mask, rel_embeddings)
+            if args is not None:
+                return native.encoder_layer(hidden_states, *args), None
+        return super().forward(hidden_states, attention_mask, query_states=query_states, relative_pos=relative_pos,
+                               rel_embeddings=rel_embeddings, output_attentions=output_attentions)
 
 
 class FlashDebertaV2Encoder(DebertaV2Encoder):
@@ -260,6 +335,7 @@ def patch_model(model, attn_implementation="flash_attention_2", fp8_qk=False, sk
         if type(old) is cls:
             if cls is FlashDisentangledSelfAttention:
                 old._mask_memo = mask_memo
+                old._own_products = False
             continue
         new = cls(config, fp8_qk=fp8_qk) if cls is FlashDisentangledSelfAttention else cls(config)
         new.load_state_dict(old.state_dict())
@@ -268,8 +344,14 @@ def patch_model(model, attn_implementation="flash_attention_2", fp8_qk=False, sk
         new.train(old.training)
         if cls is FlashDisentangledSelfAttention:
             new._mask_memo = mask_memo
+            new._own_products = False
         layer.attention.self = new
     flash = cls is FlashDisentangledSelfAttention
+    for layer in encoder.layer:
+        if flash and type(layer) is DebertaV2Layer:
+            layer.__class__ = FlashDebertaV2Layer
+        elif not flash and type(layer) is FlashDebertaV2Layer:
+            layer.__class__ = DebertaV2Layer
     # The encoder-side shortcuts live in a subclass that differs from transformers' encoder in three methods
     # only; switching the instance's class keeps copies and pickles of the model working.
     if flash and type(encoder) in (DebertaV2Encoder, FlashDebertaV2Encoder):
@@ -301,4 +383,4 @@ class FlashDebertaV2Model(DebertaV2Model):
 
 
 __all__ = ["FlashDisentangledSelfAttention", "DEBERTA_SELF_ATTENTION_CLASSES", "FlashDebertaV2Model",
-           "FlashDebertaV2Encoder", "DebertaV2Config", "patch_model"]
+           "FlashDebertaV2Encoder", "FlashDebertaV2Layer", "DebertaV2Config", "patch_model"]

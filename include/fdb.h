@@ -304,6 +304,15 @@ int32_t fdb_tile_rows(void);
 int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64_t stride_b, int64_t stride_l, int32_t batch,
                     int32_t length, int32_t* seq_start, int32_t* seq_len, void* stream);
 
+/*
+ * The linear layer in front of the attention for a batch of few rows (FDB_BF16 / FDB_F16):
+ * out [rows, cols] = x [rows, depth] . w [cols, depth]^T (+ bias [cols] or NULL).  Row strides ldx, ldw, ldo in elements, x, w, out
+ * and their rows aligned to 16 bytes; depth a multiple of 32, cols and ldo even.  The reference runs it as torch's module
+ * (src/flashdeberta/model.py:147-149).
+ */
+int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_t rows, int32_t cols, int32_t depth, int64_t ldx,
+               int64_t ldw, int64_t ldo, int32_t dtype, void* stream);
+
 /* Enqueue the device-side work-list construction from cu_seqlens. */
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens,
                        int32_t* worklist, void* stream);

@@ -1,6 +1,8 @@
-"""The native host path (csrc/fdb_torch.cpp): the mask-bounds kernel against padding.seq_bounds."""
+"""The native host path (csrc/fdb_torch.cpp) and the linear kernels (csrc/fdb_linear.hip): mask bounds against
+padding.seq_bounds, products against fp32 torch, the one-call encoder layer against the module-by-module one."""
 import pytest
 import torch
+import torch.nn.functional as F
 
 from flashdeberta_amd import _lib
 from flashdeberta_amd.padding import key_padding_mask, seq_bounds
@@ -25,3 +27,63 @@ def test_mask_bounds(dtype, B, L):
         start, length = _lib.native.mask_bounds(m)
         ref_start, ref_length, _ = seq_bounds(key_padding_mask(m))
         assert torch.equal(start, ref_start) and torch.equal(length, ref_length), (m.shape, start, ref_start, length, ref_length)
+
+
+def _rel(a, b):
+    return ((a.float() - b).norm() / b.norm()).item()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,code,tol", [(torch.bfloat16, 1, 4e-3), (torch.float16, 2, 6e-4)], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 2, 32), (16, 48, 64), (17, 768, 768), (32, 18, 96), (24, 768, 3072),   # weights streamed, eight and sixteen waves
+    (33, 64, 64), (64, 100, 128), (65, 132, 192), (257, 768, 768),              # tiles: one step, odd counts, ragged edges
+    (40, 18, 96), (70, 30, 64),                                                 # many rows, sizes the tiles do not take
+])
+def test_linear_kernels(M, N, K, dtype, code, tol):
+    g = torch.Generator(device="cuda").manual_seed(M * N + K)
+    x, w = [torch.randn(r, K + 8, device="cuda", generator=g).to(dtype)[:, :K] for r in (M, N)]   # rows with a stride of their own
+    b = torch.randn(N, device="cuda", generator=g).to(dtype)
+    out = torch.full((M + 1, N), 7.0, device="cuda", dtype=dtype)
+    for bias in (b, None):
+        rc = _lib.lib.fdb_linear(x.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), M, N, K, x.stride(0),
+                                 w.stride(0), N, code, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        ref = F.linear(x.float(), w.float(), None if bias is None else bias.float())
+        assert _rel(out[:M], ref) < tol and (out[M] == 7.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,N,K", [(1, 768, 768), (24, 2304, 768), (301, 768, 3072), (4096, 3072, 768)])
+def test_library_products_have_the_bits_of_torch(M, N, K, dtype):
+    x, w, b = [torch.randn(*s, device="cuda").to(dtype) for s in ((M, K), (N, K), (N,))]
+    assert torch.equal(_lib.native.linear(x, w, b, False), F.linear(x, w, b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L", [(1, 5), (2, 40), (3, 300), (6, 384)])   # each way of computing the projections
+def test_encoder_layer_matches_the_module_by_module_forward(B, L):
+    from transformers.models.deberta_v2.modeling_deberta_v2 import DebertaV2Layer
+
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
+
+    torch.manual_seed(L)
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=256, num_hidden_layers=1, num_attention_heads=4, intermediate_size=1024,
+                          relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True,
+                          norm_rel_ebd="layer_norm", position_biased_input=False, initializer_range=0.2)
+    model = FlashDebertaV2Model(cfg).eval().cuda().to(torch.bfloat16)
+    layer = model.encoder.layer[0]
+    x = torch.randn(B, L, 256, device="cuda").to(torch.bfloat16)
+    mask = torch.ones(B, L, device="cuda", dtype=torch.long)
+    mask[-1, L // 2:] = 0
+    rel = torch.randn(64, 256, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        got = layer(x, mask, rel_embeddings=rel)[0]
+        ref = DebertaV2Layer.forward(layer, x, mask, rel_embeddings=rel)[0]
+        assert torch.equal(got, ref)
+        calls = []
+        handle = layer.output.dense.register_forward_hook(lambda *a: calls.append(1))   # a hook on any part is honoured
+        layer(x, mask, rel_embeddings=rel)
+        handle.remove()
+        assert calls
