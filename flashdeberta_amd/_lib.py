@@ -45,10 +45,10 @@ class FdbAttnBwdArgs(ctypes.Structure):
 
 
 EXPORTS = (
-    "fdb_version", "fdb_attn_args_size", "fdb_strerror", "fdb_attn_check", "fdb_attn_fwd", "fdb_attn_fwd_part", "fdb_attn_fwd_noalloc", "fdb_attn_bwd", "fdb_attn_bwd_chain", "fdb_attn_bwd_args_size", "fdb_attn_workspace_bytes",
+    "fdb_version", "fdb_attn_args_size", "fdb_strerror", "fdb_attn_check", "fdb_attn_fwd", "fdb_attn_fwd_part", "fdb_attn_fwd_noalloc", "fdb_attn_bwd", "fdb_attn_bwd_tables", "fdb_attn_bwd_tables_workspace_bytes", "fdb_attn_bwd_chain", "fdb_attn_bwd_args_size", "fdb_attn_workspace_bytes",
     "fdb_worklist_ints",
     "fdb_worklist_max_tiles", "fdb_tile_rows", "fdb_build_worklist", "fdb_delta_lut_radius", "fdb_delta_lut", "fdb_delta_lut_window",
-    "fdb_linear", "fdb_mask_bounds", "fdb_quant_e4m3_per_head", "fdb_quant_e4m3_per_head_pair", "fdb_dequant_e4m3_per_head",
+    "fdb_linear", "fdb_column_sums", "fdb_column_sums_workspace_bytes", "fdb_mask_bounds", "fdb_quant_e4m3_per_head", "fdb_quant_e4m3_per_head_pair", "fdb_dequant_e4m3_per_head",
 )
 
 
@@ -85,6 +85,10 @@ def _load():
     lib.fdb_attn_bwd.argtypes = [ctypes.POINTER(FdbAttnBwdArgs), vp]
     lib.fdb_attn_bwd_chain.restype = ctypes.c_int
     lib.fdb_attn_bwd_chain.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, i32, i64, i64, i64, i64, i64, i32, i32, i32, i32, vp]
+    lib.fdb_attn_bwd_tables.restype = ctypes.c_int  # both: the native host path passes its own argument block
+    lib.fdb_attn_bwd_tables.argtypes = [vp, vp]
+    lib.fdb_attn_bwd_tables_workspace_bytes.restype = i64
+    lib.fdb_attn_bwd_tables_workspace_bytes.argtypes = [vp]
     lib.fdb_attn_workspace_bytes.restype = i64
     lib.fdb_attn_workspace_bytes.argtypes = [ctypes.POINTER(FdbAttnArgs)]
     lib.fdb_worklist_ints.restype = i64
@@ -102,6 +106,10 @@ def _load():
     lib.fdb_delta_lut.argtypes = [i32, i32, i32, vp]
     lib.fdb_linear.restype = ctypes.c_int
     lib.fdb_linear.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i32, vp]
+    lib.fdb_column_sums_workspace_bytes.restype = i64
+    lib.fdb_column_sums_workspace_bytes.argtypes = [i64, i64]
+    lib.fdb_column_sums.restype = ctypes.c_int
+    lib.fdb_column_sums.argtypes = [vp, i64, i64, vp, i64, i64, vp, vp, i32, vp]
     lib.fdb_mask_bounds.restype = ctypes.c_int
     lib.fdb_mask_bounds.argtypes = [vp, i32, i32, i64, i64, i32, i32, vp, vp, vp]
     lib.fdb_quant_e4m3_per_head.restype = ctypes.c_int

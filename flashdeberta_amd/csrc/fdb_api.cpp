@@ -553,11 +553,148 @@ int fdb_attn_bwd(const fdb_attn_bwd_args* a, void* stream) {
   return fdb_launch_bwd(p, a->dtype, a->head_dim, stream);
 }
 
+}  // extern "C"
+
+namespace {
+
+// Sizes of the table backward that follow from the arguments, and where the parts of its workspace lie.
+int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int64_t* bytes) {
+  if (!a) return FDB_ERR_NULL;
+  if (!a->q || !a->k || !a->v || !a->dout || !a->out || !a->pos_key || !a->pos_query || !a->dq || !a->dk || !a->dv || !a->d_pos_key ||
+      !a->d_pos_query || !a->lse)
+    return FDB_ERR_NULL;
+  if (a->dtype != FDB_BF16 && a->dtype != FDB_F16) return FDB_ERR_DTYPE;
+  if (a->head_dim != 64) return FDB_ERR_HEAD_DIM;
+  if (a->batch < 1 || a->heads < 1 || a->heads > 65535 || a->batch > 65535 || a->seqlen < 1) return FDB_ERR_SHAPE;
+  if (a->att_span < 1 || a->lut_radius < 1 || a->lut_radius > (1 << 20) || !a->delta_lut) return FDB_ERR_SPAN;
+  const void* ptrs[] = {a->q, a->k, a->v, a->dout, a->out, a->pos_key, a->pos_query, a->dq, a->dk, a->dv};
+  for (const void* ptr : ptrs)
+    if (!aligned16(ptr)) return FDB_ERR_ALIGN;
+  const int64_t strides[] = {a->q_stride_b, a->q_stride_t, a->q_stride_h, a->k_stride_b, a->k_stride_t, a->k_stride_h, a->v_stride_b,
+                             a->v_stride_t, a->v_stride_h, a->do_stride_b, a->do_stride_t, a->do_stride_h, a->out_stride_b, a->out_stride_t,
+                             a->out_stride_h, a->dq_stride_b, a->dq_stride_t, a->dq_stride_h, a->dk_stride_b, a->dk_stride_t, a->dk_stride_h,
+                             a->dv_stride_b, a->dv_stride_t, a->dv_stride_h, a->pk_stride_h, a->pk_stride_r, a->pq_stride_h, a->pq_stride_r};
+  for (int64_t s : strides)
+    if ((s * 2) % 16 != 0) return FDB_ERR_ALIGN;
+  // the loop side's rows are walked with 32-bit row strides in bytes, the tables with 24-bit ones and 32-bit offsets
+  const int64_t rows[] = {a->q_stride_t, a->k_stride_t, a->v_stride_t, a->do_stride_t};
+  for (int64_t s : rows)
+    if (s < 0 || s * 2 * 32 > INT32_MAX) return FDB_ERR_SHAPE;
+  const int64_t table_rows = 2 * (int64_t)a->att_span, tr[] = {a->pk_stride_r, a->pq_stride_r};
+  for (int64_t s : tr)
+    if (s < 0 || s * 2 >= (1 << 24) || table_rows * s * 2 > INT32_MAX) return FDB_ERR_SHAPE;
+  const int64_t tiles = ((int64_t)a->seqlen + FDB_BM - 1) / FDB_BM, pairs = (int64_t)a->batch * a->heads;
+  if (tiles * pairs > INT32_MAX) return FDB_ERR_SHAPE;
+  memset(p, 0, sizeof(*p));
+  p->B = a->batch; p->H = a->heads; p->L = a->seqlen; p->S = a->att_span; p->R = a->lut_radius; p->causal = a->causal ? 1 : 0;
+  p->pairs_per_xcd = (pairs >= 8 && tiles * pairs > 4 * (int64_t)cu_count()) ? 1 : 0;   // as in fdb_attn_bwd
+  p->stat_len = (a->seqlen + 31) / 32 * 32 + 32;
+  p->g_rows = (int32_t)(4 * tiles);
+  // Blocks of 32 relative positions a wave's row block meets: those of its tile's near steps and one more (see Zones)
+  const int32_t R = a->lut_radius, n_blk = (a->seqlen + 31) / 32;
+  const int32_t most = (FDB_BM - 1 + 2 * R + 2 * 31) / 32 + 1;
+  p->g_slots = (most < n_blk ? most : n_blk) + 1;
+  int32_t rho_max = 3 + (R + 31) / 32, rho_min = -((R + FDB_BM - 1 + 31) / 32);
+  if (rho_max > n_blk - 1) rho_max = n_blk - 1;
+  if (rho_min < -n_blk) rho_min = -n_blk;
+  p->rho_min = rho_min;
+  p->tg_groups = (rho_max - rho_min + 1 + 3) / 4;
+  p->has_far = a->seqlen > R ? 1 : 0;   // some element has |i - j| >= R
+  // Shares of the tokens for the tables' gradients: the launch has H * groups workgroups per share, two fit a CU; a share is a
+  // whole number of chunks of a batch row, at least eight row blocks each, the same number for every share.
+  const int64_t per = (int64_t)a->heads * p->tg_groups;
+  int64_t parts = 2 * (int64_t)cu_count() / per;
+  if (parts > 16) parts = 16;
+  if (parts < 1) parts = 1;
+  auto chunks_for = [&](int64_t n) {   // chunks per batch row that deal batch * chunks evenly to n shares
+    int64_t x = a->batch, y = n;
+    while (y) {
+      const int64_t t = x % y;
+      x = y;
+      y = t;
+    }
+    return n / x;
+  };
+  while (parts > 1 && (int64_t)n_blk < 8 * chunks_for(parts)) --parts;
+  const int64_t chunks = chunks_for(parts);
+  p->tg_len = (int32_t)((n_blk + chunks - 1) / chunks);
+  p->tg_chunks = (int32_t)chunks;
+  p->tg_parts = (int32_t)parts;
+  char* w = (char*)a->workspace;
+  int64_t off = 0;
+  auto take = [&](int64_t n) {
+    char* at = w ? w + off : nullptr;
+    off += align256(n);
+    return at;
+  };
+  p->neg_lse = (float*)take(pairs * p->stat_len * 4);
+  p->neg_delta = (float*)take(pairs * p->stat_len * 4);
+  p->far_q = take(pairs * 2 * p->stat_len * 2);
+  p->far_k = take(pairs * 2 * p->stat_len * 2);
+  p->g_blocks = take(pairs * p->g_rows * p->g_slots * 2048);
+  p->zero_block = take(2048);
+  p->e_parts = (float*)take(parts * per * 4 * 2 * 32 * 64 * 4);
+  p->far_parts = (float*)take(parts * a->heads * 256 * 4);
+  *bytes = off;
+  return FDB_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t fdb_attn_bwd_tables_workspace_bytes(const fdb_attn_bwd_tables_args* a) {
+  FdbBwdRingParams p;
+  int64_t bytes = 0;
+  const int rc = bwd_tables_plan(a, &p, &bytes);
+  return rc == FDB_OK ? bytes : rc;
+}
+
+int fdb_attn_bwd_tables(const fdb_attn_bwd_tables_args* a, void* stream) {
+  FdbBwdRingParams p;
+  int64_t bytes = 0;
+  const int rc = bwd_tables_plan(a, &p, &bytes);
+  if (rc != FDB_OK) return rc;
+  if (!a->workspace) return FDB_ERR_NULL;
+  if (reinterpret_cast<uintptr_t>(a->workspace) & 255u) return FDB_ERR_ALIGN;
+  p.q = (const char*)a->q; p.k = (const char*)a->k; p.v = (const char*)a->v; p.dout = (const char*)a->dout; p.out = (const char*)a->out;
+  p.pk = (const char*)a->pos_key; p.pq = (const char*)a->pos_query;
+  p.dq = (char*)a->dq; p.dk = (char*)a->dk; p.dv = (char*)a->dv; p.dpk = (char*)a->d_pos_key; p.dpq = (char*)a->d_pos_query;
+  p.lse = a->lse; p.seq_start = a->seq_start; p.seq_len = a->seq_len; p.lut = a->delta_lut;
+  p.q_sb = a->q_stride_b; p.q_st = a->q_stride_t; p.q_sh = a->q_stride_h;
+  p.k_sb = a->k_stride_b; p.k_st = a->k_stride_t; p.k_sh = a->k_stride_h;
+  p.v_sb = a->v_stride_b; p.v_st = a->v_stride_t; p.v_sh = a->v_stride_h;
+  p.g_sb = a->do_stride_b; p.g_st = a->do_stride_t; p.g_sh = a->do_stride_h;
+  p.o_sb = a->out_stride_b; p.o_st = a->out_stride_t; p.o_sh = a->out_stride_h;
+  p.dq_sb = a->dq_stride_b; p.dq_st = a->dq_stride_t; p.dq_sh = a->dq_stride_h;
+  p.dk_sb = a->dk_stride_b; p.dk_st = a->dk_stride_t; p.dk_sh = a->dk_stride_h;
+  p.dv_sb = a->dv_stride_b; p.dv_st = a->dv_stride_t; p.dv_sh = a->dv_stride_h;
+  p.pk_sh = a->pk_stride_h; p.pk_sr = a->pk_stride_r; p.pq_sh = a->pq_stride_h; p.pq_sr = a->pq_stride_r;
+  p.dp_sh = a->dp_stride_h; p.dp_sr = a->dp_stride_r;
+  p.sm_scale = a->sm_scale;
+  p.scale_log2 = a->sm_scale * 1.4426950408889634f;
+  return fdb_launch_bwd_ring(p, a->dtype, stream);
+}
+
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens, int32_t* worklist,
                        void* stream) {
   if (!cu_seqlens || !worklist) return FDB_ERR_NULL;
   if (batch < 1 || total_tokens < 0) return FDB_ERR_SHAPE;
   return fdb_launch_worklist(cu_seqlens, batch, worklist, fdb_worklist_max_tiles(total_tokens, batch), stream);
+}
+
+int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols) {
+  if (x_rows < 1 || x_cols < 1) return 0;
+  return (fdb_column_sum_parts(x_rows) + 1) * x_cols * 4;
+}
+
+int fdb_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, void* workspace,
+                    int32_t dtype, void* stream) {
+  if (!x || !out || !workspace) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  if (x_rows < 1 || x_cols < 8 || x_cols % 8 || (y && (y_rows < 1 || y_cols < 8 || y_cols % 8 || y_cols > x_cols))) return FDB_ERR_SHAPE;
+  if (!aligned16(x) || !aligned16(y) || !aligned16(workspace)) return FDB_ERR_ALIGN;
+  return fdb_launch_column_sums(x, x_rows, x_cols, y, y_rows, y_cols, out, (float*)workspace, dtype, stream);
 }
 
 int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64_t stride_b, int64_t stride_l, int32_t batch,

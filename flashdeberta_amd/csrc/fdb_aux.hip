@@ -9,6 +9,8 @@
 #include "fdb_kernels.h"
 #include "../../include/fdb.h"
 
+using namespace fdb;
+
 namespace {
 
 constexpr int kWlThreads = 256;
@@ -73,6 +75,61 @@ __global__ __launch_bounds__(kWlThreads) void fdb_worklist_kernel(const int32_t*
         wl[3 + 2 * pos] = m0;
       }
   }
+}
+
+// Column sums in two launches without atomics: every workgroup sums a share of the rows for 512 columns (eight per lane, a wave a
+// row at a time, the four waves' sums added in LDS) and leaves one row of fp32 sums; the second launch adds those.  Bound by one
+// read of x: 19 MB at [4096 x 2304].
+constexpr int kColShare = 64;   // rows per workgroup: a share of 64 rows keeps the launch wide, 64 partial rows at 4096
+
+template <class QT>
+__global__ __launch_bounds__(256) void fdb_column_sums_kernel(const char* __restrict__ x, int64_t x_rows, int64_t x_cols, const char* __restrict__ y,
+                                                              int64_t y_rows, int64_t y_cols, float* __restrict__ ws, int x_parts) {
+  __shared__ float part[4][512];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int share = blockIdx.y;   // the last one takes all of y
+  const bool second = share == x_parts;
+  const char* src = second ? y : x;
+  const int64_t rows = second ? y_rows : x_rows, cols = second ? y_cols : x_cols, col = (int64_t)blockIdx.x * 512 + 8 * lane;
+  const int64_t r0 = second ? 0 : (int64_t)share * kColShare, r1 = second ? rows : min(rows, r0 + kColShare);
+  f32x8 acc = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (col < cols) {
+#pragma unroll 8
+    for (int64_t r = r0 + wave; r < r1; r += 4) acc += QT::to_f32(QT::load(src + (r * cols + col) * 2));
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) part[wave][8 * lane + e] = acc[e];
+  __syncthreads();
+  for (int c = threadIdx.x; c < 512; c += 256)
+    if ((int64_t)blockIdx.x * 512 + c < x_cols)
+      ws[(int64_t)share * x_cols + (int64_t)blockIdx.x * 512 + c] = part[0][c] + part[1][c] + part[2][c] + part[3][c];
+}
+
+template <class QT>
+__global__ __launch_bounds__(256) void fdb_column_sums_end_kernel(const float* __restrict__ ws, int64_t cols, int parts, typename QT::scratch_t* __restrict__ out) {
+  // 64 columns per workgroup, the parts dealt to its four waves
+  __shared__ float part[4][64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t col = (int64_t)blockIdx.x * 64 + lane;
+  float sum = 0.f;
+  if (col < cols) {
+#pragma unroll 8
+    for (int s = wave; s < parts; s += 4) sum += ws[(int64_t)s * cols + col];
+  }
+  part[wave][lane] = sum;
+  __syncthreads();
+  if (wave == 0 && col < cols) out[col] = (typename QT::scratch_t)(part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]);
+}
+
+template <class QT>
+int launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
+                       hipStream_t stream) {
+  const int parts = fdb_column_sum_parts(x_rows);
+  hipLaunchKernelGGL(fdb_column_sums_kernel<QT>, dim3((unsigned)((x_cols + 511) / 512), (unsigned)(parts + (y ? 1 : 0))), dim3(256), 0, stream,
+                     (const char*)x, x_rows, x_cols, (const char*)y, y_rows, y_cols, ws, parts);
+  hipLaunchKernelGGL(fdb_column_sums_end_kernel<QT>, dim3((unsigned)((x_cols + 63) / 64)), dim3(256), 0, stream, ws, x_cols, parts + (y ? 1 : 0),
+                     (typename QT::scratch_t*)out);
+  return (int)hipGetLastError();
 }
 
 // Bounds of a padded batch's real tokens, one workgroup per row: first and last non-zero mask element and their count.
@@ -240,6 +297,15 @@ int fdb_launch_dequant(const void* y, int64_t y_st, int64_t y_sh, const float* s
   }
 #undef FDB_DQ
   return (int)hipGetLastError();
+}
+
+int fdb_column_sum_parts(int64_t rows) { return (int)((rows + kColShare - 1) / kColShare); }
+
+int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
+                           int dtype, void* stream) {
+  if (dtype == FDB_BF16) return launch_column_sums<fdb::Bf16Tr>(x, x_rows, x_cols, y, y_rows, y_cols, out, ws, (hipStream_t)stream);
+  if (dtype == FDB_F16) return launch_column_sums<fdb::F16Tr>(x, x_rows, x_cols, y, y_rows, y_cols, out, ws, (hipStream_t)stream);
+  return FDB_ERR_DTYPE;
 }
 
 int fdb_launch_mask_bounds(const void* mask, int elem_size, bool is_float, int64_t stride_b, int64_t stride_l, int32_t batch, int32_t length,

@@ -89,6 +89,54 @@ struct FdbBwdParams {
 };
 int fdb_launch_bwd(const FdbBwdParams& p, int dtype, int head_dim, void* stream);
 
+// Backward with the tables in the kernel (fdb_bwd_ring.hip): fixed layout, head_dim 64, 16-bit types, both position terms.
+struct FdbBwdRingParams {
+  const char* q;
+  const char* k;
+  const char* v;
+  const char* dout;
+  const char* out;
+  const char* pk;       // K_r, Q_r
+  const char* pq;
+  char* dq;
+  char* dk;
+  char* dv;
+  char* dpk;            // gradients of the tables, strides dp_sh, dp_sr; rows [0, 2S) are written
+  char* dpq;
+  const float* lse;     // [B*L, H]
+  const int32_t* seq_start;
+  const int32_t* seq_len;
+  const int16_t* lut;
+  // scratch: row statistics [B][H][stat_len], far sums [B][H][2][stat_len] (element type of q), G blocks
+  // [B][H][g_rows][g_slots][32 x 32] (element type of q), partial table gradients [tg_parts][H][4 tg_groups][2][32][64] and
+  // [tg_parts][H][2 tables][2 sides][64]
+  float* neg_lse;
+  float* neg_delta;
+  char* far_q;
+  char* far_k;
+  char* g_blocks;
+  char* zero_block;     // 2 KB of zeros, written by the dQ launch
+  float* e_parts;
+  float* far_parts;
+  int64_t q_sb, q_st, q_sh;
+  int64_t k_sb, k_st, k_sh;
+  int64_t v_sb, v_st, v_sh;
+  int64_t g_sb, g_st, g_sh;     // dout
+  int64_t o_sb, o_st, o_sh;     // out
+  int64_t dq_sb, dq_st, dq_sh;
+  int64_t dk_sb, dk_st, dk_sh;
+  int64_t dv_sb, dv_st, dv_sh;
+  int64_t pk_sh, pk_sr, pq_sh, pq_sr, dp_sh, dp_sr;
+  int32_t B, H, L, S, R, causal;
+  int32_t pairs_per_xcd;
+  int32_t stat_len, g_rows, g_slots;
+  int32_t rho_min, tg_groups, tg_parts, tg_chunks, tg_len;  // blocks of 32 relative positions in groups of four; shares of the tokens; chunks of
+                                                            // tg_len row blocks per batch row
+  int32_t has_far;
+  float scale_log2, sm_scale;
+};
+int fdb_launch_bwd_ring(const FdbBwdRingParams& p, int dtype, void* stream);
+
 // The chain through the position tables (fdb_chain.hip): contiguous tensors, head_dim 64, 2S = 512.
 struct FdbChainParams {
   const char* g;       // [matrices][rows][2S] score gradients
@@ -168,6 +216,9 @@ int fdb_launch_merge(const FdbKParams& p, int dtype, void* stream);
 int fdb_launch_merge_parts(const FdbKParams& p, int dtype, int head_dim, void* stream);
 int fdb_launch_linear(const void* x, const void* w, const void* bias, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldw,
                       int64_t ldo, int dtype, void* stream);  // fdb_linear.hip
+int fdb_column_sum_parts(int64_t rows);
+int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
+                           int dtype, void* stream);
 int fdb_launch_mask_bounds(const void* mask, int elem_size, bool is_float, int64_t stride_b, int64_t stride_l, int32_t batch, int32_t length,
                            int32_t* start, int32_t* len, void* stream);
 int fdb_launch_worklist(const int32_t* cu, int32_t batch, int32_t* wl, int32_t max_tiles, void* stream);

@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hipblaslt/hipblaslt.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
@@ -468,6 +469,160 @@ PyObject* py_attention_fwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// ---- backward with the tables in the kernel -----------------------------------------------------------------------------
+// A tensor of t's sizes whose memory runs like t's where t is dense (so that the gradient of a transposed view is contiguous where the
+// view's base is), else contiguous.
+Tensor empty_as(const Tensor& t) {
+  const bool ok = t.is_non_overlapping_and_dense() && t.stride(-1) == 1;
+  return ok ? at::empty_strided(t.sizes(), t.strides(), t.options()) : at::empty(t.sizes(), t.options());
+}
+
+bool backward_in_tables(const Tensor& q, const OptTensor& pk, const OptTensor& pq) {
+  return (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) && q.dim() == 4 && q.size(3) == 64 && pk && pq && q.is_cuda();
+}
+
+struct Strided {  // [B, L, H, 64] somewhere in memory
+  const void* p;
+  int64_t b, t, h;
+};
+Strided strided(const Tensor& x) { return {x.data_ptr(), x.stride(0), x.stride(1), x.stride(2)}; }
+
+struct BwdSettings {
+  double sm_scale;
+  int64_t buckets, max_relative;
+  bool causal;
+  OptTensor seq_start, seq_len;
+};
+
+struct Table {  // [H, rows, 64] somewhere in memory
+  const void* p;
+  int64_t h, r;
+};
+Table table_of(const Tensor& x) { return {x.data_ptr(), x.stride(0), x.stride(1)}; }
+
+// dq, dk, dv and the tables' gradients (one set of strides for both) into the given memory
+void backward(const Tensor& on, int64_t B, int64_t L, int64_t H, Strided q, Strided k, Strided v, Strided out, Strided dout, const Tensor& lse,
+              Table pk, Table pq, Strided dq, Strided dk, Strided dv, Table dpk, Table dpq, const BwdSettings& o) {
+  fdb_attn_bwd_tables_args a = {};
+  const auto set = [](const Strided& s, int64_t& b, int64_t& t, int64_t& h) {
+    b = s.b, t = s.t, h = s.h;
+    return s.p;
+  };
+  a.q = set(q, a.q_stride_b, a.q_stride_t, a.q_stride_h);
+  a.k = set(k, a.k_stride_b, a.k_stride_t, a.k_stride_h);
+  a.v = set(v, a.v_stride_b, a.v_stride_t, a.v_stride_h);
+  a.out = set(out, a.out_stride_b, a.out_stride_t, a.out_stride_h);
+  a.dout = set(dout, a.do_stride_b, a.do_stride_t, a.do_stride_h);
+  a.dq = const_cast<void*>(set(dq, a.dq_stride_b, a.dq_stride_t, a.dq_stride_h));
+  a.dk = const_cast<void*>(set(dk, a.dk_stride_b, a.dk_stride_t, a.dk_stride_h));
+  a.dv = const_cast<void*>(set(dv, a.dv_stride_b, a.dv_stride_t, a.dv_stride_h));
+  a.pos_key = pk.p, a.pk_stride_h = pk.h, a.pk_stride_r = pk.r;
+  a.pos_query = pq.p, a.pq_stride_h = pq.h, a.pq_stride_r = pq.r;
+  a.d_pos_key = const_cast<void*>(dpk.p), a.d_pos_query = const_cast<void*>(dpq.p);
+  a.dp_stride_h = dpk.h, a.dp_stride_r = dpk.r;
+  a.lse = (const float*)lse.data_ptr();
+  std::vector<Tensor> keep;
+  const char* what = "an int32 GPU tensor with one entry per batch row";
+  if (o.seq_start) a.seq_start = (const int32_t*)vector_arg(*o.seq_start, at::kInt, B, "seq_start", what, keep);
+  if (o.seq_len) a.seq_len = (const int32_t*)vector_arg(*o.seq_len, at::kInt, B, "seq_len", what, keep);
+  const Lut& lut = lut_for(o.buckets, o.max_relative, on);
+  a.delta_lut = (const int16_t*)lut.table.data_ptr();
+  a.lut_radius = lut.radius;
+  a.att_span = (int32_t)att_span(o.buckets, o.max_relative);
+  a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = 64, a.seqlen = (int32_t)L;
+  a.dtype = fdb_dtype_of(on.scalar_type());
+  a.causal = o.causal ? 1 : 0;
+  a.sm_scale = (float)o.sm_scale;
+  const int64_t bytes = fdb_attn_bwd_tables_workspace_bytes(&a);
+  if (bytes < 0) check((int)bytes, "fdb_attn_bwd_tables");
+  const Tensor ws = at::empty({bytes}, on.options().dtype(at::kByte));
+  a.workspace = ws.data_ptr();
+  check(fdb_attn_bwd_tables(&a, stream_of(on)), "fdb_attn_bwd_tables");
+}
+
+// dq, dk, dv, d pos_key, d pos_query of the operator
+std::array<Tensor, 5> backward_of(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& out_in, const Tensor& lse, const Tensor& dout_in,
+                                  const Tensor& pk_in, const Tensor& pq_in, const BwdSettings& o) {
+  const Tensor q = unit_last(q_in), k = unit_last(k_in), v = unit_last(v_in), out = unit_last(out_in), dout = unit_last(dout_in);
+  const int64_t B = q.size(0), L = q.size(1), H = q.size(2), D = q.size(3), span = att_span(o.buckets, o.max_relative);
+  const c10::hip::HIPGuard guard(q.get_device());
+  const Tensor pk = pos_arg(pk_in, H, D, span, "pos_key"), pq = pos_arg(pq_in, H, D, span, "pos_query");
+  const Tensor dq = empty_as(q_in), dk = empty_as(k_in), dv = empty_as(v_in);
+  const int64_t rows = std::max(pk.size(1), pq.size(1));   // one layout for both; rows past 2S take no part
+  const Tensor dpos = rows > 2 * span ? at::zeros({2, H, rows, D}, pk.options()) : at::empty({2, H, rows, D}, pk.options());
+  Tensor dpk = dpos.select(0, 0), dpq = dpos.select(0, 1);
+  backward(q, B, L, H, strided(q), strided(k), strided(v), strided(out), strided(dout), lse, table_of(pk), table_of(pq), strided(dq), strided(dk),
+           strided(dv), table_of(dpk), table_of(dpq), o);
+  if (pk.size(1) != rows) dpk = dpk.narrow(1, 0, pk.size(1));
+  if (pq.size(1) != rows) dpq = dpq.narrow(1, 0, pq.size(1));
+  return {dq, dk, dv, dpk.reshape(pk_in.sizes()), dpq.reshape(pq_in.sizes())};
+}
+
+// The fused forward and the backward above as one autograd node.
+struct AttentionNode : public torch::autograd::Function<AttentionNode> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& pk, const Tensor& pq,
+                        const Fwd* o) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    Fwd with = *o;
+    with.pos_key = pk, with.pos_query = pq;
+    with.return_lse = true;
+    auto r = ::forward(q, k, v, with);
+    ctx->save_for_backward({q, k, v, r.first, r.second, pk, pq, o->seq_start.value_or(Tensor()), o->seq_len.value_or(Tensor())});
+    const int terms = 3;
+    ctx->saved_data["sm_scale"] = std::isnan(o->sm_scale) ? 1.0 / std::sqrt((double)(q.size(3) * terms)) : o->sm_scale;
+    ctx->saved_data["buckets"] = o->buckets;
+    ctx->saved_data["max_relative"] = o->max_relative;
+    ctx->saved_data["causal"] = o->causal;
+    return r.first;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    const auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; };
+    const BwdSettings o{ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["buckets"].toInt(), ctx->saved_data["max_relative"].toInt(),
+                        ctx->saved_data["causal"].toBool(), opt(s[7]), opt(s[8])};
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto r = backward_of(s[0], s[1], s[2], s[3], s[4], grads[0], s[5], s[6], o);
+    return {r[0], r[1], r[2], r[3], r[4], Tensor()};
+  }
+};
+
+// attention_node(q, k, v, pos_key, pos_query, sm_scale, position_buckets, max_relative_positions, causal, seq_start, seq_len, out, far_splits,
+//                near_splits, workspace) -> out, differentiable; None where backward_in_tables does not serve
+PyObject* py_attention_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 15, "attention_node takes 15 arguments");
+  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v");
+  const OptTensor pk = opt_tensor_arg(x[3], "pos_key"), pq = opt_tensor_arg(x[4], "pos_query");
+  if (!backward_in_tables(q, pk, pq)) Py_RETURN_NONE;
+  Fwd o;
+  if (x[5] != Py_None) o.sm_scale = float_arg(x[5]);
+  o.buckets = int_arg(x[6]);
+  o.max_relative = int_arg(x[7]);
+  o.causal = bool_arg(x[8]);
+  o.seq_start = opt_tensor_arg(x[9], "seq_start");
+  o.seq_len = opt_tensor_arg(x[10], "seq_len");
+  o.out = opt_tensor_arg(x[11], "out");
+  o.far_splits = int_arg(x[12]);
+  o.near_splits = int_arg(x[13]);
+  o.workspace = opt_tensor_arg(x[14], "workspace");
+  return THPVariable_Wrap(AttentionNode::apply(q, k, v, *pk, *pq, (const Fwd*)&o));
+  END_HANDLE_TH_ERRORS
+}
+
+// attention_bwd(q, k, v, out, lse, dout, pos_key, pos_query, sm_scale, position_buckets, max_relative_positions, causal, seq_start, seq_len)
+//   -> (dq, dk, dv, d pos_key, d pos_query)
+PyObject* py_attention_bwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 14, "attention_bwd takes 14 arguments");
+  const BwdSettings o{float_arg(x[8]), int_arg(x[9]), int_arg(x[10]), bool_arg(x[11]), opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
+  auto r = backward_of(tensor_arg(x[0], "q"), tensor_arg(x[1], "k"), tensor_arg(x[2], "v"), tensor_arg(x[3], "out"), tensor_arg(x[4], "lse"),
+                       tensor_arg(x[5], "dout"), tensor_arg(x[6], "pos_key"), tensor_arg(x[7], "pos_query"), o);
+  PyObject* t = PyTuple_New(5);
+  for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(r[i]));
+  return t;
+  END_HANDLE_TH_ERRORS
+}
+
 // The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
 // x: pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start, seq_len
 Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, PyObject* const* x, bool own) {
@@ -499,6 +654,123 @@ Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTens
   a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)(B * L);
   run_forward(a, qkv, type, o);
   return out;
+}
+
+// One layer's attention in training, from the hidden states and the relative embeddings through the three projections (shared
+// by the tables): a node of its own.  What autograd would run as one product per projection and tensor, a reduction per bias and
+// an addition per shared tensor is here
+//   forward   q | k | v = hidden . W^T + b and Q_r | K_r = rel . W[q, k]^T + b[q, k], W the three weights on top of each other;
+//   backward  d hidden = d qkv . W,  d W = d qkv^T . hidden (+ d pos^T . rel onto the rows of q and k),  d rel = d pos . W[q, k],
+//             d b = the column sums of d qkv and d pos.
+struct LayerArgs {
+  int64_t heads = 0;
+  BwdSettings o;
+};
+struct LayerNode : public torch::autograd::Function<LayerNode> {
+  static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& hidden_in, const Tensor& rel_in, const Tensor& qw, const Tensor& qb,
+                        const Tensor& kw, const Tensor& kb, const Tensor& vw, const Tensor& vb, const LayerArgs* args) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor hidden = hidden_in.contiguous(), rel = rel_in.contiguous();
+    const c10::hip::HIPGuard guard(hidden.get_device());
+    const int64_t B = hidden.size(0), L = hidden.size(1), C = hidden.size(2), H = args->heads, D = qw.size(0) / H, W = H * D;
+    const int64_t span = att_span(args->o.buckets, args->o.max_relative), rows = 2 * span, esz = hidden.element_size();
+    const auto type = hidden.scalar_type();
+    const Tensor w = at::cat({qw, kw, vw}), b = at::cat({qb, kb, vb});
+    const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
+    gemm(hidden, type, type, false, true, 1, B * L, 3 * W, C, {hidden.data_ptr(), C}, {w.data_ptr(), C}, {qkv.data_ptr(), 3 * W}, b.data_ptr());
+    gemm(hidden, type, type, false, true, 1, rows, 2 * W, C, {rel.data_ptr(), C}, {w.data_ptr(), C}, {pos.data_ptr(), 2 * W}, b.data_ptr());
+    const Tensor out = at::empty({B, L, W}, hidden.options());
+    fdb_attn_args a = {};
+    const char* p = (const char*)qkv.data_ptr();
+    a.dtype = fdb_dtype_of(type);
+    a.q = p, a.k = p + W * esz, a.v = p + 2 * W * esz, a.out = out.data_ptr();
+    a.q_stride_b = a.k_stride_b = a.v_stride_b = L * 3 * W;
+    a.q_stride_t = a.k_stride_t = a.v_stride_t = 3 * W;
+    a.q_stride_h = a.k_stride_h = a.v_stride_h = a.o_stride_h = D;
+    a.o_stride_b = L * W, a.o_stride_t = W;
+    a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)(B * L);
+    Fwd f;
+    f.sm_scale = args->o.sm_scale, f.buckets = args->o.buckets, f.max_relative = args->o.max_relative;
+    f.seq_start = args->o.seq_start, f.seq_len = args->o.seq_len;
+    f.return_lse = true;
+    const std::array<int64_t, 3> size{H, rows, D}, stride{D, 2 * W, 1};
+    f.pos_query = pos.as_strided(size, stride, 0);
+    f.pos_key = pos.as_strided(size, stride, W);
+    const Tensor lse = run_forward(a, qkv, type, f);
+    ctx->save_for_backward({hidden, rel, w, qkv, pos, out, lse, args->o.seq_start.value_or(Tensor()), args->o.seq_len.value_or(Tensor())});
+    ctx->saved_data["heads"] = H;
+    ctx->saved_data["sm_scale"] = args->o.sm_scale;
+    ctx->saved_data["buckets"] = args->o.buckets;
+    ctx->saved_data["max_relative"] = args->o.max_relative;
+    ctx->saved_data["rel_rows"] = rel_in.size(0);
+    return out;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto s = ctx->get_saved_variables();
+    const Tensor &hidden = s[0], &rel = s[1], &w = s[2], &qkv = s[3], &pos = s[4], &out = s[5], &lse = s[6];
+    at::AutoDispatchBelowADInplaceOrView below;
+    const auto opt = [](const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; };
+    const BwdSettings o{ctx->saved_data["sm_scale"].toDouble(), ctx->saved_data["buckets"].toInt(), ctx->saved_data["max_relative"].toInt(), false, opt(s[7]), opt(s[8])};
+    const c10::hip::HIPGuard guard(hidden.get_device());
+    const int64_t B = hidden.size(0), L = hidden.size(1), C = hidden.size(2), H = ctx->saved_data["heads"].toInt(), W = w.size(0) / 3, D = W / H;
+    const int64_t rows = pos.size(0), n = B * L, esz = hidden.element_size(), rel_rows = ctx->saved_data["rel_rows"].toInt();
+    const auto type = hidden.scalar_type();
+    const Tensor dout = grads[0].contiguous();
+    const Tensor dqkv = at::empty({n, 3 * W}, hidden.options()), dpos = at::empty({rows, 2 * W}, hidden.options());
+    const auto at_col = [&](const Tensor& t, int64_t col) { return (const void*)((const char*)t.data_ptr() + col * W * esz); };
+    const auto part = [&](const Tensor& t, int64_t col) { return Strided{at_col(t, col), L * 3 * W, 3 * W, D}; };
+    const auto whole = [&](const Tensor& t) { return Strided{t.data_ptr(), L * W, W, D}; };
+    const auto table = [&](const Tensor& t, int64_t col) { return Table{at_col(t, col), D, 2 * W}; };
+    ::backward(hidden, B, L, H, part(qkv, 0), part(qkv, 1), part(qkv, 2), whole(out), whole(dout), lse, table(pos, 1), table(pos, 0), part(dqkv, 0),
+               part(dqkv, 1), part(dqkv, 2), table(dpos, 1), table(dpos, 0), o);
+    Tensor dhidden, drel, dw, db;
+    if (ctx->needs_input_grad(0)) {
+      dhidden = at::empty(hidden.sizes(), hidden.options());
+      gemm(hidden, type, type, false, false, 1, n, C, 3 * W, {dqkv.data_ptr(), 3 * W}, {w.data_ptr(), C}, {dhidden.data_ptr(), C});
+    }
+    if (ctx->needs_input_grad(1)) {
+      drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
+      gemm(hidden, type, type, false, false, 1, rows, C, 2 * W, {dpos.data_ptr(), 2 * W}, {w.data_ptr(), C}, {drel.data_ptr(), C});
+    }
+    if (ctx->needs_input_grad(2) || ctx->needs_input_grad(4) || ctx->needs_input_grad(6)) {
+      dw = at::empty({3 * W, C}, hidden.options());
+      gemm(hidden, type, type, true, false, 1, 3 * W, C, n, {dqkv.data_ptr(), 3 * W}, {hidden.data_ptr(), C}, {dw.data_ptr(), C});
+      gemm(hidden, type, type, true, false, 1, 2 * W, C, rows, {dpos.data_ptr(), 2 * W}, {rel.data_ptr(), C}, {dw.data_ptr(), C}, nullptr, true);
+    }
+    if (ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7)) {
+      db = at::empty({3 * W}, hidden.options());
+      const Tensor ws = at::empty({fdb_column_sums_workspace_bytes(n, 3 * W)}, hidden.options().dtype(at::kByte));
+      check(fdb_column_sums(dqkv.data_ptr(), n, 3 * W, dpos.data_ptr(), rows, 2 * W, db.data_ptr(), ws.data_ptr(), fdb_dtype_of(type), stream_of(hidden)),
+            "fdb_column_sums");
+    }
+    const auto rows_of = [&](const Tensor& t, int64_t i) { return t.defined() ? t.narrow(0, i * W, W) : Tensor(); };
+    return {dhidden, drel, rows_of(dw, 0), rows_of(db, 0), rows_of(dw, 1), rows_of(db, 1), rows_of(dw, 2), rows_of(db, 2), Tensor()};
+  }
+};
+
+// layer_node(hidden, rel, q_weight, q_bias, k_weight, k_bias, v_weight, v_bias, heads, sm_scale, position_buckets, max_relative_positions,
+//            seq_start, seq_len) -> context [B, L, H*D], differentiable; None for tensors it is not built for
+PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 14, "layer_node takes 14 arguments");
+  const Tensor& hidden = tensor_arg(x[0], "hidden");
+  LayerArgs a;
+  a.heads = int_arg(x[8]);
+  a.o = BwdSettings{float_arg(x[9]), int_arg(x[10]), int_arg(x[11]), false, opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
+  const auto type = hidden.scalar_type();
+  if (!hidden.is_cuda() || (type != at::kBFloat16 && type != at::kHalf) || hidden.dim() != 3 || hidden.numel() == 0 || a.heads < 1) Py_RETURN_NONE;
+  Tensor t[7];
+  for (int i = 0; i < 7; ++i) {
+    if (x[i + 1] == Py_None) Py_RETURN_NONE;
+    t[i] = tensor_arg(x[i + 1], "parameters");
+    if (t[i].scalar_type() != type || t[i].device() != hidden.device()) Py_RETURN_NONE;
+  }
+  const int64_t C = hidden.size(2), W = t[1].size(0), span = att_span(a.o.buckets, a.o.max_relative);
+  if (t[0].dim() != 2 || t[0].size(0) < 2 * span || t[0].size(1) != C || W != 64 * a.heads || C % 8) Py_RETURN_NONE;
+  for (int i = 1; i < 7; i += 2)
+    if (t[i].dim() != 2 || t[i].size(0) != W || t[i].size(1) != C || t[i + 1].dim() != 1 || t[i + 1].size(0) != W) Py_RETURN_NONE;
+  return THPVariable_Wrap(LayerNode::apply(hidden, t[0], t[1], t[2], t[3], t[4], t[5], t[6], (const LayerArgs*)&a));
+  END_HANDLE_TH_ERRORS
 }
 
 // layer_attention(hidden, weight, bias, pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start,
@@ -709,6 +981,9 @@ PyTypeObject MemoType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 PyMethodDef module_methods[] = {
     {"attention_fwd", (PyCFunction)(void*)py_attention_fwd, METH_FASTCALL, nullptr},
+    {"attention_node", (PyCFunction)(void*)py_attention_node, METH_FASTCALL, nullptr},
+    {"layer_node", (PyCFunction)(void*)py_layer_node, METH_FASTCALL, nullptr},
+    {"attention_bwd", (PyCFunction)(void*)py_attention_bwd, METH_FASTCALL, nullptr},
     {"layer_attention", (PyCFunction)(void*)py_layer_attention, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, nullptr},
     {"encoder_layer", (PyCFunction)(void*)py_encoder_layer, METH_FASTCALL, nullptr},

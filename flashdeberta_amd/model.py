@@ -58,6 +58,10 @@ def _weight_and_bias(module):
     return module.weight, module.bias
 
 
+def _hooked(module):
+    return module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+
+
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     """Same parameters as the eager module (query_proj, key_proj, value_proj[, pos_key_proj,
     pos_query_proj]), so `load_state_dict(eager.state_dict())` works (reference tests/attention.py:60).
@@ -170,6 +174,16 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         pos_key, pos_query = self._pos_layers(rel_embeddings)
         return (*fused, pos_key, pos_query, self.num_attention_heads, *self._score_settings(pos_key, pos_query), *self._bounds(attention_mask))
 
+    def _trains_as_one_node(self):
+        """Whether native.layer_node computes what the module does, step by step: plain projections shared with the tables, both
+        position terms, nothing that has to see the projections' own calls (hooks) or cast their operands (autocast)."""
+        if not (self.relative_attention and self.share_att_key and not self.fp8_qk and "c2p" in self.pos_att_type and "p2c" in self.pos_att_type) \
+                or torch.is_autocast_enabled() or torch.compiler.is_compiling() or nn_module._global_forward_hooks \
+                or nn_module._global_forward_pre_hooks or nn_module._global_backward_hooks:
+            return False
+        projections = [self._modules[n] for n in ("query_proj", "key_proj", "value_proj")]
+        return all(type(m) is torch.nn.Linear for m in projections) and not any(_hooked(m) for m in projections)
+
     def forward(self, hidden_states, attention_mask, output_attentions=False, query_states=None,
                 relative_pos=None, rel_embeddings=None):
         """-> (context [B, L, H*D], None).  `relative_pos` is ignored: the bucketed relative
@@ -184,9 +198,17 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         args = self._native_args(attention_mask, rel_embeddings, hidden_states.requires_grad) if query_states is hidden_states else None
         if args is not None:
             return native.layer_attention(hidden_states, *args, self._own_products), None
+        seq_start, seq_len = self._bounds(attention_mask)
+        if query_states is hidden_states and rel_embeddings is not None and self._trains_as_one_node():
+            sm_scale, buckets, max_distance = self._score_settings(rel_embeddings, rel_embeddings)
+            modules = self._modules
+            rel = rel_embeddings if not self.training else self.pos_dropout(rel_embeddings)
+            ctx = native.layer_node(hidden_states, rel, *[p for n in ("query_proj", "key_proj", "value_proj") for p in _weight_and_bias(modules[n])],
+                                    H, sm_scale, buckets, max_distance, seq_start, seq_len)
+            if ctx is not None:
+                return ctx, None
         pos_key, pos_query = self._pos_layers(rel_embeddings)
         sm_scale, buckets, max_distance = self._score_settings(pos_key, pos_query)
-        seq_start, seq_len = self._bounds(attention_mask)
 
         q, k, v = self._qkv(hidden_states, query_states)
         kw = {}
@@ -224,10 +246,6 @@ DEBERTA_SELF_ATTENTION_CLASSES = {
     "eager": DisentangledSelfAttention,
     "flash_attention_2": FlashDisentangledSelfAttention,
 }
-
-
-def _hooked(module):
-    return module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
 
 
 class FlashDebertaV2Layer(DebertaV2Layer):

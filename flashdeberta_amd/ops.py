@@ -270,6 +270,9 @@ def disentangled_attention_bwd(q, k, v, out, lse, dout, pos_key=None, pos_query=
     pos_query = _pos_arg(pos_query, H, D, span, "pos_query")
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D * (1 + (pos_key is not None) + (pos_query is not None)))
+    if fused_chain is None and delta is None and pos_key is not None and pos_query is not None and D == 64 and q.dtype in (torch.bfloat16, torch.float16):
+        return native.attention_bwd(q, k, v, out, lse.contiguous(), dout, pos_key, pos_query, sm_scale, position_buckets, max_relative_positions,
+                                    causal, seq_start, seq_len)
     q, k, v, dout = [x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v, dout)]
     f32 = torch.float32
     c2p = p2c = d_c2p = d_p2c = None
@@ -403,7 +406,14 @@ def disentangled_attention(q, k, v, pos_key=None, pos_query=None, **kwargs):
     required, the fixed layout in fp32 / bf16 / fp16 is differentiable (dq, dk, dv, d pos_key, d pos_query);
     the packed layout and FP8 operands become a node whose backward raises."""
     if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in (q, k, v, pos_key, pos_query)):
-        differentiable = q.dim() == 4 and q.dtype in _DTYPES and set(kwargs) <= _BWD_KW
+        differentiable = q.dim() == 4 and q.dtype in _DTYPES and kwargs.keys() <= _BWD_KW
+        if differentiable and pos_key is not None and pos_query is not None:
+            get = kwargs.get
+            out = native.attention_node(q, k, v, pos_key, pos_query, get("sm_scale"), get("position_buckets", 0),
+                                        get("max_relative_positions", 0), get("causal", False), get("seq_start"), get("seq_len"),
+                                        get("out"), get("far_splits", 0), get("near_splits", 0), get("workspace"))
+            if out is not None:
+                return out
         return (_DisentangledAttention if differentiable else _ForwardOnly).apply(kwargs, q, k, v, pos_key, pos_query)
     return disentangled_attention_fwd(q, k, v, pos_key, pos_query, **kwargs)
 

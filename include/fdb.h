@@ -247,6 +247,57 @@ size_t fdb_attn_bwd_args_size(void);
 int fdb_attn_bwd(const fdb_attn_bwd_args* a, void* stream);
 
 /*
+ * The backward with the tables in the kernel: dq, dk, dv and the gradients of K_r and Q_r themselves, from q, k, v, out, lse, dout and
+ * the tables, with no position-score tensors on either side of the call (fdb_attn_bwd and fdb_attn_bwd_chain with the products
+ * around them compute the same).  Fixed layout (padded batches through seq_start / seq_len: rows of padding of dq, dk, dv are
+ * written as zeros; causal), both position terms, FDB_BF16 / FDB_F16, head_dim 64, any table.  Strides in elements, rows of 64
+ * contiguous elements aligned to 16 bytes; rows [0, 2 * att_span) of d_pos_key / d_pos_query are written, both with the strides dp_*.
+ * workspace: fdb_attn_bwd_tables_workspace_bytes(a) bytes, 256-byte aligned (negative: the error fdb_attn_bwd_tables would return).
+ */
+typedef struct fdb_attn_bwd_tables_args {
+  const void* q;
+  const void* k;
+  const void* v;
+  const void* dout;
+  const void* out;
+  const void* pos_key;
+  const void* pos_query;
+  void* dq;
+  void* dk;
+  void* dv;
+  void* d_pos_key;
+  void* d_pos_query;
+  const float* lse;        /* [B*L, H] as the forward returns it */
+  const int32_t* seq_start;
+  const int32_t* seq_len;
+  const int16_t* delta_lut;
+  void* workspace;
+  int64_t q_stride_b, q_stride_t, q_stride_h;
+  int64_t k_stride_b, k_stride_t, k_stride_h;
+  int64_t v_stride_b, v_stride_t, v_stride_h;
+  int64_t do_stride_b, do_stride_t, do_stride_h;
+  int64_t out_stride_b, out_stride_t, out_stride_h;
+  int64_t dq_stride_b, dq_stride_t, dq_stride_h;
+  int64_t dk_stride_b, dk_stride_t, dk_stride_h;
+  int64_t dv_stride_b, dv_stride_t, dv_stride_h;
+  int64_t pk_stride_h, pk_stride_r;
+  int64_t pq_stride_h, pq_stride_r;
+  int64_t dp_stride_h, dp_stride_r;
+  int32_t batch;
+  int32_t heads;
+  int32_t head_dim;
+  int32_t seqlen;
+  int32_t att_span;
+  int32_t lut_radius;
+  int32_t dtype;
+  int32_t causal;
+  float sm_scale;
+} fdb_attn_bwd_tables_args;
+
+int64_t fdb_attn_bwd_tables_workspace_bytes(const fdb_attn_bwd_tables_args* a);
+int fdb_attn_bwd_tables(const fdb_attn_bwd_tables_args* a, void* stream);
+
+/*
  * The chain of the backward through the position tables, for `matrices` (head, term) pairs at once: with
  * g = d_scores [matrices][rows][2 * att_span] (what fdb_attn_bwd left in d_c2p_bias / d_p2c_bias, head-major),
  * the token rows x (the q rows for a c2p matrix, the k rows for a p2c matrix: row r of matrix m at
@@ -293,6 +344,15 @@ int32_t fdb_worklist_max_tiles(int32_t total_tokens, int32_t batch);
 
 /* Rows of one q-tile (the work-list granularity). */
 int32_t fdb_tile_rows(void);
+
+/*
+ * Column sums (FDB_BF16 / FDB_F16, fp32 sums, one rounding): out[c] = sum of x[:, c] over x_rows contiguous rows of x_cols, plus that of y
+ * for its y_cols <= x_cols columns (y may be NULL): the bias gradients of projections that share weights.  Columns a multiple of
+ * 8, x and y aligned to 16 bytes, workspace as asked for.
+ */
+int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols);
+int fdb_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, void* workspace,
+                    int32_t dtype, void* stream);
 
 /*
  * The bounds of a padded batch from its mask, on the device: token l of row b is real where the element at

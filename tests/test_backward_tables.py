@@ -1,0 +1,114 @@
+"""The backward with the tables in the kernel (fdb_attn_bwd_tables) and the training node of a layer: against the oracle's chain rule
+at the edges of tiles, steps, rings and zones, and against the module-by-module forward under autograd."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from flashdeberta_amd import _lib, ops
+from oracle import disentangled_oracle as O
+
+
+def _np(x):
+    return x.detach().float().cpu().numpy().astype(np.float64)
+
+
+CASES = [
+    # B, L, H, buckets, max_rel, causal, (start, length) per row or None
+    (1, 1, 1, 256, 512, False, None),
+    (2, 32, 2, 256, 512, False, None),
+    (1, 33, 1, 256, 512, True, None),
+    (1, 129, 3, 32, 64, False, None),                      # one row in the last tile, far steps on both sides
+    (2, 160, 2, 32, 64, True, None),
+    (1, 544, 1, 256, 512, False, None),                    # the first length with far steps (radius 512)
+    (1, 1153, 1, 256, 512, False, None),                   # a tile with far steps on both sides, an odd end
+    (1, 900, 2, 256, 512, True, None),
+    (3, 300, 2, 32, 64, False, [(0, 300), (37, 200), (299, 1)]),   # left and right padding, a row of one token
+    (2, 257, 1, 16, 16, False, [(0, 0), (1, 256)]),        # an empty row; a table that saturates within a step
+    (1, 300, 1, 256, 200, False, None),                    # steps of several table rows per position
+    (1, 400, 2, 0, 100, False, None),                      # no buckets
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "B%dL%dH%d_b%d_m%d_c%d%s" % (c[:6] + ("pad" if c[6] else "",)))
+def test_table_backward_matches_oracle(case, dtype):
+    B, L, H, pb, mr, causal, rows = case
+    S, D = ops.att_span(pb, mr), 64
+    g = torch.Generator().manual_seed(L * 7 + H)
+    q, k, v, dout = [torch.randn(B, L, H, D, generator=g).to(dtype) for _ in range(4)]
+    pk, pq = [torch.randn(H, 2 * S, D, generator=g).to(dtype) for _ in range(2)]
+    kw = dict(position_buckets=pb, max_relative_positions=mr, causal=causal)
+    if rows:
+        kw["seq_start"], kw["seq_len"] = [torch.tensor(x, dtype=torch.int32).cuda() for x in zip(*rows)]
+    c = [x.cuda() for x in (q, k, v, pk, pq)]
+    out, lse = ops.disentangled_attention_fwd(*c, return_lse=True, **kw)
+    got = ops.disentangled_attention_bwd(*c[:3], out, lse, dout.cuda(), *c[3:], **kw)
+    again = ops.disentangled_attention_bwd(*c[:3], out, lse, dout.cuda(), *c[3:], **kw)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    ref = [np.zeros((B, L, H, D)) for _ in range(3)] + [np.zeros((H, 2 * S, D)) for _ in range(2)]
+    t = lambda x, b, s: _np(x[b:b + 1, s]).transpose(0, 2, 1, 3)
+    for b, (start, length) in enumerate(rows or [(0, L)] * B):
+        if not length:
+            continue
+        s = slice(start, start + length)
+        r = O.disentangled_attention_backward(*[t(x, b, s) for x in (q, k, v, dout)], _np(pk), _np(pq), pb, mr, causal=causal)
+        for n in range(3):
+            ref[n][b:b + 1, s] = r[n].transpose(0, 2, 1, 3)
+        ref[3] += r[3]
+        ref[4] += r[4]
+    for name, a, r in zip(("dq", "dk", "dv", "dK_r", "dQ_r"), got, ref):
+        err = np.abs(_np(a) - r).max()
+        assert err <= 3e-2 * max(np.abs(r).max(), 1e-2), "%s: err %.3e, largest %.3e" % (name, err, np.abs(r).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols,rows2,cols2", [(1, 8, 0, 0), (63, 512, 5, 8), (64, 520, 64, 512), (65, 2304, 512, 1536), (4096, 768, 0, 0)])
+def test_column_sums(rows, cols, rows2, cols2):
+    x = torch.randn(rows, cols, device="cuda").to(torch.bfloat16)
+    y = torch.randn(rows2, cols2, device="cuda").to(torch.bfloat16) if rows2 else None
+    out = torch.empty(cols, device="cuda", dtype=torch.bfloat16)
+    ws = torch.empty(_lib.lib.fdb_column_sums_workspace_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+    assert _lib.lib.fdb_column_sums(x.data_ptr(), rows, cols, None if y is None else y.data_ptr(), rows2, cols2, out.data_ptr(), ws.data_ptr(), 1,
+                                    torch.cuda.current_stream().cuda_stream) == 0
+    ref = x.float().sum(0)
+    if y is not None:
+        ref[:cols2] += y.float().sum(0)
+    assert ((out.float() - ref).abs() <= 4e-3 * ref.abs() + 1e-4 * rows ** 0.5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,padded", [(1, 7, False), (3, 200, True), (2, 640, False)])
+def test_layer_node_matches_separate_projections(B, L, padded):
+    """The whole layer as one node against the same module with its projections called one by one (a hook on one of them
+    turns the node off): output and every gradient."""
+    from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
+
+    torch.manual_seed(L)
+    cfg = DebertaV2Config(hidden_size=192, num_attention_heads=3, relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32,
+                          max_relative_positions=64, share_att_key=True, hidden_dropout_prob=0.0, attention_probs_dropout_prob=0.0)
+    att = FlashDisentangledSelfAttention(cfg).train().cuda().to(torch.bfloat16)
+    x = torch.randn(B, L, 192, device="cuda").to(torch.bfloat16).requires_grad_()
+    rel = torch.randn(64, 192, device="cuda").to(torch.bfloat16).requires_grad_()
+    mask = torch.ones(B, L, device="cuda", dtype=torch.long)
+    if padded:
+        mask[0, L // 3:] = 0
+    dout = torch.randn(B, L, 192, device="cuda").to(torch.bfloat16)
+    leaves = [x, rel, *att.parameters()]
+
+    def grads():
+        out = att(x, mask, rel_embeddings=rel)[0]
+        return (out.detach(), out.grad_fn.name(), *torch.autograd.grad(out, leaves, dout))
+
+    one = grads()
+    handle = att.value_proj.register_forward_hook(lambda *a: None)
+    separate = grads()
+    handle.remove()
+    assert one[1] != separate[1]
+    for a, b in zip(one[:1] + one[2:], separate[:1] + separate[2:]):
+        assert (a.float() - b.float()).norm() <= 2e-2 * b.float().norm()
+    # only what is asked for
+    att.value_proj.weight.requires_grad_(False)
+    some = torch.autograd.grad(att(x, mask, rel_embeddings=rel)[0], [x, att.query_proj.bias], dout)
+    assert torch.equal(some[0], one[2]) and some[1].shape == (192,)
