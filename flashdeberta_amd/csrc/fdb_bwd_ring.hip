@@ -279,19 +279,32 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
       }
     }
   };
-  // dX^T += Y1^T dS, dV^T += dO^T P: the loop rows are the accumulators' registers
-  auto outputs = [&](const f32x16& pr, const frag (&dsf)[2], int off) __attribute__((always_inline)) {
+  // dX^T += Y1^T dS, dV^T += dO^T P: the loop rows are the accumulators' registers.  The transposed operands are asked for
+  // well ahead of their use.
+  struct Trans {
+    frag y1[2][DBLKS], y2[kDQ ? 1 : 2][DBLKS];
+  };
+  auto request_trans = [&](Trans& t, int off) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int d = 0; d < DBLKS; ++d) {
+        t.y1[c][d] = y_trans(c, d, off);
+        if constexpr (!kDQ) t.y2[c][d] = y_trans(c, d, off + 2 * kTile);
+      }
+  };
+  auto outputs = [&](const f32x16& pr, const frag (&dsf)[2], const Trans& t) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
 #pragma unroll
-      for (int d = 0; d < DBLKS; ++d) acc1[d] = QT::mma(y_trans(c, d, off), dsf[c], acc1[d]);
+      for (int d = 0; d < DBLKS; ++d) acc1[d] = QT::mma(t.y1[c][d], dsf[c], acc1[d]);
       if constexpr (!kDQ) {
         f32x8 p8;
 #pragma unroll
         for (int e = 0; e < 8; ++e) p8[e] = pr[8 * c + e];
         const frag pf = QT::from_f32(p8);
 #pragma unroll
-        for (int d = 0; d < DBLKS; ++d) acc2[d] = QT::mma(y_trans(c, d, off + 2 * kTile), pf, acc2[d]);
+        for (int d = 0; d < DBLKS; ++d) acc2[d] = QT::mma(t.y2[c][d], pf, acc2[d]);
       }
     }
   };
@@ -354,27 +367,36 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
       __syncthreads();
       if (s + 1 < z.hi) tiles_dma(s + 1, buf ^ 1);
       f32x16 sacc, dpacc;
-      if constexpr (kDQ) {
-        sacc = start16;
-        dpacc = del16;
-      } else {
+      frag yf[KS], zf[KS];   // every operand of the eight products is requested before the first of them waits for one
+      if constexpr (!kDQ) {
         sacc = start_stat(0, buf);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sacc[v] += start;
         dpacc = start_stat(1, buf);
       }
 #pragma unroll
       for (int x = 0; x < KS; ++x) {
-        sacc = QT::mma(y_frag(x, off), x1[x], sacc);
-        dpacc = QT::mma(y_frag(x, off + 2 * kTile), x2[x], dpacc);
+        yf[x] = y_frag(x, off);
+        zf[x] = y_frag(x, off + 2 * kTile);
       }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!kDQ) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sacc[v] += start;
+      }
+#pragma unroll
+      for (int x = 0; x < KS; ++x) {
+        sacc = QT::mma(yf[x], x1[x], kDQ && x == 0 ? start16 : sacc);
+        dpacc = QT::mma(zf[x], x2[x], kDQ && x == 0 ? del16 : dpacc);
+      }
+      Trans tr;
+      request_trans(tr, off);
+      __builtin_amdgcn_sched_barrier(0);
       const bool edge = xw0 + 31 >= Lb || y0 + kStep > Lb || (p.causal && (kDQ ? y0 + kStep - 1 > xw0 : xw0 + 31 > y0));
       gradients(sacc, dpacc, y0, edge);
       frag dsf[2];
       pack(dpacc, dsf);
       sum += (((dpacc[0] + dpacc[1]) + (dpacc[2] + dpacc[3])) + ((dpacc[4] + dpacc[5]) + (dpacc[6] + dpacc[7]))) +
              (((dpacc[8] + dpacc[9]) + (dpacc[10] + dpacc[11])) + ((dpacc[12] + dpacc[13]) + (dpacc[14] + dpacc[15])));
-      outputs(sacc, dsf, off);
+      outputs(sacc, dsf, tr);
     }
     far_sum[side] = sum;
   };
@@ -493,7 +515,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
       constexpr int PAR = decltype(par_tag)::value;
       constexpr int OFF = PAR * kTile;
       const int s = z.s0 + k, y0 = s * kStep;
-      wait_vmcnt<0>();
+      wait_vmcnt<kDQ ? 2 : 0>();   // the loads of the step before; the two stores of G after them may still be on their way
       asm volatile("" : "+v"(dnext));
       __syncthreads();
       tiles_dma(s + 1, PAR ^ 1);
@@ -557,6 +579,9 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
 #pragma unroll
       for (int v = 0; v < 16; ++v) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v] + cband[v]);
       const bool edge = xw0 + 31 >= Lb || y0 + kStep > Lb || (p.causal && (kDQ ? y0 + kStep - 1 > xw0 : xw0 + 31 > y0));
+      Trans tr;
+      request_trans(tr, OFF);
+      __builtin_amdgcn_sched_barrier(0);
       gradients(sacc, dpacc, y0, edge);
       // The saturated rows of a table's gradient come from the sums per lane row alone (far steps and these few elements),
       // the rows inside the radius from the blocks of G: where the two roles' far steps begin does not matter then.
@@ -584,7 +609,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
         }
       }
       wave_lds_fence();
-      outputs(sacc, dsf, OFF);
+      outputs(sacc, dsf, tr);
       frag gf[2];
       g_load(PAR ^ 1, gf);
       g_use(gf, xs_new == 0 ? kXBatches - 1 : xs_new - 1, k);
