@@ -134,10 +134,11 @@ int far_parts_wanted(const fdb_attn_args* a) {
 // (five batches of table rows) and a merge kernel follows, so a share keeps at least sixteen 32-key
 // steps, or eight when all shares together fill at most half of the slots.  (Measured, 12 heads: one
 // sequence of 1024: 0.056 -> 0.040 ms; one of 512: 0.025 -> 0.022; four of 512 in shares of eight
-// steps would go from 0.025 to 0.028.)  Two shares also pay when they need a partial second round, as
-// long as the query tiles alone fill at most 70 % of the slots (288 to 352 tiles: 5 to 8 % of the call;
-// 384: between +2 and -4 %).
-int near_parts_wanted(const fdb_attn_args* a) {
+// steps would go from 0.025 to 0.028.)  Two shares of twelve steps pay while they leave a fifth of the
+// slots free (two of 777 40.0 -> 38.3 us, two of 900 45.2 -> 43.0; three of 777, 504 shares, would lose 7 %).
+// `room`: the workspace is sized for two shares with a partial second round as well (288 to 352 query tiles), which
+// the launch does not take: dealt longest first, the tiles are 3 to 8 % faster unshared there.
+int near_parts_wanted(const fdb_attn_args* a, bool room = false) {
   if (!(a->pos_key || a->pos_query) || !a->lse || !steps32_supported(a->dtype, a->head_dim)) return 1;
   if (a->near_splits > 0) return a->near_splits;
   // A packed batch has its lengths on the device: the host goes by the mean length and by the most query tiles the
@@ -147,10 +148,9 @@ int near_parts_wanted(const fdb_attn_args* a) {
   const int steps_all = (typical + 31) / 32, steps_near = (FDB_BM + 2 * a->lut_radius + 3 * (FDB_BN - 1)) / 32;
   const int steps = steps_all < steps_near ? steps_all : steps_near;
   int best = 1;
-  // (packed batches only share when all shares fit in one round: three sequences of 1000 lose 10 % to two shares)
-  for (int n = 2; n <= FDB_MAX_FAR_PARTS && (wgs * n <= slots || (n == 2 && !a->cu_seqlens && wgs * 10 <= slots * 7)); ++n) {
+  for (int n = 2; n <= FDB_MAX_FAR_PARTS && (wgs * n <= slots || (room && n == 2 && !a->cu_seqlens && wgs * 10 <= slots * 7)); ++n) {
     const int per = steps / n;
-    if (per >= 16 || (per >= 8 && wgs * n <= slots / 2)) best = n;
+    if (per >= 16 || (n == 2 && per >= 12 && wgs * n * 5 <= slots * 4) || (per >= 8 && wgs * n <= slots / 2)) best = n;
   }
   return best;
 }
@@ -328,7 +328,7 @@ int64_t fdb_attn_workspace_bytes(const fdb_attn_args* a) {
     const int parts = key_parts_wanted(a);
     return parts > 1 ? parts * far_part_bytes(a) : 0;
   }
-  const int near = near_parts_wanted(a);
+  const int near = near_parts_wanted(a, true);
   return (far_parts_wanted(a) - 1 + (near > 1 ? near : 0)) * far_part_bytes(a);
 }
 
@@ -587,7 +587,6 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   if (tiles * pairs > INT32_MAX) return FDB_ERR_SHAPE;
   memset(p, 0, sizeof(*p));
   p->B = a->batch; p->H = a->heads; p->L = a->seqlen; p->S = a->att_span; p->R = a->lut_radius; p->causal = a->causal ? 1 : 0;
-  p->pairs_per_xcd = (pairs >= 8 && tiles * pairs > 4 * (int64_t)cu_count()) ? 1 : 0;   // as in fdb_attn_bwd
   p->stat_len = (a->seqlen + 31) / 32 * 32 + 32;
   p->g_rows = (int32_t)(4 * tiles);
   // Blocks of 32 relative positions a wave's row block meets: those of its tile's near steps and one more (see Zones)

@@ -107,23 +107,6 @@ __device__ __forceinline__ Zones zones_of(int m0, int Lb, int R, bool causal, bo
   return z;
 }
 
-// Linear workgroup id -> (tile of 128 lane rows, head, batch row): whole (batch row, head) pairs per XCD where the launcher asks
-// for it, see fdb_attn_bwd.
-__device__ __forceinline__ void block_of(const FdbBwdRingParams& p, int n, int& tile, int& h, int& b) {
-  const int tiles = (p.L + FDB_BM - 1) / FDB_BM, whole = (p.B * p.H) & ~7;
-  int pair;
-  if (p.pairs_per_xcd && n < whole * tiles) {
-    const int slot = n >> 3;
-    pair = (n & 7) + 8 * (slot / tiles);
-    tile = slot % tiles;
-  } else {
-    pair = n / tiles;
-    tile = n % tiles;
-  }
-  b = pair / p.H;
-  h = pair % p.H;
-}
-
 template <class QT, int ROLE>
 __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdRingParams p) {
   constexpr bool kDQ = ROLE == 0;
@@ -134,9 +117,12 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  int tile_x, h, b;
-  block_of(p, (int)blockIdx.x, tile_x, h, b);
-  if (kDQ && p.causal) tile_x = (p.L + FDB_BM - 1) / FDB_BM - 1 - tile_x;
+  // near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
+  const int tiles = (p.L + FDB_BM - 1) / FDB_BM;
+  int tile_x, h;
+  block_map((int)blockIdx.x, p.B * tiles, p.H, tiles, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, tile_x, h);
+  const int b = tile_x / tiles;
+  tile_x -= b * tiles;
   const int m0 = tile_x * FDB_BM;
   const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;

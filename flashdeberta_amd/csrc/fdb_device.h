@@ -257,20 +257,24 @@ __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { re
 
 // Linear workgroup id -> (query-tile index within the launch, head).  The hardware deals
 // workgroups to the 8 XCDs round-robin by linear id, and each XCD has its own L2.  In the fixed
-// layout, when the number of (sequence, head) groups is a multiple of 8, groups are dealt to XCDs
-// whole: all query tiles of a group then stream the same K and V through one L2.
-// Within a group the query tiles are dealt in the order `order` asks for, so that the workgroups
+// layout the (sequence, head) groups are dealt to XCDs whole, group g to XCD g % 8: all query tiles of a group then stream the
+// same K and V through one L2.  (Groups beyond the last multiple of 8 are spread over the XCDs.)
+// The query tiles are dealt in the order `order` asks for, that of all groups before the next one, so that the workgroups
 // with the most key tiles start first and the launch ends on the short ones: kEdgesFirst for the far
 // tiles (a query tile at either end of the sequence has the most), kMiddleFirst for the near tiles, kLastFirst for
-// the far tiles of a causal call (a query tile sees the keys before it: the last one has the most).
+// the far tiles of a causal call (a query tile sees the keys before it: the last one has the most).  Only as many groups are
+// taken together as leave their K and V in an XCD's 4 MB of L2: 96 query tiles of 16-bit head_dim 64 are 3 MB.
 enum { kNatural = 0, kEdgesFirst = 1, kMiddleFirst = 2, kLastFirst = 3 };
 __device__ __forceinline__ void block_map(int n, int nx, int heads, int tiles_per_seq, bool fixed, int order, int& xq,
                                           int& h) {
-  const int groups = fixed ? (nx / tiles_per_seq) * heads : 1;
-  if (fixed && (groups & 7) == 0) {
-    const int xcd = n & 7, slot = n >> 3;
-    const int grp = xcd + 8 * (slot / tiles_per_seq);
-    int t = slot % tiles_per_seq;
+  if (fixed) {
+    const int groups = (nx / tiles_per_seq) * heads;
+    const int most = 8 * max(1, 96 / tiles_per_seq);   // groups taken together
+    const int first = n / (most * tiles_per_seq) * most;
+    const int here = min(groups - first, most), m = n - first * tiles_per_seq;
+    const int i = m % here;
+    int t = m / here;
+    const int grp = first + (i < (here & ~7) ? (n & 7) | (i & ~7) : i);
     if (order == kLastFirst) {
       t = tiles_per_seq - 1 - t;
     } else if (order != kNatural) {
@@ -279,9 +283,6 @@ __device__ __forceinline__ void block_map(int n, int nx, int heads, int tiles_pe
     }
     xq = (grp / heads) * tiles_per_seq + t;
     h = grp % heads;
-  } else if (fixed) {
-    xq = n % nx;
-    h = n / nx;
   } else {
     // packed sequences: the work-list holds the tiles longest sequence first; all heads of a tile are
     // dealt before the next tile, so the whole launch runs from long workgroups to short ones

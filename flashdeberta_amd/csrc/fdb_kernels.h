@@ -128,7 +128,6 @@ struct FdbBwdRingParams {
   int64_t dv_sb, dv_st, dv_sh;
   int64_t pk_sh, pk_sr, pq_sh, pq_sr, dp_sh, dp_sr;
   int32_t B, H, L, S, R, causal;
-  int32_t pairs_per_xcd;
   int32_t stat_len, g_rows, g_slots;
   int32_t rho_min, tg_groups, tg_parts, tg_chunks, tg_len;  // blocks of 32 relative positions in groups of four; shares of the tokens; chunks of
                                                             // tg_len row blocks per batch row
