@@ -20,6 +20,8 @@
 
 #include <cmath>
 #include <map>
+#include <memory>
+#include <mutex>
 #include <optional>
 #include <tuple>
 #include <utility>
@@ -81,6 +83,13 @@ int fdb_dtype_of(at::ScalarType t) {
   }
 }
 
+// Memory that can be read through data_ptr(): not a wrapper around other tensors (quantised or distributed parameters, functorch's).
+bool plain_memory(const Tensor& t) {
+  constexpr c10::DispatchKeySet wrapped({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                         c10::DispatchKey::Conjugate, c10::DispatchKey::Negative, c10::DispatchKey::ZeroTensor});
+  return t.layout() == at::kStrided && !t.key_set().has_any(wrapped);
+}
+
 void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
 int64_t att_span(int64_t buckets, int64_t max_relative) { return buckets > 0 ? buckets : max_relative; }
@@ -99,10 +108,14 @@ struct GemmKey {
   }
 };
 struct GemmPlan {
+  hipblasLtHandle_t handle = nullptr;
   hipblasLtMatmulDesc_t desc = nullptr;
   hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
   hipblasLtMatmulAlgo_t algo;
   int64_t workspace = 0;
+  GemmPlan() = default;
+  GemmPlan(const GemmPlan&) = delete;
+  GemmPlan& operator=(const GemmPlan&) = delete;
   ~GemmPlan() {
     if (a) hipblasLtMatrixLayoutDestroy(a);
     if (b) hipblasLtMatrixLayoutDestroy(b);
@@ -123,60 +136,64 @@ hipDataType blas_type(at::ScalarType t) {
   }
 }
 
+// Handles, plans and the bias pointer a plan carries into its launch are shared by the threads of a program: autograd runs the
+// backward's products on its own threads, without the GIL.  Held for a lookup or a launch, never while memory is asked for.
+std::mutex g_blas_mutex;
+
 hipblasLtHandle_t blas_handle(int device) {
-  static hipblasLtHandle_t handles[64] = {};
-  if (!handles[device]) blas(hipblasLtCreate(&handles[device]), "hipblasLtCreate");
-  return handles[device];
+  static std::map<int, hipblasLtHandle_t> handles;
+  hipblasLtHandle_t& h = handles[device];
+  if (!h) blas(hipblasLtCreate(&h), "hipblasLtCreate");
+  return h;
 }
 
 // The library is column-major: D^T [N, M] = op(B)^T op(A)^T, so B's memory is its first operand and A's the second.
-std::map<GemmKey, GemmPlan> g_plans;  // reached with the GIL held
-GemmPlan& gemm_plan(const GemmKey& key) {
+std::map<GemmKey, std::shared_ptr<GemmPlan>> g_plans;
+std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
+  const std::lock_guard<std::mutex> lock(g_blas_mutex);
   const auto hit = g_plans.find(key);
   if (hit != g_plans.end()) return hit->second;
-  if (g_plans.size() >= kMostPlans) g_plans.clear();
-  GemmPlan& p = g_plans[key];
-  try {
-    blas(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F), "hipblasLtMatmulDescCreate");
-    const auto set = [&](hipblasLtMatmulDescAttributes_t what, const void* v, size_t n) { blas(hipblasLtMatmulDescSetAttribute(p.desc, what, v, n), "hipblasLtMatmulDescSetAttribute"); };
-    const hipblasOperation_t op_first = key.flags & 2 ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_second = key.flags & 1 ? HIPBLAS_OP_T : HIPBLAS_OP_N;
-    set(HIPBLASLT_MATMUL_DESC_TRANSA, &op_first, sizeof(op_first));
-    set(HIPBLASLT_MATMUL_DESC_TRANSB, &op_second, sizeof(op_second));
-    const auto in = (hipDataType)key.type, out = (hipDataType)key.out_type;
-    if (key.flags & 4) {
-      const hipblasLtEpilogue_t e = HIPBLASLT_EPILOGUE_BIAS;
-      set(HIPBLASLT_MATMUL_DESC_EPILOGUE, &e, sizeof(e));
-      set(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &in, sizeof(in));
-    }
-    // row-major [M, K] with row stride lda is column-major [K, M]
-    blas(hipblasLtMatrixLayoutCreate(&p.a, in, key.flags & 2 ? key.k : key.n, key.flags & 2 ? key.n : key.k, key.ldb), "hipblasLtMatrixLayoutCreate");
-    blas(hipblasLtMatrixLayoutCreate(&p.b, in, key.flags & 1 ? key.m : key.k, key.flags & 1 ? key.k : key.m, key.lda), "hipblasLtMatrixLayoutCreate");
-    blas(hipblasLtMatrixLayoutCreate(&p.d, out, key.n, key.m, key.ldd), "hipblasLtMatrixLayoutCreate");
-    if (key.batch > 1) {
-      const int32_t count = (int32_t)key.batch;
-      const std::pair<hipblasLtMatrixLayout_t, int64_t> ls[] = {{p.a, key.sb}, {p.b, key.sa}, {p.d, key.sd}};
-      for (const auto& l : ls) {
-        blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &count, sizeof(count)), "hipblasLtMatrixLayoutSetAttribute");
-        blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &l.second, sizeof(l.second)), "hipblasLtMatrixLayoutSetAttribute");
-      }
-    }
-    hipblasLtMatmulPreference_t pref = nullptr;
-    blas(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
-    const size_t most = at::cuda::getCUDABlasLtWorkspaceSize();  // torch's own bound, so that the choice is torch's own
-    hipblasLtMatmulHeuristicResult_t found = {};
-    int n = 0;
-    hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most, sizeof(most));
-    const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(blas_handle(key.device), p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
-    hipblasLtMatmulPreferenceDestroy(pref);
-    blas(rc, "hipblasLtMatmulAlgoGetHeuristic");
-    TORCH_CHECK(n > 0, "hipBLASLt has no kernel for this product");
-    p.algo = found.algo;
-    p.workspace = (int64_t)found.workspaceSize;
-  } catch (...) {
-    g_plans.erase(key);
-    throw;
+  const auto plan = std::make_shared<GemmPlan>();
+  GemmPlan& p = *plan;
+  p.handle = blas_handle(key.device);
+  blas(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F), "hipblasLtMatmulDescCreate");
+  const auto set = [&](hipblasLtMatmulDescAttributes_t what, const void* v, size_t n) { blas(hipblasLtMatmulDescSetAttribute(p.desc, what, v, n), "hipblasLtMatmulDescSetAttribute"); };
+  const hipblasOperation_t op_first = key.flags & 2 ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_second = key.flags & 1 ? HIPBLAS_OP_T : HIPBLAS_OP_N;
+  set(HIPBLASLT_MATMUL_DESC_TRANSA, &op_first, sizeof(op_first));
+  set(HIPBLASLT_MATMUL_DESC_TRANSB, &op_second, sizeof(op_second));
+  const auto in = (hipDataType)key.type, out = (hipDataType)key.out_type;
+  if (key.flags & 4) {
+    const hipblasLtEpilogue_t e = HIPBLASLT_EPILOGUE_BIAS;
+    set(HIPBLASLT_MATMUL_DESC_EPILOGUE, &e, sizeof(e));
+    set(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &in, sizeof(in));
   }
-  return p;
+  // row-major [M, K] with row stride lda is column-major [K, M]
+  blas(hipblasLtMatrixLayoutCreate(&p.a, in, key.flags & 2 ? key.k : key.n, key.flags & 2 ? key.n : key.k, key.ldb), "hipblasLtMatrixLayoutCreate");
+  blas(hipblasLtMatrixLayoutCreate(&p.b, in, key.flags & 1 ? key.m : key.k, key.flags & 1 ? key.k : key.m, key.lda), "hipblasLtMatrixLayoutCreate");
+  blas(hipblasLtMatrixLayoutCreate(&p.d, out, key.n, key.m, key.ldd), "hipblasLtMatrixLayoutCreate");
+  if (key.batch > 1) {
+    const int32_t count = (int32_t)key.batch;
+    const std::pair<hipblasLtMatrixLayout_t, int64_t> ls[] = {{p.a, key.sb}, {p.b, key.sa}, {p.d, key.sd}};
+    for (const auto& l : ls) {
+      blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &count, sizeof(count)), "hipblasLtMatrixLayoutSetAttribute");
+      blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &l.second, sizeof(l.second)), "hipblasLtMatrixLayoutSetAttribute");
+    }
+  }
+  hipblasLtMatmulPreference_t pref = nullptr;
+  blas(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
+  const size_t most = at::cuda::getCUDABlasLtWorkspaceSize();  // torch's own bound, so that the choice is torch's own
+  hipblasLtMatmulHeuristicResult_t found = {};
+  int n = 0;
+  hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most, sizeof(most));
+  const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(p.handle, p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
+  hipblasLtMatmulPreferenceDestroy(pref);
+  blas(rc, "hipblasLtMatmulAlgoGetHeuristic");
+  TORCH_CHECK(n > 0, "hipBLASLt has no kernel for this product");
+  p.algo = found.algo;
+  p.workspace = (int64_t)found.workspaceSize;
+  if (g_plans.size() >= kMostPlans) g_plans.clear();
+  g_plans.emplace(key, plan);
+  return plan;
 }
 
 struct Mat {  // `batch` row-major matrices, `ld` elements between rows, `stride` elements between matrices
@@ -186,13 +203,15 @@ struct Mat {  // `batch` row-major matrices, `ld` elements between rows, `stride
 void gemm(const Tensor& on, at::ScalarType type, at::ScalarType out_type, bool trans_a, bool trans_b, int64_t batch, int64_t m, int64_t n, int64_t k,
           Mat a, Mat b, Mat d, const void* bias = nullptr, bool accumulate = false) {
   const int device = on.get_device();
-  GemmPlan& p = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, batch, a.stride, b.stride, d.stride, device, (int32_t)blas_type(type), (int32_t)blas_type(out_type),
+  const auto plan = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, batch, a.stride, b.stride, d.stride, device, (int32_t)blas_type(type), (int32_t)blas_type(out_type),
                                   (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
-  if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias, sizeof(bias)), "hipblasLtMatmulDescSetAttribute");
+  GemmPlan& p = *plan;
   Tensor ws;
   if (p.workspace > 0) ws = at::empty({p.workspace}, on.options().dtype(at::kByte));
   const float one = 1.f, beta = accumulate ? 1.f : 0.f;
-  blas(hipblasLtMatmul(blas_handle(device), p.desc, &one, b.p, p.a, a.p, p.b, &beta, d.p, p.d, const_cast<void*>(d.p), p.d, &p.algo,
+  const std::lock_guard<std::mutex> lock(g_blas_mutex);
+  if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias, sizeof(bias)), "hipblasLtMatmulDescSetAttribute");
+  blas(hipblasLtMatmul(p.handle, p.desc, &one, b.p, p.a, a.p, p.b, &beta, d.p, p.d, const_cast<void*>(d.p), p.d, &p.algo,
                        p.workspace > 0 ? ws.data_ptr() : nullptr, p.workspace, (hipStream_t)stream_of(on)),
        "hipblasLtMatmul");
 }
@@ -205,9 +224,11 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
   const auto type = x_in.scalar_type();
   const bool half = type == at::kBFloat16 || type == at::kHalf;
   const int64_t k = x_in.size(-1), m = k > 0 ? x_in.numel() / k : 0;
-  if (!x_in.is_cuda() || !half || w.scalar_type() != type || (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 ||
-      w.stride(1) != 1 || k != w.size(1) || !bias || !bias->is_contiguous())
+  if (!x_in.is_cuda() || !half || !plain_memory(x_in) || !plain_memory(w) || (bias && !plain_memory(*bias)) || w.scalar_type() != type || (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 ||
+      w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) || w.device() != x_in.device() || !bias || bias->device() != x_in.device() ||
+      bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())
     return at::linear(x_in, w, bias);
+  const c10::hip::HIPGuard guard(x_in.get_device());
   const Tensor x = x_in.contiguous();
   const int64_t n = w.size(0);
   auto size = x.sizes().vec();
@@ -233,24 +254,33 @@ PyObject* py_linear(PyObject*, PyObject* const* x, Py_ssize_t n) {
 
 // ---- the delta table on the device ---------------------------------------------------------------------------------
 // One per (buckets, positions, device), built by the Python callable registered below and kept for the life of the
-// process like the host table it comes from.  Reached with the GIL held.
+// process like the host table it comes from.  Threads of a program share them, autograd's among them, which do not hold the GIL.
 struct Lut {
   Tensor table;
-  int32_t radius;
+  int32_t radius = 0;
 };
 PyObject* g_lut_source = nullptr;
-std::map<std::tuple<int64_t, int64_t, int>, Lut> g_luts;
+std::mutex g_lut_mutex;
+std::map<std::tuple<int64_t, int64_t, int>, Lut> g_luts;  // entries are never erased: references to them stay valid
 
 const Lut& lut_for(int64_t buckets, int64_t max_relative, const Tensor& on) {
   const auto key = std::make_tuple(buckets, max_relative, (int)on.get_device());
-  const auto hit = g_luts.find(key);
-  if (hit != g_luts.end()) return hit->second;
-  PyObject* dev = THPDevice_New(on.device());
-  if (!dev) throw python_error();
-  PyObject* r = PyObject_CallFunction(g_lut_source, "LLN", (long long)buckets, (long long)max_relative, dev);
-  if (!r) throw python_error();
-  Lut lut{THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(r, 1))};
-  Py_DECREF(r);
+  {
+    const std::lock_guard<std::mutex> lock(g_lut_mutex);
+    const auto hit = g_luts.find(key);
+    if (hit != g_luts.end()) return hit->second;
+  }
+  Lut lut;
+  {
+    const pybind11::gil_scoped_acquire gil;  // taken without the mutex: another thread may hold the GIL and wait for the mutex
+    PyObject* dev = THPDevice_New(on.device());
+    if (!dev) throw python_error();
+    PyObject* r = PyObject_CallFunction(g_lut_source, "LLN", (long long)buckets, (long long)max_relative, dev);
+    if (!r) throw python_error();
+    lut = {THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(r, 1))};
+    Py_DECREF(r);
+  }
+  const std::lock_guard<std::mutex> lock(g_lut_mutex);
   return g_luts.emplace(key, std::move(lut)).first->second;
 }
 
@@ -334,6 +364,8 @@ Tensor run_forward(fdb_attn_args& a, const Tensor& on, at::ScalarType qt, const 
   if (o.pos_query) pq = pos_arg(*o.pos_query, H, D, span, "pos_query");
   TORCH_CHECK_VALUE(!pk.defined() || pk.scalar_type() == qt, "pos_key dtype ", pk.scalar_type(), " does not match q dtype ", qt);
   TORCH_CHECK_VALUE(!pq.defined() || pq.scalar_type() == qt, "pos_query dtype ", pq.scalar_type(), " does not match q dtype ", qt);
+  for (const Tensor* t : {&pk, &pq})
+    TORCH_CHECK_VALUE(!t->defined() || t->device() == on.device(), "pos_key and pos_query must be on q's device ", on.device(), ", got ", t->device());
   const bool has_pos = pk.defined() || pq.defined();
   const int terms = 1 + (pk.defined() ? 1 : 0) + (pq.defined() ? 1 : 0);
   if (has_pos) {
@@ -392,6 +424,8 @@ std::pair<Tensor, Tensor> forward(const Tensor& q_in, const Tensor& k_in, const 
   }
   TORCH_CHECK_VALUE(k_in.sizes() == q_in.sizes() && v_in.sizes() == q_in.sizes(), "q, k, v must have the same shape (self-attention): ",
                     q_in.sizes(), " ", k_in.sizes(), " ", v_in.sizes());
+  TORCH_CHECK_VALUE(k_in.device() == q_in.device() && v_in.device() == q_in.device() && (!o.out || o.out->device() == q_in.device()),
+                    "q, k, v (and out) must be on one device");
   const auto qt = q_in.scalar_type();
   const bool fp8 = qt == at::kFloat8_e4m3fn;
   fdb_attn_args a = {};
@@ -543,6 +577,13 @@ void backward(const Tensor& on, int64_t B, int64_t L, int64_t H, Strided q, Stri
 // dq, dk, dv, d pos_key, d pos_query of the operator
 std::array<Tensor, 5> backward_of(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& out_in, const Tensor& lse, const Tensor& dout_in,
                                   const Tensor& pk_in, const Tensor& pq_in, const BwdSettings& o) {
+  for (const Tensor* t : {&k_in, &v_in, &out_in, &dout_in})
+    TORCH_CHECK_VALUE(t->sizes() == q_in.sizes() && t->scalar_type() == q_in.scalar_type() && t->device() == q_in.device(),
+                      "k, v, out and dout must have q's shape, dtype and device");
+  TORCH_CHECK_VALUE(lse.scalar_type() == at::kFloat && lse.device() == q_in.device() && lse.numel() == q_in.size(0) * q_in.size(1) * q_in.size(2),
+                    "lse must be the forward's float32 [B*L, H]");
+  for (const Tensor* t : {&pk_in, &pq_in})
+    TORCH_CHECK_VALUE(t->scalar_type() == q_in.scalar_type() && t->device() == q_in.device(), "pos_key and pos_query must have q's dtype and device");
   const Tensor q = unit_last(q_in), k = unit_last(k_in), v = unit_last(v_in), out = unit_last(out_in), dout = unit_last(dout_in);
   const int64_t B = q.size(0), L = q.size(1), H = q.size(2), D = q.size(3), span = att_span(o.buckets, o.max_relative);
   const c10::hip::HIPGuard guard(q.get_device());
@@ -758,12 +799,12 @@ PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
   a.heads = int_arg(x[8]);
   a.o = BwdSettings{float_arg(x[9]), int_arg(x[10]), int_arg(x[11]), false, opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
   const auto type = hidden.scalar_type();
-  if (!hidden.is_cuda() || (type != at::kBFloat16 && type != at::kHalf) || hidden.dim() != 3 || hidden.numel() == 0 || a.heads < 1) Py_RETURN_NONE;
+  if (!hidden.is_cuda() || !plain_memory(hidden) || (type != at::kBFloat16 && type != at::kHalf) || hidden.dim() != 3 || hidden.numel() == 0 || a.heads < 1) Py_RETURN_NONE;
   Tensor t[7];
   for (int i = 0; i < 7; ++i) {
     if (x[i + 1] == Py_None) Py_RETURN_NONE;
     t[i] = tensor_arg(x[i + 1], "parameters");
-    if (t[i].scalar_type() != type || t[i].device() != hidden.device()) Py_RETURN_NONE;
+    if (t[i].scalar_type() != type || t[i].device() != hidden.device() || !plain_memory(t[i])) Py_RETURN_NONE;
   }
   const int64_t C = hidden.size(2), W = t[1].size(0), span = att_span(a.o.buckets, a.o.max_relative);
   if (t[0].dim() != 2 || t[0].size(0) < 2 * span || t[0].size(1) != C || W != 64 * a.heads || C % 8) Py_RETURN_NONE;

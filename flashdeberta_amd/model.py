@@ -53,8 +53,9 @@ def _seq_bounds_of(attention_mask, memo):
 
 def _weight_and_bias(module):
     """A projection's parameters; a plain Linear's without nn.Module's attribute machinery (a quarter of a microsecond each)."""
-    if type(module) is torch.nn.Linear:
-        return module._parameters["weight"], module._parameters["bias"]
+    own = module._parameters
+    if type(module) is torch.nn.Linear and "weight" in own and "bias" in own:  # pruning and weight_norm move them elsewhere
+        return own["weight"], own["bias"]
     return module.weight, module.bias
 
 
@@ -272,11 +273,11 @@ class FlashDebertaV2Layer(DebertaV2Layer):
             return None
         shape = hidden_states.shape[-1:]
         for m in linears:
-            if type(m) is not torch.nn.Linear or m._parameters["weight"].dtype != hidden_states.dtype:
+            if type(m) is not torch.nn.Linear or m.weight.dtype != hidden_states.dtype:
                 return None
         for m in norms:
-            if type(m) is not torch.nn.LayerNorm or m.normalized_shape != shape or m._parameters["bias"] is None \
-                    or m._parameters["weight"].dtype != hidden_states.dtype:
+            if type(m) is not torch.nn.LayerNorm or m.normalized_shape != shape or m.bias is None or m.weight is None \
+                    or m.weight.dtype != hidden_states.dtype:
                 return None
         if any(_hooked(m) for m in (attention, intermediate, output, att, att_out, act, *linears, *norms,
                                       *att._modules.values())):
@@ -286,8 +287,7 @@ class FlashDebertaV2Layer(DebertaV2Layer):
             return None
         (ow, ob), (uw, ub), (dw, db) = [_weight_and_bias(m) for m in linears]
         n1, n2 = norms
-        return (*args, ow, ob, n1._parameters["weight"], n1._parameters["bias"], n1.eps, uw, ub, dw, db,
-                n2._parameters["weight"], n2._parameters["bias"], n2.eps)
+        return (*args, ow, ob, n1.weight, n1.bias, n1.eps, uw, ub, dw, db, n2.weight, n2.bias, n2.eps)
 
     def forward(self, hidden_states, attention_mask, query_states=None, relative_pos=None, rel_embeddings=None, output_attentions=False):
         if query_states is None or query_states is hidden_states:

@@ -270,7 +270,8 @@ def disentangled_attention_bwd(q, k, v, out, lse, dout, pos_key=None, pos_query=
     pos_query = _pos_arg(pos_query, H, D, span, "pos_query")
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(D * (1 + (pos_key is not None) + (pos_query is not None)))
-    if fused_chain is None and delta is None and pos_key is not None and pos_query is not None and D == 64 and q.dtype in (torch.bfloat16, torch.float16):
+    if fused_chain is None and delta is None and D == 64 and q.dtype in (torch.bfloat16, torch.float16) \
+            and all(x is not None and x.dtype == q.dtype for x in (pos_key, pos_query)):
         return native.attention_bwd(q, k, v, out, lse.contiguous(), dout, pos_key, pos_query, sm_scale, position_buckets, max_relative_positions,
                                     causal, seq_start, seq_len)
     q, k, v, dout = [x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v, dout)]

@@ -87,3 +87,77 @@ def test_encoder_layer_matches_the_module_by_module_forward(B, L):
         layer(x, mask, rel_embeddings=rel)
         handle.remove()
         assert calls
+
+
+def _attention(**kw):
+    from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
+
+    torch.manual_seed(5)
+    cfg = DebertaV2Config(hidden_size=128, num_attention_heads=2, relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32,
+                          max_relative_positions=64, share_att_key=True, hidden_dropout_prob=0.0, attention_probs_dropout_prob=0.0, **kw)
+    return FlashDisentangledSelfAttention(cfg).cuda().to(torch.bfloat16)
+
+
+@pytest.mark.gpu
+def test_projection_whose_weight_is_no_parameter():
+    """Pruning leaves `weight` an attribute beside the parameter `weight_orig`."""
+    from torch.nn.utils import prune
+
+    att = _attention().eval()
+    x, rel = torch.randn(1, 20, 128, device="cuda").to(torch.bfloat16), torch.randn(64, 128, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        ref = att(x, None, rel_embeddings=rel)[0]
+        prune.identity(att.query_proj, "weight")
+        assert torch.equal(att(x, None, rel_embeddings=rel)[0], ref)
+
+
+@pytest.mark.gpu
+def test_operands_of_another_device_or_size_are_refused():
+    x, w, b = [torch.randn(*s, device="cuda").to(torch.bfloat16) for s in ((4, 64), (64, 64), (64,))]
+    for bad in ((x, w.cpu(), b), (x, w, b.cpu()), (x, w, b[:32].contiguous())):
+        with pytest.raises(RuntimeError):
+            _lib.native.linear(*bad, True)
+    q = torch.randn(1, 40, 2, 64, device="cuda").to(torch.bfloat16)
+    pos = torch.randn(2, 64, 64, device="cuda").to(torch.bfloat16)
+    lse = torch.zeros(40, 2, device="cuda")
+    tail = (0.1, 32, 64, False, None, None)
+    for bad in ((q, q, q, q, lse, q[:, :20], pos, pos), (q, q, q, q, lse[:20], q, pos, pos), (q, q, q, q, lse, q.float(), pos, pos),
+                (q, q, q, q, lse, q, pos.cpu(), pos)):
+        with pytest.raises(ValueError):
+            _lib.native.attention_bwd(*bad, *tail)
+    with pytest.raises(ValueError):
+        _lib.native.attention_fwd(q, q.cpu(), q, pos, pos, None, None, 0.1, 32, 64, False, False, *([None] * 7), False, 0, 0, None, False, 0, None)
+
+
+@pytest.mark.gpu
+def test_threads_share_the_plans():
+    """Forward and backward of layers of many lengths from several threads: the products' plans are made, found and launched by
+    these threads and by autograd's own, which do not hold the GIL."""
+    import threading
+
+    att = _attention().train()
+    rel = torch.randn(64, 128, device="cuda").to(torch.bfloat16)
+    xs = [torch.randn(1, n, 128, device="cuda").to(torch.bfloat16).requires_grad_() for n in range(33, 53)]
+
+    def gradients(x):
+        out = att(x, None, rel_embeddings=rel)[0]
+        return torch.autograd.grad(out, [x, att.value_proj.bias], torch.ones_like(out))
+
+    got, failed = {}, []
+
+    def work(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                got[k] = [gradients(x) for x in xs[k % 2::2]]
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:   # noqa: BLE001  (reported below, in the main thread)
+            failed.append(e)
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not failed, failed
+    for k in range(4):
+        for x, g in zip(xs[k % 2::2], got[k]):
+            assert all(torch.equal(a, b) for a, b in zip(g, gradients(x)))
