@@ -3,7 +3,7 @@
 // and returns their gradients as tensors, serves the other types, head_dims and term sets.)
 // Counterpart of src/flashdeberta/ops/flash_attention.py:490-1086 and of the autograd backward of model.py:189-192.
 //
-// Two launches of one kernel, a role each, then two small ones for the tables:
+// Two roles of one kernel, as one launch or one after the other, then two small launches for the tables:
 //   role dQ    : lane side X = queries (4 waves x 32 rows, one row per lane and its partner lane ^ 32), loop side Y = keys
 //   role dK/dV : X = keys, Y = queries
 // With x a lane row, y a loop row and r' = x - y (the relative position i - j in the dQ role, j - i in the other) both roles see
@@ -107,8 +107,10 @@ __device__ __forceinline__ Zones zones_of(int m0, int Lb, int R, bool causal, bo
   return z;
 }
 
-template <class QT, int ROLE>
-__global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdRingParams p) {
+// One workgroup of a role, the wg-th of its grid.  STATS: the row statistics are there (fdb_row_stats_kernel); otherwise the dQ role,
+// launched on its own before the other, computes them on its way.
+template <class QT, int ROLE, bool STATS>
+__device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg) {
   constexpr bool kDQ = ROLE == 0;
   constexpr int KS = 4, DBLKS = 2;
   using frag = typename QT::frag;
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
   // near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
   const int tiles = (p.L + FDB_BM - 1) / FDB_BM;
   int tile_x, h;
-  block_map((int)blockIdx.x, p.B * tiles, p.H, tiles, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, tile_x, h);
+  block_map(wg, p.B * tiles, p.H, tiles, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, tile_x, h);
   const int b = tile_x / tiles;
   tile_x -= b * tiles;
   const int m0 = tile_x * FDB_BM;
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
       clear(p.dv, p.dv_sb, p.dv_st, p.dv_sh);
     }
   }
-  if (kDQ && blockIdx.x == 0 && tid < 128) *(u32x4*)(p.zero_block + tid * 16) = u32x4{0u, 0u, 0u, 0u};  // what stands in for a block of G that no step met
+  if (kDQ && wg == 0 && tid < 128) *(u32x4*)(p.zero_block + tid * 16) = u32x4{0u, 0u, 0u, 0u};  // what stands in for a block of G that no step met
   if (m0 >= Lb) return;
   auto base = [&](const char* ptr, int64_t sb, int64_t st, int64_t sh) { return ptr + (b * sb + (int64_t)tok0 * st + (int64_t)h * sh) * 2; };
   const char* qb = base(p.q, p.q_sb, p.q_st, p.q_sh);
@@ -169,7 +171,12 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
   for (int s = 0; s < KS; ++s) x2[s] = x_ok ? QT::load(x2b + ((int64_t)xr * x2_st + 16 * s + 8 * g) * 2) : QT::zero();
   const int64_t stat_row = ((int64_t)b * p.H + h) * p.stat_len;   // row statistics by (batch row, head), local row index
   float lse_x = 0.f, del_x = 0.f;   // dQ role: -lse in base 2, -Delta
-  if (kDQ) {
+  if (kDQ && STATS) {
+    if (x_ok) {
+      lse_x = p.neg_lse[stat_row + xr];
+      del_x = p.neg_delta[stat_row + xr];
+    }
+  } else if (kDQ) {
     // Delta = dO . O of this lane's row; both statistics are left for the dK/dV launch in the form it starts its products from
     const char* ob = base(p.out, p.o_sb, p.o_st, p.o_sh);
     float dot = 0.f;
@@ -676,6 +683,43 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
   }
 }
 
+template <class QT, int ROLE>
+__global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdRingParams p) {
+  bwd_ring<QT, ROLE, false>(p, (int)blockIdx.x);
+}
+
+// Both roles as one launch, the longer one's workgroups first: 2 x 288 workgroups, say, leave half of the GPU's 512 places empty
+// as two launches and fill them as one.
+template <class QT>
+__global__ __launch_bounds__(kThreads, 2) void fdb_bwd_both_kernel(const FdbBwdRingParams p) {
+  const int n = (int)(gridDim.x >> 1), wg = (int)blockIdx.x;
+  if (wg < n) bwd_ring<QT, 1, true>(p, wg);
+  else bwd_ring<QT, 0, true>(p, wg - n);
+}
+
+// The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), eight lanes a row, 32 rows a workgroup.  Bound by reading dO and O.
+template <class QT>
+__global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingParams p) {
+  const int b = (int)blockIdx.z, h = (int)blockIdx.y, c = threadIdx.x & 7, row = (int)blockIdx.x * 32 + (int)(threadIdx.x >> 3);
+  const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
+  const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
+  if (row >= Lb) return;   // a row's eight lanes leave together
+  const int64_t tok = (int64_t)tok0 + row;
+  const f32x8 o8 = QT::to_f32(QT::load(p.out + ((int64_t)b * p.o_sb + tok * p.o_st + (int64_t)h * p.o_sh + 8 * c) * 2));
+  const f32x8 g8 = QT::to_f32(QT::load(p.dout + ((int64_t)b * p.g_sb + tok * p.g_st + (int64_t)h * p.g_sh + 8 * c) * 2));
+  const float lse = p.lse[((int64_t)b * p.L + tok) * p.H + h];
+  float dot = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(o8[e], g8[e], dot);
+#pragma unroll
+  for (int x = 1; x < 8; x *= 2) dot += __shfl_xor(dot, x);
+  if (c == 0) {
+    const int64_t at = ((int64_t)b * p.H + h) * p.stat_len + row;
+    p.neg_lse[at] = lse * -1.4426950408889634f;
+    p.neg_delta[at] = -dot;
+  }
+}
+
 // ---- gradients of the tables ----------------------------------------------------------------------------------------------
 // dE_K[r] = sum_i G[i][r] q_i and dE_Q[r] = sum_i G[i][r] k_(i-r) for blocks of 32 relative positions r = 32 rho + c, from the blocks
 // [32 i x 32 c] of G the dQ launch stored.  A workgroup is four waves with four neighbouring rho of one head; it walks row blocks I
@@ -932,19 +976,32 @@ __global__ __launch_bounds__(256) void fdb_table_fold_kernel(const FdbBwdRingPar
   *out = (T)(sum * p.sm_scale);
 }
 
+// Up to so many workgroups a role, the two roles are one launch (with the statistics' own launch before it): what each leaves empty at
+// its end the other fills, while a launch of many rounds has little to fill and pays for the statistics.  Whole backward, 12 heads,
+// two launches -> one: 1x512 (48 a role) 92 -> 65 us, 8x512 (384) 139 -> 121, 2x1501 (288) 236 -> 196, 4x2048 (768) 434 -> 412,
+// 4x4096 (1536) 1195 -> 1178; 8x4096 (3072) would go from 2350 to 2395.
+constexpr unsigned kMostTogether = 2048;
+
 template <class QT>
 int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
   auto dq = fdb_bwd_ring_kernel<QT, 0>;
   auto dkv = fdb_bwd_ring_kernel<QT, 1>;
   auto tg = fdb_table_grad_kernel<QT>;
-  static std::atomic<uint64_t> set0{0}, set1{0}, set2{0};
+  auto both = fdb_bwd_both_kernel<QT>;
+  static std::atomic<uint64_t> set0{0}, set1{0}, set2{0}, set3{0};
   hipError_t e = fdb_set_lds_once((const void*)dq, kLds, set0);
   if (e == hipSuccess) e = fdb_set_lds_once((const void*)dkv, kLds, set1);
   if (e == hipSuccess) e = fdb_set_lds_once((const void*)tg, kTgLds, set2);
+  if (e == hipSuccess) e = fdb_set_lds_once((const void*)both, kLds, set3);
   if (e != hipSuccess) return (int)e;
   const unsigned tiles = (unsigned)((p.L + FDB_BM - 1) / FDB_BM), grid = tiles * (unsigned)p.H * (unsigned)p.B;
-  hipLaunchKernelGGL(dq, dim3(grid), dim3(kThreads), kLds, stream, p);
-  hipLaunchKernelGGL(dkv, dim3(grid), dim3(kThreads), kLds, stream, p);
+  if (grid <= kMostTogether) {
+    hipLaunchKernelGGL(fdb_row_stats_kernel<QT>, dim3((unsigned)((p.L + 31) / 32), (unsigned)p.H, (unsigned)p.B), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(both, dim3(2 * grid), dim3(kThreads), kLds, stream, p);
+  } else {
+    hipLaunchKernelGGL(dq, dim3(grid), dim3(kThreads), kLds, stream, p);
+    hipLaunchKernelGGL(dkv, dim3(grid), dim3(kThreads), kLds, stream, p);
+  }
   hipLaunchKernelGGL(tg, dim3((unsigned)(p.H * p.tg_parts), (unsigned)(p.tg_groups + (p.has_far ? 1 : 0))), dim3(kThreads), kTgLds, stream, p);
   hipLaunchKernelGGL(fdb_table_fold_kernel<QT>, dim3((unsigned)((2 * p.S + kFoldRows - 1) / kFoldRows), (unsigned)p.H, 2), dim3(256), 0, stream, p);
   return (int)hipGetLastError();
