@@ -363,6 +363,7 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
   p.pq_sh = a->pq_stride_h; p.pq_sr = a->pq_stride_r;
   p.B = a->batch; p.H = a->heads; p.L = a->max_seqlen;
   p.tiles_per_seq = (a->max_seqlen + FDB_BM - 1) / FDB_BM;
+  p.groups_together = fdb_groups_together(p.tiles_per_seq);
   p.R = a->lut_radius > 0 ? a->lut_radius : 1;
   p.causal = a->causal ? 1 : 0;
   p.scale_log2 = a->sm_scale * 1.4426950408889634f;
@@ -370,7 +371,6 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
   p.fill_pad = (!a->cu_seqlens && (a->seq_start || a->seq_len)) ? 1 : 0;
   const int64_t grid_x = query_tiles(a);
   if (grid_x < 1 || grid_x * a->heads > INT32_MAX) return FDB_ERR_SHAPE;
-  p.grid_x = (int32_t)grid_x;
   // Split path: the far tiles in a far-only run of the kernel (three workgroups per CU), the near
   // tiles in a second launch, which merges the two.  It needs the log-sum-exp buffer as the
   // hand-over between the two launches.
@@ -589,6 +589,8 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   p->B = a->batch; p->H = a->heads; p->L = a->seqlen; p->S = a->att_span; p->R = a->lut_radius; p->causal = a->causal ? 1 : 0;
   p->stat_len = (a->seqlen + 31) / 32 * 32 + 32;
   p->g_rows = (int32_t)(4 * tiles);
+  p->tiles = (int32_t)tiles;
+  p->groups_together = fdb_groups_together(p->tiles);
   // Blocks of 32 relative positions a wave's row block meets: those of its tile's near steps and one more (see Zones)
   const int32_t R = a->lut_radius, n_blk = (a->seqlen + 31) / 32;
   const int32_t most = (FDB_BM - 1 + 2 * R + 2 * 31) / 32 + 1;

@@ -120,11 +120,8 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   // near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
-  const int tiles = (p.L + FDB_BM - 1) / FDB_BM;
-  int tile_x, h;
-  block_map(wg, p.B * tiles, p.H, tiles, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, tile_x, h);
-  const int b = tile_x / tiles;
-  tile_x -= b * tiles;
+  int b, tile_x, h;
+  block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, b, tile_x, h);
   const int m0 = tile_x * FDB_BM;
   const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
@@ -697,23 +694,33 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_both_kernel(const FdbBwdR
   else bwd_ring<QT, 0, true>(p, wg - n);
 }
 
-// The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), eight lanes a row, 32 rows a workgroup.  Bound by reading dO and O.
+// The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), 128 rows a workgroup, two lanes a row that add up in the dQ
+// role's order, so that a batch row's gradients have the same bits whichever way it is launched.  Bound by reading dO and O.
 template <class QT>
 __global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingParams p) {
-  const int b = (int)blockIdx.z, h = (int)blockIdx.y, c = threadIdx.x & 7, row = (int)blockIdx.x * 32 + (int)(threadIdx.x >> 3);
+  const int b = (int)blockIdx.z, h = (int)blockIdx.y, g = threadIdx.x & 1, row = (int)blockIdx.x * 128 + (int)(threadIdx.x >> 1);
   const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
-  if (row >= Lb) return;   // a row's eight lanes leave together
+  if (row >= Lb) return;   // a row's two lanes leave together
   const int64_t tok = (int64_t)tok0 + row;
-  const f32x8 o8 = QT::to_f32(QT::load(p.out + ((int64_t)b * p.o_sb + tok * p.o_st + (int64_t)h * p.o_sh + 8 * c) * 2));
-  const f32x8 g8 = QT::to_f32(QT::load(p.dout + ((int64_t)b * p.g_sb + tok * p.g_st + (int64_t)h * p.g_sh + 8 * c) * 2));
+  const char* orow = p.out + ((int64_t)b * p.o_sb + tok * p.o_st + (int64_t)h * p.o_sh + 8 * g) * 2;
+  const char* grow = p.dout + ((int64_t)b * p.g_sb + tok * p.g_st + (int64_t)h * p.g_sh + 8 * g) * 2;
+  typename QT::frag o[4], d[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    o[s] = QT::load(orow + 32 * s);
+    d[s] = QT::load(grow + 32 * s);
+  }
   const float lse = p.lse[((int64_t)b * p.L + tok) * p.H + h];
   float dot = 0.f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(o8[e], g8[e], dot);
+  for (int s = 0; s < 4; ++s) {
+    const f32x8 o8 = QT::to_f32(o[s]), g8 = QT::to_f32(d[s]);
 #pragma unroll
-  for (int x = 1; x < 8; x *= 2) dot += __shfl_xor(dot, x);
-  if (c == 0) {
+    for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(o8[e], g8[e], dot);
+  }
+  dot += __shfl_xor(dot, 1);
+  if (g == 0) {
     const int64_t at = ((int64_t)b * p.H + h) * p.stat_len + row;
     p.neg_lse[at] = lse * -1.4426950408889634f;
     p.neg_delta[at] = -dot;
@@ -821,57 +828,75 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     const int n_rows = (Lb + 31) / 32;                       // row blocks of this sequence
     const int I0 = c0 * p.tg_len, I1 = min(n_rows, I0 + p.tg_len);
     if (I0 >= I1) continue;
-    const char* qb = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2;
-    const char* kb = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2;
-    const char* gb = p.g_blocks + ((int64_t)b * p.H + h) * p.g_rows * (int64_t)p.g_slots * kGBlk;
-    auto rows_dma = [&](const char* base, int64_t row_bytes, uint32_t lane_off, int blk, uint32_t dst) __attribute__((always_inline)) {
-      if (blk >= 0 && (blk + 1) * 32 <= Lb) {
-        dma16sn(base + (int64_t)(blk * 32) * row_bytes, lane_off, dst + wave_kb);
-      } else {
-        const int row = max(0, min(blk * 32 + srow, Lb - 1));   // rows outside the sequence: finite values that meet zeros
-        dma16n(base + (int64_t)row * row_bytes + chunk_off, dst + wave_kb);
-      }
+    const int full = Lb / 32;                                // those of 32 rows
+    const int rho0 = p.rho_min + 4 * group;
+    // What is fetched next: row block I of q and of G, row block J = I - 1 - rho0 of k (the wave w = 0 uses the newest).  The places in
+    // memory and the zones of I's tile are carried along: computed per row block they were two thirds of a turn's instructions.
+    int I = I0, J = I0 - 1 - rho0;
+    const int64_t q_step = p.q_st * 64, k_step = p.k_st * 64, g_step = (int64_t)p.g_slots * kGBlk;
+    const char* const q_rows = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2;
+    const char* const k_rows = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2;
+    uint64_t q_at = (uint64_t)(uintptr_t)q_rows + (uint64_t)(I * q_step), k_at = (uint64_t)(uintptr_t)k_rows + (uint64_t)(J * k_step);
+    uint64_t g_at = (uint64_t)(uintptr_t)p.g_blocks + (uint64_t)((((int64_t)b * p.H + h) * p.g_rows + I) * g_step);
+    int z0 = 0, zn = -1;   // first near step of the tile, number of near steps or -1
+    auto zone_at = [&](int row_block) __attribute__((always_inline)) {
+      const Zones z = zones_of(row_block / 4 * FDB_BM, Lb, p.R, p.causal, true);
+      z0 = z.s0;
+      zn = z.s1 > z.s0 ? z.s1 - z.s0 : -1;
+    };
+    auto clamped_dma = [&](const char* rows, int64_t step, int blk, uint32_t dst) __attribute__((always_inline)) {
+      const int row = max(0, min(blk * 32 + srow, Lb - 1));   // rows outside the sequence: finite values that meet zeros
+      dma16n(rows + (int64_t)row * (step / 32) + chunk_off, dst + wave_kb);
     };
     // block (I, rho) into a ring slot; a block of zeros where the dQ launch met no such block (no near step, or outside the
     // sequence).  Returns whether there is one.
-    auto g_dma = [&](int I, uint32_t ring) __attribute__((always_inline)) {
-      const Zones z = zones_of(max(I, 0) / 4 * FDB_BM, Lb, p.R, p.causal, true);
-      const int k = I - rho - z.s0;
-      const bool there = I >= 0 && I < n_rows && z.s1 > z.s0 && k >= 0 && k <= z.s1 - z.s0;
-      const char* src = there ? gb + ((int64_t)I * p.g_slots + k) * kGBlk : p.zero_block;
+    auto g_dma = [&](int row_block, uint64_t at, uint32_t ring) __attribute__((always_inline)) {
+      const int k = row_block - rho - z0;
+      const bool there = (uint32_t)row_block < (uint32_t)n_rows && k >= 0 && k <= zn;
+      const char* src = there ? (const char*)(uintptr_t)(at + (uint64_t)((int64_t)k * kGBlk)) : p.zero_block;
       dma16sn(src, lane * 16, g_base + ring * kGBlk);
       dma16sn(src + 1024, lane * 16, g_base + ring * kGBlk + 1024);
       return there;
     };
-    const int rho0 = p.rho_min + 4 * group;
     __syncthreads();   // the item before is done with the rings
-    // rows of k: J = I - 1 - rho; the wave w = 0 uses the newest
-    for (int w = 1; w < 4; ++w) rows_dma(kb, p.k_st * 2, k_lane, I0 - 1 - rho0 - w, kTgOffK + (uint32_t)(kKRing - w) * kTile);
-    bool prev = g_dma(I0 == 0 ? -1 : I0 - 1, kGRing - 1);
-    auto fetch = [&](int n, uint32_t ring, uint32_t kslot) __attribute__((always_inline)) {   // what row block I0 + n needs first, four loads per wave
-      rows_dma(qb, p.q_st * 2, q_lane, I0 + n, ring * kTile);
-      rows_dma(kb, p.k_st * 2, k_lane, I0 + n - 1 - rho0, kTgOffK + kslot * kTile);
-      return g_dma(I0 + n, ring);
+    for (int w = 1; w < 4; ++w) {
+      const int blk = J - w;
+      const uint32_t dst = kTgOffK + (uint32_t)(kKRing - w) * kTile;
+      if ((uint32_t)blk < (uint32_t)full) dma16sn(k_rows + blk * k_step, k_lane, dst + wave_kb);
+      else clamped_dma(k_rows, k_step, blk, dst);
+    }
+    zone_at(max(I - 1, 0));
+    bool prev = g_dma(I - 1, g_at - (uint64_t)g_step, kGRing - 1);
+    auto fetch = [&](uint32_t ring, uint32_t kslot) __attribute__((always_inline)) {   // what the next row block needs first, four loads per wave
+      if (I < full) dma16sn((const char*)(uintptr_t)q_at, q_lane, ring * kTile + wave_kb);
+      else clamped_dma(q_rows, q_step, I, ring * kTile);
+      if ((uint32_t)J < (uint32_t)full) dma16sn((const char*)(uintptr_t)k_at, k_lane, kTgOffK + kslot * kTile + wave_kb);
+      else clamped_dma(k_rows, k_step, J, kTgOffK + kslot * kTile);
+      if ((I & 3) == 0) zone_at(I);
+      const bool there = g_dma(I, g_at, ring);
+      ++I, ++J;
+      q_at += (uint64_t)q_step, k_at += (uint64_t)k_step, g_at += (uint64_t)g_step;
+      return there;
     };
-    bool cur = fetch(0, 0, 0), next = fetch(1, 1, 1);
+    bool cur = fetch(0, 0), next = fetch(1, 1);
     int kread = wave == 0 ? 0 : kKRing - wave, kfill = 2;   // ring slots of k: this wave's rows, and where the next ones go
     auto turn = [&](auto slot_tag, int n) __attribute__((always_inline)) {
       constexpr int RING = decltype(slot_tag)::value, PREV = (RING + kGRing - 1) % kGRing;
       wait_vmcnt<4>();   // this row block's loads have landed, those of the next one may still fly
       __syncthreads();
-      const bool after = fetch(n + 2, (RING + 2) % kGRing, (uint32_t)kfill);
-      if (cur && n < I1 - I0) {
+      const bool after = fetch((RING + 2) % kGRing, (uint32_t)kfill);
+      const bool for_k = cur && n < I1 - I0, for_q = (prev || cur) && (n > 0 || I0 == 0);
+      if (for_k || for_q) {   // the operands of both tables' products are requested before the first product waits for one
+        frag gk[2], gq[2], tq[2][2], tk[2][2];
+        const uint32_t kt = kTgOffK + (uint32_t)kread * kTile;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(g_base + gt[0] + RING * kGBlk + 1024 * c));
           const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(g_base + gt[1] + RING * kGBlk + 1024 * c));
-          const frag a = __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          gk[c] = __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
-          for (int d = 0; d < 2; ++d) ek[d] = QT::mma(a, trans(RING * kTile, c, d), ek[d]);
+          for (int d = 0; d < 2; ++d) tq[c][d] = trans(RING * kTile, c, d);
         }
-      }
-      if ((prev || cur) && (n > 0 || I0 == 0)) {
-        const uint32_t kt = kTgOffK + (uint32_t)kread * kTile;
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           s16x8 a;
@@ -883,8 +908,22 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
             if (RING == 0) at -= 4 * g + li + o0 >= 32 ? kGRing * kGBlk : 0;   // block I lies in slot 0, block I - 1 in the last one
             a[e] = *(LDS_AS const short*)(uintptr_t)at;
           }
+          gq[c] = __builtin_bit_cast(frag, a);
 #pragma unroll
-          for (int d = 0; d < 2; ++d) eq[d] = QT::mma(__builtin_bit_cast(frag, a), trans(kt, c, d), eq[d]);
+          for (int d = 0; d < 2; ++d) tk[c][d] = trans(kt, c, d);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (for_k) {
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) ek[d] = QT::mma(gk[c], tq[c][d], ek[d]);
+        }
+        if (for_q) {
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) eq[d] = QT::mma(gq[c], tk[c][d], eq[d]);
         }
       }
       prev = cur;
@@ -921,34 +960,35 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
 
 // Row delta of a table's gradient: the sum of dE over the parts and over the relative positions inside the radius with
 // delta(r) = delta (a range, since delta is monotone), the saturated rows' sums at its ends, times sm_scale.  A workgroup takes
-// four rows of one head and table (blockIdx.z), a wave each, and finds their ranges in one pass over the delta table; four
-// positions and four parts are asked for together (one row after the other it waited for memory a dozen times: 30 us).
+// four rows of one head and table (blockIdx.z), a wave each, which finds its range by a search 64 entries wide: two dependent
+// loads for a radius of 512.  Four positions and four parts are asked for together (one row after the other it waited for
+// memory a dozen times: 30 us).
 constexpr int kFoldRows = 4;
+
+// how many of the n entries of the monotone table are below v
+__device__ __forceinline__ int entries_below(const int16_t* lut, int n, int v, int lane) {
+  int lo = 0;
+  while (n > 64) {
+    const int step = (n + 63) / 64;
+    const int c = __popcll(__ballot(lane * step < n && lut[lo + min(lane * step, n - 1)] < v));   // probes below v: a prefix of them
+    if (c == 0) return lo;
+    lo += (c - 1) * step + 1;
+    n = min(step - 1, n - (c - 1) * step - 1);
+  }
+  return lo + __popcll(__ballot(lane < n && lut[lo + min(lane, max(n - 1, 0))] < v));
+}
 
 template <class QT>
 __global__ __launch_bounds__(256) void fdb_table_fold_kernel(const FdbBwdRingParams p) {
-  __shared__ int first[kFoldRows], last[kFoldRows];
   const int tid = threadIdx.x, d = tid & 63, h = blockIdx.y, table = blockIdx.z, row0 = blockIdx.x * kFoldRows;
-  if (tid < kFoldRows) {
-    first[tid] = p.R + 1;   // no position maps here
-    last[tid] = -p.R - 1;
-  }
-  __syncthreads();
-  for (int x = tid; x <= 2 * p.R; x += 256) {
-    const int mine = p.lut[x], before = x > 0 ? p.lut[x - 1] : -1, after = x < 2 * p.R ? p.lut[x + 1] : -1, u = mine - row0;
-    if (u >= 0 && u < kFoldRows) {
-      if (before != mine) first[u] = x - p.R;
-      if (after != mine) last[u] = x - p.R;
-    }
-  }
-  __syncthreads();
+  const int u = __builtin_amdgcn_readfirstlane(tid >> 6), row = row0 + u, entries = 2 * p.R + 1;
+  if (row >= 2 * p.S) return;
+  const int from = entries_below(p.lut, entries, row, d), to = entries_below(p.lut, entries, row + 1, d);   // the row's entries of the table
   const int r_min = 32 * p.rho_min, r_max = 32 * (p.rho_min + 4 * p.tg_groups) - 1;
   const int64_t part_len = (int64_t)p.H * (4 * p.tg_groups) * 4096;
   const float* e = p.e_parts + (int64_t)h * (4 * p.tg_groups) * 4096 + table * 2048 + d;
-  const int u = tid >> 6;
-  if (row0 + u >= 2 * p.S) return;
-  const bool low = first[u] == -p.R, high = last[u] == p.R;
-  const int r0 = max(max(first[u], -p.R + 1), r_min), r1 = min(min(last[u], p.R - 1), r_max);
+  const bool low = from == 0 && to > 0, high = to == entries && from < to;
+  const int r0 = max(max(from - p.R, -p.R + 1), r_min), r1 = min(min(to - 1 - p.R, p.R - 1), r_max);
   float sum = 0.f;
   for (int r = r0; r <= r1; r += 4) {
     const float* er[4];
@@ -972,7 +1012,7 @@ __global__ __launch_bounds__(256) void fdb_table_fold_kernel(const FdbBwdRingPar
     for (int part = 0; part < p.tg_parts; ++part) sum += f[(int64_t)part * p.H * 256] + (low && high ? f[(int64_t)part * p.H * 256 + 64] : 0.f);
   }
   typedef typename QT::scratch_t T;
-  T* out = (T*)(table == 0 ? p.dpk : p.dpq) + (int64_t)h * p.dp_sh + (int64_t)(row0 + u) * p.dp_sr + d;
+  T* out = (T*)(table == 0 ? p.dpk : p.dpq) + (int64_t)h * p.dp_sh + (int64_t)row * p.dp_sr + d;
   *out = (T)(sum * p.sm_scale);
 }
 
@@ -994,9 +1034,9 @@ int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
   if (e == hipSuccess) e = fdb_set_lds_once((const void*)tg, kTgLds, set2);
   if (e == hipSuccess) e = fdb_set_lds_once((const void*)both, kLds, set3);
   if (e != hipSuccess) return (int)e;
-  const unsigned tiles = (unsigned)((p.L + FDB_BM - 1) / FDB_BM), grid = tiles * (unsigned)p.H * (unsigned)p.B;
+  const unsigned grid = (unsigned)p.tiles * (unsigned)p.H * (unsigned)p.B;
   if (grid <= kMostTogether) {
-    hipLaunchKernelGGL(fdb_row_stats_kernel<QT>, dim3((unsigned)((p.L + 31) / 32), (unsigned)p.H, (unsigned)p.B), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(fdb_row_stats_kernel<QT>, dim3((unsigned)p.tiles, (unsigned)p.H, (unsigned)p.B), dim3(256), 0, stream, p);
     hipLaunchKernelGGL(both, dim3(2 * grid), dim3(kThreads), kLds, stream, p);
   } else {
     hipLaunchKernelGGL(dq, dim3(grid), dim3(kThreads), kLds, stream, p);

@@ -255,7 +255,7 @@ __device__ __forceinline__ float scratch_add_lo<float>(float acc, uint32_t) { re
 template <>
 __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { return acc; }
 
-// Linear workgroup id -> (query-tile index within the launch, head).  The hardware deals
+// Linear workgroup id -> (batch row, query tile, head); packed sequences: (-, work-list entry, head).  The hardware deals
 // workgroups to the 8 XCDs round-robin by linear id, and each XCD has its own L2.  In the fixed
 // layout the (sequence, head) groups are dealt to XCDs whole, group g to XCD g % 8: all query tiles of a group then stream the
 // same K and V through one L2.  (Groups beyond the last multiple of 8 are spread over the XCDs.)
@@ -263,17 +263,17 @@ __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { re
 // with the most key tiles start first and the launch ends on the short ones: kEdgesFirst for the far
 // tiles (a query tile at either end of the sequence has the most), kMiddleFirst for the near tiles, kLastFirst for
 // the far tiles of a causal call (a query tile sees the keys before it: the last one has the most).  Only as many groups are
-// taken together as leave their K and V in an XCD's 4 MB of L2: 96 query tiles of 16-bit head_dim 64 are 3 MB.
+// taken together as leave their K and V in an XCD's 4 MB of L2: 96 query tiles of 16-bit head_dim 64 are 3 MB.  The host passes
+// that number (fdb_groups_together): each division here costs every workgroup some 40 instructions before its first load.
 enum { kNatural = 0, kEdgesFirst = 1, kMiddleFirst = 2, kLastFirst = 3 };
-__device__ __forceinline__ void block_map(int n, int nx, int heads, int tiles_per_seq, bool fixed, int order, int& xq,
+__device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles_per_seq, int most, bool fixed, int order, int& b, int& t,
                                           int& h) {
   if (fixed) {
-    const int groups = (nx / tiles_per_seq) * heads;
-    const int most = 8 * max(1, 96 / tiles_per_seq);   // groups taken together
+    const int groups = batch * heads;
     const int first = n / (most * tiles_per_seq) * most;
     const int here = min(groups - first, most), m = n - first * tiles_per_seq;
-    const int i = m % here;
-    int t = m / here;
+    t = m / here;
+    const int i = m - t * here;
     const int grp = first + (i < (here & ~7) ? (n & 7) | (i & ~7) : i);
     if (order == kLastFirst) {
       t = tiles_per_seq - 1 - t;
@@ -281,14 +281,20 @@ __device__ __forceinline__ void block_map(int n, int nx, int heads, int tiles_pe
       if (order == kMiddleFirst) t = tiles_per_seq - 1 - t;
       t = (t & 1) ? tiles_per_seq - 1 - (t >> 1) : (t >> 1);  // 0, T-1, 1, T-2, ...
     }
-    xq = (grp / heads) * tiles_per_seq + t;
-    h = grp % heads;
+    b = grp / heads;
+    h = grp - b * heads;
   } else {
     // packed sequences: the work-list holds the tiles longest sequence first; all heads of a tile are
     // dealt before the next tile, so the whole launch runs from long workgroups to short ones
-    xq = n / heads;
-    h = n % heads;
+    b = 0;
+    t = n / heads;
+    h = n - t * heads;
   }
+  // the divisions run on vector registers: taken back, or every address that depends on these stays there too (the e4m3 near kernel
+  // spills 52 registers then)
+  b = __builtin_amdgcn_readfirstlane(b);
+  t = __builtin_amdgcn_readfirstlane(t);
+  h = __builtin_amdgcn_readfirstlane(h);
 }
 
 // 16 bytes per lane from global memory straight into LDS: lane l's data lands at lds_base + 16*l

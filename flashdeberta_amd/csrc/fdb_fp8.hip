@@ -86,26 +86,25 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  int xq, h;
-  block_map((int)blockIdx.x, p.grid_x, p.H, p.tiles_per_seq, p.cu == nullptr, p.causal ? kLastFirst : kEdgesFirst, xq, h);
+  int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
+  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr, p.causal ? kLastFirst : kEdgesFirst, b, tile, h);
 
-  int b, m0, tok0, Lb;
+  int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
-    if (xq >= p.wl[0]) return;
-    b = p.wl[2 + 2 * xq];
-    m0 = p.wl[3 + 2 * xq];
+    if (tile >= p.wl[0]) return;
+    b = p.wl[2 + 2 * tile];
+    m0 = p.wl[3 + 2 * tile];
     tok0 = p.cu[b];
     Lb = p.cu[b + 1] - tok0;
     qo = ko = vo = oo = 0;
   } else {
-    b = xq / p.tiles_per_seq;
-    m0 = (xq % p.tiles_per_seq) * FDB_BM;
+    m0 = tile * FDB_BM;
     tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
     const int sl = p.seq_len ? p.seq_len[b] : p.L;
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
-      fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, xq % p.tiles_per_seq, p.L, tok0, Lb,
+      fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,
                            sl < 0 ? VT::NAN_WORD : 0u, tid);
     if (m0 >= Lb) return;
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; oo = b * p.o_sb;
@@ -413,26 +412,25 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  int xq, h;
-  block_map((int)blockIdx.x, p.grid_x, p.H, p.tiles_per_seq, p.cu == nullptr, kMiddleFirst, xq, h);
+  int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
+  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr, kMiddleFirst, b, tile, h);
 
-  int b, m0, tok0, Lb;
+  int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
-    if (xq >= p.wl[0]) return;
-    b = p.wl[2 + 2 * xq];
-    m0 = p.wl[3 + 2 * xq];
+    if (tile >= p.wl[0]) return;
+    b = p.wl[2 + 2 * tile];
+    m0 = p.wl[3 + 2 * tile];
     tok0 = p.cu[b];
     Lb = p.cu[b + 1] - tok0;
     qo = ko = vo = oo = 0;
   } else {
-    b = xq / p.tiles_per_seq;
-    m0 = (xq % p.tiles_per_seq) * FDB_BM;
+    m0 = tile * FDB_BM;
     tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
     const int sl = p.seq_len ? p.seq_len[b] : p.L;
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
-      fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, xq % p.tiles_per_seq, p.L, tok0, Lb,
+      fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,
                            sl < 0 ? VT::NAN_WORD : 0u, tid);
     if (m0 >= Lb) return;
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; oo = b * p.o_sb;

@@ -7,6 +7,9 @@
 #define FDB_BM 128
 #define FDB_BN 64
 
+// (sequence, head) groups whose query tiles are dealt together, see block_map
+inline int32_t fdb_groups_together(int32_t tiles_per_seq) { return 8 * (tiles_per_seq < 96 ? 96 / tiles_per_seq : 1); }
+
 struct FdbKParams {
   const char* q;
   const char* k;
@@ -31,7 +34,7 @@ struct FdbKParams {
   int64_t pk_sh, pk_sr;
   int64_t pq_sh, pq_sr;
   int32_t B, H, L, tiles_per_seq;
-  int32_t grid_x;   // query tiles in the launch (the grid is grid_x * H workgroups)
+  int32_t groups_together;  // fdb_groups_together(tiles_per_seq)
   int32_t R;        // LUT radius
   int32_t far_done;  // near launches: the far tiles' partial results (far_parts of them) are to be merged
   int32_t far_parts; // workgroups per query tile of the far-only launch, each with its share of the far tiles and a
@@ -129,6 +132,7 @@ struct FdbBwdRingParams {
   int64_t pk_sh, pk_sr, pq_sh, pq_sr, dp_sh, dp_sr;
   int32_t B, H, L, S, R, causal;
   int32_t stat_len, g_rows, g_slots;
+  int32_t tiles, groups_together;  // query tiles of a sequence; fdb_groups_together(tiles)
   int32_t rho_min, tg_groups, tg_parts, tg_chunks, tg_len;  // blocks of 32 relative positions in groups of four; shares of the tokens; chunks of
                                                             // tg_len row blocks per batch row
   int32_t has_far;
