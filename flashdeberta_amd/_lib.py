@@ -107,7 +107,7 @@ def _load():
     lib.fdb_linear.restype = ctypes.c_int
     lib.fdb_linear.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i32, vp]
     lib.fdb_column_sums_workspace_bytes.restype = i64
-    lib.fdb_column_sums_workspace_bytes.argtypes = [i64, i64]
+    lib.fdb_column_sums_workspace_bytes.argtypes = [i64, i64, i64]
     lib.fdb_column_sums.restype = ctypes.c_int
     lib.fdb_column_sums.argtypes = [vp, i64, i64, vp, i64, i64, vp, vp, i32, vp]
     lib.fdb_mask_bounds.restype = ctypes.c_int

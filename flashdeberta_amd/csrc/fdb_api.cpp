@@ -684,9 +684,9 @@ int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_t
   return fdb_launch_worklist(cu_seqlens, batch, worklist, fdb_worklist_max_tiles(total_tokens, batch), stream);
 }
 
-int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols) {
+int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols, int64_t y_rows) {
   if (x_rows < 1 || x_cols < 1) return 0;
-  return (fdb_column_sum_parts(x_rows) + 1) * x_cols * 4;
+  return (int64_t)fdb_column_sum_parts(y_rows > x_rows ? y_rows : x_rows) * x_cols * 4;
 }
 
 int fdb_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, void* workspace,

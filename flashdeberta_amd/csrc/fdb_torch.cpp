@@ -780,7 +780,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     }
     if (ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7)) {
       db = at::empty({3 * W}, hidden.options());
-      const Tensor ws = at::empty({fdb_column_sums_workspace_bytes(n, 3 * W)}, hidden.options().dtype(at::kByte));
+      const Tensor ws = at::empty({fdb_column_sums_workspace_bytes(n, 3 * W, rows)}, hidden.options().dtype(at::kByte));
       check(fdb_column_sums(dqkv.data_ptr(), n, 3 * W, dpos.data_ptr(), rows, 2 * W, db.data_ptr(), ws.data_ptr(), fdb_dtype_of(type), stream_of(hidden)),
             "fdb_column_sums");
     }

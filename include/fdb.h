@@ -350,7 +350,7 @@ int32_t fdb_tile_rows(void);
  * for its y_cols <= x_cols columns (y may be NULL): the bias gradients of projections that share weights.  Columns a multiple of
  * 8, x and y aligned to 16 bytes, workspace as asked for.
  */
-int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols);
+int64_t fdb_column_sums_workspace_bytes(int64_t x_rows, int64_t x_cols, int64_t y_rows);  /* y_rows 0 without y */
 int fdb_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, void* workspace,
                     int32_t dtype, void* stream);
 

@@ -64,12 +64,12 @@ def test_table_backward_matches_oracle(case, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols,rows2,cols2", [(1, 8, 0, 0), (63, 512, 5, 8), (64, 520, 64, 512), (65, 2304, 512, 1536), (4096, 768, 0, 0)])
+@pytest.mark.parametrize("rows,cols,rows2,cols2", [(1, 8, 0, 0), (63, 512, 5, 8), (64, 520, 64, 512), (3, 16, 200, 8), (65, 2304, 512, 1536), (4096, 768, 0, 0)])
 def test_column_sums(rows, cols, rows2, cols2):
     x = torch.randn(rows, cols, device="cuda").to(torch.bfloat16)
     y = torch.randn(rows2, cols2, device="cuda").to(torch.bfloat16) if rows2 else None
     out = torch.empty(cols, device="cuda", dtype=torch.bfloat16)
-    ws = torch.empty(_lib.lib.fdb_column_sums_workspace_bytes(rows, cols), dtype=torch.uint8, device="cuda")
+    ws = torch.empty(_lib.lib.fdb_column_sums_workspace_bytes(rows, cols, rows2), dtype=torch.uint8, device="cuda")
     assert _lib.lib.fdb_column_sums(x.data_ptr(), rows, cols, None if y is None else y.data_ptr(), rows2, cols2, out.data_ptr(), ws.data_ptr(), 1,
                                     torch.cuda.current_stream().cuda_stream) == 0
     ref = x.float().sum(0)
