@@ -161,3 +161,18 @@ def test_threads_share_the_plans():
     for k in range(4):
         for x, g in zip(xs[k % 2::2], got[k]):
             assert all(torch.equal(a, b) for a, b in zip(g, gradients(x)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,heads,dim", [(1, 1, 64), (1, 40, 64), (257, 3, 64), (511, 12, 32), (300, 17, 128), (16391, 12, 64), (40, 400, 64)])
+def test_quantiser_walks_every_row(tokens, heads, dim):
+    """Heads fewer and more than a workgroup has rows, tokens around a thread's eight; bytes and scales are whole, hence exact."""
+    from flashdeberta_amd import quantize_e4m3_per_head_pair
+
+    g = torch.Generator(device="cuda").manual_seed(tokens + heads)
+    xs = [torch.randn(tokens, heads, dim + 8, device="cuda", generator=g).to(torch.bfloat16)[..., :dim] for _ in range(2)]
+    y0, s0, y1, s1 = quantize_e4m3_per_head_pair(*xs)
+    for x, y, s in ((xs[0], y0, s0), (xs[1], y1, s1)):
+        scale = x.float().abs().amax(dim=(0, 2)).clamp_min(1e-12) / torch.tensor(448.0, device="cuda")   # a divisor on the GPU: a Python number would become a factor 1 / 448
+        assert torch.equal(s, scale)
+        assert torch.equal(y.view(torch.uint8), (x.float() / scale[:, None]).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8))
