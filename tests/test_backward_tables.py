@@ -112,3 +112,35 @@ def test_layer_node_matches_separate_projections(B, L, padded):
     att.value_proj.weight.requires_grad_(False)
     some = torch.autograd.grad(att(x, mask, rel_embeddings=rel)[0], [x, att.query_proj.bias], dout)
     assert torch.equal(some[0], one[2]) and some[1].shape == (192,)
+
+
+@pytest.mark.gpu
+def test_node_replays_from_a_graph_and_through_saved_tensor_hooks():
+    """Forward and backward of the operator in a captured graph, replayed with eager work between, and with the saved tensors taken to
+    the host and back: the eager call's bits."""
+    B, H, L, D = 1, 2, 700, 64
+    leaves = [torch.randn(*s, device="cuda").to(torch.bfloat16).requires_grad_() for s in ((B, H, L, D),) * 3 + ((H, 512, D),) * 2]
+    dout = torch.randn(B, H, L, D, device="cuda").to(torch.bfloat16)
+
+    def step():
+        out = ops.flash_attention_with_disentangled(*leaves, position_buckets=256, max_relative_distance=512)
+        return (out.detach(), *torch.autograd.grad(out, leaves, dout))
+
+    ref = step()
+    with torch.autograd.graph.save_on_cpu():
+        assert all(torch.equal(a, b) for a, b in zip(step(), ref))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for scale in (1.0, 0.5, 2.0):
+        with torch.no_grad():
+            leaves[0].mul_(scale)
+        ref = step()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, ref))
