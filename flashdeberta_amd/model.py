@@ -63,6 +63,11 @@ def _hooked(module):
     return module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
 
 
+def _passes_through(dropout):
+    """Whether leaving a dropout's call out changes nothing: a plain one that is off or drops nothing."""
+    return type(dropout) is torch.nn.Dropout and not (dropout.training and dropout.p > 0.0)
+
+
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     """Same parameters as the eager module (query_proj, key_proj, value_proj[, pos_key_proj,
     pos_query_proj]), so `load_state_dict(eager.state_dict())` works (reference tests/attention.py:60).
@@ -253,7 +258,7 @@ class FlashDebertaV2Layer(DebertaV2Layer):
     """transformers' encoder layer whose inference in a 16-bit type is one native call (native.encoder_layer): the same
     projections, attention, GELU and post-norms, with the same bits, without a module call per step.
     Anything else -- training, recording, autocast, hooks on any part, a part of another class (adapters, quantised
-    projections, another activation) -- takes transformers' own forward.  Instances are made by `patch_model`."""
+    projections, another activation), a dropout that is on -- takes transformers' own forward.  Instances are made by `patch_model`."""
 
     def _native_args(self, hidden_states, attention_mask, rel_embeddings):
         if self.training or torch.is_grad_enabled() or hidden_states.dtype not in (torch.bfloat16, torch.float16) or not hidden_states.is_cuda \
@@ -269,7 +274,8 @@ class FlashDebertaV2Layer(DebertaV2Layer):
         act = intermediate._modules.get("intermediate_act_fn")
         linears = att_out._modules["dense"], intermediate._modules["dense"], output._modules["dense"]
         norms = att_out._modules["LayerNorm"], output._modules["LayerNorm"]
-        if getattr(act, "act", None) is not F.gelu:
+        dropouts = att_out._modules["dropout"], output._modules["dropout"]
+        if getattr(act, "act", None) is not F.gelu or not all(_passes_through(m) for m in dropouts):
             return None
         shape = hidden_states.shape[-1:]
         for m in linears:
@@ -279,7 +285,7 @@ class FlashDebertaV2Layer(DebertaV2Layer):
             if type(m) is not torch.nn.LayerNorm or m.normalized_shape != shape or m.bias is None or m.weight is None \
                     or m.weight.dtype != hidden_states.dtype:
                 return None
-        if any(_hooked(m) for m in (attention, intermediate, output, att, att_out, act, *linears, *norms,
+        if any(_hooked(m) for m in (attention, intermediate, output, att, att_out, act, *linears, *norms, *dropouts,
                                       *att._modules.values())):
             return None
         args = att._native_args(attention_mask, rel_embeddings, False)

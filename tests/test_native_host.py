@@ -1,5 +1,7 @@
 """The native host path (csrc/fdb_torch.cpp) and the linear kernels (csrc/fdb_linear.hip): mask bounds against
 padding.seq_bounds, products against fp32 torch, the one-call encoder layer against the module-by-module one."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -87,6 +89,52 @@ def test_encoder_layer_matches_the_module_by_module_forward(B, L):
         layer(x, mask, rel_embeddings=rel)
         handle.remove()
         assert calls
+
+
+def _encoder_layer(dropout=0.1):
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
+
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=128, num_hidden_layers=1, num_attention_heads=2, intermediate_size=256, relative_attention=True,
+                          pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True, norm_rel_ebd="layer_norm",
+                          position_biased_input=False, hidden_dropout_prob=dropout)
+    return FlashDebertaV2Model(cfg).eval().to(torch.bfloat16).encoder.layer[0]
+
+
+def _takes_one_call(layer):
+    """Whether the layer's inference on GPU activations would be the one native call (the decision itself needs no GPU)."""
+    hidden = SimpleNamespace(dtype=torch.bfloat16, is_cuda=True, shape=torch.Size((1, 8, 128)))
+    with torch.no_grad():
+        return layer._native_args(hidden, None, torch.zeros(64, 128, dtype=torch.bfloat16)) is not None
+
+
+@pytest.mark.parametrize("name", ["attention.output", "output"])
+def test_one_call_layer_leaves_no_dropout_out(name):
+    """Dropout kept on in an eval model, with a hook, or replaced by another module: transformers' own forward calls it."""
+    assert _takes_one_call(_encoder_layer())
+    layer = _encoder_layer()
+    part = layer.get_submodule(name)
+    part.dropout.train()
+    assert not _takes_one_call(layer)
+    part.dropout.p = 0.0   # on, and dropping nothing
+    assert _takes_one_call(layer)
+    for register in ("register_forward_hook", "register_forward_pre_hook"):
+        handle = getattr(part.dropout, register)(lambda *a: None)
+        assert not _takes_one_call(layer)
+        handle.remove()
+    part.dropout = torch.nn.Linear(128, 128)
+    assert not _takes_one_call(layer)
+
+
+@pytest.mark.gpu
+def test_dropout_kept_on_in_an_eval_model():
+    layer = _encoder_layer(0.5).cuda()
+    x, rel = torch.randn(2, 40, 128, device="cuda").to(torch.bfloat16), torch.randn(64, 128, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        first = layer(x, None, rel_embeddings=rel)[0]
+        assert torch.equal(first, layer(x, None, rel_embeddings=rel)[0])
+        layer.output.dropout.train()
+        sampled = [layer(x, None, rel_embeddings=rel)[0] for _ in range(2)]
+    assert not torch.equal(*sampled)
 
 
 def _attention(**kw):
