@@ -908,6 +908,44 @@ PyObject* py_register_lut_source(PyObject*, PyObject* fn) {
   Py_RETURN_NONE;
 }
 
+// ---- modules whose calls a fused path takes the place of --------------------------------------------------------------
+// untouched(modules, kinds) -> whether every module does what its kind (class, the class's own forward) does, unseen: exactly of
+// that class, which nobody has given another forward, no hooks on it, no `forward` of its own, not compiled by itself.  A layer
+// asks this of some twenty modules per call; in Python the look-ups took longer than the launch of a short product.
+PyObject* py_untouched(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  static PyObject* const forward = PyUnicode_InternFromString("forward");
+  static PyObject* const compiled = PyUnicode_InternFromString("_compiled_call_impl");
+  static PyObject* const hooks[] = {PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
+                                    PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
+  if (n != 2 || !PyTuple_Check(x[0]) || !PyTuple_Check(x[1]) || PyTuple_GET_SIZE(x[0]) != PyTuple_GET_SIZE(x[1])) {
+    PyErr_SetString(PyExc_TypeError, "untouched(modules, kinds) takes two tuples of one length");
+    return nullptr;
+  }
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(x[0]); ++i) {
+    PyObject *m = PyTuple_GET_ITEM(x[0], i), *kind = PyTuple_GET_ITEM(x[1], i);
+    if (!PyTuple_Check(kind) || PyTuple_GET_SIZE(kind) != 2) {
+      PyErr_SetString(PyExc_TypeError, "untouched: a kind is a pair (class, its forward)");
+      return nullptr;
+    }
+    if ((PyObject*)Py_TYPE(m) != PyTuple_GET_ITEM(kind, 0)) Py_RETURN_FALSE;
+    PyObject* f = PyObject_GetAttr((PyObject*)Py_TYPE(m), forward);
+    if (!f) return nullptr;
+    Py_DECREF(f);   // the class keeps it
+    if (f != PyTuple_GET_ITEM(kind, 1)) Py_RETURN_FALSE;
+    PyObject* d = PyObject_GenericGetDict(m, nullptr);
+    if (!d) return nullptr;
+    bool plain = !PyDict_GetItemWithError(d, forward) && !PyDict_GetItemWithError(d, compiled);
+    for (PyObject* name : hooks) {
+      PyObject* h = PyDict_GetItemWithError(d, name);
+      plain = plain && (!h || PyObject_IsTrue(h) == 0);
+    }
+    Py_DECREF(d);
+    if (PyErr_Occurred()) return nullptr;
+    if (!plain) Py_RETURN_FALSE;
+  }
+  Py_RETURN_TRUE;
+}
+
 // ---- Memo ---------------------------------------------------------------------------------------------------------
 // One remembered value, valid while the tensors it was computed from are the same objects, have not been written in place
 // (version counter), still sit in the same storage with the same dtype on the same device (`p.data = x` and `module.to(dtype)`
@@ -1030,6 +1068,7 @@ PyMethodDef module_methods[] = {
     {"encoder_layer", (PyCFunction)(void*)py_encoder_layer, METH_FASTCALL, nullptr},
     {"quantize_e4m3", (PyCFunction)(void*)py_quantize, METH_FASTCALL, nullptr},
     {"mask_bounds", (PyCFunction)(void*)py_mask_bounds, METH_FASTCALL, nullptr},
+    {"untouched", (PyCFunction)(void*)py_untouched, METH_FASTCALL, nullptr},
     {"register_lut_source", py_register_lut_source, METH_O, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -14,6 +14,7 @@ import math
 import torch
 import torch.nn.functional as F
 from torch.nn.modules import module as nn_module
+from transformers.activations import GELUActivation
 from transformers.models.deberta_v2.modeling_deberta_v2 import (
     DebertaV2Attention,
     DebertaV2Config,
@@ -59,13 +60,19 @@ def _weight_and_bias(module):
     return module.weight, module.bias
 
 
-def _hooked(module):
-    return module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+def _kind(cls):
+    """A class as native.untouched asks for it: with what it computes as long as nobody gives it another forward."""
+    return cls, cls.forward
 
 
-def _passes_through(dropout):
-    """Whether leaving a dropout's call out changes nothing: a plain one that is off or drops nothing."""
-    return type(dropout) is torch.nn.Dropout and not (dropout.training and dropout.p > 0.0)
+_LINEAR, _DROPOUT = _kind(torch.nn.Linear), _kind(torch.nn.Dropout)
+
+
+def _stands_in(modules, kinds):
+    """Whether computing what these kinds of modules do without calling them is unseen by the program: native.untouched, and
+    no hooks on all modules."""
+    return native.untouched(modules, kinds) and not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
+                                                     or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
 
 
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
@@ -78,7 +85,8 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     Outside training the three input projections run as one GEMM over the concatenated weights
     (a copy kept per module, rebuilt when a parameter is replaced or written in place), and K_r / Q_r
     are remembered for as long as the relative embeddings handed in are the same tensor (an encoder
-    patched by `patch_model` hands in the same tensor until its embedding table changes)."""
+    patched by `patch_model` hands in the same tensor until its embedding table changes); both only
+    while the projections are plain linear layers that nobody has hooked or given another forward."""
 
     # Projections of a few rows by the library's own kernels, which start sooner than hipBLASLt's but add up in another order;
     # off in a patched encoder, whose twelve layers turn one differing rounding of a 16-bit type into a percent.
@@ -89,8 +97,14 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         self.fp8_qk = bool(getattr(config, "fp8_qk", False)) if fp8_qk is None else bool(fp8_qk)
         self._qkv_memo, self._pos_memo, self._mask_memo, self._pos8_memo = _Memo(), _Memo(), _Memo(), _Memo()
 
+    def _plain_projections(self):
+        """Whether products with the projections' weights are all that the query, key and value projections do."""
+        modules = self._modules
+        return _stands_in((modules["query_proj"], modules["key_proj"], modules["value_proj"]), (_LINEAR, _LINEAR, _LINEAR))
+
     def _fused_qkv(self):
-        """Concatenated [3*H*D, hidden] weight and bias of the query, key and value projections."""
+        """Concatenated [3*H*D, hidden] weight and bias of the query, key and value projections (plain ones), None where only
+        some have a bias."""
         modules = self._modules
         (qw, qb), (kw, kb), (vw, vb) = [_weight_and_bias(modules[n]) for n in ("query_proj", "key_proj", "value_proj")]
         with_bias = qb is not None and kb is not None and vb is not None
@@ -111,14 +125,14 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         H, D = self.num_attention_heads, self.attention_head_size
         # the concatenated weights are a copy made outside autograd: only where nothing is being recorded
         recording = torch.is_grad_enabled() and (hidden_states.requires_grad or self.query_proj.weight.requires_grad)
-        fused = None if (self.training or recording or query_states is not hidden_states) else self._fused_qkv()
+        fused = None if (self.training or recording or query_states is not hidden_states or not self._plain_projections()) else self._fused_qkv()
         if fused is not None:
             qkv = F.linear(hidden_states, fused[0], fused[1]).view(B, L, 3, H, D)
             return qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
         return (self.query_proj(query_states).view(B, L, H, D), self.key_proj(hidden_states).view(B, L, H, D),
                 self.value_proj(hidden_states).view(B, L, H, D))
 
-    def _pos_layers(self, rel_embeddings):
+    def _pos_layers(self, rel_embeddings, plain=False):
         """K_r, Q_r as [H, 2S, D] views of the projected relative embeddings
         (reference model.py:159-177; the slice to 2S rows is transformers modeling_deberta_v2.py:295)."""
         if not self.relative_attention or rel_embeddings is None:
@@ -132,8 +146,11 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             qproj = modules["query_proj" if self.share_att_key else "pos_query_proj"]
         key = None
         recording = torch.is_grad_enabled() and (rel_embeddings.requires_grad or self.query_proj.weight.requires_grad)
-        if not self.training and not recording:  # a remembered K_r / Q_r must not carry an autograd graph
-            key = (rel_embeddings,) + tuple(p for m in (kproj, qproj) if m is not None for p in _weight_and_bias(m) if p is not None)
+        projections = tuple(m for m in (kproj, qproj) if m is not None)
+        # a remembered K_r / Q_r must not carry an autograd graph, and depends on nothing but the embeddings and the weights
+        # (`plain`: the caller knows that about these projections)
+        if not self.training and not recording and (plain or _stands_in(projections, (_LINEAR,) * len(projections))):
+            key = (rel_embeddings,) + tuple(p for m in projections for p in _weight_and_bias(m) if p is not None)
             hit = self._pos_memo.get(key, tuple(self.pos_att_type))
             if hit is not None:
                 return hit
@@ -168,27 +185,26 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     def _native_args(self, attention_mask, rel_embeddings, hidden_requires_grad):
         """What follows the hidden states in a call of native.layer_attention, or None where that path does not serve:
         in training or while anything is recorded (the concatenated weights are a copy made outside autograd), under
-        autocast, with FP8 operands, or with projections that have no weights to concatenate."""
+        autocast, with FP8 operands, or with projections that are more than products with weights to concatenate."""
         if self.training or self.fp8_qk or torch.is_autocast_enabled():
             return None
         if torch.is_grad_enabled() and (hidden_requires_grad or (rel_embeddings is not None and rel_embeddings.requires_grad)
                                         or any(p.requires_grad for p in self.parameters())):
             return None
-        fused = self._fused_qkv()
+        fused = self._fused_qkv() if self._plain_projections() else None
         if fused is None:
             return None
-        pos_key, pos_query = self._pos_layers(rel_embeddings)
+        pos_key, pos_query = self._pos_layers(rel_embeddings, self.share_att_key)
         return (*fused, pos_key, pos_query, self.num_attention_heads, *self._score_settings(pos_key, pos_query), *self._bounds(attention_mask))
 
     def _trains_as_one_node(self):
         """Whether native.layer_node computes what the module does, step by step: plain projections shared with the tables, both
-        position terms, nothing that has to see the projections' own calls (hooks) or cast their operands (autocast)."""
+        position terms, nothing that has to see the projections' own calls (hooks, a forward of their own) or cast their operands
+        (autocast)."""
         if not (self.relative_attention and self.share_att_key and not self.fp8_qk and "c2p" in self.pos_att_type and "p2c" in self.pos_att_type) \
-                or torch.is_autocast_enabled() or torch.compiler.is_compiling() or nn_module._global_forward_hooks \
-                or nn_module._global_forward_pre_hooks or nn_module._global_backward_hooks:
+                or torch.is_autocast_enabled() or torch.compiler.is_compiling():
             return False
-        projections = [self._modules[n] for n in ("query_proj", "key_proj", "value_proj")]
-        return all(type(m) is torch.nn.Linear for m in projections) and not any(_hooked(m) for m in projections)
+        return self._plain_projections()
 
     def forward(self, hidden_states, attention_mask, output_attentions=False, query_states=None,
                 relative_pos=None, rel_embeddings=None):
@@ -254,39 +270,41 @@ DEBERTA_SELF_ATTENTION_CLASSES = {
 }
 
 
+# the parts of a layer that its one native call takes the place of, in the order FlashDebertaV2Layer._native_args names them
+_LAYER_PARTS = (*(_kind(c) for c in (DebertaV2Attention, DebertaV2Intermediate, DebertaV2Output, FlashDisentangledSelfAttention, DebertaV2SelfOutput,
+                                     GELUActivation)), *(_LINEAR,) * 3, *(_kind(torch.nn.LayerNorm),) * 2, *(_DROPOUT,) * 2)
+
+
 class FlashDebertaV2Layer(DebertaV2Layer):
     """transformers' encoder layer whose inference in a 16-bit type is one native call (native.encoder_layer): the same
     projections, attention, GELU and post-norms, with the same bits, without a module call per step.
-    Anything else -- training, recording, autocast, hooks on any part, a part of another class (adapters, quantised
-    projections, another activation), a dropout that is on -- takes transformers' own forward.  Instances are made by `patch_model`."""
+    Anything else -- training, recording, autocast, hooks on any part, a part with a forward of its own or of another class
+    (adapters, quantised projections, another activation), a dropout that is on -- takes transformers' own forward.  Instances are
+    made by `patch_model`."""
 
     def _native_args(self, hidden_states, attention_mask, rel_embeddings):
         if self.training or torch.is_grad_enabled() or hidden_states.dtype not in (torch.bfloat16, torch.float16) or not hidden_states.is_cuda \
-                or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks or torch.compiler.is_compiling():
+                or torch.compiler.is_compiling():
             return None
         own = self._modules
         attention, intermediate, output = own["attention"], own["intermediate"], own["output"]
         if type(attention) is not DebertaV2Attention or type(intermediate) is not DebertaV2Intermediate or type(output) is not DebertaV2Output:
             return None
         att, att_out = attention._modules["self"], attention._modules["output"]
-        if type(att) is not FlashDisentangledSelfAttention or type(att_out) is not DebertaV2SelfOutput:
+        if type(att_out) is not DebertaV2SelfOutput:
             return None
         act = intermediate._modules.get("intermediate_act_fn")
         linears = att_out._modules["dense"], intermediate._modules["dense"], output._modules["dense"]
         norms = att_out._modules["LayerNorm"], output._modules["LayerNorm"]
         dropouts = att_out._modules["dropout"], output._modules["dropout"]
-        if getattr(act, "act", None) is not F.gelu or not all(_passes_through(m) for m in dropouts):
+        if not _stands_in((attention, intermediate, output, att, att_out, act, *linears, *norms, *dropouts), _LAYER_PARTS):
             return None
-        shape = hidden_states.shape[-1:]
-        for m in linears:
-            if type(m) is not torch.nn.Linear or m.weight.dtype != hidden_states.dtype:
-                return None
-        for m in norms:
-            if type(m) is not torch.nn.LayerNorm or m.normalized_shape != shape or m.bias is None or m.weight is None \
-                    or m.weight.dtype != hidden_states.dtype:
-                return None
-        if any(_hooked(m) for m in (attention, intermediate, output, att, att_out, act, *linears, *norms, *dropouts,
-                                      *att._modules.values())):
+        if act.act is not F.gelu or any(m.training and m.p > 0.0 for m in dropouts):
+            return None
+        shape, dtype = hidden_states.shape[-1:], hidden_states.dtype
+        if any(m.weight.dtype != dtype for m in linears):
+            return None
+        if any(m.normalized_shape != shape or m.bias is None or m.weight is None or m.weight.dtype != dtype for m in norms):
             return None
         args = att._native_args(attention_mask, rel_embeddings, False)
         if args is None:

@@ -125,6 +125,67 @@ def test_one_call_layer_leaves_no_dropout_out(name):
     assert not _takes_one_call(layer)
 
 
+def _changes(part):
+    """Ways in which a program changes what calling a module does, each with its undoing."""
+    handles = [part.register_forward_hook, part.register_forward_pre_hook, part.register_full_backward_hook]
+    for register in handles:
+        handle = register(lambda *a: None)
+        yield
+        handle.remove()
+    part.forward = part.forward
+    yield
+    del part.forward
+    cls, old = type(part), type(part).forward
+    cls.forward = lambda self, *a, **k: old(self, *a, **k)
+    try:
+        yield
+    finally:
+        cls.forward = old
+    part.__class__ = type("Other", (cls,), {})
+    yield
+    part.__class__ = cls
+
+
+PARTS = ["attention", "attention.self", "attention.self.query_proj", "attention.self.key_proj", "attention.self.value_proj", "attention.output",
+         "attention.output.dense", "attention.output.dropout", "attention.output.LayerNorm", "intermediate", "intermediate.dense",
+         "intermediate.intermediate_act_fn", "output", "output.dense", "output.dropout", "output.LayerNorm"]
+
+
+@pytest.mark.parametrize("name", PARTS)
+def test_one_call_layer_leaves_changed_parts_to_their_own_call(name):
+    layer = _encoder_layer()
+    for _ in _changes(layer.get_submodule(name)):
+        assert not _takes_one_call(layer)
+    assert _takes_one_call(layer)
+
+
+@pytest.mark.parametrize("name", ["query_proj", "key_proj", "value_proj"])
+def test_changed_projections_are_called(name):
+    """The attention's own ways round its projections' calls: the concatenated weights, the remembered tables, the training node."""
+    att = _attention("cpu")
+    rel = torch.randn(64, 128).to(torch.bfloat16)
+    called = []
+    plain = torch.nn.Linear.forward
+
+    def fused(att):
+        with torch.no_grad():
+            return att.eval()._native_args(None, rel, False) is not None, att.train()._trains_as_one_node()
+
+    assert fused(att) == (True, True)
+    for _ in _changes(att.get_submodule(name)):
+        assert fused(att) == (False, False)
+    part = att.get_submodule(name)
+    part.forward = lambda x: called.append(1) or plain(part, x)
+    with torch.no_grad():
+        att.eval()._qkv(rel[None], rel[None])
+        assert len(called) == 1
+        att._pos_layers(rel)
+        att._pos_layers(rel)
+    assert len(called) == (1 if name == "value_proj" else 3)   # the tables are not remembered past a forward nobody has looked into
+    del part.forward
+    assert fused(att) == (True, True)
+
+
 @pytest.mark.gpu
 def test_dropout_kept_on_in_an_eval_model():
     layer = _encoder_layer(0.5).cuda()
@@ -137,13 +198,13 @@ def test_dropout_kept_on_in_an_eval_model():
     assert not torch.equal(*sampled)
 
 
-def _attention(**kw):
+def _attention(device="cuda", **kw):
     from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
 
     torch.manual_seed(5)
     cfg = DebertaV2Config(hidden_size=128, num_attention_heads=2, relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32,
                           max_relative_positions=64, share_att_key=True, hidden_dropout_prob=0.0, attention_probs_dropout_prob=0.0, **kw)
-    return FlashDisentangledSelfAttention(cfg).cuda().to(torch.bfloat16)
+    return FlashDisentangledSelfAttention(cfg).to(device).to(torch.bfloat16)
 
 
 @pytest.mark.gpu
