@@ -66,6 +66,7 @@ def _kind(cls):
 
 
 _LINEAR, _DROPOUT = _kind(torch.nn.Linear), _kind(torch.nn.Dropout)
+_SHARED_PARTS = _LINEAR, _LINEAR, _LINEAR, _DROPOUT
 
 
 def _stands_in(modules, kinds):
@@ -132,9 +133,11 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         return (self.query_proj(query_states).view(B, L, H, D), self.key_proj(hidden_states).view(B, L, H, D),
                 self.value_proj(hidden_states).view(B, L, H, D))
 
-    def _pos_layers(self, rel_embeddings, plain=False):
+    def _pos_layers(self, rel_embeddings, plain=False, dropped=None):
         """K_r, Q_r as [H, 2S, D] views of the projected relative embeddings
-        (reference model.py:159-177; the slice to 2S rows is transformers modeling_deberta_v2.py:295)."""
+        (reference model.py:159-177; the slice to 2S rows is transformers modeling_deberta_v2.py:295).
+        plain: the caller knows that nobody has touched these projections and pos_dropout; dropped: what pos_dropout gave for these embeddings, if the
+        caller has called it."""
         if not self.relative_attention or rel_embeddings is None:
             return None, None
         # the position projections exist only for the terms the module has (transformers :170-178)
@@ -147,16 +150,17 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         key = None
         recording = torch.is_grad_enabled() and (rel_embeddings.requires_grad or self.query_proj.weight.requires_grad)
         projections = tuple(m for m in (kproj, qproj) if m is not None)
+        dropout = modules["pos_dropout"]
         # a remembered K_r / Q_r must not carry an autograd graph, and depends on nothing but the embeddings and the weights
-        # (`plain`: the caller knows that about these projections)
-        if not self.training and not recording and (plain or _stands_in(projections, (_LINEAR,) * len(projections))):
+        if not self.training and not recording and (plain or _stands_in((*projections, dropout), (*(_LINEAR,) * len(projections), _DROPOUT))) \
+                and not (dropout.training and dropout.p > 0.0):
             key = (rel_embeddings,) + tuple(p for m in projections for p in _weight_and_bias(m) if p is not None)
             hit = self._pos_memo.get(key, tuple(self.pos_att_type))
             if hit is not None:
                 return hit
         H, D = self.num_attention_heads, self.attention_head_size
         span = self.pos_ebd_size
-        rel = self.pos_dropout(rel_embeddings)[0:2 * span]
+        rel = (dropout(rel_embeddings) if dropped is None else dropped)[0:2 * span]
 
         def heads(x):  # [2S, H*D] -> [H, 2S, D] without a copy
             return x.view(x.shape[0], H, D).transpose(0, 1)
@@ -191,10 +195,13 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         if torch.is_grad_enabled() and (hidden_requires_grad or (rel_embeddings is not None and rel_embeddings.requires_grad)
                                         or any(p.requires_grad for p in self.parameters())):
             return None
-        fused = self._fused_qkv() if self._plain_projections() else None
+        modules = self._modules
+        parts = modules["query_proj"], modules["key_proj"], modules["value_proj"], modules.get("pos_dropout")
+        shared = self.relative_attention and self.share_att_key   # the tables come from these parts alone
+        fused = self._fused_qkv() if (_stands_in(parts, _SHARED_PARTS) if shared else self._plain_projections()) else None
         if fused is None:
             return None
-        pos_key, pos_query = self._pos_layers(rel_embeddings, self.share_att_key)
+        pos_key, pos_query = self._pos_layers(rel_embeddings, shared)
         return (*fused, pos_key, pos_query, self.num_attention_heads, *self._score_settings(pos_key, pos_query), *self._bounds(attention_mask))
 
     def _trains_as_one_node(self):
@@ -221,15 +228,16 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         if args is not None:
             return native.layer_attention(hidden_states, *args, self._own_products), None
         seq_start, seq_len = self._bounds(attention_mask)
+        rel = None
         if query_states is hidden_states and rel_embeddings is not None and self._trains_as_one_node():
             sm_scale, buckets, max_distance = self._score_settings(rel_embeddings, rel_embeddings)
             modules = self._modules
-            rel = rel_embeddings if not self.training else self.pos_dropout(rel_embeddings)
+            rel = self.pos_dropout(rel_embeddings)
             ctx = native.layer_node(hidden_states, rel, *[p for n in ("query_proj", "key_proj", "value_proj") for p in _weight_and_bias(modules[n])],
                                     H, sm_scale, buckets, max_distance, seq_start, seq_len)
             if ctx is not None:
                 return ctx, None
-        pos_key, pos_query = self._pos_layers(rel_embeddings)
+        pos_key, pos_query = self._pos_layers(rel_embeddings, dropped=rel)
         sm_scale, buckets, max_distance = self._score_settings(pos_key, pos_query)
 
         q, k, v = self._qkv(hidden_states, query_states)

@@ -6,7 +6,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from flashdeberta_amd import _lib
+from flashdeberta_amd import _lib, model
 from flashdeberta_amd.padding import key_padding_mask, seq_bounds
 
 
@@ -186,6 +186,40 @@ def test_changed_projections_are_called(name):
     assert fused(att) == (True, True)
 
 
+@pytest.mark.parametrize("how", ["on", "hook", "forward"])
+@pytest.mark.parametrize("node", [True, False], ids=["node", "no_node"])
+def test_dropout_of_the_relative_embeddings_is_called_once(node, how, monkeypatch):
+    """In an eval module, whether anything is recorded or not, and whether or not the training node takes the call."""
+    att = _attention("cpu", hidden_dropout_prob=0.5).eval()
+    rel, x = torch.randn(64, 128).to(torch.bfloat16), torch.randn(1, 8, 128).to(torch.bfloat16)
+    calls, seen = [], []
+    if how == "forward":
+        att.pos_dropout.forward = lambda r: calls.append(1) or r * 2
+    else:
+        att.pos_dropout.train(how == "on")
+        att.pos_dropout.register_forward_hook(lambda *a: calls.append(1)) if how == "hook" else None
+
+    def layer_node(hidden, rel, *rest):
+        seen.append(rel)
+        return hidden if node else None
+
+    monkeypatch.setattr(model, "native", SimpleNamespace(layer_node=layer_node, untouched=_lib.native.untouched))
+    monkeypatch.setattr(model.ops, "disentangled_attention", lambda q, k, v, pos_key, pos_query, **kw: seen.append(pos_key) or q)
+    att(x, None, rel_embeddings=rel)   # recorded: the weights require gradients
+    assert len(seen) == (1 if node else 2)
+    given = seen[0].detach()
+    if how == "on":
+        assert (given == 0).any() and ((given == 0) | (given == (2 * rel).to(given.dtype))).all()
+    else:
+        assert torch.equal(given, rel * 2 if how == "forward" else rel) and len(calls) == 1
+    if not node:
+        assert torch.equal(seen[1], F.linear(given, att.key_proj.weight, att.key_proj.bias).view(64, 2, 64).transpose(0, 1))
+    with torch.no_grad():   # not recorded: the tables are not remembered past a dropout that is more than nothing
+        att._pos_layers(rel)
+        first, second = att._pos_layers(rel)[0], att._pos_layers(rel)[0]
+    assert not torch.equal(first, second) if how == "on" else len(calls) == 4
+
+
 @pytest.mark.gpu
 def test_dropout_kept_on_in_an_eval_model():
     layer = _encoder_layer(0.5).cuda()
@@ -198,12 +232,13 @@ def test_dropout_kept_on_in_an_eval_model():
     assert not torch.equal(*sampled)
 
 
-def _attention(device="cuda", **kw):
+def _attention(device="cuda", hidden_dropout_prob=0.0, **kw):
     from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
 
     torch.manual_seed(5)
     cfg = DebertaV2Config(hidden_size=128, num_attention_heads=2, relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32,
-                          max_relative_positions=64, share_att_key=True, hidden_dropout_prob=0.0, attention_probs_dropout_prob=0.0, **kw)
+                          max_relative_positions=64, share_att_key=True, hidden_dropout_prob=hidden_dropout_prob,
+                          attention_probs_dropout_prob=0.0, **kw)
     return FlashDisentangledSelfAttention(cfg).to(device).to(torch.bfloat16)
 
 
