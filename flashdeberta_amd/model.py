@@ -66,7 +66,6 @@ def _kind(cls):
 
 
 _LINEAR, _DROPOUT = _kind(torch.nn.Linear), _kind(torch.nn.Dropout)
-_SHARED_PARTS = _LINEAR, _LINEAR, _LINEAR, _DROPOUT
 
 
 def _stands_in(modules, kinds):
@@ -74,6 +73,10 @@ def _stands_in(modules, kinds):
     no hooks on all modules."""
     return native.untouched(modules, kinds) and not (nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
                                                      or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
+
+
+_PROJECTIONS = "query_proj", "key_proj", "value_proj", "pos_key_proj", "pos_query_proj"
+_PARTS = {n: (_LINEAR,) * n + (_DROPOUT,) for n in (3, 4, 5)}
 
 
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
@@ -103,6 +106,25 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         modules = self._modules
         return _stands_in((modules["query_proj"], modules["key_proj"], modules["value_proj"]), (_LINEAR, _LINEAR, _LINEAR))
 
+    def _plain_parts(self):
+        """The same for all parts: the projections of the relative embeddings and their dropout among them."""
+        modules = self._modules
+        if not self.relative_attention:
+            return self._plain_projections()
+        parts = [modules[n] for n in ("query_proj", "key_proj", "value_proj")]
+        if not self.share_att_key:
+            parts += [modules[n] for n in ("pos_key_proj", "pos_query_proj") if n in modules]
+        return _stands_in((*parts, modules["pos_dropout"]), _PARTS[len(parts)])
+
+    def _recording(self, *inputs):
+        """Whether autograd records what is computed from these tensors and the projections' weights, the ones that are read: a
+        DataParallel replica holds its weights as plain attributes and has no parameters."""
+        if not torch.is_grad_enabled():
+            return False
+        modules = self._modules
+        weights = [p for n in _PROJECTIONS if n in modules for p in _weight_and_bias(modules[n])]
+        return any(x is not None and x.requires_grad for x in (*inputs, *weights))
+
     def _fused_qkv(self):
         """Concatenated [3*H*D, hidden] weight and bias of the query, key and value projections (plain ones), None where only
         some have a bias."""
@@ -125,8 +147,8 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         B, L, _ = hidden_states.shape
         H, D = self.num_attention_heads, self.attention_head_size
         # the concatenated weights are a copy made outside autograd: only where nothing is being recorded
-        recording = torch.is_grad_enabled() and (hidden_states.requires_grad or self.query_proj.weight.requires_grad)
-        fused = None if (self.training or recording or query_states is not hidden_states or not self._plain_projections()) else self._fused_qkv()
+        fused = None if (self.training or query_states is not hidden_states or not self._plain_parts() or self._recording(hidden_states)) \
+            else self._fused_qkv()
         if fused is not None:
             qkv = F.linear(hidden_states, fused[0], fused[1]).view(B, L, 3, H, D)
             return qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
@@ -136,7 +158,7 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     def _pos_layers(self, rel_embeddings, plain=False, dropped=None):
         """K_r, Q_r as [H, 2S, D] views of the projected relative embeddings
         (reference model.py:159-177; the slice to 2S rows is transformers modeling_deberta_v2.py:295).
-        plain: the caller knows that nobody has touched these projections and pos_dropout; dropped: what pos_dropout gave for these embeddings, if the
+        plain: the caller knows that nobody has touched the parts and that nothing is recorded; dropped: what pos_dropout gave for these embeddings, if the
         caller has called it."""
         if not self.relative_attention or rel_embeddings is None:
             return None, None
@@ -148,13 +170,10 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         if "p2c" in self.pos_att_type:
             qproj = modules["query_proj" if self.share_att_key else "pos_query_proj"]
         key = None
-        recording = torch.is_grad_enabled() and (rel_embeddings.requires_grad or self.query_proj.weight.requires_grad)
-        projections = tuple(m for m in (kproj, qproj) if m is not None)
         dropout = modules["pos_dropout"]
         # a remembered K_r / Q_r must not carry an autograd graph, and depends on nothing but the embeddings and the weights
-        if not self.training and not recording and (plain or _stands_in((*projections, dropout), (*(_LINEAR,) * len(projections), _DROPOUT))) \
-                and not (dropout.training and dropout.p > 0.0):
-            key = (rel_embeddings,) + tuple(p for m in projections for p in _weight_and_bias(m) if p is not None)
+        if not self.training and (plain or self._plain_parts() and not self._recording(rel_embeddings)) and not (dropout.training and dropout.p > 0.0):
+            key = (rel_embeddings,) + tuple(p for m in (kproj, qproj) if m is not None for p in _weight_and_bias(m) if p is not None)
             hit = self._pos_memo.get(key, tuple(self.pos_att_type))
             if hit is not None:
                 return hit
@@ -186,22 +205,18 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         arbitrary masks)."""
         return (None, None) if attention_mask is None else _seq_bounds_of(attention_mask, self._mask_memo)
 
-    def _native_args(self, attention_mask, rel_embeddings, hidden_requires_grad):
+    def _native_args(self, attention_mask, rel_embeddings, hidden_states=None):
         """What follows the hidden states in a call of native.layer_attention, or None where that path does not serve:
         in training or while anything is recorded (the concatenated weights are a copy made outside autograd), under
         autocast, with FP8 operands, or with projections that are more than products with weights to concatenate."""
         if self.training or self.fp8_qk or torch.is_autocast_enabled():
             return None
-        if torch.is_grad_enabled() and (hidden_requires_grad or (rel_embeddings is not None and rel_embeddings.requires_grad)
-                                        or any(p.requires_grad for p in self.parameters())):
+        if not self._plain_parts() or self._recording(hidden_states, rel_embeddings):
             return None
-        modules = self._modules
-        parts = modules["query_proj"], modules["key_proj"], modules["value_proj"], modules.get("pos_dropout")
-        shared = self.relative_attention and self.share_att_key   # the tables come from these parts alone
-        fused = self._fused_qkv() if (_stands_in(parts, _SHARED_PARTS) if shared else self._plain_projections()) else None
+        fused = self._fused_qkv()
         if fused is None:
             return None
-        pos_key, pos_query = self._pos_layers(rel_embeddings, shared)
+        pos_key, pos_query = self._pos_layers(rel_embeddings, plain=True)
         return (*fused, pos_key, pos_query, self.num_attention_heads, *self._score_settings(pos_key, pos_query), *self._bounds(attention_mask))
 
     def _trains_as_one_node(self):
@@ -224,7 +239,7 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
             query_states = hidden_states
         B, L, _ = hidden_states.shape
         H, D = self.num_attention_heads, self.attention_head_size
-        args = self._native_args(attention_mask, rel_embeddings, hidden_states.requires_grad) if query_states is hidden_states else None
+        args = self._native_args(attention_mask, rel_embeddings, hidden_states) if query_states is hidden_states else None
         if args is not None:
             return native.layer_attention(hidden_states, *args, self._own_products), None
         seq_start, seq_len = self._bounds(attention_mask)
@@ -314,7 +329,7 @@ class FlashDebertaV2Layer(DebertaV2Layer):
             return None
         if any(m.normalized_shape != shape or m.bias is None or m.weight is None or m.weight.dtype != dtype for m in norms):
             return None
-        args = att._native_args(attention_mask, rel_embeddings, False)
+        args = att._native_args(attention_mask, rel_embeddings)
         if args is None:
             return None
         (ow, ob), (uw, ub), (dw, db) = [_weight_and_bias(m) for m in linears]

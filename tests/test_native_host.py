@@ -169,7 +169,7 @@ def test_changed_projections_are_called(name):
 
     def fused(att):
         with torch.no_grad():
-            return att.eval()._native_args(None, rel, False) is not None, att.train()._trains_as_one_node()
+            return att.eval()._native_args(None, rel) is not None, att.train()._trains_as_one_node()
 
     assert fused(att) == (True, True)
     for _ in _changes(att.get_submodule(name)):
@@ -220,6 +220,42 @@ def test_dropout_of_the_relative_embeddings_is_called_once(node, how, monkeypatc
     assert not torch.equal(first, second) if how == "on" else len(calls) == 4
 
 
+def _replica(module):
+    """What DataParallel computes on each device: a module whose weights are attributes carrying the graph back to the parameters."""
+    copy = module._replicate_for_data_parallel()
+    for name, child in module._modules.items():
+        copy._modules[name] = _replica(child)
+    for name, p in module._parameters.items():
+        setattr(copy, name, p * 1) if p is not None else copy._parameters.__setitem__(name, None)
+    return copy
+
+
+@pytest.mark.parametrize("share", [True, False], ids=["shared", "separate"])
+def test_weights_that_are_no_parameters_are_recorded(share):
+    """Eval mode with gradients on: a replica's projections, and any single weight that is not frozen, keep the inference paths off."""
+    att = _attention("cpu", share_att_key=share).eval()
+    rel, x = torch.randn(64, 128).to(torch.bfloat16), torch.randn(1, 8, 128).to(torch.bfloat16)
+
+    def recorded(a):
+        q, k, v = a._qkv(x, x)
+        pos_key, pos_query = a._pos_layers(rel)
+        return a._native_args(None, rel, x) is None, [t.requires_grad for t in (q, k, v, pos_key, pos_query)]
+
+    replica = _replica(att)
+    assert not list(replica.parameters())
+    assert recorded(replica) == (True, [True] * 5)
+    replica._qkv(x, x)[2].float().sum().backward()
+    assert att.value_proj.weight.grad is not None
+    for p in att.parameters():
+        p.requires_grad_(False)
+    assert recorded(att) == (False, [False] * 5)
+    for name, expected in (("query_proj", [1, 0, 0, 0, share]), ("key_proj", [0, 1, 0, share, 0]), ("value_proj", [0, 0, 1, 0, 0])) + \
+            (() if share else (("pos_key_proj", [0, 0, 0, 1, 0]), ("pos_query_proj", [0, 0, 0, 0, 1]))):
+        p = att.get_submodule(name).weight.requires_grad_(True)
+        assert recorded(att) == (True, [bool(e) for e in expected]), name
+        p.requires_grad_(False)
+
+
 @pytest.mark.gpu
 def test_dropout_kept_on_in_an_eval_model():
     layer = _encoder_layer(0.5).cuda()
@@ -232,12 +268,12 @@ def test_dropout_kept_on_in_an_eval_model():
     assert not torch.equal(*sampled)
 
 
-def _attention(device="cuda", hidden_dropout_prob=0.0, **kw):
+def _attention(device="cuda", hidden_dropout_prob=0.0, share_att_key=True, **kw):
     from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
 
     torch.manual_seed(5)
     cfg = DebertaV2Config(hidden_size=128, num_attention_heads=2, relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32,
-                          max_relative_positions=64, share_att_key=True, hidden_dropout_prob=hidden_dropout_prob,
+                          max_relative_positions=64, share_att_key=share_att_key, hidden_dropout_prob=hidden_dropout_prob,
                           attention_probs_dropout_prob=0.0, **kw)
     return FlashDisentangledSelfAttention(cfg).to(device).to(torch.bfloat16)
 
