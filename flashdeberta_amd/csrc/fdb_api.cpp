@@ -630,8 +630,8 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   };
   p->neg_lse = (float*)take(pairs * p->stat_len * 4);
   p->neg_delta = (float*)take(pairs * p->stat_len * 4);
-  p->far_q = take(pairs * 2 * p->stat_len * 2);
-  p->far_k = take(pairs * 2 * p->stat_len * 2);
+  p->far_q = (float*)take(pairs * 2 * p->stat_len * 4);
+  p->far_k = (float*)take(pairs * 2 * p->stat_len * 4);
   p->g_blocks = take(pairs * p->g_rows * p->g_slots * 2048);
   p->zero_block = take(2048);
   p->e_parts = (float*)take(parts * per * 4 * 2 * 32 * 64 * 4);

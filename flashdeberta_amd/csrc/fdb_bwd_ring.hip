@@ -658,10 +658,11 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
         for (int e = 0; e < 4; ++e) acc1[d][4 * q4 + e] = (acc1[d][4 * q4 + e] + far0 * r0[e] + far1 * r1[e]) * p.sm_scale;
       }
     if (g == 0) {
-      // ... and what the tables' saturated rows take from this row, [delta(+R), delta(-R)], rounded like every other score gradient
-      typename QT::scratch_t* fs = (typename QT::scratch_t*)(kDQ ? p.far_q : p.far_k) + ((int64_t)b * p.H + h) * 2 * p.stat_len + xr;
-      fs[0] = (typename QT::scratch_t)(kDQ ? sat0 : sat1);
-      fs[p.stat_len] = (typename QT::scratch_t)(kDQ ? sat1 : sat0);
+      // ... and what the tables' saturated rows take from this row, [delta(+R), delta(-R)]: sums over a whole sequence and without
+      // the soft-max scale, which in fp16 would leave its range long before the gradients made of them do
+      float* fs = (kDQ ? p.far_q : p.far_k) + ((int64_t)b * p.H + h) * 2 * p.stat_len + xr;
+      fs[0] = kDQ ? sat0 : sat1;
+      fs[p.stat_len] = kDQ ? sat1 : sat0;
     }
   }
   auto write = [&](char* ptr, int64_t sb, int64_t st, int64_t sh, const f32x16 (&acc)[DBLKS]) {
@@ -763,7 +764,6 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     f32x8 acc[2][2];
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[t >> 1][t & 1] = f32x8{0, 0, 0, 0, 0, 0, 0, 0};
-    using T = typename QT::scratch_t;
     const int r8 = lane >> 3, c8 = lane & 7;
     for (int it = it0; it < it1; ++it) {
       const int b = it / p.tg_chunks, c = it % p.tg_chunks;
@@ -772,15 +772,15 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
       const int i1 = min(Lb, (c + 1) * p.tg_len * 32);
       const char* qr = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh + 8 * c8) * 2;
       const char* kr = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh + 8 * c8) * 2;
-      const T* fq = (const T*)p.far_q + ((int64_t)b * p.H + h) * 2 * p.stat_len;
-      const T* fk = (const T*)p.far_k + ((int64_t)b * p.H + h) * 2 * p.stat_len;
+      const float* fq = p.far_q + ((int64_t)b * p.H + h) * 2 * p.stat_len;
+      const float* fk = p.far_k + ((int64_t)b * p.H + h) * 2 * p.stat_len;
 #pragma unroll 4
       for (int i = c * p.tg_len * 32 + 8 * wave + r8; i < i1; i += 32) {
         const f32x8 q = QT::to_f32(QT::load(qr + (int64_t)i * p.q_st * 2)), k = QT::to_f32(QT::load(kr + (int64_t)i * p.k_st * 2));
-        acc[0][0] += (float)fq[i] * q;
-        acc[0][1] += (float)fq[p.stat_len + i] * q;
-        acc[1][0] += (float)fk[i] * k;
-        acc[1][1] += (float)fk[p.stat_len + i] * k;
+        acc[0][0] += fq[i] * q;
+        acc[0][1] += fq[p.stat_len + i] * q;
+        acc[1][0] += fk[i] * k;
+        acc[1][1] += fk[p.stat_len + i] * k;
       }
     }
     float* s = (float*)smem;   // [32 row classes][4][64]

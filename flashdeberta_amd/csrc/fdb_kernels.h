@@ -110,13 +110,13 @@ struct FdbBwdRingParams {
   const int32_t* seq_start;
   const int32_t* seq_len;
   const int16_t* lut;
-  // scratch: row statistics [B][H][stat_len], far sums [B][H][2][stat_len] (element type of q), G blocks
-  // [B][H][g_rows][g_slots][32 x 32] (element type of q), partial table gradients [tg_parts][H][4 tg_groups][2][32][64] and
+  // scratch: row statistics [B][H][stat_len], far sums [B][H][2][stat_len], G blocks [B][H][g_rows][g_slots][32 x 32] (element type
+  // of q), partial table gradients [tg_parts][H][4 tg_groups][2][32][64] and
   // [tg_parts][H][2 tables][2 sides][64]
   float* neg_lse;
   float* neg_delta;
-  char* far_q;
-  char* far_k;
+  float* far_q;
+  float* far_k;
   char* g_blocks;
   char* zero_block;     // 2 KB of zeros, written by the dQ launch
   float* e_parts;

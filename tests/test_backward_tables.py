@@ -63,6 +63,40 @@ def test_table_backward_matches_oracle(case, dtype):
         assert err <= 3e-2 * max(np.abs(r).max(), 1e-2), "%s: err %.3e, largest %.3e" % (name, err, np.abs(r).max())
 
 
+def _rel(a, r):
+    return np.linalg.norm(_np(a) - r) / np.linalg.norm(r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_saturated_rows_of_a_key_that_all_queries_attend_to(dtype):
+    """Loss-scaled gradients: the far queries' score gradients of one key add up to 1.4e5, beyond fp16, while everything that leaves
+    the backward (which takes the soft-max scale, 1 / 13.9) is finite there."""
+    B, L, H, D, pb, mr = 1, 900, 1, 64, 32, 64
+    g = torch.Generator().manual_seed(3)
+    q = 1.2 + 0.05 * torch.randn(B, L, H, D, generator=g)
+    k, v = [0.05 * torch.randn(B, L, H, D, generator=g) for _ in range(2)]
+    k[:, 0] += 1.2          # q . k_0 / 13.9 = 6.6: half of every row's probability
+    v[:, 0] += 12.0         # dO . v_0 = 770
+    dout = 1.0 + 0.05 * torch.randn(B, L, H, D, generator=g)
+    pk, pq = [0.05 * torch.randn(H, 2 * pb, D, generator=g) for _ in range(2)]
+    q, k, v, dout, pk, pq = [x.to(dtype) for x in (q, k, v, dout, pk, pq)]
+    kw = dict(position_buckets=pb, max_relative_positions=mr)
+    c = [x.cuda() for x in (q, k, v, pk, pq)]
+    out, lse = ops.disentangled_attention_fwd(*c, return_lse=True, **kw)
+    got = ops.disentangled_attention_bwd(*c[:3], out, lse, dout.cuda(), *c[3:], **kw)
+    t = lambda x: _np(x).transpose(0, 2, 1, 3)
+    ref = O.disentangled_attention_backward(*[t(x) for x in (q, k, v, dout)], _np(pk), _np(pq), pb, mr)
+    ref = [r.transpose(0, 2, 1, 3) for r in ref[:3]] + list(ref[3:])
+    # the sum itself, from what it becomes: d pos_query of the saturated rows is the far sums of all keys times the keys
+    assert np.abs(ref[4]).max() * np.sqrt(3 * D) / 1.3 > 65504 > max(np.abs(r).max() for r in ref)
+    for name, a, r in zip(("dq", "dk", "dv", "dK_r", "dQ_r"), got, ref):
+        assert torch.isfinite(a).all(), name
+        # scores, score gradients and results are rounded to the type once each, independently: half a unit in the last place each at
+        # most, less than two in the 2-norm of the whole
+        assert _rel(a, r) <= torch.finfo(dtype).eps, (name, _rel(a, r))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols,rows2,cols2", [(1, 8, 0, 0), (63, 512, 5, 8), (64, 520, 64, 512), (3, 16, 200, 8), (65, 2304, 512, 1536), (4096, 768, 0, 0)])
 def test_column_sums(rows, cols, rows2, cols2):
