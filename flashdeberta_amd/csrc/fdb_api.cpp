@@ -136,9 +136,9 @@ int far_parts_wanted(const fdb_attn_args* a) {
 // sequence of 1024: 0.056 -> 0.040 ms; one of 512: 0.025 -> 0.022; four of 512 in shares of eight
 // steps would go from 0.025 to 0.028.)  Two shares of twelve steps pay while they leave a fifth of the
 // slots free (two of 777 40.0 -> 38.3 us, two of 900 45.2 -> 43.0; three of 777, 504 shares, would lose 7 %).
-// `room`: the workspace is sized for two shares with a partial second round as well (288 to 352 query tiles), which
-// the launch does not take: dealt longest first, the tiles are 3 to 8 % faster unshared there.
-int near_parts_wanted(const fdb_attn_args* a, bool room = false) {
+// Two shares with a partial second round (288 to 352 query tiles) are not taken: dealt longest first, the tiles are 3 to 8 %
+// faster unshared there.
+int near_parts_wanted(const fdb_attn_args* a) {
   if (!(a->pos_key || a->pos_query) || !a->lse || !steps32_supported(a->dtype, a->head_dim)) return 1;
   if (a->near_splits > 0) return a->near_splits;
   // A packed batch has its lengths on the device: the host goes by the mean length and by the most query tiles the
@@ -148,7 +148,7 @@ int near_parts_wanted(const fdb_attn_args* a, bool room = false) {
   const int steps_all = (typical + 31) / 32, steps_near = (FDB_BM + 2 * a->lut_radius + 3 * (FDB_BN - 1)) / 32;
   const int steps = steps_all < steps_near ? steps_all : steps_near;
   int best = 1;
-  for (int n = 2; n <= FDB_MAX_FAR_PARTS && (wgs * n <= slots || (room && n == 2 && !a->cu_seqlens && wgs * 10 <= slots * 7)); ++n) {
+  for (int n = 2; n <= FDB_MAX_FAR_PARTS && wgs * n <= slots; ++n) {
     const int per = steps / n;
     if (per >= 16 || (n == 2 && per >= 12 && wgs * n * 5 <= slots * 4) || (per >= 8 && wgs * n <= slots / 2)) best = n;
   }
@@ -328,7 +328,7 @@ int64_t fdb_attn_workspace_bytes(const fdb_attn_args* a) {
     const int parts = key_parts_wanted(a);
     return parts > 1 ? parts * far_part_bytes(a) : 0;
   }
-  const int near = near_parts_wanted(a, true);
+  const int near = near_parts_wanted(a);
   return (far_parts_wanted(a) - 1 + (near > 1 ? near : 0)) * far_part_bytes(a);
 }
 
