@@ -100,11 +100,10 @@ int64_t att_span(int64_t buckets, int64_t max_relative) { return buckets > 0 ? b
 // short batch.  Here both are kept per (shape, strides, type, epilogue) and the call is the launch alone.
 //   D [M, N] (row stride ldd) = op(A) op(B) (+ bias over N) (+ D): row-major matrices, A [M, K] or its transpose, B [K, N] or its transpose.
 struct GemmKey {
-  int64_t m, n, k, lda, ldb, ldd, batch, sa, sb, sd;
-  int32_t device, type, out_type, flags;  // flags: 1 A transposed, 2 B transposed, 4 bias, 8 accumulate onto D
+  int64_t m, n, k, lda, ldb, ldd;
+  int32_t device, type, flags;  // flags: 1 A transposed, 2 B transposed, 4 bias, 8 accumulate onto D
   bool operator<(const GemmKey& o) const {
-    return std::tie(m, n, k, lda, ldb, ldd, batch, sa, sb, sd, device, type, out_type, flags) <
-           std::tie(o.m, o.n, o.k, o.lda, o.ldb, o.ldd, o.batch, o.sa, o.sb, o.sd, o.device, o.type, o.out_type, o.flags);
+    return std::tie(m, n, k, lda, ldb, ldd, device, type, flags) < std::tie(o.m, o.n, o.k, o.lda, o.ldb, o.ldd, o.device, o.type, o.flags);
   }
 };
 struct GemmPlan {
@@ -127,14 +126,7 @@ constexpr size_t kMostPlans = 512;  // a plan is a few hundred bytes; a program 
 
 void blas(hipblasStatus_t s, const char* what) { TORCH_CHECK(s == HIPBLAS_STATUS_SUCCESS, what, " failed: hipBLASLt status ", (int)s); }
 
-hipDataType blas_type(at::ScalarType t) {
-  switch (t) {
-    case at::kFloat: return HIP_R_32F;
-    case at::kBFloat16: return HIP_R_16BF;
-    case at::kHalf: return HIP_R_16F;
-    default: TORCH_CHECK_VALUE(false, "unsupported dtype ", t);
-  }
-}
+hipDataType blas_type(at::ScalarType t) { return t == at::kBFloat16 ? HIP_R_16BF : HIP_R_16F; }  // the callers refuse other types
 
 // Handles, plans and the bias pointer a plan carries into its launch are shared by the threads of a program: autograd runs the
 // backward's products on its own threads, without the GIL.  Held for a lookup or a launch, never while memory is asked for.
@@ -161,24 +153,16 @@ std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
   const hipblasOperation_t op_first = key.flags & 2 ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_second = key.flags & 1 ? HIPBLAS_OP_T : HIPBLAS_OP_N;
   set(HIPBLASLT_MATMUL_DESC_TRANSA, &op_first, sizeof(op_first));
   set(HIPBLASLT_MATMUL_DESC_TRANSB, &op_second, sizeof(op_second));
-  const auto in = (hipDataType)key.type, out = (hipDataType)key.out_type;
+  const auto type = (hipDataType)key.type;
   if (key.flags & 4) {
     const hipblasLtEpilogue_t e = HIPBLASLT_EPILOGUE_BIAS;
     set(HIPBLASLT_MATMUL_DESC_EPILOGUE, &e, sizeof(e));
-    set(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &in, sizeof(in));
+    set(HIPBLASLT_MATMUL_DESC_BIAS_DATA_TYPE, &type, sizeof(type));
   }
   // row-major [M, K] with row stride lda is column-major [K, M]
-  blas(hipblasLtMatrixLayoutCreate(&p.a, in, key.flags & 2 ? key.k : key.n, key.flags & 2 ? key.n : key.k, key.ldb), "hipblasLtMatrixLayoutCreate");
-  blas(hipblasLtMatrixLayoutCreate(&p.b, in, key.flags & 1 ? key.m : key.k, key.flags & 1 ? key.k : key.m, key.lda), "hipblasLtMatrixLayoutCreate");
-  blas(hipblasLtMatrixLayoutCreate(&p.d, out, key.n, key.m, key.ldd), "hipblasLtMatrixLayoutCreate");
-  if (key.batch > 1) {
-    const int32_t count = (int32_t)key.batch;
-    const std::pair<hipblasLtMatrixLayout_t, int64_t> ls[] = {{p.a, key.sb}, {p.b, key.sa}, {p.d, key.sd}};
-    for (const auto& l : ls) {
-      blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_BATCH_COUNT, &count, sizeof(count)), "hipblasLtMatrixLayoutSetAttribute");
-      blas(hipblasLtMatrixLayoutSetAttribute(l.first, HIPBLASLT_MATRIX_LAYOUT_STRIDED_BATCH_OFFSET, &l.second, sizeof(l.second)), "hipblasLtMatrixLayoutSetAttribute");
-    }
-  }
+  blas(hipblasLtMatrixLayoutCreate(&p.a, type, key.flags & 2 ? key.k : key.n, key.flags & 2 ? key.n : key.k, key.ldb), "hipblasLtMatrixLayoutCreate");
+  blas(hipblasLtMatrixLayoutCreate(&p.b, type, key.flags & 1 ? key.m : key.k, key.flags & 1 ? key.k : key.m, key.lda), "hipblasLtMatrixLayoutCreate");
+  blas(hipblasLtMatrixLayoutCreate(&p.d, type, key.n, key.m, key.ldd), "hipblasLtMatrixLayoutCreate");
   hipblasLtMatmulPreference_t pref = nullptr;
   blas(hipblasLtMatmulPreferenceCreate(&pref), "hipblasLtMatmulPreferenceCreate");
   const size_t most = at::cuda::getCUDABlasLtWorkspaceSize();  // torch's own bound, so that the choice is torch's own
@@ -196,15 +180,14 @@ std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
   return plan;
 }
 
-struct Mat {  // `batch` row-major matrices, `ld` elements between rows, `stride` elements between matrices
+struct Mat {  // a row-major matrix, `ld` elements between rows
   const void* p;
-  int64_t ld, stride = 0;
+  int64_t ld;
 };
-void gemm(const Tensor& on, at::ScalarType type, at::ScalarType out_type, bool trans_a, bool trans_b, int64_t batch, int64_t m, int64_t n, int64_t k,
-          Mat a, Mat b, Mat d, const void* bias = nullptr, bool accumulate = false) {
-  const int device = on.get_device();
-  const auto plan = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, batch, a.stride, b.stride, d.stride, device, (int32_t)blas_type(type), (int32_t)blas_type(out_type),
-                                  (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
+void gemm(const Tensor& on, bool trans_a, bool trans_b, int64_t m, int64_t n, int64_t k, Mat a, Mat b, Mat d, const void* bias = nullptr,
+          bool accumulate = false) {
+  const auto plan = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, (int32_t)on.get_device(), (int32_t)blas_type(on.scalar_type()),
+                                      (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
   GemmPlan& p = *plan;
   Tensor ws;
   if (p.workspace > 0) ws = at::empty({p.workspace}, on.options().dtype(at::kByte));
@@ -240,7 +223,7 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
     if (rc == 0) return out;
     if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
   }
-  gemm(x, type, type, false, true, 1, m, n, k, {x.data_ptr(), k}, {w.data_ptr(), w.stride(0)}, {out.data_ptr(), n}, b);
+  gemm(x, false, true, m, n, k, {x.data_ptr(), k}, {w.data_ptr(), w.stride(0)}, {out.data_ptr(), n}, b);
   return out;
 }
 
@@ -718,8 +701,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const auto type = hidden.scalar_type();
     const Tensor w = at::cat({qw, kw, vw}), b = at::cat({qb, kb, vb});
     const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
-    gemm(hidden, type, type, false, true, 1, B * L, 3 * W, C, {hidden.data_ptr(), C}, {w.data_ptr(), C}, {qkv.data_ptr(), 3 * W}, b.data_ptr());
-    gemm(hidden, type, type, false, true, 1, rows, 2 * W, C, {rel.data_ptr(), C}, {w.data_ptr(), C}, {pos.data_ptr(), 2 * W}, b.data_ptr());
+    gemm(hidden, false, true, B * L, 3 * W, C, {hidden.data_ptr(), C}, {w.data_ptr(), C}, {qkv.data_ptr(), 3 * W}, b.data_ptr());
+    gemm(hidden, false, true, rows, 2 * W, C, {rel.data_ptr(), C}, {w.data_ptr(), C}, {pos.data_ptr(), 2 * W}, b.data_ptr());
     const Tensor out = at::empty({B, L, W}, hidden.options());
     fdb_attn_args a = {};
     const char* p = (const char*)qkv.data_ptr();
@@ -767,16 +750,16 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     Tensor dhidden, drel, dw, db;
     if (ctx->needs_input_grad(0)) {
       dhidden = at::empty(hidden.sizes(), hidden.options());
-      gemm(hidden, type, type, false, false, 1, n, C, 3 * W, {dqkv.data_ptr(), 3 * W}, {w.data_ptr(), C}, {dhidden.data_ptr(), C});
+      gemm(hidden, false, false, n, C, 3 * W, {dqkv.data_ptr(), 3 * W}, {w.data_ptr(), C}, {dhidden.data_ptr(), C});
     }
     if (ctx->needs_input_grad(1)) {
       drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
-      gemm(hidden, type, type, false, false, 1, rows, C, 2 * W, {dpos.data_ptr(), 2 * W}, {w.data_ptr(), C}, {drel.data_ptr(), C});
+      gemm(hidden, false, false, rows, C, 2 * W, {dpos.data_ptr(), 2 * W}, {w.data_ptr(), C}, {drel.data_ptr(), C});
     }
     if (ctx->needs_input_grad(2) || ctx->needs_input_grad(4) || ctx->needs_input_grad(6)) {
       dw = at::empty({3 * W, C}, hidden.options());
-      gemm(hidden, type, type, true, false, 1, 3 * W, C, n, {dqkv.data_ptr(), 3 * W}, {hidden.data_ptr(), C}, {dw.data_ptr(), C});
-      gemm(hidden, type, type, true, false, 1, 2 * W, C, rows, {dpos.data_ptr(), 2 * W}, {rel.data_ptr(), C}, {dw.data_ptr(), C}, nullptr, true);
+      gemm(hidden, true, false, 3 * W, C, n, {dqkv.data_ptr(), 3 * W}, {hidden.data_ptr(), C}, {dw.data_ptr(), C});
+      gemm(hidden, true, false, 2 * W, C, rows, {dpos.data_ptr(), 2 * W}, {rel.data_ptr(), C}, {dw.data_ptr(), C}, nullptr, true);
     }
     if (ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7)) {
       db = at::empty({3 * W}, hidden.options());
