@@ -112,6 +112,7 @@ struct GemmPlan {
   hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
   hipblasLtMatmulAlgo_t algo;
   int64_t workspace = 0;
+  bool usable = false;   // the library has a kernel for this product
   GemmPlan() = default;
   GemmPlan(const GemmPlan&) = delete;
   GemmPlan& operator=(const GemmPlan&) = delete;
@@ -171,8 +172,7 @@ std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
   hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most, sizeof(most));
   const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(p.handle, p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
   hipblasLtMatmulPreferenceDestroy(pref);
-  blas(rc, "hipblasLtMatmulAlgoGetHeuristic");
-  TORCH_CHECK(n > 0, "hipBLASLt has no kernel for this product");
+  p.usable = rc == HIPBLAS_STATUS_SUCCESS && n > 0;   // a plan without a kernel is kept, too: the next call need not ask again
   p.algo = found.algo;
   p.workspace = (int64_t)found.workspaceSize;
   if (g_plans.size() >= kMostPlans) g_plans.clear();
@@ -180,23 +180,40 @@ std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
   return plan;
 }
 
-struct Mat {  // a row-major matrix, `ld` elements between rows
-  const void* p;
-  int64_t ld;
+struct Mat {  // the first `rows` rows of a row-major matrix; one of more dimensions is contiguous, its leading ones taken together
+  const Tensor& t;
+  int64_t rows;
+  int64_t cols() const { return t.size(-1); }
+  int64_t ld() const { return t.dim() == 2 ? t.stride(0) : cols(); }   // a dimension of one may have any stride
+  Tensor view() const { return t.dim() == 2 ? t.narrow(0, 0, rows) : t.view({-1, cols()}).narrow(0, 0, rows); }
 };
-void gemm(const Tensor& on, bool trans_a, bool trans_b, int64_t m, int64_t n, int64_t k, Mat a, Mat b, Mat d, const void* bias = nullptr,
-          bool accumulate = false) {
-  const auto plan = gemm_plan(GemmKey{m, n, k, a.ld, b.ld, d.ld, (int32_t)on.get_device(), (int32_t)blas_type(on.scalar_type()),
+// The product by hipBLASLt; false where that has no kernel for it or does not start the one it named.
+bool library_product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias = nullptr, bool accumulate = false) {
+  const Tensor& on = d.t;
+  const auto plan = gemm_plan(GemmKey{trans_a ? a.cols() : a.rows, trans_b ? b.rows : b.cols(), trans_a ? a.rows : a.cols(), a.ld(), b.ld(), d.ld(),
+                                      (int32_t)on.get_device(), (int32_t)blas_type(on.scalar_type()),
                                       (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
   GemmPlan& p = *plan;
+  if (!p.usable) return false;
   Tensor ws;
   if (p.workspace > 0) ws = at::empty({p.workspace}, on.options().dtype(at::kByte));
   const float one = 1.f, beta = accumulate ? 1.f : 0.f;
   const std::lock_guard<std::mutex> lock(g_blas_mutex);
-  if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias, sizeof(bias)), "hipblasLtMatmulDescSetAttribute");
-  blas(hipblasLtMatmul(p.handle, p.desc, &one, b.p, p.a, a.p, p.b, &beta, d.p, p.d, const_cast<void*>(d.p), p.d, &p.algo,
-                       p.workspace > 0 ? ws.data_ptr() : nullptr, p.workspace, (hipStream_t)stream_of(on)),
-       "hipblasLtMatmul");
+  const void* bias_at = bias ? bias->data_ptr() : nullptr;
+  if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias_at, sizeof(bias_at)), "hipblasLtMatmulDescSetAttribute");
+  return hipblasLtMatmul(p.handle, p.desc, &one, b.t.data_ptr(), p.a, a.t.data_ptr(), p.b, &beta, d.t.data_ptr(), p.d, d.t.data_ptr(), p.d, &p.algo,
+                         p.workspace > 0 ? ws.data_ptr() : nullptr, p.workspace, (hipStream_t)stream_of(on)) == HIPBLAS_STATUS_SUCCESS;
+}
+// The same product by torch, whose own route does not end at hipBLASLt.
+void torch_product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias = nullptr, bool accumulate = false) {
+  const Tensor x = trans_a ? a.view().t() : a.view(), y = trans_b ? b.view().t() : b.view();
+  Tensor out = d.view();
+  if (bias) at::addmm_out(out, bias->narrow(0, 0, y.size(1)), x, y);
+  else if (accumulate) out.addmm_(x, y);
+  else at::mm_out(out, x, y);
+}
+void product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias = nullptr, bool accumulate = false) {
+  if (!library_product(a, trans_a, b, trans_b, d, bias, accumulate)) torch_product(a, trans_a, b, trans_b, d, bias, accumulate);
 }
 
 // x [..., K] . w [N, K]^T + bias -> [..., N], as torch's linear computes it, bit for bit (the heuristic's choice is the same).
@@ -217,14 +234,26 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
   auto size = x.sizes().vec();
   size.back() = n;
   const Tensor out = at::empty(size, x.options());
-  const void* b = bias->data_ptr();
   if (own && (m <= 32 || (k <= 1536 && ((m + 63) / 64) * ((n + 63) / 64) <= 256))) {
-    const int rc = fdb_linear(x.data_ptr(), w.data_ptr(), b, out.data_ptr(), (int32_t)m, (int32_t)n, (int32_t)k, k, w.stride(0), n, fdb_dtype_of(type), stream_of(x));
+    const int rc = fdb_linear(x.data_ptr(), w.data_ptr(), bias->data_ptr(), out.data_ptr(), (int32_t)m, (int32_t)n, (int32_t)k, k, w.stride(0), n, fdb_dtype_of(type), stream_of(x));
     if (rc == 0) return out;
     if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
   }
-  gemm(x, false, true, m, n, k, {x.data_ptr(), k}, {w.data_ptr(), w.stride(0)}, {out.data_ptr(), n}, b);
-  return out;
+  return library_product({x, m}, false, {w, n}, true, {out, m}, &*bias) ? out : at::linear(x_in, w, bias);
+}
+
+// product(a, rows_a, trans_a, b, rows_b, trans_b, d, rows_d, bias or None, accumulate, library): into d, by hipBLASLt (whether it has
+// done it) or by torch
+PyObject* py_product(PyObject*, PyObject* const* x, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n == 11, "product takes 11 arguments");
+  const Mat a{tensor_arg(x[0], "a"), int_arg(x[1])}, b{tensor_arg(x[3], "b"), int_arg(x[4])}, d{tensor_arg(x[6], "d"), int_arg(x[7])};
+  const OptTensor bias = opt_tensor_arg(x[8], "bias");
+  bool done = true;
+  if (bool_arg(x[10])) done = library_product(a, bool_arg(x[2]), b, bool_arg(x[5]), d, bias ? &*bias : nullptr, bool_arg(x[9]));
+  else torch_product(a, bool_arg(x[2]), b, bool_arg(x[5]), d, bias ? &*bias : nullptr, bool_arg(x[9]));
+  return PyBool_FromLong(done);
+  END_HANDLE_TH_ERRORS
 }
 
 // linear(x, weight, bias, own) -> x . weight^T + bias
@@ -701,8 +730,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const auto type = hidden.scalar_type();
     const Tensor w = at::cat({qw, kw, vw}), b = at::cat({qb, kb, vb});
     const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
-    gemm(hidden, false, true, B * L, 3 * W, C, {hidden.data_ptr(), C}, {w.data_ptr(), C}, {qkv.data_ptr(), 3 * W}, b.data_ptr());
-    gemm(hidden, false, true, rows, 2 * W, C, {rel.data_ptr(), C}, {w.data_ptr(), C}, {pos.data_ptr(), 2 * W}, b.data_ptr());
+    product({hidden, B * L}, false, {w, 3 * W}, true, {qkv, B * L}, &b);
+    product({rel, rows}, false, {w, 2 * W}, true, {pos, rows}, &b);
     const Tensor out = at::empty({B, L, W}, hidden.options());
     fdb_attn_args a = {};
     const char* p = (const char*)qkv.data_ptr();
@@ -750,16 +779,16 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     Tensor dhidden, drel, dw, db;
     if (ctx->needs_input_grad(0)) {
       dhidden = at::empty(hidden.sizes(), hidden.options());
-      gemm(hidden, false, false, n, C, 3 * W, {dqkv.data_ptr(), 3 * W}, {w.data_ptr(), C}, {dhidden.data_ptr(), C});
+      product({dqkv, n}, false, {w, 3 * W}, false, {dhidden, n});
     }
     if (ctx->needs_input_grad(1)) {
       drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
-      gemm(hidden, false, false, rows, C, 2 * W, {dpos.data_ptr(), 2 * W}, {w.data_ptr(), C}, {drel.data_ptr(), C});
+      product({dpos, rows}, false, {w, 2 * W}, false, {drel, rows});
     }
     if (ctx->needs_input_grad(2) || ctx->needs_input_grad(4) || ctx->needs_input_grad(6)) {
       dw = at::empty({3 * W, C}, hidden.options());
-      gemm(hidden, true, false, 3 * W, C, n, {dqkv.data_ptr(), 3 * W}, {hidden.data_ptr(), C}, {dw.data_ptr(), C});
-      gemm(hidden, true, false, 2 * W, C, rows, {dpos.data_ptr(), 2 * W}, {rel.data_ptr(), C}, {dw.data_ptr(), C}, nullptr, true);
+      product({dqkv, n}, true, {hidden, n}, false, {dw, 3 * W});
+      product({dpos, rows}, true, {rel, rows}, false, {dw, 2 * W}, nullptr, true);
     }
     if (ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7)) {
       db = at::empty({3 * W}, hidden.options());
@@ -1047,6 +1076,7 @@ PyMethodDef module_methods[] = {
     {"layer_node", (PyCFunction)(void*)py_layer_node, METH_FASTCALL, nullptr},
     {"attention_bwd", (PyCFunction)(void*)py_attention_bwd, METH_FASTCALL, nullptr},
     {"layer_attention", (PyCFunction)(void*)py_layer_attention, METH_FASTCALL, nullptr},
+    {"product", (PyCFunction)(void*)py_product, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, nullptr},
     {"encoder_layer", (PyCFunction)(void*)py_encoder_layer, METH_FASTCALL, nullptr},
     {"quantize_e4m3", (PyCFunction)(void*)py_quantize, METH_FASTCALL, nullptr},

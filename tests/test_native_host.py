@@ -63,6 +63,39 @@ def test_library_products_have_the_bits_of_torch(M, N, K, dtype):
     assert torch.equal(_lib.native.linear(x, w, b, False), F.linear(x, w, b))
 
 
+# Every form of a product that a layer has: (transposed a, transposed b, bias, accumulated, a with 2 dimensions, 3, or 3
+# with one of them of size one and any stride); the rows that take part are the first of more.
+FORMS = [(False, True, True, False, 3), (False, True, True, False, 4), (False, True, True, False, 2), (False, False, False, False, 2), (True, False, False, False, 3),
+         (True, False, False, True, 2)]
+
+
+@pytest.mark.parametrize("route", [pytest.param(("cpu", False), id="torch_cpu"), pytest.param(("cuda", False), id="torch", marks=pytest.mark.gpu),
+                                   pytest.param(("cuda", True), id="library", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: "%s%s%s%s%d" % ("t" if f[0] else "n", "t" if f[1] else "n", "b" if f[2] else "", "+" if f[3] else "", f[4]))
+def test_products_and_their_second_route(form, route):
+    """hipBLASLt's product and the one that stands in where it has no kernel compute the same forms."""
+    trans_a, trans_b, with_bias, accumulate, dims = form
+    device, library = route
+    m, n, k = 48, 32, 64
+    g = torch.Generator().manual_seed(m + sum(form))
+    normal = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(device)
+    rows_a, rows_b = (k, n if trans_b else k) if trans_a else (m, n if trans_b else k)
+    cols_a = m if trans_a else k
+    a = normal(rows_a + 16, cols_a) if dims == 2 else normal(2, rows_a // 2, cols_a) if dims == 3 else normal(2, rows_a, cols_a)[1:].transpose(0, 1)
+    assert dims == 2 or a.is_contiguous()
+    b, d, bias = normal(rows_b + 16, k if trans_b else n), normal(m + 16, n), normal(n + 16) if with_bias else None
+    before = d.clone()
+    assert _lib.native.product(a, rows_a, trans_a, b, rows_b, trans_b, d, m, bias, accumulate, library) is True
+    x, y = a.reshape(-1, a.shape[-1])[:rows_a].double(), b[:rows_b].double()
+    ref = (x.t() if trans_a else x) @ (y.t() if trans_b else y)
+    if with_bias:
+        ref = ref + bias[:n].double()
+    if accumulate:
+        ref = ref + before[:m].double()
+    assert torch.equal(d[m:], before[m:])
+    assert ((d[:m].double() - ref).norm() / ref.norm()).item() <= 2.0 ** -8   # one rounding of the result to bf16
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,L", [(1, 5), (2, 40), (3, 300), (6, 384)])   # each way of computing the projections
 def test_encoder_layer_matches_the_module_by_module_forward(B, L):
