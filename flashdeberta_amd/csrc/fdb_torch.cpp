@@ -67,6 +67,16 @@ bool bool_arg(PyObject* o) {
   return v != 0;
 }
 
+// What an entry does once its arguments are read -- allocations, searches for a kernel, launches that wait for a place in a queue --
+// is done without the interpreter's lock, so that the threads of a program do not wait for one another.
+using NoGil = pybind11::gil_scoped_release;
+
+[[noreturn]] void throw_python() {  // the pending Python error, carried out of the scope that holds the lock
+  python_error e;
+  e.persist();
+  throw e;
+}
+
 // Negative codes are argument errors (ValueError), positive ones HIP errors (RuntimeError).
 void check(int code, const char* what) {
   if (code == 0) return;
@@ -100,14 +110,14 @@ int64_t att_span(int64_t buckets, int64_t max_relative) { return buckets > 0 ? b
 // short batch.  Here both are kept per (shape, strides, type, epilogue) and the call is the launch alone.
 //   D [M, N] (row stride ldd) = op(A) op(B) (+ bias over N) (+ D): row-major matrices, A [M, K] or its transpose, B [K, N] or its transpose.
 struct GemmKey {
+  hipblasLtHandle_t handle;
   int64_t m, n, k, lda, ldb, ldd;
-  int32_t device, type, flags;  // flags: 1 A transposed, 2 B transposed, 4 bias, 8 accumulate onto D
+  int32_t type, flags;  // flags: 1 A transposed, 2 B transposed, 4 bias, 8 accumulate onto D
   bool operator<(const GemmKey& o) const {
-    return std::tie(m, n, k, lda, ldb, ldd, device, type, flags) < std::tie(o.m, o.n, o.k, o.lda, o.ldb, o.ldd, o.device, o.type, o.flags);
+    return std::tie(handle, m, n, k, lda, ldb, ldd, type, flags) < std::tie(o.handle, o.m, o.n, o.k, o.lda, o.ldb, o.ldd, o.type, o.flags);
   }
 };
 struct GemmPlan {
-  hipblasLtHandle_t handle = nullptr;
   hipblasLtMatmulDesc_t desc = nullptr;
   hipblasLtMatrixLayout_t a = nullptr, b = nullptr, d = nullptr;
   hipblasLtMatmulAlgo_t algo;
@@ -129,26 +139,19 @@ void blas(hipblasStatus_t s, const char* what) { TORCH_CHECK(s == HIPBLAS_STATUS
 
 hipDataType blas_type(at::ScalarType t) { return t == at::kBFloat16 ? HIP_R_16BF : HIP_R_16F; }  // the callers refuse other types
 
-// Handles, plans and the bias pointer a plan carries into its launch are shared by the threads of a program: autograd runs the
-// backward's products on its own threads, without the GIL.  Held for a lookup or a launch, never while memory is asked for.
-std::mutex g_blas_mutex;
-
-hipblasLtHandle_t blas_handle(int device) {
-  static std::map<int, hipblasLtHandle_t> handles;
-  hipblasLtHandle_t& h = handles[device];
-  if (!h) blas(hipblasLtCreate(&h), "hipblasLtCreate");
-  return h;
-}
-
 // The library is column-major: D^T [N, M] = op(B)^T op(A)^T, so B's memory is its first operand and A's the second.
+// A plan belongs to a handle of torch's, and torch lends a handle of a device to one thread at a time: the bias pointer that a plan
+// carries into its launch, and the launch, need no lock.  The mutex is held for a look into the map alone.
+std::mutex g_plans_mutex;
 std::map<GemmKey, std::shared_ptr<GemmPlan>> g_plans;
 std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
-  const std::lock_guard<std::mutex> lock(g_blas_mutex);
-  const auto hit = g_plans.find(key);
-  if (hit != g_plans.end()) return hit->second;
+  {
+    const std::lock_guard<std::mutex> lock(g_plans_mutex);
+    const auto hit = g_plans.find(key);
+    if (hit != g_plans.end()) return hit->second;
+  }
   const auto plan = std::make_shared<GemmPlan>();
   GemmPlan& p = *plan;
-  p.handle = blas_handle(key.device);
   blas(hipblasLtMatmulDescCreate(&p.desc, HIPBLAS_COMPUTE_32F, HIP_R_32F), "hipblasLtMatmulDescCreate");
   const auto set = [&](hipblasLtMatmulDescAttributes_t what, const void* v, size_t n) { blas(hipblasLtMatmulDescSetAttribute(p.desc, what, v, n), "hipblasLtMatmulDescSetAttribute"); };
   const hipblasOperation_t op_first = key.flags & 2 ? HIPBLAS_OP_T : HIPBLAS_OP_N, op_second = key.flags & 1 ? HIPBLAS_OP_T : HIPBLAS_OP_N;
@@ -170,12 +173,13 @@ std::shared_ptr<GemmPlan> gemm_plan(const GemmKey& key) {
   hipblasLtMatmulHeuristicResult_t found = {};
   int n = 0;
   hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &most, sizeof(most));
-  const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(p.handle, p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
+  const hipblasStatus_t rc = hipblasLtMatmulAlgoGetHeuristic(key.handle, p.desc, p.a, p.b, p.d, p.d, pref, 1, &found, &n);
   hipblasLtMatmulPreferenceDestroy(pref);
   p.usable = rc == HIPBLAS_STATUS_SUCCESS && n > 0;   // a plan without a kernel is kept, too: the next call need not ask again
   p.algo = found.algo;
   p.workspace = (int64_t)found.workspaceSize;
-  if (g_plans.size() >= kMostPlans) g_plans.clear();
+  const std::lock_guard<std::mutex> lock(g_plans_mutex);
+  if (g_plans.size() >= kMostPlans) g_plans.clear();   // one that another thread is using lives until it is done
   g_plans.emplace(key, plan);
   return plan;
 }
@@ -190,18 +194,18 @@ struct Mat {  // the first `rows` rows of a row-major matrix; one of more dimens
 // The product by hipBLASLt; false where that has no kernel for it or does not start the one it named.
 bool library_product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias = nullptr, bool accumulate = false) {
   const Tensor& on = d.t;
-  const auto plan = gemm_plan(GemmKey{trans_a ? a.cols() : a.rows, trans_b ? b.rows : b.cols(), trans_a ? a.rows : a.cols(), a.ld(), b.ld(), d.ld(),
-                                      (int32_t)on.get_device(), (int32_t)blas_type(on.scalar_type()),
+  const hipblasLtHandle_t handle = at::cuda::getCurrentCUDABlasLtHandle();   // the callers have made d's device the current one
+  const auto plan = gemm_plan(GemmKey{handle, trans_a ? a.cols() : a.rows, trans_b ? b.rows : b.cols(), trans_a ? a.rows : a.cols(), a.ld(), b.ld(), d.ld(),
+                                      (int32_t)blas_type(on.scalar_type()),
                                       (trans_a ? 1 : 0) | (trans_b ? 2 : 0) | (bias ? 4 : 0) | (accumulate ? 8 : 0)});
   GemmPlan& p = *plan;
   if (!p.usable) return false;
   Tensor ws;
   if (p.workspace > 0) ws = at::empty({p.workspace}, on.options().dtype(at::kByte));
   const float one = 1.f, beta = accumulate ? 1.f : 0.f;
-  const std::lock_guard<std::mutex> lock(g_blas_mutex);
   const void* bias_at = bias ? bias->data_ptr() : nullptr;
   if (bias) blas(hipblasLtMatmulDescSetAttribute(p.desc, HIPBLASLT_MATMUL_DESC_BIAS_POINTER, &bias_at, sizeof(bias_at)), "hipblasLtMatmulDescSetAttribute");
-  return hipblasLtMatmul(p.handle, p.desc, &one, b.t.data_ptr(), p.a, a.t.data_ptr(), p.b, &beta, d.t.data_ptr(), p.d, d.t.data_ptr(), p.d, &p.algo,
+  return hipblasLtMatmul(handle, p.desc, &one, b.t.data_ptr(), p.a, a.t.data_ptr(), p.b, &beta, d.t.data_ptr(), p.d, d.t.data_ptr(), p.d, &p.algo,
                          p.workspace > 0 ? ws.data_ptr() : nullptr, p.workspace, (hipStream_t)stream_of(on)) == HIPBLAS_STATUS_SUCCESS;
 }
 // The same product by torch, whose own route does not end at hipBLASLt.
@@ -249,9 +253,14 @@ PyObject* py_product(PyObject*, PyObject* const* x, Py_ssize_t n) {
   TORCH_CHECK_TYPE(n == 11, "product takes 11 arguments");
   const Mat a{tensor_arg(x[0], "a"), int_arg(x[1])}, b{tensor_arg(x[3], "b"), int_arg(x[4])}, d{tensor_arg(x[6], "d"), int_arg(x[7])};
   const OptTensor bias = opt_tensor_arg(x[8], "bias");
+  const bool trans_a = bool_arg(x[2]), trans_b = bool_arg(x[5]), accumulate = bool_arg(x[9]), library = bool_arg(x[10]);
   bool done = true;
-  if (bool_arg(x[10])) done = library_product(a, bool_arg(x[2]), b, bool_arg(x[5]), d, bias ? &*bias : nullptr, bool_arg(x[9]));
-  else torch_product(a, bool_arg(x[2]), b, bool_arg(x[5]), d, bias ? &*bias : nullptr, bool_arg(x[9]));
+  {
+    const NoGil released;
+    const c10::OptionalDeviceGuard guard(d.t.device());
+    if (library) done = library_product(a, trans_a, b, trans_b, d, bias ? &*bias : nullptr, accumulate);
+    else torch_product(a, trans_a, b, trans_b, d, bias ? &*bias : nullptr, accumulate);
+  }
   return PyBool_FromLong(done);
   END_HANDLE_TH_ERRORS
 }
@@ -260,7 +269,15 @@ PyObject* py_product(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_linear(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 4, "linear takes 4 arguments");
-  return THPVariable_Wrap(project(tensor_arg(x[0], "x"), tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), bool_arg(x[3])));
+  const Tensor &in = tensor_arg(x[0], "x"), &weight = tensor_arg(x[1], "weight");
+  const OptTensor bias = opt_tensor_arg(x[2], "bias");
+  const bool own = bool_arg(x[3]);
+  Tensor out;
+  {
+    const NoGil released;
+    out = project(in, weight, bias, own);
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 
@@ -286,9 +303,9 @@ const Lut& lut_for(int64_t buckets, int64_t max_relative, const Tensor& on) {
   {
     const pybind11::gil_scoped_acquire gil;  // taken without the mutex: another thread may hold the GIL and wait for the mutex
     PyObject* dev = THPDevice_New(on.device());
-    if (!dev) throw python_error();
+    if (!dev) throw_python();
     PyObject* r = PyObject_CallFunction(g_lut_source, "LLN", (long long)buckets, (long long)max_relative, dev);
-    if (!r) throw python_error();
+    if (!r) throw_python();
     lut = {THPVariable_Unpack(PyTuple_GET_ITEM(r, 0)), (int32_t)PyLong_AsLong(PyTuple_GET_ITEM(r, 1))};
     Py_DECREF(r);
   }
@@ -344,10 +361,12 @@ void launch_forward(fdb_attn_args& a, const Tensor& on, bool need_lse, const Fwd
       a.workspace_bytes = w.numel();
     }
   } else if (o.ask && a.cu_seqlens) {
+    const pybind11::gil_scoped_acquire gil;
     PyObject* r = PyObject_CallFunction(o.ask, "K", (unsigned long long)(uintptr_t)&a);
-    if (!r) throw python_error();
-    ws_bytes = int_arg(r);
+    if (!r) throw_python();
+    ws_bytes = PyLong_AsLongLong(r);
     Py_DECREF(r);
+    if (ws_bytes == -1 && PyErr_Occurred()) throw_python();
   } else {
     ws_bytes = fdb_attn_workspace_bytes(&a);
   }
@@ -502,7 +521,12 @@ PyObject* py_attention_fwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   o.no_alloc = bool_arg(x[23]);
   o.part = int_arg(x[24]);
   o.ask = x[25];
-  auto r = forward(tensor_arg(x[0], "q"), tensor_arg(x[1], "k"), tensor_arg(x[2], "v"), o);
+  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v");
+  std::pair<Tensor, Tensor> r;
+  {
+    const NoGil released;
+    r = forward(q, k, v, o);
+  }
   PyObject* out = nullptr;
   if (x[18] != Py_None) {
     out = x[18];
@@ -658,7 +682,12 @@ PyObject* py_attention_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
   o.far_splits = int_arg(x[12]);
   o.near_splits = int_arg(x[13]);
   o.workspace = opt_tensor_arg(x[14], "workspace");
-  return THPVariable_Wrap(AttentionNode::apply(q, k, v, *pk, *pq, (const Fwd*)&o));
+  Tensor out;
+  {
+    const NoGil released;
+    out = AttentionNode::apply(q, k, v, *pk, *pq, (const Fwd*)&o);
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 
@@ -668,31 +697,42 @@ PyObject* py_attention_bwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 14, "attention_bwd takes 14 arguments");
   const BwdSettings o{float_arg(x[8]), int_arg(x[9]), int_arg(x[10]), bool_arg(x[11]), opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
-  auto r = backward_of(tensor_arg(x[0], "q"), tensor_arg(x[1], "k"), tensor_arg(x[2], "v"), tensor_arg(x[3], "out"), tensor_arg(x[4], "lse"),
-                       tensor_arg(x[5], "dout"), tensor_arg(x[6], "pos_key"), tensor_arg(x[7], "pos_query"), o);
+  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v"), &out = tensor_arg(x[3], "out"), &lse = tensor_arg(x[4], "lse"),
+               &dout = tensor_arg(x[5], "dout"), &pk = tensor_arg(x[6], "pos_key"), &pq = tensor_arg(x[7], "pos_query");
+  std::array<Tensor, 5> r;
+  {
+    const NoGil released;
+    r = backward_of(q, k, v, out, lse, dout, pk, pq, o);
+  }
   PyObject* t = PyTuple_New(5);
   for (int i = 0; i < 5; ++i) PyTuple_SET_ITEM(t, i, THPVariable_Wrap(r[i]));
   return t;
   END_HANDLE_TH_ERRORS
 }
 
-// The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
 // x: pos_key, pos_query, heads, sm_scale, position_buckets, max_relative_positions, seq_start, seq_len
-Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, PyObject* const* x, bool own) {
+struct LayerCall {
+  Fwd o;
+  int64_t heads;
+  explicit LayerCall(PyObject* const* x) : heads(int_arg(x[2])) {
+    o.pos_key = opt_tensor_arg(x[0], "pos_key");
+    o.pos_query = opt_tensor_arg(x[1], "pos_query");
+    o.sm_scale = float_arg(x[3]);
+    o.buckets = int_arg(x[4]);
+    o.max_relative = int_arg(x[5]);
+    o.seq_start = opt_tensor_arg(x[6], "seq_start");
+    o.seq_len = opt_tensor_arg(x[7], "seq_len");
+  }
+};
+
+// The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
+Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, const LayerCall& call, bool own) {
   TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be [B, L, hidden]");
   const Tensor qkv = project(hidden, weight, bias, own);
   TORCH_CHECK(qkv.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", qkv.device());
   const auto type = qkv.scalar_type();
   TORCH_CHECK_VALUE(fdb_dtype_of(type) >= 0, "unsupported dtype ", type);
-  const int64_t B = qkv.size(0), L = qkv.size(1), H = int_arg(x[2]), D = qkv.size(2) / (3 * H), width = H * D;
-  Fwd o;
-  o.pos_key = opt_tensor_arg(x[0], "pos_key");
-  o.pos_query = opt_tensor_arg(x[1], "pos_query");
-  o.sm_scale = float_arg(x[3]);
-  o.buckets = int_arg(x[4]);
-  o.max_relative = int_arg(x[5]);
-  o.seq_start = opt_tensor_arg(x[6], "seq_start");
-  o.seq_len = opt_tensor_arg(x[7], "seq_len");
+  const int64_t B = qkv.size(0), L = qkv.size(1), H = call.heads, D = qkv.size(2) / (3 * H), width = H * D;
   const c10::hip::HIPGuard guard(qkv.get_device());
   const Tensor out = at::empty({B, L, width}, qkv.options());
   fdb_attn_args a = {};
@@ -705,7 +745,7 @@ Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTens
   a.q_stride_h = a.k_stride_h = a.v_stride_h = a.o_stride_h = D;
   a.o_stride_b = L * width, a.o_stride_t = width;
   a.batch = (int32_t)B, a.heads = (int32_t)H, a.head_dim = (int32_t)D, a.max_seqlen = (int32_t)L, a.total_tokens = (int32_t)(B * L);
-  run_forward(a, qkv, type, o);
+  run_forward(a, qkv, type, call.o);
   return out;
 }
 
@@ -822,7 +862,12 @@ PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
   if (t[0].dim() != 2 || t[0].size(0) < 2 * span || t[0].size(1) != C || W != 64 * a.heads || C % 8) Py_RETURN_NONE;
   for (int i = 1; i < 7; i += 2)
     if (t[i].dim() != 2 || t[i].size(0) != W || t[i].size(1) != C || t[i + 1].dim() != 1 || t[i + 1].size(0) != W) Py_RETURN_NONE;
-  return THPVariable_Wrap(LayerNode::apply(hidden, t[0], t[1], t[2], t[3], t[4], t[5], t[6], (const LayerArgs*)&a));
+  Tensor out;
+  {
+    const NoGil released;
+    out = LayerNode::apply(hidden, t[0], t[1], t[2], t[3], t[4], t[5], t[6], (const LayerArgs*)&a);
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 
@@ -831,7 +876,16 @@ PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 12, "layer_attention takes 12 arguments");
-  return THPVariable_Wrap(layer_attention(tensor_arg(x[0], "hidden"), tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), x + 3, bool_arg(x[11])));
+  const Tensor &hidden = tensor_arg(x[0], "hidden"), &weight = tensor_arg(x[1], "weight");
+  const OptTensor bias = opt_tensor_arg(x[2], "bias");
+  const LayerCall call(x + 3);
+  const bool own = bool_arg(x[11]);
+  Tensor out;
+  {
+    const NoGil released;
+    out = layer_attention(hidden, weight, bias, call, own);
+  }
+  return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
 
@@ -844,15 +898,32 @@ PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 23, "encoder_layer takes 23 arguments");
   const Tensor& hidden = tensor_arg(x[0], "hidden");
-  const auto norm = [](Tensor y, const Tensor& residual, PyObject* const* p) {
-    return at::layer_norm(y.add_(residual), {y.size(-1)}, tensor_arg(p[0], "norm_weight"), tensor_arg(p[1], "norm_bias"), float_arg(p[2]));
+  struct Norm {
+    const Tensor &weight, &bias;
+    double eps;
+    explicit Norm(PyObject* const* p) : weight(tensor_arg(p[0], "norm_weight")), bias(tensor_arg(p[1], "norm_bias")), eps(float_arg(p[2])) {}
+    Tensor operator()(Tensor y, const Tensor& residual) const { return at::layer_norm(y.add_(residual), {y.size(-1)}, weight, bias, eps); }
   };
-  const Tensor context = layer_attention(hidden, tensor_arg(x[1], "weight"), opt_tensor_arg(x[2], "bias"), x + 3, false);
-  const c10::hip::HIPGuard guard(hidden.get_device());
-  const Tensor attended = norm(project(context, tensor_arg(x[11], "out_weight"), opt_tensor_arg(x[12], "out_bias"), false), hidden, x + 13);
-  const Tensor up = project(attended, tensor_arg(x[16], "up_weight"), opt_tensor_arg(x[17], "up_bias"), false);
-  at::gelu_(const_cast<Tensor&>(up));
-  return THPVariable_Wrap(norm(project(up, tensor_arg(x[18], "down_weight"), opt_tensor_arg(x[19], "down_bias"), false), attended, x + 20));
+  struct Linear {
+    const Tensor& weight;
+    OptTensor bias;
+    explicit Linear(PyObject* const* p) : weight(tensor_arg(p[0], "weight")), bias(opt_tensor_arg(p[1], "bias")) {}
+    Tensor operator()(const Tensor& y) const { return project(y, weight, bias, false); }
+  };
+  const Linear in(x + 1), out(x + 11), up(x + 16), down(x + 18);
+  const LayerCall call(x + 3);
+  const Norm norm1(x + 13), norm2(x + 20);
+  Tensor next;
+  {
+    const NoGil released;
+    const Tensor context = layer_attention(hidden, in.weight, in.bias, call, false);
+    const c10::hip::HIPGuard guard(hidden.get_device());
+    const Tensor attended = norm1(out(context), hidden);
+    Tensor inner = up(attended);
+    at::gelu_(inner);
+    next = norm2(down(inner), attended);
+  }
+  return THPVariable_Wrap(std::move(next));
   END_HANDLE_TH_ERRORS
 }
 
@@ -869,26 +940,32 @@ PyObject* py_quantize(PyObject*, PyObject* const* x, Py_ssize_t n) {
     TORCH_CHECK_VALUE(t->is_cuda() && t->scalar_type() == at::kBFloat16, name, pair ? " expects bfloat16 GPU tensors" : " expects a bfloat16 GPU tensor");
   TORCH_CHECK_VALUE(a0.sizes() == a1.sizes(), name, ": shapes differ: ", a0.sizes(), " ", a1.sizes());
   const int64_t H = a0.size(-2), D = a0.size(-1);
-  Tensor r0 = a0.reshape({-1, H, D}), r1 = pair ? a1.reshape({-1, H, D}) : r0;
-  if (r0.strides() != r1.strides() || r0.stride(2) != 1) r0 = r0.contiguous(), r1 = r1.contiguous();
-  const c10::hip::HIPGuard guard(r0.get_device());
-  const int64_t tokens = r0.size(0), count = pair ? 2 : 1;
-  const Tensor y = at::empty({count, tokens, H, D}, r0.options().dtype(at::kFloat8_e4m3fn));
-  const Tensor scale = at::empty({count, H}, r0.options().dtype(at::kFloat));
-  const Tensor ws = at::empty({count * H}, r0.options().dtype(at::kInt));
-  char* y0 = (char*)y.data_ptr();
-  float* s0 = (float*)scale.data_ptr();
-  if (pair)
-    check(fdb_quant_e4m3_per_head_pair(r0.data_ptr(), r1.data_ptr(), r0.stride(0), r0.stride(1), y0, y0 + tokens * H * D, H * D, D, s0, s0 + H,
-                                       (uint32_t*)ws.data_ptr(), (int32_t)tokens, (int32_t)H, (int32_t)D, stream_of(r0)),
-          "fdb_quant_e4m3_per_head_pair");
-  else
-    check(fdb_quant_e4m3_per_head(r0.data_ptr(), r0.stride(0), r0.stride(1), y0, H * D, D, s0, (uint32_t*)ws.data_ptr(), (int32_t)tokens,
-                                  (int32_t)H, (int32_t)D, stream_of(r0)),
-          "fdb_quant_e4m3_per_head");
-  if (!pair) return Py_BuildValue("NN", THPVariable_Wrap(y.select(0, 0).reshape(a0.sizes())), THPVariable_Wrap(scale.select(0, 0)));
-  return Py_BuildValue("NNNN", THPVariable_Wrap(y.select(0, 0).reshape(a0.sizes())), THPVariable_Wrap(scale.select(0, 0)),
-                       THPVariable_Wrap(y.select(0, 1).reshape(a1.sizes())), THPVariable_Wrap(scale.select(0, 1)));
+  Tensor y0, y1, s0, s1;
+  {
+    const NoGil released;
+    Tensor r0 = a0.reshape({-1, H, D}), r1 = pair ? a1.reshape({-1, H, D}) : r0;
+    if (r0.strides() != r1.strides() || r0.stride(2) != 1) r0 = r0.contiguous(), r1 = r1.contiguous();
+    const c10::hip::HIPGuard guard(r0.get_device());
+    const int64_t tokens = r0.size(0), count = pair ? 2 : 1;
+    const Tensor y = at::empty({count, tokens, H, D}, r0.options().dtype(at::kFloat8_e4m3fn));
+    const Tensor scale = at::empty({count, H}, r0.options().dtype(at::kFloat));
+    const Tensor ws = at::empty({count * H}, r0.options().dtype(at::kInt));
+    char* y_at = (char*)y.data_ptr();
+    float* s_at = (float*)scale.data_ptr();
+    if (pair)
+      check(fdb_quant_e4m3_per_head_pair(r0.data_ptr(), r1.data_ptr(), r0.stride(0), r0.stride(1), y_at, y_at + tokens * H * D, H * D, D, s_at, s_at + H,
+                                         (uint32_t*)ws.data_ptr(), (int32_t)tokens, (int32_t)H, (int32_t)D, stream_of(r0)),
+            "fdb_quant_e4m3_per_head_pair");
+    else
+      check(fdb_quant_e4m3_per_head(r0.data_ptr(), r0.stride(0), r0.stride(1), y_at, H * D, D, s_at, (uint32_t*)ws.data_ptr(), (int32_t)tokens,
+                                    (int32_t)H, (int32_t)D, stream_of(r0)),
+            "fdb_quant_e4m3_per_head");
+    y0 = y.select(0, 0).reshape(a0.sizes()), s0 = scale.select(0, 0);
+    if (pair) y1 = y.select(0, 1).reshape(a1.sizes()), s1 = scale.select(0, 1);
+  }
+  if (!pair) return Py_BuildValue("NN", THPVariable_Wrap(std::move(y0)), THPVariable_Wrap(std::move(s0)));
+  return Py_BuildValue("NNNN", THPVariable_Wrap(std::move(y0)), THPVariable_Wrap(std::move(s0)), THPVariable_Wrap(std::move(y1)),
+                       THPVariable_Wrap(std::move(s1)));
   END_HANDLE_TH_ERRORS
 }
 
@@ -904,12 +981,17 @@ PyObject* py_mask_bounds(PyObject*, PyObject* const* x, Py_ssize_t n) {
   const int64_t B = m.size(0), L = m.size(-1);
   if (B < 1 || L < 1 || (m.dim() > 2 && m.size(-2) != L)) Py_RETURN_NONE;
   const int64_t step = m.stride(-1) + (m.dim() > 2 ? m.stride(-2) : 0);  // a square mask's diagonal says which tokens are real
-  const c10::hip::HIPGuard guard(m.get_device());
-  const Tensor out = at::empty({2, B}, m.options().dtype(at::kInt));
-  int32_t* p = (int32_t*)out.data_ptr();
-  check(fdb_mask_bounds(m.data_ptr(), (int32_t)m.element_size(), real ? 1 : 0, m.stride(0), step, (int32_t)B, (int32_t)L, p, p + B, stream_of(m)),
-        "fdb_mask_bounds");
-  return Py_BuildValue("NN", THPVariable_Wrap(out.select(0, 0)), THPVariable_Wrap(out.select(0, 1)));
+  Tensor start, length;
+  {
+    const NoGil released;
+    const c10::hip::HIPGuard guard(m.get_device());
+    const Tensor out = at::empty({2, B}, m.options().dtype(at::kInt));
+    int32_t* p = (int32_t*)out.data_ptr();
+    check(fdb_mask_bounds(m.data_ptr(), (int32_t)m.element_size(), real ? 1 : 0, m.stride(0), step, (int32_t)B, (int32_t)L, p, p + B, stream_of(m)),
+          "fdb_mask_bounds");
+    start = out.select(0, 0), length = out.select(0, 1);
+  }
+  return Py_BuildValue("NN", THPVariable_Wrap(std::move(start)), THPVariable_Wrap(std::move(length)));
   END_HANDLE_TH_ERRORS
 }
 

@@ -1,5 +1,7 @@
 """The native host path (csrc/fdb_torch.cpp) and the linear kernels (csrc/fdb_linear.hip): mask bounds against
 padding.seq_bounds, products against fp32 torch, the one-call encoder layer against the module-by-module one."""
+import sys
+import threading
 from types import SimpleNamespace
 
 import pytest
@@ -342,12 +344,71 @@ def test_operands_of_another_device_or_size_are_refused():
         _lib.native.attention_fwd(q, q.cpu(), q, pos, pos, None, None, 0.1, 32, 64, False, False, *([None] * 7), False, 0, 0, None, False, 0, None)
 
 
+def _lets_others_run(call):
+    """Whether another thread gets the interpreter during one of many calls.  Nobody asks for it back in the meantime (the switch
+    interval is longer than the test), so it does only if the call itself lets go."""
+    gate, ran = threading.Lock(), []
+    gate.acquire()
+    old = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    other = threading.Thread(target=lambda: gate.acquire() and ran.append(1))
+    other.start()
+    gate.release()
+    try:
+        for _ in range(3000):
+            call()
+            if ran:
+                return True
+        return False
+    finally:
+        sys.setswitchinterval(old)
+        other.join()
+
+
+def _refused(call):
+    def run():
+        try:
+            call()
+        except RuntimeError:
+            pass
+    return run
+
+
+def test_interpreter_lock_on_the_host():
+    """The entries whose first part runs on CPU tensors, too: a projection, and (refused after it) the layers around one."""
+    x, w, b = torch.randn(1, 64, 64), torch.randn(192, 64), torch.randn(192)
+    norm, square = (b[:64], b[:64], 1e-7), (w[:64], b[:64])
+    rest = (None, None, 1, 0.1, 0, 0, None, None)
+    assert not _lets_others_run(lambda: _lib.native.untouched((), ()))
+    assert _lets_others_run(lambda: _lib.native.linear(x, w, b, False))
+    assert _lets_others_run(_refused(lambda: _lib.native.layer_attention(x, w, b, *rest, False)))
+    assert _lets_others_run(_refused(lambda: _lib.native.encoder_layer(x, w, b, *rest, *square, *norm, *square, *square, *norm)))
+
+
+@pytest.mark.gpu
+def test_interpreter_lock_on_the_gpu():
+    from flashdeberta_amd import ops
+
+    g = lambda *s: torch.randn(*s, device="cuda").to(torch.bfloat16)
+    q, pos, mask = g(1, 40, 2, 64), g(2, 64, 64), torch.ones(2, 40, device="cuda")
+    kw = dict(position_buckets=32, max_relative_positions=64)
+    out, lse = ops.disentangled_attention_fwd(q, q, q, pos, pos, return_lse=True, **kw)
+    att, x, rel = _attention().train(), g(1, 40, 128), g(64, 128)
+    leaf = q.clone().requires_grad_()
+    cu = torch.tensor([0, 40], dtype=torch.int32, device="cuda")
+    for call in (lambda: ops.disentangled_attention_fwd(q, q, q, pos, pos, **kw),
+                 lambda: ops.disentangled_attention_fwd(q[0], q[0], q[0], pos, pos, cu_seqlens=cu, max_seqlen=40, **kw),   # asks Python on its way
+                 lambda: ops.disentangled_attention_bwd(q, q, q, out, lse, q, pos, pos, **kw), lambda: ops.disentangled_attention(leaf, q, q, pos, pos, **kw),
+                 lambda: att(x, None, rel_embeddings=rel), lambda: _lib.native.mask_bounds(mask), lambda: ops.quantize_e4m3_per_head(q),
+                 lambda: ops.quantize_e4m3_per_head_pair(q, q)):
+        assert _lets_others_run(call)
+        torch.cuda.synchronize()
+
+
 @pytest.mark.gpu
 def test_threads_share_the_plans():
     """Forward and backward of layers of many lengths from several threads: the products' plans are made, found and launched by
     these threads and by autograd's own, which do not hold the GIL."""
-    import threading
-
     att = _attention().train()
     rel = torch.randn(64, 128, device="cuda").to(torch.bfloat16)
     xs = [torch.randn(1, n, 128, device="cuda").to(torch.bfloat16).requires_grad_() for n in range(33, 53)]
