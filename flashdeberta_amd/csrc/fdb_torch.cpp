@@ -35,6 +35,8 @@ using at::Tensor;
 using OptTensor = std::optional<Tensor>;
 
 // ---- Python arguments -------------------------------------------------------------------------------------------
+// What an entry uses after it has let go of the interpreter's lock it holds by a reference of its own: another thread may put
+// another tensor into the Python object meanwhile.
 const Tensor& tensor_arg(PyObject* o, const char* name) {
   TORCH_CHECK_TYPE(THPVariable_Check(o), name, " must be a tensor");
   return THPVariable_Unpack(o);
@@ -251,7 +253,8 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
 PyObject* py_product(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 11, "product takes 11 arguments");
-  const Mat a{tensor_arg(x[0], "a"), int_arg(x[1])}, b{tensor_arg(x[3], "b"), int_arg(x[4])}, d{tensor_arg(x[6], "d"), int_arg(x[7])};
+  const Tensor ta = tensor_arg(x[0], "a"), tb = tensor_arg(x[3], "b"), td = tensor_arg(x[6], "d");
+  const Mat a{ta, int_arg(x[1])}, b{tb, int_arg(x[4])}, d{td, int_arg(x[7])};
   const OptTensor bias = opt_tensor_arg(x[8], "bias");
   const bool trans_a = bool_arg(x[2]), trans_b = bool_arg(x[5]), accumulate = bool_arg(x[9]), library = bool_arg(x[10]);
   bool done = true;
@@ -269,7 +272,7 @@ PyObject* py_product(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_linear(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 4, "linear takes 4 arguments");
-  const Tensor &in = tensor_arg(x[0], "x"), &weight = tensor_arg(x[1], "weight");
+  const Tensor in = tensor_arg(x[0], "x"), weight = tensor_arg(x[1], "weight");
   const OptTensor bias = opt_tensor_arg(x[2], "bias");
   const bool own = bool_arg(x[3]);
   Tensor out;
@@ -521,7 +524,7 @@ PyObject* py_attention_fwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   o.no_alloc = bool_arg(x[23]);
   o.part = int_arg(x[24]);
   o.ask = x[25];
-  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v");
+  const Tensor q = tensor_arg(x[0], "q"), k = tensor_arg(x[1], "k"), v = tensor_arg(x[2], "v");
   std::pair<Tensor, Tensor> r;
   {
     const NoGil released;
@@ -668,7 +671,7 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
 PyObject* py_attention_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 15, "attention_node takes 15 arguments");
-  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v");
+  const Tensor q = tensor_arg(x[0], "q"), k = tensor_arg(x[1], "k"), v = tensor_arg(x[2], "v");
   const OptTensor pk = opt_tensor_arg(x[3], "pos_key"), pq = opt_tensor_arg(x[4], "pos_query");
   if (!backward_in_tables(q, pk, pq)) Py_RETURN_NONE;
   Fwd o;
@@ -697,8 +700,8 @@ PyObject* py_attention_bwd(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 14, "attention_bwd takes 14 arguments");
   const BwdSettings o{float_arg(x[8]), int_arg(x[9]), int_arg(x[10]), bool_arg(x[11]), opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
-  const Tensor &q = tensor_arg(x[0], "q"), &k = tensor_arg(x[1], "k"), &v = tensor_arg(x[2], "v"), &out = tensor_arg(x[3], "out"), &lse = tensor_arg(x[4], "lse"),
-               &dout = tensor_arg(x[5], "dout"), &pk = tensor_arg(x[6], "pos_key"), &pq = tensor_arg(x[7], "pos_query");
+  const Tensor q = tensor_arg(x[0], "q"), k = tensor_arg(x[1], "k"), v = tensor_arg(x[2], "v"), out = tensor_arg(x[3], "out"), lse = tensor_arg(x[4], "lse"),
+               dout = tensor_arg(x[5], "dout"), pk = tensor_arg(x[6], "pos_key"), pq = tensor_arg(x[7], "pos_query");
   std::array<Tensor, 5> r;
   {
     const NoGil released;
@@ -846,7 +849,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
 PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 14, "layer_node takes 14 arguments");
-  const Tensor& hidden = tensor_arg(x[0], "hidden");
+  const Tensor hidden = tensor_arg(x[0], "hidden");
   LayerArgs a;
   a.heads = int_arg(x[8]);
   a.o = BwdSettings{float_arg(x[9]), int_arg(x[10]), int_arg(x[11]), false, opt_tensor_arg(x[12], "seq_start"), opt_tensor_arg(x[13], "seq_len")};
@@ -876,7 +879,7 @@ PyObject* py_layer_node(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 12, "layer_attention takes 12 arguments");
-  const Tensor &hidden = tensor_arg(x[0], "hidden"), &weight = tensor_arg(x[1], "weight");
+  const Tensor hidden = tensor_arg(x[0], "hidden"), weight = tensor_arg(x[1], "weight");
   const OptTensor bias = opt_tensor_arg(x[2], "bias");
   const LayerCall call(x + 3);
   const bool own = bool_arg(x[11]);
@@ -897,15 +900,15 @@ PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 23, "encoder_layer takes 23 arguments");
-  const Tensor& hidden = tensor_arg(x[0], "hidden");
+  const Tensor hidden = tensor_arg(x[0], "hidden");
   struct Norm {
-    const Tensor &weight, &bias;
+    const Tensor weight, bias;
     double eps;
     explicit Norm(PyObject* const* p) : weight(tensor_arg(p[0], "norm_weight")), bias(tensor_arg(p[1], "norm_bias")), eps(float_arg(p[2])) {}
     Tensor operator()(Tensor y, const Tensor& residual) const { return at::layer_norm(y.add_(residual), {y.size(-1)}, weight, bias, eps); }
   };
   struct Linear {
-    const Tensor& weight;
+    const Tensor weight;
     OptTensor bias;
     explicit Linear(PyObject* const* p) : weight(tensor_arg(p[0], "weight")), bias(opt_tensor_arg(p[1], "bias")) {}
     Tensor operator()(const Tensor& y) const { return project(y, weight, bias, false); }
@@ -933,7 +936,7 @@ PyObject* py_quantize(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 2, "quantize_e4m3 takes 2 arguments");
   const bool pair = x[1] != Py_None;
-  const Tensor& a0 = tensor_arg(x[0], "x0");
+  const Tensor a0 = tensor_arg(x[0], "x0");
   const Tensor a1 = pair ? tensor_arg(x[1], "x1") : a0;
   const char* name = pair ? "quantize_e4m3_per_head_pair" : "quantize_e4m3_per_head";
   for (const Tensor* t : {&a0, &a1})
@@ -975,7 +978,7 @@ PyObject* py_quantize(PyObject*, PyObject* const* x, Py_ssize_t n) {
 PyObject* py_mask_bounds(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK_TYPE(n == 1, "mask_bounds takes 1 argument");
-  const Tensor& m = tensor_arg(x[0], "mask");
+  const Tensor m = tensor_arg(x[0], "mask");
   const bool real = m.is_floating_point();
   if (!m.is_cuda() || m.is_complex() || m.dim() < 2 || m.dim() > 4 || (real && m.element_size() == 1)) Py_RETURN_NONE;
   const int64_t B = m.size(0), L = m.size(-1);
