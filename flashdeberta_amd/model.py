@@ -76,7 +76,7 @@ def _stands_in(modules, kinds):
 
 
 _PROJECTIONS = "query_proj", "key_proj", "value_proj", "pos_key_proj", "pos_query_proj"
-_PARTS = {n: (_LINEAR,) * n + (_DROPOUT,) for n in (3, 4, 5)}
+_PARTS = _LINEAR, _LINEAR, _LINEAR, _DROPOUT
 
 
 class FlashDisentangledSelfAttention(DisentangledSelfAttention):
@@ -108,13 +108,14 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
 
     def _plain_parts(self):
         """The same for all parts: the projections of the relative embeddings and their dropout among them."""
-        modules = self._modules
         if not self.relative_attention:
             return self._plain_projections()
-        parts = [modules[n] for n in ("query_proj", "key_proj", "value_proj")]
-        if not self.share_att_key:
-            parts += [modules[n] for n in ("pos_key_proj", "pos_query_proj") if n in modules]
-        return _stands_in((*parts, modules["pos_dropout"]), _PARTS[len(parts)])
+        modules = self._modules
+        parts = modules["query_proj"], modules["key_proj"], modules["value_proj"], modules["pos_dropout"]
+        if self.share_att_key:
+            return _stands_in(parts, _PARTS)
+        own = tuple(modules[n] for n in ("pos_key_proj", "pos_query_proj") if n in modules)
+        return _stands_in(parts + own, _PARTS + (_LINEAR,) * len(own))
 
     def _recording(self, *inputs):
         """Whether autograd records what is computed from these tensors and the projections' weights, the ones that are read: a
