@@ -21,9 +21,10 @@
 //       dK_r: dE_K[r] = sum_i G[i][r] q_i,   dQ_r: dE_Q[r] = sum_i G[i][r] k_(i-r),
 //     which fdb_table_grad_kernel accumulates over all tokens for its relative positions (the rows of G read back shifted
 //     against each other for the second one) and fdb_table_fold_kernel sums over the positions of a table row.
-// Against gathers from score tensors and score gradients collected per table row (fdb_bwd.hip), bf16, 12 heads:
-//   B = 8, L = 4096   dQ 1377 -> 1000 us, dK/dV 1553 -> 1230 us; score products, chain and transposes 600 -> 300 us (tables)
-//   B = 8, L = 512    68 + 66 -> 43 + 43 us; around them 90 -> 41 us
+// Against gathers from score tensors and score gradients collected per table row (fdb_bwd.hip), bf16, 12 heads, mean of a launch
+// (a box or its warmth moves these by up to 8 %):
+//   B = 8, L = 4096   dQ 1377 -> 956 us, dK/dV 1553 -> 1125 us; score products, chain and transposes 600 -> 309 us (tables)
+//   B = 8, L = 512    68 + 66 -> 83 us (both as one launch); around them 90 -> 46 us (row statistics, tables)
 // A near step is bound like the forward's by what its waves issue (with two waves per SIMD, one instruction per 4.5 clocks each)
 // next to its 28 (dQ) or 32 MFMAs; a far step by MFMA plus VALU time.
 //
