@@ -1047,6 +1047,10 @@ PyObject* py_untouched(PyObject*, PyObject* const* x, Py_ssize_t n) {
 // One remembered value, valid while the tensors it was computed from are the same objects, have not been written in place
 // (version counter), still sit in the same storage with the same dtype on the same device (`p.data = x` and `module.to(dtype)`
 // swap those under an unchanged object), and `extra` compares equal.  The tensors are held weakly.
+// A value belongs to the stream it was computed on, where whatever uses it, and whatever its memory is given to afterwards, comes
+// after it; each stream has its own, for the last few streams.  One that is recorded into a graph belongs to that capture: outside
+// it nothing has computed it yet, and a graph that took one from outside would keep, replay after replay, what followed from a mask
+// or a weight then, in memory that is given back once the program has changed either.
 struct Stamp {
   c10::weak_intrusive_ptr<c10::TensorImpl> impl;
   const void* data;
@@ -1054,11 +1058,26 @@ struct Stamp {
   at::ScalarType dtype;
   at::Device device;
 };
-struct MemoState {
+struct Place {
+  int64_t device = -1, stream = 0;
+  unsigned long long capture = 0;
+  bool operator==(const Place& o) const { return device == o.device && stream == o.stream && capture == o.capture; }
+};
+struct Remembered {
+  Place place;
   std::vector<Stamp> stamps;
   PyObject* extra = nullptr;
   PyObject* value = nullptr;
+  Remembered() = default;
+  Remembered(const Remembered&) = delete;
+  Remembered& operator=(const Remembered&) = delete;
+  ~Remembered() {
+    Py_XDECREF(extra);
+    Py_XDECREF(value);
+  }
 };
+typedef std::vector<std::shared_ptr<Remembered>> MemoState;   // the latest first
+constexpr size_t kMostStreams = 4;
 struct MemoObject {
   PyObject_HEAD
   MemoState* state;
@@ -1068,17 +1087,49 @@ bool tracked(const Tensor& t) { return t.defined() && !t.is_inference(); }  // i
 bool plain(const Tensor& t) { return t.has_storage(); }
 const void* address(const Tensor& t) { return plain(t) ? t.data_ptr() : nullptr; }
 
-void memo_clear(MemoState* s) {
-  s->stamps.clear();
-  Py_CLEAR(s->extra);
-  Py_CLEAR(s->value);
+Place place_of(PyObject* tensors) {
+  Place p;
+  if (PyTuple_GET_SIZE(tensors) == 0) return p;
+  const Tensor& t = tensor_arg(PyTuple_GET_ITEM(tensors, 0), "tensors");
+  if (!t.is_cuda()) return p;
+  const auto stream = c10::hip::getCurrentHIPStream(t.get_device());
+  p.device = t.get_device();
+  p.stream = stream.id();
+  if (p.stream != 0) {  // the default stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    const hipError_t e = hipStreamGetCaptureInfo(stream.stream(), &status, &id);
+    TORCH_CHECK(e == hipSuccess, "hipStreamGetCaptureInfo failed: ", hipGetErrorString(e));
+    if (status != hipStreamCaptureStatusNone) p.capture = id;
+  }
+  return p;
+}
+
+// values whose capture is over, or another one: moved out, to be given back when nothing here is being walked over
+MemoState drop_captures(MemoState& all, const Place& now) {
+  MemoState gone;
+  for (size_t i = all.size(); i-- > 0;)
+    if (all[i]->place.capture != 0 && all[i]->place.capture != now.capture) {
+      gone.push_back(std::move(all[i]));
+      all.erase(all.begin() + i);
+    }
+  return gone;
 }
 PyObject* memo_get(PyObject* self, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  MemoState* s = ((MemoObject*)self)->state;
+  MemoState& all = *((MemoObject*)self)->state;
   TORCH_CHECK_TYPE(n >= 1 && n <= 2 && PyTuple_Check(x[0]), "get(tensors, extra=None) takes a tuple of tensors");
+  if (all.empty()) Py_RETURN_NONE;
+  const Place now = place_of(x[0]);
+  const MemoState gone = drop_captures(all, now);
+  std::shared_ptr<Remembered> s;
+  for (const auto& r : all)
+    if (r->place == now) {
+      s = r;
+      break;
+    }
   const Py_ssize_t count = PyTuple_GET_SIZE(x[0]);
-  if (!s->value || (size_t)count != s->stamps.size()) Py_RETURN_NONE;
+  if (!s || (size_t)count != s->stamps.size()) Py_RETURN_NONE;
   PyObject* extra = n > 1 ? x[1] : Py_None;
   if (extra != s->extra) {
     const int same = PyObject_RichCompareBool(extra, s->extra, Py_EQ);
@@ -1098,23 +1149,31 @@ PyObject* memo_get(PyObject* self, PyObject* const* x, Py_ssize_t n) {
 }
 PyObject* memo_put(PyObject* self, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  MemoState* s = ((MemoObject*)self)->state;
   TORCH_CHECK_TYPE(n >= 2 && n <= 3 && PyTuple_Check(x[0]), "put(tensors, value, extra=None) takes a tuple of tensors");
   const Py_ssize_t count = PyTuple_GET_SIZE(x[0]);
-  std::vector<Stamp> stamps;
-  bool all = true;
-  for (Py_ssize_t i = 0; i < count && all; ++i) {
+  const auto fresh = std::make_shared<Remembered>();
+  fresh->place = place_of(x[0]);
+  bool all_tracked = true;
+  for (Py_ssize_t i = 0; i < count && all_tracked; ++i) {
     const Tensor& t = tensor_arg(PyTuple_GET_ITEM(x[0], i), "tensors");
-    all = tracked(t);
-    if (all) stamps.push_back(Stamp{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), address(t), (int64_t)t._version(), t.scalar_type(), t.device()});
+    all_tracked = tracked(t);
+    if (all_tracked) fresh->stamps.push_back(Stamp{c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr()), address(t), (int64_t)t._version(), t.scalar_type(), t.device()});
   }
-  memo_clear(s);
-  if (all) {
-    s->stamps = std::move(stamps);
-    s->extra = n > 2 ? x[2] : Py_None;
-    Py_INCREF(s->extra);
-    s->value = x[1];
-    Py_INCREF(s->value);
+  MemoState& all = *((MemoObject*)self)->state;
+  MemoState gone = drop_captures(all, fresh->place);
+  for (size_t i = all.size(); i-- > 0;)
+    if (all[i]->place == fresh->place) {
+      gone.push_back(std::move(all[i]));
+      all.erase(all.begin() + i);
+    }
+  if (all_tracked) {
+    Py_INCREF(fresh->extra = n > 2 ? x[2] : Py_None);
+    Py_INCREF(fresh->value = x[1]);
+    all.insert(all.begin(), fresh);
+    if (all.size() > kMostStreams) {
+      gone.push_back(std::move(all.back()));
+      all.pop_back();
+    }
   }
   Py_INCREF(x[1]);
   return x[1];
@@ -1129,16 +1188,18 @@ PyObject* memo_new(PyTypeObject* type, PyObject*, PyObject*) {
   return (PyObject*)m;
 }
 int memo_traverse(PyObject* self, visitproc visit, void* arg) {
-  MemoState* s = ((MemoObject*)self)->state;
-  if (s) {
-    Py_VISIT(s->extra);
-    Py_VISIT(s->value);
-  }
+  const MemoState* all = ((MemoObject*)self)->state;
+  if (all)
+    for (const auto& r : *all) {
+      if (r.use_count() > 1) continue;   // a call that is running holds it, too
+      Py_VISIT(r->extra);
+      Py_VISIT(r->value);
+    }
   return 0;
 }
 int memo_gc_clear(PyObject* self) {
-  MemoState* s = ((MemoObject*)self)->state;
-  if (s) memo_clear(s);
+  MemoState gone;
+  if (MemoState* all = ((MemoObject*)self)->state) gone.swap(*all);
   return 0;
 }
 void memo_dealloc(PyObject* self) {
@@ -1178,7 +1239,7 @@ PyMODINIT_FUNC PyInit__native(void) {
   MemoType.tp_name = "flashdeberta_amd._native.Memo";
   MemoType.tp_basicsize = sizeof(MemoObject);
   MemoType.tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC;
-  MemoType.tp_doc = "One remembered value, valid while the tensors it was computed from are unchanged.";
+  MemoType.tp_doc = "One remembered value, valid while the tensors it was computed from are unchanged, on the stream it was computed on.";
   MemoType.tp_new = memo_new;
   MemoType.tp_traverse = memo_traverse;
   MemoType.tp_clear = memo_gc_clear;

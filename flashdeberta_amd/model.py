@@ -34,7 +34,8 @@ from .padding import key_padding_mask, seq_bounds
 
 # One remembered value, valid while the tensors it was computed from are the same objects, have not been written in
 # place, still sit in the same storage with the same dtype on the same device, and `extra` compares equal; the tensors
-# are held weakly: get(tensors, extra=None), put(tensors, value, extra=None).
+# are held weakly: get(tensors, extra=None), put(tensors, value, extra=None).  Each of the last four streams has its own, and
+# so has a graph that is being recorded: it computes what it needs anew, from the masks and weights as they are at a replay.
 _Memo = native.Memo
 
 
@@ -87,7 +88,7 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     absmax scales before the kernel (bf16 inputs only).
 
     Outside training the three input projections run as one GEMM over the concatenated weights
-    (a copy kept per module, rebuilt when a parameter is replaced or written in place), and K_r / Q_r
+    (a copy kept per module and stream, rebuilt when a parameter is replaced or written in place), and K_r / Q_r
     are remembered for as long as the relative embeddings handed in are the same tensor (an encoder
     patched by `patch_model` hands in the same tensor until its embedding table changes); both only
     while the projections are plain linear layers that nobody has hooked or given another forward."""

@@ -314,6 +314,73 @@ def _attention(device="cuda", hidden_dropout_prob=0.0, share_att_key=True, **kw)
 
 
 @pytest.mark.gpu
+def test_remembered_values_stay_on_their_stream():
+    att = _attention().eval()
+    rel, mask = torch.randn(64, 128, device="cuda").to(torch.bfloat16), torch.ones(2, 40, device="cuda")
+    remembered = lambda: (att._fused_qkv()[0], att._pos_layers(rel)[0], att._bounds(mask)[1])
+    same = lambda a, b: [x is y for x, y in zip(a, b)] == [True] * 3
+    streams = [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(6)]
+    torch.cuda.synchronize()
+    with torch.no_grad():
+        seen = []
+        for stream in streams[:4]:
+            with torch.cuda.stream(stream):
+                seen.append(remembered())
+                assert same(remembered(), seen[-1])
+        assert all(not any(x is y for x, y in zip(a, b)) for i, a in enumerate(seen) for b in seen[:i])
+        for stream, values in zip(streams, seen):   # taking turns, each stream finds its own
+            with torch.cuda.stream(stream):
+                assert same(remembered(), values)
+        for stream in streams[4:]:   # no more than a few are kept
+            with torch.cuda.stream(stream):
+                remembered()
+        assert not any(x is y for x, y in zip(remembered(), seen[0]))
+        torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_captured_encoder_follows_its_mask_and_weights():
+    """A graph recorded after eager calls on the same mask and weights: replays see what has been written into either since, and eager
+    calls between them do not take what only a replay computes."""
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
+
+    torch.manual_seed(11)
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=128, num_hidden_layers=2, num_attention_heads=2, intermediate_size=256, relative_attention=True,
+                          pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True, norm_rel_ebd="layer_norm",
+                          position_biased_input=False, initializer_range=0.2)
+    net = FlashDebertaV2Model(cfg).eval().cuda().to(torch.bfloat16)
+    ids = torch.randint(0, 100, (3, 50), device="cuda")
+    lengths = lambda *n: (torch.arange(50, device="cuda") < torch.tensor(n, device="cuda")[:, None]).long()
+    mask = lengths(50, 40, 30)
+    call = lambda m: net(input_ids=ids, attention_mask=m).last_hidden_state
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            call(mask)
+        torch.cuda.current_stream().wait_stream(side)
+        call(mask)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            captured = call(mask)
+        with torch.cuda.stream(side):   # the stream of the capture, which has not computed anything yet
+            assert torch.isfinite(call(mask)).all()
+        torch.cuda.synchronize()
+        layer = net.encoder.layer[1].attention.self
+        for step, n in enumerate(((50, 40, 30), (20, 50, 1), (7, 8, 50))):
+            mask.copy_(lengths(*n))
+            ids.copy_(torch.randint(0, 100, (3, 50), device="cuda"))
+            if step == 2:
+                layer.key_proj.weight.mul_(-1.5)
+                net.encoder.rel_embeddings.weight.mul_(0.5)
+            ref = call(lengths(*n))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(captured, ref), step
+            assert torch.equal(call(mask), ref)
+
+
+@pytest.mark.gpu
 def test_projection_whose_weight_is_no_parameter():
     """Pruning leaves `weight` an attribute beside the parameter `weight_orig`."""
     from torch.nn.utils import prune
