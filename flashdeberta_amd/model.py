@@ -10,6 +10,7 @@ here); attention-probability dropout is not applied (nor is it on the reference'
 on the relative embeddings remains, model.py:159-160).
 """
 import math
+import threading
 
 import torch
 import torch.nn.functional as F
@@ -66,7 +67,7 @@ def _kind(cls):
     return cls, cls.forward
 
 
-_LINEAR, _DROPOUT = _kind(torch.nn.Linear), _kind(torch.nn.Dropout)
+_LINEAR, _LAYER_NORM, _DROPOUT = _kind(torch.nn.Linear), _kind(torch.nn.LayerNorm), _kind(torch.nn.Dropout)
 
 
 def _stands_in(modules, kinds):
@@ -297,7 +298,7 @@ DEBERTA_SELF_ATTENTION_CLASSES = {
 
 # the parts of a layer that its one native call takes the place of, in the order FlashDebertaV2Layer._native_args names them
 _LAYER_PARTS = (*(_kind(c) for c in (DebertaV2Attention, DebertaV2Intermediate, DebertaV2Output, FlashDisentangledSelfAttention, DebertaV2SelfOutput,
-                                     GELUActivation)), *(_LINEAR,) * 3, *(_kind(torch.nn.LayerNorm),) * 2, *(_DROPOUT,) * 2)
+                                     GELUActivation)), *(_LINEAR,) * 3, *(_LAYER_NORM,) * 2, *(_DROPOUT,) * 2)
 
 
 class FlashDebertaV2Layer(DebertaV2Layer):
@@ -347,15 +348,27 @@ class FlashDebertaV2Layer(DebertaV2Layer):
                                rel_embeddings=rel_embeddings, output_attentions=output_attentions)
 
 
+_forwarding = threading.local()   # the encoder whose forward this thread is in
+
+
 class FlashDebertaV2Encoder(DebertaV2Encoder):
     """transformers' encoder minus work the fused attention never reads: with `_fdb_skip_dense` it builds
     neither the [1, L, L] int64 relative-position tensor nor the [B, 1, L, L] mask (transformers
     modeling_deberta_v2.py:601-626), and outside training it hands the layers one relative-embedding tensor
     object for as long as the table and its LayerNorm are unchanged, so that each layer's K_r / Q_r stay
-    valid from forward to forward.  Instances are made by `patch_model`, which switches the class of an
+    valid from forward to forward.  A forward that autograd records (an eval model that is fine-tuned) computes
+    the tensor with its graph, each time.  Instances are made by `patch_model`, which switches the class of an
     existing encoder."""
 
     _fdb_skip_dense = True
+
+    def forward(self, *args, **kwargs):
+        outer = getattr(_forwarding, "encoder", None)
+        _forwarding.encoder = self
+        try:
+            return super().forward(*args, **kwargs)
+        finally:
+            _forwarding.encoder = outer
 
     def get_rel_pos(self, hidden_states, query_states=None, relative_pos=None):
         if self._fdb_skip_dense:
@@ -374,7 +387,10 @@ class FlashDebertaV2Encoder(DebertaV2Encoder):
         if memo is None:
             memo = self._fdb_rel_memo = _Memo()
         norm = self.LayerNorm if "layer_norm" in self.norm_rel_ebd else None
-        key = (self.rel_embeddings.weight,) + (tuple(norm.parameters()) if norm is not None else ())
+        key = (self.rel_embeddings.weight,) + (() if norm is None else tuple(p for p in (norm.weight, norm.bias) if p is not None))
+        recorded = getattr(_forwarding, "encoder", None) is self and torch.is_grad_enabled() and any(p.requires_grad for p in key)
+        if recorded or not (norm is None or _stands_in((norm,), (_LAYER_NORM,))):
+            return super().get_rel_embedding()
         hit = memo.get(key)
         if hit is None:
             with torch.no_grad():

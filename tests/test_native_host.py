@@ -291,6 +291,59 @@ def test_weights_that_are_no_parameters_are_recorded(share):
         p.requires_grad_(False)
 
 
+@pytest.mark.parametrize("norm", ["layer_norm", "none"])
+def test_relative_embeddings_of_a_recorded_forward_carry_their_graph(norm):
+    """Fine-tuning an eval model: what the encoder hands to its layers leads back to the table and its norm, also of a replica."""
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
+
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=128, num_hidden_layers=1, num_attention_heads=2, intermediate_size=256, relative_attention=True,
+                          pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True, norm_rel_ebd=norm)
+    encoder = FlashDebertaV2Model(cfg).eval().encoder
+    seen = []
+
+    class Layer(torch.nn.Module):
+        def forward(self, hidden_states, attention_mask, rel_embeddings=None, **kwargs):
+            seen.append(rel_embeddings)
+            return hidden_states, None
+
+    encoder.layer = torch.nn.ModuleList([Layer()])
+    x, mask = torch.randn(1, 8, 128), torch.ones(1, 8)
+    run = lambda e: e(x, mask) and seen.pop()
+    leaves = [encoder.rel_embeddings.weight] + ([encoder.LayerNorm.weight, encoder.LayerNorm.bias] if norm == "layer_norm" else [])
+    for _ in range(2):
+        assert all(g is not None for g in torch.autograd.grad(run(encoder).sum(), leaves, allow_unused=True))
+    assert all(g is not None for g in torch.autograd.grad(run(_replica(encoder)).sum(), leaves, allow_unused=True))
+    with torch.no_grad():
+        assert run(encoder) is run(encoder)
+    for p in leaves:
+        p.requires_grad_(False)
+    assert run(encoder) is run(encoder) and not run(encoder).requires_grad
+    if norm == "layer_norm":
+        for _ in _changes(encoder.LayerNorm):
+            assert run(encoder) is not run(encoder)
+
+
+@pytest.mark.gpu
+def test_gradients_of_an_eval_model_are_those_of_training_without_dropout():
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
+
+    torch.manual_seed(13)
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=128, num_hidden_layers=2, num_attention_heads=2, intermediate_size=256, relative_attention=True,
+                          pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True, norm_rel_ebd="layer_norm",
+                          position_biased_input=False, hidden_dropout_prob=0.0, attention_probs_dropout_prob=0.0)
+    net = FlashDebertaV2Model(cfg).cuda().to(torch.bfloat16)
+    ids, mask = torch.randint(0, 100, (2, 60), device="cuda"), torch.ones(2, 60, device="cuda", dtype=torch.long)
+    mask[1, 40:] = 0
+    names, leaves = zip(*[(n, p) for n, p in net.named_parameters() if p.requires_grad])
+    got = []
+    for mode in (True, False, False):
+        out = net.train(mode)(input_ids=ids, attention_mask=mask).last_hidden_state
+        got.append(torch.autograd.grad((out * mask[:, :, None]).float().square().sum(), leaves, allow_unused=True))
+    for name, a, *rest in zip(names, *got):
+        assert all(torch.equal(a, b) if a is not None else b is None for b in rest), name
+        assert a is not None or "rel_embeddings" not in name
+
+
 @pytest.mark.gpu
 def test_dropout_kept_on_in_an_eval_model():
     layer = _encoder_layer(0.5).cuda()
