@@ -132,7 +132,9 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         """Concatenated [3*H*D, hidden] weight and bias of the query, key and value projections (plain ones), None where only
         some have a bias."""
         modules = self._modules
-        (qw, qb), (kw, kb), (vw, vb) = [_weight_and_bias(modules[n]) for n in ("query_proj", "key_proj", "value_proj")]
+        qw, qb = _weight_and_bias(modules["query_proj"])
+        kw, kb = _weight_and_bias(modules["key_proj"])
+        vw, vb = _weight_and_bias(modules["value_proj"])
         with_bias = qb is not None and kb is not None and vb is not None
         if not with_bias and not (qb is None and kb is None and vb is None):
             return None
@@ -161,8 +163,8 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
     def _pos_layers(self, rel_embeddings, plain=False, dropped=None):
         """K_r, Q_r as [H, 2S, D] views of the projected relative embeddings
         (reference model.py:159-177; the slice to 2S rows is transformers modeling_deberta_v2.py:295).
-        plain: the caller knows that nobody has touched the parts and that nothing is recorded; dropped: what pos_dropout gave for these embeddings, if the
-        caller has called it."""
+        plain: the caller knows that nobody has touched the parts and that nothing is recorded; dropped: what pos_dropout
+        gave for these embeddings, if the caller has called it."""
         if not self.relative_attention or rel_embeddings is None:
             return None, None
         # the position projections exist only for the terms the module has (transformers :170-178)
@@ -176,8 +178,12 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         dropout = modules["pos_dropout"]
         # a remembered K_r / Q_r must not carry an autograd graph, and depends on nothing but the embeddings and the weights
         if not self.training and (plain or self._plain_parts() and not self._recording(rel_embeddings)) and not (dropout.training and dropout.p > 0.0):
-            key = (rel_embeddings,) + tuple(p for m in (kproj, qproj) if m is not None for p in _weight_and_bias(m) if p is not None)
-            hit = self._pos_memo.get(key, tuple(self.pos_att_type))
+            key, terms = (rel_embeddings,), tuple(self.pos_att_type)
+            for m in (kproj, qproj):
+                if m is not None:
+                    weight, bias = _weight_and_bias(m)
+                    key += (weight, bias) if bias is not None else (weight,)
+            hit = self._pos_memo.get(key, terms)
             if hit is not None:
                 return hit
         H, D = self.num_attention_heads, self.attention_head_size
@@ -190,7 +196,7 @@ class FlashDisentangledSelfAttention(DisentangledSelfAttention):
         pos_key = heads(kproj(rel)) if kproj is not None else None
         pos_query = heads(qproj(rel)) if qproj is not None else None
         if key is not None:
-            self._pos_memo.put(key, (pos_key, pos_query), tuple(self.pos_att_type))
+            self._pos_memo.put(key, (pos_key, pos_query), terms)
         return pos_key, pos_query
 
     def _score_settings(self, pos_key, pos_query):
