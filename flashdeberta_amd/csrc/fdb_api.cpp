@@ -714,7 +714,23 @@ int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_
       (rows + 15) / 16 > 65535)
     return FDB_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || (reinterpret_cast<uintptr_t>(bias) & 1u)) return FDB_ERR_ALIGN;
+  if (rows > 32 && fdb_gemm(x, w, bias, nullptr, out, rows, cols, depth, ldx, ldw, ldo, 0, FDB_GEMM_PLAIN, dtype, stream) == FDB_OK) return FDB_OK;
   return fdb_launch_linear(x, w, bias, out, rows, cols, depth, ldx, ldw, ldo, dtype, stream);
+}
+
+int fdb_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t rows, int32_t cols, int32_t depth, int64_t ldx,
+             int64_t ldw, int64_t ldo, int64_t ldr, int32_t epilogue, int32_t dtype, void* stream) {
+  const bool added = epilogue == FDB_GEMM_RESIDUAL;
+  if (!x || !w || !out || (added && !residual)) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  if (epilogue < FDB_GEMM_PLAIN || epilogue > FDB_GEMM_RESIDUAL) return FDB_ERR_UNSUPPORTED;
+  if (rows < 1 || cols < 8 || depth < 64 || cols % 8 || depth % 64 || ldx < depth || ldw < depth || ldo < cols || (added && ldr < cols) ||
+      rows > (1 << 24) || cols > (1 << 24) || ldx > (1 << 22) || ldw > (1 << 22))  // 256 rows of x and of w within a lane's 32-bit offset
+    return FDB_ERR_SHAPE;
+  if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || ldo % 8 || (added && (!aligned16(residual) || ldr % 8)) ||
+      (reinterpret_cast<uintptr_t>(bias) & 7u))
+    return FDB_ERR_ALIGN;
+  return fdb_launch_gemm(x, w, bias, residual, out, rows, cols, depth, ldx, ldw, ldo, ldr, epilogue, dtype, stream);
 }
 
 int32_t fdb_delta_lut_radius(int32_t position_buckets, int32_t max_position) {

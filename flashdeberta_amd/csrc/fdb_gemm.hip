@@ -1,0 +1,248 @@
+// Products of more rows than fdb_linear.hip streams, for the layers around the attention: out = epilogue(x . w^T + bias), 16-bit types.
+//
+// hipBLASLt does the plain product as fast; what is gained is what follows it.  An encoder layer adds the residual to two of its products
+// and takes the GELU of a third, each a pass of its own over memory that is as long as a tenth of the layer.  Here these happen on the
+// tile that is being written.  [4096 rows, bf16, on the GPU alone, in a replayed graph; product and pass by torch -> here]
+//   768 -> 768 + residual 17.0 -> 9.8 us,  768 -> 3072 + GELU 37.8 -> 27.7,  3072 -> 768 + residual 30.6 -> 26.9;
+// with 1500 rows 11.6 -> 7.3, 22.1 -> 16.2 and 21.7 -> 18.3.
+//
+// The sums run over the contraction in order, 32 at a time, in one accumulator, and are rounded where torch's separate passes round:
+// the bits are those of torch's product, GELU and addition (where the library does not split the contraction).
+//
+// What bounds it (4096 x 3072 x 768, tile 256 x 192, 22.7 us without an epilogue): with the loads of its stages left out 19.1, with the products
+// alone 21.2, with neither 11.9 (launch, first loads, operands, 25 MB of results): the matrix cores, whose clock falls under such operands to
+// the rate of a large library product, plus a start and an end that one round of workgroups does not overlap with them.  Measured
+// and no faster: operands read a stage ahead into registers, loads issued between the products instead of ahead of them, more
+// stages, rows padded against a stride of whole channels.  GELU through erff instead of the table: 35 us instead of 27.7.
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include <atomic>
+
+#include "fdb_device.h"
+#include "fdb_kernels.h"
+#include "../../include/fdb.h"
+
+using namespace fdb;
+
+namespace {
+
+__device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+
+// GELU of a 16-bit value, rounded to its type, as torch's elementwise kernel computes it.  erff and what goes with it are some 45 vector
+// instructions an element and no memory time hides them here; a bf16 has so few values that matter (2^-14 <= |x| < 8: 17 binades of 128
+// and a sign) that each workgroup tabulates them while its first tiles are on their way, and looks the others up.
+__device__ __forceinline__ float gelu(float x) { return x * 0.5f * (1.f + erff(x * 0.70710678118654752440f)); }
+constexpr uint32_t kGeluLow = (127 - 14) << 7, kGeluHigh = (127 + 3) << 7, kGeluCount = kGeluHigh - kGeluLow;   // bit patterns of bf16 magnitudes
+constexpr int kGeluBytes = 2 * kGeluCount * 2;   // [sign][magnitude - low]
+
+enum { kPlain = FDB_GEMM_PLAIN, kGelu = FDB_GEMM_GELU, kResidual = FDB_GEMM_RESIDUAL };   // out = y, gelu(y) or y + residual, y = x . w^T + bias rounded to the type
+
+struct GemmParams {
+  const char *x, *w, *bias, *residual;
+  char* out;
+  int64_t ldx, ldw, ldo, ldr;   // elements
+  int32_t M, N, K, tiles_n, tiles;
+};
+
+// A workgroup of WM x WN waves makes TM x TN outputs, PER_CU of them share a CU; stages of kDepth of the contraction go straight from global
+// memory into one of STAGES LDS buffers, rows of 128 bytes, slot (row, s) = chunk s ^ swz(row) (sixteen rows' same chunk: sixteen bank groups).
+constexpr int kDepth = 64;
+__device__ __forceinline__ int swz(int row) { return 4 * ((row >> 1) & 1) | (-(row >> 2) & 3); }
+
+template <int TM_, int TN_, int WM_, int WN_, int STAGES_, int PER_CU_>
+struct GemmShape {
+  static constexpr int TM = TM_, TN = TN_, WM = WM_, WN = WN_, STAGES = STAGES_, PER_CU = PER_CU_;
+  static constexpr int NW = WM * WN, FM = TM / (16 * WM), FN = TN / (16 * WN);
+  static constexpr int ROWB = 2 * kDepth, RPI = 1024 / ROWB;   // bytes of a row, rows a wave's load fills
+  static constexpr int XI = TM / RPI, WI = TN / RPI, LOADS = (XI + WI) / NW;
+  static constexpr int STAGE = (TM + TN) * ROWB, PITCH = TN * 2 + 16;
+  static constexpr int TILES = STAGES * STAGE > TM * PITCH ? STAGES * STAGE : TM * PITCH;
+  static constexpr int lds_bytes(bool table) { return TILES + (table ? kGeluBytes : 0); }
+  static_assert(PER_CU * TILES <= 160 * 1024, "LDS budget");   // a workgroup with a table may be alone with one fewer
+  static_assert(TM % (16 * WM) == 0 && TN % (16 * WN) == 0 && TM % RPI == 0 && TN % RPI == 0 && (XI + WI) % NW == 0, "whole fragments, whole loads");
+};
+
+template <class QT, int EPI, class S>
+__global__ __launch_bounds__(64 * S::NW, S::PER_CU * S::NW / 4) void fdb_gemm_kernel(const GemmParams p) {
+  constexpr int TM = S::TM, TN = S::TN, STAGES = S::STAGES;
+  using frag = typename QT::frag;
+  using elem = typename QT::scratch_t;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, kg = lane >> 4;
+  const int wm = wave / S::WN, wn = wave % S::WN;
+  // every XCD takes a run of tiles, whose rows of x and w then pass through one L2
+  const int n = blockIdx.x, xcd = n & 7, each = p.tiles >> 3, more = p.tiles & 7;
+  const int tile = xcd * each + min(xcd, more) + (n >> 3);
+  const int tm = tile / p.tiles_n, tn = tile - tm * p.tiles_n;
+  const int m0 = tm * TM, n0 = tn * TN;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_AS char*)smem;
+  const char* xb = p.x + (int64_t)m0 * p.ldx * 2;
+  const char* wb = p.w + (int64_t)n0 * p.ldw * 2;
+  uint32_t off[S::LOADS];
+#pragma unroll
+  for (int j = 0; j < S::LOADS; ++j) {
+    const int c = wave + S::NW * j, row = c * S::RPI + (lane >> 3);   // rows past the end re-read the last one
+    const uint32_t chunk = (uint32_t)(((lane & 7) ^ swz(row)) * 16);
+    if (c < S::XI) off[j] = (uint32_t)(min(m0 + row, p.M - 1) - m0) * (uint32_t)(p.ldx * 2) + chunk;
+    else off[j] = (uint32_t)(min(n0 + row - TM, p.N - 1) - n0) * (uint32_t)(p.ldw * 2) + chunk;
+  }
+  auto fill = [&](int t, int buf) __attribute__((always_inline)) {
+    const uint32_t dst = lds0 + (uint32_t)buf * S::STAGE + (uint32_t)wave * 1024u;
+#pragma unroll
+    for (int j = 0; j < S::LOADS; ++j)
+      dma16sn((wave + S::NW * j < S::XI ? xb : wb) + (int64_t)t * S::ROWB, off[j], dst + j * S::NW * 1024u);
+  };
+  f32x4 acc[S::FM][S::FN];
+#pragma unroll
+  for (int i = 0; i < S::FM; ++i)
+#pragma unroll
+    for (int j = 0; j < S::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = p.K / kDepth;
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t)
+    if (t < steps) fill(t, t);
+  constexpr bool TABLE = EPI == kGelu && std::is_same<QT, Bf16Tr>::value;
+  if constexpr (TABLE) {
+    uint16_t* table = (uint16_t*)(smem + S::TILES);
+    for (uint32_t e = tid; e < kGeluCount; e += 64 * S::NW) {
+      const float v = __builtin_bit_cast(float, (kGeluLow + e) << 16), t = erff(v * 0.70710678118654752440f);
+      ((__bf16*)table)[e] = (__bf16)(v * 0.5f * (1.f + t));
+      ((__bf16*)table)[kGeluCount + e] = (__bf16)(-v * 0.5f * (1.f - t));
+    }
+  }
+  const uint32_t xrow = (uint32_t)((wm * S::FM * 16 + r) * S::ROWB), wrow = (uint32_t)((TM + wn * S::FN * 16 + r) * S::ROWB), f = (uint32_t)swz(r);
+  int buf = 0;
+#pragma unroll 1
+  for (int t = 0; t < steps; ++t) {
+    // this wave's loads of stage t have landed, those of the STAGES - 2 after it may still fly
+    if (t + STAGES - 1 <= steps) wait_vmcnt<(STAGES - 2) * S::LOADS>();
+    else wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();   // ... and everybody's; everybody has read the buffer of stage t - 1
+    asm volatile("" ::: "memory");
+    if (t + STAGES - 1 < steps) fill(t + STAGES - 1, buf == 0 ? STAGES - 1 : buf - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t at = lds0 + (uint32_t)buf * S::STAGE;
+#pragma unroll
+    for (int s = 0; s < kDepth / 32; ++s) {
+      frag xf[S::FM], wf[S::FN];
+      const uint32_t slot = ((uint32_t)(4 * s + kg) ^ f) * 16;
+#pragma unroll
+      for (int j = 0; j < S::FN; ++j) wf[j] = *(LDS_AS const frag*)(uintptr_t)(at + wrow + slot + j * 16 * S::ROWB);
+#pragma unroll
+      for (int i = 0; i < S::FM; ++i) xf[i] = *(LDS_AS const frag*)(uintptr_t)(at + xrow + slot + i * 16 * S::ROWB);
+#pragma unroll
+      for (int i = 0; i < S::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < S::FN; ++j) acc[i][j] = mma16(wf[j], xf[i], acc[i][j]);
+    }
+    buf = buf == STAGES - 1 ? 0 : buf + 1;
+  }
+  __syncthreads();   // the staged tiles have been read: their memory takes the result
+#pragma unroll
+  for (int j = 0; j < S::FN; ++j) {
+    const int col = (wn * S::FN + j) * 16 + 4 * kg;
+    f32x4 b = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias && n0 + col < p.N) b = QT::load4(p.bias + (int64_t)(n0 + col) * 2);
+#pragma unroll
+    for (int i = 0; i < S::FM; ++i) {
+      f32x4 y = acc[i][j] + b;
+      if constexpr (TABLE) {
+        typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+        const u16x4 bits = __builtin_bit_cast(u16x4, QT::pack4(y));
+        u16x4 looked;
+        uint32_t most = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t at = (bits[e] & 0x7FFFu) - kGeluLow;
+          most = max(most, at);
+          looked[e] = ((const uint16_t*)(smem + S::TILES))[min(at, kGeluCount - 1) + (bits[e] >> 15) * kGeluCount];
+        }
+        if (__any(most >= kGeluCount)) {   // tiny, large, infinite or not a number
+#pragma unroll
+          for (int e = 0; e < 4; ++e) y[e] = gelu((float)(elem)y[e]);
+        } else {
+          *(u16x4*)(smem + ((wm * S::FM + i) * 16 + r) * S::PITCH + col * 2) = looked;
+          continue;
+        }
+      } else if constexpr (EPI == kGelu) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = gelu((float)(elem)y[e]);
+      }
+      QT::store4(smem + ((wm * S::FM + i) * 16 + r) * S::PITCH + col * 2, y[0], y[1], y[2], y[3]);
+    }
+  }
+  __syncthreads();
+  constexpr int CH = TN / 8;
+  for (int c = tid; c < TM * CH; c += 64 * S::NW) {
+    const int row = c / CH, col = (c - row * CH) * 8, m = m0 + row, nn = n0 + col;
+    if (m < p.M && nn < p.N) {
+      frag y = *(const frag*)(smem + row * S::PITCH + col * 2);
+      if constexpr (EPI == kResidual) y = QT::from_f32(QT::to_f32(y) + QT::to_f32(QT::load(p.residual + ((int64_t)m * p.ldr + nn) * 2)));
+      *(frag*)(p.out + ((int64_t)m * p.ldo + nn) * 2) = y;
+    }
+  }
+}
+
+template <class QT, int EPI, class S>
+int launch_shape(GemmParams p, hipStream_t stream) {
+  auto kern = fdb_gemm_kernel<QT, EPI, S>;
+  constexpr int lds = S::lds_bytes(EPI == kGelu && std::is_same<QT, Bf16Tr>::value);
+  static std::atomic<uint64_t> lds_set{0};
+  const hipError_t e = fdb_set_lds_once((const void*)kern, lds, lds_set);
+  if (e != hipSuccess) return (int)e;
+  p.tiles_n = (p.N + S::TN - 1) / S::TN;
+  p.tiles = (p.M + S::TM - 1) / S::TM * p.tiles_n;
+  hipLaunchKernelGGL(kern, dim3(p.tiles), dim3(64 * S::NW), lds, stream, p);
+  return (int)hipGetLastError();
+}
+
+using S32x64 = GemmShape<32, 64, 2, 2, 4, 3>;
+using S64x64 = GemmShape<64, 64, 2, 2, 3, 3>;
+using S64x192Deep = GemmShape<64, 192, 2, 4, 4, 1>;   // alone on its CU: four stages instead of a second workgroup
+using S64x192 = GemmShape<64, 192, 2, 4, 2, 2>;
+using S256x192 = GemmShape<256, 192, 4, 2, 2, 1>;
+
+int64_t tiles_of(int64_t M, int64_t N, int tm, int tn) { return (M + tm - 1) / tm * ((N + tn - 1) / tn); }
+
+// The smallest tile whose workgroups make one round of the chip; beyond that the tile that loads the least.  bf16, replayed graph, us, in the
+// order of the list, * the chosen one ([M x K] . [K x N] and what follows):
+//   512 x 768 x 768   5.4* 6.2 8.9 8.2 18.9      1500 x 768 x 768    7.7 7.3* 8.9 8.5 19.2      1024 x 3072 x 768  22.9 17.2 12.3* 14.3 24.3
+//   4096 x 768 x 3072 44.6 32.3 26.9* 34.6 59.7  2048 x 3072 x 768  43.1 27.5 22.9 17.4* 25.2   8192 x 768 x 768  26.3 19.6 19.0 15.3* 23.1
+//   3000 x 3072 x 768 61.0 39.8 32.7 27.9 26.4*  4096 x 3072 x 768  82.3 50.5 42.8 31.1 27.7*   8192 x 3072 x 768  155 97.3 81.4 58.1 53.4*
+// (64 x 96, 128 x 96, 128 x 128, 128 x 144, 128 x 192 and 256 x 256, with two to five stages, lie between these.)
+template <class QT, int EPI>
+int launch_gemm(const GemmParams& p, hipStream_t stream) {
+  if (tiles_of(p.M, p.N, 32, 64) <= 256) return launch_shape<QT, EPI, S32x64>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 64) <= 480) return launch_shape<QT, EPI, S64x64>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 192) <= 256) return launch_shape<QT, EPI, S64x192Deep>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 192) <= 512) return launch_shape<QT, EPI, S64x192>(p, stream);
+  return launch_shape<QT, EPI, S256x192>(p, stream);
+}
+
+template <class QT>
+int launch_type(const GemmParams& p, int epilogue, hipStream_t stream) {
+  if (epilogue == kGelu) return launch_gemm<QT, kGelu>(p, stream);
+  if (epilogue == kResidual) return launch_gemm<QT, kResidual>(p, stream);
+  return launch_gemm<QT, kPlain>(p, stream);
+}
+
+}  // namespace
+
+// Where this kernel is the faster one, and adds up as the library does.  Up to 32 rows the weights are streamed by many waves that share the
+// contraction.  A long contraction over few tiles is split by the library ([512 x 3072] . [3072 x 768] + residual 13.5 us there, 13.9 here; 1500 rows
+// 21.7 and 18.3).  A plain product has nothing to gain from 512 tiles of 64 x 192 up (4096 and 3000 rows to 2304 columns: 19.3 and 16.7 us there, 20.8
+// and 19.7 here; 2048, 1024 and 512 rows 15.5, 11.2 and 8.1 there, 12.7, 9.4 and 7.1 here).
+extern "C" int32_t fdb_gemm_serves(int64_t M, int64_t N, int64_t K, int32_t epilogue) {
+  if (M <= 32 || N < 8 || K < kDepth || N % 8 || K % kDepth || M > (1 << 24) || N > (1 << 24)) return 0;
+  if (K > 1536 && tiles_of(M, N, 64, 64) <= 256) return 0;
+  return epilogue != kPlain || tiles_of(M, N, 64, 192) <= 512;
+}
+
+int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx,
+                    int64_t ldw, int64_t ldo, int64_t ldr, int epilogue, int dtype, void* stream) {
+  const GemmParams p{(const char*)x, (const char*)w, (const char*)bias, (const char*)residual, (char*)out, ldx, ldw, ldo, ldr, M, N, K, 0, 0};
+  return dtype == FDB_BF16 ? launch_type<Bf16Tr>(p, epilogue, (hipStream_t)stream) : launch_type<F16Tr>(p, epilogue, (hipStream_t)stream);
+}

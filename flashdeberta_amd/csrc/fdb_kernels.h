@@ -219,6 +219,8 @@ int fdb_launch_merge(const FdbKParams& p, int dtype, void* stream);
 int fdb_launch_merge_parts(const FdbKParams& p, int dtype, int head_dim, void* stream);
 int fdb_launch_linear(const void* x, const void* w, const void* bias, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldw,
                       int64_t ldo, int dtype, void* stream);  // fdb_linear.hip
+int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx,
+                    int64_t ldw, int64_t ldo, int64_t ldr, int epilogue, int dtype, void* stream);  // fdb_gemm.hip
 int fdb_column_sum_parts(int64_t rows);
 int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
                            int dtype, void* stream);

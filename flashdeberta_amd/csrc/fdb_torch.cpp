@@ -222,30 +222,47 @@ void product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias
   if (!library_product(a, trans_a, b, trans_b, d, bias, accumulate)) torch_product(a, trans_a, b, trans_b, d, bias, accumulate);
 }
 
-// x [..., K] . w [N, K]^T + bias -> [..., N], as torch's linear computes it, bit for bit (the heuristic's choice is the same).
-// With `own`, a product of few rows takes the library's kernels instead: up to 32 rows, or while 64 x 64 tiles make one round
-// of workgroups and the contraction is short; beyond that hipBLASLt's larger tiles and its split contraction are faster by more
-// than its call costs the host.
-Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool own) {
+// x [..., K] . w [N, K]^T + bias -> [..., N], followed by GELU or an addition of `residual` [..., N] where asked for, as torch computes
+// them one after the other: bit for bit (the library's choice is torch's, and fdb_gemm adds up as it does).  With `own`, a product of at
+// most 32 rows takes the library's streaming kernel, whose waves share the contraction.
+enum class Then { nothing, gelu, add };
+Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool own, Then then = Then::nothing, const Tensor* residual = nullptr) {
   const auto type = x_in.scalar_type();
   const bool half = type == at::kBFloat16 || type == at::kHalf;
   const int64_t k = x_in.size(-1), m = k > 0 ? x_in.numel() / k : 0;
+  const auto rest = [&](Tensor y) {
+    if (then == Then::add) y.add_(*residual);
+    else if (then == Then::gelu) at::gelu_(y);
+    return y;
+  };
   if (!x_in.is_cuda() || !half || !plain_memory(x_in) || !plain_memory(w) || (bias && !plain_memory(*bias)) || w.scalar_type() != type || (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 ||
       w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) || w.device() != x_in.device() || !bias || bias->device() != x_in.device() ||
       bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())
-    return at::linear(x_in, w, bias);
+    return rest(at::linear(x_in, w, bias));
   const c10::hip::HIPGuard guard(x_in.get_device());
   const Tensor x = x_in.contiguous();
   const int64_t n = w.size(0);
   auto size = x.sizes().vec();
   size.back() = n;
   const Tensor out = at::empty(size, x.options());
-  if (own && (m <= 32 || (k <= 1536 && ((m + 63) / 64) * ((n + 63) / 64) <= 256))) {
+  if (m <= 32 && own) {
     const int rc = fdb_linear(x.data_ptr(), w.data_ptr(), bias->data_ptr(), out.data_ptr(), (int32_t)m, (int32_t)n, (int32_t)k, k, w.stride(0), n, fdb_dtype_of(type), stream_of(x));
-    if (rc == 0) return out;
+    if (rc == 0) return rest(out);
     if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
   }
-  return library_product({x, m}, false, {w, n}, true, {out, m}, &*bias) ? out : at::linear(x_in, w, bias);
+  const int epilogue = then == Then::gelu ? FDB_GEMM_GELU : then == Then::add ? FDB_GEMM_RESIDUAL : FDB_GEMM_PLAIN;
+  if (fdb_gemm_serves(m, n, k, epilogue)) {
+    Tensor r;
+    if (then == Then::add && residual->scalar_type() == type && residual->sizes() == out.sizes() && residual->device() == x.device() && plain_memory(*residual))
+      r = residual->contiguous();
+    if (then != Then::add || r.defined()) {
+      const int rc = fdb_gemm(x.data_ptr(), w.data_ptr(), bias->data_ptr(), r.defined() ? r.data_ptr() : nullptr, out.data_ptr(), (int32_t)m, (int32_t)n,
+                              (int32_t)k, k, w.stride(0), n, n, epilogue, fdb_dtype_of(type), stream_of(x));
+      if (rc == 0) return out;
+      if (rc > 0) check(rc, "fdb_gemm");
+    }
+  }
+  return rest(library_product({x, m}, false, {w, n}, true, {out, m}, &*bias) ? out : at::linear(x_in, w, bias));
 }
 
 // product(a, rows_a, trans_a, b, rows_b, trans_b, d, rows_d, bias or None, accumulate, library): into d, by hipBLASLt (whether it has
@@ -905,13 +922,13 @@ PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
     const Tensor weight, bias;
     double eps;
     explicit Norm(PyObject* const* p) : weight(tensor_arg(p[0], "norm_weight")), bias(tensor_arg(p[1], "norm_bias")), eps(float_arg(p[2])) {}
-    Tensor operator()(Tensor y, const Tensor& residual) const { return at::layer_norm(y.add_(residual), {y.size(-1)}, weight, bias, eps); }
+    Tensor operator()(const Tensor& y) const { return at::layer_norm(y, {y.size(-1)}, weight, bias, eps); }
   };
   struct Linear {
     const Tensor weight;
     OptTensor bias;
     explicit Linear(PyObject* const* p) : weight(tensor_arg(p[0], "weight")), bias(opt_tensor_arg(p[1], "bias")) {}
-    Tensor operator()(const Tensor& y) const { return project(y, weight, bias, false); }
+    Tensor operator()(const Tensor& y, Then then, const Tensor* residual = nullptr) const { return project(y, weight, bias, false, then, residual); }
   };
   const Linear in(x + 1), out(x + 11), up(x + 16), down(x + 18);
   const LayerCall call(x + 3);
@@ -921,10 +938,8 @@ PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
     const NoGil released;
     const Tensor context = layer_attention(hidden, in.weight, in.bias, call, false);
     const c10::hip::HIPGuard guard(hidden.get_device());
-    const Tensor attended = norm1(out(context), hidden);
-    Tensor inner = up(attended);
-    at::gelu_(inner);
-    next = norm2(down(inner), attended);
+    const Tensor attended = norm1(out(context, Then::add, &hidden));
+    next = norm2(down(up(attended, Then::gelu), Then::add, &attended));
   }
   return THPVariable_Wrap(std::move(next));
   END_HANDLE_TH_ERRORS

@@ -373,6 +373,18 @@ int fdb_mask_bounds(const void* mask, int32_t elem_size, int32_t is_float, int64
 int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_t rows, int32_t cols, int32_t depth, int64_t ldx,
                int64_t ldw, int64_t ldo, int32_t dtype, void* stream);
 
+/*
+ * Products of more rows and what follows them in an encoder layer (FDB_BF16 / FDB_F16), y = x [rows, depth] . w [cols, depth]^T + bias (or
+ * NULL) rounded to the type:  out = y, gelu(y) (the exact one, x / 2 * (1 + erf(x / sqrt 2))) or y + residual [rows, cols].  Row strides in
+ * elements; x, w, out, residual and their rows aligned to 16 bytes, bias to 8; depth a multiple of 64, cols of 8.  out overlaps nothing else.
+ * fdb_gemm_serves: whether this is the faster way for a size (host, no GPU).  The reference runs modules one by one
+ * (transformers' DebertaV2Layer).
+ */
+enum { FDB_GEMM_PLAIN = 0, FDB_GEMM_GELU = 1, FDB_GEMM_RESIDUAL = 2 };
+int fdb_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t rows, int32_t cols, int32_t depth, int64_t ldx,
+             int64_t ldw, int64_t ldo, int64_t ldr, int32_t epilogue, int32_t dtype, void* stream);
+int32_t fdb_gemm_serves(int64_t rows, int64_t cols, int64_t depth, int32_t epilogue);
+
 /* Enqueue the device-side work-list construction from cu_seqlens. */
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens,
                        int32_t* worklist, void* stream);
