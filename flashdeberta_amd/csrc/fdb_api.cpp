@@ -4,6 +4,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include <hip/hip_runtime.h>
@@ -105,13 +106,42 @@ bool has_far_launch(const fdb_attn_args* a) {
          longest > radius + FDB_BN - 1;
 }
 
+int near_parts_wanted(const fdb_attn_args* a);
+
+// Whether the near launch walks the far tiles, too, and the far launch is left out.  A far tile costs the near kernel some four times what it
+// costs the far kernel, but a launch of few far tiles costs 6 to 8 us whatever it does, and while every query tile has a workgroup slot the
+// near launch lasts as long as its longest query tile, in mid-sequence, which has few far tiles or none.  12 heads, bf16, two launches -> one:
+//   3 x 777 39.7 -> 30.0 us, 1 x 700 28.4 -> 21.3, 8 x 640 46.0 -> 36.9, 8 x 777 80.9 -> 67.7, 4 x 1024 56.9 -> 51.2, 1 x 1300 44.0 -> 40.7;
+// kept as two where one is slower: 2 x 1300 58.4 (62.5), 2 x 1501 61.6 (71.0), 6 x 1024 81.6 (82.4).
+bool near_takes_all(const fdb_attn_args* a) {
+  if (!has_far_launch(a) || !steps32_supported(a->dtype, a->head_dim) || a->cu_seqlens || a->causal || a->far_splits > 0 || a->near_splits > 0) return false;
+  if (a->max_seqlen > 16 * FDB_BM) return false;
+  const int tiles = (a->max_seqlen + FDB_BM - 1) / FDB_BM, n64 = (a->max_seqlen + FDB_BN - 1) / FDB_BN, radius = a->lut_radius > 0 ? a->lut_radius : 1;
+  int most_near = 0, most_far = 0, far_tiles = 0;
+  for (int t = 0; t < tiles; ++t) {
+    const int m0 = t * FDB_BM, lim = m0 - (FDB_BN - 1) - radius;
+    const int t0 = lim >= 0 ? std::min(n64, lim / FDB_BN + 1) : 0, t1 = std::max(t0, std::min(n64, (m0 + FDB_BM - 1 + radius + FDB_BN - 1) / FDB_BN));
+    most_near = std::max(most_near, t1 - t0);
+    most_far = std::max(most_far, n64 - (t1 - t0));
+    far_tiles += n64 - (t1 - t0);
+  }
+  // microseconds, from the sizes above: a near step takes 1.43 in a launch that ends on its short tiles, 1.6 where all have the same length
+  // and some share a compute unit, and 0.85 of a slot's time where there are several rounds; the far launch has its longest workgroup or its total
+  const int64_t wgs = (int64_t)tiles * a->batch * a->heads;
+  const double all = (double)far_tiles * a->batch * a->heads / cu_count();
+  const int parts = near_parts_wanted(a);
+  const double alone = 2 * n64 * (wgs * parts <= cu_count() ? 1.43 : 1.6) - 2 * most_near * 1.43;
+  const double more = std::max(alone / parts, wgs > 2 * cu_count() ? 1.7 * all : 0.0), far = std::max(3.0 + 0.65 * most_far, 6.0 + 0.43 * all);
+  return more < far;
+}
+
 // Workgroups per query tile of the far-only launch.  That launch keeps three workgroups on a CU; when
 // the query tiles fill at most half of those slots, the far keys of a tile are shared out among as many
 // workgroups as still fit in one round, every share keeping at least eight tiles.  (Measured: 384 query
 // tiles on 768 slots gain 9 % of the whole call from two shares; shares that need a second round of
 // workgroups, e.g. three for 512 query tiles, gain nothing.)
 int far_parts_wanted(const fdb_attn_args* a) {
-  if (!has_far_launch(a) || !steps32_supported(a->dtype, a->head_dim)) return 1;
+  if (!has_far_launch(a) || near_takes_all(a) || !steps32_supported(a->dtype, a->head_dim)) return 1;
   if (a->far_splits > 0) return a->far_splits;
   // A packed batch has its lengths on the device: the host goes by the mean length (the kernel divides each query
   // tile's own far tiles among the shares, whatever they are), and only shares when that mean leaves far tiles at all.
@@ -376,7 +406,8 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
   // hand-over between the two launches.
   if ((a->pos_key || a->pos_query) && a->lse && pair_supported(a->dtype, a->head_dim)) {
     const bool fp8 = fdb_fp8_pair_supported(a->dtype, a->head_dim);
-    const bool need_far = has_far_launch(a);  // otherwise no tile of any query tile is far
+    p.near_all = launch_mask == 0 && near_takes_all(a) ? 1 : 0;
+    const bool need_far = has_far_launch(a) && !p.near_all;  // otherwise no tile of any query tile is far
     // as many workgroups per query tile as wanted and as the workspace holds partial results for
     p.far_parts = need_far ? far_parts_wanted(a) : 1;
     p.near_parts = near_parts_wanted(a);

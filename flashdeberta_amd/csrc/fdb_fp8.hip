@@ -459,8 +459,8 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   if (p.causal) j_end = min(Lb, m0 + FDB_BM);
   const int n_tiles = (j_end + FDB_BN - 1) / FDB_BN;
   const int lim = m0 - (FDB_BN - 1) - p.R;
-  const int t0 = lim >= 0 ? min(n_tiles, lim / FDB_BN + 1) : 0;
-  const int t1 = max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
+  const int t0 = lim >= 0 && !p.near_all ? min(n_tiles, lim / FDB_BN + 1) : 0;
+  const int t1 = p.near_all ? n_tiles : max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
   int s0 = 2 * t0;
   int s1 = max(s0, min(2 * t1, (j_end + kStep - 1) / kStep));
   if (p.near_parts > 1) {

@@ -37,6 +37,7 @@ struct FdbKParams {
   int32_t groups_together;  // fdb_groups_together(tiles_per_seq)
   int32_t R;        // LUT radius
   int32_t far_done;  // near launches: the far tiles' partial results (far_parts of them) are to be merged
+  int32_t near_all;  // near launches: they walk every key tile, no far launch precedes them
   int32_t far_parts; // workgroups per query tile of the far-only launch, each with its share of the far tiles and a
                      // partial result of its own (the first in out / lse, the others in workspace slots 0 ..)
   int32_t near_parts; // workgroups per query tile of the near launch; above 1 each leaves the partial result of

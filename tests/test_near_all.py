@@ -1,0 +1,64 @@
+"""The near launch with all key tiles, taken where a far launch would have little to do: against the oracle, around the tile edges, and
+against the pair of launches, which far_splits=1 asks for."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from flashdeberta_amd import _lib, ops
+from oracle import disentangled_oracle as O
+
+EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _inputs(B, L, H, terms, dtype):
+    g = torch.Generator().manual_seed(B * L)
+    q, k, v = [torch.randn(B, L, H, 64, generator=g).to(dtype) for _ in range(3)]
+    pk, pq = [torch.randn(H, 512, 64, generator=g).to(dtype) if t else None for t in terms]
+    return q, k, v, pk, pq
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("B,L,terms", [(1, 577, (1, 1)), (1, 640, (1, 1)), (2, 641, (1, 0)), (1, 777, (0, 1)), (1, 1024, (1, 1)), (1, 1153, (1, 1))])
+def test_all_key_tiles_in_the_near_launch(B, L, terms, dtype):
+    q, k, v, pk, pq = _inputs(B, L, 2, terms, dtype)
+    n = lambda x: None if x is None else x.float().numpy().astype(np.float64)
+    t = lambda x: n(x).transpose(0, 2, 1, 3)
+    ref, ref_lse = O.disentangled_attention(t(q), t(k), t(v), n(pk), n(pq), 256, 512, return_lse=True)
+    d = lambda x: None if x is None else x.cuda()
+    kw = dict(position_buckets=256, max_relative_positions=512, return_lse=True)
+    out, lse = ops.disentangled_attention_fwd(d(q), d(k), d(v), d(pk), d(pq), **kw)
+    two, two_lse = ops.disentangled_attention_fwd(d(q), d(k), d(v), d(pk), d(pq), far_splits=1, **kw)
+    # scores of standard deviation 1.0 to 1.4 carry a rounding of the scaled query and of c2p, the output a rounding of the probabilities and one of its own
+    for got, got_lse in ((out, lse), (two, two_lse)):
+        assert np.abs(got.float().cpu().numpy().transpose(0, 2, 1, 3) - ref).max() <= 3 * EPS[dtype] * max(1.0, np.abs(ref).max())
+        assert np.abs(got_lse.view(B, L, 2).cpu().numpy().transpose(0, 2, 1) - ref_lse).max() <= 2 * EPS[dtype]
+
+
+@pytest.mark.gpu
+def test_padded_rows_in_the_near_launch():
+    q, k, v, pk, pq = [x.cuda() for x in _inputs(3, 777, 2, (1, 1), torch.bfloat16)]
+    kw = dict(position_buckets=256, max_relative_positions=512)
+    start, length = [torch.tensor(x, dtype=torch.int32, device="cuda") for x in ((0, 100, 776), (777, 640, 1))]
+    out = ops.disentangled_attention_fwd(q, k, v, pk, pq, seq_start=start, seq_len=length, **kw)
+    for b in range(3):
+        s, n = int(start[b]), int(length[b])
+        alone = ops.disentangled_attention_fwd(*[x[b:b + 1, s:s + n].contiguous() for x in (q, k, v)], pk, pq, far_splits=1, **kw)
+        assert (out[b, s:s + n] - alone[0]).abs().max() <= 4 * EPS[torch.bfloat16]
+        assert out[b].isfinite().all() and (out[b, :s] == 0).all() and (out[b, s + n:] == 0).all()
+
+
+def test_calls_that_keep_two_launches():
+    """A far share of its own has a workspace slot: none is asked for where the near launch takes all, whatever the number of near shares."""
+    a = _lib.FdbAttnArgs()
+    for n in ("q", "k", "v", "out", "pos_key", "pos_query", "lse", "delta_lut"):
+        setattr(a, n, 0x1000)
+    a.batch, a.heads, a.head_dim, a.dtype, a.att_span, a.lut_radius, a.max_seqlen, a.total_tokens = 1, 1, 64, _lib.FDB_BF16, 256, 512, 2048, 2048
+    part = lambda rows: rows * (64 * 2 + 4)
+    ws = lambda: _lib.lib.fdb_attn_workspace_bytes(ctypes.byref(a))
+    assert ws() % part(2048) == 0
+    near = ws() // part(2048)
+    a.far_splits = 2
+    assert ws() == (1 + near) * part(2048)
