@@ -764,6 +764,36 @@ int fdb_gemm(const void* x, const void* w, const void* bias, const void* residua
   return fdb_launch_gemm(x, w, bias, residual, out, rows, cols, depth, ldx, ldw, ldo, ldr, epilogue, dtype, stream);
 }
 
+int fdb_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0, void* out1,
+              int32_t dtype, void* stream) {
+  if (!w || rows0 < 0 || rows1 < 0 || (rows0 && (!x0 || !out0)) || (rows1 && (!x1 || !out1))) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  const auto deep = [](int32_t rows, int32_t depth) { return rows == 0 || (depth >= 64 && depth % 64 == 0 && depth <= (1 << 22)); };
+  if (rows0 + rows1 < 1 || rows0 > (1 << 26) || rows1 > (1 << 26) || cols < 64 || cols % 64 || cols > (1 << 22) || !deep(rows0, depth0) || !deep(rows1, depth1)) return FDB_ERR_SHAPE;
+  if (!aligned16(x0) || !aligned16(x1) || !aligned16(w) || !aligned16(out0) || !aligned16(out1)) return FDB_ERR_ALIGN;
+  return fdb_launch_dgrad(x0, rows0, depth0, x1, rows1, depth1, w, cols, out0, out1, dtype, stream);
+}
+
+int64_t fdb_wgrad_workspace_bytes(int32_t rows0, int32_t rows1, int32_t x_cols, int32_t y_cols) {
+  if (rows0 < 1 || rows1 < 1 || x_cols < 64 || y_cols < 64) return FDB_ERR_SHAPE;
+  return (int64_t)fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols, y_cols, cu_count()) * x_cols * (y_cols + 1) * 4;
+}
+
+int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
+              void* dw, void* db, void* workspace, int32_t dtype, void* stream) {
+  if (!x0 || !y0 || !x1 || !y1 || !dw || !db || !workspace) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  // 64-column panels; the second pair belongs to whole tiles of 128 columns; rows within a lane's 24-bit product
+  if (rows0 < 1 || rows1 < 1 || rows0 > (1 << 26) || rows1 > (1 << 26) || x_cols0 < 64 || x_cols0 % 64 || x_cols0 > (1 << 22) || x_cols1 < 128 || x_cols1 % 128 || x_cols1 > x_cols0 ||
+      y_cols < 64 || y_cols % 64 || y_cols > (1 << 22))
+    return FDB_ERR_SHAPE;
+  for (const void* x : {x0, y0, x1, y1, (const void*)dw, (const void*)db, (const void*)workspace})
+    if (!aligned16(x)) return FDB_ERR_ALIGN;
+  if (reinterpret_cast<uintptr_t>(workspace) & 31u) return FDB_ERR_ALIGN;
+  return fdb_launch_wgrad(x0, y0, rows0, x_cols0, x1, y1, rows1, x_cols1, y_cols, dw, db, (float*)workspace, fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols0, y_cols, cu_count()), dtype,
+                          stream);
+}
+
 int32_t fdb_delta_lut_radius(int32_t position_buckets, int32_t max_position) {
   if (!lut_config_ok(position_buckets, max_position)) return FDB_ERR_LUT_ARGS;
   const int32_t span = position_buckets > 0 ? position_buckets : max_position;

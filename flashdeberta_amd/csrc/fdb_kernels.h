@@ -222,6 +222,11 @@ int fdb_launch_linear(const void* x, const void* w, const void* bias, void* out,
                       int64_t ldo, int dtype, void* stream);  // fdb_linear.hip
 int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx,
                     int64_t ldw, int64_t ldo, int64_t ldr, int epilogue, int dtype, void* stream);  // fdb_gemm.hip
+int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0,
+                     void* out1, int dtype, void* stream);  // fdb_grad.hip
+int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols, int cus);
+int fdb_launch_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
+                     void* dw, void* db, float* ws, int32_t shares, int dtype, void* stream);
 int fdb_column_sum_parts(int64_t rows);
 int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
                            int dtype, void* stream);

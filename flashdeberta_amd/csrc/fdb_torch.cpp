@@ -837,25 +837,43 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     ::backward(hidden, B, L, H, part(qkv, 0), part(qkv, 1), part(qkv, 2), whole(out), whole(dout), lse, table(pos, 1), table(pos, 0), part(dqkv, 0),
                part(dqkv, 1), part(dqkv, 2), table(dpos, 1), table(dpos, 0), o);
     Tensor dhidden, drel, dw, db;
-    if (ctx->needs_input_grad(0)) {
-      dhidden = at::empty(hidden.sizes(), hidden.options());
-      product({dqkv, n}, false, {w, 3 * W}, false, {dhidden, n});
+    const bool for_hidden = ctx->needs_input_grad(0), for_rel = ctx->needs_input_grad(1);
+    const bool for_weights = ctx->needs_input_grad(2) || ctx->needs_input_grad(4) || ctx->needs_input_grad(6);
+    const bool for_biases = ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7);
+    const int code = fdb_dtype_of(type);
+    // tokens and tables in one launch; a negative code is a size or an alignment these kernels are not built for: two products then
+    if (for_hidden) dhidden = at::empty(hidden.sizes(), hidden.options());
+    if (for_rel) drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
+    if (for_hidden || for_rel) {
+      const int rc = n > INT32_MAX || C > INT32_MAX || !fdb_dgrad_serves(for_hidden ? n : 0, for_rel ? rows : 0, C) ? (int)FDB_ERR_SHAPE : fdb_dgrad(dqkv.data_ptr(), for_hidden ? (int32_t)n : 0, (int32_t)(3 * W), dpos.data_ptr(), for_rel ? (int32_t)rows : 0, (int32_t)(2 * W), w.data_ptr(),
+                               (int32_t)C, for_hidden ? dhidden.data_ptr() : nullptr, for_rel ? drel.data_ptr() : nullptr, code, stream_of(hidden));
+      if (rc > 0) check(rc, "fdb_dgrad");
+      if (rc < 0 && for_hidden) product({dqkv, n}, false, {w, 3 * W}, false, {dhidden, n});
+      if (rc < 0 && for_rel) product({dpos, rows}, false, {w, 2 * W}, false, {drel, rows});
     }
-    if (ctx->needs_input_grad(1)) {
-      drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
-      product({dpos, rows}, false, {w, 2 * W}, false, {drel, rows});
-    }
-    if (ctx->needs_input_grad(2) || ctx->needs_input_grad(4) || ctx->needs_input_grad(6)) {
+    bool sums_done = false;
+    if (for_weights) {
       dw = at::empty({3 * W, C}, hidden.options());
-      product({dqkv, n}, true, {hidden, n}, false, {dw, 3 * W});
-      product({dpos, rows}, true, {rel, rows}, false, {dw, 2 * W}, nullptr, true);
+      db = at::empty({3 * W}, hidden.options());
+      int rc = FDB_ERR_SHAPE;
+      if (n <= INT32_MAX && C % 64 == 0) {
+        const Tensor ws = at::empty({fdb_wgrad_workspace_bytes((int32_t)n, (int32_t)rows, (int32_t)(3 * W), (int32_t)C)}, hidden.options().dtype(at::kByte));
+        rc = fdb_wgrad(dqkv.data_ptr(), hidden.data_ptr(), (int32_t)n, (int32_t)(3 * W), dpos.data_ptr(), rel.data_ptr(), (int32_t)rows, (int32_t)(2 * W), (int32_t)C, dw.data_ptr(),
+                       db.data_ptr(), ws.data_ptr(), code, stream_of(hidden));
+        if (rc > 0) check(rc, "fdb_wgrad");
+      }
+      sums_done = rc == 0;
+      if (rc < 0) {
+        product({dqkv, n}, true, {hidden, n}, false, {dw, 3 * W});
+        product({dpos, rows}, true, {rel, rows}, false, {dw, 2 * W}, nullptr, true);
+      }
     }
-    if (ctx->needs_input_grad(3) || ctx->needs_input_grad(5) || ctx->needs_input_grad(7)) {
+    if (for_biases && !sums_done) {
       db = at::empty({3 * W}, hidden.options());
       const Tensor ws = at::empty({fdb_column_sums_workspace_bytes(n, 3 * W, rows)}, hidden.options().dtype(at::kByte));
-      check(fdb_column_sums(dqkv.data_ptr(), n, 3 * W, dpos.data_ptr(), rows, 2 * W, db.data_ptr(), ws.data_ptr(), fdb_dtype_of(type), stream_of(hidden)),
-            "fdb_column_sums");
+      check(fdb_column_sums(dqkv.data_ptr(), n, 3 * W, dpos.data_ptr(), rows, 2 * W, db.data_ptr(), ws.data_ptr(), code, stream_of(hidden)), "fdb_column_sums");
     }
+    if (!for_biases) db = Tensor();
     const auto rows_of = [&](const Tensor& t, int64_t i) { return t.defined() ? t.narrow(0, i * W, W) : Tensor(); };
     return {dhidden, drel, rows_of(dw, 0), rows_of(db, 0), rows_of(dw, 1), rows_of(db, 1), rows_of(dw, 2), rows_of(db, 2), Tensor()};
   }

@@ -385,6 +385,21 @@ int fdb_gemm(const void* x, const void* w, const void* bias, const void* residua
              int64_t ldw, int64_t ldo, int64_t ldr, int32_t epilogue, int32_t dtype, void* stream);
 int32_t fdb_gemm_serves(int64_t rows, int64_t cols, int64_t depth, int32_t epilogue);
 
+/*
+ * The products of a layer's training backward (FDB_BF16 / FDB_F16; contiguous row-major matrices aligned to 16 bytes, the workspace to 32;
+ * depth and all column counts multiples of 64).  Two problems that share weights are one launch each:
+ *   fdb_dgrad: out_i [rows_i, cols] = x_i [rows_i, depth_i] . w, the first depth_i rows of w [.., cols] (rows_i 0: none);
+ *   fdb_wgrad: dw [x_cols0, y_cols] = x0^T . y0, and + x1^T . y1 on its first x_cols1 rows (a multiple of 128), fp32 sums over all rows, one
+ *              rounding; db [x_cols0] = the column sums of x0 (+ x1).
+ * The reference's layers run them as autograd's products per module (src/flashdeberta/model.py:147-192).
+ */
+int fdb_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0, void* out1,
+              int32_t dtype, void* stream);
+int32_t fdb_dgrad_serves(int64_t rows0, int64_t rows1, int64_t cols);  /* host: whether fdb_dgrad is the faster way */
+int64_t fdb_wgrad_workspace_bytes(int32_t rows0, int32_t rows1, int32_t x_cols0, int32_t y_cols);
+int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
+              void* dw, void* db, void* workspace, int32_t dtype, void* stream);
+
 /* Enqueue the device-side work-list construction from cu_seqlens. */
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens,
                        int32_t* worklist, void* stream);
