@@ -774,6 +774,17 @@ int fdb_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int
   return fdb_launch_dgrad(x0, rows0, depth0, x1, rows1, depth1, w, cols, out0, out1, dtype, stream);
 }
 
+int fdb_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream) {
+  if (!w || !b || !w_out || !b_out) return FDB_ERR_NULL;
+  if (b_bytes < 16 || b_bytes % 16 || w_bytes < b_bytes || w_bytes % 16 || w_bytes > (1ll << 40)) return FDB_ERR_SHAPE;
+  for (int i = 0; i < 3; ++i) {
+    if (!w[i] || !b[i]) return FDB_ERR_NULL;
+    if (!aligned16(w[i]) || !aligned16(b[i])) return FDB_ERR_ALIGN;
+  }
+  if (!aligned16(w_out) || !aligned16(b_out)) return FDB_ERR_ALIGN;
+  return fdb_launch_join(w, b, w_out, b_out, w_bytes, b_bytes, stream);
+}
+
 int64_t fdb_wgrad_workspace_bytes(int32_t rows0, int32_t rows1, int32_t x_cols, int32_t y_cols) {
   if (rows0 < 1 || rows1 < 1 || x_cols < 64 || y_cols < 64) return FDB_ERR_SHAPE;
   return (int64_t)fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols, y_cols, cu_count()) * x_cols * (y_cols + 1) * 4;

@@ -321,6 +321,34 @@ int fdb_launch_dequant(const void* y, int64_t y_st, int64_t y_sh, const float* s
   return (int)hipGetLastError();
 }
 
+namespace {
+// Three weights and three biases under one another (blockIdx.y: which), sixteen bytes a lane, four lines a thread in flight: the two launches
+// that torch's cat takes are 7.5 us for 3.5 MB, this one 3.
+struct Join {
+  const u32x4 *w[3], *b[3];
+};
+__global__ __launch_bounds__(256) void fdb_join_kernel(const Join from, u32x4* __restrict__ w, u32x4* __restrict__ b, int64_t w_len, int64_t b_len) {
+  const int which = blockIdx.y;
+  const u32x4* src = which == 0 ? from.w[0] : which == 1 ? from.w[1] : from.w[2];
+  const int64_t at = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+  u32x4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (at + 256 * j < w_len) v[j] = src[at + 256 * j];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (at + 256 * j < w_len) w[which * w_len + at + 256 * j] = v[j];
+  if (at < b_len) b[which * b_len + at] = (which == 0 ? from.b[0] : which == 1 ? from.b[1] : from.b[2])[at];
+}
+}  // namespace
+int fdb_launch_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream) {
+  Join from;
+  for (int i = 0; i < 3; ++i) from.w[i] = (const u32x4*)w[i], from.b[i] = (const u32x4*)b[i];
+  hipLaunchKernelGGL(fdb_join_kernel, dim3((unsigned)((w_bytes / 16 + 1023) / 1024), 3), dim3(256), 0, (hipStream_t)stream, from, (u32x4*)w_out, (u32x4*)b_out, w_bytes / 16,
+                     b_bytes / 16);
+  return (int)hipGetLastError();
+}
+
 int fdb_column_sum_parts(int64_t rows) { return (int)((rows + kColShare - 1) / kColShare); }
 
 int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,

@@ -227,6 +227,7 @@ int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* 
 int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols, int cus);
 int fdb_launch_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
                      void* dw, void* db, float* ws, int32_t shares, int dtype, void* stream);
+int fdb_launch_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream);
 int fdb_column_sum_parts(int64_t rows);
 int fdb_launch_column_sums(const void* x, int64_t x_rows, int64_t x_cols, const void* y, int64_t y_rows, int64_t y_cols, void* out, float* ws,
                            int dtype, void* stream);

@@ -779,6 +779,32 @@ struct LayerArgs {
   int64_t heads = 0;
   BwdSettings o;
 };
+// The three weights and the three biases under one another.
+std::pair<Tensor, Tensor> joined(const Tensor& qw, const Tensor& qb, const Tensor& kw, const Tensor& kb, const Tensor& vw, const Tensor& vb, at::ScalarType type, void* stream) {
+  bool plain = true;
+  for (const Tensor* t : {&qw, &kw, &vw, &qb, &kb, &vb}) plain = plain && t->is_contiguous();
+  if (plain) {
+    const Tensor w = at::empty({3 * qw.size(0), qw.size(1)}, qw.options()), b = at::empty({3 * qb.size(0)}, qb.options());
+    const void* const ws[3] = {qw.data_ptr(), kw.data_ptr(), vw.data_ptr()};
+    const void* const bs[3] = {qb.data_ptr(), kb.data_ptr(), vb.data_ptr()};
+    const int rc = fdb_join(ws, bs, w.data_ptr(), b.data_ptr(), qw.numel() * 2, qb.numel() * 2, stream);
+    if (rc == 0) return {w, b};
+    if (rc > 0) check(rc, "fdb_join");
+  }
+  return {at::cat({qw, kw, vw}), at::cat({qb, kb, vb})};
+}
+// out [rows, cols] = the first rows of x . the first cols rows of w^T + b
+void projected(const Tensor& x, int64_t rows, const Tensor& w, const Tensor& b, int64_t cols, const Tensor& out) {
+  const int64_t k = x.size(-1);
+  if (fdb_gemm_serves(rows, cols, k, FDB_GEMM_PLAIN)) {
+    const int rc = fdb_gemm(x.data_ptr(), w.data_ptr(), b.data_ptr(), nullptr, out.data_ptr(), (int32_t)rows, (int32_t)cols, (int32_t)k, k, k, cols, 0, FDB_GEMM_PLAIN,
+                            fdb_dtype_of(x.scalar_type()), stream_of(x));
+    if (rc == 0) return;
+    if (rc > 0) check(rc, "fdb_gemm");
+  }
+  product({x, rows}, false, {w, cols}, true, {out, rows}, &b);
+}
+
 struct LayerNode : public torch::autograd::Function<LayerNode> {
   static Tensor forward(torch::autograd::AutogradContext* ctx, const Tensor& hidden_in, const Tensor& rel_in, const Tensor& qw, const Tensor& qb,
                         const Tensor& kw, const Tensor& kb, const Tensor& vw, const Tensor& vb, const LayerArgs* args) {
@@ -788,10 +814,11 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     const int64_t B = hidden.size(0), L = hidden.size(1), C = hidden.size(2), H = args->heads, D = qw.size(0) / H, W = H * D;
     const int64_t span = att_span(args->o.buckets, args->o.max_relative), rows = 2 * span, esz = hidden.element_size();
     const auto type = hidden.scalar_type();
-    const Tensor w = at::cat({qw, kw, vw}), b = at::cat({qb, kb, vb});
+    Tensor w, b;
+    std::tie(w, b) = joined(qw, qb, kw, kb, vw, vb, type, stream_of(hidden));
     const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
-    product({hidden, B * L}, false, {w, 3 * W}, true, {qkv, B * L}, &b);
-    product({rel, rows}, false, {w, 2 * W}, true, {pos, rows}, &b);
+    projected(hidden, B * L, w, b, 3 * W, qkv);
+    projected(rel, rows, w, b, 2 * W, pos);
     const Tensor out = at::empty({B, L, W}, hidden.options());
     fdb_attn_args a = {};
     const char* p = (const char*)qkv.data_ptr();

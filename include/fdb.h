@@ -400,6 +400,12 @@ int64_t fdb_wgrad_workspace_bytes(int32_t rows0, int32_t rows1, int32_t x_cols0,
 int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
               void* dw, void* db, void* workspace, int32_t dtype, void* stream);
 
+/*
+ * Three contiguous weights of w_bytes each and three biases of b_bytes under one another, in one launch: what the projections of a layer are
+ * joined into for one product.  Pointers aligned to 16 bytes, sizes multiples of 16, no bias longer than a weight.
+ */
+int fdb_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream);
+
 /* Enqueue the device-side work-list construction from cu_seqlens. */
 int fdb_build_worklist(const int32_t* cu_seqlens, int32_t batch, int32_t total_tokens,
                        int32_t* worklist, void* stream);

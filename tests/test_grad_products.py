@@ -71,6 +71,17 @@ def test_wgrad(rows, x_cols, y_cols, dtype):
     _close(db[:x_cols[0]], sums, scale, dtype, "db")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [(8, 8), (64, 64), (192, 344), (768, 768)])
+def test_join(rows, cols):
+    w = [torch.randn(rows, cols, device="cuda").to(torch.bfloat16) for _ in range(3)]
+    b = [torch.randn(rows, device="cuda").to(torch.bfloat16) for _ in range(3)]
+    out, bias = torch.full((3 * rows + 1, cols), 7.0, device="cuda", dtype=torch.bfloat16), torch.full((3 * rows + 8,), 7.0, device="cuda", dtype=torch.bfloat16)
+    at = lambda ts: (ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    assert _lib.lib.fdb_join(at(w), at(b), out.data_ptr(), bias.data_ptr(), 2 * rows * cols, 2 * rows, torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out[:-1], torch.cat(w)) and torch.equal(bias[:-8], torch.cat(b)) and (out[-1] == 7.0).all() and (bias[-8:] == 7.0).all()
+
+
 def test_where_dgrad_serves():
     serves = _lib.lib.fdb_dgrad_serves
     assert serves(1, 0, 64) and serves(8192, 512, 768) and not serves(8192, 512, 1024) and serves(16384, 512, 768)
