@@ -149,12 +149,14 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   const int64_t x1_st = kDQ ? p.q_st : p.k_st, x2_st = kDQ ? p.g_st : p.v_st;
   const char* y1b = kDQ ? kb : qb;
   const char* y2b = kDQ ? vb : gb;
-  const uint32_t y1_rsb = (uint32_t)((kDQ ? p.k_st : p.q_st) * 2), y2_rsb = (uint32_t)((kDQ ? p.v_st : p.g_st) * 2);
+  const uint32_t y1_rsb = own_sgpr((uint32_t)((kDQ ? p.k_st : p.q_st) * 2)), y2_rsb = own_sgpr((uint32_t)((kDQ ? p.v_st : p.g_st) * 2));
   const char* pkb = p.pk + (int64_t)h * p.pk_sh * 2;
   const char* pqb = p.pq + (int64_t)h * p.pq_sh * 2;
   const char* txb = kDQ ? pkb : pqb;   // the table the lane side meets, and the loop side's
   const char* tyb = kDQ ? pqb : pkb;
-  const uint32_t tx_rowb = (uint32_t)((kDQ ? p.pk_sr : p.pq_sr) * 2), ty_rowb = (uint32_t)((kDQ ? p.pq_sr : p.pk_sr) * 2);
+  const uint32_t tx_rowb = own_sgpr((uint32_t)((kDQ ? p.pk_sr : p.pq_sr) * 2)), ty_rowb = own_sgpr((uint32_t)((kDQ ? p.pq_sr : p.pk_sr) * 2));
+  const uint16_t* lut = own_sgpr((const uint16_t*)p.lut);
+  const int R = (int)own_sgpr((uint32_t)p.R);
   const float x_scale = p.scale_log2;
 
   const int xw0 = m0 + wave * 32, xr = xw0 + li;
@@ -224,7 +226,7 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   int r_tab = 0;
   auto batch_delta = [&]() __attribute__((always_inline)) {
     const int r = kDQ ? r_tab : -r_tab;
-    const int d = (int)((const uint16_t*)p.lut)[max(-p.R, min(p.R, r)) + p.R];
+    const int d = (int)lut[(uint32_t)(max(-R, min(R, r)) + R)];
     r_tab -= 32;
     return d;
   };
@@ -739,10 +741,13 @@ __global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingPara
 // The last group of a head collects the saturated rows' sums per token: two rows (delta(+R), delta(-R)) of each table, weights per token.
 // A wave issues about one instruction per 4.5 clocks and a row block is only eight MFMAs, so the loop is written for few
 // instructions: it is unrolled over the four ring slots of G, which makes every LDS address a lane constant plus an immediate
-// (address arithmetic and remainders per row block had made it 2.5 times as long), and loads run two row blocks ahead.
+// (address arithmetic and remainders per row block had made it 2.5 times as long), and loads run two row blocks ahead.  What wraps
+// from slot 0 to the last one does so by a mask of the address: chosen by comparisons, sixteen of them stayed in scalar
+// registers and the rest of the loop's went to lanes of vector ones (28.2 us where this takes 26.3; B = 8, L = 512, 12 heads).
 constexpr int kGBlk = 2048, kGRing = 4, kKRing = 6;
 constexpr int kTgOffK = kGRing * kTile, kTgOffG = kTgOffK + kKRing * kTile, kTgLds = kTgOffG + 4 * kGRing * kGBlk;
 static_assert(kTgLds <= 80 * 1024, "two workgroups per CU");
+static_assert(kTgOffG % (kGRing * kGBlk) == 0, "a wave's ring of G wraps by a mask of its address");
 
 template <class QT>
 __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBwdRingParams p) {
@@ -820,7 +825,11 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(yt[2 * d + 1] + tile + 2048 * c + 1024));
     return __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  const uint32_t q_lane = (uint32_t)srow * (uint32_t)(p.q_st * 2) + chunk_off, k_lane = (uint32_t)srow * (uint32_t)(p.k_st * 2) + chunk_off;
+  const int R = (int)own_sgpr((uint32_t)p.R);
+  const bool causal = p.causal != 0;
+  const char* const zeros = own_sgpr((const char*)p.zero_block);
+  const uint32_t q_rowb = own_sgpr((uint32_t)(p.q_st * 2)), k_rowb = own_sgpr((uint32_t)(p.k_st * 2)), g_step = own_sgpr((uint32_t)(p.g_slots * kGBlk));
+  const uint32_t q_lane = (uint32_t)srow * q_rowb + chunk_off, k_lane = (uint32_t)srow * k_rowb + chunk_off;
   const uint32_t u_lane = g_base + (uint32_t)(li * 66 + g * 256);   // G element (row 4 g + li, column li) of ring slot 0
   for (int it = it0; it < it1; ++it) {
     const int b = it / p.tg_chunks, c0 = it % p.tg_chunks;
@@ -834,27 +843,27 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     // What is fetched next: row block I of q and of G, row block J = I - 1 - rho0 of k (the wave w = 0 uses the newest).  The places in
     // memory and the zones of I's tile are carried along: computed per row block they were two thirds of a turn's instructions.
     int I = I0, J = I0 - 1 - rho0;
-    const int64_t q_step = p.q_st * 64, k_step = p.k_st * 64, g_step = (int64_t)p.g_slots * kGBlk;
+    const uint64_t q_step = (uint64_t)q_rowb * 32, k_step = (uint64_t)k_rowb * 32;
     const char* const q_rows = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2;
     const char* const k_rows = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2;
-    uint64_t q_at = (uint64_t)(uintptr_t)q_rows + (uint64_t)(I * q_step), k_at = (uint64_t)(uintptr_t)k_rows + (uint64_t)(J * k_step);
-    uint64_t g_at = (uint64_t)(uintptr_t)p.g_blocks + (uint64_t)((((int64_t)b * p.H + h) * p.g_rows + I) * g_step);
+    uint64_t q_at = (uint64_t)(uintptr_t)q_rows + (uint64_t)(uint32_t)I * q_step, k_at = (uint64_t)(uintptr_t)k_rows + (uint64_t)((int64_t)J * (int64_t)k_step);
+    uint64_t g_at = (uint64_t)(uintptr_t)p.g_blocks + (uint64_t)(((int64_t)b * p.H + h) * p.g_rows + I) * g_step;
     int z0 = 0, zn = -1;   // first near step of the tile, number of near steps or -1
     auto zone_at = [&](int row_block) __attribute__((always_inline)) {
-      const Zones z = zones_of(row_block / 4 * FDB_BM, Lb, p.R, p.causal, true);
+      const Zones z = zones_of(row_block / 4 * FDB_BM, Lb, R, causal, true);
       z0 = z.s0;
       zn = z.s1 > z.s0 ? z.s1 - z.s0 : -1;
     };
-    auto clamped_dma = [&](const char* rows, int64_t step, int blk, uint32_t dst) __attribute__((always_inline)) {
+    auto clamped_dma = [&](const char* rows, uint32_t rowb, int blk, uint32_t dst) __attribute__((always_inline)) {
       const int row = max(0, min(blk * 32 + srow, Lb - 1));   // rows outside the sequence: finite values that meet zeros
-      dma16n(rows + (int64_t)row * (step / 32) + chunk_off, dst + wave_kb);
+      dma16n(rows + (uint64_t)(uint32_t)row * rowb + chunk_off, dst + wave_kb);
     };
     // block (I, rho) into a ring slot; a block of zeros where the dQ launch met no such block (no near step, or outside the
     // sequence).  Returns whether there is one.
     auto g_dma = [&](int row_block, uint64_t at, uint32_t ring) __attribute__((always_inline)) {
       const int k = row_block - rho - z0;
       const bool there = (uint32_t)row_block < (uint32_t)n_rows && k >= 0 && k <= zn;
-      const char* src = there ? (const char*)(uintptr_t)(at + (uint64_t)((int64_t)k * kGBlk)) : p.zero_block;
+      const char* src = there ? (const char*)(uintptr_t)(at + (uint64_t)((int64_t)k * kGBlk)) : zeros;
       dma16sn(src, lane * 16, g_base + ring * kGBlk);
       dma16sn(src + 1024, lane * 16, g_base + ring * kGBlk + 1024);
       return there;
@@ -863,20 +872,20 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     for (int w = 1; w < 4; ++w) {
       const int blk = J - w;
       const uint32_t dst = kTgOffK + (uint32_t)(kKRing - w) * kTile;
-      if ((uint32_t)blk < (uint32_t)full) dma16sn(k_rows + blk * k_step, k_lane, dst + wave_kb);
-      else clamped_dma(k_rows, k_step, blk, dst);
+      if ((uint32_t)blk < (uint32_t)full) dma16sn(k_rows + (uint64_t)(uint32_t)blk * k_step, k_lane, dst + wave_kb);
+      else clamped_dma(k_rows, k_rowb, blk, dst);
     }
     zone_at(max(I - 1, 0));
-    bool prev = g_dma(I - 1, g_at - (uint64_t)g_step, kGRing - 1);
+    bool prev = g_dma(I - 1, g_at - g_step, kGRing - 1);
     auto fetch = [&](uint32_t ring, uint32_t kslot) __attribute__((always_inline)) {   // what the next row block needs first, four loads per wave
       if (I < full) dma16sn((const char*)(uintptr_t)q_at, q_lane, ring * kTile + wave_kb);
-      else clamped_dma(q_rows, q_step, I, ring * kTile);
+      else clamped_dma(q_rows, q_rowb, I, ring * kTile);
       if ((uint32_t)J < (uint32_t)full) dma16sn((const char*)(uintptr_t)k_at, k_lane, kTgOffK + kslot * kTile + wave_kb);
-      else clamped_dma(k_rows, k_step, J, kTgOffK + kslot * kTile);
+      else clamped_dma(k_rows, k_rowb, J, kTgOffK + kslot * kTile);
       if ((I & 3) == 0) zone_at(I);
       const bool there = g_dma(I, g_at, ring);
       ++I, ++J;
-      q_at += (uint64_t)q_step, k_at += (uint64_t)k_step, g_at += (uint64_t)g_step;
+      q_at += q_step, k_at += k_step, g_at += g_step;
       return there;
     };
     bool cur = fetch(0, 0), next = fetch(1, 1);
@@ -906,7 +915,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
             // row of G behind (key row 16 c + 8 (e/4) + 4 g + e%4, position li), counted from block I - 1 on: o0 + 4 g + li
             const int o0 = 16 * c + 8 * (e >> 2) + (e & 3);
             uint32_t at = u_lane + PREV * kGBlk + o0 * 64;
-            if (RING == 0) at -= 4 * g + li + o0 >= 32 ? kGRing * kGBlk : 0;   // block I lies in slot 0, block I - 1 in the last one
+            if (RING == 0) at = (at & (kGRing * kGBlk - 1)) | g_base;   // block I lies in slot 0, block I - 1 in the last one
             a[e] = *(LDS_AS const short*)(uintptr_t)at;
           }
           gq[c] = __builtin_bit_cast(frag, a);

@@ -297,6 +297,23 @@ __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles
   h = __builtin_amdgcn_readfirstlane(h);
 }
 
+// A kernel argument in scalar registers of its own.  The compiler loads arguments sixteen registers at a time; where a loop wants
+// more scalar registers than there are, it keeps such a group in lanes of a vector register and brings all sixteen back
+// (sixteen v_readlane) for the one argument a step uses.  50 of some 330 instructions of a near step in e4m3: 889 -> 883 us at B = 4,
+// L = 8192, 12 heads; 124 in the loops of the backward's launch of both roles: 75.4 -> 71.2 us at B = 8, L = 512, twelve heads.  The 16-bit
+// near kernel keeps none in its loops, and is slower with the copies.
+__device__ __forceinline__ uint32_t own_sgpr(uint32_t x) {
+  uint32_t r;
+  asm("s_mov_b32 %0, %1" : "=&s"(r) : "s"(__builtin_amdgcn_readfirstlane(x)));
+  return r;
+}
+template <class T>
+__device__ __forceinline__ const T* own_sgpr(const T* x) {
+  const uint64_t a = (uint64_t)(uintptr_t)x;
+  const uint32_t lo = own_sgpr((uint32_t)a), hi = own_sgpr((uint32_t)(a >> 32));
+  return (const T*)(uintptr_t)(((uint64_t)hi << 32) | lo);
+}
+
 // 16 bytes per lane from global memory straight into LDS: lane l's data lands at lds_base + 16*l
 // (lds_base: byte offset in the workgroup's LDS, the same in every lane).  Issued through asm so
 // that the compiler keeps no account of it: the kernel waits for these loads itself, with

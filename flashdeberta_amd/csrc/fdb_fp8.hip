@@ -441,7 +441,9 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   char* ob = p.out + (oo + (int64_t)tok0 * p.o_st + (int64_t)h * p.o_sh) * 2;
   const char* pkb = C2P ? p.pk + (int64_t)h * p.pk_sh : nullptr;
   const char* pqb = P2C ? p.pq + (int64_t)h * p.pq_sh : nullptr;
-  const uint32_t k_rsb = (uint32_t)p.k_st, v_rsb = (uint32_t)(p.v_st * 2);
+  const uint32_t k_rsb = own_sgpr((uint32_t)p.k_st), v_rsb = own_sgpr((uint32_t)(p.v_st * 2));
+  const uint16_t* lut = own_sgpr((const uint16_t*)p.lut);
+  const int R = (int)own_sgpr((uint32_t)p.R);
   // units: the content product and the sum are in s_q s_k; C arrives in s_q s_kr (and scaled by 2^-kCShift), P in s_k s_qr
   const float s_q = p.qs[h], s_k = p.ks[h];
   const float x_scale = p.scale_log2 * s_q * s_k;
@@ -509,19 +511,17 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   };
   int r_tab = r_hi0 - row8;  // relative position of this thread's row of a batch; runs down by 32 per batch
   auto batch_delta = [&]() __attribute__((always_inline)) {
-    const int d = (int)((const uint16_t*)p.lut)[max(-p.R, min(p.R, r_tab)) + p.R];
+    const int d = (int)lut[(uint32_t)(max(-R, min(R, r_tab)) + R)];
     r_tab -= 32;
     return d;
   };
-  const uint32_t ek_lds = lds0 + (uint32_t)(EK - smem) + half_kb, eq_lds = lds0 + (uint32_t)(EQ - smem) + half_kb;
-  const uint32_t pk_rowb = (uint32_t)p.pk_sr, pq_rowb = (uint32_t)p.pq_sr;  // the host bounds them (24-bit row strides)
+  // The ring this wave's loads fill, E_K (waves 0, 1) or E_Q (waves 2, 3): chosen once, so that a step loads without a branch.
+  const bool ring_k = C2P && (!P2C || wave < 2), ring_on = (wave < 2) == ring_k;
+  const uint32_t ring_lds = lds0 + (uint32_t)((ring_k ? EK : EQ) - smem) + half_kb;
+  const char* ring_src = own_sgpr(ring_k ? pkb : pqb);
+  const uint32_t ring_rowb = own_sgpr((uint32_t)(ring_k ? p.pk_sr : p.pq_sr));  // the host bounds them (24-bit row strides)
   auto batch_dma = [&](int delta, int slot) __attribute__((always_inline)) {
-    const uint32_t seg = (uint32_t)slot * (32 * kRow8);
-    if (wave < 2) {
-      if constexpr (C2P) dma16sn(pkb, __umul24((uint32_t)delta, pk_rowb) + chunk8, ek_lds + seg);
-    } else {
-      if constexpr (P2C) dma16sn(pqb, __umul24((uint32_t)delta, pq_rowb) + chunk8, eq_lds + seg);
-    }
+    if ((C2P && P2C) || ring_on) dma16sn(ring_src, __umul24((uint32_t)delta, ring_rowb) + chunk8, ring_lds + (uint32_t)slot * (32 * kRow8));
   };
 
   f32x16 o_acc[DBLKS];
