@@ -266,8 +266,11 @@ __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { re
 // taken together as leave their K and V in an XCD's 4 MB of L2: 96 query tiles of 16-bit head_dim 64 are 3 MB.  The host passes
 // that number (fdb_groups_together): each division here costs every workgroup some 40 instructions before its first load.
 enum { kNatural = 0, kEdgesFirst = 1, kMiddleFirst = 2, kLastFirst = 3 };
-__device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles_per_seq, int most, bool fixed, int order, int& b, int& t,
-                                          int& h) {
+__device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles_per_seq, int most, bool fixed, int order, int& b_out, int& t_out,
+                                          int& h_out) {
+  // Not the caller's variables: the compiler makes one store, to a chosen address, of the two branches' stores, and the numbers then
+  // pass through scratch memory before a workgroup's first load.  Forward of 1 x 4096, 16 heads: 119.5 -> 117.9 us.
+  int b, t, h;
   if (fixed) {
     const int groups = batch * heads;
     const int first = n / (most * tiles_per_seq) * most;
@@ -292,9 +295,9 @@ __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles
   }
   // the divisions run on vector registers: taken back, or every address that depends on these stays there too (the e4m3 near kernel
   // spills 52 registers then)
-  b = __builtin_amdgcn_readfirstlane(b);
-  t = __builtin_amdgcn_readfirstlane(t);
-  h = __builtin_amdgcn_readfirstlane(h);
+  b_out = __builtin_amdgcn_readfirstlane(b);
+  t_out = __builtin_amdgcn_readfirstlane(t);
+  h_out = __builtin_amdgcn_readfirstlane(h);
 }
 
 // A kernel argument in scalar registers of its own.  The compiler loads arguments sixteen registers at a time; where a loop wants
