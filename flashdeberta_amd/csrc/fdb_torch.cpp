@@ -222,11 +222,28 @@ void product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias
   if (!library_product(a, trans_a, b, trans_b, d, bias, accumulate)) torch_product(a, trans_a, b, trans_b, d, bias, accumulate);
 }
 
+// The projections of a padded batch's real rows, x [batch * length, k]: the attention reads no other row of them.  Whether it was done.
+struct Lengths {
+  const OptTensor &start, &len;
+};
+bool project_real(const Tensor& x, const Tensor& w, const Tensor& b, int64_t cols, const Tensor& out, int64_t batch, int64_t length, const Lengths& real) {
+  const OptTensor &start = real.start, &len = real.len;
+  const int64_t k = x.size(-1);
+  if (!len || !fdb_gemm_real_serves(batch, length, cols, k, k)) return false;
+  for (const OptTensor* t : {&start, &len})
+    if (*t && ((*t)->scalar_type() != at::kInt || !(*t)->is_contiguous() || (*t)->numel() != batch || (*t)->device() != x.device() || !plain_memory(**t))) return false;
+  const int rc = fdb_gemm_real(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), start ? (const int32_t*)start->data_ptr() : nullptr, (const int32_t*)len->data_ptr(),
+                               (int32_t)batch, (int32_t)length, (int32_t)cols, (int32_t)k, k, w.stride(0), cols, fdb_dtype_of(x.scalar_type()), stream_of(x));
+  if (rc > 0) check(rc, "fdb_gemm_real");
+  return rc == 0;   // a negative code: a size or an alignment it is not built for
+}
+
 // x [..., K] . w [N, K]^T + bias -> [..., N], followed by GELU or an addition of `residual` [..., N] where asked for, as torch computes
 // them one after the other: bit for bit (the library's choice is torch's, and fdb_gemm adds up as it does).  With `own`, a product of at
 // most 32 rows takes the library's streaming kernel, whose waves share the contraction.
 enum class Then { nothing, gelu, add };
-Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool own, Then then = Then::nothing, const Tensor* residual = nullptr) {
+// With `real`, only the rows that a padded batch's lengths name have to be there.
+Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool own, Then then = Then::nothing, const Tensor* residual = nullptr, const Lengths* real = nullptr) {
   const auto type = x_in.scalar_type();
   const bool half = type == at::kBFloat16 || type == at::kHalf;
   const int64_t k = x_in.size(-1), m = k > 0 ? x_in.numel() / k : 0;
@@ -250,6 +267,7 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
     if (rc == 0) return rest(out);
     if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
   }
+  if (real && then == Then::nothing && x.dim() == 3 && project_real(x, w, *bias, n, out, x.size(0), x.size(1), *real)) return out;
   const int epilogue = then == Then::gelu ? FDB_GEMM_GELU : then == Then::add ? FDB_GEMM_RESIDUAL : FDB_GEMM_PLAIN;
   if (fdb_gemm_serves(m, n, k, epilogue)) {
     Tensor r;
@@ -748,7 +766,8 @@ struct LayerCall {
 // The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
 Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, const LayerCall& call, bool own) {
   TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be [B, L, hidden]");
-  const Tensor qkv = project(hidden, weight, bias, own);
+  const Lengths real{call.o.seq_start, call.o.seq_len};
+  const Tensor qkv = project(hidden, weight, bias, own, Then::nothing, nullptr, &real);
   TORCH_CHECK(qkv.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", qkv.device());
   const auto type = qkv.scalar_type();
   TORCH_CHECK_VALUE(fdb_dtype_of(type) >= 0, "unsupported dtype ", type);
@@ -772,7 +791,7 @@ Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTens
 // One layer's attention in training, from the hidden states and the relative embeddings through the three projections (shared
 // by the tables): a node of its own.  What autograd would run as one product per projection and tensor, a reduction per bias and
 // an addition per shared tensor is here
-//   forward   q | k | v = hidden . W^T + b and Q_r | K_r = rel . W[q, k]^T + b[q, k], W the three weights on top of each other;
+//   forward   q | k | v = hidden . W^T + b (of a long padded batch the real rows) and Q_r | K_r = rel . W[q, k]^T + b[q, k], W the three weights on top of each other;
 //   backward  d hidden = d qkv . W,  d W = d qkv^T . hidden (+ d pos^T . rel onto the rows of q and k),  d rel = d pos . W[q, k],
 //             d b = the column sums of d qkv and d pos.
 struct LayerArgs {
@@ -817,7 +836,7 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     Tensor w, b;
     std::tie(w, b) = joined(qw, qb, kw, kb, vw, vb, type, stream_of(hidden));
     const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
-    projected(hidden, B * L, w, b, 3 * W, qkv);
+    if (!project_real(hidden, w, b, 3 * W, qkv, B, L, {args->o.seq_start, args->o.seq_len})) projected(hidden, B * L, w, b, 3 * W, qkv);
     projected(rel, rows, w, b, 2 * W, pos);
     const Tensor out = at::empty({B, L, W}, hidden.options());
     fdb_attn_args a = {};
@@ -956,8 +975,8 @@ PyObject* py_layer_attention(PyObject*, PyObject* const* x, Py_ssize_t n) {
 
 // encoder_layer(hidden, weight, bias, pos_key, ..., seq_len [as layer_attention], out_weight, out_bias, norm1_weight, norm1_bias, eps1,
 //               up_weight, up_bias, down_weight, down_bias, norm2_weight, norm2_bias, eps2) -> hidden states of the next layer
-// A whole post-norm encoder layer with GELU; the caller has checked that the layer is one.  Every product, sum, norm and GELU is
-// the one its modules would run, in the same order, so the result has the same bits: in a 16-bit type twelve layers turn one
+// A whole post-norm encoder layer with GELU; the caller has checked that the layer is one.  Products, sums, norms and GELU round where its
+// modules' would, and the products add up in the same order, so the result has the same bits: in a 16-bit type twelve layers turn one
 // differing rounding into a percent.
 PyObject* py_encoder_layer(PyObject*, PyObject* const* x, Py_ssize_t n) {
   HANDLE_TH_ERRORS

@@ -386,6 +386,16 @@ int fdb_gemm(const void* x, const void* w, const void* bias, const void* residua
 int32_t fdb_gemm_serves(int64_t rows, int64_t cols, int64_t depth, int32_t epilogue);
 
 /*
+ * fdb_gemm's plain product for the real rows of a padded batch, x and out [batch * seqlen, ..]: of sequence b the rows seq_start[b] (NULL: 0) up
+ * to seq_start[b] + seq_len[b] (negative: none), clamped to its seqlen rows, as fdb_attn_args reads them.  The other rows of out are not
+ * written.  batch <= 64, all rows of x within 2 GB.  fdb_gemm_real_serves: whether it is the faster way for a size (host, no GPU).
+ * The reference projects padding along with the text (src/flashdeberta/model.py:147-149).
+ */
+int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
+                  int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream);
+int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t cols, int64_t depth, int64_t ldx);
+
+/*
  * The products of a layer's training backward (FDB_BF16 / FDB_F16; contiguous row-major matrices aligned to 16 bytes, the workspace to 32;
  * depth and all column counts multiples of 64).  Two problems that share weights are one launch each:
  *   fdb_dgrad: out_i [rows_i, cols] = x_i [rows_i, depth_i] . w, the first depth_i rows of w [.., cols] (rows_i 0: none);
