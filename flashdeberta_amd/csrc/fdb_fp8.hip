@@ -19,7 +19,10 @@
 //                     in two LDS rings, C through a per-wave fp16 scratch that holds both blocks of a step, P by lane
 //                     rotations) on 64-byte rows: 4 score MFMAs per step instead of 16.  The three products have the units s_q s_k, s_q s_kr
 //                     and s_k s_qr: the content product accumulates on top of C * (s_kr / s_k), P enters as
-//                     fma(P, s_qr / s_q, .), and one factor s_q s_k sm_scale log2(e) converts the sum.
+//                     fma(P, s_qr / s_q, .), and one factor s_q s_k sm_scale log2(e) converts the sum.  Where the far launch would have
+//                     little to do it walks the far tiles, too, first and without rings: P is the product of the keys with one
+//                     row of Q_r, the MFMA's other operand in every column, and C a number per row, in fp32.  Nothing is folded into
+//                     an e4m3 query there: the output's error against 64 bits is a half to a quarter of the two launches'.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -397,7 +400,7 @@ __device__ __forceinline__ void lds_wait_all8() { asm volatile("s_waitcnt lgkmcn
 // (168 registers per lane at three workgroups per CU do not hold them), which is why the ring of E_Q has a sixth batch: the
 // batch a step's loads overwrite must not be one that a wave still reads in that step.  Per wave and step one e4m3 MFMA
 // each for the content product and C, two for P, four bf16 MFMAs for P V.
-template <bool C2P, bool P2C>
+template <bool C2P, bool P2C, bool ALL>
 __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams p) {
   constexpr int D = 64, DBLKS = 2;
   using VT = Bf16Tr;
@@ -461,16 +464,23 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   if (p.causal) j_end = min(Lb, m0 + FDB_BM);
   const int n_tiles = (j_end + FDB_BN - 1) / FDB_BN;
   const int lim = m0 - (FDB_BN - 1) - p.R;
-  const int t0 = lim >= 0 && !p.near_all ? min(n_tiles, lim / FDB_BN + 1) : 0;
-  const int t1 = p.near_all ? n_tiles : max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
+  const int t0 = lim >= 0 ? min(n_tiles, lim / FDB_BN + 1) : 0;
+  const int t1 = max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
   int s0 = 2 * t0;
   int s1 = max(s0, min(2 * t1, (j_end + kStep - 1) / kStep));
+  int all0 = s0, all1 = s1;  // ALL: the far steps on both sides with them
+  if constexpr (ALL) all0 = 0, all1 = (j_end + kStep - 1) / kStep;
   if (p.near_parts > 1) {
-    const int all = s1 - s0, part = (int)blockIdx.y;
-    s1 = s0 + (int)((int64_t)all * (part + 1) / p.near_parts);
-    s0 = s0 + (int)((int64_t)all * part / p.near_parts);
+    const int all = all1 - all0, part = (int)blockIdx.y;
+    all1 = all0 + (int)((int64_t)all * (part + 1) / p.near_parts);
+    all0 = all0 + (int)((int64_t)all * part / p.near_parts);
   }
+  s0 = ALL ? min(max(s0, all0), all1) : all0;
+  s1 = ALL ? max(s0, min(s1, all1)) : all1;
   const int n_steps = s1 - s0;
+  // ALL: the far steps left and right of them, walked first, as t = -n_far .. -1
+  const int n_left = ALL ? s0 - all0 : 0, n_right = ALL ? all1 - s1 : 0, n_far = n_left + n_right;
+  auto far_step_at = [&](int t) __attribute__((always_inline)) { return t < -n_right ? s0 + n_right + t : t < 0 ? all1 + t : s0; };
   const int n_full = max(0, min(n_steps, (p.causal ? min(Lb, m0) : Lb) / kStep - s0));
   // u = r_hi0 - r counts downwards from the first step's largest r; batch = u / 32, ring slot = batch mod 5 (E_K) or 6 (E_Q).  Wave w's
   // block bk at step k is batch k + 4 - w - bk, MFMA row m its row 31 - m: r = iw0 - 32 s - 32 + 32 bk + m.
@@ -574,22 +584,114 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   int slot_k = 4 - wave, slot_q = 4 - wave;  // ring slots of this wave's block 0
   const int ring_n = wave < 2 ? kRingBatchesK : kRingBatchesQ;  // the ring this wave's loads fill
   int slot_dma = wave < 2 ? 0 : 5;                              // and the slot of it that the step's loads fill
+  // ALL: what the far steps of a side start from (side 0: left of the near steps, delta(R); 1: right of them, delta(-R))
+  float row_add = 0.f;                          // C of the row, in the exponent's unit
+  i32x8 eq = {0, 0, 0, 0, 0, 0, 0, 0};          // the row of Q_r that all keys of the side meet
+  auto side_begins = [&](int side) __attribute__((always_inline)) {
+    const int delta = p.lut[side == 0 ? 2 * p.R : 0];
+    if constexpr (P2C) {
+      const char* row = pqb + (int64_t)delta * p.pq_sr + 32 * g;
+      eq = frag8(*(const u32x4*)row, *(const u32x4*)(row + 16));
+    }
+    if constexpr (C2P) {
+      const char* row = pkb + (int64_t)delta * p.pk_sr + 32 * g;
+      const i32x8 kr = frag8(*(const u32x4*)row, *(const u32x4*)(row + 16));
+      float acc = 0.f;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) {
+        const f32x4 q4 = e4m3x4((uint32_t)qf[w]), k4 = e4m3x4((uint32_t)kr[w]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_fmaf(q4[e], k4[e], acc);
+      }
+      row_add = wave_half_sum(acc) * (p.scale_log2 * s_q * p.pks[h]);
+    }
+    asm volatile("" ::"v"(eq));  // consumed ahead of the loop, like the query
+  };
   // ---- prologue -----------------------------------------------------------------------------------------------
-  if (n_steps > 0) {
-    k_dma(s0, 0);
-    v_dma(s0, 0);
-    int d0[6];
+  auto near_begins = [&]() __attribute__((always_inline)) {
+    if constexpr (C2P) c_store(mma8_sa<127 - kCShift>(ring_frag(ek0, 3 - wave), qf, zero), 1);  // block 1 of step 0
+  };
+  if (n_steps + n_far > 0) {
+    k_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1);
+    v_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1);
+    if (!ALL || n_steps > 0) {
+      int d0[6];
 #pragma unroll
-    for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
+      for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
 #pragma unroll
-    for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
+      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
 #pragma unroll
-    for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
-    dnext = d0[5];
+      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
+      dnext = d0[5];
+    }
+    if constexpr (ALL)
+      if (n_far > 0) side_begins(n_left > 0 ? 0 : 1);
     wait_vmcnt<0>();
     __syncthreads();
-    if constexpr (C2P) c_store(mma8_sa<127 - kCShift>(ring_frag(ek0, 3 - wave), qf, zero), 1);  // block 1 of step 0
+    if constexpr (!ALL) near_begins();
   }
+
+  auto read_v = [&](vfrag (&vfr)[2][DBLKS], uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int d = 0; d < DBLKS; ++d) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + buf + 2048 * c));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + buf + 2048 * c + 1024));
+        vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+  };
+  auto mask_keys = [&](f32x16& sacc, int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
+      if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+    }
+  };
+  // online soft-max in base 2 over a step's scores sacc * x_scale + add, O^T += V^T P^T
+  auto take = [&](auto mask_tag, const f32x16& sacc, float add, const vfrag (&vfr)[2][DBLKS]) __attribute__((always_inline)) {
+    constexpr bool MASK = decltype(mask_tag)::value;
+    vfrag pf[2];
+    float l_blk = 0.f;
+    auto probs = [&](float off) __attribute__((always_inline)) {
+      l_blk = 0.f;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        f32x8 pv;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * c + (e ^ 3)], x_scale, off));
+        pf[c] = VT::from_f32(pv);
+        l_blk = sum8(pv, l_blk);
+      }
+    };
+    bool slow = __any(m_run == -INFINITY);
+    if (!slow) {
+      probs(add - m_run);
+      slow = __any(!(l_blk <= 256.f));
+    }
+    if (slow) {
+      float mx = sacc[0];
+#pragma unroll
+      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
+      mx = __builtin_fmaf(wave_half_max(mx), x_scale, add);
+      if (__any(mx > m_run + kLazyTau)) {
+        const float m_new = (mx > m_run + kLazyTau) ? mx : m_run;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+        m_run = m_new;
+#pragma unroll
+        for (int d = 0; d < DBLKS; ++d)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
+      }
+      probs((MASK && m_run == -INFINITY) ? 0.f : add - m_run);
+    }
+    l_run += l_blk;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
+  };
 
   auto step = [&](auto mask_tag, auto par_tag, int k) __attribute__((always_inline)) {
     constexpr bool MASK = decltype(mask_tag)::value;
@@ -637,14 +739,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
         rotate16<28>(xs, px, std::make_integer_sequence<int, 16>{});
     }
     vfrag vfr[2][DBLKS];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int d = 0; d < DBLKS; ++d) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + PAR * N8::V_BYTES + 2048 * c));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + PAR * N8::V_BYTES + 2048 * c + 1024));
-        vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      }
+    read_v(vfr, PAR * N8::V_BYTES);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (C2P || P2C) {
       lds_wait_all8();
@@ -659,57 +754,42 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
       if constexpr (C2P) sacc[v] = __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)craw[v]), rho_c, sacc[v]);
       if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], rho_p, sacc[v]);
     }
-    if constexpr (MASK) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
-        if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
-      }
-    }
-    vfrag pf[2];
-    float l_blk = 0.f;
-    auto probs = [&](float off) __attribute__((always_inline)) {
-      l_blk = 0.f;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x8 pv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[8 * c + (e ^ 3)], x_scale, off));
-        pf[c] = VT::from_f32(pv);
-        l_blk = sum8(pv, l_blk);
-      }
-    };
-    bool slow = __any(m_run == -INFINITY);
-    if (!slow) {
-      probs(-m_run);
-      slow = __any(!(l_blk <= 256.f));
-    }
-    if (slow) {
-      float mx = sacc[0];
-#pragma unroll
-      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
-      mx = wave_half_max(mx) * x_scale;
-      if (__any(mx > m_run + kLazyTau)) {
-        const float m_new = (mx > m_run + kLazyTau) ? mx : m_run;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        l_run *= alpha;
-        m_run = m_new;
-#pragma unroll
-        for (int d = 0; d < DBLKS; ++d)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
-      }
-      probs((MASK && m_run == -INFINITY) ? 0.f : -m_run);
-    }
-    l_run += l_blk;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
+    if constexpr (MASK) mask_keys(sacc, j0);
+    take(mask_tag, sacc, 0.f, vfr);
     slot_k = slot_k == kRingBatchesK - 1 ? 0 : slot_k + 1;
     slot_q = slot_q == kRingBatchesQ - 1 ? 0 : slot_q + 1;
     slot_dma = slot_dma == ring_n - 1 ? 0 : slot_dma + 1;
   };
+  // ---- far steps (ALL): their K and V go through the two buffers so that the first near step finds its own in buffer 0
+  auto far_steps = [&](auto mask_tag, int t, int end) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (; t < end; ++t) {
+      const int s = far_step_at(t), next = far_step_at(t + 1), par = t & 1;
+      wait_vmcnt<0>();
+      __syncthreads();
+      k_dma(next, par ^ 1);
+      v_dma(next, par ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const i32x8 kf = lds_frag8(kx0 + par * N8::K_BYTES, kx1 + par * N8::K_BYTES);
+      vfrag vfr[2][DBLKS];
+      read_v(vfr, par * N8::V_BYTES);
+      f32x16 sacc = mma8(kf, qf, zero);
+      if constexpr (P2C) {
+        const f32x16 pacc = mma8(kf, eq, zero);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sacc[v] = __builtin_fmaf(pacc[v], rho_p, sacc[v]);
+      }
+      if constexpr (decltype(mask_tag)::value)
+        if ((s + 1) * kStep > Lb) mask_keys(sacc, s * kStep);
+      take(mask_tag, sacc, row_add, vfr);
+    }
+  };
+  if constexpr (ALL) {
+    far_steps(std::false_type{}, -n_far, -n_right);
+    if (n_left > 0 && n_right > 0) side_begins(1);
+    far_steps(std::true_type{}, -n_right, 0);
+    if (n_steps > 0) near_begins();  // the rings' rows have been waited for, here or in the first far step
+  }
   {
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
@@ -756,20 +836,20 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
             l_tot > 0.f ? (m_run + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f : -INFINITY;
       return;
     }
-    const int n_far = p.far_done ? p.far_parts : 0;
+    const int far_parts = !ALL && p.far_done ? p.far_parts : 0;
     float w_far[FDB_MAX_FAR_PARTS], w_near = 1.f, m_out = m_run;
     const char* far_row[FDB_MAX_FAR_PARTS];
 #pragma unroll
     for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) {
       w_far[s] = -INFINITY;
       far_row[s] = orow;
-      if (s < n_far) {
+      if (s < far_parts) {
         const float* lp = s == 0 ? p.lse : far_part_lse(p, s, D * 2);
         w_far[s] = lp[tok * p.H + h] * 1.4426950408889634f;
         if (s > 0) far_row[s] = far_part_out(p, s, D * 2) + (tok * p.H + h) * (D * 2);
       }
     }
-    if (n_far > 0) {
+    if (far_parts > 0) {
       m_out = m_run + __builtin_amdgcn_logf(l_tot);
 #pragma unroll
       for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) m_out = fmaxf(m_out, w_far[s]);
@@ -778,7 +858,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
     float denom = w_near * l_tot;
 #pragma unroll
     for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) {
-      w_far[s] = (s < n_far && w_far[s] != -INFINITY) ? __builtin_amdgcn_exp2f(w_far[s] - m_out) : 0.f;
+      w_far[s] = (s < far_parts && w_far[s] != -INFINITY) ? __builtin_amdgcn_exp2f(w_far[s] - m_out) : 0.f;
       denom += w_far[s];
     }
     const float inv = denom > 0.f ? 1.f / denom : 0.f;
@@ -791,7 +871,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
         float f0 = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
 #pragma unroll
         for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s)
-          if (s < n_far) {
+          if (s < far_parts) {
             const f32x4 far4 = VT::load4(far_row[s] + off);
             const float sf = w_far[s] * inv;
             f0 += far4[0] * sf; f1 += far4[1] * sf; f2 += far4[2] * sf; f3 += far4[3] * sf;
@@ -803,9 +883,9 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   }
 }
 
-template <bool C2P, bool P2C>
+template <bool C2P, bool P2C, bool ALL>
 int launch_near8_one(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  auto kern = fdb_near8_kernel<C2P, P2C>;
+  auto kern = fdb_near8_kernel<C2P, P2C, ALL>;
   constexpr int lds = N8::lds_bytes(C2P, P2C);
   static_assert(lds <= 52 * 1024, "three workgroups per CU: with 53 KB a CU was seen to take only two");
   static std::atomic<uint64_t> lds_set{0};
@@ -814,6 +894,13 @@ int launch_near8_one(const FdbKParams& p, int grid_x, hipStream_t stream) {
   hipLaunchKernelGGL(kern, dim3((unsigned)grid_x * p.H, p.near_parts > 1 ? (unsigned)p.near_parts : 1u, 1), dim3(kThreads), lds,
                      stream, p);
   return (int)hipGetLastError();
+}
+template <bool ALL>
+int launch_near8(const FdbKParams& p, int grid_x, hipStream_t stream) {
+  if (p.pk && p.pq) return launch_near8_one<true, true, ALL>(p, grid_x, stream);
+  if (p.pk) return launch_near8_one<true, false, ALL>(p, grid_x, stream);
+  if (p.pq) return launch_near8_one<false, true, ALL>(p, grid_x, stream);
+  return FDB_ERR_UNSUPPORTED;
 }
 
 }  // namespace
@@ -830,8 +917,5 @@ int fdb_launch_far8(const FdbKParams& p, int grid_x, void* stream_) {
 
 int fdb_launch_near8(const FdbKParams& p, int grid_x, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
-  if (p.pk && p.pq) return launch_near8_one<true, true>(p, grid_x, stream);
-  if (p.pk) return launch_near8_one<true, false>(p, grid_x, stream);
-  if (p.pq) return launch_near8_one<false, true>(p, grid_x, stream);
-  return FDB_ERR_UNSUPPORTED;
+  return p.near_all ? launch_near8<true>(p, grid_x, stream) : launch_near8<false>(p, grid_x, stream);
 }

@@ -27,6 +27,11 @@
 //   reference point, so the sum leaves for the exponential as it is.
 // LDS: K 2 x 4 KB + V 2 x 4 KB + rings 2 x 20 KB + scratch 17 KB = 73 KB.
 //
+// Where the far launch would have little to do (near_takes_all in fdb_api.cpp) the launch walks the far tiles, too (ALL).  Beyond the
+// table's reach a step needs neither rings nor scratch: every key of a side has the same relative rows, and the scores are formed as the far
+// launch forms them, with the row of Q_r added to the query and c2p as a number per query row, kept in fp32.  (The scratch would round
+// that number to 16 bits, once for all far keys of the row: the log-sum-exp's error was up to 2.6 times the two launches' that way.)
+//
 // Staging goes global -> LDS directly (global_load_lds_dwordx4: no staging registers, no LDS write
 // instructions of the waves' own) and runs one step ahead: right after the one barrier of step s (every
 // wave is done with step s-1) a wave issues its share of K(s+1) and V(s+1) into the buffers step s does not
@@ -98,7 +103,7 @@ __device__ __forceinline__ float lds_elem_f32(uint32_t addr) {
 }
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <class QT, class VT, bool C2P, bool P2C>
+template <class QT, class VT, bool C2P, bool P2C, bool ALL>
 __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams p) {
   constexpr int D = 64, KS = 4, DBLKS = 2;
   using qfrag = typename QT::frag;
@@ -167,16 +172,24 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   if (p.causal) j_end = min(Lb, m0 + FDB_BM);
   const int n_tiles = (j_end + FDB_BN - 1) / FDB_BN;
   const int lim = m0 - (FDB_BN - 1) - p.R;
-  const int t0 = lim >= 0 && !p.near_all ? min(n_tiles, lim / FDB_BN + 1) : 0;
-  const int t1 = p.near_all ? n_tiles : max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
+  const int t0 = lim >= 0 ? min(n_tiles, lim / FDB_BN + 1) : 0;
+  const int t1 = max(t0, min(n_tiles, (m0 + FDB_BM - 1 + p.R + FDB_BN - 1) / FDB_BN));
   int s0 = 2 * t0;                                                         // first 32-key step
   int s1 = max(s0, min(2 * t1, (j_end + kStep - 1) / kStep));              // one past the last
+  int all0 = s0, all1 = s1;                                                // ALL: the far steps on both sides with them
+  if constexpr (ALL) all0 = 0, all1 = (j_end + kStep - 1) / kStep;
   if (p.near_parts > 1) {  // this workgroup's share of the steps
-    const int all = s1 - s0, part = (int)blockIdx.y;
-    s1 = s0 + (int)((int64_t)all * (part + 1) / p.near_parts);
-    s0 = s0 + (int)((int64_t)all * part / p.near_parts);
+    const int all = all1 - all0, part = (int)blockIdx.y;
+    all1 = all0 + (int)((int64_t)all * (part + 1) / p.near_parts);
+    all0 = all0 + (int)((int64_t)all * part / p.near_parts);
   }
+  s0 = ALL ? min(max(s0, all0), all1) : all0;
+  s1 = ALL ? max(s0, min(s1, all1)) : all1;
   const int n_steps = s1 - s0;
+  // ALL: the far steps left and right of them, walked first (the near steps then keep nothing of theirs in registers), as t = -n_far .. -1
+  const int n_left = ALL ? s0 - all0 : 0, n_right = ALL ? all1 - s1 : 0, n_far = n_left + n_right;
+  auto far_step_at = [&](int t) __attribute__((always_inline)) { return t < -n_right ? s0 + n_right + t : t < 0 ? all1 + t : s0; };
+
   const int n_full = max(0, min(n_steps, (p.causal ? min(Lb, m0) : Lb) / kStep - s0));  // steps k < n_full need no mask
 
   // relative positions of the workgroup at step k = s - s0: r in [r_hi0 - 32k - 159, r_hi0 - 32k];
@@ -240,7 +253,8 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
 #pragma unroll
     for (int v = 0; v < 16; ++v) o_acc[d][v] = 0.f;
   float m_run = -INFINITY, l_run = 0.f;
-  // the content product's accumulator starts from minus the row's reference point (0 before the row has one)
+  float row_add = 0.f;  // ALL: what a row's scores of the range at hand have in common, c2p of the far keys or nothing
+  // the content product's accumulator starts from row_add minus the row's reference point (0 before the row has one)
   f32x16 negm;
 #pragma unroll
   for (int v = 0; v < 16; ++v) negm[v] = 0.f;
@@ -309,23 +323,34 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   };
   int slot_rd = 4 - wave;  // ring slot of this wave's block 0
   int slot_dma = 0;        // ring slot the step's loads fill
-  // ---- prologue: step 0's K and ring batches 0..4 on their way to LDS -------------------------------------
+  // ALL: what the far steps of a side start from (side 0: left of the near steps, delta(R); 1: right of them, delta(-R))
+  qfrag qx[ALL ? KS : 1];
+  auto range_begins = [&](float add) __attribute__((always_inline)) {
+    row_add = add;
+    const float nm = add - (m_run == -INFINITY ? 0.f : m_run);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) negm[v] = nm;
+  };
+  auto side_begins = [&](int side) __attribute__((always_inline)) {
+    const int delta = p.lut[side == 0 ? 2 * p.R : 0];
+    float acc = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int off = (16 * s + 8 * g) * 2;
+      f32x8 q8 = QT::to_f32(i < Lb ? QT::load(qb + (int64_t)i * p.q_st * 2 + off) : QT::zero());
+      if constexpr (C2P) {
+        const f32x8 a = QT::to_f32(QT::load(pkb + (int64_t)delta * p.pk_sr * 2 + off));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc = __builtin_fmaf(a[e], q8[e], acc);
+      }
+      if constexpr (P2C) q8 += QT::to_f32(QT::load(pqb + (int64_t)delta * p.pq_sr * 2 + off));
+      qx[s] = QT::from_f32(q8 * x_scale);
+    }
+    range_begins(C2P ? wave_half_sum(acc) * x_scale : 0.f);
+  };
+  // ---- prologue: the first step's K and V and ring batches 0..4 on their way to LDS ------------------------
   // All table values first, then all rows: the loads of one kind are in flight together.
-  if (n_steps > 0) {
-    k_dma(s0, 0, false);  // K and V need no table value: on their way while the table is read
-    v_dma(s0, 0, false);
-    int d0[6];
-#pragma unroll
-    for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
-    // (taken here, all at once: the compiler, which does not count the direct loads, would otherwise wait for
-    // each value at its use, behind all the direct loads issued before it)
-#pragma unroll
-    for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
-#pragma unroll
-    for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
-    dnext = d0[5];
-    wait_vmcnt<0>();
-    __syncthreads();  // the prologue's ring rows
+  auto near_begins = [&]() __attribute__((always_inline)) {
     ring_read(1, 3 - wave);  // block 1 of step 0
     if constexpr (C2P) {
       f32x16 c1;
@@ -333,7 +358,102 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
       for (int x = 0; x < KS; ++x) c1 = QT::mma(ac[x], qf[x], x == 0 ? zero : c1);
       c_store(c1, 1);
     }
+  };
+  if (n_steps + n_far > 0) {
+    k_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);  // K and V need no table value: on their way while the table is read
+    v_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);
+    if (!ALL || n_steps > 0) {
+      int d0[6];
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
+      // (taken here, all at once: the compiler, which does not count the direct loads, would otherwise wait for
+      // each value at its use, behind all the direct loads issued before it)
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
+#pragma unroll
+      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
+      dnext = d0[5];
+    }
+    if constexpr (ALL)
+      if (__builtin_expect(n_far > 0, 0)) side_begins(n_left > 0 ? 0 : 1);  // (far code out of the way of the tiles that have none)
+    wait_vmcnt<0>();
+    __syncthreads();  // the prologue's ring rows
+    if constexpr (!ALL) near_begins();
   }
+
+  // V^T operands of the step in the buffer at byte `buf` of V's two
+  auto read_v = [&](vfrag (&vfr)[2][DBLKS], uint32_t buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int d = 0; d < DBLKS; ++d) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + buf + 2048 * c));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + buf + 2048 * c + 1024));
+        vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+  };
+  auto mask_keys = [&](f32x16& sacc, int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
+      if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+    }
+  };
+  // Online soft-max in base 2 over a step's scores, O^T += V^T P^T.
+  // sacc = score - reference point.  The probabilities are formed first; the half-row sum of a step bounds its
+  // largest one, so while it stays under 2^kLazyTau nothing has to move and no maximum is taken.  Otherwise (or
+  // before a row has a reference point) the wave takes the maximum, moves the reference points of the rows that
+  // need it, shifts the step's scores and forms the probabilities again.
+  auto take = [&](f32x16& sacc, const vfrag (&vfr)[2][DBLKS]) __attribute__((always_inline)) {
+    vfrag pf[2];
+    float l_blk = 0.f;
+    auto probs = [&]() __attribute__((always_inline)) {
+      l_blk = 0.f;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        f32x8 pv;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(sacc[8 * c + (e ^ 3)]);  // the V^T operand takes the keys in ascending order
+        pf[c] = VT::from_f32(pv);
+        l_blk = sum8(pv, l_blk);
+      }
+    };
+    const bool first = m_run == -INFINITY;
+    bool slow = __any(first);
+    if (!slow) {
+      probs();
+      slow = __any(!(l_blk <= 256.f));  // 2^kLazyTau; also true for an overflow
+    }
+    if (slow) {
+      float mx = sacc[0];
+#pragma unroll
+      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
+      mx = wave_half_max(mx);  // relative to the reference point (to 0 while the row has none)
+      const bool mv = first ? mx > -INFINITY : mx > kLazyTau;
+      if (__any(mv)) {
+        const float shift = mv ? mx : 0.f;
+        const float alpha = first ? 0.f : __builtin_amdgcn_exp2f(-shift);  // 1 where nothing moves
+        if (mv) m_run = (first ? 0.f : m_run) + shift;
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < DBLKS; ++d)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sacc[v] -= shift;
+        float nm = m_run == -INFINITY ? 0.f : -m_run;
+        if constexpr (ALL) nm += row_add;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) negm[v] = nm;
+      }
+      probs();
+    }
+    l_run += l_blk;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
+  };
 
   auto step = [&](auto mask_tag, auto par_tag, auto next_tag, int k) __attribute__((always_inline)) {
     constexpr bool MASK = decltype(mask_tag)::value;
@@ -411,14 +531,7 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     }
     // V^T operands requested here, ahead of the soft-max, so that the four MFMAs at the end of the step find them
     vfrag vfr[2][DBLKS];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int d = 0; d < DBLKS; ++d) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + PAR * NCfg::V_BYTES + 2048 * c));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + PAR * NCfg::V_BYTES + 2048 * c + 1024));
-        vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-      }
+    read_v(vfr, PAR * NCfg::V_BYTES);
     __builtin_amdgcn_sched_barrier(0);
     // one wait for the band of C and the rotated P (issued as asm: the compiler keeps no count of them)
     if constexpr (C2P || P2C) {
@@ -434,68 +547,43 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
       if constexpr (C2P) sacc[v] += cband[v];
       if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v]);
     }
-    // ---- mask, online soft-max in base 2, O^T += V^T P^T ---------------------------------------------------
-    if constexpr (MASK) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
-        if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
-      }
-    }
-    // sacc = score - reference point.  The probabilities are formed first; the half-row sum of a step bounds its
-    // largest one, so while it stays under 2^kLazyTau nothing has to move and no maximum is taken.  Otherwise (or
-    // before a row has a reference point) the wave takes the maximum, moves the reference points of the rows that
-    // need it, shifts the step's scores and forms the probabilities again.
-    vfrag pf[2];
-    float l_blk = 0.f;
-    auto probs = [&]() __attribute__((always_inline)) {
-      l_blk = 0.f;
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        f32x8 pv;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pv[e] = __builtin_amdgcn_exp2f(sacc[8 * c + (e ^ 3)]);  // the V^T operand takes the keys in ascending order
-        pf[c] = VT::from_f32(pv);
-        l_blk = sum8(pv, l_blk);
-      }
-    };
-    const bool first = m_run == -INFINITY;
-    bool slow = __any(first);
-    if (!slow) {
-      probs();
-      slow = __any(!(l_blk <= 256.f));  // 2^kLazyTau; also true for an overflow
-    }
-    if (slow) {
-      float mx = sacc[0];
-#pragma unroll
-      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
-      mx = wave_half_max(mx);  // relative to the reference point (to 0 while the row has none)
-      const bool mv = first ? mx > -INFINITY : mx > kLazyTau;
-      if (__any(mv)) {
-        const float shift = mv ? mx : 0.f;
-        const float alpha = first ? 0.f : __builtin_amdgcn_exp2f(-shift);  // 1 where nothing moves
-        if (mv) m_run = (first ? 0.f : m_run) + shift;
-        l_run *= alpha;
-#pragma unroll
-        for (int d = 0; d < DBLKS; ++d)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sacc[v] -= shift;
-        const float nm = m_run == -INFINITY ? 0.f : -m_run;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) negm[v] = nm;
-      }
-      probs();
-    }
-    l_run += l_blk;
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
+    if constexpr (MASK) mask_keys(sacc, j0);
+    take(sacc, vfr);
     slot_rd = slot_rd == kRingBatches - 1 ? 0 : slot_rd + 1;
     slot_dma = slot_dma == kRingBatches - 1 ? 0 : slot_dma + 1;
   };
+  // ---- far steps (ALL): their K and V go through the two buffers so that the first near step finds its own in buffer 0
+  auto far_steps = [&](auto mask_tag, int t, int end) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (; t < end; ++t) {
+      const int s = far_step_at(t), next = far_step_at(t + 1), par = t & 1;
+      wait_vmcnt<0>();
+      __syncthreads();
+      k_dma(next, par ^ 1, false);
+      v_dma(next, par ^ 1, false);
+      __builtin_amdgcn_sched_barrier(0);
+      qfrag kf[KS];
+#pragma unroll
+      for (int x = 0; x < KS; ++x) kf[x] = *(LDS_AS const qfrag*)(uintptr_t)(klx[x] + par * NCfg::K_BYTES);
+      vfrag vfr[2][DBLKS];
+      read_v(vfr, par * NCfg::V_BYTES);
+      f32x16 sacc;
+#pragma unroll
+      for (int x = 0; x < KS; ++x) sacc = QT::mma(kf[x], qx[x], x == 0 ? negm : sacc);
+      if constexpr (decltype(mask_tag)::value)
+        if ((s + 1) * kStep > Lb) mask_keys(sacc, s * kStep);
+      take(sacc, vfr);
+    }
+  };
+  if constexpr (ALL) {
+    if (__builtin_expect(n_far > 0, 0)) {
+      far_steps(std::false_type{}, -n_far, -n_right);
+      if (n_left > 0 && n_right > 0) side_begins(1);
+      far_steps(std::true_type{}, -n_right, 0);
+      range_begins(0.f);
+    }
+    if (n_steps > 0) near_begins();  // the rings' rows have been waited for, above or in the first far step
+  }
   {
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
@@ -553,20 +641,20 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     }
     // far partial results: part 0 in out / lse, the others in the workspace (rows normalised over their
     // keys, log-sum-exp -inf where a row had none)
-    const int n_far = p.far_done ? p.far_parts : 0;
+    const int far_parts = !ALL && p.far_done ? p.far_parts : 0;
     float w_far[FDB_MAX_FAR_PARTS], w_near = 1.f, m_out = m_run;
     const char* far_row[FDB_MAX_FAR_PARTS];
 #pragma unroll
     for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) {
       w_far[s] = -INFINITY;  // log-sum-exp in base 2 until the maximum is known
       far_row[s] = orow;
-      if (s < n_far) {
+      if (s < far_parts) {
         const float* lp = s == 0 ? p.lse : far_part_lse(p, s, D * 2);
         w_far[s] = lp[tok * p.H + h] * 1.4426950408889634f;
         if (s > 0) far_row[s] = far_part_out(p, s, D * 2) + (tok * p.H + h) * (D * 2);
       }
     }
-    if (n_far > 0) {
+    if (far_parts > 0) {
       m_out = m_run + __builtin_amdgcn_logf(l_tot);
 #pragma unroll
       for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) m_out = fmaxf(m_out, w_far[s]);
@@ -575,7 +663,7 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     float denom = w_near * l_tot;
 #pragma unroll
     for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s) {
-      w_far[s] = (s < n_far && w_far[s] != -INFINITY) ? __builtin_amdgcn_exp2f(w_far[s] - m_out) : 0.f;
+      w_far[s] = (s < far_parts && w_far[s] != -INFINITY) ? __builtin_amdgcn_exp2f(w_far[s] - m_out) : 0.f;
       denom += w_far[s];
     }
     const float inv = denom > 0.f ? 1.f / denom : 0.f;
@@ -588,7 +676,7 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
         float f0 = 0.f, f1 = 0.f, f2 = 0.f, f3 = 0.f;
 #pragma unroll
         for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s)
-          if (s < n_far) {
+          if (s < far_parts) {
             const f32x4 far4 = VT::load4(far_row[s] + off);
             const float sf = w_far[s] * inv;
             f0 += far4[0] * sf; f1 += far4[1] * sf; f2 += far4[2] * sf; f3 += far4[3] * sf;
@@ -600,9 +688,9 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   }
 }
 
-template <class QT, bool C2P, bool P2C>
+template <class QT, bool C2P, bool P2C, bool ALL>
 int launch_near_one(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  auto kern = fdb_near_kernel<QT, QT, C2P, P2C>;
+  auto kern = fdb_near_kernel<QT, QT, C2P, P2C, ALL>;
   constexpr int lds = NCfg::lds_bytes(C2P, P2C);
   static_assert(lds <= 80 * 1024, "two workgroups per CU");
   static std::atomic<uint64_t> lds_set{0};
@@ -613,12 +701,16 @@ int launch_near_one(const FdbKParams& p, int grid_x, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-template <class QT>
+template <class QT, bool ALL>
 int launch_near_pos(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  if (p.pk && p.pq) return launch_near_one<QT, true, true>(p, grid_x, stream);
-  if (p.pk) return launch_near_one<QT, true, false>(p, grid_x, stream);
-  if (p.pq) return launch_near_one<QT, false, true>(p, grid_x, stream);
+  if (p.pk && p.pq) return launch_near_one<QT, true, true, ALL>(p, grid_x, stream);
+  if (p.pk) return launch_near_one<QT, true, false, ALL>(p, grid_x, stream);
+  if (p.pq) return launch_near_one<QT, false, true, ALL>(p, grid_x, stream);
   return FDB_ERR_UNSUPPORTED;
+}
+template <class QT>
+int launch_near(const FdbKParams& p, int grid_x, hipStream_t stream) {
+  return p.near_all ? launch_near_pos<QT, true>(p, grid_x, stream) : launch_near_pos<QT, false>(p, grid_x, stream);
 }
 
 }  // namespace
@@ -629,7 +721,7 @@ bool fdb_near32_supported(int dtype, int head_dim) {
 
 int fdb_launch_near32(const FdbKParams& p, int dtype, int grid_x, void* stream_) {
   hipStream_t stream = (hipStream_t)stream_;
-  if (dtype == FDB_BF16) return launch_near_pos<Bf16Tr>(p, grid_x, stream);
-  if (dtype == FDB_F16) return launch_near_pos<F16Tr>(p, grid_x, stream);
+  if (dtype == FDB_BF16) return launch_near<Bf16Tr>(p, grid_x, stream);
+  if (dtype == FDB_F16) return launch_near<F16Tr>(p, grid_x, stream);
   return FDB_ERR_UNSUPPORTED;
 }
