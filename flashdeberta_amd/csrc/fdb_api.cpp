@@ -106,33 +106,27 @@ bool has_far_launch(const fdb_attn_args* a) {
          longest > radius + FDB_BN - 1;
 }
 
-int near_parts_wanted(const fdb_attn_args* a);
-
-// Whether the near launch walks the far tiles, too, and the far launch is left out.  A far tile costs the near kernel some four times what it
-// costs the far kernel, but a launch of few far tiles costs 6 to 8 us whatever it does, and while every query tile has a workgroup slot the
-// near launch lasts as long as its longest query tile, in mid-sequence, which has few far tiles or none.  12 heads, bf16, two launches -> one:
-//   3 x 777 39.7 -> 30.0 us, 1 x 700 28.4 -> 21.3, 8 x 640 46.0 -> 36.9, 8 x 777 80.9 -> 67.7, 4 x 1024 56.9 -> 51.2, 1 x 1300 44.0 -> 40.7;
-// kept as two where one is slower: 2 x 1300 58.4 (62.5), 2 x 1501 61.6 (71.0), 6 x 1024 81.6 (82.4).
+// Whether the near launch walks the far tiles, too, and the far launch is left out.  A far step costs a near workgroup, two of which share a CU,
+// more than it costs a far one, three of which do; but the far launch costs 6 to 8 us whatever it does, a first and a last round of
+// its own, and a partial result that is written and read again.  So the far tiles decide, counted for the query tile at an end of the sequence, which
+// has the most of them: the line is where the calls measured change sides.  12 heads unless stated, two launches -> one, us:
+//   radius 512       bf16                    e4m3                      radius 64 and 256   bf16                    e4m3
+//   1 x 700          28.7 -> 22.1            28.0 -> 21.4              8 x 300, 64         27.6 -> 21.4            25.7 -> 18.7
+//   3 x 777          39.9 -> 31.1            38.8 -> 30.2              3 x 777, 64         30.4 -> 25.4            29.0 -> 24.2
+//   16 x 1024        170.2 -> 146.1          124.9 -> 110.5            16 x 1024, 64       112.5 -> 101.9          96.0 -> 83.8
+//   2 x 1501         61.7 -> 57.1            57.9 -> 52.4              4 x 1501, 64        69.0 -> 69.8            55.9 -> 53.1
+//   16 x 1501        296.5 -> 267.6          221.5 -> 202.7            2 x 2048, 64        54.9 -> 61.2 (kept)     49.6 -> 59.2 (kept)
+//   3 x 2048         109.3 -> 111.6          82.7 -> 79.3              1 x 2048, 4 h., 64  32.7 -> 41.6 (kept)     32.0 -> 42.4 (kept)
+//   8 x 2048         223.3 -> 213.7          177.3 -> 170.6            8 x 1024, 256       78.3 -> 67.9            61.2 -> 52.7
+//   1 x 2048, 4 h.   42.2 -> 27.6            41.3 -> 27.4              8 x 1501, 256       131.0 -> 124.0          111.0 -> 103.1
+// fp16 runs as bf16 does (16 x 1501 304.2 -> 279.4, 3 x 2048 114.4 -> 115.4).  Without a workspace, when nothing is shared: 1 x 2048, 4 heads 61.5 -> 54.7, 1 x 1300
+// 53.9 -> 44.4, 1 x 700 35.0 -> 27.1 (e4m3 60.8 -> 54.4, 52.6 -> 42.7, 34.2 -> 26.9).
 bool near_takes_all(const fdb_attn_args* a) {
   if (!has_far_launch(a) || !steps32_supported(a->dtype, a->head_dim) || a->cu_seqlens || a->causal || a->far_splits > 0 || a->near_splits > 0) return false;
   if (a->max_seqlen > 16 * FDB_BM) return false;
-  const int tiles = (a->max_seqlen + FDB_BM - 1) / FDB_BM, n64 = (a->max_seqlen + FDB_BN - 1) / FDB_BN, radius = a->lut_radius > 0 ? a->lut_radius : 1;
-  int most_near = 0, most_far = 0, far_tiles = 0;
-  for (int t = 0; t < tiles; ++t) {
-    const int m0 = t * FDB_BM, lim = m0 - (FDB_BN - 1) - radius;
-    const int t0 = lim >= 0 ? std::min(n64, lim / FDB_BN + 1) : 0, t1 = std::max(t0, std::min(n64, (m0 + FDB_BM - 1 + radius + FDB_BN - 1) / FDB_BN));
-    most_near = std::max(most_near, t1 - t0);
-    most_far = std::max(most_far, n64 - (t1 - t0));
-    far_tiles += n64 - (t1 - t0);
-  }
-  // microseconds, from the sizes above: a near step takes 1.43 in a launch that ends on its short tiles, 1.6 where all have the same length
-  // and some share a compute unit, and 0.85 of a slot's time where there are several rounds; the far launch has its longest workgroup or its total
-  const int64_t wgs = (int64_t)tiles * a->batch * a->heads;
-  const double all = (double)far_tiles * a->batch * a->heads / cu_count();
-  const int parts = near_parts_wanted(a);
-  const double alone = 2 * n64 * (wgs * parts <= cu_count() ? 1.43 : 1.6) - 2 * most_near * 1.43;
-  const double more = std::max(alone / parts, wgs > 2 * cu_count() ? 1.7 * all : 0.0), far = std::max(3.0 + 0.65 * most_far, 6.0 + 0.43 * all);
-  return more < far;
+  const int radius = a->lut_radius > 0 ? a->lut_radius : 1;
+  const int tiles = (a->max_seqlen + FDB_BN - 1) / FDB_BN, near = (FDB_BM - 1 + radius + FDB_BN - 1) / FDB_BN;   // of the first query tile
+  return tiles - near <= 22;
 }
 
 // Workgroups per query tile of the far-only launch.  That launch keeps three workgroups on a CU; when

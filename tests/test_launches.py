@@ -1,0 +1,54 @@
+"""The launches that calls take (tests/launches.py: on the host, without a GPU)."""
+import pytest
+
+from flashdeberta_amd import _lib
+from launches import P, launches
+
+
+def _forward(batch, seqlen, heads=12, dtype=_lib.FDB_BF16, radius=512, workspace=0, **more):
+    a = _lib.FdbAttnArgs()
+    for n in ("q", "k", "v", "out", "pos_key", "pos_query", "lse", "delta_lut", "q_scale", "k_scale", "pk_scale", "pq_scale"):
+        setattr(a, n, 0x1000)
+    a.batch, a.heads, a.head_dim, a.dtype, a.max_seqlen, a.total_tokens = batch, heads, 64, dtype, seqlen, batch * seqlen
+    a.att_span, a.lut_radius, a.sm_scale = radius // 2, radius, 0.1
+    a.workspace, a.workspace_bytes = 0x100000 if workspace else None, workspace
+    for n, v in more.items():
+        setattr(a, n, v)
+    return "fdb_attn_fwd", [a, None]
+
+
+def _kinds(made):
+    """far, near (the near steps alone), all (the near launch with the far tiles) or merge, and the shares"""
+    out = []
+    for name, _, shares, _ in made:
+        all_tiles = "near" in name and name.split("EEv10FdbKParams")[0].endswith("Lb1E")
+        out.append(("merge" if "merge" in name else "far" if "far8" in name or "attn_kernel" in name else "all" if all_tiles else "near", shares))
+    return out
+
+
+ALL = 1 << 32   # a workspace for whatever the call wants
+
+
+@pytest.mark.parametrize("dtype", [_lib.FDB_BF16, _lib.FDB_F16, _lib.FDB_FP8_E4M3], ids=["bf16", "fp16", "e4m3"])
+def test_where_the_near_launch_takes_the_far_tiles(dtype):
+    """By the sizes alone: a caller without a workspace, whose tiles are not shared, takes the same kernels."""
+    call = lambda *a, **kw: _forward(*a, dtype=dtype, **kw)
+    cases = [
+        (call(1, 575, workspace=ALL), [("near", 2), ("merge", 1)]),          # no key is far
+        (call(1, 576, workspace=ALL), [("all", 2), ("merge", 1)]),
+        (call(1, 576), [("all", 1)]),
+        (call(1, 2048, 4, workspace=ALL), [("all", 4), ("merge", 1)]),
+        (call(1, 2048, 4), [("all", 1)]),
+        (call(2, 1501), [("all", 1)]),
+        (call(64, 700), [("all", 1)]),
+        (call(1, 2049), [("far", 1), ("near", 1)]),
+        (call(8, 4096), [("far", 1), ("near", 1)]),
+        (call(1, 1600, radius=64), [("all", 1)]),                            # 22 far tiles at the end of the sequence
+        (call(1, 1601, radius=64), [("far", 1), ("near", 1)]),
+        (call(1, 1000, causal=1), [("far", 1), ("near", 1)]),
+        (call(1, 1000, far_splits=1), [("far", 1), ("near", 1)]),
+        (call(1, 1000, near_splits=1), [("far", 1), ("near", 1)]),
+        (call(1, 1000, cu_seqlens=0x1000, worklist=0x1000), [("far", 1), ("near", 1)]),
+    ]
+    for (_, want), (rc, made) in zip(cases, launches([c for c, _ in cases])):
+        assert rc == 0 and _kinds(made) == want, (want, made)
