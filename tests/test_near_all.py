@@ -64,10 +64,11 @@ def test_calls_that_keep_two_launches():
     assert ws() == (1 + near) * part(2048)
 
 
-def _rms(B, L, H, kind, **kw):
-    """Root mean squares of the errors of the output and of the log-sum-exp [L, H], first batch row, against 64 bits on the operands as the kernels get them."""
+def _errors(B, L, H, kind, buckets=256, most=512, **kw):
+    """Errors of the output [L, H, 64] and of the log-sum-exp [L, H], first batch row, against 64 bits on the operands as the kernels get them."""
     q, k, v, pk, pq = _inputs(B, L, H, (1, 1), torch.float16 if kind == "fp16" else torch.bfloat16)
-    call, given = dict(position_buckets=256, max_relative_positions=512, return_lse=True, **kw), [x.cuda() for x in (q, k, v, pk, pq)]
+    pk, pq = pk[:, :2 * buckets], pq[:, :2 * buckets]
+    call, given = dict(position_buckets=buckets, max_relative_positions=most, return_lse=True, **kw), [x.cuda() for x in (q, k, v, pk, pq)]
     exact = [x.double() for x in (q, k, v, pk, pq)]
     if kind == "e4m3":
         eight = [ops.quantize_e4m3_per_head(x) for x in (given[0].view(B * L, H, 64), given[1].view(B * L, H, 64), given[3].transpose(0, 1), given[4].transpose(0, 1))]
@@ -77,11 +78,16 @@ def _rms(B, L, H, kind, **kw):
         given = [q8.view(B, L, H, 64), k8.view(B, L, H, 64), given[2], pk8.transpose(0, 1), pq8.transpose(0, 1)]
         call.update(q_scale=qs, k_scale=ks, pos_key_scale=pks, pos_query_scale=pqs)
     rows = lambda x: x[:1].numpy().transpose(0, 2, 1, 3)
-    ref, ref_lse = O.disentangled_attention(*[rows(x) for x in exact[:3]], exact[3].numpy(), exact[4].numpy(), 256, 512, return_lse=True)
+    ref, ref_lse = O.disentangled_attention(*[rows(x) for x in exact[:3]], exact[3].numpy(), exact[4].numpy(), buckets, most, return_lse=True)
     out, lse = ops.disentangled_attention_fwd(*given, **call)
     e = out[0].double().cpu().numpy() - ref[0].transpose(1, 0, 2)
-    el = lse.view(B, L, H)[0].double().cpu().numpy() - ref_lse[0].T
-    return np.sqrt((e * e).mean()), np.sqrt((el * el).mean()), np.sqrt((el[[0, 1, L - 2, L - 1]] ** 2).mean())
+    return e, lse.view(B, L, H)[0].double().cpu().numpy() - ref_lse[0].T
+
+
+def _rms(*args, **kw):
+    """... their root mean squares, and that of the log-sum-exp of the two rows at either end"""
+    e, el = _errors(*args, **kw)
+    return np.sqrt((e * e).mean()), np.sqrt((el * el).mean()), np.sqrt((el[[0, 1, -2, -1]] ** 2).mean())
 
 
 @pytest.mark.gpu
@@ -99,3 +105,15 @@ def test_e4m3_far_keys_add_nothing_to_the_rounding_of_c2p():
     """In e4m3 the near steps' c2p is cut to 16 bits, the far ones' is not: at the ends of 1500 tokens, where 700 at most are near, the log-sum-exp's
     error is that share (and less) of a call's whose keys are all near."""
     assert _rms(1, 1500, 4, "e4m3")[2] <= 700 / 1500 * 1.25 * _rms(1, 512, 12, "e4m3")[2]   # 32 rows: a root mean square known to a quarter
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "e4m3"])
+@pytest.mark.parametrize("shared", [True, False])
+# all near but one key; ragged last steps that are near and far ones; shares that hold no near step, far ones of either side or of both; the most tiles
+@pytest.mark.parametrize("L,H,buckets,most", [(577, 3, 256, 512), (193, 2, 32, 64), (641, 1, 32, 64), (1537, 2, 32, 64), (1600, 12, 32, 64), (1000, 1, 128, 256), (2048, 2, 256, 512), (1985, 12, 256, 512)])
+def test_far_steps_and_shares(L, H, buckets, most, shared, kind):
+    e, el = _errors(1, L, H, kind, buckets, most, **({} if shared else dict(workspace=torch.empty(256, dtype=torch.uint8, device="cuda"))))
+    eps = EPS[torch.float16 if kind == "fp16" else torch.bfloat16]
+    # as above; outputs are of magnitude 1 at most at these lengths, and e4m3's near c2p is cut to fp16: a score of 4 by 2^-9
+    assert np.abs(e).max() <= 3 * eps and np.abs(el).max() <= 2 * eps
