@@ -134,15 +134,18 @@ def test_strided_inputs_and_reference_call_shape():
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("B,L,pb,mr", [(2, 1500, 256, 512), (1, 700, 32, 64), (2, 300, 256, 512)])
 def test_one_kernel_and_two_kernel_paths_agree(dtype, B, L, pb, mr):
-    """With a log-sum-exp buffer the library runs the far tiles and the near tiles as two launches;
-    without one a single kernel walks every tile.  Both must match the oracle and each other."""
+    """With a log-sum-exp buffer the library runs the far tiles and the near tiles as two launches, or
+    as one near launch where few tiles are far (far_splits=1 asks for two); without one a single kernel walks
+    every tile.  All must match the oracle and each other."""
     q, k, v, pk, pq = _inputs(B, L, 3, 64, pb, mr, dtype, 77, 1.0)
     args = [_dev(x) for x in (q, k, v, pk, pq)]
     kw = dict(position_buckets=pb, max_relative_positions=mr)
-    two = ops.disentangled_attention_fwd(*args, **kw)
+    two = ops.disentangled_attention_fwd(*args, far_splits=1, **kw)
+    own = ops.disentangled_attention_fwd(*args, **kw)
     one = ops.disentangled_attention_fwd(*args, single_kernel=True, **kw)
     ref = _oracle_blhd(q, k, v, pk, pq, pb, mr)
     _check(two, ref, TOL[dtype], "two launches")
+    _check(own, ref, TOL[dtype], "the library's choice")
     _check(one, ref, TOL[dtype], "one launch")
     assert (two.float() - one.float()).abs().max().item() <= TOL[dtype]
 
@@ -160,10 +163,11 @@ def test_two_launch_variants(causal, c2p, p2c, D, L):
     kernels (one or two position terms, causal, head_dim 32 / 64, ragged tails)."""
     q, k, v, pk, pq = _inputs(2, L, 2, D, 256, 512, torch.bfloat16, 31 + L, 1.0, c2p, p2c)
     ref, ref_lse = _oracle_blhd(q, k, v, pk, pq, 256, 512, causal=causal, return_lse=True)
-    out, lse = ops.disentangled_attention_fwd(_dev(q), _dev(k), _dev(v), _dev(pk), _dev(pq), position_buckets=256,
-                                              max_relative_positions=512, causal=causal, return_lse=True)
-    _check(out, ref, TOL[torch.bfloat16], "out")
-    _check(lse.view(2, L, 2), ref_lse, 4 * TOL[torch.bfloat16], "lse")
+    for choice in (dict(far_splits=1), {}):  # two launches by request, then whatever the library takes
+        out, lse = ops.disentangled_attention_fwd(_dev(q), _dev(k), _dev(v), _dev(pk), _dev(pq), position_buckets=256,
+                                                  max_relative_positions=512, causal=causal, return_lse=True, **choice)
+        _check(out, ref, TOL[torch.bfloat16], "out")
+        _check(lse.view(2, L, 2), ref_lse, 4 * TOL[torch.bfloat16], "lse")
 
 
 @pytest.mark.parametrize("splits", [2, 3, 4])
@@ -475,7 +479,7 @@ def _digit_run(term, dtype, D, L, pb, mr, layout, n_heads_per_call=3, **kw):
     return got
 
 
-@pytest.mark.parametrize("variant", ["plain", "packed", "left", "shared", "d32", "short_table"])
+@pytest.mark.parametrize("variant", ["plain", "packed", "left", "shared", "d32", "short_table", "one", "one_left", "one_short_table"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("term", ["c2p", "p2c"])
 def test_delta_indices_bit_exact_on_the_16_bit_kernels(term, dtype, variant):
@@ -484,8 +488,11 @@ def test_delta_indices_bit_exact_on_the_16_bit_kernels(term, dtype, variant):
     L = 1300 with 256 buckets over 512 positions has far tiles on both sides, both zone edges and the linear,
     logarithmic and saturated parts of the table.  Variants: the plain fixed layout, a packed batch, a batch
     padded on the left, far keys shared by three and near steps by two workgroups, head_dim 32, and a short
-    table (32 buckets over 64 positions, L = 300) whose zones all fall inside one query tile."""
-    D, L, pb, mr, layout, kw = 64, 1300, 256, 512, "plain", {}
+    table (32 buckets over 64 positions, L = 300) whose zones all fall inside one query tile.  far_splits=1 asks for
+    the two launches; the variants "one" leave the choice to the library, which takes a near launch of all tiles."""
+    D, L, pb, mr, layout, kw = 64, 1300, 256, 512, "plain", dict(far_splits=1)
+    if variant.startswith("one"):
+        variant, kw = variant[4:], {}
     if variant in ("packed", "left"):
         layout = variant
     if variant == "shared":
@@ -626,8 +633,8 @@ def _fp8_pair_model(q8, qs, k8, ks, v, pk8, pks, pq8, pqs, pb, mr, causal=False)
     every (query tile of 128, key tile of 64) pair that is near, and for the far ones the kernel's documented
     rounding -- the folded query (s_q q + s_qr Q_r[delta]) sm_scale log2(e) s_k, formed in fp32 and rounded to e4m3
     once more with a power-of-two exponent of its row (its largest entry scaled into [128, 256)), the
-    content->position term as a per-row constant.  A call with no far launch (no sequence beyond radius + 63) is the
-    plain oracle."""
+    content->position term as a per-row constant.  A call with no far key (no sequence beyond radius + 63) is the
+    plain oracle, and so is one whose far tiles go through the near launch."""
     B, L, H, D = q8.shape
     has_pos = pk8 is not None or pq8 is not None
     c = 1.0 / np.sqrt(D * (1 + (pk8 is not None) + (pq8 is not None)))
@@ -779,8 +786,8 @@ def test_fp8_dequantisation_exact():
     assert torch.equal(got_t, ref)
 
 
-# single=False: the far / near pair of launches with e4m3 MFMA contractions (the default at head_dim 64);
-# single=True: the one-kernel e4m3 path
+# single=False: the far / near pair of launches with e4m3 MFMA contractions (far_splits=1: the library would take one near launch for
+# so few far tiles); single=True: the one-kernel e4m3 path
 @pytest.mark.parametrize("single", [False, True])
 @pytest.mark.parametrize("L,pb,mr", [(300, 32, 64), (1100, 256, 512)])
 def test_fp8_attention(L, pb, mr, single):
@@ -795,7 +802,7 @@ def test_fp8_attention(L, pb, mr, single):
         pq8, pqs = ops.quantize_e4m3_per_head(pq.cuda().transpose(0, 1))
         out = ops.disentangled_attention_fwd(q8, k8, v.cuda(), pk8.transpose(0, 1), pq8.transpose(0, 1), position_buckets=pb,
                                              max_relative_positions=mr, q_scale=qs, k_scale=ks, pos_key_scale=pks,
-                                             pos_query_scale=pqs, single_kernel=single)
+                                             pos_query_scale=pqs, single_kernel=single, far_splits=1)
         ref_dq = _oracle_blhd(dq(q8, qs), dq(k8, ks), v, dq(pk8, pks).transpose(0, 1), dq(pq8, pqs).transpose(0, 1), pb, mr)
         if single:
             return out, ref_dq, ref_dq
@@ -1772,6 +1779,7 @@ def test_random_fp8_variants(seed):
     if pair:  # far and near keys of a query tile shared out among workgroups, as the library would for few tiles
         kw["far_splits"], kw["near_splits"] = int(r.randint(4)), int(r.randint(4))
         what += " shares %d/%d" % (kw["far_splits"], kw["near_splits"])
+        pair = packed or causal or kw["far_splits"] > 0 or kw["near_splits"] > 0  # left to the library, one near launch takes the far tiles, too
 
     def reference(sl, batch):
         if not pair:

@@ -50,7 +50,7 @@ def test_padded_rows_in_the_near_launch():
         assert out[b].isfinite().all() and (out[b, :s] == 0).all() and (out[b, s + n:] == 0).all()
 
 
-def test_calls_that_keep_two_launches():
+def test_workspace_of_a_far_share():
     """A far share of its own has a workspace slot: none is asked for where the near launch takes all, whatever the number of near shares."""
     a = _lib.FdbAttnArgs()
     for n in ("q", "k", "v", "out", "pos_key", "pos_query", "lse", "delta_lut"):
