@@ -739,7 +739,10 @@ int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_
       (rows + 15) / 16 > 65535)
     return FDB_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || (reinterpret_cast<uintptr_t>(bias) & 1u)) return FDB_ERR_ALIGN;
-  if (rows > 32 && fdb_gemm(x, w, bias, nullptr, out, rows, cols, depth, ldx, ldw, ldo, 0, FDB_GEMM_PLAIN, dtype, stream) == FDB_OK) return FDB_OK;
+  if (rows > 32) {  // a negative code: a size or an alignment those tiles are not built for; a positive one is the runtime's
+    const int rc = fdb_gemm(x, w, bias, nullptr, out, rows, cols, depth, ldx, ldw, ldo, 0, FDB_GEMM_PLAIN, dtype, stream);
+    if (rc >= 0) return rc;
+  }
   return fdb_launch_linear(x, w, bias, out, rows, cols, depth, ldx, ldw, ldo, dtype, stream);
 }
 

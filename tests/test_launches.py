@@ -52,3 +52,13 @@ def test_where_the_near_launch_takes_the_far_tiles(dtype):
     ]
     for (_, want), (rc, made) in zip(cases, launches([c for c, _ in cases])):
         assert rc == 0 and _kinds(made) == want, (want, made)
+
+
+def _linear(rows, cols, depth, ldo=None, bias=P(0x1000)):
+    return "fdb_linear", [P(0x1000), P(0x1000), bias, P(0x1000), rows, cols, depth, depth, depth, ldo or cols, _lib.FDB_BF16, None]
+
+
+def test_an_error_of_the_runtime_ends_the_linear_layer():
+    for rows in (24, 100):
+        (rc, made), = launches([_linear(rows, 768, 768)], fails=1)
+        assert rc == 719 and len(made) == 1, (rc, made)
