@@ -38,7 +38,8 @@ __device__ __forceinline__ float gelu(float x) { return x * 0.5f * (1.f + erff(x
 constexpr uint32_t kGeluLow = (127 - 14) << 7, kGeluHigh = (127 + 3) << 7, kGeluCount = kGeluHigh - kGeluLow;   // bit patterns of bf16 magnitudes
 constexpr int kGeluBytes = 2 * kGeluCount * 2;   // [sign][magnitude - low]
 
-enum { kPlain = FDB_GEMM_PLAIN, kGelu = FDB_GEMM_GELU, kResidual = FDB_GEMM_RESIDUAL };   // out = y, gelu(y) or y + residual, y = x . w^T + bias rounded to the type
+enum { kPlain = FDB_GEMM_PLAIN, kGelu = FDB_GEMM_GELU, kResidual = FDB_GEMM_RESIDUAL, kNarrow = FDB_GEMM_NARROW };   // out = y, gelu(y) or y + residual, y = x . w^T +
+                                                                                   // bias rounded to the type; y by fours of columns, bias anywhere
 
 struct GemmParams {
   const char *x, *w, *bias, *residual;
@@ -148,7 +149,14 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
   for (int j = 0; j < S::FN; ++j) {
     const int col = (wn * S::FN + j) * 16 + 4 * kg;
     f32x4 b = {0.f, 0.f, 0.f, 0.f};
-    if (p.bias && n0 + col < p.N) b = QT::load4(p.bias + (int64_t)(n0 + col) * 2);
+    if (p.bias && n0 + col < p.N) {
+      if constexpr (EPI == kNarrow) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = (float)((const elem*)p.bias)[n0 + col + e];
+      } else {
+        b = QT::load4(p.bias + (int64_t)(n0 + col) * 2);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < S::FM; ++i) {
       f32x4 y = acc[i][j] + b;
@@ -178,11 +186,15 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
     }
   }
   __syncthreads();
-  constexpr int CH = TN / 8;
+  constexpr int CW = EPI == kNarrow ? 4 : 8, CH = TN / CW;
   for (int c = tid; c < TM * CH; c += 64 * S::NW) {
-    const int row = c / CH, col = (c - row * CH) * 8, m = m0 + row, nn = n0 + col;
+    const int row = c / CH, col = (c - row * CH) * CW, m = m0 + row, nn = n0 + col;
     if (m < rows.count && nn < p.N) {
       const int64_t at = rows.base(m0) + rows.from_base(m0, row);
+      if constexpr (EPI == kNarrow) {
+        *(u32x2*)(p.out + (at * p.ldo + nn) * 2) = *(const u32x2*)(smem + row * S::PITCH + col * 2);
+        continue;
+      }
       frag y = *(const frag*)(smem + row * S::PITCH + col * 2);
       if constexpr (EPI == kResidual) y = QT::from_f32(QT::to_f32(y) + QT::to_f32(QT::load(p.residual + (at * p.ldr + nn) * 2)));
       *(frag*)(p.out + (at * p.ldo + nn) * 2) = y;
@@ -340,6 +352,7 @@ template <class QT>
 int launch_type(const GemmParams& p, int epilogue, hipStream_t stream) {
   if (epilogue == kGelu) return launch_gemm<QT, kGelu>(p, stream);
   if (epilogue == kResidual) return launch_gemm<QT, kResidual>(p, stream);
+  if (epilogue == kNarrow) return launch_gemm<QT, kNarrow>(p, stream);
   return launch_gemm<QT, kPlain>(p, stream);
 }
 

@@ -4,7 +4,7 @@
 // launch costs 2.5.  Up to 32 rows fdb_linear_kernel streams the weights: one workgroup per 16 output columns, eight or
 // sixteen waves that share the contraction, so that even a [768 x 768] weight is on its way through 48 x 8 waves at once, each
 // with four steps' loads in flight.  In a replayed graph, [24 x 768] . [768 x 2304]: 4.0 us against hipBLASLt's 4.8.
-// Beyond that fdb_gemm.hip's tiles, for the sizes they take: [64 / 200 x 768] . [768 x 2304] 5.3 / 5.6 us.
+// Beyond that fdb_gemm.hip's tiles, for the sizes they take (columns and output rows by eights, or by fours where the streaming makes more than one round): [64 / 200 x 768] . [768 x 2304] 5.3 / 5.6 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

@@ -46,6 +46,23 @@ def test_tiles_and_their_remainders(M, N, K, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("M,N,K", [(33, 4, 64), (200, 772, 128), (1030, 516, 64), (1601, 1364, 64), (3000, 1164, 64), (5000, 1404, 64)])   # streamed, then each tile
+@pytest.mark.parametrize("pitch,shift", [(0, 0), (4, 0), (0, 1), (4, 3), (8, 2)])   # of the output's rows beyond N, and elements the bias is off 8 bytes by
+def test_linear_by_fours(M, N, K, pitch, shift, dtype):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = [(torch.randn(r, K, device="cuda", generator=g) * s).to(dtype) for r, s in ((M, 1.0), (N, K ** -0.5))]
+    bias = torch.randn(N + shift, device="cuda", generator=g).to(dtype)[shift:]
+    out = torch.full((M + 1, N + pitch), 7.0, device="cuda", dtype=dtype)
+    assert _lib.lib.fdb_linear(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), M, N, K, K, K, N + pitch,
+                               {torch.bfloat16: _lib.FDB_BF16, torch.float16: _lib.FDB_F16}[dtype], torch.cuda.current_stream().cuda_stream) == 0
+    assert (out[M] == 7.0).all() and (out[:, N:] == 7.0).all()
+    ref = x.double() @ w.double().t() + bias.double()
+    bound = torch.finfo(dtype).eps / 2 * ref.abs() * 1.01 + 1e-5   # one rounding of the result; the fp32 sums' own is smaller by 2^-10
+    assert ((out[:M, :N].double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 def test_gelu_of_every_value_is_torchs(dtype):
     """The product of zeros leaves the bias: all 65536 patterns, in rows of their own and beside ordinary values."""
     every = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(dtype)

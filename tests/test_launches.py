@@ -62,3 +62,12 @@ def test_an_error_of_the_runtime_ends_the_linear_layer():
     for rows in (24, 100):
         (rc, made), = launches([_linear(rows, 768, 768)], fails=1)
         assert rc == 719 and len(made) == 1, (rc, made)
+
+
+def test_linear_layers_of_many_rows_are_tiled():
+    """Columns or output rows by fours, a bias on any element, too: the streaming kernel reads all weights for every 32 rows.  It keeps what makes one
+    workgroup a compute unit, and what the tiles are not built for."""
+    calls = [_linear(200, 772, 768), _linear(200, 768, 768, ldo=772), _linear(200, 768, 768, bias=P(0x1002)), _linear(100, 768, 768), _linear(32, 772, 768),
+             _linear(160, 772, 768), _linear(200, 770, 768), _linear(200, 768, 96)]
+    for (rc, made), tiled in zip(launches(calls), [True] * 4 + [False] * 4):
+        assert rc == 0 and len(made) == 1 and ("fdb_gemm_kernel" in made[0][0]) == tiled, made
