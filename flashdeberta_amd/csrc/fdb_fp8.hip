@@ -631,26 +631,83 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
     if constexpr (!ALL) near_begins();
   }
 
-  auto read_v = [&](vfrag (&vfr)[2][DBLKS], uint32_t buf) __attribute__((always_inline)) {
+  // A far step (ALL) has the number far_step_at(k), k = -n_far .. -1, and goes without rings and scratch.
+  auto step = [&](auto far_tag, auto mask_tag, auto par_tag, int k) __attribute__((always_inline)) {
+    constexpr bool FAR = decltype(far_tag)::value, MASK = decltype(mask_tag)::value;
+    constexpr int PAR = decltype(par_tag)::value;
+    const int s = FAR ? far_step_at(k) : s0 + k, next = FAR ? far_step_at(k + 1) : s + 1;
+    const int j0 = s * kStep;
+    wait_vmcnt<0>();
+    if constexpr (!FAR) asm volatile("" : "+v"(dnext));
+    __syncthreads();
+    k_dma(next, PAR ^ 1);
+    v_dma(next, PAR ^ 1);
+    if constexpr (!FAR) batch_dma(dnext, slot_dma);  // batch k + 5 in place of batch k (E_K) or k - 1 (E_Q)
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!FAR) dnext = batch_delta();
+    const i32x8 kf = lds_frag8(kx0 + PAR * N8::K_BYTES, kx1 + PAR * N8::K_BYTES);
+    f32x16 sacc, cnew, pacc[2];
+    if constexpr (C2P && !FAR) cnew = mma8_sa<127 - kCShift>(ring_frag(ek0, slot_k), qf, zero);
+    if constexpr (P2C && !FAR) pacc[1] = mma8(kf, ring_frag(eq0, slot_q == 0 ? kRingBatchesQ - 1 : slot_q - 1), zero);
+    if constexpr (P2C && !FAR) pacc[0] = mma8(kf, ring_frag(eq0, slot_q), zero);
+    if constexpr (P2C && FAR) pacc[0] = mma8(kf, eq, zero);
+    sacc = mma8(kf, qf, zero);
+    uint32_t craw[16];
+    if constexpr (C2P && !FAR) {
+      c_store(cnew, PAR);
+      wave_lds_fence();
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        craw[4 * q + 0] = lds_u16_asm<0>(c_rd[PAR][q]);
+        craw[4 * q + 1] = lds_u16_asm<2>(c_rd[PAR][q]);
+        craw[4 * q + 2] = lds_u16_asm<4>(c_rd[PAR][q]);
+        craw[4 * q + 3] = lds_u16_asm<6>(c_rd[PAR][q]);
+      }
+      wave_lds_fence();
+    }
+    float px[16];
+    if constexpr (P2C && !FAR) {
+      float xs[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int c = 8 * (v >> 2) + 3 - (v & 3);  // jj - 4g
+        xs[v] = (xl < 32 - c) ? pacc[1][v] : pacc[0][v];
+      }
+      if (g == 0)
+        rotate16<32>(xs, px, std::make_integer_sequence<int, 16>{});
+      else
+        rotate16<28>(xs, px, std::make_integer_sequence<int, 16>{});
+    }
+    vfrag vfr[2][DBLKS];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int d = 0; d < DBLKS; ++d) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + buf + 2048 * c));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + buf + 2048 * c + 1024));
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + PAR * N8::V_BYTES + 2048 * c));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + PAR * N8::V_BYTES + 2048 * c + 1024));
         vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
-  };
-  auto mask_keys = [&](f32x16& sacc, int j0) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr ((C2P || P2C) && !FAR) {
+      lds_wait_all8();
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        if constexpr (C2P) asm volatile("" : "+v"(craw[v]));
+        if constexpr (P2C) asm volatile("" : "+v"(px[v]));
+      }
+    }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
-      if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+      if constexpr (C2P && !FAR) sacc[v] = __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)craw[v]), rho_c, sacc[v]);
+      if constexpr (P2C) sacc[v] = __builtin_fmaf(FAR ? pacc[0][v] : px[v], rho_p, sacc[v]);
     }
-  };
-  // online soft-max in base 2 over a step's scores sacc * x_scale + add, O^T += V^T P^T
-  auto take = [&](auto mask_tag, const f32x16& sacc, float add, const vfrag (&vfr)[2][DBLKS]) __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
+    if constexpr (MASK) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
+        if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+      }
+    }
     vfrag pf[2];
     float l_blk = 0.f;
     auto probs = [&](float off) __attribute__((always_inline)) {
@@ -666,14 +723,15 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
     };
     bool slow = __any(m_run == -INFINITY);
     if (!slow) {
-      probs(add - m_run);
+      probs(FAR ? row_add - m_run : -m_run);
       slow = __any(!(l_blk <= 256.f));
     }
     if (slow) {
       float mx = sacc[0];
 #pragma unroll
       for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
-      mx = __builtin_fmaf(wave_half_max(mx), x_scale, add);
+      mx = wave_half_max(mx) * x_scale;
+      if constexpr (FAR) mx += row_add;
       if (__any(mx > m_run + kLazyTau)) {
         const float m_new = (mx > m_run + kLazyTau) ? mx : m_run;
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -684,135 +742,59 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
 #pragma unroll
           for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
       }
-      probs((MASK && m_run == -INFINITY) ? 0.f : add - m_run);
+      probs((MASK && m_run == -INFINITY) ? 0.f : FAR ? row_add - m_run : -m_run);
     }
     l_run += l_blk;
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
-  };
-
-  auto step = [&](auto mask_tag, auto par_tag, int k) __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
-    constexpr int PAR = decltype(par_tag)::value;
-    const int s = s0 + k;
-    const int j0 = s * kStep;
-    wait_vmcnt<0>();
-    asm volatile("" : "+v"(dnext));
-    __syncthreads();
-    k_dma(s + 1, PAR ^ 1);
-    v_dma(s + 1, PAR ^ 1);
-    batch_dma(dnext, slot_dma);  // batch k + 5 in place of batch k (E_K) or k - 1 (E_Q)
-    __builtin_amdgcn_sched_barrier(0);
-    dnext = batch_delta();
-    const i32x8 kf = lds_frag8(kx0 + PAR * N8::K_BYTES, kx1 + PAR * N8::K_BYTES);
-    f32x16 sacc, cnew, pacc[2];
-    if constexpr (C2P) cnew = mma8_sa<127 - kCShift>(ring_frag(ek0, slot_k), qf, zero);
-    if constexpr (P2C) pacc[1] = mma8(kf, ring_frag(eq0, slot_q == 0 ? kRingBatchesQ - 1 : slot_q - 1), zero);
-    if constexpr (P2C) pacc[0] = mma8(kf, ring_frag(eq0, slot_q), zero);
-    sacc = mma8(kf, qf, zero);
-    uint32_t craw[16];
-    if constexpr (C2P) {
-      c_store(cnew, PAR);
-      wave_lds_fence();
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        craw[4 * q + 0] = lds_u16_asm<0>(c_rd[PAR][q]);
-        craw[4 * q + 1] = lds_u16_asm<2>(c_rd[PAR][q]);
-        craw[4 * q + 2] = lds_u16_asm<4>(c_rd[PAR][q]);
-        craw[4 * q + 3] = lds_u16_asm<6>(c_rd[PAR][q]);
-      }
-      wave_lds_fence();
-    }
-    float px[16];
-    if constexpr (P2C) {
-      float xs[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int c = 8 * (v >> 2) + 3 - (v & 3);  // jj - 4g
-        xs[v] = (xl < 32 - c) ? pacc[1][v] : pacc[0][v];
-      }
-      if (g == 0)
-        rotate16<32>(xs, px, std::make_integer_sequence<int, 16>{});
-      else
-        rotate16<28>(xs, px, std::make_integer_sequence<int, 16>{});
-    }
-    vfrag vfr[2][DBLKS];
-    read_v(vfr, PAR * N8::V_BYTES);
-    __builtin_amdgcn_sched_barrier(0);
-    if constexpr (C2P || P2C) {
-      lds_wait_all8();
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        if constexpr (C2P) asm volatile("" : "+v"(craw[v]));
-        if constexpr (P2C) asm volatile("" : "+v"(px[v]));
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      if constexpr (C2P) sacc[v] = __builtin_fmaf((float)__builtin_bit_cast(_Float16, (uint16_t)craw[v]), rho_c, sacc[v]);
-      if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], rho_p, sacc[v]);
-    }
-    if constexpr (MASK) mask_keys(sacc, j0);
-    take(mask_tag, sacc, 0.f, vfr);
+    if constexpr (FAR) return;
     slot_k = slot_k == kRingBatchesK - 1 ? 0 : slot_k + 1;
     slot_q = slot_q == kRingBatchesQ - 1 ? 0 : slot_q + 1;
     slot_dma = slot_dma == ring_n - 1 ? 0 : slot_dma + 1;
   };
-  // ---- far steps (ALL): their K and V go through the two buffers so that the first near step finds its own in buffer 0
-  auto far_steps = [&](auto mask_tag, int t, int end) __attribute__((always_inline)) {
-#pragma unroll 1
-    for (; t < end; ++t) {
-      const int s = far_step_at(t), next = far_step_at(t + 1), par = t & 1;
-      wait_vmcnt<0>();
-      __syncthreads();
-      k_dma(next, par ^ 1);
-      v_dma(next, par ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-      const i32x8 kf = lds_frag8(kx0 + par * N8::K_BYTES, kx1 + par * N8::K_BYTES);
-      vfrag vfr[2][DBLKS];
-      read_v(vfr, par * N8::V_BYTES);
-      f32x16 sacc = mma8(kf, qf, zero);
-      if constexpr (P2C) {
-        const f32x16 pacc = mma8(kf, eq, zero);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sacc[v] = __builtin_fmaf(pacc[v], rho_p, sacc[v]);
-      }
-      if constexpr (decltype(mask_tag)::value)
-        if ((s + 1) * kStep > Lb) mask_keys(sacc, s * kStep);
-      take(mask_tag, sacc, row_add, vfr);
-    }
-  };
-  if constexpr (ALL) {
-    far_steps(std::false_type{}, -n_far, -n_right);
-    if (n_left > 0 && n_right > 0) side_begins(1);
-    far_steps(std::true_type{}, -n_right, 0);
-    if (n_steps > 0) near_begins();  // the rings' rows have been waited for, here or in the first far step
-  }
   {
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
+    if constexpr (ALL) {
+      // K and V go through the two buffers so that the first near step finds its own in buffer 0
+      auto far_steps = [&](int t, int end) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (; t < end; ++t) {
+          if (t & 1) step(std::true_type{}, std::false_type{}, T1{}, t);
+          else step(std::true_type{}, std::false_type{}, T0{}, t);
+        }
+      };
+      if (n_far > 0) {
+        const bool ragged = n_right > 0 && all1 * kStep > Lb;   // the last far step reaches past the end
+        far_steps(-n_far, -n_right);
+        if (n_left > 0 && n_right > 0) side_begins(1);
+        far_steps(-n_right, ragged ? -1 : 0);
+        if (ragged) step(std::true_type{}, std::true_type{}, T1{}, -1);
+      }
+      if (n_steps > 0) near_begins();  // the rings' rows have been waited for, above or in the first far step
+    }
     int k = 0;
 #pragma unroll 1
     for (; k + 1 < n_full; k += 2) {
-      step(std::false_type{}, T0{}, k);
-      step(std::false_type{}, T1{}, k + 1);
+      step(std::false_type{}, std::false_type{}, T0{}, k);
+      step(std::false_type{}, std::false_type{}, T1{}, k + 1);
     }
     if (k < n_full) {
-      step(std::false_type{}, T0{}, k);
+      step(std::false_type{}, std::false_type{}, T0{}, k);
       ++k;
     }
     if ((k & 1) && k < n_steps) {
-      step(std::true_type{}, T1{}, k);
+      step(std::false_type{}, std::true_type{}, T1{}, k);
       ++k;
     }
 #pragma unroll 1
     for (; k + 1 < n_steps; k += 2) {
-      step(std::true_type{}, T0{}, k);
-      step(std::true_type{}, T1{}, k + 1);
+      step(std::false_type{}, std::true_type{}, T0{}, k);
+      step(std::false_type{}, std::true_type{}, T1{}, k + 1);
     }
-    if (k < n_steps) step(std::true_type{}, T0{}, k);
+    if (k < n_steps) step(std::false_type{}, std::true_type{}, T0{}, k);
   }
   wait_vmcnt<0>();  // none of the last step's direct loads may still be writing LDS when the workgroup ends
 

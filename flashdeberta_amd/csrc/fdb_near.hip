@@ -381,30 +381,123 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     if constexpr (!ALL) near_begins();
   }
 
-  // V^T operands of the step in the buffer at byte `buf` of V's two
-  auto read_v = [&](vfrag (&vfr)[2][DBLKS], uint32_t buf) __attribute__((always_inline)) {
+  // A far step (ALL) has the number far_step_at(k), k = -n_far .. -1, and goes without rings, C and P.
+  auto step = [&](auto far_tag, auto mask_tag, auto par_tag, auto next_tag, int k) __attribute__((always_inline)) {
+    constexpr bool FAR = decltype(far_tag)::value, MASK = decltype(mask_tag)::value;
+    constexpr int PAR = decltype(par_tag)::value;  // parity of the step: its K / V buffers, its half of the scratch
+    constexpr bool NEXT_INSIDE = decltype(next_tag)::value;  // the next step's keys all lie inside the sequence
+    const int s = FAR ? far_step_at(k) : s0 + k, next = FAR ? far_step_at(k + 1) : s + 1;
+    const int j0 = s * kStep;
+    // This wave's direct loads of the step before -- K, V and the new ring batch of this step -- have landed;
+    // behind the barrier everyone's have, and every wave is done with the buffers the loads below overwrite.
+    wait_vmcnt<0>();
+    // The table value fetched a step ago is among the loads just waited for; taking it here keeps the compiler,
+    // which does not count the direct loads, from waiting for it further down, behind this step's direct loads.
+    if constexpr (!FAR) asm volatile("" : "+v"(dnext));
+    __syncthreads();
+    // ---- staging for the next step, straight into LDS ----------------------------------------------------------
+    // It runs unconditionally, past the last step too (row and table indices are clamped, and nobody reads
+    // what the last steps fetch), so every step issues the same loads and the one wait above covers them.
+    k_dma(next, PAR ^ 1, NEXT_INSIDE);
+    v_dma(next, PAR ^ 1, NEXT_INSIDE);
+    if constexpr (!FAR) batch_dma(dnext, slot_dma);          // batch k + 5 in place of batch k
+    __builtin_amdgcn_sched_barrier(0);   // the table load stays behind the direct loads
+    if constexpr (!FAR) dnext = batch_delta();               // of batch k + 6, used a step from now
+    // ---- operands of the step out of LDS ------------------------------------------------------------------
+    qfrag kf[KS];
+#pragma unroll
+    for (int x = 0; x < KS; ++x) kf[x] = *(LDS_AS const qfrag*)(uintptr_t)(klx[x] + PAR * NCfg::K_BYTES);
+    if constexpr (!FAR) ring_read(PAR, slot_rd);
+    // ---- the sixteen MFMAs of the four score products, in two pairs of chains that alternate (no MFMA waits for
+    // its own previous link): C's new block with P's block 1 (whose operands are this step's keys and the rows
+    // kept from the step before), then P's block 0 with the content product.  What follows C -- the write to the
+    // scratch and the reads of the skewed band -- runs under the second pair.
+    f32x16 sacc, cnew, pacc[2];
+    if constexpr (!FAR) {
+#pragma unroll
+      for (int x = 0; x < KS; ++x) {
+        if constexpr (C2P) cnew = QT::mma(ac[x], qf[x], x == 0 ? zero : cnew);
+        if constexpr (P2C) pacc[1] = QT::mma(kf[x], aq[PAR ^ 1][x], x == 0 ? zero : pacc[1]);
+      }
+#pragma unroll
+      for (int x = 0; x < KS; ++x) {
+        if constexpr (P2C) pacc[0] = QT::mma(kf[x], aq[PAR][x], x == 0 ? zero : pacc[0]);
+        sacc = QT::mma(kf[x], qf[x], x == 0 ? negm : sacc);
+      }
+    } else {
+#pragma unroll
+      for (int x = 0; x < KS; ++x) sacc = QT::mma(kf[x], qx[x], x == 0 ? negm : sacc);
+    }
+    float cband[16];
+    if constexpr (C2P && !FAR) {
+      c_store(cnew, PAR);
+      wave_lds_fence();  // the LDS unit runs one wave's operations in order; this keeps the compiler from moving them
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        cband[4 * q + 0] = lds_elem_f32<QT, 0>(c_rd[PAR][q]);
+        cband[4 * q + 1] = lds_elem_f32<QT, 2>(c_rd[PAR][q]);
+        cband[4 * q + 2] = lds_elem_f32<QT, 4>(c_rd[PAR][q]);
+        cband[4 * q + 3] = lds_elem_f32<QT, 6>(c_rd[PAR][q]);
+      }
+      wave_lds_fence();
+    }
+    // P with the keys as MFMA rows, like the content product: register v of lane (g, n) holds
+    // P[jj(v, g)][32 bk + n], and element (jj, i = li) wants column li + 32 - jj of that row, i.e. the same
+    // register of another lane of its own half: lane (li - jj) mod 32, block 1 if li >= jj.  Each source lane is
+    // read by exactly one lane, which wants block 1 from it if n + jj < 32 and block 0 otherwise: the source
+    // picks (a compare of its lane constant with a constant of the register), and a rotation of each half-wave
+    // by 32 - jj moves it: ds_swizzle in rotate mode, no address registers; the halves differ by 4 in jj, so each
+    // half runs its own sixteen under its half of the execution mask.
+    float px[16];
+    if constexpr (P2C && !FAR) {
+      float xs[16];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int c = 8 * (v >> 2) + 3 - (v & 3);  // jj - 4g
+        xs[v] = (xl < 32 - c) ? pacc[1][v] : pacc[0][v];
+      }
+      if (g == 0)
+        rotate16<32>(xs, px, std::make_integer_sequence<int, 16>{});
+      else
+        rotate16<28>(xs, px, std::make_integer_sequence<int, 16>{});
+    }
+    // V^T operands requested here, ahead of the soft-max, so that the four MFMAs at the end of the step find them
+    vfrag vfr[2][DBLKS];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int d = 0; d < DBLKS; ++d) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + buf + 2048 * c));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + buf + 2048 * c + 1024));
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d] + PAR * NCfg::V_BYTES + 2048 * c));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(vlx[2 * d + 1] + PAR * NCfg::V_BYTES + 2048 * c + 1024));
         vfr[c][d] = __builtin_bit_cast(vfrag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       }
-  };
-  auto mask_keys = [&](f32x16& sacc, int j0) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    // one wait for the band of C and the rotated P (issued as asm: the compiler keeps no count of them)
+    if constexpr ((C2P || P2C) && !FAR) {
+      lds_wait_all();
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        if constexpr (C2P && std::is_same<QT, Bf16Tr>::value) asm volatile("" : "+v"(cband[v]));
+        if constexpr (P2C) asm volatile("" : "+v"(px[v]));
+      }
+    }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
-      if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+      if constexpr (C2P && !FAR) sacc[v] += cband[v];
+      if constexpr (P2C && !FAR) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v]);
     }
-  };
-  // Online soft-max in base 2 over a step's scores, O^T += V^T P^T.
-  // sacc = score - reference point.  The probabilities are formed first; the half-row sum of a step bounds its
-  // largest one, so while it stays under 2^kLazyTau nothing has to move and no maximum is taken.  Otherwise (or
-  // before a row has a reference point) the wave takes the maximum, moves the reference points of the rows that
-  // need it, shifts the step's scores and forms the probabilities again.
-  auto take = [&](f32x16& sacc, const vfrag (&vfr)[2][DBLKS]) __attribute__((always_inline)) {
+    // ---- mask, online soft-max in base 2, O^T += V^T P^T ---------------------------------------------------
+    if constexpr (MASK) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int j = j0 + 8 * (v >> 2) + 4 * g + 3 - (v & 3);
+        if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
+      }
+    }
+    // sacc = score - reference point.  The probabilities are formed first; the half-row sum of a step bounds its
+    // largest one, so while it stays under 2^kLazyTau nothing has to move and no maximum is taken.  Otherwise (or
+    // before a row has a reference point) the wave takes the maximum, moves the reference points of the rows that
+    // need it, shifts the step's scores and forms the probabilities again.
     vfrag pf[2];
     float l_blk = 0.f;
     auto probs = [&]() __attribute__((always_inline)) {
@@ -453,168 +546,60 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int d = 0; d < DBLKS; ++d) o_acc[d] = VT::mma(vfr[c][d], pf[c], o_acc[d]);
-  };
-
-  auto step = [&](auto mask_tag, auto par_tag, auto next_tag, int k) __attribute__((always_inline)) {
-    constexpr bool MASK = decltype(mask_tag)::value;
-    constexpr int PAR = decltype(par_tag)::value;  // parity of the step: its K / V buffers, its half of the scratch
-    constexpr bool NEXT_INSIDE = decltype(next_tag)::value;  // the next step's keys all lie inside the sequence
-    const int s = s0 + k;
-    const int j0 = s * kStep;
-    // This wave's direct loads of the step before -- K, V and the new ring batch of this step -- have landed;
-    // behind the barrier everyone's have, and every wave is done with the buffers the loads below overwrite.
-    wait_vmcnt<0>();
-    // The table value fetched a step ago is among the loads just waited for; taking it here keeps the compiler,
-    // which does not count the direct loads, from waiting for it further down, behind this step's direct loads.
-    asm volatile("" : "+v"(dnext));
-    __syncthreads();
-    // ---- staging for the next step, straight into LDS ----------------------------------------------------------
-    // It runs unconditionally, past the last step too (row and table indices are clamped, and nobody reads
-    // what the last steps fetch), so every step issues the same loads and the one wait above covers them.
-    k_dma(s + 1, PAR ^ 1, NEXT_INSIDE);
-    v_dma(s + 1, PAR ^ 1, NEXT_INSIDE);
-    batch_dma(dnext, slot_dma);          // batch k + 5 in place of batch k
-    __builtin_amdgcn_sched_barrier(0);   // the table load stays behind the direct loads
-    dnext = batch_delta();               // of batch k + 6, used a step from now
-    // ---- operands of the step out of LDS ------------------------------------------------------------------
-    qfrag kf[KS];
-#pragma unroll
-    for (int x = 0; x < KS; ++x) kf[x] = *(LDS_AS const qfrag*)(uintptr_t)(klx[x] + PAR * NCfg::K_BYTES);
-    ring_read(PAR, slot_rd);
-    // ---- the sixteen MFMAs of the four score products, in two pairs of chains that alternate (no MFMA waits for
-    // its own previous link): C's new block with P's block 1 (whose operands are this step's keys and the rows
-    // kept from the step before), then P's block 0 with the content product.  What follows C -- the write to the
-    // scratch and the reads of the skewed band -- runs under the second pair.
-    f32x16 sacc, cnew, pacc[2];
-#pragma unroll
-    for (int x = 0; x < KS; ++x) {
-      if constexpr (C2P) cnew = QT::mma(ac[x], qf[x], x == 0 ? zero : cnew);
-      if constexpr (P2C) pacc[1] = QT::mma(kf[x], aq[PAR ^ 1][x], x == 0 ? zero : pacc[1]);
-    }
-#pragma unroll
-    for (int x = 0; x < KS; ++x) {
-      if constexpr (P2C) pacc[0] = QT::mma(kf[x], aq[PAR][x], x == 0 ? zero : pacc[0]);
-      sacc = QT::mma(kf[x], qf[x], x == 0 ? negm : sacc);
-    }
-    float cband[16];
-    if constexpr (C2P) {
-      c_store(cnew, PAR);
-      wave_lds_fence();  // the LDS unit runs one wave's operations in order; this keeps the compiler from moving them
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        cband[4 * q + 0] = lds_elem_f32<QT, 0>(c_rd[PAR][q]);
-        cband[4 * q + 1] = lds_elem_f32<QT, 2>(c_rd[PAR][q]);
-        cband[4 * q + 2] = lds_elem_f32<QT, 4>(c_rd[PAR][q]);
-        cband[4 * q + 3] = lds_elem_f32<QT, 6>(c_rd[PAR][q]);
-      }
-      wave_lds_fence();
-    }
-    // P with the keys as MFMA rows, like the content product: register v of lane (g, n) holds
-    // P[jj(v, g)][32 bk + n], and element (jj, i = li) wants column li + 32 - jj of that row, i.e. the same
-    // register of another lane of its own half: lane (li - jj) mod 32, block 1 if li >= jj.  Each source lane is
-    // read by exactly one lane, which wants block 1 from it if n + jj < 32 and block 0 otherwise: the source
-    // picks (a compare of its lane constant with a constant of the register), and a rotation of each half-wave
-    // by 32 - jj moves it: ds_swizzle in rotate mode, no address registers; the halves differ by 4 in jj, so each
-    // half runs its own sixteen under its half of the execution mask.
-    float px[16];
-    if constexpr (P2C) {
-      float xs[16];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int c = 8 * (v >> 2) + 3 - (v & 3);  // jj - 4g
-        xs[v] = (xl < 32 - c) ? pacc[1][v] : pacc[0][v];
-      }
-      if (g == 0)
-        rotate16<32>(xs, px, std::make_integer_sequence<int, 16>{});
-      else
-        rotate16<28>(xs, px, std::make_integer_sequence<int, 16>{});
-    }
-    // V^T operands requested here, ahead of the soft-max, so that the four MFMAs at the end of the step find them
-    vfrag vfr[2][DBLKS];
-    read_v(vfr, PAR * NCfg::V_BYTES);
-    __builtin_amdgcn_sched_barrier(0);
-    // one wait for the band of C and the rotated P (issued as asm: the compiler keeps no count of them)
-    if constexpr (C2P || P2C) {
-      lds_wait_all();
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        if constexpr (C2P && std::is_same<QT, Bf16Tr>::value) asm volatile("" : "+v"(cband[v]));
-        if constexpr (P2C) asm volatile("" : "+v"(px[v]));
-      }
-    }
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      if constexpr (C2P) sacc[v] += cband[v];
-      if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v]);
-    }
-    if constexpr (MASK) mask_keys(sacc, j0);
-    take(sacc, vfr);
+    if constexpr (FAR) return;
     slot_rd = slot_rd == kRingBatches - 1 ? 0 : slot_rd + 1;
     slot_dma = slot_dma == kRingBatches - 1 ? 0 : slot_dma + 1;
   };
-  // ---- far steps (ALL): their K and V go through the two buffers so that the first near step finds its own in buffer 0
-  auto far_steps = [&](auto mask_tag, int t, int end) __attribute__((always_inline)) {
-#pragma unroll 1
-    for (; t < end; ++t) {
-      const int s = far_step_at(t), next = far_step_at(t + 1), par = t & 1;
-      wait_vmcnt<0>();
-      __syncthreads();
-      k_dma(next, par ^ 1, false);
-      v_dma(next, par ^ 1, false);
-      __builtin_amdgcn_sched_barrier(0);
-      qfrag kf[KS];
-#pragma unroll
-      for (int x = 0; x < KS; ++x) kf[x] = *(LDS_AS const qfrag*)(uintptr_t)(klx[x] + par * NCfg::K_BYTES);
-      vfrag vfr[2][DBLKS];
-      read_v(vfr, par * NCfg::V_BYTES);
-      f32x16 sacc;
-#pragma unroll
-      for (int x = 0; x < KS; ++x) sacc = QT::mma(kf[x], qx[x], x == 0 ? negm : sacc);
-      if constexpr (decltype(mask_tag)::value)
-        if ((s + 1) * kStep > Lb) mask_keys(sacc, s * kStep);
-      take(sacc, vfr);
-    }
-  };
-  if constexpr (ALL) {
-    if (__builtin_expect(n_far > 0, 0)) {
-      far_steps(std::false_type{}, -n_far, -n_right);
-      if (n_left > 0 && n_right > 0) side_begins(1);
-      far_steps(std::true_type{}, -n_right, 0);
-      range_begins(0.f);
-    }
-    if (n_steps > 0) near_begins();  // the rings' rows have been waited for, above or in the first far step
-  }
   {
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
     using Y = std::true_type;
     using N = std::false_type;
+    if constexpr (ALL) {
+      // K and V go through the two buffers so that the first near step finds its own in buffer 0
+      auto far_steps = [&](int t, int end) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (; t < end; ++t) {
+          if (t & 1) step(Y{}, N{}, T1{}, N{}, t);
+          else step(Y{}, N{}, T0{}, N{}, t);
+        }
+      };
+      if (__builtin_expect(n_far > 0, 0)) {
+        const bool ragged = n_right > 0 && all1 * kStep > Lb;   // the last far step reaches past the end
+        far_steps(-n_far, -n_right);
+        if (n_left > 0 && n_right > 0) side_begins(1);
+        far_steps(-n_right, ragged ? -1 : 0);
+        if (ragged) step(Y{}, Y{}, T1{}, N{}, -1);
+        range_begins(0.f);
+      }
+      if (n_steps > 0) near_begins();  // the rings' rows have been waited for, above or in the first far step
+    }
     int k = 0;
     // the bulk: unmasked steps whose successor is unmasked too (its rows need no clamping)
 #pragma unroll 1
     for (; k + 2 < n_full; k += 2) {
-      step(N{}, T0{}, Y{}, k);
-      step(N{}, T1{}, Y{}, k + 1);
+      step(N{}, N{}, T0{}, Y{}, k);
+      step(N{}, N{}, T1{}, Y{}, k + 1);
     }
 #pragma unroll 1
     for (; k + 1 < n_full; k += 2) {
-      step(N{}, T0{}, N{}, k);
-      step(N{}, T1{}, N{}, k + 1);
+      step(N{}, N{}, T0{}, N{}, k);
+      step(N{}, N{}, T1{}, N{}, k + 1);
     }
     if (k < n_full) {
-      step(N{}, T0{}, N{}, k);
+      step(N{}, N{}, T0{}, N{}, k);
       ++k;
     }
     if ((k & 1) && k < n_steps) {
-      step(Y{}, T1{}, N{}, k);
+      step(N{}, Y{}, T1{}, N{}, k);
       ++k;
     }
 #pragma unroll 1
     for (; k + 1 < n_steps; k += 2) {
-      step(Y{}, T0{}, N{}, k);
-      step(Y{}, T1{}, N{}, k + 1);
+      step(N{}, Y{}, T0{}, N{}, k);
+      step(N{}, Y{}, T1{}, N{}, k + 1);
     }
-    if (k < n_steps) step(Y{}, T0{}, N{}, k);
+    if (k < n_steps) step(N{}, Y{}, T0{}, N{}, k);
   }
   wait_vmcnt<0>();  // the last step's direct loads: none may still be writing LDS when the workgroup ends
 
