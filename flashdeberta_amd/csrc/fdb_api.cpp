@@ -766,8 +766,8 @@ int fdb_gemm(const void* x, const void* w, const void* bias, const void* residua
   return fdb_launch_gemm(x, w, bias, residual, out, rows, cols, depth, ldx, ldw, ldo, ldr, epilogue, dtype, stream);
 }
 
-int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
-                  int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream) {
+static int gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
+                     int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t dtype, void* stream) {
   if (!x || !w || !out || !seq_len) return FDB_ERR_NULL;
   if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
   const int64_t rows = (int64_t)batch * seqlen;
@@ -775,7 +775,17 @@ int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, con
       cols > (1 << 24) || ldx > (1 << 22) || ldw > (1 << 22) || rows * ldx * 2 > INT32_MAX)  // all rows of x and 192 of w within a lane's 32-bit offset
     return FDB_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || ldo % 8 || (reinterpret_cast<uintptr_t>(bias) & 7u)) return FDB_ERR_ALIGN;
-  return fdb_launch_gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, cu_count(), dtype, stream);
+  return fdb_launch_gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, clear, cu_count(), dtype, stream);
+}
+
+int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
+                  int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream) {
+  return gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, false, dtype, stream);
+}
+
+int fdb_gemm_real_cleared(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch,
+                          int32_t seqlen, int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream) {
+  return gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, true, dtype, stream);
 }
 
 int fdb_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0, void* out1,

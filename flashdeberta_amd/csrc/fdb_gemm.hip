@@ -231,6 +231,7 @@ struct RealParams {
   GemmParams g;
   const int32_t *start, *length;   // [batch]: the first real row of a sequence (NULL: 0) and how many (negative: none)
   int32_t batch, seqlen, cus, narrow, span;   // narrow: tiles of 160 columns across; span: half of the power of two from batch up
+  int32_t clear;   // the rows of padding become zeros
 };
 using R64 = GemmShape<64, 192, 2, 4, 4, 1>;
 using R128 = GemmShape<128, 192, 2, 4, 3, 1>;
@@ -296,6 +297,13 @@ __global__ __launch_bounds__(512, 2) void fdb_gemm_real_kernel(const RealParams 
     else if (height == 192) make_tile<QT, kPlain, R192>(p.g, rows, tm, tn, smem);
     else if (wide == p.g.tiles_n) make_tile<QT, kPlain, R256>(p.g, rows, tm, tn, smem);
     else make_tile<QT, kPlain, R256x160>(p.g, rows, tm, tn, smem);
+  }
+  if (!p.clear) return;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int i = blockIdx.x * 8 + wave; i < p.batch * p.seqlen; i += gridDim.x * 8) {   // a row a wave
+    const int b = __builtin_amdgcn_readfirstlane(i / p.seqlen), row = i - b * p.seqlen, b_first = __builtin_amdgcn_readlane(first, b);
+    if (row >= b_first && row < b_first + __builtin_amdgcn_readlane(len, b)) continue;
+    for (int col = 8 * lane; col < p.g.N; col += 8 * 64) *(u32x4*)(p.g.out + ((int64_t)i * p.g.ldo + col) * 2) = u32x4{0, 0, 0, 0};
   }
 }
 
@@ -382,9 +390,9 @@ extern "C" int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t N
 }
 
 int fdb_launch_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* start, const int32_t* length, int32_t batch, int32_t seqlen,
-                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, int32_t cus, int dtype, void* stream) {
+                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t cus, int dtype, void* stream) {
   RealParams p{};
   p.g = GemmParams{(const char*)x, (const char*)w, (const char*)bias, nullptr, (char*)out, ldx, ldw, ldo, 0, batch * seqlen, N, K, 0, 0};
-  p.start = start, p.length = length, p.batch = batch, p.seqlen = seqlen, p.cus = cus;
+  p.start = start, p.length = length, p.batch = batch, p.seqlen = seqlen, p.cus = cus, p.clear = clear;
   return dtype == FDB_BF16 ? launch_real<Bf16Tr>(p, (hipStream_t)stream) : launch_real<F16Tr>(p, (hipStream_t)stream);
 }

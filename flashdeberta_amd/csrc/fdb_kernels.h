@@ -225,7 +225,7 @@ int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* 
 // The plain product where columns and output rows come by fours only, or the bias lies on any element: for fdb_linear, not an epilogue of fdb_gemm's.
 enum { FDB_GEMM_NARROW = 3 };
 int fdb_launch_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* start, const int32_t* length, int32_t batch, int32_t seqlen,
-                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, int32_t cus, int dtype, void* stream);
+                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t cus, int dtype, void* stream);
 int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0,
                      void* out1, int dtype, void* stream);  // fdb_grad.hip
 int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols, int cus);

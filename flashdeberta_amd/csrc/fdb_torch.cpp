@@ -226,14 +226,16 @@ void product(Mat a, bool trans_a, Mat b, bool trans_b, Mat d, const Tensor* bias
 struct Lengths {
   const OptTensor &start, &len;
 };
-bool project_real(const Tensor& x, const Tensor& w, const Tensor& b, int64_t cols, const Tensor& out, int64_t batch, int64_t length, const Lengths& real) {
+// `cleared`: with zeros in the rows of padding, which are not written otherwise.
+bool project_real(const Tensor& x, const Tensor& w, const Tensor& b, int64_t cols, const Tensor& out, int64_t batch, int64_t length, const Lengths& real, bool cleared) {
   const OptTensor &start = real.start, &len = real.len;
   const int64_t k = x.size(-1);
   if (!len || !fdb_gemm_real_serves(batch, length, cols, k, k)) return false;
   for (const OptTensor* t : {&start, &len})
     if (*t && ((*t)->scalar_type() != at::kInt || !(*t)->is_contiguous() || (*t)->numel() != batch || (*t)->device() != x.device() || !plain_memory(**t))) return false;
-  const int rc = fdb_gemm_real(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), start ? (const int32_t*)start->data_ptr() : nullptr, (const int32_t*)len->data_ptr(),
-                               (int32_t)batch, (int32_t)length, (int32_t)cols, (int32_t)k, k, w.stride(0), cols, fdb_dtype_of(x.scalar_type()), stream_of(x));
+  const auto entry = cleared ? fdb_gemm_real_cleared : fdb_gemm_real;
+  const int rc = entry(x.data_ptr(), w.data_ptr(), b.data_ptr(), out.data_ptr(), start ? (const int32_t*)start->data_ptr() : nullptr, (const int32_t*)len->data_ptr(),
+                       (int32_t)batch, (int32_t)length, (int32_t)cols, (int32_t)k, k, w.stride(0), cols, fdb_dtype_of(x.scalar_type()), stream_of(x));
   if (rc > 0) check(rc, "fdb_gemm_real");
   return rc == 0;   // a negative code: a size or an alignment it is not built for
 }
@@ -267,7 +269,7 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
     if (rc == 0) return rest(out);
     if (rc > 0) check(rc, "fdb_linear");  // a negative code: a size or alignment it is not built for
   }
-  if (real && then == Then::nothing && x.dim() == 3 && project_real(x, w, *bias, n, out, x.size(0), x.size(1), *real)) return out;
+  if (real && then == Then::nothing && x.dim() == 3 && project_real(x, w, *bias, n, out, x.size(0), x.size(1), *real, false)) return out;
   const int epilogue = then == Then::gelu ? FDB_GEMM_GELU : then == Then::add ? FDB_GEMM_RESIDUAL : FDB_GEMM_PLAIN;
   if (fdb_gemm_serves(m, n, k, epilogue)) {
     Tensor r;
@@ -836,7 +838,8 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     Tensor w, b;
     std::tie(w, b) = joined(qw, qb, kw, kb, vw, vb, type, stream_of(hidden));
     const Tensor qkv = at::empty({B * L, 3 * W}, hidden.options()), pos = at::empty({rows, 2 * W}, hidden.options());
-    if (!project_real(hidden, w, b, 3 * W, qkv, B, L, {args->o.seq_start, args->o.seq_len})) projected(hidden, B * L, w, b, 3 * W, qkv);
+    // rows of padding: nothing of the node reads them, but hooks on its saved tensors do
+    if (!project_real(hidden, w, b, 3 * W, qkv, B, L, {args->o.seq_start, args->o.seq_len}, true)) projected(hidden, B * L, w, b, 3 * W, qkv);
     projected(rel, rows, w, b, 2 * W, pos);
     const Tensor out = at::empty({B, L, W}, hidden.options());
     fdb_attn_args a = {};

@@ -393,6 +393,9 @@ int32_t fdb_gemm_serves(int64_t rows, int64_t cols, int64_t depth, int32_t epilo
  */
 int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
                   int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream);
+/* ... with zeros in the other rows: for a result that others look at, too (a training layer saves it for its backward) */
+int fdb_gemm_real_cleared(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch,
+                          int32_t seqlen, int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, int32_t dtype, void* stream);
 int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t cols, int64_t depth, int64_t ldx);
 
 /*

@@ -22,10 +22,11 @@ def _lengths(kind, batch, seqlen):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("cleared", [False, True], ids=["left", "cleared"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("kind", ["full", "none", "one", "clamped", "ragged", "third"])
 @pytest.mark.parametrize("batch,seqlen,N,K", [(1, 1500, 2304, 64), (8, 512, 2304, 128), (64, 33, 1544, 64), (47, 170, 3080, 64), (63, 260, 2304, 64), (5, 2999, 200, 192), (3, 700, 3072, 320)])
-def test_real_rows(batch, seqlen, N, K, kind, dtype):
+def test_real_rows(batch, seqlen, N, K, kind, dtype, cleared):
     g = torch.Generator(device="cuda").manual_seed(batch + N)
     x, w = [(torch.randn(r, K, device="cuda", generator=g) * s).to(dtype) for r, s in ((batch * seqlen, 1.0), (N, K ** -0.5))]
     bias = torch.randn(N, device="cuda", generator=g).to(dtype)
@@ -38,10 +39,11 @@ def test_real_rows(batch, seqlen, N, K, kind, dtype):
     x[~real] = float("nan")   # whatever padding holds
     out = torch.full((batch * seqlen, N), 7.0, device="cuda", dtype=dtype)
     start, length = [torch.tensor(t, dtype=torch.int32, device="cuda") for t in (starts, lens)]
-    assert _lib.lib.fdb_gemm_real(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), None if max(starts) == 0 else start.data_ptr(), length.data_ptr(), batch,
-                                  seqlen, N, K, K, K, N, {torch.bfloat16: _lib.FDB_BF16, torch.float16: _lib.FDB_F16}[dtype],
-                                  torch.cuda.current_stream().cuda_stream) == 0
-    assert (out[~real] == 7.0).all()
+    entry = _lib.lib.fdb_gemm_real_cleared if cleared else _lib.lib.fdb_gemm_real
+    assert entry(x.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), None if max(starts) == 0 else start.data_ptr(), length.data_ptr(), batch,
+                 seqlen, N, K, K, K, N, {torch.bfloat16: _lib.FDB_BF16, torch.float16: _lib.FDB_F16}[dtype],
+                 torch.cuda.current_stream().cuda_stream) == 0
+    assert (out[~real] == (0.0 if cleared else 7.0)).all()
     ref = x[real].double() @ w.double().t() + bias.double()
     bound = torch.finfo(dtype).eps / 2 * ref.abs() * 1.01 + 1e-5   # one rounding of the result; the fp32 sums' own is smaller by 2^-10
     assert ((out[real].double() - ref).abs() <= bound).all()
@@ -70,12 +72,18 @@ def test_nothing_reads_the_rows_left_out(side):
     mask = ((at < lens[:, None]) if side == "right" else (at >= L - lens[:, None])).long()
     grad = torch.randn(B, L, 768, device="cuda").to(torch.bfloat16)
     seen = []
+
+    def pack(t):   # what a hook on the saved tensors meets: no memory that nobody has written
+        assert t.dtype == torch.float32 or not t.is_floating_point() or t.isfinite().all(), t.shape
+        return t
+
     for poison in (0.0, float("nan"), float("nan")):
         hold = [torch.full((n,), poison, device="cuda", dtype=torch.bfloat16) for n in [B * L * 2304] * 4 + [B * L * 768] * 6 + [512 * 1536] * 4]
         del hold   # what the calls below are given
         with torch.no_grad():
             inferred = layer.eval()(x, mask, rel_embeddings=rel)[0]
-        out = layer.train()(x, mask, rel_embeddings=rel)[0]
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+            out = layer.train()(x, mask, rel_embeddings=rel)[0]
         seen.append([inferred, out, *torch.autograd.grad(out, [x, rel, *layer.parameters()], grad)])
     assert all(torch.isfinite(t).all() for t in seen[0])
     for other in seen[1:]:
