@@ -377,10 +377,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // Padded fixed layout: the rows of `out` outside a batch row's real tokens, written by the workgroup whose tile index t
 // covers them in absolute terms (rows [128 t, 128 t + 128), two threads per row of ROW_BYTES): zeros, or `word` = the
-// element type's NaN pattern for a batch row the caller marked with a negative token count.
+// element type's NaN pattern for a batch row the caller marked with a negative token count.  With lse_bh (the head's log-sum-exp of the
+// sequence's first row, `heads` floats from one row to the next or NULL) also those: 0 or NaN.
 template <int ROW_BYTES>
 __device__ __forceinline__ void fill_pad_rows(char* out_bh, int64_t row_stride_bytes, int t, int L, int tok0, int Lb,
-                                              uint32_t word, int tid) {
+                                              uint32_t word, int tid, float* lse_bh = nullptr, int heads = 0) {
   static_assert(ROW_BYTES % 32 == 0, "two threads per row, 16-byte stores");
   const int row = t * 128 + (tid >> 1);
   if (row >= L || (row >= tok0 && row < tok0 + Lb)) return;
@@ -388,6 +389,7 @@ __device__ __forceinline__ void fill_pad_rows(char* out_bh, int64_t row_stride_b
   const u32x4 w = {word, word, word, word};
 #pragma unroll
   for (int c = 0; c < ROW_BYTES / 32; ++c) *(u32x4*)(dst + 16 * c) = w;
+  if (lse_bh && (tid & 1) == 0) lse_bh[(int64_t)row * heads] = word ? __builtin_nanf("") : 0.f;
 }
 
 // Number of direct loads (dma16 / dma16s) a wave issues per K/V tile of the far-only staging: the waits

@@ -98,7 +98,7 @@ typedef struct fdb_attn_args {
   const void* pos_key;     /* K_r or NULL (no content->position term)  */
   const void* pos_query;   /* Q_r or NULL (no position->content term)  */
   void* out;
-  float* lse;              /* [B*max_seqlen*H] (fixed) / [T*H] (varlen), token-major, or NULL */
+  float* lse;              /* [B*max_seqlen*H] (fixed) / [T*H] (varlen), token-major, or NULL; rows of padding like those of out */
   const int32_t* cu_seqlens; /* device int32[batch+1] or NULL                                 */
   int32_t* worklist;       /* device int32[fdb_worklist_ints(...)], filled by fdb_build_worklist */
   const int32_t* seq_start; /* fixed layout only, device int32[batch] or NULL: first real token of each row */

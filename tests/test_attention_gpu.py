@@ -612,9 +612,10 @@ def test_empty_rows_and_empty_sequences(near):
     q, k, v, pk, pq = _inputs(3, 300, H, D, pb, mr, torch.bfloat16, 41, 1.0)
     kw = dict(position_buckets=pb, max_relative_positions=mr, near_splits=near)
     out = torch.full((3, 300, H, D), 7.0, dtype=torch.bfloat16, device="cuda")
-    ops.disentangled_attention_fwd(_dev(q), _dev(k), _dev(v), _dev(pk), _dev(pq), out=out,
-                                   seq_len=torch.tensor(lens, dtype=torch.int32).cuda(), **kw)
+    _, lse = ops.disentangled_attention_fwd(_dev(q), _dev(k), _dev(v), _dev(pk), _dev(pq), out=out, return_lse=True,
+                                            seq_len=torch.tensor(lens, dtype=torch.int32).cuda(), **kw)
     assert (out[1] == 0).all() and (out[2, 77:] == 0).all()
+    assert (lse.view(3, 300, H)[1] == 0).all() and (lse.view(3, 300, H)[2, 77:] == 0).all()
     cu = torch.tensor([0, 300, 300, 377], dtype=torch.int32)
     packed = torch.cat([q[0], q[2, :77]]), torch.cat([k[0], k[2, :77]]), torch.cat([v[0], v[2, :77]])
     outp = ops.disentangled_attention_fwd(*[_dev(x) for x in packed], _dev(pk), _dev(pq), cu_seqlens=cu.cuda(),

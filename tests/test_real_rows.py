@@ -74,7 +74,7 @@ def test_nothing_reads_the_rows_left_out(side):
     seen = []
 
     def pack(t):   # what a hook on the saved tensors meets: no memory that nobody has written
-        assert t.dtype == torch.float32 or not t.is_floating_point() or t.isfinite().all(), t.shape
+        assert not t.is_floating_point() or t.isfinite().all(), t.shape
         return t
 
     for poison in (0.0, float("nan"), float("nan")):
