@@ -72,19 +72,6 @@ constexpr int32_t kRadiusCap = 1 << 22;
 
 static_assert(FDB_MAX_FAR_SPLITS == FDB_MAX_FAR_PARTS, "public and internal limit of the far splits");
 
-// Compute units of the current device (256 if it cannot be asked).
-int cu_count() {
-  static std::atomic<int> cached[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cached[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-    cached[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 int64_t query_tiles(const fdb_attn_args* a) {
   return a->cu_seqlens ? fdb_worklist_max_tiles(a->total_tokens, a->batch)
                        : (int64_t)a->batch * ((a->max_seqlen + FDB_BM - 1) / FDB_BM);
@@ -144,7 +131,7 @@ int far_parts_wanted(const fdb_attn_args* a) {
     typical = a->total_tokens / a->batch;
     if (typical < 2 * a->lut_radius + FDB_BM) return 1;
   }
-  const int64_t wgs = query_tiles(a) * a->heads, slots = 3 * (int64_t)cu_count();
+  const int64_t wgs = query_tiles(a) * a->heads, slots = 3 * (int64_t)fdb_cu_count();
   if (wgs >= slots) return 1;
   const int n64 = (typical + FDB_BN - 1) / FDB_BN;
   const int near64 = (FDB_BM + 2 * a->lut_radius + 3 * (FDB_BN - 1)) / FDB_BN;  // of a query tile in mid-sequence
@@ -168,7 +155,7 @@ int near_parts_wanted(const fdb_attn_args* a) {
   // A packed batch has its lengths on the device: the host goes by the mean length and by the most query tiles the
   // token count allows (the kernel divides each query tile's own steps among the shares, whatever they are).
   const int32_t typical = a->cu_seqlens ? a->total_tokens / a->batch : a->max_seqlen;
-  const int64_t wgs = query_tiles(a) * a->heads, slots = 2 * (int64_t)cu_count();
+  const int64_t wgs = query_tiles(a) * a->heads, slots = 2 * (int64_t)fdb_cu_count();
   const int steps_all = (typical + 31) / 32, steps_near = (FDB_BM + 2 * a->lut_radius + 3 * (FDB_BN - 1)) / 32;
   const int steps = steps_all < steps_near ? steps_all : steps_near;
   int best = 1;
@@ -195,7 +182,7 @@ int key_parts_wanted(const fdb_attn_args* a) {
   // tiles' soft-max does not meet otherwise (a row's first tile always shows it a key) and is not written for
   if (a->causal) return 1;
   if (a->far_splits > 0) return a->far_splits;
-  const int64_t wgs = query_tiles(a) * a->heads, slots = cu_count();
+  const int64_t wgs = query_tiles(a) * a->heads, slots = fdb_cu_count();
   int n = (int)(slots / wgs);
   if (n > FDB_MAX_FAR_PARTS) n = FDB_MAX_FAR_PARTS;
   while (n > 1 && n64 / n < 2) --n;
@@ -211,6 +198,18 @@ int64_t far_part_bytes(const fdb_attn_args* a) {
 }
 
 }  // namespace
+
+int fdb_cu_count() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
 
 // ---- the entry point that allocates nothing ---------------------------------------------------------
 // Its scratch lives in the library's own device image: one copy per GPU, held until the process ends.
@@ -572,7 +571,7 @@ int fdb_attn_bwd(const fdb_attn_bwd_args* a, void* stream) {
   // causal 2.83 -> 2.03); a launch of at most two rounds is a little faster with the tiles of a pair spread out.
   const int64_t tiles = ((int64_t)a->seqlen + FDB_BM - 1) / FDB_BM, pairs = (int64_t)a->batch * a->heads;
   if (tiles * pairs > INT32_MAX) return FDB_ERR_SHAPE;
-  p.pairs_per_xcd = (pairs >= 8 && tiles * pairs > 4 * (int64_t)cu_count()) ? 1 : 0;
+  p.pairs_per_xcd = (pairs >= 8 && tiles * pairs > 4 * (int64_t)fdb_cu_count()) ? 1 : 0;
   // the ring holds a step's window, a partly stored group and, with chunked stores, up to seven or three more complete groups
   p.store_chunks = !has_pos ? 1 : a->lut_window + 4 + 28 <= FDB_BWD_RING ? 8 : a->lut_window + 4 + 12 <= FDB_BWD_RING ? 4 : 1;
   return fdb_launch_bwd(p, a->dtype, a->head_dim, stream);
@@ -629,7 +628,7 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   // Shares of the tokens for the tables' gradients: the launch has H * groups workgroups per share, two fit a CU; a share is a
   // whole number of chunks of a batch row, at least eight row blocks each, the same number for every share.
   const int64_t per = (int64_t)a->heads * p->tg_groups;
-  int64_t parts = 2 * (int64_t)cu_count() / per;
+  int64_t parts = 2 * (int64_t)fdb_cu_count() / per;
   if (parts > 16) parts = 16;
   if (parts < 1) parts = 1;
   auto chunks_for = [&](int64_t n) {   // chunks per batch row that deal batch * chunks evenly to n shares
@@ -745,7 +744,7 @@ int fdb_linear(const void* x, const void* w, const void* bias, void* out, int32_
     // compute unit each.  Streamed / tiled, bf16, us: 160 x 772 x 768 4.2 / 5.0, 200 x 772 x 768 6.0 / 5.0, 64 x 2308 x 768 6.0 / 5.0,
     // 300 x 2308 x 768 14.6 / 5.8, 4096 x 772 x 768 53.3 / 12.4; 160 x 772 x 3072 10.5 / 13.0, 200 x 772 x 3072 19.2 / 13.0, 300 x 3076 x 3072 68.3 / 17.4.
     const int64_t streamed = (int64_t)((cols + 15) / 16) * ((rows + 31) / 32);
-    if (wide || streamed > cu_count())
+    if (wide || streamed > fdb_cu_count())
       return fdb_launch_gemm(x, w, bias, nullptr, out, rows, cols, depth, ldx, ldw, ldo, 0, wide ? (int)FDB_GEMM_PLAIN : (int)FDB_GEMM_NARROW, dtype, stream);
   }
   return fdb_launch_linear(x, w, bias, out, rows, cols, depth, ldx, ldw, ldo, dtype, stream);
@@ -775,7 +774,7 @@ static int gemm_real(const void* x, const void* w, const void* bias, void* out, 
       cols > (1 << 24) || ldx > (1 << 22) || ldw > (1 << 22) || rows * ldx * 2 > INT32_MAX)  // all rows of x and 192 of w within a lane's 32-bit offset
     return FDB_ERR_SHAPE;
   if (!aligned16(x) || !aligned16(w) || !aligned16(out) || ldx % 8 || ldw % 8 || ldo % 8 || (reinterpret_cast<uintptr_t>(bias) & 7u)) return FDB_ERR_ALIGN;
-  return fdb_launch_gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, clear, cu_count(), dtype, stream);
+  return fdb_launch_gemm_real(x, w, bias, out, seq_start, seq_len, batch, seqlen, cols, depth, ldx, ldw, ldo, clear, dtype, stream);
 }
 
 int fdb_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
@@ -811,7 +810,7 @@ int fdb_join(const void* const w[3], const void* const b[3], void* w_out, void* 
 
 int64_t fdb_wgrad_workspace_bytes(int32_t rows0, int32_t rows1, int32_t x_cols, int32_t y_cols) {
   if (rows0 < 1 || rows1 < 1 || x_cols < 64 || y_cols < 64) return FDB_ERR_SHAPE;
-  return (int64_t)fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols, y_cols, cu_count()) * x_cols * (y_cols + 1) * 4;
+  return (int64_t)fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols, y_cols) * x_cols * (y_cols + 1) * 4;
 }
 
 int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
@@ -825,7 +824,7 @@ int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, co
   for (const void* x : {x0, y0, x1, y1, (const void*)dw, (const void*)db, (const void*)workspace})
     if (!aligned16(x)) return FDB_ERR_ALIGN;
   if (reinterpret_cast<uintptr_t>(workspace) & 31u) return FDB_ERR_ALIGN;
-  return fdb_launch_wgrad(x0, y0, rows0, x_cols0, x1, y1, rows1, x_cols1, y_cols, dw, db, (float*)workspace, fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols0, y_cols, cu_count()), dtype,
+  return fdb_launch_wgrad(x0, y0, rows0, x_cols0, x1, y1, rows1, x_cols1, y_cols, dw, db, (float*)workspace, fdb_wgrad_shares((int64_t)rows0 + rows1, x_cols0, y_cols), dtype,
                           stream);
 }
 

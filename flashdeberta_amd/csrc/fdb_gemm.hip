@@ -349,10 +349,11 @@ int64_t tiles_of(int64_t M, int64_t N, int tm, int tn) { return (M + tm - 1) / t
 // (64 x 96, 128 x 96, 128 x 128, 128 x 144, 128 x 192 and 256 x 256, with two to five stages, lie between these.)
 template <class QT, int EPI>
 int launch_gemm(const GemmParams& p, hipStream_t stream) {
-  if (tiles_of(p.M, p.N, 32, 64) <= 256) return launch_shape<QT, EPI, S32x64>(p, stream);
-  if (tiles_of(p.M, p.N, 64, 64) <= 480) return launch_shape<QT, EPI, S64x64>(p, stream);
-  if (tiles_of(p.M, p.N, 64, 192) <= 256) return launch_shape<QT, EPI, S64x192Deep>(p, stream);
-  if (tiles_of(p.M, p.N, 64, 192) <= 512) return launch_shape<QT, EPI, S64x192>(p, stream);
+  const int64_t cus = fdb_cu_count();
+  if (tiles_of(p.M, p.N, 32, 64) <= cus) return launch_shape<QT, EPI, S32x64>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 64) * 8 <= cus * 15) return launch_shape<QT, EPI, S64x64>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 192) <= cus) return launch_shape<QT, EPI, S64x192Deep>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 192) <= 2 * cus) return launch_shape<QT, EPI, S64x192>(p, stream);
   return launch_shape<QT, EPI, S256x192>(p, stream);
 }
 
@@ -368,12 +369,12 @@ int launch_type(const GemmParams& p, int epilogue, hipStream_t stream) {
 
 // Where this kernel is the faster one, and adds up as the library does.  Up to 32 rows the weights are streamed by many waves that share the
 // contraction.  A long contraction over few tiles is split by the library ([512 x 3072] . [3072 x 768] + residual 13.5 us there, 13.9 here; 1500 rows
-// 21.7 and 18.3).  A plain product has nothing to gain from 512 tiles of 64 x 192 up (4096 and 3000 rows to 2304 columns: 19.3 and 16.7 us there, 20.8
+// 21.7 and 18.3).  A plain product has nothing to gain beyond two tiles of 64 x 192 a compute unit (4096 and 3000 rows to 2304 columns: 19.3 and 16.7 us there, 20.8
 // and 19.7 here; 2048, 1024 and 512 rows 15.5, 11.2 and 8.1 there, 12.7, 9.4 and 7.1 here).
 extern "C" int32_t fdb_gemm_serves(int64_t M, int64_t N, int64_t K, int32_t epilogue) {
   if (M <= 32 || N < 8 || K < kDepth || N % 8 || K % kDepth || M > (1 << 24) || N > (1 << 24)) return 0;
-  if (K > 1536 && tiles_of(M, N, 64, 64) <= 256) return 0;
-  return epilogue != kPlain || tiles_of(M, N, 64, 192) <= 512;
+  if (K > 1536 && tiles_of(M, N, 64, 64) <= fdb_cu_count()) return 0;
+  return epilogue != kPlain || tiles_of(M, N, 64, 192) <= 2 * fdb_cu_count();
 }
 
 int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* residual, void* out, int32_t M, int32_t N, int32_t K, int64_t ldx,
@@ -386,13 +387,13 @@ int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* 
 extern "C" int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t N, int64_t K, int64_t ldx) {
   const int64_t M = batch * seqlen;
   if (batch < 1 || batch > kRealSequences || seqlen < 1 || N < 8 || K < kDepth || N % 8 || K % kDepth || M > (1 << 24) || N > (1 << 24)) return 0;
-  return M * ldx * 2 <= INT32_MAX && tiles_of(M, N, 64, 192) > 512;
+  return M * ldx * 2 <= INT32_MAX && tiles_of(M, N, 64, 192) > 2 * fdb_cu_count();
 }
 
 int fdb_launch_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* start, const int32_t* length, int32_t batch, int32_t seqlen,
-                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t cus, int dtype, void* stream) {
+                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int dtype, void* stream) {
   RealParams p{};
   p.g = GemmParams{(const char*)x, (const char*)w, (const char*)bias, nullptr, (char*)out, ldx, ldw, ldo, 0, batch * seqlen, N, K, 0, 0};
-  p.start = start, p.length = length, p.batch = batch, p.seqlen = seqlen, p.cus = cus, p.clear = clear;
+  p.start = start, p.length = length, p.batch = batch, p.seqlen = seqlen, p.cus = fdb_cu_count(), p.clear = clear;
   return dtype == FDB_BF16 ? launch_real<Bf16Tr>(p, (hipStream_t)stream) : launch_real<F16Tr>(p, (hipStream_t)stream);
 }

@@ -342,7 +342,7 @@ int launch_dgrad(DgradParams p, hipStream_t stream) {
 template <class QT>
 int launch_dgrad_rows(const DgradParams& p, hipStream_t stream) {
   const int64_t tiles = (int64_t)(tiles_of(p.rows[0], 64) + tiles_of(p.rows[1], 64)) * tiles_of(p.cols, 128);
-  return tiles <= 512 ? launch_dgrad<QT, 64>(p, stream) : launch_dgrad<QT, 128>(p, stream);
+  return tiles <= 2 * fdb_cu_count() ? launch_dgrad<QT, 64>(p, stream) : launch_dgrad<QT, 128>(p, stream);
 }
 
 template <class QT>
@@ -366,16 +366,16 @@ int launch_wgrad(WgradParams p, void* dw, void* db, hipStream_t stream) {
 // Shares of the contraction: as many as have a place of their own on the chip, each with six stages at least (a share's partial result
 // costs as much as three).  12 heads, 1 / 2 / 3 / 4 / 5 shares: 4096 tokens 71.9 42.0 35.7 31.2* 41.4 us, 1000 tokens 30.6 23.0 22.9 23.3* 27.7, 300 tokens
 // 21.3 19.0* 20.3 22.5 24.3; 16 heads, 4096 tokens 73.9 47.0* 59.6 54.7 52.7.  A library product each and the column sums: 52.9, 33.5, -, 60.7.
-int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols, int cus) {
+int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols) {
   const int64_t tiles = (int64_t)tiles_of(x_cols, WShape::TM) * tiles_of(y_cols, WShape::TN), stages = tiles_of(rows, kDepth);
-  return (int)std::max<int64_t>(1, std::min<int64_t>({2 * cus / tiles, stages / 6, 16}));
+  return (int)std::max<int64_t>(1, std::min<int64_t>({2 * fdb_cu_count() / tiles, stages / 6, 16}));
 }
 
 // Where one launch beats a library product each: unless a second round of workgroups is mostly empty (16 heads, 8192 tokens: 544 tiles,
 // 70.1 us against 58.5; 12 heads, 408 tiles, 31.0 against 43.9).
 extern "C" int32_t fdb_dgrad_serves(int64_t rows0, int64_t rows1, int64_t cols) {
-  const int64_t tiles = (tiles_of(rows0, 128) + tiles_of(rows1, 128)) * (int64_t)tiles_of(cols, 128), rounds = (tiles + 511) / 512;
-  return tiles >= 384 * rounds || rounds == 1;
+  const int64_t tiles = (tiles_of(rows0, 128) + tiles_of(rows1, 128)) * (int64_t)tiles_of(cols, 128), places = 2 * fdb_cu_count(), rounds = (tiles + places - 1) / places;
+  return 4 * tiles >= 3 * places * rounds || rounds == 1;
 }
 
 int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0,

@@ -191,6 +191,9 @@ inline hipError_t fdb_set_lds_once(const void* kern, int lds_bytes, std::atomic<
 // Most workgroups per query tile a far-only launch is split into.
 #define FDB_MAX_FAR_PARTS 4
 
+// Compute units of the current device (256 if it cannot be asked).
+int fdb_cu_count();
+
 // Launchers return the hipError_t of the launch as int.
 // fdb_launch_attn, by mode:
 //   FDB_MODE_FUSED      one kernel walks every key tile;
@@ -225,10 +228,10 @@ int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* 
 // The plain product where columns and output rows come by fours only, or the bias lies on any element: for fdb_linear, not an epilogue of fdb_gemm's.
 enum { FDB_GEMM_NARROW = 3 };
 int fdb_launch_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* start, const int32_t* length, int32_t batch, int32_t seqlen,
-                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t cus, int dtype, void* stream);
+                         int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int dtype, void* stream);
 int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0,
                      void* out1, int dtype, void* stream);  // fdb_grad.hip
-int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols, int cus);
+int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols);
 int fdb_launch_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, const void* x1, const void* y1, int32_t rows1, int32_t x_cols1, int32_t y_cols,
                      void* dw, void* db, float* ws, int32_t shares, int dtype, void* stream);
 int fdb_launch_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream);

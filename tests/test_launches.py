@@ -71,3 +71,25 @@ def test_linear_layers_of_many_rows_are_tiled():
              _linear(160, 772, 768), _linear(200, 770, 768), _linear(200, 768, 96)]
     for (rc, made), tiled in zip(launches(calls), [True] * 4 + [False] * 4):
         assert rc == 0 and len(made) == 1 and ("fdb_gemm_kernel" in made[0][0]) == tiled, made
+
+
+def _gemm(rows, cols, depth, epilogue):
+    return "fdb_gemm", [P(0x1000)] * 5 + [rows, cols, depth, depth, depth, cols, cols, epilogue, _lib.FDB_BF16, None]
+
+
+def _dgrad(rows, cols):
+    return "fdb_dgrad", [P(0x1000), rows, 3 * cols, P(0x1000), 0, 64, P(0x1000), cols, P(0x1000), P(0x1000), _lib.FDB_BF16, None]
+
+
+def test_thresholds_of_the_products_follow_the_compute_units():
+    """A device of half the compute units takes the kernels for half the rows, and serves it where this one serves twice as many."""
+    rows = [256, 512, 1024, 1536, 2048, 3072, 4096, 8192, 16384]
+    sizes = [(r, c, d, e) for r in rows for c in (768, 2304, 3072) for d in (768, 3072) for e in (0, 2)]
+    asked = lambda part: ([_gemm(r // part, c, d, e) for r, c, d, e in sizes] + [_dgrad(r // part, c) for r in rows for c in (768, 1024)]
+                          + [("fdb_gemm_serves", [r // part, c, d, e]) for r, c, d, e in sizes] + [("fdb_gemm_real_serves", [8 // part, r // 8, c, d, d]) for r, c, d, e in sizes]
+                          + [("fdb_dgrad_serves", [r // part, 0, c]) for r in rows for c in (768, 1024)])
+    whole, half = launches(asked(1), cus=256), launches(asked(2), cus=128)
+    kernels = lambda made: [name for name, *_ in made]
+    for call, (rc, made), (rc_half, made_half) in zip(asked(1), whole, half):
+        assert rc == rc_half and kernels(made) == kernels(made_half), (call, made, made_half)
+    assert len({k for _, made in whole for k in kernels(made)}) > 10   # every tile is among them
