@@ -83,8 +83,8 @@ def test_where_it_serves():
                                          (dict(x=24), "ALIGN"), (dict(bias=20), "ALIGN"), (dict(ldo=68), "ALIGN"), (dict(residual=0), "NULL"), (dict(residual=8), "ALIGN"),
                                          (dict(ldr=56), "SHAPE"), (dict(dtype=0), "DTYPE"), (dict(epilogue=3), "UNSUPPORTED")])
 def test_refused_on_the_host(change, code):
-    codes = {"NULL": -1}
+    codes = {"NULL": -1, "DTYPE": -2, "ALIGN": -4, "SHAPE": -5, "UNSUPPORTED": -10}
     kw = dict(x=16, w=32, bias=48, residual=64, out=80, rows=64, cols=64, depth=64, ldx=64, ldw=64, ldo=64, ldr=64, epilogue=RESIDUAL, dtype=_lib.FDB_BF16)
     kw.update(change)
     rc = _lib.lib.fdb_gemm(*[v or None if k in ("x", "w", "bias", "residual", "out") else v for k, v in kw.items()], None)
-    assert rc < 0 and (code not in codes or rc == codes[code]), (rc, code)
+    assert rc == codes[code], (rc, code)

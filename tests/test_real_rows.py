@@ -55,6 +55,20 @@ def test_where_it_serves():
     assert not serves(65, 512, 2304, 768, 768) and not serves(8, 512, 2304, 100, 104) and not serves(64, 65536, 2304, 768, 768)
 
 
+@pytest.mark.parametrize("entry", ["fdb_gemm_real", "fdb_gemm_real_cleared"])
+@pytest.mark.parametrize("change,code", [
+    (dict(x=0), -1), (dict(w=0), -1), (dict(out=0), -1), (dict(length=0), -1), (dict(dtype=_lib.FDB_F32), -2), (dict(dtype=_lib.FDB_FP8_E4M3), -2),
+    (dict(batch=0), -5), (dict(batch=65), -5), (dict(seqlen=0), -5), (dict(batch=64, seqlen=(1 << 18) + 1), -5), (dict(cols=12), -5), (dict(cols=0), -5), (dict(depth=96), -5),
+    (dict(depth=32), -5), (dict(ldx=56), -5), (dict(ldw=56), -5), (dict(ldo=56), -5), (dict(ldx=(1 << 22) + 8), -5), (dict(ldw=(1 << 22) + 8), -5),
+    (dict(batch=64, seqlen=1 << 18, ldx=64), -5),    # rows of x past 2 GB
+    (dict(x=24), -4), (dict(w=40), -4), (dict(out=88), -4), (dict(bias=52), -4), (dict(ldx=68), -4), (dict(ldw=68), -4), (dict(ldo=68), -4)])
+def test_refused_on_the_host(change, code, entry):
+    kw = dict(x=16, w=32, bias=48, out=80, start=0, length=96, batch=8, seqlen=64, cols=64, depth=64, ldx=64, ldw=64, ldo=64, dtype=_lib.FDB_BF16)
+    kw.update(change)
+    args = [v or None if k in ("x", "w", "bias", "out", "start", "length") else v for k, v in kw.items()]
+    assert getattr(_lib.lib, entry)(*args, None) == code
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("side", ["right", "left"])
 def test_nothing_reads_the_rows_left_out(side):
