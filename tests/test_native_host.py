@@ -126,6 +126,33 @@ def test_encoder_layer_matches_the_module_by_module_forward(B, L):
         assert calls
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("width", [768, 1024])
+@pytest.mark.parametrize("B,L", [(2, 40), (3, 300), (6, 256), (8, 384), (5, 999)])   # every tile, and from (8, 384) on the products of real rows
+def test_encoder_layer_bits_at_the_widths_of_the_models(B, L, width, dtype):
+    """The layer as one call against its modules, and its attention against the library's product of all rows."""
+    from transformers.models.deberta_v2.modeling_deberta_v2 import DebertaV2Layer
+
+    from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model, ops
+
+    torch.manual_seed(width + L)
+    cfg = DebertaV2Config(vocab_size=100, hidden_size=width, num_hidden_layers=1, num_attention_heads=width // 64, intermediate_size=4 * width,
+                          relative_attention=True, pos_att_type="p2c|c2p", position_buckets=32, max_relative_positions=64, share_att_key=True,
+                          norm_rel_ebd="layer_norm", position_biased_input=False, initializer_range=0.05)
+    layer = FlashDebertaV2Model(cfg).eval().cuda().to(dtype).encoder.layer[0]
+    x, rel = torch.randn(B, L, width, device="cuda").to(dtype), torch.randn(64, width, device="cuda").to(dtype)
+    lengths = torch.tensor([L] + [L - (b * L) // (B + 1) for b in range(1, B)], device="cuda")
+    mask = (torch.arange(L, device="cuda") < lengths[:, None]).long()
+    with torch.no_grad():
+        assert torch.equal(layer(x, mask, rel_embeddings=rel)[0], DebertaV2Layer.forward(layer, x, mask, rel_embeddings=rel)[0])
+        att = layer.attention.self
+        q, k, v = [F.linear(x, p.weight, p.bias).view(B, L, -1, 64) for p in (att.query_proj, att.key_proj, att.value_proj)]
+        pk, pq = [F.linear(rel, p.weight, p.bias).view(64, -1, 64).transpose(0, 1) for p in (att.key_proj, att.query_proj)]
+        ref = ops.disentangled_attention_fwd(q, k, v, pk, pq, position_buckets=32, max_relative_positions=64, seq_len=lengths.int())
+        assert torch.equal(att(x, mask, rel_embeddings=rel)[0], ref.view(B, L, width))
+
+
 def _encoder_layer(dropout=0.1):
     from flashdeberta_amd import DebertaV2Config, FlashDebertaV2Model
 
