@@ -300,11 +300,17 @@ __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles
   h_out = __builtin_amdgcn_readfirstlane(h);
 }
 
+// The 16-bit products by tiles of 16 x 16 outputs, and where they keep a row of 128 bytes in LDS: slot (row, s) holds chunk s ^ swz16(row), so that
+// sixteen rows' same chunk lies in sixteen bank groups.
+__device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ int swz16(int row) { return 4 * ((row >> 1) & 1) | (-(row >> 2) & 3); }
+
 // A kernel argument in scalar registers of its own.  The compiler loads arguments sixteen registers at a time; where a loop wants
 // more scalar registers than there are, it keeps such a group in lanes of a vector register and brings all sixteen back
-// (sixteen v_readlane) for the one argument a step uses.  50 of some 330 instructions of a near step in e4m3: 889 -> 883 us at B = 4,
-// L = 8192, 12 heads; 124 in the loops of the backward's launch of both roles: 75.4 -> 71.2 us at B = 8, L = 512, twelve heads.  The 16-bit
-// near kernel keeps none in its loops, and is slower with the copies.
+// (sixteen v_readlane) for the one argument a step uses: 124 in the loops of the backward's launch of both roles, 75.4 -> 71.2 us at B = 8,
+// L = 512, twelve heads; 50 of some 330 instructions of a near step in e4m3, whose time did not change beyond its noise.  The 16-bit near
+// kernel keeps none in its loops, and is slower with the copies.
 __device__ __forceinline__ uint32_t own_sgpr(uint32_t x) {
   uint32_t r;
   asm("s_mov_b32 %0, %1" : "=&s"(r) : "s"(__builtin_amdgcn_readfirstlane(x)));

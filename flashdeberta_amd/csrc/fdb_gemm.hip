@@ -28,9 +28,6 @@ using namespace fdb;
 
 namespace {
 
-__device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f32x4 mma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
 // GELU of a 16-bit value, rounded to its type, as torch's elementwise kernel computes it.  erff and what goes with it are some 45 vector
 // instructions an element and no memory time hides them here; a bf16 has so few values that matter (2^-14 <= |x| < 8: 17 binades of 128
 // and a sign) that each workgroup tabulates them while its first tiles are on their way, and looks the others up.
@@ -49,9 +46,8 @@ struct GemmParams {
 };
 
 // A workgroup of WM x WN waves makes TM x TN outputs, PER_CU of them share a CU; stages of kDepth of the contraction go straight from global
-// memory into one of STAGES LDS buffers, rows of 128 bytes, slot (row, s) = chunk s ^ swz(row) (sixteen rows' same chunk: sixteen bank groups).
+// memory into one of STAGES LDS buffers, rows of 128 bytes, slot (row, s) = chunk s ^ swz16(row) (sixteen rows' same chunk: sixteen bank groups).
 constexpr int kDepth = 64;
-__device__ __forceinline__ int swz(int row) { return 4 * ((row >> 1) & 1) | (-(row >> 2) & 3); }
 
 template <int TM_, int TN_, int WM_, int WN_, int STAGES_, int PER_CU_, int STAGED_ = TN_>
 struct GemmShape {   // STAGED: rows of w that are fetched, TN or what makes whole loads for every wave
@@ -88,7 +84,7 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
 #pragma unroll
   for (int j = 0; j < S::LOADS; ++j) {
     const int c = wave + S::NW * j, row = c * S::RPI + (lane >> 3);   // rows past the end re-read the last one
-    const uint32_t chunk = (uint32_t)(((lane & 7) ^ swz(row)) * 16);
+    const uint32_t chunk = (uint32_t)(((lane & 7) ^ swz16(row)) * 16);
     if (c < S::XI) off[j] = rows.from_base(m0, row) * (uint32_t)(p.ldx * 2) + chunk;
     else off[j] = (uint32_t)(min(n0 + row - TM, p.N - 1) - n0) * (uint32_t)(p.ldw * 2) + chunk;
   }
@@ -116,7 +112,7 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
       ((__bf16*)table)[kGeluCount + e] = (__bf16)(-v * 0.5f * (1.f - t));
     }
   }
-  const uint32_t xrow = (uint32_t)((wm * S::FM * 16 + r) * S::ROWB), wrow = (uint32_t)((TM + wn * S::FN * 16 + r) * S::ROWB), f = (uint32_t)swz(r);
+  const uint32_t xrow = (uint32_t)((wm * S::FM * 16 + r) * S::ROWB), wrow = (uint32_t)((TM + wn * S::FN * 16 + r) * S::ROWB), f = (uint32_t)swz16(r);
   int buf = 0;
 #pragma unroll 1
   for (int t = 0; t < steps; ++t) {

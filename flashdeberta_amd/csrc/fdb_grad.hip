@@ -20,19 +20,15 @@ using namespace fdb;
 
 namespace {
 
-__device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f32x4 mma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-
-// LDS rows are 128 bytes, slot (row, s) = chunk s ^ swz(row), as in fdb_gemm.hip.  An operand whose contraction runs down its rows is staged in
+// LDS rows are 128 bytes, slot (row, s) = chunk s ^ swz16(row), as in fdb_gemm.hip.  An operand whose contraction runs down its rows is staged in
 // panels of 64 rows (one stage of the contraction) by 64 columns and read transposed.
 constexpr int kDepth = 64, kRow = 128, kPanel = kDepth * kRow;
-__device__ __forceinline__ int swz(int row) { return 4 * ((row >> 1) & 1) | (-(row >> 2) & 3); }
 
 // This lane's part of the address of a transposed operand: 16 columns from 16 * f on, contraction 8 * kg + 4 * h + 0..3 of the 32 at
 // hand; f, h and the 32 are left to the instruction's offset where they do not touch the swizzle.
 __device__ __forceinline__ uint32_t tr_lane(int lane, int f, int h) {
   const int s16 = lane & 15, row = 8 * (lane >> 4) + 4 * h + (s16 >> 2);
-  return (uint32_t)(row * kRow + (((2 * (f & 3) + ((s16 >> 1) & 1)) ^ swz(row)) * 16) + (s16 & 1) * 8);
+  return (uint32_t)(row * kRow + (((2 * (f & 3) + ((s16 >> 1) & 1)) ^ swz16(row)) * 16) + (s16 & 1) * 8);
 }
 template <class QT>
 __device__ __forceinline__ typename QT::frag tr_frag(uint32_t lo, uint32_t hi, int offset) {   // the offset travels in the instructions
@@ -85,10 +81,10 @@ __global__ __launch_bounds__(256, 2) void fdb_dgrad_kernel(const DgradParams p) 
     const int c = wave + S::NW * j;
     if (j < S::XLOADS) {
       const int row = 8 * c + (lane >> 3);
-      off[j] = (uint32_t)(min(m0 + row, rows - 1) - m0) * (uint32_t)(depth * 2) + (uint32_t)(((lane & 7) ^ swz(row)) * 16);
+      off[j] = (uint32_t)(min(m0 + row, rows - 1) - m0) * (uint32_t)(depth * 2) + (uint32_t)(((lane & 7) ^ swz16(row)) * 16);
     } else {
       const int w = c - S::TM / 8, row = 8 * (w & 7) + (lane >> 3);
-      off[j] = (uint32_t)row * (uint32_t)(cols * 2) + (uint32_t)(min(n0 + 64 * (w >> 3), cols - 64) * 2) + (uint32_t)(((lane & 7) ^ swz(row)) * 16);
+      off[j] = (uint32_t)row * (uint32_t)(cols * 2) + (uint32_t)(min(n0 + 64 * (w >> 3), cols - 64) * 2) + (uint32_t)(((lane & 7) ^ swz16(row)) * 16);
     }
   }
   auto fill = [&](int buf) __attribute__((always_inline)) {
@@ -107,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void fdb_dgrad_kernel(const DgradParams p) 
 #pragma unroll
   for (int t = 0; t < S::STAGES - 1; ++t)
     if (t < steps) fill(t);
-  const uint32_t xrow = lds0 + (uint32_t)((wm * 16 * S::FM + r) * kRow), f = (uint32_t)swz(r);
+  const uint32_t xrow = lds0 + (uint32_t)((wm * 16 * S::FM + r) * kRow), f = (uint32_t)swz16(r);
   uint32_t wlane[4][2];
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -187,7 +183,7 @@ __global__ __launch_bounds__(64 * WShape::NW, 2) void fdb_wgrad_kernel(const Wgr
 #pragma unroll
   for (int j = 0; j < S::LOADS; ++j) {
     const int c = wave + S::NW * j, row = 8 * (c & 7) + (lane >> 3);
-    const uint32_t chunk = (uint32_t)(((lane & 7) ^ swz(row)) * 16);
+    const uint32_t chunk = (uint32_t)(((lane & 7) ^ swz16(row)) * 16);
 #pragma unroll
     for (int w = 0; w < 2; ++w)
       off[w][j] = (uint32_t)row * (uint32_t)((j < S::XLOADS ? p.x_cols[w] : p.y_cols) * 2) + chunk +

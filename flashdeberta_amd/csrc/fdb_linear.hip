@@ -4,7 +4,8 @@
 // launch costs 2.5.  Up to 32 rows fdb_linear_kernel streams the weights: one workgroup per 16 output columns, eight or
 // sixteen waves that share the contraction, so that even a [768 x 768] weight is on its way through 48 x 8 waves at once, each
 // with four steps' loads in flight.  In a replayed graph, [24 x 768] . [768 x 2304]: 4.0 us against hipBLASLt's 4.8.
-// Beyond that fdb_gemm.hip's tiles, for the sizes they take (columns and output rows by eights, or by fours where the streaming makes more than one round): [64 / 200 x 768] . [768 x 2304] 5.3 / 5.6 us.
+// Beyond that fdb_gemm.hip's tiles, for the sizes they take (columns and output rows by eights, or by fours where the streaming makes more
+// than one round): [64 / 200 x 768] . [768 x 2304] 5.3 / 5.6 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -17,9 +18,6 @@ using namespace fdb;
 namespace {
 
 constexpr int kLinCols = 16;
-
-__device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f32x4 mma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
 // out [M, N] = x [M, K] . w [N, K]^T + bias.  Contraction steps of 32 go round the waves; MT row blocks of 16 per
 // workgroup share every weight fragment.  A lane reads 16 bytes of a row, four lanes 64 contiguous bytes.

@@ -254,8 +254,8 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
     else if (then == Then::gelu) at::gelu_(y);
     return y;
   };
-  if (!x_in.is_cuda() || !half || !plain_memory(x_in) || !plain_memory(w) || (bias && !plain_memory(*bias)) || w.scalar_type() != type || (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 ||
-      w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) || w.device() != x_in.device() || !bias || bias->device() != x_in.device() ||
+  if (!x_in.is_cuda() || !half || !plain_memory(x_in) || !plain_memory(w) || (bias && !plain_memory(*bias)) || w.scalar_type() != type ||
+      (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 || w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) || w.device() != x_in.device() || !bias || bias->device() != x_in.device() ||
       bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())
     return rest(at::linear(x_in, w, bias));
   const c10::hip::HIPGuard guard(x_in.get_device());
@@ -894,8 +894,10 @@ struct LayerNode : public torch::autograd::Function<LayerNode> {
     if (for_hidden) dhidden = at::empty(hidden.sizes(), hidden.options());
     if (for_rel) drel = rel_rows > rows ? at::zeros({rel_rows, C}, hidden.options()) : at::empty({rel_rows, C}, hidden.options());
     if (for_hidden || for_rel) {
-      const int rc = n > INT32_MAX || C > INT32_MAX || !fdb_dgrad_serves(for_hidden ? n : 0, for_rel ? rows : 0, C) ? (int)FDB_ERR_SHAPE : fdb_dgrad(dqkv.data_ptr(), for_hidden ? (int32_t)n : 0, (int32_t)(3 * W), dpos.data_ptr(), for_rel ? (int32_t)rows : 0, (int32_t)(2 * W), w.data_ptr(),
-                               (int32_t)C, for_hidden ? dhidden.data_ptr() : nullptr, for_rel ? drel.data_ptr() : nullptr, code, stream_of(hidden));
+      int rc = FDB_ERR_SHAPE;
+      if (n <= INT32_MAX && C <= INT32_MAX && fdb_dgrad_serves(for_hidden ? n : 0, for_rel ? rows : 0, C))
+        rc = fdb_dgrad(dqkv.data_ptr(), for_hidden ? (int32_t)n : 0, (int32_t)(3 * W), dpos.data_ptr(), for_rel ? (int32_t)rows : 0, (int32_t)(2 * W),
+                       w.data_ptr(), (int32_t)C, for_hidden ? dhidden.data_ptr() : nullptr, for_rel ? drel.data_ptr() : nullptr, code, stream_of(hidden));
       if (rc > 0) check(rc, "fdb_dgrad");
       if (rc < 0 && for_hidden) product({dqkv, n}, false, {w, 3 * W}, false, {dhidden, n});
       if (rc < 0 && for_rel) product({dpos, rows}, false, {w, 2 * W}, false, {drel, rows});
