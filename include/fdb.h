@@ -325,6 +325,8 @@ int fdb_attn_bwd_chain(const void* d_scores, const void* x, const void* x_second
  * constant; launch of their own) and the near keys; the partial results go through the workspace, one slot of
  * rows * heads * (head_dim * sizeof(v element) + 4) bytes each (rows: those of the lse buffer): far_splits - 1
  * slots, plus near_splits slots if near_splits > 1 (a small merge kernel then follows the two launches).
+ * Where few keys are far (fixed layout, head_dim 64, up to 2048 tokens, not causal) one launch walks them all, unless
+ * far_splits or near_splits ask for two; its shares are the near ones.
  * The workspace is optional: without it (or with a smaller one) the call first gives up the near splits,
  * then uses as many far splits as fit, down to one, with the same result up to rounding.  Calls that one kernel
  * serves (fp32, head_dim 128, no position term, no lse buffer) share ALL key tiles of a query tile among up to
