@@ -383,11 +383,12 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // Padded fixed layout: the rows of `out` outside a batch row's real tokens, written by the workgroup whose tile index t
 // covers them in absolute terms (rows [128 t, 128 t + 128), two threads per row of ROW_BYTES): zeros, or `word` = the
-// element type's NaN pattern for a batch row the caller marked with a negative token count.  With lse_bh (the head's log-sum-exp of the
-// sequence's first row, `heads` floats from one row to the next or NULL) also those: 0 or NaN.
+// element type's NaN pattern for a batch row the caller marked with a negative token count.  With lse_b (the log-sum-exps of the
+// sequence's first row, `heads` of them a row, or NULL) also those: 0 or NaN.  All heads of a row by the first head's workgroups: by each head's own, up to
+// eight XCDs' caches would write parts of one line.
 template <int ROW_BYTES>
 __device__ __forceinline__ void fill_pad_rows(char* out_bh, int64_t row_stride_bytes, int t, int L, int tok0, int Lb,
-                                              uint32_t word, int tid, float* lse_bh = nullptr, int heads = 0) {
+                                              uint32_t word, int tid, float* lse_b = nullptr, int heads = 0) {
   static_assert(ROW_BYTES % 32 == 0, "two threads per row, 16-byte stores");
   const int row = t * 128 + (tid >> 1);
   if (row >= L || (row >= tok0 && row < tok0 + Lb)) return;
@@ -395,7 +396,8 @@ __device__ __forceinline__ void fill_pad_rows(char* out_bh, int64_t row_stride_b
   const u32x4 w = {word, word, word, word};
 #pragma unroll
   for (int c = 0; c < ROW_BYTES / 32; ++c) *(u32x4*)(dst + 16 * c) = w;
-  if (lse_bh && (tid & 1) == 0) lse_bh[(int64_t)row * heads] = word ? __builtin_nanf("") : 0.f;
+  if (lse_b)
+    for (int h = tid & 1; h < heads; h += 2) lse_b[(int64_t)row * heads + h] = word ? __builtin_nanf("") : 0.f;
 }
 
 // Number of direct loads (dma16 / dma16s) a wave issues per K/V tile of the far-only staging: the waits

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
       fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,
-                           sl < 0 ? VT::NAN_WORD : 0u, tid, p.lse ? p.lse + (int64_t)b * p.L * p.H + h : nullptr, p.H);
+                           sl < 0 ? VT::NAN_WORD : 0u, tid, p.lse && h == 0 ? p.lse + (int64_t)b * p.L * p.H : nullptr, p.H);
     if (m0 >= Lb) return;
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; oo = b * p.o_sb;
   }
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
       fill_pad_rows<kRowV>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,
-                           sl < 0 ? VT::NAN_WORD : 0u, tid, p.lse ? p.lse + (int64_t)b * p.L * p.H + h : nullptr, p.H);
+                           sl < 0 ? VT::NAN_WORD : 0u, tid, p.lse && h == 0 ? p.lse + (int64_t)b * p.L * p.H : nullptr, p.H);
     if (m0 >= Lb) return;
     qo = b * p.q_sb; ko = b * p.k_sb; vo = b * p.v_sb; oo = b * p.o_sb;
   }

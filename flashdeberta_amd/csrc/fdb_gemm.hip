@@ -276,7 +276,7 @@ __global__ __launch_bounds__(512, 2) void fdb_gemm_real_kernel(const RealParams 
   consider(128, p.g.tiles_n, 192);
   consider(64, p.g.tiles_n, 192);
   // Ahead of the tiles, under whose loads and products the stores drain (after them: 8 x 512 15.2 -> 16.5 us), and past the caches, since nobody
-  // reads the rows: a training layer of 8 x 512 takes 217 us without clearing, 218.5 so, 220 with ordinary stores.
+  // reads the rows: a training layer of 8 x 512 takes up to 1.5 us of 216 longer for it, 2.6 with ordinary stores.
   if (p.clear) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int i = blockIdx.x * 8 + wave; i < p.batch * p.seqlen; i += gridDim.x * 8) {   // a row a wave
