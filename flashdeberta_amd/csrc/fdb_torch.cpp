@@ -255,8 +255,8 @@ Tensor project(const Tensor& x_in, const Tensor& w, const OptTensor& bias, bool 
     return y;
   };
   if (!x_in.is_cuda() || !half || !plain_memory(x_in) || !plain_memory(w) || (bias && !plain_memory(*bias)) || w.scalar_type() != type ||
-      (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 || w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) || w.device() != x_in.device() || !bias || bias->device() != x_in.device() ||
-      bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())
+      (bias && bias->scalar_type() != type) || m < 2 || w.dim() != 2 || w.stride(1) != 1 || w.stride(0) < k || k != w.size(1) ||
+      w.device() != x_in.device() || !bias || bias->device() != x_in.device() || bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())
     return rest(at::linear(x_in, w, bias));
   const c10::hip::HIPGuard guard(x_in.get_device());
   const Tensor x = x_in.contiguous();
