@@ -94,26 +94,29 @@ bool has_far_launch(const fdb_attn_args* a) {
 }
 
 // Whether the near launch walks the far tiles, too, and the far launch is left out.  A far step costs a near workgroup, two of which share a CU,
-// more than it costs a far one, three of which do; but the far launch costs 6 to 8 us whatever it does, a first and a last round of
-// its own, and a partial result that is written and read again.  So the far tiles decide, counted for the query tile at an end of the sequence, which
-// has the most of them: the line is where the calls measured change sides.  12 heads unless stated, two launches -> one, us:
-//   radius 512       bf16                    e4m3                      radius 64 and 256   bf16                    e4m3
-//   1 x 700          28.7 -> 22.1            28.0 -> 21.4              8 x 300, 64         27.6 -> 21.4            25.7 -> 18.7
-//   3 x 777          39.9 -> 31.1            38.8 -> 30.2              3 x 777, 64         30.4 -> 25.4            29.0 -> 24.2
-//   16 x 1024        170.2 -> 146.1          124.9 -> 110.5            16 x 1024, 64       112.5 -> 101.9          96.0 -> 83.8
-//   2 x 1501         61.7 -> 57.1            57.9 -> 52.4              4 x 1501, 64        69.0 -> 69.8            55.9 -> 53.1
-//   16 x 1501        296.5 -> 267.6          221.5 -> 202.7            2 x 2048, 64        54.9 -> 61.2 (kept)     49.6 -> 59.2 (kept)
-//   3 x 2048         109.3 -> 111.6          82.7 -> 79.3              1 x 2048, 4 h., 64  32.7 -> 41.6 (kept)     32.0 -> 42.4 (kept)
-//   8 x 2048         223.3 -> 213.7          177.3 -> 170.6            8 x 1024, 256       78.3 -> 67.9            61.2 -> 52.7
-//   1 x 2048, 4 h.   42.2 -> 27.6            41.3 -> 27.4              8 x 1501, 256       131.0 -> 124.0          111.0 -> 103.1
-// fp16 runs as bf16 does (16 x 1501 304.2 -> 279.4, 3 x 2048 114.4 -> 115.4).  Without a workspace, when nothing is shared: 1 x 2048, 4 heads 61.5 -> 54.7, 1 x 1300
-// 53.9 -> 44.4, 1 x 700 35.0 -> 27.1 (e4m3 60.8 -> 54.4, 52.6 -> 42.7, 34.2 -> 26.9).
+// more than it costs a far one, three of which do; but the far launch costs 6 to 8 us whatever it does, a first and a last round of its own, and a
+// partial result that is written and read again.  So it goes by the far tiles of the query tile at an end of the sequence, which has the most of them:
+// up to 8 for any batch, and while every query tile has a compute unit to itself, where the launch lasts as long as one tile, up to 6 more than a tile in
+// mid-sequence has near ones.  Replays back to back (60 ms of each, so at the clock that lasts), two launches -> one, us, 12 heads unless stated:
+//   far at an end, radius   bf16              e4m3                 alone on a compute unit   bf16             e4m3
+//   3    512  3 x 777       38.8 -> 30.0      38.5 -> 28.9         11  512  1 x 1300         43.4 -> 31.6     41.6 -> 30.3
+//   1    512  64 x 700      356 -> 329        269 -> 243           14  512  1 x 1501         46.9 -> 42.4     44.0 -> 37.7
+//   6    512  4 x 1024      56.0 -> 47.7      50.7 -> 43.0         22  512  1 x 2048         59.2 -> 54.2     55.9 -> 49.1
+//   6    512  16 x 1024     164 -> 147        125 -> 110           22  512  1 x 2048, 4 h.   41.1 -> 26.7     40.7 -> 26.5
+//   8    512  5 x 1152      80.7 -> 81.0      62.5 -> 56.8         18  256  1 x 1501         43.1 -> 37.7     39.9 -> 34.7
+//   8    64   16 x 704      78.5 -> 73.8      67.8 -> 56.5         22  256  1 x 1750         47.7 -> 44.2 (kept; unshared 47.0 -> 50.6)
+//   8    256  8 x 896       69.1 -> 63.6      54.2 -> 45.7         13  64   1 x 1024         29.9 -> 29.9 (kept)
+//   11   512  4 x 1300      82.6 -> 86.5      64.7 -> 61.1 (kept)  18  64   1 x 1300         34.3 -> 36.9 (kept)
+//   14   512  8 x 1501      155 -> 151 (kept) 22  512  3 x 2048    110 -> 119 (kept)   13  64  8 x 1024  62.9 -> 64.5 (kept)   21  64  4 x 1501  69.5 -> 79.2 (kept)
+// fp16 runs as bf16 does (3 x 777 39.5 -> 31.5, 4 x 1300 84.7 -> 91.1).  Unshared for want of a workspace: 1 x 1300 53.2 -> 43.9, 1 x 2048 with 4 heads 60.3 -> 57.0
+// (e4m3 52.6 -> 42.2, 60.2 -> 56.1).
 bool near_takes_all(const fdb_attn_args* a) {
   if (!has_far_launch(a) || !steps32_supported(a->dtype, a->head_dim) || a->cu_seqlens || a->causal || a->far_splits > 0 || a->near_splits > 0) return false;
   if (a->max_seqlen > 16 * FDB_BM) return false;
   const int radius = a->lut_radius > 0 ? a->lut_radius : 1;
-  const int tiles = (a->max_seqlen + FDB_BN - 1) / FDB_BN, near = (FDB_BM - 1 + radius + FDB_BN - 1) / FDB_BN;   // of the first query tile
-  return tiles - near <= 22;
+  const int at_an_end = (a->max_seqlen + FDB_BN - 1) / FDB_BN - (FDB_BM - 1 + radius + FDB_BN - 1) / FDB_BN;
+  const int near_in_the_middle = (FDB_BM + 2 * radius + 3 * (FDB_BN - 1)) / FDB_BN;
+  return at_an_end <= 8 || (query_tiles(a) * a->heads <= fdb_cu_count() && at_an_end <= near_in_the_middle + 6);
 }
 
 // Workgroups per query tile of the far-only launch.  That launch keeps three workgroups on a CU; when

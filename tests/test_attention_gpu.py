@@ -1782,7 +1782,10 @@ def test_random_fp8_variants(seed):
     if pair:  # far and near keys of a query tile shared out among workgroups, as the library would for few tiles
         kw["far_splits"], kw["near_splits"] = int(r.randint(4)), int(r.randint(4))
         what += " shares %d/%d" % (kw["far_splits"], kw["near_splits"])
-        pair = packed or causal or kw["far_splits"] > 0 or kw["near_splits"] > 0  # left to the library, one near launch takes the far tiles, too
+        # left to the library, one near launch takes the far tiles, too, where they are few (so few query tiles have a compute unit each)
+        radius = ops.delta_lut_host(pb, mr)[1]
+        few = -(-L // 64) - (190 + radius) // 64 <= max(8, (317 + 2 * radius) // 64 + 6)
+        pair = packed or causal or kw["far_splits"] > 0 or kw["near_splits"] > 0 or not few
 
     def reference(sl, batch):
         if not pair:

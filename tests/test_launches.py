@@ -39,12 +39,15 @@ def test_where_the_near_launch_takes_the_far_tiles(dtype):
         (call(1, 576), [("all", 1)]),
         (call(1, 2048, 4, workspace=ALL), [("all", 4), ("merge", 1)]),
         (call(1, 2048, 4), [("all", 1)]),
-        (call(2, 1501), [("all", 1)]),
-        (call(64, 700), [("all", 1)]),
+        (call(64, 1152), [("all", 1)]),                                      # 8 far tiles at an end of the sequence
+        (call(64, 1153), [("far", 1), ("near", 1)]),
+        (call(2, 1152, 14), [("all", 1)]),
+        (call(2, 1280, 12), [("all", 1)]),                                   # 240 query tiles on 256 compute units
+        (call(2, 1300, 12), [("far", 1), ("near", 1)]),                      # 264
         (call(1, 2049), [("far", 1), ("near", 1)]),
         (call(8, 4096), [("far", 1), ("near", 1)]),
-        (call(1, 1600, radius=64), [("all", 1)]),                            # 22 far tiles at the end of the sequence
-        (call(1, 1601, radius=64), [("far", 1), ("near", 1)]),
+        (call(1, 960, radius=64), [("all", 1)]),                             # 12 far tiles at an end, 6 near ones in the middle
+        (call(1, 961, radius=64), [("far", 1), ("near", 1)]),
         (call(1, 1000, causal=1), [("far", 1), ("near", 1)]),
         (call(1, 1000, far_splits=1), [("far", 1), ("near", 1)]),
         (call(1, 1000, near_splits=1), [("far", 1), ("near", 1)]),
@@ -52,6 +55,9 @@ def test_where_the_near_launch_takes_the_far_tiles(dtype):
     ]
     for (_, want), (rc, made) in zip(cases, launches([c for c, _ in cases])):
         assert rc == 0 and _kinds(made) == want, (want, made)
+    (_, whole), = launches([call(1, 1300)], cus=132)
+    (_, short), = launches([call(1, 1300)], cus=131)
+    assert _kinds(whole) == [("all", 1)] and _kinds(short)[0][0] == "far"
 
 
 def _linear(rows, cols, depth, ldo=None, bias=P(0x1000)):
