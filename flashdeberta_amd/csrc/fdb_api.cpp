@@ -430,18 +430,22 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
     return fdb_launch_attn(p, a->dtype, a->head_dim, (int)grid_x, FDB_MODE_NEAR_RING, stream);
   }
   if (launch_mask != 0) return FDB_ERR_UNSUPPORTED;  // a single kernel has no parts
+  const auto launch = [&]() {
+    if (a->dtype == FDB_F32 && a->head_dim == 64 && (a->pos_key || a->pos_query)) return fdb_launch_near_f32(p, (int)grid_x, stream);
+    return fdb_launch_attn(p, a->dtype, a->head_dim, (int)grid_x, FDB_MODE_FUSED, stream);
+  };
   // as many shares of the keys as wanted and as the workspace holds partial results for
   p.key_parts = key_parts_wanted(a);
   const int64_t slots_have = a->workspace ? a->workspace_bytes / far_part_bytes(a) : 0;
   if (p.key_parts > slots_have) p.key_parts = slots_have >= 2 ? (int)slots_have : 1;
   if (p.key_parts <= 1) {
     p.key_parts = 1;
-    return fdb_launch_attn(p, a->dtype, a->head_dim, (int)grid_x, FDB_MODE_FUSED, stream);
+    return launch();
   }
   p.ws_slots = p.key_parts;
   p.ws = (char*)a->workspace;
   p.ws_rows = lse_rows(a);
-  const int rc_attn = fdb_launch_attn(p, a->dtype, a->head_dim, (int)grid_x, FDB_MODE_FUSED, stream);
+  const int rc_attn = launch();
   if (rc_attn != 0) return rc_attn;
   return fdb_launch_merge_parts(p, a->dtype, a->head_dim, stream);
 }

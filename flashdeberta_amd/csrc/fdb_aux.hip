@@ -494,8 +494,11 @@ __global__ __launch_bounds__(256) void fdb_merge_parts_kernel(const FdbKParams p
     w[s] = w[s] != -INFINITY ? __builtin_amdgcn_exp2f(w[s] - m) : 0.f;
     denom += w[s];
   }
-  const float inv = denom > 0.f ? 1.f / denom : 0.f;
-  float acc[4] = {0.f, 0.f, 0.f, 0.f};
+  // a real token sees a key: none above 0 is a row of NaN, or of scores that are all -inf and have no soft-max
+  const float inv = denom > 0.f ? 1.f / denom : __builtin_nanf("");
+  float acc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = denom > 0.f ? 0.f : inv;
 #pragma unroll
   for (int s = 0; s < FDB_MAX_FAR_PARTS; ++s)
     if (s < p.key_parts && w[s] > 0.f) {
@@ -505,7 +508,7 @@ __global__ __launch_bounds__(256) void fdb_merge_parts_kernel(const FdbKParams p
       for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(x[e], f, acc[e]);
     }
   VT::store4(dst, acc[0], acc[1], acc[2], acc[3]);
-  if (cc == 0 && p.lse) p.lse[row] = denom > 0.f ? (m + __builtin_amdgcn_logf(denom)) * 0.6931471805599453f : -INFINITY;
+  if (cc == 0 && p.lse) p.lse[row] = denom > 0.f ? (m + __builtin_amdgcn_logf(denom)) * 0.6931471805599453f : inv;
 }
 
 template <class VT>

@@ -210,6 +210,8 @@ bool fdb_near_supported(int dtype, int head_dim);
 // (16-bit element types, head_dim 64); merges the far partial like the ring mode.
 bool fdb_near32_supported(int dtype, int head_dim);
 int fdb_launch_near32(const FdbKParams& p, int dtype, int grid_x, void* stream);
+// fp32 at head_dim 64 with a position term: every key tile in one launch (p.key_parts shares of them, as in the one-kernel mode).
+int fdb_launch_near_f32(const FdbKParams& p, int grid_x, void* stream);
 // The same pair of launches for OCP e4m3 q / k / K_r / Q_r with bf16 v (head_dim 64): e4m3 MFMA contractions over
 // the whole head_dim for the three score products (fdb_fp8.hip).
 bool fdb_fp8_pair_supported(int dtype, int head_dim);

@@ -1,0 +1,65 @@
+"""The fp32 forward with position terms at head_dim 64 (csrc/fdb_near_f32.hip): around its steps of 32 keys and tiles of 128 queries, far steps on
+either side, shares of the keys, and rows that have no soft-max."""
+import numpy as np
+import pytest
+import torch
+
+from flashdeberta_amd import ops
+from oracle import disentangled_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+BOTH, C2P, P2C = (1, 1), (1, 0), (0, 1)
+
+
+def _inputs(B, L, H, span, terms):
+    g = torch.Generator().manual_seed(B * L)
+    q, k, v = [torch.randn(B, L, H, 64, generator=g) for _ in range(3)]
+    pk, pq = [torch.randn(H, 2 * span, 64, generator=g) if t else None for t in terms]
+    return q, k, v, pk, pq
+
+
+def _oracle(q, k, v, pk, pq, buckets, most, **kw):
+    n = lambda x: None if x is None else x.numpy().astype(np.float64)
+    t = lambda x: n(x).transpose(0, 2, 1, 3)
+    out, lse = O.disentangled_attention(t(q), t(k), t(v), n(pk), n(pq), buckets, most, return_lse=True, **kw)
+    return out.transpose(0, 2, 1, 3), lse.transpose(0, 2, 1)
+
+
+@pytest.mark.parametrize("B,L,buckets,most,terms,causal,shares", [
+    (2, 1, 32, 64, BOTH, False, 0), (1, 31, 32, 64, BOTH, False, 0), (1, 32, 256, 512, BOTH, False, 2), (1, 33, 32, 64, BOTH, True, 0),
+    (1, 97, 32, 64, BOTH, False, 4), (1, 128, 256, 512, C2P, False, 0), (2, 129, 32, 64, P2C, False, 3),
+    (1, 222, 32, 64, BOTH, False, 0), (1, 255, 0, 48, BOTH, True, 0), (1, 511, 32, 64, BOTH, False, 2), (1, 639, 256, 512, BOTH, False, 4),
+    (1, 700, 32, 64, C2P, False, 1), (1, 705, 32, 64, P2C, True, 0), (1, 737, 256, 512, BOTH, False, 1), (1, 1300, 256, 512, BOTH, True, 0)])
+def test_against_the_oracle(B, L, buckets, most, terms, causal, shares):
+    q, k, v, pk, pq = x = _inputs(B, L, 2, ops.att_span(buckets, most), terms)
+    ref, ref_lse = _oracle(*x, buckets, most, causal=causal)
+    out, lse = ops.disentangled_attention_fwd(*[None if t is None else t.cuda() for t in x], position_buckets=buckets, max_relative_positions=most, causal=causal,
+                                              return_lse=True, far_splits=shares)
+    # scores are sums of at most 3 x 64 products of unit normal values: 2^-24 of sums up to about 40 each step, and the same again in the exponent
+    assert np.abs(out.cpu().numpy() - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max())
+    assert np.abs(lse.view(B, L, 2).cpu().numpy() - ref_lse).max() <= 2e-5
+
+
+@pytest.mark.parametrize("shares", [1, 2, 4])
+def test_rows_without_a_soft_max(shares):
+    """A query of NaN, one whose scores are all -inf, and keys whose scores are -inf for every query, a whole share of them."""
+    q, k, v, pk, _ = _inputs(1, 300, 2, 32, C2P)
+    pk[..., 0] = 0.0
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    k[0, :160, :, 0] = -float("inf")
+    q[0, 7] = float("nan")
+    args = dict(position_buckets=32, max_relative_positions=64, far_splits=shares)
+    call = lambda *x: ops.disentangled_attention_fwd(*[t.cuda() for t in x], None, return_lse=True, **args)
+    out, lse = [t.cpu() for t in call(q, k, v, pk)]
+    rows = [i for i in range(300) if i != 7]
+    assert out[0, 7].isnan().all() and lse.view(300, 2)[7].isnan().all()
+    assert out[0, rows].isfinite().all() and lse.view(300, 2)[rows].isfinite().all()
+    seen = [t.clone() for t in (q, k, v)]
+    seen[1][0, :160] = 5.0   # what these keys and values hold otherwise does not count
+    seen[1][0, :160, :, 0] = -float("inf")
+    seen[2][0, :160] = 3.0
+    assert torch.equal(call(*seen, pk)[0].cpu()[0, rows], out[0, rows])
+    k[0, :, :, 0] = -float("inf")
+    out, lse = [t.cpu() for t in call(q, k, v, pk)]
+    assert out.isnan().all() and lse.isnan().all()
