@@ -48,7 +48,7 @@ EXPORTS = (
     "fdb_version", "fdb_attn_args_size", "fdb_strerror", "fdb_attn_check", "fdb_attn_fwd", "fdb_attn_fwd_part", "fdb_attn_fwd_noalloc",
     "fdb_attn_bwd", "fdb_attn_bwd_tables", "fdb_attn_bwd_tables_workspace_bytes", "fdb_attn_bwd_chain", "fdb_attn_bwd_args_size",
     "fdb_attn_workspace_bytes", "fdb_worklist_ints", "fdb_worklist_max_tiles", "fdb_tile_rows", "fdb_build_worklist",
-    "fdb_delta_lut_radius", "fdb_delta_lut", "fdb_delta_lut_window", "fdb_linear", "fdb_gemm", "fdb_gemm_serves", "fdb_gemm_real",
+    "fdb_delta_lut_radius", "fdb_delta_lut", "fdb_delta_lut_window", "fdb_linear", "fdb_layer_small", "fdb_layer_small_serves", "fdb_gemm", "fdb_gemm_serves", "fdb_gemm_real",
     "fdb_gemm_real_cleared", "fdb_gemm_real_serves", "fdb_join", "fdb_dgrad", "fdb_dgrad_serves", "fdb_wgrad", "fdb_wgrad_workspace_bytes",
     "fdb_column_sums", "fdb_column_sums_workspace_bytes", "fdb_mask_bounds", "fdb_quant_e4m3_per_head", "fdb_quant_e4m3_per_head_pair",
     "fdb_dequant_e4m3_per_head",
@@ -109,6 +109,10 @@ def _load():
     lib.fdb_delta_lut.argtypes = [i32, i32, i32, vp]
     lib.fdb_linear.restype = ctypes.c_int
     lib.fdb_linear.argtypes = [vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i32, vp]
+    lib.fdb_layer_small.restype = ctypes.c_int
+    lib.fdb_layer_small.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i64, i64, i64, i64, i64, i64, i32, i32, ctypes.c_float, i32, vp]
+    lib.fdb_layer_small_serves.restype = i32
+    lib.fdb_layer_small_serves.argtypes = [i64, i64, i64, i64]
     lib.fdb_gemm.restype = ctypes.c_int
     lib.fdb_gemm.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i64, i64, i64, i64, i32, i32, vp]
     lib.fdb_gemm_serves.restype = i32

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 LIB = os.path.join(PKG, "libfdb_hip.so")
 NATIVE = os.path.join(PKG, "_native.so")
-SOURCES = ["fdb_api.cpp", "fdb_attn.hip", "fdb_near.hip", "fdb_near_f32.hip", "fdb_fp8.hip", "fdb_aux.hip", "fdb_bwd.hip", "fdb_bwd_ring.hip", "fdb_chain.hip", "fdb_linear.hip", "fdb_gemm.hip", "fdb_grad.hip"]
+SOURCES = ["fdb_api.cpp", "fdb_attn.hip", "fdb_near.hip", "fdb_near_f32.hip", "fdb_small.hip", "fdb_fp8.hip", "fdb_aux.hip", "fdb_bwd.hip", "fdb_bwd_ring.hip", "fdb_chain.hip", "fdb_linear.hip", "fdb_gemm.hip", "fdb_grad.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-x", "hip",

@@ -772,6 +772,26 @@ int fdb_gemm(const void* x, const void* w, const void* bias, const void* residua
   return fdb_launch_gemm(x, w, bias, residual, out, rows, cols, depth, ldx, ldw, ldo, ldr, epilogue, dtype, stream);
 }
 
+int fdb_layer_small(const void* x, const void* w, const void* bias, const void* pos_key, const void* pos_query, void* out, const int32_t* seq_start, const int32_t* seq_len,
+                    const int16_t* delta_lut, int32_t batch, int32_t seqlen, int32_t heads, int32_t depth, int64_t ldx, int64_t ldw, int64_t pk_stride_h,
+                    int64_t pk_stride_r, int64_t pq_stride_h, int64_t pq_stride_r, int32_t att_span, int32_t lut_radius, float sm_scale, int32_t dtype, void* stream) {
+  if (!x || !w || !pos_key || !pos_query || !out) return FDB_ERR_NULL;
+  if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
+  if (batch < 1 || heads < 1 || heads > 65535 || seqlen < 1 || seqlen > 32 || depth < 64 || depth % 64 || ldx < depth || ldw < depth || ldx > (1 << 22) || ldw > (1 << 22) ||
+      (int64_t)batch * heads > INT32_MAX)
+    return FDB_ERR_SHAPE;
+  if (att_span < 1 || lut_radius < 1 || !delta_lut) return FDB_ERR_SPAN;
+  for (const void* t : {x, w, pos_key, pos_query, (const void*)out})
+    if (!aligned16(t)) return FDB_ERR_ALIGN;
+  if (reinterpret_cast<uintptr_t>(bias) & 7u) return FDB_ERR_ALIGN;
+  for (int64_t s : {ldx, ldw, pk_stride_h, pk_stride_r, pq_stride_h, pq_stride_r})
+    if (s % 8) return FDB_ERR_ALIGN;
+  for (int64_t s : {pk_stride_r, pq_stride_r})   // table rows by 24-bit strides and 32-bit offsets, in bytes
+    if (s < 0 || s * 2 >= (1 << 24) || 2 * (int64_t)att_span * s * 2 > INT32_MAX) return FDB_ERR_SHAPE;
+  return fdb_launch_small(x, w, bias, pos_key, pos_query, out, seq_start, seq_len, delta_lut, batch, seqlen, heads, depth, ldx, ldw, pk_stride_h, pk_stride_r, pq_stride_h,
+                          pq_stride_r, lut_radius, sm_scale, dtype, stream);
+}
+
 static int gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* seq_start, const int32_t* seq_len, int32_t batch, int32_t seqlen,
                      int32_t cols, int32_t depth, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int32_t dtype, void* stream) {
   if (!x || !w || !out || !seq_len) return FDB_ERR_NULL;

@@ -229,6 +229,9 @@ int fdb_launch_gemm(const void* x, const void* w, const void* bias, const void* 
                     int64_t ldw, int64_t ldo, int64_t ldr, int epilogue, int dtype, void* stream);  // fdb_gemm.hip
 // The plain product where columns and output rows come by fours only, or the bias lies on any element: for fdb_linear, not an epilogue of fdb_gemm's.
 enum { FDB_GEMM_NARROW = 3 };
+int fdb_launch_small(const void* x, const void* w, const void* bias, const void* pos_key, const void* pos_query, void* out, const int32_t* start, const int32_t* length,
+                     const int16_t* lut, int32_t batch, int32_t seqlen, int32_t heads, int32_t depth, int64_t ldx, int64_t ldw, int64_t pk_sh, int64_t pk_sr, int64_t pq_sh,
+                     int64_t pq_sr, int32_t radius, float sm_scale, int dtype, void* stream);
 int fdb_launch_gemm_real(const void* x, const void* w, const void* bias, void* out, const int32_t* start, const int32_t* length, int32_t batch, int32_t seqlen,
                          int32_t N, int32_t K, int64_t ldx, int64_t ldw, int64_t ldo, bool clear, int dtype, void* stream);
 int fdb_launch_dgrad(const void* x0, int32_t rows0, int32_t depth0, const void* x1, int32_t rows1, int32_t depth1, const void* w, int32_t cols, void* out0,

@@ -765,9 +765,41 @@ struct LayerCall {
   }
 };
 
+// The whole layer in one launch where it is that small (fdb_layer_small); undefined where it is not, or where the tensors are not what that takes.
+Tensor layer_small(const Tensor& hidden, const Tensor& w, const OptTensor& bias, const LayerCall& call) {
+  const auto type = hidden.scalar_type();
+  const Fwd& o = call.o;
+  if (hidden.dim() != 3 || (type != at::kBFloat16 && type != at::kHalf) || !hidden.is_cuda() || !o.pos_key || !o.pos_query) return {};
+  const int64_t B = hidden.size(0), L = hidden.size(1), C = hidden.size(2), H = call.heads, span = att_span(o.buckets, o.max_relative);
+  if (!fdb_layer_small_serves(B, L, H, C) || w.dim() != 2 || w.size(0) != 3 * 64 * H || w.size(1) != C || w.stride(1) != 1 || span < 1 ||
+      (bias && (bias->dim() != 1 || bias->size(0) != w.size(0) || !bias->is_contiguous())))
+    return {};
+  const Tensor* const all[] = {&hidden, &w, bias ? &*bias : &w, &*o.pos_key, &*o.pos_query};
+  for (const Tensor* t : all)
+    if (t->scalar_type() != type || t->device() != hidden.device() || !plain_memory(*t)) return {};
+  const Tensor pk = pos_arg(*o.pos_key, H, 64, span, "pos_key"), pq = pos_arg(*o.pos_query, H, 64, span, "pos_query");
+  const c10::hip::HIPGuard guard(hidden.get_device());
+  const Tensor x = hidden.contiguous(), out = at::empty({B, L, H * 64}, x.options());
+  const Lut& lut = lut_for(o.buckets, o.max_relative, x);
+  std::vector<Tensor> keep;
+  const char* what = "an int32 GPU tensor with one entry per batch row";
+  const int32_t* const start = o.seq_start ? (const int32_t*)vector_arg(*o.seq_start, at::kInt, B, "seq_start", what, keep) : nullptr;
+  const int32_t* const len = o.seq_len ? (const int32_t*)vector_arg(*o.seq_len, at::kInt, B, "seq_len", what, keep) : nullptr;
+  const float scale = (float)(std::isnan(o.sm_scale) ? 1.0 / std::sqrt(64.0 * 3) : o.sm_scale);
+  const int rc = fdb_layer_small(x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr, pk.data_ptr(), pq.data_ptr(), out.data_ptr(), start, len,
+                                 (const int16_t*)lut.table.data_ptr(), (int32_t)B, (int32_t)L, (int32_t)H, (int32_t)C, C, w.stride(0), pk.stride(0), pk.stride(1), pq.stride(0),
+                                 pq.stride(1), (int32_t)span, lut.radius, scale, fdb_dtype_of(type), stream_of(x));
+  if (rc > 0) check(rc, "fdb_layer_small");
+  return rc == 0 ? out : Tensor();   // a negative code: an alignment or a stride it is not built for
+}
+
 // The three input projections as one product over the concatenated weights, and the attention on its columns where they lie.
 Tensor layer_attention(const Tensor& hidden, const Tensor& weight, const OptTensor& bias, const LayerCall& call, bool own) {
   TORCH_CHECK_VALUE(hidden.dim() == 3, "hidden_states must be [B, L, hidden]");
+  if (own) {   // (adds up in another order than the library, like the streamed products)
+    const Tensor done = layer_small(hidden, weight, bias, call);
+    if (done.defined()) return done;
+  }
   const Lengths real{call.o.seq_start, call.o.seq_len};
   const Tensor qkv = project(hidden, weight, bias, own, Then::nothing, nullptr, &real);
   TORCH_CHECK(qkv.is_cuda(), "disentangled_attention_fwd runs on the GPU only; got device ", qkv.device());

@@ -401,6 +401,18 @@ int fdb_gemm_real_cleared(const void* x, const void* w, const void* bias, void* 
 int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t cols, int64_t depth, int64_t ldx);
 
 /*
+ * A whole attention layer of short texts (FDB_BF16 / FDB_F16, head_dim 64, up to 32 tokens): out [batch, seqlen, heads * 64] = the attention of
+ * q | k | v = x [batch * seqlen, depth] . w [3 * heads * 64, depth]^T + bias (or NULL), rounded to the type, with both position terms as fdb_attn_fwd
+ * takes them (seq_start, seq_len likewise; not causal; no log-sum-exps).  Row strides ldx, ldw and the tables' strides in elements; all rows aligned to 16
+ * bytes, bias to 8; depth a multiple of 64.  fdb_layer_small_serves: whether it is the faster way for a size (host, no GPU).  The reference runs
+ * four modules and two kernels (src/flashdeberta/model.py:130-252).
+ */
+int fdb_layer_small(const void* x, const void* w, const void* bias, const void* pos_key, const void* pos_query, void* out, const int32_t* seq_start, const int32_t* seq_len,
+                    const int16_t* delta_lut, int32_t batch, int32_t seqlen, int32_t heads, int32_t depth, int64_t ldx, int64_t ldw, int64_t pk_stride_h,
+                    int64_t pk_stride_r, int64_t pq_stride_h, int64_t pq_stride_r, int32_t att_span, int32_t lut_radius, float sm_scale, int32_t dtype, void* stream);
+int32_t fdb_layer_small_serves(int64_t batch, int64_t seqlen, int64_t heads, int64_t depth);
+
+/*
  * The products of a layer's training backward (FDB_BF16 / FDB_F16; contiguous row-major matrices aligned to 16 bytes, the workspace to 32;
  * depth and all column counts multiples of 64).  Two problems that share weights are one launch each:
  *   fdb_dgrad: out_i [rows_i, cols] = x_i [rows_i, depth_i] . w, the first depth_i rows of w [.., cols] (rows_i 0: none);
