@@ -777,8 +777,8 @@ int fdb_layer_small(const void* x, const void* w, const void* bias, const void* 
                     int64_t pk_stride_r, int64_t pq_stride_h, int64_t pq_stride_r, int32_t att_span, int32_t lut_radius, float sm_scale, int32_t dtype, void* stream) {
   if (!x || !w || !pos_key || !pos_query || !out) return FDB_ERR_NULL;
   if (dtype != FDB_BF16 && dtype != FDB_F16) return FDB_ERR_DTYPE;
-  if (batch < 1 || heads < 1 || heads > 65535 || seqlen < 1 || seqlen > 32 || depth < 64 || depth % 64 || ldx < depth || ldw < depth || ldx > (1 << 22) || ldw > (1 << 22) ||
-      (int64_t)batch * heads > INT32_MAX)
+  if (batch < 1 || heads < 1 || heads > 65535 || seqlen < 1 || seqlen > 128 || depth < 64 || depth % 64 || ldx < depth || ldw < depth || ldx > (1 << 22) || ldw > (1 << 22) ||
+      (int64_t)batch * heads > INT32_MAX || 3 * 64 * (int64_t)heads * ldw * 2 > INT32_MAX)   // a head's rows of w within a lane's 32-bit offset
     return FDB_ERR_SHAPE;
   if (att_span < 1 || lut_radius < 1 || !delta_lut) return FDB_ERR_SPAN;
   for (const void* t : {x, w, pos_key, pos_query, (const void*)out})

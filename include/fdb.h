@@ -401,7 +401,7 @@ int fdb_gemm_real_cleared(const void* x, const void* w, const void* bias, void* 
 int32_t fdb_gemm_real_serves(int64_t batch, int64_t seqlen, int64_t cols, int64_t depth, int64_t ldx);
 
 /*
- * A whole attention layer of short texts (FDB_BF16 / FDB_F16, head_dim 64, up to 32 tokens): out [batch, seqlen, heads * 64] = the attention of
+ * A whole attention layer of short texts (FDB_BF16 / FDB_F16, head_dim 64, up to 128 tokens): out [batch, seqlen, heads * 64] = the attention of
  * q | k | v = x [batch * seqlen, depth] . w [3 * heads * 64, depth]^T + bias (or NULL), rounded to the type, with both position terms as fdb_attn_fwd
  * takes them (seq_start, seq_len likewise; not causal; no log-sum-exps).  Row strides ldx, ldw and the tables' strides in elements; all rows aligned to 16
  * bytes, bias to 8; depth a multiple of 64.  fdb_layer_small_serves: whether it is the faster way for a size (host, no GPU).  The reference runs

@@ -15,8 +15,10 @@ CODE = {torch.bfloat16: _lib.FDB_BF16, torch.float16: _lib.FDB_F16}
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("B,L,H,C,buckets,most,bounds", [
     (1, 1, 1, 64, 256, 512, None), (1, 24, 12, 768, 256, 512, None), (2, 31, 3, 128, 256, 512, None), (3, 32, 2, 192, 32, 64, None), (1, 32, 4, 1024, 0, 20, None),
-    (7, 17, 5, 320, 16, 16, None),   # a table that saturates within the block
-    (5, 32, 2, 256, 256, 512, [(0, 32), (0, 1), (3, 29), (31, 1), (10, 0)]), (4, 9, 3, 64, 32, 64, [(-2, 9), (0, 20), (0, -1), (4, 3)])])
+    (1, 33, 2, 64, 256, 512, None), (2, 64, 3, 128, 32, 64, None), (1, 65, 2, 64, 256, 512, None), (1, 97, 2, 128, 32, 64, None), (2, 128, 2, 256, 256, 512, None),
+    (1, 128, 3, 320, 16, 16, None), (7, 17, 5, 320, 16, 16, None),   # a table that saturates within the block
+    (5, 32, 2, 256, 256, 512, [(0, 32), (0, 1), (3, 29), (31, 1), (10, 0)]), (4, 9, 3, 64, 32, 64, [(-2, 9), (0, 20), (0, -1), (4, 3)]),
+    (5, 60, 2, 192, 256, 512, [(0, 60), (0, 32), (0, 33), (27, 33), (5, -1)]), (6, 120, 2, 64, 32, 64, [(0, 120), (0, 64), (0, 65), (119, 1), (20, 33), (0, 97)])])
 def test_against_64_bits(B, L, H, C, buckets, most, bounds, dtype):
     g = torch.Generator().manual_seed(B * 100 + L)
     rnd = lambda *s, k=1.0: (torch.randn(*s, generator=g) * k).to(dtype)
@@ -52,7 +54,7 @@ def test_against_64_bits(B, L, H, C, buckets, most, bounds, dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("B,L,heads,padded", [(1, 24, 12, False), (4, 32, 12, True), (2, 33, 12, True), (21, 20, 12, True), (22, 20, 12, True), (3, 7, 6, False)])
+@pytest.mark.parametrize("B,L,heads,padded", [(1, 24, 12, False), (4, 32, 12, True), (2, 33, 12, True), (21, 20, 12, True), (22, 20, 12, True), (3, 7, 6, False), (2, 64, 12, True), (5, 100, 6, True), (2, 129, 12, True)])
 def test_layer_with_and_without(B, L, heads, padded):
     """The module's inference on either side of the sizes it takes, against its projections and the operator one by one, also from a graph."""
     from flashdeberta_amd import DebertaV2Config, FlashDisentangledSelfAttention
@@ -82,12 +84,12 @@ def test_layer_with_and_without(B, L, heads, padded):
 def test_where_it_serves():
     serves = _lib.lib.fdb_layer_small_serves
     assert serves(1, 24, 12, 768) and serves(21, 32, 12, 768) and not serves(22, 32, 12, 768)   # a workgroup a compute unit (256)
-    assert not serves(1, 33, 12, 768) and not serves(1, 24, 12, 100) and not serves(0, 24, 12, 768)
+    assert not serves(4, 129, 12, 768) and serves(1, 64, 12, 768) and not serves(3, 128, 12, 768) and serves(4, 97, 12, 768) and not serves(1, 24, 12, 100) and not serves(0, 24, 12, 768)
 
 
 @pytest.mark.parametrize("change,code", [
     (dict(x=0), -1), (dict(w=0), -1), (dict(pk=0), -1), (dict(pq=0), -1), (dict(out=0), -1), (dict(dtype=_lib.FDB_F32), -2), (dict(x=24), -4), (dict(w=40), -4), (dict(bias=52), -4),
-    (dict(pk=72), -4), (dict(out=88), -4), (dict(ldx=68), -4), (dict(pqr=68), -4), (dict(batch=0), -5), (dict(seqlen=33), -5), (dict(seqlen=0), -5), (dict(depth=96), -5), (dict(ldw=56), -5),
+    (dict(pk=72), -4), (dict(out=88), -4), (dict(ldx=68), -4), (dict(pqr=68), -4), (dict(batch=0), -5), (dict(seqlen=129), -5), (dict(seqlen=0), -5), (dict(depth=96), -5), (dict(ldw=56), -5),
     (dict(pkr=-64), -5), (dict(pkr=1 << 23), -5), (dict(pkr=1 << 22, span=1 << 9), -5), (dict(span=0), -6), (dict(lut=0), -6), (dict(radius=0), -6)])
 def test_refused_on_the_host(change, code):
     kw = dict(x=16, w=32, bias=48, pk=64, pq=80, out=96, start=0, length=0, lut=128, batch=2, seqlen=24, heads=2, depth=64, ldx=64, ldw=64, pkh=64, pkr=64, pqh=64, pqr=64, span=32,
