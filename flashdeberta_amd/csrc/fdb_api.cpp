@@ -390,6 +390,7 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
   p.B = a->batch; p.H = a->heads; p.L = a->max_seqlen;
   p.tiles_per_seq = (a->max_seqlen + FDB_BM - 1) / FDB_BM;
   p.groups_together = fdb_groups_together(p.tiles_per_seq);
+  p.by_length = fdb_deals_by_length(p.seq_len, p.B, (int64_t)p.tiles_per_seq * p.B * p.H, fdb_cu_count());
   p.R = a->lut_radius > 0 ? a->lut_radius : 1;
   p.causal = a->causal ? 1 : 0;
   p.scale_log2 = a->sm_scale * 1.4426950408889634f;
@@ -622,6 +623,7 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   p->g_rows = (int32_t)(4 * tiles);
   p->tiles = (int32_t)tiles;
   p->groups_together = fdb_groups_together(p->tiles);
+  p->by_length = fdb_deals_by_length(a->seq_len, p->B, 2 * tiles * pairs, fdb_cu_count());
   // Blocks of 32 relative positions a wave's row block meets: those of its tile's near steps and one more (see Zones)
   const int32_t R = a->lut_radius, n_blk = (a->seqlen + 31) / 32;
   const int32_t most = (FDB_BM - 1 + 2 * R + 2 * 31) / 32 + 1;

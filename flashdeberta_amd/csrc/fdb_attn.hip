@@ -250,8 +250,8 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in scalar registers: what depends on it alone stays scalar
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
-  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr,
-            MODE == kFarOnly ? (p.causal ? kLastFirst : kEdgesFirst) : (MODE == kNearRing ? kMiddleFirst : kNatural), b, tile, h);
+  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr,
+            MODE == kFarOnly ? (p.causal ? kLastFirst : kEdgesFirst) : (MODE == kNearRing ? kMiddleFirst : kNatural), lane, b, tile, h);
 
   int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;

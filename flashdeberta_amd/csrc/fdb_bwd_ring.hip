@@ -110,7 +110,8 @@ __device__ __forceinline__ Zones zones_of(int m0, int Lb, int R, bool causal, bo
 
 // One workgroup of a role, the wg-th of its grid.  STATS: the row statistics are there (fdb_row_stats_kernel); otherwise the dQ role,
 // launched on its own before the other, computes them on its way.
-template <class QT, int ROLE, bool STATS>
+// BY_LENGTH: a padded batch dealt by the lengths of its sequences (an instantiation of its own: its registers cost the other 1 to 3 %).
+template <class QT, int ROLE, bool STATS, bool BY_LENGTH>
 __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg) {
   constexpr bool kDQ = ROLE == 0;
   constexpr int KS = 4, DBLKS = 2;
@@ -122,7 +123,8 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   // near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
   int b, tile_x, h;
-  block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, b, tile_x, h);
+  if constexpr (BY_LENGTH) padded_map(wg, p.seq_start, p.seq_len, p.B, p.H, p.tiles, p.L, lane, b, tile_x, h);
+  else block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, b, tile_x, h);
   const int m0 = tile_x * FDB_BM;
   const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
@@ -684,18 +686,25 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   }
 }
 
-template <class QT, int ROLE>
+template <class QT, int ROLE, bool BY_LENGTH>
 __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdRingParams p) {
-  bwd_ring<QT, ROLE, false>(p, (int)blockIdx.x);
+  bwd_ring<QT, ROLE, false, BY_LENGTH>(p, (int)blockIdx.x);
 }
 
 // Both roles as one launch, the longer one's workgroups first: 2 x 288 workgroups, say, leave half of the GPU's 512 places empty
 // as two launches and fill them as one.
-template <class QT>
+template <class QT, bool BY_LENGTH>
 __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_both_kernel(const FdbBwdRingParams p) {
-  const int n = (int)(gridDim.x >> 1), wg = (int)blockIdx.x;
-  if (wg < n) bwd_ring<QT, 1, true>(p, wg);
-  else bwd_ring<QT, 0, true>(p, wg - n);
+  const int wg = (int)blockIdx.x;
+  if constexpr (BY_LENGTH) {   // both roles of a tile's heads one after the other: the short texts of both end the launch
+    const int pair = wg / (2 * p.H), h = wg - pair * 2 * p.H;
+    if (h < p.H) bwd_ring<QT, 1, true, true>(p, pair * p.H + h);
+    else bwd_ring<QT, 0, true, true>(p, pair * p.H + h - p.H);
+  } else {
+    const int n = (int)(gridDim.x >> 1);
+    if (wg < n) bwd_ring<QT, 1, true, false>(p, wg);
+    else bwd_ring<QT, 0, true, false>(p, wg - n);
+  }
 }
 
 // The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), 128 rows a workgroup, two lanes a row that add up in the dQ
@@ -1040,12 +1049,12 @@ __global__ __launch_bounds__(256) void fdb_table_fold_kernel(const FdbBwdRingPar
 // 4x4096 (1536) 1195 -> 1178; 8x4096 (3072) would go from 2350 to 2395.
 constexpr unsigned kMostTogether = 2048;
 
-template <class QT>
+template <class QT, bool BY_LENGTH>
 int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
-  auto dq = fdb_bwd_ring_kernel<QT, 0>;
-  auto dkv = fdb_bwd_ring_kernel<QT, 1>;
+  auto dq = fdb_bwd_ring_kernel<QT, 0, BY_LENGTH>;
+  auto dkv = fdb_bwd_ring_kernel<QT, 1, BY_LENGTH>;
   auto tg = fdb_table_grad_kernel<QT>;
-  auto both = fdb_bwd_both_kernel<QT>;
+  auto both = fdb_bwd_both_kernel<QT, BY_LENGTH>;
   static std::atomic<uint64_t> set0{0}, set1{0}, set2{0}, set3{0};
   hipError_t e = fdb_set_lds_once((const void*)dq, kLds, set0);
   if (e == hipSuccess) e = fdb_set_lds_once((const void*)dkv, kLds, set1);
@@ -1069,8 +1078,8 @@ int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
 
 int fdb_launch_bwd_ring(const FdbBwdRingParams& p, int dtype, void* stream) {
   switch (dtype) {
-    case FDB_BF16: return launch_all<Bf16Tr>(p, (hipStream_t)stream);
-    case FDB_F16: return launch_all<F16Tr>(p, (hipStream_t)stream);
+    case FDB_BF16: return p.by_length ? launch_all<Bf16Tr, true>(p, (hipStream_t)stream) : launch_all<Bf16Tr, false>(p, (hipStream_t)stream);
+    case FDB_F16: return p.by_length ? launch_all<F16Tr, true>(p, (hipStream_t)stream) : launch_all<F16Tr, false>(p, (hipStream_t)stream);
     default: return FDB_ERR_DTYPE;
   }
 }

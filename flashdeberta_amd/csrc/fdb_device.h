@@ -6,6 +6,8 @@
 
 #include <type_traits>
 
+#include "fdb_kernels.h"
+
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(8))) float f32x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
@@ -298,6 +300,57 @@ __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles
   b_out = __builtin_amdgcn_readfirstlane(b);
   t_out = __builtin_amdgcn_readfirstlane(t);
   h_out = __builtin_amdgcn_readfirstlane(h);
+}
+
+// Linear workgroup id -> (batch row, query tile, head) of a padded batch (host: fdb_deals_by_length).  The dispatcher takes workgroups in order and waits
+// for a place where the next one belongs: a workgroup without tokens among the first leaves a place that stays empty, and one of a long text
+// among the last makes the launch end late.  So the tiles with tokens come first, the highest tile of all sequences before the next lower one and in
+// each the longest sequence first; a launch ends on the shortest texts, and on the tiles of padding, which are only cleared.  All heads of a tile
+// are dealt before the next.  Lengths between a quarter and all of the longest, 12 heads, bf16, us, block_map -> here: near launch 32 x 128 15.2 -> 13.4, 8 x 512 31.2 ->
+// 24.9, 16 x 256 20.2 -> 17.7, 16 x 512 48.0 -> 36.3 (where 52 of 512 places stood empty for 20 us), 64 x 128 24.4 -> 22.3; both roles of the backward 8 x 512 69.2 ->
+// 53.4, 16 x 512 117 -> 99.8, 32 x 128 38.5 -> 37.5.  Every wave finds its place itself, a lane a sequence: how many of the tiles at hand have tokens is a count of lanes,
+// the length of the sequence with a given rank is found bit by bit.
+__device__ __forceinline__ void padded_map(int n, const int32_t* start, const int32_t* length, int batch, int heads, int tiles_per_seq, int most, int lane, int& b_out,
+                                           int& t_out, int& h_out) {
+  int mine = -1;   // this lane's sequence: its tokens
+  if (lane < batch) mine = min(max(length[lane], 0), most - (start ? min(max(start[lane], 0), most) : 0));
+  int u = (int)((uint32_t)n / (uint32_t)heads);
+  const int h = n - u * heads;
+  int t = tiles_per_seq - 1, rank = -1;
+  for (; t >= 0; --t) {
+    const int here = __popcll(__ballot(mine > t * FDB_BM));
+    if (u < here) {
+      rank = u;
+      break;
+    }
+    u -= here;
+  }
+  if (rank < 0) {   // padding
+    for (t = 0; t < tiles_per_seq; ++t) {
+      const int here = __popcll(__ballot(mine > t * FDB_BM));
+      if (u < batch - here) {
+        rank = here + u;
+        break;
+      }
+      u -= batch - here;
+    }
+  }
+  int of = 0;   // the length of that rank: the largest that more than `rank` sequences reach
+  for (int bit = 31 - __builtin_clz(most); bit >= 0; --bit) {
+    const int x = of | (1 << bit);
+    if (__popcll(__ballot(mine >= x)) > rank) of = x;
+  }
+  uint64_t same = __ballot(mine == of);
+  for (int before = rank - __popcll(__ballot(mine > of)); before > 0; --before) same &= same - 1;
+  b_out = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)same) - 1);
+  t_out = __builtin_amdgcn_readfirstlane(t);
+  h_out = __builtin_amdgcn_readfirstlane(h);
+}
+// Where workgroup n belongs: block_map's order, or that of a padded batch.
+template <class Params>
+__device__ __forceinline__ void place_of(int n, const Params& p, int tiles_per_seq, bool fixed, int order, int lane, int& b, int& t, int& h) {
+  if (p.by_length) padded_map(n, p.seq_start, p.seq_len, p.B, p.H, tiles_per_seq, p.L, lane, b, t, h);
+  else block_map(n, p.B, p.H, tiles_per_seq, p.groups_together, fixed, order, b, t, h);
 }
 
 // The 16-bit products by tiles of 16 x 16 outputs, and where they keep a row of 128 bytes in LDS: slot (row, s) holds chunk s ^ swz16(row), so that

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
-  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr, p.causal ? kLastFirst : kEdgesFirst, b, tile, h);
+  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr, p.causal ? kLastFirst : kEdgesFirst, lane, b, tile, h);
 
   int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
-  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr, kMiddleFirst, b, tile, h);
+  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr, kMiddleFirst, lane, b, tile, h);
 
   int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;

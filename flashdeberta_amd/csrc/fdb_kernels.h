@@ -10,6 +10,12 @@
 // (sequence, head) groups whose query tiles are dealt together, see block_map
 inline int32_t fdb_groups_together(int32_t tiles_per_seq) { return 8 * (tiles_per_seq < 96 ? 96 / tiles_per_seq : 1); }
 
+// Whether a padded batch's workgroups are dealt by the lengths of its sequences (padded_map): a lane a sequence, and more workgroups (of all roles) than
+// compute units; fewer have a unit each whatever the order.
+inline bool fdb_deals_by_length(const int32_t* seq_len, int64_t batch, int64_t workgroups, int64_t cus) {
+  return seq_len && batch > 1 && batch <= 64 && workgroups > cus;
+}
+
 struct FdbKParams {
   const char* q;
   const char* k;
@@ -35,6 +41,7 @@ struct FdbKParams {
   int64_t pq_sh, pq_sr;
   int32_t B, H, L, tiles_per_seq;
   int32_t groups_together;  // fdb_groups_together(tiles_per_seq)
+  int32_t by_length;        // fdb_deals_by_length
   int32_t R;        // LUT radius
   int32_t far_done;  // near launches: the far tiles' partial results (far_parts of them) are to be merged
   int32_t near_all;  // near launches: they walk every key tile, no far launch precedes them
@@ -138,6 +145,7 @@ struct FdbBwdRingParams {
                                                             // tg_len row blocks per batch row
   int32_t has_far;
   float scale_log2, sm_scale;
+  int32_t by_length;   // fdb_deals_by_length (last: an argument among the others moves the sixteen-register loads of the rest, and the dQ role spills more)
 };
 int fdb_launch_bwd_ring(const FdbBwdRingParams& p, int dtype, void* stream);
 

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
-  block_map((int)blockIdx.x, p.B, p.H, p.tiles_per_seq, p.groups_together, p.cu == nullptr, kMiddleFirst, b, tile, h);
+  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr, kMiddleFirst, lane, b, tile, h);
 
   int m0, tok0, Lb;
   int64_t qo, ko, vo, oo;
