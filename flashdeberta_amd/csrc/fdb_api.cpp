@@ -654,6 +654,7 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   p->tg_len = (int32_t)((n_blk + chunks - 1) / chunks);
   p->tg_chunks = (int32_t)chunks;
   p->tg_parts = (int32_t)parts;
+  p->tg_items = (int32_t)(a->batch * chunks / parts);
   char* w = (char*)a->workspace;
   int64_t off = 0;
   auto take = [&](int64_t n) {

@@ -748,17 +748,24 @@ __global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingPara
 // and I, picked element by element (sixteen 2-byte LDS reads per lane); everything else is transposing reads and MFMAs, 64 fp32
 // sums per lane kept for the life of the workgroup.  Bound by the reading of G: 1 GB at B = 8, L = 4096, 12 heads.
 // The last group of a head collects the saturated rows' sums per token: two rows (delta(+R), delta(-R)) of each table, weights per token.
-// A wave issues about one instruction per 4.5 clocks and a row block is only eight MFMAs, so the loop is written for few
-// instructions: it is unrolled over the four ring slots of G, which makes every LDS address a lane constant plus an immediate
-// (address arithmetic and remainders per row block had made it 2.5 times as long), and loads run two row blocks ahead.  What wraps
-// from slot 0 to the last one does so by a mask of the address: chosen by comparisons, sixteen of them stayed in scalar
-// registers and the rest of the loop's went to lanes of vector ones (28.2 us where this takes 26.3; B = 8, L = 512, 12 heads).
-constexpr int kGBlk = 2048, kGRing = 4, kKRing = 6;
+// A wave issues about one instruction per 4.5 clocks and a row block is only eight MFMAs (a third of two waves' turn), so the loop is
+// written for few instructions: it is unrolled over the four ring slots of G, which makes every LDS address a lane constant plus an
+// immediate; what 32 turns need to know of G's blocks (which there are, where they lie) is worked out at once, a row block per lane, and
+// is then one bit and one value read from a lane; rows are clamped in vector registers, without a branch.  190 -> 118 instructions a turn, of
+// which 90 scalar ones were found to be more than half of what the waves issued (and 89 -> 16 scalar registers spilled to lanes):
+// 12 heads, us, 8 x 512 padded 25.3 -> 19.4, 2 x 1501 31.8 -> 26.6, 8 x 4096 270 -> 260.  Loads run two row blocks ahead.  No faster: eight
+// waves, half of them for either table, which doubles the scalar instructions (25.3 -> 26.5), and the operands asked for ahead of the next loads.
+// A launch without divisions and scalar loads ahead of each sequence: 19.4 -> 17.4 and 26.6 -> 25.8.  What is left beside the turns (0.33 us
+// for two workgroups of a CU) is the writing of the shares' sums, 25 MB of them.
+constexpr int kGBlk = 2048, kGRing = 4, kKRing = 8;
 constexpr int kTgOffK = kGRing * kTile, kTgOffG = kTgOffK + kKRing * kTile, kTgLds = kTgOffG + 4 * kGRing * kGBlk;
 static_assert(kTgLds <= 80 * 1024, "two workgroups per CU");
 static_assert(kTgOffG % (kGRing * kGBlk) == 0, "a wave's ring of G wraps by a mask of its address");
 
-template <class QT>
+// BY_LENGTH (a padded batch of up to 64 sequences): a part takes an equal share of the row blocks that hold tokens, wherever in a sequence that
+// begins and ends, instead of chunks of the batch's rows, of which one part may have twice as many with tokens as another (8 x 512, lengths of 148 to
+// 512, 28 row blocks in the longest of four parts: 26.2 -> 25.3 us with what follows as it was).
+template <class QT, bool BY_LENGTH>
 __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBwdRingParams p) {
   using frag = typename QT::frag;
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -766,13 +773,44 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  const int h = (int)blockIdx.x % p.H, part = (int)blockIdx.x / p.H, group = p.tg_groups - (int)blockIdx.y - (p.has_far ? 0 : 1);  // the saturated rows first
-  // this part's items: (batch row, chunk of row blocks)
-  const int items = p.B * p.tg_chunks;
-  const int it0 = (int)((int64_t)items * part / p.tg_parts), it1 = (int)((int64_t)items * (part + 1) / p.tg_parts);
+  const int h = (int)blockIdx.x, part = (int)blockIdx.y, group = p.tg_groups - (int)blockIdx.z - (p.has_far ? 0 : 1);  // the saturated rows first
+  // this part's items: (batch row, chunk of row blocks), as many as any other's
+  int it0 = part * p.tg_items, it1 = it0 + p.tg_items;
+  int first = 0, len = 0, before = 0, lo = 0, hi = 0;   // BY_LENGTH: this lane's sequence and the row blocks ahead of it; this part's of all
+  if constexpr (BY_LENGTH) {
+    if (lane < p.B) {
+      if (p.seq_start) first = min(max(p.seq_start[lane], 0), p.L);
+      len = min(max(p.seq_len[lane], 0), p.L - first);
+    }
+    const int blocks = (len + 31) / 32;
+    before = blocks;
+#pragma unroll
+    for (int x = 1; x < 64; x <<= 1) {
+      const int other = __shfl_up(before, x);
+      before += lane >= x ? other : 0;
+    }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(before, 63), share = (total + (uint32_t)p.tg_parts - 1) / (uint32_t)p.tg_parts;
+    lo = (int)min(total, share * (uint32_t)part), hi = (int)min(total, lo + share);
+    it0 = __popcll(__ballot(lane < p.B && before <= lo));   // sequences that end ahead of it
+    before -= blocks;
+    it1 = __popcll(__ballot(lane < p.B && before < hi));
+  }
+  // the row blocks [I0, I1) of sequence b that are the item's
+  auto item = [&](int it, int n_rows, int& I0, int& I1) __attribute__((always_inline)) {
+    if constexpr (BY_LENGTH) {
+      const int ahead = __builtin_amdgcn_readlane(before, it);
+      I0 = max(0, lo - ahead), I1 = min(n_rows, hi - ahead);
+    } else {
+      I0 = (int)((uint32_t)it % (uint32_t)p.tg_chunks) * p.tg_len, I1 = min(n_rows, I0 + p.tg_len);
+    }
+  };
   auto seq_of = [&](int b, int& tok0, int& Lb) __attribute__((always_inline)) {
-    tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
-    Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
+    if constexpr (BY_LENGTH) {
+      tok0 = __builtin_amdgcn_readlane(first, b), Lb = __builtin_amdgcn_readlane(len, b);
+    } else {
+      tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
+      Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
+    }
   };
   if (group == p.tg_groups) {
     // the saturated rows: a wave takes eight rows at a time, sixteen bytes of a row per lane
@@ -781,16 +819,17 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     for (int t = 0; t < 4; ++t) acc[t >> 1][t & 1] = f32x8{0, 0, 0, 0, 0, 0, 0, 0};
     const int r8 = lane >> 3, c8 = lane & 7;
     for (int it = it0; it < it1; ++it) {
-      const int b = it / p.tg_chunks, c = it % p.tg_chunks;
-      int tok0, Lb;
+      const int b = BY_LENGTH ? it : (int)((uint32_t)it / (uint32_t)p.tg_chunks);
+      int tok0, Lb, I0, I1;
       seq_of(b, tok0, Lb);
-      const int i1 = min(Lb, (c + 1) * p.tg_len * 32);
+      item(it, (Lb + 31) / 32, I0, I1);
+      const int i1 = min(Lb, I1 * 32);
       const char* qr = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh + 8 * c8) * 2;
       const char* kr = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh + 8 * c8) * 2;
       const float* fq = p.far_q + ((int64_t)b * p.H + h) * 2 * p.stat_len;
       const float* fk = p.far_k + ((int64_t)b * p.H + h) * 2 * p.stat_len;
 #pragma unroll 4
-      for (int i = c * p.tg_len * 32 + 8 * wave + r8; i < i1; i += 32) {
+      for (int i = I0 * 32 + 8 * wave + r8; i < i1; i += 32) {
         const f32x8 q = QT::to_f32(QT::load(qr + (int64_t)i * p.q_st * 2)), k = QT::to_f32(QT::load(kr + (int64_t)i * p.k_st * 2));
         acc[0][0] += fq[i] * q;
         acc[0][1] += fq[p.stat_len + i] * q;
@@ -829,92 +868,93 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     for (int x = 0; x < 2; ++x) gt[x] = (uint32_t)((8 * x + 4 * (grp >> 1) + (s16 >> 2)) * 64 + (16 * (grp & 1) + 4 * (s16 & 3)) * 2);
   }
   const uint32_t g_base = lds0 + kTgOffG + (uint32_t)wave * (kGRing * kGBlk);
-  auto trans = [&](uint32_t tile, int c, int d) __attribute__((always_inline)) {
-    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(yt[2 * d] + tile + 2048 * c));
-    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(yt[2 * d + 1] + tile + 2048 * c + 1024));
+  auto pair = [&](uint32_t lo_at, uint32_t hi_at) __attribute__((always_inline)) {
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)lo_at);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)hi_at);
     return __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
   const int R = (int)own_sgpr((uint32_t)p.R);
   const bool causal = p.causal != 0;
   const char* const zeros = own_sgpr((const char*)p.zero_block);
   const uint32_t q_rowb = own_sgpr((uint32_t)(p.q_st * 2)), k_rowb = own_sgpr((uint32_t)(p.k_st * 2)), g_step = own_sgpr((uint32_t)(p.g_slots * kGBlk));
-  const uint32_t q_lane = (uint32_t)srow * q_rowb + chunk_off, k_lane = (uint32_t)srow * k_rowb + chunk_off;
   const uint32_t u_lane = g_base + (uint32_t)(li * 66 + g * 256);   // G element (row 4 g + li, column li) of ring slot 0
   for (int it = it0; it < it1; ++it) {
-    const int b = it / p.tg_chunks, c0 = it % p.tg_chunks;
-    int tok0, Lb;
+    const int b = BY_LENGTH ? it : (int)((uint32_t)it / (uint32_t)p.tg_chunks);
+    int tok0, Lb, I0, I1;
     seq_of(b, tok0, Lb);
     const int n_rows = (Lb + 31) / 32;                       // row blocks of this sequence
-    const int I0 = c0 * p.tg_len, I1 = min(n_rows, I0 + p.tg_len);
-    if (I0 >= I1) continue;
-    const int full = Lb / 32;                                // those of 32 rows
+    item(it, n_rows, I0, I1);
     const int rho0 = p.rho_min + 4 * group;
-    // What is fetched next: row block I of q and of G, row block J = I - 1 - rho0 of k (the wave w = 0 uses the newest).  The places in
-    // memory and the zones of I's tile are carried along: computed per row block they were two thirds of a turn's instructions.
-    int I = I0, J = I0 - 1 - rho0;
-    const uint64_t q_step = (uint64_t)q_rowb * 32, k_step = (uint64_t)k_rowb * 32;
-    const char* const q_rows = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2;
-    const char* const k_rows = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2;
-    uint64_t q_at = (uint64_t)(uintptr_t)q_rows + (uint64_t)(uint32_t)I * q_step, k_at = (uint64_t)(uintptr_t)k_rows + (uint64_t)((int64_t)J * (int64_t)k_step);
-    uint64_t g_at = (uint64_t)(uintptr_t)p.g_blocks + (uint64_t)(((int64_t)b * p.H + h) * p.g_rows + I) * g_step;
-    int z0 = 0, zn = -1;   // first near step of the tile, number of near steps or -1
-    auto zone_at = [&](int row_block) __attribute__((always_inline)) {
-      const Zones z = zones_of(row_block / 4 * FDB_BM, Lb, R, causal, true);
-      z0 = z.s0;
-      zn = z.s1 > z.s0 ? z.s1 - z.s0 : -1;
+    // block (I, rho) can only be there with a row block of k at I - rho, or one past the last: the turns outside do nothing
+    const bool lead = I0 <= max(rho0, 0);                    // no item before has a turn: the key rows ahead of the first row block are this one's as well
+    I0 = max(I0, rho0), I1 = min(I1, n_rows + rho0 + 4);
+    if (I0 >= I1) continue;
+    const int last = I1 - I0;   // one more turn than row blocks: the last block's rows of k that precede it
+    const char* const q_rows = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2 + chunk_off;
+    const char* const k_rows = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2 + chunk_off;
+    // What the turns n0 .. n0 + 31 and the loads they ask for have to know of G, a row block n = n0 - 1 + lane per lane: where block (I0 + n, rho)
+    // begins in its row, and which of them there are (a near step the dQ launch met, inside the sequence), go into which table's products.
+    int n0 = 0;
+    uint32_t g_off = 0;
+    uint64_t there = 0, for_k = 0, for_q = 0;
+    auto window = [&](int n) __attribute__((always_inline)) {
+      n0 = n;
+      const int row_block = I0 + n - 1 + lane;
+      const Zones z = zones_of(max(row_block, 0) / 4 * FDB_BM, Lb, R, causal, true);
+      const int at = row_block - rho - z.s0;
+      const bool is = (uint32_t)row_block < (uint32_t)n_rows && at >= 0 && z.s1 > z.s0 && at <= z.s1 - z.s0;
+      g_off = is ? (uint32_t)at * kGBlk : 0;
+      there = __ballot(is);
+      const bool mine = n - 1 + lane < last;
+      for_k = there & __ballot(mine);
+      for_q = there | there << 1;
+      if (n == 0 && !lead) for_q &= ~2ull;
     };
-    auto clamped_dma = [&](const char* rows, uint32_t rowb, int blk, uint32_t dst) __attribute__((always_inline)) {
-      const int row = max(0, min(blk * 32 + srow, Lb - 1));   // rows outside the sequence: finite values that meet zeros
-      dma16n(rows + (uint64_t)(uint32_t)row * rowb + chunk_off, dst + wave_kb);
+    // What is fetched next: row block I of q and of G, row block I - 1 - rho0 of k (the wave w = 0 uses the newest).  Rows outside the sequence
+    // are finite values that meet zeros in G.
+    int q_row = I0 * 32 + srow, k_row = (I0 - 1 - rho0) * 32 + srow;
+    uint64_t g_at = (uint64_t)(uintptr_t)p.g_blocks + (uint64_t)(((int64_t)b * p.H + h) * p.g_rows + I0 - 1) * g_step;
+    uint32_t k_to = 0, k_from = (uint32_t)(-wave & (kKRing - 1)) * kTile;   // ring places of k: the next load's, this wave's rows
+    auto rows_dma = [&](const char* rows, uint32_t rowb, int row, uint32_t dst) __attribute__((always_inline)) {
+      dma16n(rows + (uint64_t)(uint32_t)max(0, min(row, Lb - 1)) * rowb, dst + wave_kb);
     };
-    // block (I, rho) into a ring slot; a block of zeros where the dQ launch met no such block (no near step, or outside the
-    // sequence).  Returns whether there is one.
-    auto g_dma = [&](int row_block, uint64_t at, uint32_t ring) __attribute__((always_inline)) {
-      const int k = row_block - rho - z0;
-      const bool there = (uint32_t)row_block < (uint32_t)n_rows && k >= 0 && k <= zn;
-      const char* src = there ? (const char*)(uintptr_t)(at + (uint64_t)((int64_t)k * kGBlk)) : zeros;
-      dma16sn(src, lane * 16, g_base + ring * kGBlk);
-      dma16sn(src + 1024, lane * 16, g_base + ring * kGBlk + 1024);
-      return there;
+    auto g_dma = [&](int j, uint32_t ring) __attribute__((always_inline)) {   // block n0 - 1 + j; zeros where there is none
+      const uint64_t at = g_at + (uint32_t)__builtin_amdgcn_readlane(g_off, j);
+      dma16sn_pair((there >> j) & 1 ? (const char*)(uintptr_t)at : zeros, lane * 16, g_base + ring * kGBlk);
+      g_at += g_step;
+    };
+    auto fetch = [&](int j, uint32_t ring) __attribute__((always_inline)) {   // what row block n0 - 1 + j needs first, four loads per wave
+      rows_dma(q_rows, q_rowb, q_row, ring * kTile);
+      rows_dma(k_rows, k_rowb, k_row, kTgOffK + k_to);
+      g_dma(j, ring);
+      q_row += 32, k_row += 32;
+      k_to = (k_to + kTile) & (kKRing * kTile - 1);
     };
     __syncthreads();   // the item before is done with the rings
-    for (int w = 1; w < 4; ++w) {
-      const int blk = J - w;
-      const uint32_t dst = kTgOffK + (uint32_t)(kKRing - w) * kTile;
-      if ((uint32_t)blk < (uint32_t)full) dma16sn(k_rows + (uint64_t)(uint32_t)blk * k_step, k_lane, dst + wave_kb);
-      else clamped_dma(k_rows, k_rowb, blk, dst);
-    }
-    zone_at(max(I - 1, 0));
-    bool prev = g_dma(I - 1, g_at - g_step, kGRing - 1);
-    auto fetch = [&](uint32_t ring, uint32_t kslot) __attribute__((always_inline)) {   // what the next row block needs first, four loads per wave
-      if (I < full) dma16sn((const char*)(uintptr_t)q_at, q_lane, ring * kTile + wave_kb);
-      else clamped_dma(q_rows, q_rowb, I, ring * kTile);
-      if ((uint32_t)J < (uint32_t)full) dma16sn((const char*)(uintptr_t)k_at, k_lane, kTgOffK + kslot * kTile + wave_kb);
-      else clamped_dma(k_rows, k_rowb, J, kTgOffK + kslot * kTile);
-      if ((I & 3) == 0) zone_at(I);
-      const bool there = g_dma(I, g_at, ring);
-      ++I, ++J;
-      q_at += q_step, k_at += k_step, g_at += g_step;
-      return there;
-    };
-    bool cur = fetch(0, 0), next = fetch(1, 1);
-    int kread = wave == 0 ? 0 : kKRing - wave, kfill = 2;   // ring slots of k: this wave's rows, and where the next ones go
-    auto turn = [&](auto slot_tag, int n) __attribute__((always_inline)) {
+    for (int w = 1; w < 4; ++w) rows_dma(k_rows, k_rowb, k_row - 32 * w, kTgOffK + (uint32_t)(kKRing - w) * kTile);
+    window(0);
+    g_dma(0, kGRing - 1);
+    fetch(1, 0);
+    fetch(2, 1);
+    auto turn = [&](auto slot_tag, int j) __attribute__((always_inline)) {   // row block n = n0 - 1 + j
       constexpr int RING = decltype(slot_tag)::value, PREV = (RING + kGRing - 1) % kGRing;
       wait_vmcnt<4>();   // this row block's loads have landed, those of the next one may still fly
       __syncthreads();
-      const bool after = fetch((RING + 2) % kGRing, (uint32_t)kfill);
-      const bool for_k = cur && n < I1 - I0, for_q = (prev || cur) && (n > 0 || I0 == 0);
-      if (for_k || for_q) {   // the operands of both tables' products are requested before the first product waits for one
+      fetch(j + 2, (RING + 2) % kGRing);
+      const bool now_k = (for_k >> j) & 1, now_q = (for_q >> j) & 1;
+      if (now_k || now_q) {   // the operands of both tables' products are requested before the first product waits for one
         frag gk[2], gq[2], tq[2][2], tk[2][2];
-        const uint32_t kt = kTgOffK + (uint32_t)kread * kTile;
+        uint32_t kt[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          kt[x] = yt[x] + k_from;
+          asm("" : "+v"(kt[x]));   // the constant part of the address belongs into the instruction
+        }
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(g_base + gt[0] + RING * kGBlk + 1024 * c));
-          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS s16x4*)(uintptr_t)(g_base + gt[1] + RING * kGBlk + 1024 * c));
-          gk[c] = __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+          gk[c] = pair(g_base + gt[0] + RING * kGBlk + 1024 * c, g_base + gt[1] + RING * kGBlk + 1024 * c);
 #pragma unroll
-          for (int d = 0; d < 2; ++d) tq[c][d] = trans(RING * kTile, c, d);
+          for (int d = 0; d < 2; ++d) tq[c][d] = pair(yt[2 * d] + RING * kTile + 2048 * c, yt[2 * d + 1] + RING * kTile + 2048 * c + 1024);
         }
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
@@ -929,40 +969,39 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
           }
           gq[c] = __builtin_bit_cast(frag, a);
 #pragma unroll
-          for (int d = 0; d < 2; ++d) tk[c][d] = trans(kt, c, d);
+          for (int d = 0; d < 2; ++d) tk[c][d] = pair(kt[2 * d] + kTgOffK + 2048 * c, kt[2 * d + 1] + kTgOffK + 2048 * c + 1024);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (for_k) {
+        if (now_k) {
 #pragma unroll
           for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int d = 0; d < 2; ++d) ek[d] = QT::mma(gk[c], tq[c][d], ek[d]);
         }
-        if (for_q) {
+        if (now_q) {
 #pragma unroll
           for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int d = 0; d < 2; ++d) eq[d] = QT::mma(gq[c], tk[c][d], eq[d]);
         }
       }
-      prev = cur;
-      cur = next;
-      next = after;
-      kread = kread == kKRing - 1 ? 0 : kread + 1;
-      kfill = kfill == kKRing - 1 ? 0 : kfill + 1;
+      k_from = (k_from + kTile) & (kKRing * kTile - 1);
     };
-    const int last = I1 - I0;   // one more turn than row blocks: the last block's rows of k that precede it
     int n = 0;
 #pragma unroll 1
-    for (; n + 3 <= last; n += 4) {
-      turn(std::integral_constant<int, 0>{}, n);
-      turn(std::integral_constant<int, 1>{}, n + 1);
-      turn(std::integral_constant<int, 2>{}, n + 2);
-      turn(std::integral_constant<int, 3>{}, n + 3);
+    for (;;) {
+      if (n - n0 == 32) window(n);
+      const int j = n - n0 + 1;
+      if (n + 3 > last) break;
+      turn(std::integral_constant<int, 0>{}, j);
+      turn(std::integral_constant<int, 1>{}, j + 1);
+      turn(std::integral_constant<int, 2>{}, j + 2);
+      turn(std::integral_constant<int, 3>{}, j + 3);
+      n += 4;
     }
-    if (n <= last) turn(std::integral_constant<int, 0>{}, n);
-    if (n + 1 <= last) turn(std::integral_constant<int, 1>{}, n + 1);
-    if (n + 2 <= last) turn(std::integral_constant<int, 2>{}, n + 2);
+    if (n <= last) turn(std::integral_constant<int, 0>{}, n - n0 + 1);
+    if (n + 1 <= last) turn(std::integral_constant<int, 1>{}, n - n0 + 2);
+    if (n + 2 <= last) turn(std::integral_constant<int, 2>{}, n - n0 + 3);
     wait_vmcnt<0>();
   }
   // [part][head][rho][table][position][d]
@@ -1053,7 +1092,7 @@ template <class QT, bool BY_LENGTH>
 int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
   auto dq = fdb_bwd_ring_kernel<QT, 0, BY_LENGTH>;
   auto dkv = fdb_bwd_ring_kernel<QT, 1, BY_LENGTH>;
-  auto tg = fdb_table_grad_kernel<QT>;
+  auto tg = fdb_table_grad_kernel<QT, BY_LENGTH>;
   auto both = fdb_bwd_both_kernel<QT, BY_LENGTH>;
   static std::atomic<uint64_t> set0{0}, set1{0}, set2{0}, set3{0};
   hipError_t e = fdb_set_lds_once((const void*)dq, kLds, set0);
@@ -1069,7 +1108,7 @@ int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
     hipLaunchKernelGGL(dq, dim3(grid), dim3(kThreads), kLds, stream, p);
     hipLaunchKernelGGL(dkv, dim3(grid), dim3(kThreads), kLds, stream, p);
   }
-  hipLaunchKernelGGL(tg, dim3((unsigned)(p.H * p.tg_parts), (unsigned)(p.tg_groups + (p.has_far ? 1 : 0))), dim3(kThreads), kTgLds, stream, p);
+  hipLaunchKernelGGL(tg, dim3((unsigned)p.H, (unsigned)p.tg_parts, (unsigned)(p.tg_groups + (p.has_far ? 1 : 0))), dim3(kThreads), kTgLds, stream, p);
   hipLaunchKernelGGL(fdb_table_fold_kernel<QT>, dim3((unsigned)((2 * p.S + kFoldRows - 1) / kFoldRows), (unsigned)p.H, 2), dim3(256), 0, stream, p);
   return (int)hipGetLastError();
 }

@@ -421,6 +421,14 @@ __device__ __forceinline__ void dma16sn(const void* base, uint32_t lane_off, uin
   const uint64_t sb = ((uint64_t)bhi << 32) | blo;
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(sb), "s"(lb) : "memory");
 }
+// Two loads 1024 bytes apart on both sides (the instruction's offset counts for both addresses).
+__device__ __forceinline__ void dma16sn_pair(const void* base, uint32_t lane_off, uint32_t lds_base) {
+  const uint32_t lb = __builtin_amdgcn_readfirstlane(lds_base);
+  const uint64_t b64 = (uint64_t)(uintptr_t)base;
+  const uint32_t blo = __builtin_amdgcn_readfirstlane((uint32_t)b64), bhi = __builtin_amdgcn_readfirstlane((uint32_t)(b64 >> 32));
+  const uint64_t sb = ((uint64_t)bhi << 32) | blo;
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n\tglobal_load_lds_dwordx4 %0, %1 offset:1024" : : "v"(lane_off), "s"(sb), "s"(lb) : "memory");
+}
 
 // Wait until at most N vector-memory loads of this wave are outstanding (loads complete in issue
 // order).  Issued through the builtin rather than asm, so that the compiler's own count of its

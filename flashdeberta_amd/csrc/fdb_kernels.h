@@ -146,6 +146,7 @@ struct FdbBwdRingParams {
   int32_t has_far;
   float scale_log2, sm_scale;
   int32_t by_length;   // fdb_deals_by_length (last: an argument among the others moves the sixteen-register loads of the rest, and the dQ role spills more)
+  int32_t tg_items;    // chunks a share takes
 };
 int fdb_launch_bwd_ring(const FdbBwdRingParams& p, int dtype, void* stream);
 

@@ -207,3 +207,35 @@ def test_node_replays_from_a_graph_and_through_saved_tensor_hooks():
         graph.replay()
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(captured, ref))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,H,rows", [
+    (1, 1100, 26, None),                                   # one share of more row blocks than the tables of what is there hold (32 turns)
+    (1, 2300, 12, None),                                   # several such shares, the last of them shorter
+    (2, 2300, 12, [(9, 2222), (0, 71)]),                   # shares of equal numbers of row blocks
+    (7, 700, 12, [(0, 700), (0, 0), (699, 1), (0, 33), (100, 600), (0, 320), (37, 511)]),   # shares that begin and end inside sequences
+    (64, 130, 6, [(n % 5, 2 * n) for n in range(64)]),
+])
+def test_table_gradients_of_any_share(B, L, H, rows):
+    """The tables' gradients of all heads in one call, few and large shares of the tokens, against one call a head, many and small ones: both round the same
+    sums to the type once, so they differ by its epsilon at most, and by the order of the fp32 sums."""
+    dtype = torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(L + H)
+    q, k, v, dout = [torch.randn(B, L, H, 64, device="cuda", generator=g).to(dtype) for _ in range(4)]
+    pk, pq = [torch.randn(H, 512, 64, device="cuda", generator=g).to(dtype) for _ in range(2)]
+    kw = dict(position_buckets=256, max_relative_positions=512)
+    if rows:
+        kw["seq_start"], kw["seq_len"] = [torch.tensor(x, dtype=torch.int32).cuda() for x in zip(*rows)]
+    out, lse = ops.disentangled_attention_fwd(q, k, v, pk, pq, return_lse=True, **kw)
+    got = ops.disentangled_attention_bwd(q, k, v, out, lse, dout, pk, pq, **kw)[3:]
+    ref = [torch.zeros_like(pk), torch.zeros_like(pq)]
+    for h in range(H):
+        one = [x[:, :, h:h + 1].contiguous() for x in (q, k, v, out)] + [lse[:, h:h + 1].contiguous(), dout[:, :, h:h + 1].contiguous()]
+        for r, x in zip(ref, ops.disentangled_attention_bwd(*one, pk[h:h + 1], pq[h:h + 1], **kw)[3:]):
+            r[h:h + 1] = x
+    eps = torch.finfo(dtype).eps
+    for a, r in zip(got, ref):
+        a, r = a.double(), r.double()
+        off = (a - r).abs() - eps * r.abs()
+        assert float(off.max()) <= 2.0 ** -24 * L * float(r.abs().max()), "%.3e of %.3e" % (float(off.max()), float(r.abs().max()))
