@@ -241,7 +241,7 @@ __global__ __launch_bounds__(64 * WShape::NW, 2) void fdb_wgrad_kernel(const Wgr
 #pragma unroll
     for (int j = 0; j < S::FN; ++j) ylane[j][h] = lds0 + (uint32_t)(S::TM / 64 + ((wn * S::FN + j) >> 2)) * kPanel + tr_lane(lane, wn * S::FN + j, h);
   }
-  auto multiply = [&](auto ragged, uint32_t at, int rows) __attribute__((always_inline)) {
+  auto multiply = [&](uint32_t at) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       frag xf[S::FM], yf[S::FN];
@@ -249,17 +249,6 @@ __global__ __launch_bounds__(64 * WShape::NW, 2) void fdb_wgrad_kernel(const Wgr
       for (int i = 0; i < S::FM; ++i) xf[i] = tr_frag<QT>(at + xlane[i][0], at + xlane[i][1], s * 32 * kRow);
 #pragma unroll
       for (int j = 0; j < S::FN; ++j) yf[j] = tr_frag<QT>(at + ylane[j][0], at + ylane[j][1], s * 32 * kRow);
-      if constexpr (decltype(ragged)::value) {   // rows past the last one: zeros on both sides, whatever the row they re-read holds
-        const elem zero = (elem)0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bool real = 32 * s + 8 * kg + e < rows;
-#pragma unroll
-          for (int i = 0; i < S::FM; ++i) xf[i][e] = real ? xf[i][e] : zero;
-#pragma unroll
-          for (int j = 0; j < S::FN; ++j) yf[j][e] = real ? yf[j][e] : zero;
-        }
-      }
 #pragma unroll
       for (int i = 0; i < S::FM; ++i)
 #pragma unroll
@@ -282,8 +271,12 @@ __global__ __launch_bounds__(64 * WShape::NW, 2) void fdb_wgrad_kernel(const Wgr
     if (t + S::STAGES - 1 < t1) fill(buf == 0 ? S::STAGES - 1 : buf - 1);
     __builtin_amdgcn_sched_barrier(0);
     const int real = t < first ? rows0 - t * kDepth : rows1 - (t - first) * kDepth;
-    if (real >= kDepth) multiply(std::false_type{}, (uint32_t)buf * S::STAGE, kDepth);
-    else multiply(std::true_type{}, (uint32_t)buf * S::STAGE, real);
+    if (real < kDepth) {   // rows past the last one: zeros on both sides, whatever the row they re-read holds
+      for (int c = tid; c < (S::TM + S::TN) / 64 * kDepth * 8; c += 64 * S::NW)
+        if (((c >> 3) & (kDepth - 1)) >= real) *(u32x4*)(smem + buf * S::STAGE + c * 16) = u32x4{0u, 0u, 0u, 0u};
+      __syncthreads();
+    }
+    multiply((uint32_t)buf * S::STAGE);
     buf = buf == S::STAGES - 1 ? 0 : buf + 1;
   }
   // the result by way of the LDS, in whole rows of the tile
