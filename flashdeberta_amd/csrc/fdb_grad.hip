@@ -5,7 +5,7 @@
 //   d W = d qkv^T . hidden + [d pos^T . rel] on the rows of q and k, one contraction over tokens and table rows, and d b, the column sums of
 //   d qkv and d pos, from the tiles as they pass (a product with ones).
 // 8 x 512 tokens, 12 heads, bf16, against a library product each (the second weight product onto the first one's rounded result) and two
-// launches for the column sums: 35.9 -> 21.1 us and 52.9 -> 31.2; 1000 tokens 23.9 -> 17.0 and 33.5 -> 23.3.
+// launches for the column sums: 35.9 -> 21.1 us and 52.9 -> 29; 1000 tokens 23.9 -> 14.5 and 33.5 -> 23.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -48,22 +48,20 @@ struct DgradParams {
   char* out[2];
   int32_t rows[2], depth[2], tiles[2], cols, tiles_n;
 };
-template <int ROWS>
+template <int ROWS, int WM_, int WN_, int STAGES_, int PER_CU_>
 struct DShape {
-  static constexpr int TM = ROWS, TN = 128, STAGES = ROWS == 64 ? 3 : 2, FM = TM / 32, FN = 4, NW = 4, PITCH = TN * 2 + 16;
+  static constexpr int TM = ROWS, TN = 128, WM = WM_, WN = WN_, NW = WM * WN, STAGES = STAGES_, PER_CU = PER_CU_, FM = TM / WM / 16, FN = TN / WN / 16, PITCH = TN * 2 + 16;
   static constexpr int STAGE = TM * kRow + TN / 64 * kPanel, LOADS = STAGE / 1024 / NW, XLOADS = TM / 8 / NW;
   static constexpr int LDS = STAGES * STAGE;
-  static_assert(TM * PITCH <= LDS && 2 * LDS <= 160 * 1024, "two workgroups per CU");
+  static_assert(TM * PITCH <= LDS && PER_CU * LDS <= 160 * 1024, "LDS budget");
 };
 
-template <class QT, int ROWS>
-__global__ __launch_bounds__(256, 2) void fdb_dgrad_kernel(const DgradParams p) {
-  using S = DShape<ROWS>;
-  static_assert(S::NW == 4, "four waves");
+template <class QT, class S>
+__global__ __launch_bounds__(64 * S::NW, S::PER_CU * S::NW / 4) void fdb_dgrad_kernel(const DgradParams p) {
   using frag = typename QT::frag;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane & 15, kg = lane >> 4;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / S::WN, wn = wave % S::WN;
   // every XCD takes a run of tiles
   const int all = p.tiles[0] + p.tiles[1], n = blockIdx.x, xcd = n & 7, each = all >> 3, more = all & 7;
   int tile = xcd * each + min(xcd, more) + (n >> 3);
@@ -104,11 +102,11 @@ __global__ __launch_bounds__(256, 2) void fdb_dgrad_kernel(const DgradParams p) 
   for (int t = 0; t < S::STAGES - 1; ++t)
     if (t < steps) fill(t);
   const uint32_t xrow = lds0 + (uint32_t)((wm * 16 * S::FM + r) * kRow), f = (uint32_t)swz16(r);
-  uint32_t wlane[4][2];
+  uint32_t wlane[S::FN][2];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < S::FN; ++j)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) wlane[j][h] = lds0 + S::TM * kRow + (uint32_t)wn * kPanel + tr_lane(lane, j, h);
+    for (int h = 0; h < 2; ++h) wlane[j][h] = lds0 + S::TM * kRow + (uint32_t)((wn * S::FN + j) >> 2) * kPanel + tr_lane(lane, wn * S::FN + j, h);
   int buf = 0;
 #pragma unroll 1
   for (int t = 0; t < steps; ++t) {
@@ -137,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void fdb_dgrad_kernel(const DgradParams p) 
   for (int i = 0; i < S::FM; ++i)
 #pragma unroll
     for (int j = 0; j < S::FN; ++j)
-      QT::store4(smem + ((wm * S::FM + i) * 16 + r) * S::PITCH + (64 * wn + 16 * j + 4 * kg) * 2, acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+      QT::store4(smem + ((wm * S::FM + i) * 16 + r) * S::PITCH + ((wn * S::FN + j) * 16 + 4 * kg) * 2, acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
   __syncthreads();
   constexpr int CH = S::TN / 8;
   for (int c = tid; c < S::TM * CH; c += 64 * S::NW) {
@@ -153,7 +151,7 @@ struct WgradParams {
   int32_t rows[2], x_cols[2], y_cols, tiles_n, tiles, shares;
 };
 // 128 x 128 outputs by four waves, two stages, two workgroups per CU, of which one multiplies while the other waits at its barrier.  8 x 512
-// tokens, 12 heads, with the fold, best number of shares: 31.2 us; 128 x 192 by eight waves, three stages, alone on its CU 36.0, 128 x 64
+// tokens, 12 heads, with the fold, best number of shares: 31.2 us (29.0 since rows past the last one are zeroed in the LDS); 128 x 192 by eight waves, three stages, alone on its CU 36.0, 128 x 64
 // 36.6, 64 x 192 33.5, 128 x 256 34.4, 128 x 128 by eight waves 38.4 and 44.0.
 struct WShape {
   static constexpr int TM = 128, TN = 128, WN = 2, STAGES = 2, PER_CU = 2, NW = 4, FM = 4, FN = 4;
@@ -314,10 +312,9 @@ __global__ __launch_bounds__(256) void fdb_wgrad_fold_kernel(const float* __rest
 
 int tiles_of(int64_t n, int t) { return (int)((n + t - 1) / t); }
 
-template <class QT, int ROWS>
+template <class QT, class S>
 int launch_dgrad(DgradParams p, hipStream_t stream) {
-  using S = DShape<ROWS>;
-  auto kern = fdb_dgrad_kernel<QT, ROWS>;
+  auto kern = fdb_dgrad_kernel<QT, S>;
   static std::atomic<uint64_t> lds_set{0};
   const hipError_t e = fdb_set_lds_once((const void*)kern, S::LDS, lds_set);
   if (e != hipSuccess) return (int)e;
@@ -326,12 +323,17 @@ int launch_dgrad(DgradParams p, hipStream_t stream) {
   hipLaunchKernelGGL(kern, dim3(p.tiles[0] + p.tiles[1]), dim3(64 * S::NW), S::LDS, stream, p);
   return (int)hipGetLastError();
 }
-// Tiles of 64 rows while they make one round of two workgroups a CU, of 128 beyond: 8192 tokens, 12 heads 39.2 -> 31.0 us, 4096 tokens, 16 heads
-// 46.8 -> 35.9.
+// Eight waves a tile: a stage is 0.35 us of latency and barrier for a workgroup that has its CU to itself, and half of it for two that share one, so
+// a tile of 64 rows while each has a CU (four waves, us: 12 heads, 1000 tokens 16.5 -> 14.5, 16 heads, 300 tokens 20.6 -> 18.1), then one of 128 while
+// that is so, four stages deep (64 rows, two workgroups a CU: 12 heads, 4096 tokens 22.2 -> 21.1, 3000 tokens 21.0 -> 20.1; 16 heads, 2048 tokens 26.3 -> 25.5),
+// then two of 128 a CU (four waves: 12 heads, 6000 tokens 30.1 -> 29.2, 8192 34.2 -> 33.4, 16 heads, 4096 tokens 38.2 -> 35.5; 256 rows by eight waves 42.5).
+// Waves that lie across the 128 columns (2 x 4) where x is the shorter side, along the rows where it is not (the other way round: 16.8 and 22.0 us).
 template <class QT>
 int launch_dgrad_rows(const DgradParams& p, hipStream_t stream) {
-  const int64_t tiles = (int64_t)(tiles_of(p.rows[0], 64) + tiles_of(p.rows[1], 64)) * tiles_of(p.cols, 128);
-  return tiles <= 2 * fdb_cu_count() ? launch_dgrad<QT, 64>(p, stream) : launch_dgrad<QT, 128>(p, stream);
+  auto tiles = [&](int rows) { return (int64_t)(tiles_of(p.rows[0], rows) + tiles_of(p.rows[1], rows)) * tiles_of(p.cols, 128); };
+  if (tiles(64) <= fdb_cu_count()) return launch_dgrad<QT, DShape<64, 2, 4, 3, 2>>(p, stream);
+  if (tiles(128) <= fdb_cu_count()) return launch_dgrad<QT, DShape<128, 4, 2, 4, 1>>(p, stream);
+  return launch_dgrad<QT, DShape<128, 4, 2, 2, 2>>(p, stream);
 }
 
 template <class QT>

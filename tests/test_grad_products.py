@@ -37,6 +37,13 @@ def test_dgrad(rows, depth, cols, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,depth,cols", [((3000, 65), (64, 192), 768), ((2561, 0), (128, 64), 832), ((129, 4100), (448, 256), 640)])
+def test_dgrad_of_one_round_of_tall_tiles(rows, depth, cols):
+    """More tiles of 64 rows than compute units and no more of 128: fewer stages than the ring has, as many, and more."""
+    test_dgrad(rows, depth, cols, torch.bfloat16)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("rows,x_cols,y_cols", [((1, 1), (192, 128), 64), ((63, 64), (384, 256), 128), ((65, 129), (320, 256), 192), ((200, 512), (576, 384), 256),
                                                 ((1000, 512), (2304, 1536), 768), ((4096, 512), (2304, 1536), 768), ((700, 64), (192, 128), 1024)])
