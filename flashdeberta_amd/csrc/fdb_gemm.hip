@@ -332,8 +332,9 @@ int launch_shape(GemmParams p, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-using S32x64 = GemmShape<32, 64, 2, 2, 4, 3>;
+using S32x64 = GemmShape<32, 64, 1, 4, 4, 3>;
 using S64x64 = GemmShape<64, 64, 2, 2, 3, 3>;
+using S64x64Eight = GemmShape<64, 64, 2, 4, 3, 3>;   // while each has a CU to itself: half the instructions of a stage in a row
 using S64x192Deep = GemmShape<64, 192, 2, 4, 4, 1>;   // alone on its CU: four stages instead of a second workgroup
 using S64x192 = GemmShape<64, 192, 2, 4, 2, 2>;
 using S256x192 = GemmShape<256, 192, 4, 2, 2, 1>;
@@ -345,11 +346,14 @@ int64_t tiles_of(int64_t M, int64_t N, int tm, int tn) { return (M + tm - 1) / t
 //   512 x 768 x 768   5.4* 6.2 8.9 8.2 18.9      1500 x 768 x 768    7.7 7.3* 8.9 8.5 19.2      1024 x 3072 x 768  22.9 17.2 12.3* 14.3 24.3
 //   4096 x 768 x 3072 44.6 32.3 26.9* 34.6 59.7  2048 x 3072 x 768  43.1 27.5 22.9 17.4* 25.2   8192 x 768 x 768  26.3 19.6 19.0 15.3* 23.1
 //   3000 x 3072 x 768 61.0 39.8 32.7 27.9 26.4*  4096 x 3072 x 768  82.3 50.5 42.8 31.1 27.7*   8192 x 3072 x 768  155 97.3 81.4 58.1 53.4*
+// The first by waves side by side, 1 x 4 instead of 2 x 2: 5.2 -> 5.0, [300 x 768] . [768 x 768] 5.0 -> 4.7.  The second by eight waves instead of four: 512 x 1536 x 768
+// 5.8 -> 5.5, 1024 x 768 x 768 6.2 -> 5.7; beyond a tile a compute unit four are the faster: 1500 x 768 x 768 7.1 and 7.2, 512 x 2304 x 768 6.8 and 7.1.
 // (64 x 96, 128 x 96, 128 x 128, 128 x 144, 128 x 192 and 256 x 256, with two to five stages, lie between these.)
 template <class QT, int EPI>
 int launch_gemm(const GemmParams& p, hipStream_t stream) {
   const int64_t cus = fdb_cu_count();
   if (tiles_of(p.M, p.N, 32, 64) <= cus) return launch_shape<QT, EPI, S32x64>(p, stream);
+  if (tiles_of(p.M, p.N, 64, 64) <= cus) return launch_shape<QT, EPI, S64x64Eight>(p, stream);
   if (tiles_of(p.M, p.N, 64, 64) * 8 <= cus * 15) return launch_shape<QT, EPI, S64x64>(p, stream);
   if (tiles_of(p.M, p.N, 64, 192) <= cus) return launch_shape<QT, EPI, S64x192Deep>(p, stream);
   if (tiles_of(p.M, p.N, 64, 192) <= 2 * cus) return launch_shape<QT, EPI, S64x192>(p, stream);

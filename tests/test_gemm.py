@@ -45,6 +45,13 @@ def test_tiles_and_their_remainders(M, N, K, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1030, 1160, 64), (1030, 1160, 256), (961, 1032, 192)])
+def test_tiles_of_64_by_four_waves(M, N, K):
+    """More tiles of 64 x 64 than compute units, up to where wider ones begin; (1030, 520) is eight waves'."""
+    test_tiles_and_their_remainders(M, N, K, torch.bfloat16)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("M,N,K", [(33, 4, 64), (200, 772, 128), (1030, 516, 64), (1601, 1364, 64), (3000, 1164, 64), (5000, 1404, 64)])   # streamed, then each tile
 @pytest.mark.parametrize("pitch,shift", [(0, 0), (4, 0), (0, 1), (4, 3), (8, 2)])   # of the output's rows beyond N, and elements the bias is off 8 bytes by
