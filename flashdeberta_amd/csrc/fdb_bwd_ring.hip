@@ -755,7 +755,8 @@ __global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingPara
 // which 90 scalar ones were found to be more than half of what the waves issued (and 89 -> 16 scalar registers spilled to lanes):
 // 12 heads, us, 8 x 512 padded 25.3 -> 19.4, 2 x 1501 31.8 -> 26.6, 8 x 4096 270 -> 260.  Loads run two row blocks ahead.  No faster: eight
 // waves, half of them for either table, which doubles the scalar instructions (25.3 -> 26.5), and the operands asked for ahead of the next loads.
-// A launch without divisions and scalar loads ahead of each sequence: 19.4 -> 17.4 and 26.6 -> 25.8.  What is left beside the turns (0.33 us
+// A launch without divisions and scalar loads ahead of each sequence: 19.4 -> 17.4 and 26.6 -> 25.8.  The
+// groups in rising order with the saturated rows' last: falling, with those first, the backward of 2 x 1501 takes 195 us where this takes 190.5.  What is left beside the turns (0.33 us
 // for two workgroups of a CU) is the writing of the shares' sums, 25 MB of them.
 constexpr int kGBlk = 2048, kGRing = 4, kKRing = 8;
 constexpr int kTgOffK = kGRing * kTile, kTgOffG = kTgOffK + kKRing * kTile, kTgLds = kTgOffG + 4 * kGRing * kGBlk;
@@ -773,7 +774,7 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  const int h = (int)blockIdx.x, part = (int)blockIdx.y, group = p.tg_groups - (int)blockIdx.z - (p.has_far ? 0 : 1);  // the saturated rows first
+  const int h = (int)blockIdx.x, part = (int)blockIdx.y, group = (int)blockIdx.z;  // the saturated rows last
   // this part's items: (batch row, chunk of row blocks), as many as any other's
   int it0 = part * p.tg_items, it1 = it0 + p.tg_items;
   int first = 0, len = 0, before = 0, lo = 0, hi = 0;   // BY_LENGTH: this lane's sequence and the row blocks ahead of it; this part's of all
@@ -885,10 +886,8 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_table_grad_kernel(const FdbBw
     const int n_rows = (Lb + 31) / 32;                       // row blocks of this sequence
     item(it, n_rows, I0, I1);
     const int rho0 = p.rho_min + 4 * group;
-    // block (I, rho) can only be there with a row block of k at I - rho, or one past the last: the turns outside do nothing
-    const bool lead = I0 <= max(rho0, 0);                    // no item before has a turn: the key rows ahead of the first row block are this one's as well
-    I0 = max(I0, rho0), I1 = min(I1, n_rows + rho0 + 4);
     if (I0 >= I1) continue;
+    const bool lead = I0 == 0;                               // the key rows ahead of the first row block are this item's as well
     const int last = I1 - I0;   // one more turn than row blocks: the last block's rows of k that precede it
     const char* const q_rows = p.q + ((int64_t)b * p.q_sb + (int64_t)tok0 * p.q_st + (int64_t)h * p.q_sh) * 2 + chunk_off;
     const char* const k_rows = p.k + ((int64_t)b * p.k_sb + (int64_t)tok0 * p.k_st + (int64_t)h * p.k_sh) * 2 + chunk_off;
