@@ -670,6 +670,7 @@ int bwd_tables_plan(const fdb_attn_bwd_tables_args* a, FdbBwdRingParams* p, int6
   p->zero_block = take(2048);
   p->e_parts = (float*)take(parts * per * 4 * 2 * 32 * 64 * 4);
   p->far_parts = (float*)take(parts * a->heads * 256 * 4);
+  p->places = (FdbPlace*)take(2 * tiles * pairs * (int64_t)sizeof(FdbPlace));   // (also without lengths: the size is asked for without them as well)
   *bytes = off;
   return FDB_OK;
 }

@@ -249,11 +249,11 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // in scalar registers: what depends on it alone stays scalar
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
+  int b, tile, h, tok0, sl;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
   place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr,
-            MODE == kFarOnly ? (p.causal ? kLastFirst : kEdgesFirst) : (MODE == kNearRing ? kMiddleFirst : kNatural), lane, b, tile, h);
+            MODE == kFarOnly ? (p.causal ? kLastFirst : kEdgesFirst) : (MODE == kNearRing ? kMiddleFirst : kNatural), lane, b, tile, h, tok0, sl);
 
-  int m0, tok0, Lb;
+  int m0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
     if (tile >= p.wl[0]) return;
@@ -264,8 +264,6 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
     qo = ko = vo = oo = 0;
   } else {
     m0 = tile * FDB_BM;
-    tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
-    const int sl = p.seq_len ? p.seq_len[b] : p.L;  // negative: a batch row the caller could not express, NaN throughout
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
       fill_pad_rows<D * VT::SZ>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * VT::SZ, p.o_st * VT::SZ, tile,

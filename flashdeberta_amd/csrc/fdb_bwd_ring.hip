@@ -108,11 +108,14 @@ __device__ __forceinline__ Zones zones_of(int m0, int Lb, int R, bool causal, bo
   return z;
 }
 
+// near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
+__device__ __forceinline__ int order_of(const FdbBwdRingParams& p, bool dq) { return p.causal ? (dq ? kLastFirst : kNatural) : kMiddleFirst; }
+
 // One workgroup of a role, the wg-th of its grid.  STATS: the row statistics are there (fdb_row_stats_kernel); otherwise the dQ role,
 // launched on its own before the other, computes them on its way.
-// BY_LENGTH: a padded batch dealt by the lengths of its sequences (an instantiation of its own: its registers cost the other 1 to 3 %).
+// BY_LENGTH: of a padded batch, whose place `at` is read from the table of find_places (an instantiation of its own: its registers cost the other 1 to 3 %).
 template <class QT, int ROLE, bool STATS, bool BY_LENGTH>
-__device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg) {
+__device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg, const FdbPlace* at) {
   constexpr bool kDQ = ROLE == 0;
   constexpr int KS = 4, DBLKS = 2;
   using frag = typename QT::frag;
@@ -121,13 +124,12 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  // near steps cost twice a far one, so the tiles with the most of them start first (causal: those with the most steps)
   int b, tile_x, h;
-  if constexpr (BY_LENGTH) padded_map(wg, p.seq_start, p.seq_len, p.B, p.H, p.tiles, p.L, lane, b, tile_x, h);
-  else block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, p.causal ? (kDQ ? kLastFirst : kNatural) : kMiddleFirst, b, tile_x, h);
+  if constexpr (BY_LENGTH) b = (int)own_sgpr((uint32_t)at->b), tile_x = (int)own_sgpr((uint32_t)at->tile), h = (int)own_sgpr((uint32_t)at->h);
+  else block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, order_of(p, kDQ), b, tile_x, h);
   const int m0 = tile_x * FDB_BM;
-  const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
-  const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
+  const int tok0 = BY_LENGTH ? (int)own_sgpr((uint32_t)at->tok0) : p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
+  const int Lb = BY_LENGTH ? (int)own_sgpr((uint32_t)at->tokens) : p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
   if (p.seq_start || p.seq_len) {  // rows of padding have no gradient
     auto clear = [&](char* t, int64_t sb, int64_t st, int64_t sh) {
       fill_pad_rows<kRowBytes>(t + ((int64_t)b * sb + (int64_t)h * sh) * 2, st * 2, tile_x, p.L, tok0, Lb, 0u, tid);
@@ -688,7 +690,8 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
 
 template <class QT, int ROLE, bool BY_LENGTH>
 __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdRingParams p) {
-  bwd_ring<QT, ROLE, false, BY_LENGTH>(p, (int)blockIdx.x);
+  const int wg = (int)blockIdx.x;
+  bwd_ring<QT, ROLE, false, BY_LENGTH>(p, wg, BY_LENGTH ? p.places + (ROLE == 0 ? wg : (int)gridDim.x + wg) : nullptr);
 }
 
 // Both roles as one launch, the longer one's workgroups first: 2 x 288 workgroups, say, leave half of the GPU's 512 places empty
@@ -696,22 +699,87 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_ring_kernel(const FdbBwdR
 template <class QT, bool BY_LENGTH>
 __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_both_kernel(const FdbBwdRingParams p) {
   const int wg = (int)blockIdx.x;
-  if constexpr (BY_LENGTH) {   // both roles of a tile's heads one after the other: the short texts of both end the launch
-    const int pair = wg / (2 * p.H), h = wg - pair * 2 * p.H;
-    if (h < p.H) bwd_ring<QT, 1, true, true>(p, pair * p.H + h);
-    else bwd_ring<QT, 0, true, true>(p, pair * p.H + h - p.H);
+  if constexpr (BY_LENGTH) {
+    const FdbPlace* at = p.places + wg;
+    if (at->keys) bwd_ring<QT, 1, true, true>(p, at->n, at);
+    else bwd_ring<QT, 0, true, true>(p, at->n, at);
   } else {
     const int n = (int)(gridDim.x >> 1);
-    if (wg < n) bwd_ring<QT, 1, true, false>(p, wg);
-    else bwd_ring<QT, 0, true, false>(p, wg - n);
+    if (wg < n) bwd_ring<QT, 1, true, false>(p, wg, nullptr);
+    else bwd_ring<QT, 0, true, false>(p, wg - n, nullptr);
   }
+}
+
+// The places of both roles' workgroups of a padded batch (fdb_deals_by_length), batch rows x 2 of them by this workgroup, the `at`-th of tiles * heads.  The order
+// is padded_map's, or block_map's where the mask hides little.  together: one launch, both roles of a tile's heads one after the other, the short texts of both end it;
+// otherwise dQ's places, then the others.
+// A table, because the roles have no registers to spare: with padded_map at its start the dQ role spilt 19 instead of 14 and took 705 us instead of 640 (8 x 3000).
+__device__ __forceinline__ void find_places(const FdbBwdRingParams& p, int at, bool together) {
+  __shared__ int first[64], tokens[64], sorted[64], row[64], dealt;
+  const int tid = (int)threadIdx.x, batch = p.B, heads = p.H, all = p.tiles * heads * batch;
+  if (tid < 64) {
+    int tok0 = 0, mine = 0;
+    if (tid < batch) {
+      if (p.seq_start) tok0 = min(max(p.seq_start[tid], 0), p.L);
+      mine = min(max(p.seq_len[tid], 0), p.L - tok0);
+    }
+    const bool deals = padded_batch_deals(mine, batch, p.L, tid);
+    const int blocks = tid < batch ? (mine + 31) >> 5 : -1;
+    int rank = 0;
+    for (int x = 0; x < batch; ++x) {
+      const int other = __builtin_amdgcn_readlane(blocks, x);
+      rank += other > blocks || (other == blocks && x < tid) ? 1 : 0;
+    }
+    first[tid] = tok0, tokens[tid] = mine;
+    if (tid < batch) sorted[rank] = blocks, row[rank] = tid;
+    if (tid == 0) dealt = deals;
+  }
+  __syncthreads();
+  const int n = at * batch + tid;
+  if (tid >= batch || n >= all) return;
+  auto put = [&](int slot, int b, int t, int h, bool keys) {
+    p.places[slot] = FdbPlace{b, t, h, first[b], tokens[b], n, keys ? 1 : 0, 0};
+  };
+  if (!dealt) {
+#pragma unroll
+    for (int keys = 0; keys < 2; ++keys) {
+      int b, t, h;
+      block_place(n, batch, heads, p.tiles, p.groups_together, order_of(p, keys == 0), b, t, h);
+      put(together == (keys != 0) ? n : all + n, b, t, h, keys != 0);
+    }
+    return;
+  }
+  int u = n / heads, t = p.tiles - 1, here = 0;
+  const int h = n - u * heads;
+  for (; t >= 0; --t) {   // `here` sequences have tokens in tile t
+    while (here < batch && sorted[here] > t * (FDB_BM / 32)) ++here;
+    if (u < here) break;
+    u -= here;
+  }
+  if (t < 0) {   // padding
+    for (t = 0; t < p.tiles; ++t) {
+      while (here > 0 && sorted[here - 1] <= t * (FDB_BM / 32)) --here;
+      if (u < batch - here) break;
+      u -= batch - here;
+    }
+    u += here;
+  }
+  const int b = row[u], pair = n / heads * 2 * heads + h;
+  put(together ? pair : all + n, b, t, h, true);
+  put(together ? pair + heads : n, b, t, h, false);
 }
 
 // The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), 128 rows a workgroup, two lanes a row that add up in the dQ
 // role's order, so that a batch row's gradients have the same bits whichever way it is launched.  Bound by reading dO and O.
-template <class QT>
+// PLACES: with the workgroups' places, the first layer of the grid (the only one: those alone).
+template <class QT, bool PLACES>
 __global__ __launch_bounds__(256) void fdb_row_stats_kernel(const FdbBwdRingParams p) {
-  const int b = (int)blockIdx.z, h = (int)blockIdx.y, g = threadIdx.x & 1, row = (int)blockIdx.x * 128 + (int)(threadIdx.x >> 1);
+  if constexpr (PLACES)
+    if (blockIdx.z == 0) {
+      find_places(p, (int)(blockIdx.y * gridDim.x + blockIdx.x), gridDim.z > 1);
+      return;
+    }
+  const int b = (int)blockIdx.z - (PLACES ? 1 : 0), h = (int)blockIdx.y, g = threadIdx.x & 1, row = (int)blockIdx.x * 128 + (int)(threadIdx.x >> 1);
   const int tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;
   if (row >= Lb) return;   // a row's two lanes leave together
@@ -1101,9 +1169,10 @@ int launch_all(const FdbBwdRingParams& p, hipStream_t stream) {
   if (e != hipSuccess) return (int)e;
   const unsigned grid = (unsigned)p.tiles * (unsigned)p.H * (unsigned)p.B;
   if (grid <= kMostTogether) {
-    hipLaunchKernelGGL(fdb_row_stats_kernel<QT>, dim3((unsigned)p.tiles, (unsigned)p.H, (unsigned)p.B), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((fdb_row_stats_kernel<QT, BY_LENGTH>), dim3((unsigned)p.tiles, (unsigned)p.H, (unsigned)p.B + (BY_LENGTH ? 1 : 0)), dim3(256), 0, stream, p);
     hipLaunchKernelGGL(both, dim3(2 * grid), dim3(kThreads), kLds, stream, p);
   } else {
+    if (BY_LENGTH) hipLaunchKernelGGL((fdb_row_stats_kernel<QT, true>), dim3((unsigned)p.tiles, (unsigned)p.H), dim3(256), 0, stream, p);
     hipLaunchKernelGGL(dq, dim3(grid), dim3(kThreads), kLds, stream, p);
     hipLaunchKernelGGL(dkv, dim3(grid), dim3(kThreads), kLds, stream, p);
   }

@@ -268,26 +268,29 @@ __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { re
 // taken together as leave their K and V in an XCD's 4 MB of L2: 96 query tiles of 16-bit head_dim 64 are 3 MB.  The host passes
 // that number (fdb_groups_together): each division here costs every workgroup some 40 instructions before its first load.
 enum { kNatural = 0, kEdgesFirst = 1, kMiddleFirst = 2, kLastFirst = 3 };
+__device__ __forceinline__ void block_place(int n, int batch, int heads, int tiles_per_seq, int most, int order, int& b, int& t, int& h) {   // the fixed layout's; a lane each
+  const int groups = batch * heads;
+  const int first = n / (most * tiles_per_seq) * most;
+  const int here = min(groups - first, most), m = n - first * tiles_per_seq;
+  t = m / here;
+  const int i = m - t * here;
+  const int grp = first + (i < (here & ~7) ? (n & 7) | (i & ~7) : i);
+  if (order == kLastFirst) {
+    t = tiles_per_seq - 1 - t;
+  } else if (order != kNatural) {
+    if (order == kMiddleFirst) t = tiles_per_seq - 1 - t;
+    t = (t & 1) ? tiles_per_seq - 1 - (t >> 1) : (t >> 1);  // 0, T-1, 1, T-2, ...
+  }
+  b = grp / heads;
+  h = grp - b * heads;
+}
 __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles_per_seq, int most, bool fixed, int order, int& b_out, int& t_out,
                                           int& h_out) {
   // Not the caller's variables: the compiler makes one store, to a chosen address, of the two branches' stores, and the numbers then
   // pass through scratch memory before a workgroup's first load.  Forward of 1 x 4096, 16 heads: 119.5 -> 117.9 us.
   int b, t, h;
   if (fixed) {
-    const int groups = batch * heads;
-    const int first = n / (most * tiles_per_seq) * most;
-    const int here = min(groups - first, most), m = n - first * tiles_per_seq;
-    t = m / here;
-    const int i = m - t * here;
-    const int grp = first + (i < (here & ~7) ? (n & 7) | (i & ~7) : i);
-    if (order == kLastFirst) {
-      t = tiles_per_seq - 1 - t;
-    } else if (order != kNatural) {
-      if (order == kMiddleFirst) t = tiles_per_seq - 1 - t;
-      t = (t & 1) ? tiles_per_seq - 1 - (t >> 1) : (t >> 1);  // 0, T-1, 1, T-2, ...
-    }
-    b = grp / heads;
-    h = grp - b * heads;
+    block_place(n, batch, heads, tiles_per_seq, most, order, b, t, h);
   } else {
     // packed sequences: the work-list holds the tiles longest sequence first; all heads of a tile are
     // dealt before the next tile, so the whole launch runs from long workgroups to short ones
@@ -302,23 +305,42 @@ __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles
   h_out = __builtin_amdgcn_readfirstlane(h);
 }
 
-// Linear workgroup id -> (batch row, query tile, head) of a padded batch (host: fdb_deals_by_length).  The dispatcher takes workgroups in order and waits
+// Whether a padded batch is dealt by the lengths of its sequences: a quarter of them or more leave at least a quarter of the row empty.  mine: the tokens of
+// this lane's sequence.
+__device__ __forceinline__ bool padded_batch_deals(int mine, int batch, int most, int lane) { return 4 * __popcll(__ballot(lane < batch && mine < most - most / 4)) >= batch; }
+
+// Linear workgroup id -> (batch row, query tile, head) of a padded batch (host: fdb_deals_by_length), with the row's first token and its length as the call gives it;
+// false: block_map's order is the one to take.  The dispatcher takes workgroups in order and waits
 // for a place where the next one belongs: a workgroup without tokens among the first leaves a place that stays empty, and one of a long text
 // among the last makes the launch end late.  So the tiles with tokens come first, the highest tile of all sequences before the next lower one and in
 // each the longest sequence first; a launch ends on the shortest texts, and on the tiles of padding, which are only cleared.  All heads of a tile
-// are dealt before the next.  Lengths between a quarter and all of the longest, 12 heads, bf16, us, block_map -> here: near launch 32 x 128 15.2 -> 13.4, 8 x 512 31.2 ->
-// 24.9, 16 x 256 20.2 -> 17.7, 16 x 512 48.0 -> 36.3 (where 52 of 512 places stood empty for 20 us), 64 x 128 24.4 -> 22.3; both roles of the backward 8 x 512 69.2 ->
-// 53.4, 16 x 512 117 -> 99.8, 32 x 128 38.5 -> 37.5.  Every wave finds its place itself, a lane a sequence: how many of the tiles at hand have tokens is a count of lanes,
-// the length of the sequence with a given rank is found bit by bit.
-__device__ __forceinline__ void padded_map(int n, const int32_t* start, const int32_t* length, int batch, int heads, int tiles_per_seq, int most, int lane, int& b_out,
-                                           int& t_out, int& h_out) {
-  int mine = -1;   // this lane's sequence: its tokens
-  if (lane < batch) mine = min(max(length[lane], 0), most - (start ? min(max(start[lane], 0), most) : 0));
+// are dealt before the next.
+// Lengths between a quarter and all in no order, 12 heads, bf16, us, block_map -> here (two draws where they differ in sign):
+//   forward   32 x 128 12.8 -> 11.5   64 x 256 48.4 -> 45.9   8 x 512 28.8 -> 22.0, 29.6 -> 30.0   64 x 512 124 -> 112   8 x 1024 78.0 -> 60.8   8 x 2048 166 -> 149
+//             4 x 4096 263 -> 253, 232 -> 242   8 x 4096 439 -> 383   4 x 8192 749 -> 713   16 heads 4 x 2048 111 -> 116, 118 -> 108   2 x 8192 528 -> 508
+//             fp32 8 x 512 138 -> 94   head_dim 128 8 x 2048 371 -> 257   e4m3 8 x 2048 138 -> 127   causal 8 x 384, 16 heads 18.8 -> 19.7   8 x 1024 68.5 -> 50.4
+//   backward  32 x 128 124 -> 118   64 x 256 206 -> 196   8 x 512 99.5 -> 79.1   64 x 512 551 -> 490   8 x 1024 238 -> 208   8 x 2048 558 -> 516
+//             8 x 4096 1604 -> 1393   4 x 8192 2806 -> 2564   16 heads 4 x 2048 379 -> 393, 394 -> 357   2 x 8192 2266 -> 2378
+// One sequence of 64 long and the others a quarter of it, mostly padding: forward 64 x 128 14.2 -> 15.6, 64 x 512 37.9 -> 39.3, 32 x 1024 60.6 -> 52.1.
+// Where a mask hides little, the order gives up the heads' places on the XCDs for nothing: lengths all the same, forward 64 x 512 165 -> 172, 8 x 4096 609 -> 679,
+// backward 32 x 1024 1140 -> 1211, 16 x 4096 4564 -> 5102; of three quarters to all between -7 and +7 %.  So it takes a quarter of the sequences to leave a quarter empty.
+// Every wave finds its place itself, a lane a sequence: how many of the tiles at hand have tokens is a count of lanes,
+// the length of the sequence with a given rank, in blocks of 32 tokens, is found bit by bit.
+__device__ __forceinline__ bool padded_map(int n, const int32_t* start, const int32_t* length, int batch, int heads, int tiles_per_seq, int most, int lane, int& b_out,
+                                           int& t_out, int& h_out, int& tok0_out, int& len_out) {
+  int first = 0, len = 0, mine = 0;   // this lane's sequence
+  if (lane < batch) {
+    if (start) first = min(max(start[lane], 0), most);
+    len = length[lane];
+    mine = min(max(len, 0), most - first);
+  }
+  if (!padded_batch_deals(mine, batch, most, lane)) return false;
+  const int blocks = (mine + 31) >> 5;
   int u = (int)((uint32_t)n / (uint32_t)heads);
   const int h = n - u * heads;
   int t = tiles_per_seq - 1, rank = -1;
   for (; t >= 0; --t) {
-    const int here = __popcll(__ballot(mine > t * FDB_BM));
+    const int here = __popcll(__ballot(blocks > t * (FDB_BM / 32)));
     if (u < here) {
       rank = u;
       break;
@@ -327,7 +349,7 @@ __device__ __forceinline__ void padded_map(int n, const int32_t* start, const in
   }
   if (rank < 0) {   // padding
     for (t = 0; t < tiles_per_seq; ++t) {
-      const int here = __popcll(__ballot(mine > t * FDB_BM));
+      const int here = __popcll(__ballot(blocks > t * (FDB_BM / 32)));
       if (u < batch - here) {
         rank = here + u;
         break;
@@ -336,21 +358,28 @@ __device__ __forceinline__ void padded_map(int n, const int32_t* start, const in
     }
   }
   int of = 0;   // the length of that rank: the largest that more than `rank` sequences reach
-  for (int bit = 31 - __builtin_clz(most); bit >= 0; --bit) {
+  for (int bit = 31 - __builtin_clz((most + 31) >> 5); bit >= 0; --bit) {
     const int x = of | (1 << bit);
-    if (__popcll(__ballot(mine >= x)) > rank) of = x;
+    if (__popcll(__ballot(blocks >= x)) > rank) of = x;
   }
-  uint64_t same = __ballot(mine == of);
-  for (int before = rank - __popcll(__ballot(mine > of)); before > 0; --before) same &= same - 1;
-  b_out = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)same) - 1);
+  uint64_t same = __ballot(lane < batch && blocks == of);
+  for (int before = rank - __popcll(__ballot(blocks > of)); before > 0; --before) same &= same - 1;
+  const int b = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)same) - 1);
+  b_out = b;
   t_out = __builtin_amdgcn_readfirstlane(t);
   h_out = __builtin_amdgcn_readfirstlane(h);
+  tok0_out = __builtin_amdgcn_readlane(first, b);
+  len_out = __builtin_amdgcn_readlane(len, b);
+  return true;
 }
-// Where workgroup n belongs: block_map's order, or that of a padded batch.
+// Where workgroup n belongs: block_map's order, or that of a padded batch.  Fixed layout: the batch row's first token and its length as the call gives it
+// (negative: a batch row the caller could not express, NaN throughout).
 template <class Params>
-__device__ __forceinline__ void place_of(int n, const Params& p, int tiles_per_seq, bool fixed, int order, int lane, int& b, int& t, int& h) {
-  if (p.by_length) padded_map(n, p.seq_start, p.seq_len, p.B, p.H, tiles_per_seq, p.L, lane, b, t, h);
-  else block_map(n, p.B, p.H, tiles_per_seq, p.groups_together, fixed, order, b, t, h);
+__device__ __forceinline__ void place_of(int n, const Params& p, int tiles_per_seq, bool fixed, int order, int lane, int& b, int& t, int& h, int& tok0, int& len) {
+  if (p.by_length && padded_map(n, p.seq_start, p.seq_len, p.B, p.H, tiles_per_seq, p.L, lane, b, t, h, tok0, len)) return;
+  block_map(n, p.B, p.H, tiles_per_seq, p.groups_together, fixed, order, b, t, h);
+  tok0 = fixed && p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
+  len = fixed && p.seq_len ? p.seq_len[b] : p.L;
 }
 
 // The 16-bit products by tiles of 16 x 16 outputs, and where they keep a row of 128 bytes in LDS: slot (row, s) holds chunk s ^ swz16(row), so that

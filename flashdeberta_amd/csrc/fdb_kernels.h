@@ -10,8 +10,8 @@
 // (sequence, head) groups whose query tiles are dealt together, see block_map
 inline int32_t fdb_groups_together(int32_t tiles_per_seq) { return 8 * (tiles_per_seq < 96 ? 96 / tiles_per_seq : 1); }
 
-// Whether a padded batch's workgroups are dealt by the lengths of its sequences (padded_map): a lane a sequence, and more workgroups (of all roles) than
-// compute units; fewer have a unit each whatever the order.
+// Whether a padded batch's workgroups may be dealt by the lengths of its sequences (padded_map, which looks at the lengths): a lane a sequence, and more
+// workgroups (of all roles) than compute units; fewer have a unit each whatever the order.
 inline bool fdb_deals_by_length(const int32_t* seq_len, int64_t batch, int64_t workgroups, int64_t cus) {
   return seq_len && batch > 1 && batch <= 64 && workgroups > cus;
 }
@@ -100,6 +100,11 @@ struct FdbBwdParams {
 };
 int fdb_launch_bwd(const FdbBwdParams& p, int dtype, int head_dim, void* stream);
 
+// Where a workgroup of the backward's roles works in a padded batch: the n-th of its role; the batch row's first token and its number of tokens.
+struct FdbPlace {
+  int32_t b, tile, h, tok0, tokens, n, keys, unused;   // keys: the dK/dV role
+};
+
 // Backward with the tables in the kernel (fdb_bwd_ring.hip): fixed layout, head_dim 64, 16-bit types, both position terms.
 struct FdbBwdRingParams {
   const char* q;
@@ -145,8 +150,10 @@ struct FdbBwdRingParams {
                                                             // tg_len row blocks per batch row
   int32_t has_far;
   float scale_log2, sm_scale;
-  int32_t by_length;   // fdb_deals_by_length (last: an argument among the others moves the sixteen-register loads of the rest, and the dQ role spills more)
+  // last: an argument among the others moves the sixteen-register loads of the rest, and the dQ role spills more
+  int32_t by_length;   // fdb_deals_by_length
   int32_t tg_items;    // chunks a share takes
+  FdbPlace* places;    // by_length: two for every (batch row, query tile, head)
 };
 int fdb_launch_bwd_ring(const FdbBwdRingParams& p, int dtype, void* stream);
 

@@ -120,10 +120,10 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
-  int b, tile, h;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
-  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr, kMiddleFirst, lane, b, tile, h);
+  int b, tile, h, tok0, sl;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
+  place_of((int)blockIdx.x, p, p.tiles_per_seq, p.cu == nullptr, kMiddleFirst, lane, b, tile, h, tok0, sl);
 
-  int m0, tok0, Lb;
+  int m0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
     if (tile >= p.wl[0]) return;
@@ -134,8 +134,6 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
     qo = ko = vo = oo = 0;
   } else {
     m0 = tile * FDB_BM;
-    tok0 = p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
-    const int sl = p.seq_len ? p.seq_len[b] : p.L;  // negative: a batch row the caller could not express, NaN throughout
     Lb = min(max(sl, 0), p.L - tok0);
     if (p.fill_pad && blockIdx.y == 0)
       fill_pad_rows<kRowBytes>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,

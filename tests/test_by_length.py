@@ -1,11 +1,12 @@
 """Padded batches whose workgroups are dealt by the lengths of their sequences (padded_map in csrc/fdb_device.h): the bits of the same sequences in a batch of more
 than 64, which is dealt in the plain order."""
+import ctypes
 import random
 
 import pytest
 import torch
 
-from flashdeberta_amd import ops
+from flashdeberta_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +56,78 @@ def test_bits_of_the_plain_order(B, L, H, dtype, kind):
     grads = dtype != torch.float32 and min(lens) >= 0
     for a, b in zip(_call(x, starts, lens, 0, grads), _call(x, starts, lens, 65, grads)):
         assert torch.equal(a, b)
+
+
+class _BwdArgs(ctypes.Structure):   # fdb_attn_bwd_tables_args of include/fdb.h
+    _fields_ = [(n, ctypes.c_void_p) for n in "q k v dout out pos_key pos_query dq dk dv d_pos_key d_pos_query lse seq_start seq_len delta_lut workspace".split()] + \
+        [(f"{t}_stride_{x}", ctypes.c_int64) for t in "q k v do out dq dk dv".split() for x in "bth"] + [(f"{t}_stride_{x}", ctypes.c_int64) for t in "pk pq dp".split() for x in "hr"] + \
+        [(n, ctypes.c_int32) for n in "batch heads head_dim seqlen att_span lut_radius dtype causal".split()] + [("sm_scale", ctypes.c_float)]
+
+
+def _plain_order(B, H, tiles, causal, keys):
+    """block_map: the (sequence, head) groups of an L2's share at a time, a group on one XCD, a tile of all of them before the next."""
+    most, out = 8 * (96 // tiles if tiles < 96 else 1), []
+    for first in range(0, B * H, most):
+        here = min(B * H - first, most)
+        for m in range(tiles * here):
+            t, i = divmod(m, here)
+            n = first * tiles + m
+            g = first + (n % 8 | i & ~7 if i < here & ~7 else i)
+            if causal:
+                t = t if keys else tiles - 1 - t
+            else:
+                t = tiles - 1 - t
+                t = tiles - 1 - t // 2 if t % 2 else t // 2
+            out.append((g // H, t, g % H))
+    return out
+
+
+def _order_by_length(lens, H, tiles):
+    order = sorted(range(len(lens)), key=lambda b: (-((lens[b] + 31) // 32), b))
+    real = [(b, t) for t in reversed(range(tiles)) for b in order if lens[b] > 128 * t]
+    padding = [(b, t) for t in range(tiles) for b in order if lens[b] <= 128 * t]
+    return [(b, t, h) for b, t in real + padding for h in range(H)]
+
+
+@pytest.mark.parametrize("lens,L,H,causal", [
+    ([300, 300, 300], 300, 30, False), ([512] * 8, 512, 12, True), ([400, 384, 512, 384], 512, 17, False),   # a mask that hides little or nothing
+    ([400, 383, 512, 384], 512, 17, False), ([120, 128, 33, 0, 97] * 4, 128, 7, False), ([300, 700, -1, 699, 64, 0, 1], 700, 9, False),
+    ([64, 65, 128, 31, 32, 33, 500, 7] * 8, 520, 8, False), ([520] * 64, 520, 8, False)])   # the last two: the roles as two launches
+def test_places_of_the_backward(lens, L, H, causal):
+    """The order in which the backward's workgroups are dealt, as its table has it."""
+    B, tiles = len(lens), (L + 127) // 128
+    S, (lut, radius) = 64, ops.delta_lut_device(32, 64, torch.device("cuda", 0))
+    new = lambda *s: torch.zeros(*s, device="cuda", dtype=torch.bfloat16)
+    x, tables = [new(B, L, H, 64) for _ in range(8)], [new(H, S, 64) for _ in range(4)]
+    lse, length = torch.zeros(B * L, H, device="cuda"), torch.tensor(lens, dtype=torch.int32, device="cuda")
+    a = _BwdArgs()
+    for name, t in zip("q k v dout out dq dk dv pos_key pos_query d_pos_key d_pos_query lse seq_len delta_lut".split(), x + tables + [lse, length, lut]):
+        setattr(a, name, t.data_ptr())
+    for t in "q k v do out dq dk dv".split():
+        for n, s in zip("bth", (L * H * 64, H * 64, 64)):
+            setattr(a, f"{t}_stride_{n}", s)
+    for t in "pk pq dp".split():
+        setattr(a, t + "_stride_h", S * 64), setattr(a, t + "_stride_r", 64)
+    a.batch, a.heads, a.head_dim, a.seqlen, a.att_span, a.lut_radius, a.dtype, a.causal, a.sm_scale = B, H, 64, L, S // 2, radius, _lib.FDB_BF16, causal, 0.1
+    size = _lib.lib.fdb_attn_bwd_tables_workspace_bytes(ctypes.byref(a))
+    seq_len, a.seq_len = a.seq_len, None
+    assert size == _lib.lib.fdb_attn_bwd_tables_workspace_bytes(ctypes.byref(a))   # whoever asks does not have the lengths yet
+    a.seq_len = seq_len
+    ws = torch.full((size,), 0xFF, dtype=torch.uint8, device="cuda")
+    a.workspace = ws.data_ptr()
+    assert _lib.lib.fdb_attn_bwd_tables(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    n = B * tiles * H
+    got = ws[size - (2 * n * 32 + 255) // 256 * 256:][:2 * n * 32].view(torch.int32).view(2 * n, 8).tolist()
+    real = [min(max(l, 0), L) for l in lens]
+    if 4 * sum(l < L - L // 4 for l in real) < B:
+        dq, keys = [_plain_order(B, H, tiles, causal, k) for k in (False, True)]
+        mixed = [("k", i) for i in range(n)] + [("q", i) for i in range(n)]
+    else:
+        dq = keys = _order_by_length(real, H, tiles)
+        mixed = [(r, H * i + h) for i in range(n // H) for r in "kq" for h in range(H)]
+    if n > 2048:
+        mixed = [("q", i) for i in range(n)] + [("k", i) for i in range(n)]
+    want = [((keys if r == "k" else dq)[i], i, r == "k") for r, i in mixed]
+    assert sorted(dq) == sorted(keys) == [(b, t, h) for b in range(B) for t in range(tiles) for h in range(H)]
+    assert [((b, t, h), i, k == 1) for b, t, h, _, _, i, k, _ in got] == want
+    assert [(first, tokens) for _, _, _, first, tokens, _, _, _ in got] == [(0, real[b]) for (b, _, _), _, _ in want]
