@@ -321,6 +321,8 @@ __device__ __forceinline__ bool padded_batch_deals(int mine, int batch, int most
 //             fp32 8 x 512 138 -> 94   head_dim 128 8 x 2048 371 -> 257   e4m3 8 x 2048 138 -> 127   causal 8 x 384, 16 heads 18.8 -> 19.7   8 x 1024 68.5 -> 50.4
 //   backward  32 x 128 124 -> 118   64 x 256 206 -> 196   8 x 512 99.5 -> 79.1   64 x 512 551 -> 490   8 x 1024 238 -> 208   8 x 2048 558 -> 516
 //             8 x 4096 1604 -> 1393   4 x 8192 2806 -> 2564   16 heads 4 x 2048 379 -> 393, 394 -> 357   2 x 8192 2266 -> 2378
+//   causal, both roles and the rest of the backward, the key tiles mirrored (find_places)   8 x 512 92 -> 87   8 x 1024 175 -> 170   8 x 2048 355 -> 325   32 x 256 104.5 -> 103
+//             48 x 384 234 -> 217   32 x 1024 578 -> 534   16 heads 4 x 4096 641 -> 613   2 x 8192 1342 -> 1343   causal forward 16 x 512 36.3 -> 32.7   8 x 2048 122 -> 101
 // One sequence of 64 long and the others a quarter of it, mostly padding: forward 64 x 128 14.2 -> 15.6, 64 x 512 37.9 -> 39.3, 32 x 1024 60.6 -> 52.1.
 // Where a mask hides little, the order gives up the heads' places on the XCDs for nothing: lengths all the same, forward 64 x 512 165 -> 172, 8 x 4096 609 -> 679,
 // backward 32 x 1024 1140 -> 1211, 16 x 4096 4564 -> 5102; of three quarters to all between -7 and +7 %.  So it takes a quarter of the sequences to leave a quarter empty.

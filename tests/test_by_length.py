@@ -27,12 +27,12 @@ def _bounds(kind, B, L):
     return starts, lens
 
 
-def _call(x, starts, lens, more, grads):
+def _call(x, starts, lens, more, grads, causal=False):
     """Forward (and backward) of the batch and, `more`, as many empty sequences behind it."""
     q, k, v, pk, pq, dout = x
     wide = lambda t: torch.cat([t, torch.zeros(more, *t.shape[1:], device="cuda", dtype=t.dtype)]) if more else t
     vec = lambda t: torch.tensor(list(t) + [0] * more, dtype=torch.int32, device="cuda")
-    kw = dict(position_buckets=32, max_relative_positions=64, seq_start=vec(starts) if any(starts) else None, seq_len=vec(lens))
+    kw = dict(position_buckets=32, max_relative_positions=64, causal=causal, seq_start=vec(starts) if any(starts) else None, seq_len=vec(lens))
     q, k, v, dout = [wide(t) for t in (q, k, v, dout)]
     hold = torch.full((q.numel() * 4,), float("nan"), device="cuda", dtype=q.dtype)
     del hold   # what the outputs are given
@@ -44,17 +44,18 @@ def _call(x, starts, lens, more, grads):
     return [t.nan_to_num(nan=12345.0) for t in res]
 
 
+@pytest.mark.parametrize("causal", [False, True], ids=["all", "causal"])
 @pytest.mark.parametrize("kind", ["ragged", "equal", "left", "odd"])
 @pytest.mark.parametrize("B,L,H,dtype", [(2, 600, 32, torch.bfloat16), (64, 130, 3, torch.float16), (33, 129, 5, torch.bfloat16), (23, 385, 4, torch.bfloat16), (9, 1100, 6, torch.float16),
                                          (40, 200, 4, torch.float32), (64, 520, 8, torch.bfloat16)])   # the last: the backward's roles as two launches
-def test_bits_of_the_plain_order(B, L, H, dtype, kind):
+def test_bits_of_the_plain_order(B, L, H, dtype, kind, causal):
     g = torch.Generator(device="cuda").manual_seed(B + L)
     rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dtype)
     x = rnd(B, L, H, 64), rnd(B, L, H, 64), rnd(B, L, H, 64), rnd(H, 64, 64), rnd(H, 64, 64), rnd(B, L, H, 64)
     starts, lens = _bounds(kind, B, L)
     assert B * ((L + 127) // 128) * H > 256
     grads = dtype != torch.float32 and min(lens) >= 0
-    for a, b in zip(_call(x, starts, lens, 0, grads), _call(x, starts, lens, 65, grads)):
+    for a, b in zip(_call(x, starts, lens, 0, grads, causal), _call(x, starts, lens, 65, grads, causal)):
         assert torch.equal(a, b)
 
 
@@ -82,9 +83,10 @@ def _plain_order(B, H, tiles, causal, keys):
     return out
 
 
-def _order_by_length(lens, H, tiles):
+def _order_by_length(lens, H, tiles, mirrored):
+    """mirrored: the causal key tiles, of which the first has the most queries: as far from the text's end as the query tile of that turn is from its beginning."""
     order = sorted(range(len(lens)), key=lambda b: (-((lens[b] + 31) // 32), b))
-    real = [(b, t) for t in reversed(range(tiles)) for b in order if lens[b] > 128 * t]
+    real = [(b, (lens[b] - 1) // 128 - t if mirrored else t) for t in reversed(range(tiles)) for b in order if lens[b] > 128 * t]
     padding = [(b, t) for t in range(tiles) for b in order if lens[b] <= 128 * t]
     return [(b, t, h) for b, t in real + padding for h in range(H)]
 
@@ -92,7 +94,8 @@ def _order_by_length(lens, H, tiles):
 @pytest.mark.parametrize("lens,L,H,causal", [
     ([300, 300, 300], 300, 30, False), ([512] * 8, 512, 12, True), ([400, 384, 512, 384], 512, 17, False),   # a mask that hides little or nothing
     ([400, 383, 512, 384], 512, 17, False), ([120, 128, 33, 0, 97] * 4, 128, 7, False), ([300, 700, -1, 699, 64, 0, 1], 700, 9, False),
-    ([64, 65, 128, 31, 32, 33, 500, 7] * 8, 520, 8, False), ([520] * 64, 520, 8, False)])   # the last two: the roles as two launches
+    ([400, 383, 512, 384], 512, 17, True), ([120, 128, 33, 0, 97] * 4, 128, 7, True), ([300, 700, -1, 699, 129, 0, 1], 700, 9, True),
+    ([64, 65, 128, 31, 32, 33, 500, 7] * 8, 520, 8, False), ([520] * 64, 520, 8, False), ([64, 65, 128, 31, 32, 257, 500, 7] * 8, 520, 8, True)])   # the last three: the roles as two launches
 def test_places_of_the_backward(lens, L, H, causal):
     """The order in which the backward's workgroups are dealt, as its table has it."""
     B, tiles = len(lens), (L + 127) // 128
@@ -123,7 +126,7 @@ def test_places_of_the_backward(lens, L, H, causal):
         dq, keys = [_plain_order(B, H, tiles, causal, k) for k in (False, True)]
         mixed = [("k", i) for i in range(n)] + [("q", i) for i in range(n)]
     else:
-        dq = keys = _order_by_length(real, H, tiles)
+        dq, keys = [_order_by_length(real, H, tiles, causal and k) for k in (False, True)]
         mixed = [(r, H * i + h) for i in range(n // H) for r in "kq" for h in range(H)]
     if n > 2048:
         mixed = [("q", i) for i in range(n)] + [("k", i) for i in range(n)]
