@@ -11,10 +11,21 @@
 // four score products, and between its 32 MFMAs a step hands C through the scratch and P from lane to lane and fetches V.
 //
 // What bounds it: the fp32 matrix cores (8 x 512, 16 heads: 32 steps of a workgroup in 187 us, 83 % of it products).  The kernel this took the place of
-// gathered the table rows of every block from global memory, 32 cache lines an instruction, and contracted C's shared block twice.  us, before -> here:
-//   1 x 48, 12 heads 18.4 -> 16.9   1 x 512, 12 41.7 -> 36.2   2 x 300, 12 53.5 -> 39.8    8 x 512, 16 240 -> 187
-//   1 x 1024, 12     124 -> 97.9    3 x 777, 12 190 -> 146     4 x 1000, 12 387 -> 310     2 x 2048, 12 578 -> 499
-// Errors against 64 bits are those of the other kernel or a little smaller (1 x 512 3.66e-7 and 3.65e-7 of the output's norm, 1 x 2048 8.0e-7 and 8.7e-7).
+// gathered the table rows of every block from global memory, 32 cache lines an instruction, and contracted C's shared block twice.  Whole calls, replayed
+// (packed ones: one after the other), us, before -> here, 12 heads unless stated; 512 and 64 are the tables' reach:
+//                           both terms                                           c2p alone                      p2c alone
+//                           fixed          causal         packed                 fixed          causal          fixed          causal
+//   1 x 48,  512            23.7 -> 21.5   23.4 -> 21.7   20.6 -> 19.0           18.0 -> 16.8   18.0 -> 17.1    17.9 -> 17.9   17.9 -> 18.1
+//   1 x 300, 512            56.5 -> 42.9   78.3 -> 64.2   54.6 -> 40.4           41.5 -> 31.9   54.1 -> 43.0    42.2 -> 36.1   55.2 -> 52.5
+//   1 x 512, 512            45.0 -> 39.9   121  -> 97.6   43.4 -> 38.6           34.7 -> 31.0   82.7 -> 64.4    35.1 -> 34.2   84.6 -> 80.1
+//   3 x 777, 512            191  -> 147    160  -> 130    216  -> 171            129  -> 95.1   113  -> 88.4    132  -> 120    115  -> 108
+//   8 x 512, 512, 16 heads  244  -> 192    190  -> 149    368  -> 276            164  -> 124    130  -> 98.5    168  -> 156    130  -> 122
+//   64 x 64, 512            59.9 -> 56.0   61.8 -> 57.7   88.7 -> 65.8           46.5 -> 41.7   48.0 -> 43.1    45.3 -> 45.0   47.1 -> 46.4
+//   2 x 2048, 512           580  -> 492    401  -> 342    613  -> 509            436  -> 369    304  -> 259     443  -> 428    310  -> 298
+//   4 x 4096, 512           2725 -> 2425   1660 -> 1485   2 x 8192, 512  4430 -> 4140   2710 -> 2530
+//   2 x 2048, 64            375  -> 357    269  -> 255    4 x 4096, 64   1960 -> 1920   1260 -> 1220   2 x 8192, 64  3650 -> 3620   2300 -> 2260
+// Errors against 64 bits are no larger (of the output's norm, before and here: 1 x 512 3.66e-7 and 3.61e-7, 1 x 2048 5.35e-7 and 5.16e-7, 1 x 4096 with a
+// reach of 64 7.19e-7 and 6.88e-7).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -167,8 +178,9 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
   };
   // V[8 q + 4 g + e][32 d + li], element v = 4 q + e of block d: chunk 8 d + li / 4 of a row whose slots are swapped by halves where its bit 2 is set
   const uint32_t v_lane = (uint32_t)(4 * g * kRow + (((li >> 2) ^ (8 * g)) * 16) + (li & 3) * 4);
+  auto v_row = [](int v) { return (uint32_t)((8 * (v >> 2) + (v & 3)) * kRow); };
   auto v_elem = [&](int par, int d, int v) __attribute__((always_inline)) {
-    return *(LDS_AS const float*)(uintptr_t)(Vs + par * kTile + (v_lane ^ (128 * d)) + (8 * (v >> 2) + (v & 3)) * kRow);
+    return *(LDS_AS const float*)(uintptr_t)(Vs + par * kTile + (v_lane ^ (128 * d)) + v_row(v));
   };
   // Scratch: row li = this lane's query; the block a step contracts goes to the half of the step's parity, element (jj, li) wants column
   // (32 par + li + 32 - jj) mod 64.  The four of jj = 8 q + 4 g + 0 .. 3 are the run that ends there for jj = 8 q + 4 g; columns 64 .. 67 repeat 0 .. 3.
@@ -218,82 +230,12 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
     }
   };
 
-  auto step = [&](auto far_tag, auto par_tag, int k) __attribute__((always_inline)) {
-    constexpr bool FAR = decltype(far_tag)::value;
-    constexpr int PAR = decltype(par_tag)::value;
-    const int s = FAR ? far_step_at(k) : s0 + k, j0 = s * kStep;
-    wait_vmcnt<0>();   // this wave's direct loads of the step before, and the table values
-    if constexpr (!FAR) asm volatile("" : "+v"(dnext[0]), "+v"(dnext[1]));   // (taken here: the compiler does not count the direct loads)
-    __syncthreads();   // ... and everybody's; every wave is done with what this step's loads overwrite
-    kv_dma(FAR ? far_step_at(k + 1) : s + 1, PAR ^ 1);   // past the last step, too: rows and table indices are clamped, nobody reads it
-    if constexpr (!FAR) {
-      batch_dma(dnext, slot_dma);   // batch k + 5 in place of batch k
-      __builtin_amdgcn_sched_barrier(0);
-      batch_delta(dnext);           // of batch k + 6
-    }
-    const Operand kf = lds_rows(Ks + PAR * kTile, k_lane);
-    f32x16 sacc, cnew, p0, p1;
-    float px[16], cb[16], vr[2][16];
-    if constexpr (FAR) {
-#pragma unroll
-      for (int n = 0; n < 32; ++n) {
-        sacc = mma1(kf, qx, n, n == 0 ? zero : sacc);
-        vr[n >> 4][n & 15] = v_elem(PAR, n >> 4, n & 15);
-      }
-    } else {
-      Operand ac;
-      if constexpr (C2P) ac = lds_rows(EK + slot_rd * kTile, e_lane);
-      if constexpr (P2C) {
-        aq[PAR] = lds_rows(EQ + slot_rd * kTile, e_lane);
-#pragma unroll
-        for (int n = 0; n < 32; ++n) p1 = mma1(kf, aq[PAR ^ 1], n, n == 0 ? zero : p1);
-      }
-      if constexpr (C2P) {
-#pragma unroll
-        for (int n = 0; n < 32; ++n) cnew = mma1(ac, qf, n, n == 0 ? zero : cnew);
-      }
-      if constexpr (P2C) {
-#pragma unroll
-        for (int n = 0; n < 32; ++n) {
-          p0 = mma1(kf, aq[PAR], n, n == 0 ? zero : p0);
-          if constexpr (C2P) {
-            if (n >= 8 && n < 12) c_store(cnew, PAR, n - 8);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      if constexpr (C2P) {
-        if constexpr (!P2C) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) c_store(cnew, PAR, q);
-        }
-        wave_lds_fence();   // the LDS unit runs one wave's operations in order; this keeps the compiler from moving them
-      }
-#pragma unroll
-      for (int n = 0; n < 32; ++n) {
-        sacc = mma1(kf, qf, n, n == 0 ? zero : sacc);
-        if constexpr (C2P) {
-          if (n < 8) {
-#pragma unroll
-            for (int e = 2 * (n & 1); e < 2 * (n & 1) + 2; ++e) cb[4 * (n >> 1) + e] = *(LDS_AS const float*)(uintptr_t)(c_rd[PAR][n >> 1] + 4 * (3 - e));
-          }
-        }
-        if constexpr (P2C) {
-          if (n >= 2 && n < 18) {
-            const int v = n - 2, c = 8 * (v >> 2) + (v & 3);
-            px[v] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((int)p_from[v], __builtin_bit_cast(int, xl < 32 - c ? p1[v] : p0[v])));
-          }
-        }
-        vr[n >> 4][n & 15] = v_elem(PAR, n >> 4, n & 15);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        if constexpr (C2P) sacc[v] += cb[v];
-        if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v]);
-      }
-    }
-    // ---- mask, online soft-max in base 2, O^T += V^T P^T -----------------------------------------------------------------------------
+  // mask, online soft-max in base 2, O^T += V^T P^T: the scores of the keys from j0 on, to which `add` is still to be added, and their values.
+  // BY_SUM: a far step, whose products wait for its soft-max.  Its probabilities are formed against the reference point as it is, and their sum says whether
+  // that is high enough (a sum bounds its largest term); the maximum is looked for only where it is not.  A near step's maximum is found while its last
+  // products run.
+  auto absorb = [&](auto by_sum, f32x16& sacc, const float (&vr)[2][16], int j0, float add) __attribute__((always_inline)) {
+    constexpr bool BY_SUM = decltype(by_sum)::value;
     if (j0 + kStep > Lb || (p.causal && j0 + kStep - 1 > m0)) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
@@ -301,13 +243,13 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
         if (j >= Lb || (p.causal && j > i)) sacc[v] = -INFINITY;
       }
     }
-    const float add = FAR ? row_add : 0.f;
-    float mx = sacc[0];
+    auto row_max = [&]() __attribute__((always_inline)) {
+      float mx = sacc[0];
 #pragma unroll
-    for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
-    mx = wave_half_max(mx) + add;
-    if (__any(mx > m_run + kLazyTau)) {
-      const float m_new = mx > m_run + kLazyTau ? mx : m_run;
+      for (int v = 1; v < 16; ++v) mx = fmaxf(mx, sacc[v]);
+      return wave_half_max(mx) + add;
+    };
+    auto refer_to = [&](float m_new) __attribute__((always_inline)) {
       const float alpha = m_run == m_new ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
       m_run = m_new;
       l_run *= alpha;
@@ -315,17 +257,129 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
       for (int d = 0; d < 2; ++d)
 #pragma unroll
         for (int v = 0; v < 16; ++v) o_acc[d][v] *= alpha;
-    }
-    const float off = add - (m_run == -INFINITY ? 0.f : m_run);   // -inf: the row has met no key it sees (shares, the ends of a sequence)
+    };
     f32x8 pv[2];
+    auto probs = [&]() __attribute__((always_inline)) {
+      const float off = add - (m_run == -INFINITY ? 0.f : m_run);   // -inf: the row has met no key it sees (shares, the ends of a sequence)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) pv[v >> 3][v & 7] = __builtin_amdgcn_exp2f(sacc[v] + off);
-    l_run = sum8(pv[1], sum8(pv[0], l_run));
+      for (int v = 0; v < 16; ++v) pv[v >> 3][v & 7] = __builtin_amdgcn_exp2f(sacc[v] + off);
+    };
+    if constexpr (BY_SUM) {
+      probs();
+      float sum = sum8(pv[1], sum8(pv[0], 0.f));
+      const bool moves = m_run == -INFINITY || !(sum <= 256.f);   // 2^kLazyTau; also a sum that overflows
+      if (__any(moves)) {
+        const float m_new = fmaxf(m_run, row_max());
+        refer_to(wave_half_max(moves ? 1.f : 0.f) > 0.f ? m_new : m_run);   // a row's two lanes together
+        probs();
+        sum = sum8(pv[1], sum8(pv[0], 0.f));
+      }
+      l_run += sum;
+    } else {
+      const float mx = row_max();
+      if (__any(mx > m_run + kLazyTau)) refer_to(mx > m_run + kLazyTau ? mx : m_run);
+      probs();
+      l_run = sum8(pv[1], sum8(pv[0], l_run));
+    }
 #pragma unroll
     for (int v = 0; v < 16; ++v)
 #pragma unroll
       for (int d = 0; d < 2; ++d) o_acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[d][v], pv[v >> 3][v & 7], o_acc[d], 0, 0, 0);
-    if constexpr (FAR) return;
+  };
+
+  // A far step's K is in registers when it begins and its V when its scores are done, so the barrier that the next step's loads need comes
+  // there, and the next K is read and what follows it is loaded while this step's soft-max and products run.  The buffer is an address here and no
+  // constant: two forms of the step in one loop cost 64 moves of the sums between them.  With a step's barrier and reads ahead of its products and a maximum
+  // ahead of its exponentials, far steps lost to the kernel before them: 2 x 8192 with a reach of 64 3650 us there, 3970 so, 3780 without the former, 3620 without both.
+  Operand kf_far;
+  auto far_begins = [&](int t) __attribute__((always_inline)) {   // step t's K and V are there; those of t + 1 are asked for
+    wait_vmcnt<0>();
+    __syncthreads();
+    kv_dma(far_step_at(t + 1), (t & 1) ^ 1);
+    kf_far = lds_rows(Ks + (t & 1) * kTile, k_lane);
+  };
+  auto far_step = [&](int t) __attribute__((always_inline)) {
+    f32x16 sacc;
+    float vr[2][16];
+    uint32_t v_at[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      v_at[d] = Vs + (t & 1) * kTile + (v_lane ^ (128 * d));
+      asm("" : "+v"(v_at[d]));   // the constant part of the address belongs into the instruction
+    }
+#pragma unroll
+    for (int n = 0; n < 32; ++n) {
+      sacc = mma1(kf_far, qx, n, n == 0 ? zero : sacc);
+      vr[n >> 4][n & 15] = *(LDS_AS const float*)(uintptr_t)(v_at[n >> 4] + v_row(n & 15));
+    }
+    far_begins(t + 1);   // (after the last one, too: the first near step's, and once more in the other buffer, which that step's loads take over)
+    absorb(std::true_type{}, sacc, vr, far_step_at(t) * kStep, row_add);
+  };
+  auto step = [&](auto par_tag, int k) __attribute__((always_inline)) {
+    constexpr int PAR = decltype(par_tag)::value;
+    const int s = s0 + k, j0 = s * kStep;
+    wait_vmcnt<0>();   // this wave's direct loads of the step before, and the table values
+    asm volatile("" : "+v"(dnext[0]), "+v"(dnext[1]));   // (taken here: the compiler does not count the direct loads)
+    __syncthreads();   // ... and everybody's; every wave is done with what this step's loads overwrite
+    kv_dma(s + 1, PAR ^ 1);   // past the last step, too: rows and table indices are clamped, nobody reads it
+    batch_dma(dnext, slot_dma);   // batch k + 5 in place of batch k
+    __builtin_amdgcn_sched_barrier(0);
+    batch_delta(dnext);           // of batch k + 6
+    const Operand kf = lds_rows(Ks + PAR * kTile, k_lane);
+    f32x16 sacc, cnew, p0, p1;
+    float px[16], cb[16], vr[2][16];
+    Operand ac;
+    if constexpr (C2P) ac = lds_rows(EK + slot_rd * kTile, e_lane);
+    if constexpr (P2C) {
+      aq[PAR] = lds_rows(EQ + slot_rd * kTile, e_lane);
+#pragma unroll
+      for (int n = 0; n < 32; ++n) p1 = mma1(kf, aq[PAR ^ 1], n, n == 0 ? zero : p1);
+    }
+    if constexpr (C2P) {
+#pragma unroll
+      for (int n = 0; n < 32; ++n) cnew = mma1(ac, qf, n, n == 0 ? zero : cnew);
+    }
+    if constexpr (P2C) {
+#pragma unroll
+      for (int n = 0; n < 32; ++n) {
+        p0 = mma1(kf, aq[PAR], n, n == 0 ? zero : p0);
+        if constexpr (C2P) {
+          if (n >= 8 && n < 12) c_store(cnew, PAR, n - 8);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (C2P) {
+      if constexpr (!P2C) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) c_store(cnew, PAR, q);
+      }
+      wave_lds_fence();   // the LDS unit runs one wave's operations in order; this keeps the compiler from moving them
+    }
+#pragma unroll
+    for (int n = 0; n < 32; ++n) {
+      sacc = mma1(kf, qf, n, n == 0 ? zero : sacc);
+      if constexpr (C2P) {
+        if (n < 8) {
+#pragma unroll
+          for (int e = 2 * (n & 1); e < 2 * (n & 1) + 2; ++e) cb[4 * (n >> 1) + e] = *(LDS_AS const float*)(uintptr_t)(c_rd[PAR][n >> 1] + 4 * (3 - e));
+        }
+      }
+      if constexpr (P2C) {
+        if (n >= 2 && n < 18) {
+          const int v = n - 2, c = 8 * (v >> 2) + (v & 3);
+          px[v] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((int)p_from[v], __builtin_bit_cast(int, xl < 32 - c ? p1[v] : p0[v])));
+        }
+      }
+      vr[n >> 4][n & 15] = v_elem(PAR, n >> 4, n & 15);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      if constexpr (C2P) sacc[v] += cb[v];
+      if constexpr (P2C) sacc[v] = __builtin_fmaf(px[v], x_scale, sacc[v]);
+    }
+    absorb(std::false_type{}, sacc, vr, j0, 0.f);
     slot_rd = slot_rd == kBatches - 1 ? 0 : slot_rd + 1;
     slot_dma = slot_dma == kBatches - 1 ? 0 : slot_dma + 1;
   };
@@ -342,17 +396,16 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
       for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
       dnext[0] = d0[5][0], dnext[1] = d0[5][1];
     }
-    using Y = std::true_type;
-    using N = std::false_type;
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
     if (n_far > 0) {
-      side_begins(n_left > 0 ? 0 : 1);
+      far_begins(-n_far);
 #pragma unroll 1
-      for (int t = -n_far; t < 0; ++t) {   // K and V through the two buffers so that the first near step finds its own in buffer 0
-        if (t == -n_right && n_left > 0) side_begins(1);
-        if (t & 1) step(Y{}, T1{}, t);
-        else step(Y{}, T0{}, t);
+      for (int side = n_left > 0 ? 0 : 1, t = -n_far; t < 0; ++side) {   // K and V through the two buffers so that the first near step finds its own in buffer 0
+        side_begins(side);
+        const int last = side == 0 ? -n_right : 0;
+#pragma unroll 1
+        for (; t < last; ++t) far_step(t);
       }
     }
     if (n_steps > 0) {
@@ -370,10 +423,10 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
       int k = 0;
 #pragma unroll 1
       for (; k + 1 < n_steps; k += 2) {
-        step(N{}, T0{}, k);
-        step(N{}, T1{}, k + 1);
+        step(T0{}, k);
+        step(T1{}, k + 1);
       }
-      if (k < n_steps) step(N{}, T0{}, k);
+      if (k < n_steps) step(T0{}, k);
     }
     wait_vmcnt<0>();  // the last step's direct loads: none may still be writing LDS when the workgroup ends
   }

@@ -63,3 +63,23 @@ def test_rows_without_a_soft_max(shares):
     k[0, :, :, 0] = -float("inf")
     out, lse = [t.cpu() for t in call(q, k, v, pk)]
     assert out.isnan().all() and lse.isnan().all()
+
+
+@pytest.mark.parametrize("rise", [1, -1])
+@pytest.mark.parametrize("L,terms,causal,shares", [(700, BOTH, False, 1), (641, C2P, False, 3), (993, P2C, False, 2), (900, BOTH, True, 0), (193, BOTH, False, 1)])
+def test_scores_that_rise_through_the_far_steps(L, terms, causal, shares, rise):
+    """A far step finds its reference point too low by the sum of its probabilities: scores that rise by 60 towards either end, by jumps and slowly."""
+    q, k, v, pk, pq = x = _inputs(1, L, 2, 32, terms)
+    j = torch.arange(L)
+    height = (j if rise > 0 else L - 1 - j) / L
+    q[..., 0], k[..., 0] = 3.0, (torch.where(j % 64 < 32, height, (height * 6).floor() / 6) * 20.0 * (64.0 * (1 + sum(terms))) ** 0.5)[None, :, None]
+    q[0, 5] = 0.0   # a row that sees none of it
+    for t in (pk, pq):
+        if t is not None:
+            t[..., 0] = 0.0
+    ref, ref_lse = _oracle(*x, 32, 64, causal=causal)
+    out, lse = ops.disentangled_attention_fwd(*[None if t is None else t.cuda() for t in x], position_buckets=32, max_relative_positions=64, causal=causal, return_lse=True,
+                                              far_splits=shares)
+    # a score of 60 carries 2^-24 of itself from each of some ten sums that are as large: 4e-5 of a probability, and as much of lse
+    assert np.abs(out.cpu().numpy() - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
+    assert np.abs(lse.view(1, L, 2).cpu().numpy() - ref_lse).max() <= 1e-4
