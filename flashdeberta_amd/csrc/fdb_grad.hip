@@ -323,17 +323,27 @@ int launch_dgrad(DgradParams p, hipStream_t stream) {
   hipLaunchKernelGGL(kern, dim3(p.tiles[0] + p.tiles[1]), dim3(64 * S::NW), S::LDS, stream, p);
   return (int)hipGetLastError();
 }
-// Eight waves a tile: a stage is 0.35 us of latency and barrier for a workgroup that has its CU to itself, and half of it for two that share one, so
-// a tile of 64 rows while each has a CU (four waves, us: 12 heads, 1000 tokens 16.5 -> 14.5, 16 heads, 300 tokens 20.6 -> 18.1), then one of 128 while
-// that is so, four stages deep (64 rows, two workgroups a CU: 12 heads, 4096 tokens 22.2 -> 21.1, 3000 tokens 21.0 -> 20.1; 16 heads, 2048 tokens 26.3 -> 25.5),
-// then two of 128 a CU (four waves: 12 heads, 6000 tokens 30.1 -> 29.2, 8192 34.2 -> 33.4, 16 heads, 4096 tokens 38.2 -> 35.5; 256 rows by eight waves 42.5).
+// Eight waves a tile where it has its CU to itself: a stage is 0.35 us of latency and barrier for such a workgroup, and half of it for two that share one; four
+// waves a tile where two share a CU, the matrix cores are busy and a wave's operands serve more products.  Whole launches, replayed, bf16, 512 table rows, us:
+//   tiles of 64 (128) rows      64 x 8 waves   64 x 4   128 x 8, four stages   128 x 8, two a CU   128 x 4
+//   12 heads,  1024 tokens  144 (72)   19.1*   21.2   24.4    29.0    29.2      16 heads, 1600   264 (136)  29.4   28.1*  30.1   36.4   36.8
+//              2500         288 (144)  24.3    23.8*  24.8    28.9    29.2      24 heads, 1024   288 (144)  43.9   36.9*  40.8   51.2   51.8
+//              3000         330 (168)  26.6    26.9   24.9*   29.1    29.4      16 heads, 2048   320 (160)  33.3   30.4   30.2*  36.4   36.9
+//              4096         432 (216)  27.2    27.0   25.2*   29.7    30.1      24 heads, 2048   480 (240)  52.8   50.4   42.7*  51.6   52.3
+//              6144         624 (312)  38.1    40.0   43.3    32.2*   33.8      16 heads, 5000   696 (352)  49.8   51.9   54.6   41.9*  42.6
+//              8192         816 (408)  45.0    43.5   43.6    35.8    36.1*     24 heads, 3500   756 (384)  75.4   75.3   77.1   63.3   61.1*
+//              20000       1926 (966)  88.2    85.5   83.2    73.2    70.3*     16 heads, 7000   944 (472)  62.4   59.3   55.3   49.7   48.2*
+//              16384       1584 (792)  78.6    79.3   81.7    65.0    64.1*     24 heads, 8192  1632 (816)   165    159    151    128    118*
 // Waves that lie across the 128 columns (2 x 4) where x is the shorter side, along the rows where it is not (the other way round: 16.8 and 22.0 us).
 template <class QT>
 int launch_dgrad_rows(const DgradParams& p, hipStream_t stream) {
+  const int64_t cus = fdb_cu_count();
   auto tiles = [&](int rows) { return (int64_t)(tiles_of(p.rows[0], rows) + tiles_of(p.rows[1], rows)) * tiles_of(p.cols, 128); };
-  if (tiles(64) <= fdb_cu_count()) return launch_dgrad<QT, DShape<64, 2, 4, 3, 2>>(p, stream);
-  if (tiles(128) <= fdb_cu_count()) return launch_dgrad<QT, DShape<128, 4, 2, 4, 1>>(p, stream);
-  return launch_dgrad<QT, DShape<128, 4, 2, 2, 2>>(p, stream);
+  if (tiles(64) <= cus) return launch_dgrad<QT, DShape<64, 2, 4, 3, 2>>(p, stream);
+  if (tiles(64) * 8 <= cus * 9) return launch_dgrad<QT, DShape<64, 2, 2, 3, 2>>(p, stream);   // few CUs have two
+  if (tiles(128) <= cus) return launch_dgrad<QT, DShape<128, 4, 2, 4, 1>>(p, stream);
+  if (tiles(128) * 2 < cus * 3) return launch_dgrad<QT, DShape<128, 4, 2, 2, 2>>(p, stream);   // most CUs have one
+  return launch_dgrad<QT, DShape<128, 2, 2, 2, 2>>(p, stream);
 }
 
 template <class QT>
@@ -362,8 +372,10 @@ int fdb_wgrad_shares(int64_t rows, int64_t x_cols, int64_t y_cols) {
   return (int)std::max<int64_t>(1, std::min<int64_t>({2 * fdb_cu_count() / tiles, stages / 6, 16}));
 }
 
-// Where one launch beats a library product each: unless a second round of workgroups is mostly empty (16 heads, 8192 tokens: 544 tiles,
-// 70.1 us against 58.5; 12 heads, 408 tiles, 31.0 against 43.9).
+// Where one launch beats a library product each: unless a second round of workgroups, or the last of more, is mostly empty.  Tiles, this and the library
+// (torch.mm of each), us: 16 heads 512 50.3 and 61 | 544 75.2 and 64.3 | 664 75.8 and 71.5 | 912 87.0 and 87.5 | 1056 115 and 94.3 | 1288 123 and 127;
+// 12 heads 498 39.5 and 50.1 | 600 58.9 and 55.2 | 792 64.1 and 66.5 | 966 70.3 and 72.5; 24 heads 528 108 and 87 | 816 118 and 116 | 996 132 and 129 |
+// 1200 171 and 175 | 1368 183 and 191.  (600 tiles at 16 heads, 75.6 and 84, and 1584 at 24, 230 and 214, fall on the wrong side.)
 extern "C" int32_t fdb_dgrad_serves(int64_t rows0, int64_t rows1, int64_t cols) {
   const int64_t tiles = (tiles_of(rows0, 128) + tiles_of(rows1, 128)) * (int64_t)tiles_of(cols, 128), places = 2 * fdb_cu_count(), rounds = (tiles + places - 1) / places;
   return 4 * tiles >= 3 * places * rounds || rounds == 1;

@@ -19,7 +19,8 @@ def _close(got, ref, scale, dtype, what):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("rows,depth,cols", [((1, 0), (64, 64), 64), ((0, 65), (64, 128), 128), ((64, 63), (192, 128), 192), ((200, 129), (320, 64), 448), ((1000, 512), (2304, 1536), 768),
-                                             ((5500, 130), (64, 128), 768)])   # the last: tiles of 128 rows
+                                             ((5500, 130), (64, 128), 768), ((9000, 65), (64, 192), 768),   # tiles of 128 rows: most compute units have one, most have two
+                                             ((2700, 129), (128, 64), 768), ((2497, 0), (64, 64), 832)])   # tiles of 64 rows: a few compute units have two
 def test_dgrad(rows, depth, cols, dtype):
     g = torch.Generator(device="cuda").manual_seed(sum(rows))
     w = torch.randn(max(depth), cols, device="cuda", generator=g).to(dtype)
