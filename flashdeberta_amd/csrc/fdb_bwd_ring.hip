@@ -711,8 +711,8 @@ __global__ __launch_bounds__(kThreads, 2) void fdb_bwd_both_kernel(const FdbBwdR
 }
 
 // The places of both roles' workgroups of a padded batch (fdb_deals_by_length), batch rows x 2 of them by this workgroup, the `at`-th of tiles * heads.  The order
-// is padded_map's, or block_map's where the mask hides little.  together: one launch, both roles of a tile's heads one after the other, the short texts of both end it;
-// otherwise dQ's places, then the others.
+// is padded_map's, or block_map's where the mask hides little.  together: one launch, the roles take turns of 64, the short texts of both end it; otherwise dQ's
+// places, then the others.
 // A table, because the roles have no registers to spare: with padded_map at its start the dQ role spilt 19 instead of 14 and took 705 us instead of 640 (8 x 3000).
 __device__ __forceinline__ void find_places(const FdbBwdRingParams& p, int at, bool together) {
   __shared__ int first[64], tokens[64], sorted[64], row[64], dealt;
@@ -749,30 +749,48 @@ __device__ __forceinline__ void find_places(const FdbBwdRingParams& p, int at, b
     }
     return;
   }
-  int u = n / heads, t = p.tiles - 1, here = 0;
-  const int h = n - u * heads;
-  for (; t >= 0; --t) {   // `here` sequences have tokens in tile t
-    while (here < batch && sorted[here] > t * (FDB_BM / 32)) ++here;
-    if (u < here) break;
-    u -= here;
+  const int unit = 64, part = n / unit, at_unit = n - part * unit, in_part = min(unit, all - part * unit);
+  const int slot_keys = together ? 2 * part * unit + at_unit : all + n, slot_dq = together ? slot_keys + in_part : n;
+  int real = 0;
+  for (int x = 0; x < batch; ++x) real += (sorted[x] + FDB_BM / 32 - 1) / (FDB_BM / 32);
+  int u = n < real * heads ? n : ~(n - real * heads);
+  if (u >= 0 && !p.causal) {
+    int ahead = 0, here = 0, of_class = p.tiles;
+    for (;; --of_class) {   // `here` sequences of that many tiles
+      for (here = 0; ahead + here < batch && sorted[ahead + here] > (of_class - 1) * (FDB_BM / 32);) ++here;
+      if (u < here * of_class * heads) break;
+      u -= here * of_class * heads;
+      ahead += here;
+    }
+#pragma unroll
+    for (int keys = 0; keys < 2; ++keys) {
+      int x, t, h;
+      block_place(u, here, heads, of_class, groups_of(of_class), order_of(p, keys == 0), x, t, h);
+      put(keys ? slot_keys : slot_dq, row[ahead + x], t, h, keys != 0);
+    }
+    return;
   }
-  int t_keys = t;
-  if (t < 0) {   // padding
-    for (t = 0; t < p.tiles; ++t) {
+  const bool padding = u < 0;
+  if (padding) u = ~u;
+  const int pair = u / heads, h = u - pair * heads;
+  u = pair;
+  int t, here = padding ? batch : 0;
+  for (t = padding ? 0 : p.tiles - 1;; t += padding ? 1 : -1) {
+    if (padding) {
       while (here > 0 && sorted[here - 1] <= t * (FDB_BM / 32)) --here;
       if (u < batch - here) break;
       u -= batch - here;
+    } else {
+      while (here < batch && sorted[here] > t * (FDB_BM / 32)) ++here;
+      if (u < here) break;
+      u -= here;
     }
-    u += here;
-    t_keys = t;
-  } else if (p.causal) {
-    // The queries of a key tile are those from its own to the end of the text, as many as the mirrored query tile has keys.  Backward, highest key tile first ->
-    // mirrored (the plain order): 8 x 1024 192 -> 170 us (175), 8 x 2048 328 -> 290 (330), 4 x 4096 with 16 heads 715 -> 613 (641), 48 x 384 204 -> 210 (223).
-    t_keys = (sorted[u] - 1) / (FDB_BM / 32) - t;
   }
-  const int b = row[u], pair = n / heads * 2 * heads + h;
-  put(together ? pair : all + n, b, t_keys, h, true);
-  put(together ? pair + heads : n, b, t, h, false);
+  if (padding) u += here;
+  // Causal: the queries of a key tile are those from its own to the end of the text, as many as the mirrored query tile has keys.  Backward, highest key tile first ->
+  // mirrored (the plain order): 8 x 1024 192 -> 170 us (175), 8 x 2048 328 -> 290 (330), 4 x 4096 with 16 heads 715 -> 613 (641), 48 x 384 204 -> 210 (223).
+  put(slot_keys, row[u], padding ? t : (sorted[u] - 1) / (FDB_BM / 32) - t, h, true);
+  put(slot_dq, row[u], t, h, false);
 }
 
 // The row statistics by themselves: -lse in base 2 and -Delta = -(dO . O), 128 rows a workgroup, two lanes a row that add up in the dQ

@@ -312,24 +312,28 @@ __device__ __forceinline__ bool padded_batch_deals(int mine, int batch, int most
 // Linear workgroup id -> (batch row, query tile, head) of a padded batch (host: fdb_deals_by_length), with the row's first token and its length as the call gives it;
 // false: block_map's order is the one to take.  The dispatcher takes workgroups in order and waits
 // for a place where the next one belongs: a workgroup without tokens among the first leaves a place that stays empty, and one of a long text
-// among the last makes the launch end late.  So the tiles with tokens come first, the highest tile of all sequences before the next lower one and in
-// each the longest sequence first; a launch ends on the shortest texts, and on the tiles of padding, which are only cleared.  All heads of a tile
-// are dealt before the next.
-// Lengths between a quarter and all in no order, 12 heads, bf16, us, block_map -> here (two draws where they differ in sign):
-//   forward   32 x 128 12.8 -> 11.5   64 x 256 48.4 -> 45.9   8 x 512 28.8 -> 22.0, 29.6 -> 30.0   64 x 512 124 -> 112   8 x 1024 78.0 -> 60.8   8 x 2048 166 -> 149
-//             4 x 4096 263 -> 253, 232 -> 242   8 x 4096 439 -> 383   4 x 8192 749 -> 713   16 heads 4 x 2048 111 -> 116, 118 -> 108   2 x 8192 528 -> 508
-//             fp32 8 x 512 138 -> 94   head_dim 128 8 x 2048 371 -> 257   e4m3 8 x 2048 138 -> 127   causal 8 x 384, 16 heads 18.8 -> 19.7   8 x 1024 68.5 -> 50.4
-//   backward  32 x 128 124 -> 118   64 x 256 206 -> 196   8 x 512 99.5 -> 79.1   64 x 512 551 -> 490   8 x 1024 238 -> 208   8 x 2048 558 -> 516
-//             8 x 4096 1604 -> 1393   4 x 8192 2806 -> 2564   16 heads 4 x 2048 379 -> 393, 394 -> 357   2 x 8192 2266 -> 2378
-//   causal, both roles and the rest of the backward, the key tiles mirrored (find_places)   8 x 512 92 -> 87   8 x 1024 175 -> 170   8 x 2048 355 -> 325   32 x 256 104.5 -> 103
-//             48 x 384 234 -> 217   32 x 1024 578 -> 534   16 heads 4 x 4096 641 -> 613   2 x 8192 1342 -> 1343   causal forward 16 x 512 36.3 -> 32.7   8 x 2048 122 -> 101
-// One sequence of 64 long and the others a quarter of it, mostly padding: forward 64 x 128 14.2 -> 15.6, 64 x 512 37.9 -> 39.3, 32 x 1024 60.6 -> 52.1.
-// Where a mask hides little, the order gives up the heads' places on the XCDs for nothing: lengths all the same, forward 64 x 512 165 -> 172, 8 x 4096 609 -> 679,
-// backward 32 x 1024 1140 -> 1211, 16 x 4096 4564 -> 5102; of three quarters to all between -7 and +7 %.  So it takes a quarter of the sequences to leave a quarter empty.
-// Every wave finds its place itself, a lane a sequence: how many of the tiles at hand have tokens is a count of lanes,
+// among the last makes the launch end late.  So the tiles with tokens come first: of the sequences with the most tiles, then of those with one less, each such class
+// dealt as block_map deals a batch of that many tiles, so that a head's tiles share an XCD and few heads are under way at a time.  A launch ends on the shortest texts, and
+// on the tiles of padding, which are only cleared, by heads.  Under a causal mask the highest tile has the most keys: there the highest tile of all sequences comes
+// before the next lower one, in each the longest sequence first (by classes 8 x 2048 forward 101 -> 110 us, 8 x 1024 backward 170 -> 189).
+// bf16, us, block_map -> here; ragged: lengths of a quarter to all in no order; one: one text of the full length, the others a quarter of it; half: all half:
+//   forward   ragged  12 heads 32 x 128 13.6 -> 11.9   64 x 256 48.4 -> 45.9   17 x 512 47.2 -> 41.5   25 x 512 58.5 -> 48.7   64 x 512 124 -> 110   7 x 1024 69.6 -> 61.0
+//                     8 x 2048 168 -> 145   4 x 4096 230 -> 220   4 x 8192 814 -> 723   16 heads 14 x 512 31.5 -> 28.3   8 x 512 30.1 -> 30.7   7 x 640 35.4 -> 37.6   2 x 4096 203 -> 196
+//             one     64 x 128 18.2 -> 16.2   48 x 256 22.9 -> 18.0   64 x 512 50.1 -> 39.6   7 x 2048 91.5 -> 74.4   4 x 8192 461 -> 367   16 heads 2 x 8192 413 -> 396
+//             half    64 x 64 12.6 -> 12.6   64 x 512 63 -> 66   32 x 1024 94 -> 97 (the clearing of 25 MB and 50 ends the launch)   8 x 2048 116 -> 96   4 x 8192 546 -> 348
+//             fp32 8 x 512 138 -> 94   head_dim 128 8 x 2048 371 -> 257   e4m3 8 x 2048 138 -> 127   (these three before the classes)   causal 16 x 512 36.3 -> 32.7   8 x 2048 122 -> 101
+//   backward  (all launches of it)  ragged  12 heads 17 x 512 220 -> 162   25 x 512 242 -> 200   7 x 1024 243 -> 211   8 x 2048 558 -> 505   4 x 8192 3130 -> 2730   16 heads 2 x 4096 654 -> 653
+//             one     8 x 1024 169 -> 107   7 x 2048 261 -> 200   4 x 4096 572 -> 436   16 heads 2 x 8192 1476 -> 1463   half  64 x 512 323 -> 306   4 x 4096 503 -> 433
+//             causal  8 x 512 92 -> 87   8 x 1024 175 -> 170   8 x 2048 355 -> 325   32 x 1024 578 -> 534   16 heads 4 x 4096 641 -> 613   2 x 8192 1342 -> 1343
+// The highest tile first without a mask, too, gave up a head's place on an XCD: one, 16 heads 2 x 8192 forward 432, backward 1600; ragged 4 x 4096 240.  Tiles of padding in
+// turns of eight with the others leave the places of an XCD unevenly filled (half 64 x 512 107), ahead of all others they hold those up (69).
+// Where a mask hides little, an order by lengths gives up block_map's balance for nothing: of three quarters to all it was between -7 and +7 %, highest tile first.
+// So it takes a quarter of the sequences to leave a quarter empty.
+// Every wave finds its place itself, a lane a sequence: how many sequences have a number of tiles is a count of lanes,
 // the length of the sequence with a given rank, in blocks of 32 tokens, is found bit by bit.
-__device__ __forceinline__ bool padded_map(int n, const int32_t* start, const int32_t* length, int batch, int heads, int tiles_per_seq, int most, int lane, int& b_out,
-                                           int& t_out, int& h_out, int& tok0_out, int& len_out) {
+__device__ __forceinline__ int groups_of(int tiles) { return 8 * (tiles < 96 ? (int)(96u / (uint32_t)tiles) : 1); }   // fdb_groups_together
+__device__ __forceinline__ bool padded_map(int n, const int32_t* start, const int32_t* length, int batch, int heads, int tiles_per_seq, int most, int order, bool causal,
+                                           int lane, int& b_out, int& t_out, int& h_out, int& tok0_out, int& len_out) {
   int first = 0, len = 0, mine = 0;   // this lane's sequence
   if (lane < batch) {
     if (start) first = min(max(start[lane], 0), most);
@@ -337,36 +341,50 @@ __device__ __forceinline__ bool padded_map(int n, const int32_t* start, const in
     mine = min(max(len, 0), most - first);
   }
   if (!padded_batch_deals(mine, batch, most, lane)) return false;
-  const int blocks = (mine + 31) >> 5;
-  int u = (int)((uint32_t)n / (uint32_t)heads);
-  const int h = n - u * heads;
-  int t = tiles_per_seq - 1, rank = -1;
-  for (; t >= 0; --t) {
-    const int here = __popcll(__ballot(blocks > t * (FDB_BM / 32)));
-    if (u < here) {
-      rank = u;
-      break;
+  const int blocks = (mine + 31) >> 5, tiles = (mine + FDB_BM - 1) / FDB_BM;   // (none beyond the batch)
+  int all = 0;   // with tokens
+  for (int bit = 0; (tiles_per_seq >> bit) != 0; ++bit) all += __popcll(__ballot((tiles >> bit) & 1)) << bit;
+  all *= heads;
+  int u = n < all ? n : ~(n - all);
+  int rank, t, h;
+  if (u < 0 || causal || tiles_per_seq == 1) {   // all heads of a tile after the other
+    const bool padding = u < 0;
+    u = padding ? ~u : u;
+    const int pair = (int)((uint32_t)u / (uint32_t)heads);
+    h = u - pair * heads;
+    u = pair;
+    int here;
+    for (t = padding ? 0 : tiles_per_seq - 1;; t += padding ? 1 : -1) {
+      here = __popcll(__ballot(tiles > t));
+      const int those = padding ? batch - here : here;
+      if (u < those) break;
+      u -= those;
     }
-    u -= here;
-  }
-  if (rank < 0) {   // padding
-    for (t = 0; t < tiles_per_seq; ++t) {
-      const int here = __popcll(__ballot(blocks > t * (FDB_BM / 32)));
-      if (u < batch - here) {
-        rank = here + u;
-        break;
-      }
-      u -= batch - here;
+    rank = padding ? here + u : u;
+  } else {
+    int here, ahead = 0, of_class = tiles_per_seq;   // the sequences of that many tiles
+    for (;; --of_class) {
+      here = __popcll(__ballot(tiles == of_class));
+      const int those = here * of_class * heads;
+      if (u < those) break;
+      u -= those;
+      ahead += here;
     }
+    block_place(u, here, heads, of_class, groups_of(of_class), order, rank, t, h);
+    rank = __builtin_amdgcn_readfirstlane(rank) + ahead;
   }
   int of = 0;   // the length of that rank: the largest that more than `rank` sequences reach
   for (int bit = 31 - __builtin_clz((most + 31) >> 5); bit >= 0; --bit) {
     const int x = of | (1 << bit);
     if (__popcll(__ballot(blocks >= x)) > rank) of = x;
   }
-  uint64_t same = __ballot(lane < batch && blocks == of);
-  for (int before = rank - __popcll(__ballot(blocks > of)); before > 0; --before) same &= same - 1;
-  const int b = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)same) - 1);
+  // of the sequences of that length, the one with as many ahead of it as are still to be skipped (the counts by all lanes, ahead of any condition)
+  const bool same = lane < batch && blocks == of;
+  const uint64_t same_lanes = __ballot(same);
+  const int skip = rank - __popcll(__ballot(blocks > of));
+  const int ahead_of_me = __builtin_amdgcn_mbcnt_hi((uint32_t)(same_lanes >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same_lanes, 0u));
+  const uint64_t it = __ballot(same && ahead_of_me == skip);
+  const int b = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)it) - 1);
   b_out = b;
   t_out = __builtin_amdgcn_readfirstlane(t);
   h_out = __builtin_amdgcn_readfirstlane(h);
@@ -378,7 +396,7 @@ __device__ __forceinline__ bool padded_map(int n, const int32_t* start, const in
 // (negative: a batch row the caller could not express, NaN throughout).
 template <class Params>
 __device__ __forceinline__ void place_of(int n, const Params& p, int tiles_per_seq, bool fixed, int order, int lane, int& b, int& t, int& h, int& tok0, int& len) {
-  if (p.by_length && padded_map(n, p.seq_start, p.seq_len, p.B, p.H, tiles_per_seq, p.L, lane, b, t, h, tok0, len)) return;
+  if (p.by_length && padded_map(n, p.seq_start, p.seq_len, p.B, p.H, tiles_per_seq, p.L, order, p.causal != 0, lane, b, t, h, tok0, len)) return;
   block_map(n, p.B, p.H, tiles_per_seq, p.groups_together, fixed, order, b, t, h);
   tok0 = fixed && p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   len = fixed && p.seq_len ? p.seq_len[b] : p.L;

@@ -59,6 +59,35 @@ def test_bits_of_the_plain_order(B, L, H, dtype, kind, causal):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("kind", ["ragged", "left", "odd"])
+@pytest.mark.parametrize("B,L,H,D,dtype,more", [
+    (12, 400, 10, 32, torch.bfloat16, {}), (10, 900, 6, 32, torch.float16, {}), (9, 800, 7, 32, torch.bfloat16, dict(causal=True)),   # near launch alone, and with a far one
+    (20, 300, 8, 128, torch.bfloat16, {}), (9, 700, 8, 128, torch.float16, dict(causal=True)), (30, 200, 8, 128, torch.float32, {}), (20, 260, 8, 32, torch.float32, dict(causal=True)),
+    (14, 500, 8, 64, torch.float16, dict(single_kernel=True)), (14, 500, 8, 64, torch.float32, dict(causal=True)),
+    (20, 380, 8, 64, "e4m3", {}), (12, 1100, 5, 64, "e4m3", {}), (12, 1000, 5, 64, "e4m3", dict(causal=True)), (12, 500, 9, 128, "e4m3", {})])
+def test_bits_of_the_plain_order_in_every_kernel(B, L, H, D, dtype, more, kind):
+    """The forward of the other head_dims, types and launches."""
+    fp8 = dtype == "e4m3"
+    g = torch.Generator(device="cuda").manual_seed(B + L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).to(torch.bfloat16 if fp8 else dtype)
+    q, k, v, pk, pq = rnd(B, L, H, D), rnd(B, L, H, D), rnd(B, L, H, D), rnd(H, 64, D), rnd(H, 64, D)
+    kw = dict(position_buckets=32, max_relative_positions=64, return_lse=not more.get("single_kernel"), **more)
+    if fp8:
+        q, kw["q_scale"], k, kw["k_scale"] = ops.quantize_e4m3_per_head_pair(q, k)
+        (pk, kw["pos_key_scale"]), (pq, kw["pos_query_scale"]) = [(y.transpose(0, 1), z) for y, z in (ops.quantize_e4m3_per_head(t.transpose(0, 1)) for t in (pk, pq))]
+    starts, lens = _bounds(kind, B, L)
+    assert B * ((L + 127) // 128) * H >= 400   # no shares of the keys either way
+    got = []
+    for extra in (0, 65):
+        wide = lambda t: torch.cat([t.view(torch.uint8), torch.zeros(extra, *t.view(torch.uint8).shape[1:], device="cuda", dtype=torch.uint8)]).view(t.dtype)
+        vec = lambda t: torch.tensor(list(t) + [0] * extra, dtype=torch.int32, device="cuda")
+        res = ops.disentangled_attention_fwd(wide(q), wide(k), wide(v), pk, pq, seq_start=vec(starts) if any(starts) else None, seq_len=vec(lens), **kw)
+        out, lse = res if kw["return_lse"] else (res, None)
+        got.append([out[:B].nan_to_num(nan=12345.0)] + ([] if lse is None else [lse.view(B + extra, -1)[:B].nan_to_num(nan=12345.0)]))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 class _BwdArgs(ctypes.Structure):   # fdb_attn_bwd_tables_args of include/fdb.h
     _fields_ = [(n, ctypes.c_void_p) for n in "q k v dout out pos_key pos_query dq dk dv d_pos_key d_pos_query lse seq_start seq_len delta_lut workspace".split()] + \
         [(f"{t}_stride_{x}", ctypes.c_int64) for t in "q k v do out dq dk dv".split() for x in "bth"] + [(f"{t}_stride_{x}", ctypes.c_int64) for t in "pk pq dp".split() for x in "hr"] + \
@@ -83,12 +112,19 @@ def _plain_order(B, H, tiles, causal, keys):
     return out
 
 
-def _order_by_length(lens, H, tiles, mirrored):
-    """mirrored: the causal key tiles, of which the first has the most queries: as far from the text's end as the query tile of that turn is from its beginning."""
+def _order_by_length(lens, H, tiles, causal, keys):
+    """The sequences with the most tiles first, those of a number of tiles as a batch of their own; causal: the highest tile of all sequences first, of key tiles the one as
+    far from the text's end as the query tile of that turn is from its beginning.  Then the tiles of padding."""
     order = sorted(range(len(lens)), key=lambda b: (-((lens[b] + 31) // 32), b))
-    real = [(b, (lens[b] - 1) // 128 - t if mirrored else t) for t in reversed(range(tiles)) for b in order if lens[b] > 128 * t]
-    padding = [(b, t) for t in range(tiles) for b in order if lens[b] <= 128 * t]
-    return [(b, t, h) for b, t in real + padding for h in range(H)]
+    of = lambda b: (lens[b] + 127) // 128
+    if causal:
+        real = [(b, of(b) - 1 - t if keys else t, h) for t in reversed(range(tiles)) for b in order if of(b) > t for h in range(H)]
+    else:
+        real = []
+        for n in range(tiles, 0, -1):
+            alike = [b for b in order if of(b) == n]
+            real += [(alike[x], t, h) for x, t, h in _plain_order(len(alike), H, n, False, keys)]
+    return real + [(b, t, h) for t in range(tiles) for b in order if of(b) <= t for h in range(H)]
 
 
 @pytest.mark.parametrize("lens,L,H,causal", [
@@ -126,8 +162,8 @@ def test_places_of_the_backward(lens, L, H, causal):
         dq, keys = [_plain_order(B, H, tiles, causal, k) for k in (False, True)]
         mixed = [("k", i) for i in range(n)] + [("q", i) for i in range(n)]
     else:
-        dq, keys = [_order_by_length(real, H, tiles, causal and k) for k in (False, True)]
-        mixed = [(r, H * i + h) for i in range(n // H) for r in "kq" for h in range(H)]
+        dq, keys = [_order_by_length(real, H, tiles, causal, k) for k in (False, True)]
+        mixed = [(r, i) for first in range(0, n, 64) for r in "kq" for i in range(first, min(n, first + 64))]
     if n > 2048:
         mixed = [("q", i) for i in range(n)] + [("k", i) for i in range(n)]
     want = [((keys if r == "k" else dq)[i], i, r == "k") for r, i in mixed]
