@@ -1989,3 +1989,25 @@ def test_packed_batch_of_few_long_sequences_shares_its_far_keys(monkeypatch):
         sl = slice(off, off + n)
         _check(auto[sl][None], _oracle_blhd(q[:, sl], k[:, sl], v[:, sl], pk, pq, pb, mr), TOL[torch.bfloat16], "length %d" % n)
         off += n
+
+
+@pytest.mark.parametrize("dtype,D,terms", [(torch.float32, 128, True), (torch.float32, 32, True), (torch.bfloat16, 128, True), (torch.float16, 128, True),
+                                           (torch.float32, 64, False), (torch.bfloat16, 64, False), (torch.float16, 32, False)])
+@pytest.mark.parametrize("shares", [1, 2, 4])
+def test_rows_without_a_soft_max_in_shares_of_one_kernel(dtype, D, terms, shares):
+    """fdb_merge_parts_kernel in every type and head_dim: a query of NaN has a row of NaN and no effect on others, keys that are all at -inf leave no soft-max to any row."""
+    q, k, v, pk, pq = _inputs(1, 300, 2, D, 32, 64, dtype, 5, 1.0, terms, terms)
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    kw = dict(position_buckets=32 if terms else 0, max_relative_positions=64 if terms else 0, far_splits=shares, return_lse=True)
+    call = lambda *x: [t.float().cpu() for t in ops.disentangled_attention_fwd(*[None if t is None else t.cuda() for t in (*x, pk, pq)], **kw)]
+    whole, whole_lse = call(q, k, v)
+    q[0, 7] = float("nan")
+    out, lse = call(q, k, v)
+    rows = [i for i in range(300) if i != 7]
+    assert out[0, 7].isnan().all() and lse.view(300, 2)[7].isnan().all()
+    # the others' sums may be referred to another point, which rounds them anew: probabilities and output to the type, sums and log-sum-exps (up to about 10) in fp32
+    assert (out - whole)[0, rows].abs().max() <= 4 * torch.finfo(dtype).eps * max(1.0, whole.abs().max().item()) and whole.isfinite().all()
+    assert (lse - whole_lse).view(300, 2)[rows].abs().max() <= 16 * 10 * 2.0 ** -23
+    k[0, :, :, 0] = -float("inf")
+    out, lse = call(q, k, v)
+    assert out.isnan().all() and lse.isnan().all()

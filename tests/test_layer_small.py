@@ -53,6 +53,16 @@ def test_against_64_bits(B, L, H, C, buckets, most, bounds, dtype):
         assert np.abs(got[b, s:e] - ref).max() <= 5 * EPS[dtype] * max(1.0, np.abs(ref).max())
 
 
+def _alone(x, w, bias, pos_key, pos_query, heads, scale, buckets, most, start, length):
+    (B, L, C), out = x.shape, torch.empty_like(x)
+    lut, radius = ops.delta_lut_device(buckets, most, x.device)
+    pk, pq = [t.reshape(heads, -1, 64) if t.dim() == 4 else t for t in (pos_key, pos_query)]
+    p = lambda t: None if t is None else t.data_ptr()
+    rc = _lib.lib.fdb_layer_small(p(x), p(w), p(bias), p(pk), p(pq), p(out), p(start), p(length), p(lut), B, L, heads, C, C, w.stride(0), pk.stride(0), pk.stride(1), pq.stride(0),
+                                  pq.stride(1), ops.att_span(buckets, most), radius, scale, CODE[x.dtype], torch.cuda.current_stream().cuda_stream)
+    return rc, out
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,L,heads,padded", [(1, 24, 12, False), (4, 32, 12, True), (2, 33, 12, True), (21, 20, 12, True), (22, 20, 12, True), (3, 7, 6, False), (2, 64, 12, True), (5, 100, 6, True), (2, 129, 12, True)])
 def test_layer_with_and_without(B, L, heads, padded):
@@ -68,6 +78,15 @@ def test_layer_with_and_without(B, L, heads, padded):
     mask = (torch.arange(L, device="cuda") < lens[:, None]).long() if padded else None
     with torch.no_grad():
         got = att(x, mask, rel_embeddings=rel)[0]
+        # Which way it went: one launch allocates nothing but its result, and has the bits of that launch by itself
+        serves = bool(_lib.lib.fdb_layer_small_serves(B, L, heads, 64 * heads))
+        allocated = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+        before = allocated()
+        again = att(x, mask, rel_embeddings=rel)[0]
+        assert (allocated() - before == 1) == serves and torch.equal(got, again)
+        if serves:
+            rc, alone = _alone(x, *att._native_args(mask, rel, x))
+            assert rc == 0 and torch.equal(got, alone)
         handle = att.value_proj.register_forward_hook(lambda *a: None)   # its modules are called
         ref = att(x, mask, rel_embeddings=rel)[0]
         handle.remove()
