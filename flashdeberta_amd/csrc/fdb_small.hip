@@ -8,7 +8,7 @@
 // keys of a query block where there are two or more.  The rows of either table that the blocks' relative positions name are on their way while
 // the projections are made.
 //
-// What bounds it: the weights on their way into one CU's LDS (1 x 24: 3.8 of 8.1 us; 84 KB on their way at a time, about what a latency of 0.9 us lets
+// What bounds it: the weights on their way into one CU's LDS (1 x 24: 3.8 of 8.1 us; four stages of 28 KB on their way at a time, about what a latency of 1.1 us lets
 // through; five stages instead of four, where they fit, 9.3 -> 9.1 us a pass), then one wave's chain of products, exponentials and LDS trips (1.6); and the host.
 // Pass of a layer, two launches -> one, us (12 heads, depth 768, bf16, passes back to back):
 //   1 x 24 13.8 -> 9.1   4 x 24 14.2 -> 9.1   16 x 32 14.9 -> 9.5   21 x 32 15.3 -> 9.9     1 x 48 14.4 -> 11.2   8 x 64 15.6 -> 11.4   21 x 64 18.7 -> 12.8
@@ -358,7 +358,12 @@ int launch(const SmallParams& p, hipStream_t stream) {
 
 // One workgroup fills a CU (160 KB of LDS), so a round of them is where it is faster: 24 x 32 at 12 heads, 288 workgroups, 16.1 us as two launches and
 // 17.1 here, 48 x 32 24.5 and 25.1; 32 x 64 22.4 and 22.7.  Beyond 64 tokens the workgroup's own time, which grows with the depth, is that of two launches
-// for few rows, whose time grows with the batch: at 12 heads 1 x 100 15.6 and 17.2, 3 x 128 17.4 and 17.5, 4 x 100 17.7 and 17.3, 12 x 128 23.4 and 18.0.
+// for few rows, whose time grows with the batch: at 12 heads 1 x 100 15.6 and 17.2, 3 x 128 17.4 and 17.5, 4 x 100 17.7 and 17.3, 12 x 128 23.4 and 18.0.  Other widths, a
+// layer replayed one by one (its start of about 18 us included), two launches and one:
+//   6 heads, depth 384     1 x 80  32.7 and 32.8   2 x 100 34.4 and 34.1   2 x 128 34.4 and 34.3   16 x 128 38.4 and 34.5   40 x 128 46.6 and 39.1
+//   16 heads, depth 1024   1 x 80  49.4 and 47.3   1 x 100 51.2 and 48.3   4 x 128 53.5 and 51.1   8 x 100 54.3 and 51.6   16 x 128 58.3 and 51.8   1 x 48 45.4 and 41.0
+//   24 heads, depth 1536   1 x 80  55.1 and 60.7   2 x 100 61.4 and 61.5   4 x 100 64.8 and 60.7   8 x 100 68.5 and 61.9   10 x 128 69.9 and 61.6   1 x 48 53.1 and 52.8
+// (so at 16 heads the line is on the safe side by up to 5 %).
 extern "C" int32_t fdb_layer_small_serves(int64_t batch, int64_t seqlen, int64_t heads, int64_t depth) {
   return batch >= 1 && heads >= 1 && seqlen >= 1 && seqlen <= 128 && depth >= kDepth && depth % kDepth == 0 && batch <= (1 << 16) && heads <= (1 << 16) &&
          batch * heads <= fdb_cu_count() && (seqlen <= 64 || 2 * batch * seqlen > depth);

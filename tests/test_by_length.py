@@ -163,7 +163,7 @@ def test_places_of_the_backward(lens, L, H, causal):
         mixed = [("k", i) for i in range(n)] + [("q", i) for i in range(n)]
     else:
         dq, keys = [_order_by_length(real, H, tiles, causal, k) for k in (False, True)]
-        mixed = [(r, i) for first in range(0, n, 64) for r in "kq" for i in range(first, min(n, first + 64))]
+        mixed = [(r, i) for first in range(0, n, 32) for r in "kq" for i in range(first, min(n, first + 32))]
     if n > 2048:
         mixed = [("q", i) for i in range(n)] + [("k", i) for i in range(n)]
     want = [((keys if r == "k" else dq)[i], i, r == "k") for r, i in mixed]
