@@ -49,6 +49,7 @@ struct FdbKParams {
                      // partial result of its own (the first in out / lse, the others in workspace slots 0 ..)
   int32_t near_parts; // workgroups per query tile of the near launch; above 1 each leaves the partial result of
                       // its share of the steps in workspace slot far_parts-1 + part, and fdb_launch_merge follows
+  int32_t near_teams; // 16-bit near launches: teams of four waves in a workgroup, which share its steps out among them
   int32_t key_parts; // one-kernel mode: workgroups per query tile, each with an equal share of the key tiles and a
                      // partial result of its own in workspace slot `part`; fdb_launch_merge_parts follows (1: no sharing)
   int32_t ws_slots;  // partial results in the workspace: far_parts-1, plus near_parts if that is above 1; key_parts in the one-kernel mode

@@ -32,6 +32,10 @@
 // launch forms them, with the row of Q_r added to the query and c2p as a number per query row, kept in fp32.  (The scratch would round
 // that number to 16 bits, once for all far keys of the row: the log-sum-exp's error was up to 2.6 times the two launches' that way.)
 //
+// Where every workgroup has a CU to itself (near_takes_teams in fdb_api.cpp) it is two teams of four waves, each with LDS, rings and half of the steps of its own:
+// two waves a SIMD again.  They meet at the same barriers, and the second one's sums come to the first through LDS at the end.  Barriers of a team's own (a count in LDS
+// that its waves poll) were 1 to 5 % slower than the workgroup's.
+//
 // Staging goes global -> LDS directly (global_load_lds_dwordx4: no staging registers, no LDS write
 // instructions of the waves' own) and runs one step ahead: right after the one barrier of step s (every
 // wave is done with step s-1) a wave issues its share of K(s+1) and V(s+1) into the buffers step s does not
@@ -104,20 +108,22 @@ __device__ __forceinline__ float lds_elem_f32(uint32_t addr) {
 }
 __device__ __forceinline__ void lds_wait_all() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-template <class QT, class VT, bool C2P, bool P2C, bool ALL>
-__global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams p) {
+template <class QT, class VT, bool C2P, bool P2C, int TEAMS, bool ALL>
+__global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const FdbKParams p) {
   constexpr int D = 64, KS = 4, DBLKS = 2;
   using qfrag = typename QT::frag;
   using vfrag = typename VT::frag;
   static_assert(QT::SZ == 2 && VT::SZ == 2, "16-bit element types only");
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kNThreads) : 0;
+  char* smem = smem_all + team * NCfg::lds_bytes(C2P, P2C);
   char* Ks = smem;                      // [2][32][128]: step k reads buffer k & 1
   char* Vs = Ks + 2 * NCfg::K_BYTES;    // [2][32][128], likewise
   char* EK = Vs + 2 * NCfg::V_BYTES;    // [192][128] rows K_r[delta(r)], slot = (r_hi0 - r) mod 192
   char* EQ = EK + (C2P ? NCfg::RING_BYTES : 0);
   char* scr_raw = EQ + (P2C ? NCfg::RING_BYTES : 0);  // C's scratch (absent without the c2p term)
 
-  const int tid = threadIdx.x;
+  const int tid = TEAMS > 1 ? threadIdx.x % kNThreads : threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile, h, tok0, sl;   // tile: the query tile of sequence b, or the entry of a packed call's work-list
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   } else {
     m0 = tile * FDB_BM;
     Lb = min(max(sl, 0), p.L - tok0);
-    if (p.fill_pad && blockIdx.y == 0)
+    if (p.fill_pad && blockIdx.y == 0 && team == 0)
       fill_pad_rows<kRowBytes>(p.out + ((int64_t)b * p.o_sb + (int64_t)h * p.o_sh) * 2, p.o_st * 2, tile, p.L, tok0, Lb,
                                sl < 0 ? VT::NAN_WORD : 0u, tid, p.lse && h == 0 ? p.lse + (int64_t)b * p.L * p.H : nullptr, p.H);
     if (m0 >= Lb) return;
@@ -177,10 +183,16 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   int s1 = max(s0, min(2 * t1, (j_end + kStep - 1) / kStep));              // one past the last
   int all0 = s0, all1 = s1;                                                // ALL: the far steps on both sides with them
   if constexpr (ALL) all0 = 0, all1 = (j_end + kStep - 1) / kStep;
-  if (p.near_parts > 1) {  // this workgroup's share of the steps
-    const int all = all1 - all0, part = (int)blockIdx.y;
-    all1 = all0 + (int)((int64_t)all * (part + 1) / p.near_parts);
-    all0 = all0 + (int)((int64_t)all * part / p.near_parts);
+  int more_barriers = 0;   // TEAMS: those the other team meets and this one, with a step fewer, does not
+  if (TEAMS > 1 || p.near_parts > 1) {  // this workgroup's, or team's, share of the steps
+    const int all = all1 - all0, part = (int)blockIdx.y * TEAMS + team, parts = p.near_parts * TEAMS;
+    auto begin = [&](int x) __attribute__((always_inline)) { return (int)((int64_t)all * x / parts); };
+    if constexpr (TEAMS > 1) {
+      const int mine = begin(part + 1) - begin(part), other = begin((part ^ 1) + 1) - begin(part ^ 1);
+      more_barriers = max(0, (other > 0 ? other + 1 : 0) - (mine > 0 ? mine + 1 : 0));
+    }
+    all1 = all0 + begin(part + 1);
+    all0 = all0 + begin(part);
   }
   s0 = ALL ? min(max(s0, all0), all1) : all0;
   s1 = ALL ? max(s0, min(s1, all1)) : all1;
@@ -605,7 +617,36 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   wait_vmcnt<0>();  // the last step's direct loads: none may still be writing LDS when the workgroup ends
 
   // ---- epilogue: merge with the far tiles' partial result, normalise, store ------------------------------
-  const float l_tot = wave_half_sum(l_run);
+  float l_tot = wave_half_sum(l_run);
+  if constexpr (TEAMS > 1) {
+    static_assert(TEAMS == 2 && NCfg::lds_bytes(C2P, P2C) >= 34 * kNThreads * 4, "the second team's sums in its own part of the LDS");
+    for (; more_barriers > 0; --more_barriers) __syncthreads();
+    __syncthreads();   // nobody reads the second team's rings and tiles any more
+    f32x4* sums = (f32x4*)(smem_all + NCfg::lds_bytes(C2P, P2C)) + tid;   // [8][256]: sixteen bytes a lane, then the reference points and the rows' sums
+    float* row = (float*)(smem_all + NCfg::lds_bytes(C2P, P2C) + 32 * kNThreads * 4) + tid;
+    if (team == 1) {
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o_acc[x >> 2][4 * (x & 3) + e];
+        sums[x * kNThreads] = y;
+      }
+      row[0] = m_run, row[kNThreads] = l_tot;
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float m_other = row[0], l_other = row[kNThreads], m_both = fmaxf(m_run, m_other);
+    const float w = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_both), w_other = m_other == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_other - m_both);
+    m_run = m_both;
+    l_tot = l_tot * w + l_other * w_other;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const f32x4 y = sums[x * kNThreads];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o_acc[x >> 2][4 * (x & 3) + e] = o_acc[x >> 2][4 * (x & 3) + e] * w + y[e] * w_other;
+    }
+  }
   if (i < Lb) {
     char* orow = ob + (int64_t)i * p.o_st * 2;
     const int64_t tok = p.cu ? (int64_t)tok0 + i : (int64_t)b * p.L + tok0 + i;
@@ -629,29 +670,30 @@ __global__ __launch_bounds__(kNThreads, 2) void fdb_near_kernel(const FdbKParams
   }
 }
 
-template <class QT, bool C2P, bool P2C, bool ALL>
+template <class QT, bool C2P, bool P2C, int TEAMS, bool ALL>
 int launch_near_one(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  auto kern = fdb_near_kernel<QT, QT, C2P, P2C, ALL>;
-  constexpr int lds = NCfg::lds_bytes(C2P, P2C);
-  static_assert(lds <= 80 * 1024, "two workgroups per CU");
+  auto kern = fdb_near_kernel<QT, QT, C2P, P2C, TEAMS, ALL>;
+  constexpr int lds = TEAMS * NCfg::lds_bytes(C2P, P2C);
+  static_assert(lds <= TEAMS * 80 * 1024, "two workgroups, or the two teams of one, per CU");
   static std::atomic<uint64_t> lds_set{0};
   hipError_t e = fdb_set_lds_once((const void*)kern, lds, lds_set);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid_x * p.H, p.near_parts > 1 ? (unsigned)p.near_parts : 1u, 1), dim3(kNThreads),
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid_x * p.H, p.near_parts > 1 ? (unsigned)p.near_parts : 1u, 1), dim3(kNThreads * TEAMS),
                      lds, stream, p);
   return (int)hipGetLastError();
 }
 
-template <class QT, bool ALL>
+template <class QT, int TEAMS, bool ALL>
 int launch_near_pos(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  if (p.pk && p.pq) return launch_near_one<QT, true, true, ALL>(p, grid_x, stream);
-  if (p.pk) return launch_near_one<QT, true, false, ALL>(p, grid_x, stream);
-  if (p.pq) return launch_near_one<QT, false, true, ALL>(p, grid_x, stream);
+  if (p.pk && p.pq) return launch_near_one<QT, true, true, TEAMS, ALL>(p, grid_x, stream);
+  if (p.pk) return launch_near_one<QT, true, false, TEAMS, ALL>(p, grid_x, stream);
+  if (p.pq) return launch_near_one<QT, false, true, TEAMS, ALL>(p, grid_x, stream);
   return FDB_ERR_UNSUPPORTED;
 }
 template <class QT>
 int launch_near(const FdbKParams& p, int grid_x, hipStream_t stream) {
-  return p.near_all ? launch_near_pos<QT, true>(p, grid_x, stream) : launch_near_pos<QT, false>(p, grid_x, stream);
+  if (p.near_teams > 1) return p.near_all ? launch_near_pos<QT, 2, true>(p, grid_x, stream) : launch_near_pos<QT, 2, false>(p, grid_x, stream);
+  return p.near_all ? launch_near_pos<QT, 1, true>(p, grid_x, stream) : launch_near_pos<QT, 1, false>(p, grid_x, stream);
 }
 
 }  // namespace

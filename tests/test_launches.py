@@ -99,3 +99,14 @@ def test_thresholds_of_the_products_follow_the_compute_units():
     for call, (rc, made), (rc_half, made_half) in zip(asked(1), whole, half):
         assert rc == rc_half and kernels(made) == kernels(made_half), (call, made, made_half)
     assert len({k for _, made in whole for k in kernels(made)}) > 10   # every tile is among them
+
+
+def test_where_near_workgroups_are_two_teams():
+    """Where each has a compute unit to itself and ten steps or more; two shares that do not have one each become one of two teams."""
+    cases = [(_forward(1, 288), 256, 1), (_forward(1, 289), 512, 1), (_forward(1, 128, 12), 256, 1), (_forward(3, 777), 512, 1), (_forward(4, 777), 256, 1),
+             (_forward(1, 1024, workspace=ALL), 512, 2), (_forward(1, 2048, workspace=ALL), 512, 1), (_forward(1, 2048, 4, workspace=ALL), 512, 4),
+             (_forward(1, 512, workspace=ALL), 256, 2), (_forward(1, 1536, workspace=ALL), 256, 3), (_forward(1, 1300, workspace=ALL), 256, 2),
+             (_forward(2, 1024, workspace=ALL, causal=1), 512, 1), (_forward(3, 777, dtype=_lib.FDB_FP8_E4M3), 256, 1)]
+    for (_, threads, shares), (rc, made) in zip(cases, launches([c for c, _, _ in cases])):
+        near = [m for m in made if "near" in m[0]]
+        assert rc == 0 and [m[2:] for m in near] == [(shares, threads)], (made, threads, shares)

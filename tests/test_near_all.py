@@ -118,3 +118,35 @@ def test_far_steps_and_shares(L, H, buckets, most, shared, kind):
     eps = EPS[torch.float16 if kind == "fp16" else torch.bfloat16]
     # as above; outputs are of magnitude 1 at most at these lengths, and e4m3's near c2p is cut to fp16: a score of 4 by 2^-9
     assert np.abs(e).max() <= 3 * eps and np.abs(el).max() <= 2 * eps
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("causal", [False, True], ids=["all", "causal"])
+@pytest.mark.parametrize("L,terms,buckets,most", [(289, (1, 1), 32, 64), (320, (1, 0), 256, 512), (321, (0, 1), 32, 64), (352, (1, 1), 256, 512), (900, (1, 1), 32, 64)])
+def test_two_teams(L, terms, buckets, most, causal, dtype):
+    """Workgroups of two teams at even and odd numbers of steps, far ones among them, in padded rows down to no step for a team or for both, and packed."""
+    lens = [L, 1, 33, 0, 64, L - 1]
+    q, k, v, pk, pq = _inputs(len(lens), L, 2, terms, dtype)
+    pk, pq = [None if x is None else x[:, :2 * buckets] for x in (pk, pq)]
+    d = lambda x: None if x is None else x.cuda()
+    kw = dict(position_buckets=buckets, max_relative_positions=most, causal=causal, return_lse=True)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    out, lse = ops.disentangled_attention_fwd(d(q), d(k), d(v), d(pk), d(pq), seq_len=i32(lens), **kw)
+    rows = lambda x: torch.cat([x[b, :m] for b, m in enumerate(lens)])
+    packed, packed_lse = ops.disentangled_attention_fwd(*[d(rows(x)) for x in (q, k, v)], d(pk), d(pq), cu_seqlens=i32(np.cumsum([0] + lens)), max_seqlen=L, **kw)
+    lse = lse.view(len(lens), L, 2)
+    assert torch.equal(out[:, L - 1:][[1, 2, 3, 4]], torch.zeros_like(out[:4, :1])) and (out[3] == 0).all()
+    n = lambda x: None if x is None else x.float().numpy().astype(np.float64)
+    at = 0
+    for b, m in enumerate(lens):
+        if m == 0:
+            continue
+        t = lambda x: n(x[b:b + 1, :m]).transpose(0, 2, 1, 3)
+        ref, ref_lse = O.disentangled_attention(t(q), t(k), t(v), n(pk), n(pq), buckets, most, causal=causal, return_lse=True)
+        ref, ref_lse = ref[0].transpose(1, 0, 2), ref_lse[0].T
+        for got, got_lse in ((out[b, :m], lse[b, :m]), (packed[at:at + m], packed_lse.view(-1, 2)[at:at + m])):
+            # scores and probabilities are rounded as in every near launch, see above
+            assert np.abs(got.float().cpu().numpy() - ref).max() <= 3 * EPS[dtype] * max(1.0, np.abs(ref).max()), (b, m)
+            assert np.abs(got_lse.cpu().numpy() - ref_lse).max() <= 2 * EPS[dtype], (b, m)
+        at += m
