@@ -237,6 +237,7 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   constexpr bool FAR_ONLY = MODE == kFarOnly, RING = MODE == kNearRing;
   static_assert(!RING || (!FP8 && QT::SZ == 2 && (C2P || P2C)), "the ring mode is for the position terms of the 16-bit types");
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  read_arguments(p);
   constexpr bool KV_ALIAS = C::kv_alias(C2P, P2C);
   static_assert(!KV_ALIAS || MODE == kFused, "only the fused mode shares one buffer between K and V");
   char* Ks = smem;
@@ -372,8 +373,8 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   const int part = (FAR_ONLY || (MODE == kFused && p.key_parts > 1)) ? (int)blockIdx.y : 0;
   int t_lo = 0, t_hi = n_tiles;
   if (MODE == kFused && p.key_parts > 1) {
-    t_lo = (int)((int64_t)n_tiles * part / p.key_parts);
-    t_hi = (int)((int64_t)n_tiles * (part + 1) / p.key_parts);
+    t_lo = share_begins(n_tiles, part, p.key_parts);
+    t_hi = share_begins(n_tiles, part + 1, p.key_parts);
     const int n0 = t_near0, n1 = t_near1;
     t_near0 = min(max(n0, t_lo), t_hi);
     t_near1 = min(max(n1, t_lo), t_hi);
@@ -381,7 +382,7 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   int zl0 = t_lo, zl1 = t_near0, zr0 = t_near1, zr1 = t_hi;
   if (FAR_ONLY && p.far_parts > 1) {
     const int n_far = t_near0 + (n_tiles - t_near1);
-    const int o_lo = (int)((int64_t)n_far * part / p.far_parts), o_hi = (int)((int64_t)n_far * (part + 1) / p.far_parts);
+    const int o_lo = share_begins(n_far, part, p.far_parts), o_hi = share_begins(n_far, part + 1, p.far_parts);
     zl0 = min(o_lo, t_near0);
     zl1 = min(o_hi, t_near0);
     zr0 = t_near1 + max(o_lo - t_near0, 0);

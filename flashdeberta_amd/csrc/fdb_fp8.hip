@@ -87,6 +87,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   constexpr int D = 64, DBLKS = 2;
   using VT = Bf16Tr;
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  read_arguments(p);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
@@ -135,7 +136,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   const int part = (int)blockIdx.y;
   if (p.far_parts > 1) {
     const int n_far = t_near0 + (n_tiles - t_near1);
-    const int o_lo = (int)((int64_t)n_far * part / p.far_parts), o_hi = (int)((int64_t)n_far * (part + 1) / p.far_parts);
+    const int o_lo = share_begins(n_far, part, p.far_parts), o_hi = share_begins(n_far, part + 1, p.far_parts);
     zl0 = min(o_lo, t_near0);
     zl1 = min(o_hi, t_near0);
     zr0 = t_near1 + max(o_lo - t_near0, 0);
@@ -405,6 +406,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   using VT = Bf16Tr;
   using vfrag = typename VT::frag;
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  read_arguments(p);
   char* Ks = smem;                    // [2][32][64]: step k reads buffer k & 1
   char* Vs = Ks + 2 * N8::K_BYTES;    // [2][32][128]
   char* EK = Vs + 2 * N8::V_BYTES;    // [160][64] rows K_r[delta(r)]: batch u / 32 of u = r_hi0 - r in slot batch mod 5; E_Q: [192][64], mod 6
@@ -469,8 +471,8 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   if constexpr (ALL) all0 = 0, all1 = (j_end + kStep - 1) / kStep;
   if (p.near_parts > 1) {
     const int all = all1 - all0, part = (int)blockIdx.y;
-    all1 = all0 + (int)((int64_t)all * (part + 1) / p.near_parts);
-    all0 = all0 + (int)((int64_t)all * part / p.near_parts);
+    all1 = all0 + share_begins(all, part + 1, p.near_parts);
+    all0 = all0 + share_begins(all, part, p.near_parts);
   }
   s0 = ALL ? min(max(s0, all0), all1) : all0;
   s1 = ALL ? max(s0, min(s1, all1)) : all1;

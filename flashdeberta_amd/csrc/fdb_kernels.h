@@ -174,6 +174,10 @@ int fdb_launch_chain(const FdbChainParams& p, int dtype, void* stream);
 
 // Workspace slot `slot`: its output rows and its log-sum-exps (row_bytes = head_dim * element size).
 #if defined(__HIPCC__)
+// A kernel's first instruction: one argument of every 64 bytes that are not read at once anyway.  Left to itself the compiler reads the arguments where they
+// are used, each new 64 bytes of them after a wait for memory of their own.
+__device__ __forceinline__ void read_arguments(const FdbKParams& p) { asm volatile("" ::"s"(p.q_sb), "s"(p.o_sb)); }
+
 __device__ __forceinline__ char* ws_slot_out(const FdbKParams& p, int slot, int row_bytes) {
   return p.ws + (int64_t)slot * p.ws_rows * p.H * row_bytes;
 }

@@ -115,6 +115,7 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
   using vfrag = typename VT::frag;
   static_assert(QT::SZ == 2 && VT::SZ == 2, "16-bit element types only");
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  read_arguments(p);
   const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kNThreads) : 0;
   char* smem = smem_all + team * NCfg::lds_bytes(C2P, P2C);
   char* Ks = smem;                      // [2][32][128]: step k reads buffer k & 1
@@ -159,19 +160,6 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
   const int iw0 = m0 + wave * 32;
   const int i = iw0 + li;
 
-  qfrag qf[KS];
-#pragma unroll
-  for (int s = 0; s < KS; ++s)
-    qf[s] = (i < Lb) ? QT::load(qb + ((int64_t)i * p.q_st + 16 * s + 8 * g) * 2) : QT::zero();
-  // Consume the query loads here: left pending into the loop, their first use would make the
-  // compiler wait for every outstanding vector-memory load at the top of each step.
-#pragma unroll
-  for (int s = 0; s < KS; ++s) asm volatile("" ::"v"(qf[s]));
-  // the query operand carries the soft-max scale (in base 2): the content product and C leave the MFMA in the
-  // exponent's unit; P, which the keys make, is scaled where it is added
-#pragma unroll
-  for (int s = 0; s < KS; ++s) qf[s] = QT::from_f32(QT::to_f32(qf[s]) * x_scale);
-
   // ---- the near range: the 64-key tiles the far-only run skips, walked 32 keys at a time -----------
   int j_end = Lb;
   if (p.causal) j_end = min(Lb, m0 + FDB_BM);
@@ -186,13 +174,13 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
   int more_barriers = 0;   // TEAMS: those the other team meets and this one, with a step fewer, does not
   if (TEAMS > 1 || p.near_parts > 1) {  // this workgroup's, or team's, share of the steps
     const int all = all1 - all0, part = (int)blockIdx.y * TEAMS + team, parts = p.near_parts * TEAMS;
-    auto begin = [&](int x) __attribute__((always_inline)) { return (int)((int64_t)all * x / parts); };
+    const int from = share_begins(all, part, parts), to = share_begins(all, part + 1, parts);
     if constexpr (TEAMS > 1) {
-      const int mine = begin(part + 1) - begin(part), other = begin((part ^ 1) + 1) - begin(part ^ 1);
+      const int mine = to - from, other = team == 0 ? share_begins(all, part + 2, parts) - to : from - share_begins(all, part - 1, parts);
       more_barriers = max(0, (other > 0 ? other + 1 : 0) - (mine > 0 ? mine + 1 : 0));
     }
-    all1 = all0 + begin(part + 1);
-    all0 = all0 + begin(part);
+    all1 = all0 + to;
+    all0 = all0 + from;
   }
   s0 = ALL ? min(max(s0, all0), all1) : all0;
   s1 = ALL ? max(s0, min(s1, all1)) : all1;
@@ -257,6 +245,33 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
     if constexpr (C2P) dma16sn(pkb, __umul24((uint32_t)delta, pk_rowb) + chunk_off, ek_lds + seg);
     if constexpr (P2C) dma16sn(pqb, __umul24((uint32_t)delta, pq_rowb) + chunk_off, eq_lds + seg);
   };
+
+  // ---- prologue: the table values, the query rows, the first step's K and V and ring batches 0..4 are asked for ahead of everything that can be worked out
+  // while they are on their way.  All table values first, then all rows: the loads of one kind are in flight together.
+  qfrag qf[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s)
+    qf[s] = (i < Lb) ? QT::load(qb + ((int64_t)i * p.q_st + 16 * s + 8 * g) * 2) : QT::zero();
+  if (n_steps + n_far > 0) {
+    const bool rings = !ALL || n_steps > 0;
+    int d0[6];
+    if (rings) {
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
+    }
+    k_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);  // K and V need no table value: on their way while the table is read
+    v_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);
+    if (rings) {
+      // (taken here, all at once: the compiler, which does not count the direct loads, would otherwise wait for
+      // each value at its use, behind all the direct loads issued before it)
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
+#pragma unroll
+      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
+      dnext = d0[5];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
 
   f32x16 o_acc[DBLKS];
 #pragma unroll
@@ -359,8 +374,6 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
     }
     range_begins(C2P ? wave_half_sum(acc) * x_scale : 0.f);
   };
-  // ---- prologue: the first step's K and V and ring batches 0..4 on their way to LDS ------------------------
-  // All table values first, then all rows: the loads of one kind are in flight together.
   auto near_begins = [&]() __attribute__((always_inline)) {
     ring_read(1, 3 - wave);  // block 1 of step 0
     if constexpr (C2P) {
@@ -370,21 +383,16 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
       c_store(c1, 1);
     }
   };
+  // the query operand carries the soft-max scale (in base 2): the content product and C leave the MFMA in the
+  // exponent's unit; P, which the keys make, is scaled where it is added
+  auto scale_query = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = QT::from_f32(QT::to_f32(qf[s]) * x_scale);
+  };
   if (n_steps + n_far > 0) {
-    k_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);  // K and V need no table value: on their way while the table is read
-    v_dma(ALL ? far_step_at(-n_far) : s0, n_far & 1, false);
-    if (!ALL || n_steps > 0) {
-      int d0[6];
-#pragma unroll
-      for (int bt = 0; bt < 6; ++bt) d0[bt] = batch_delta();
-      // (taken here, all at once: the compiler, which does not count the direct loads, would otherwise wait for
-      // each value at its use, behind all the direct loads issued before it)
-#pragma unroll
-      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt]));
-#pragma unroll
-      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
-      dnext = d0[5];
-    }
+    scale_query();
     if constexpr (ALL)
       if (__builtin_expect(n_far > 0, 0)) side_begins(n_left > 0 ? 0 : 1);  // (far code out of the way of the tiles that have none)
     wait_vmcnt<0>();

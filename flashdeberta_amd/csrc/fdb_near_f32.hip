@@ -60,6 +60,7 @@ __device__ __forceinline__ f32x16 mma1(const Operand& a, const Operand& b, int n
 template <bool C2P, bool P2C>
 __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  read_arguments(p);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
@@ -106,8 +107,6 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
 #pragma unroll
     for (int x = 0; x < 8; ++x) qf.a[x] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-#pragma unroll
-  for (int x = 0; x < 8; ++x) qf.a[x] *= x_scale;   // the soft-max scale, in base 2
 
   // ---- the steps: [0, s0) far left of the query tile (every r >= R), [s0, s1) near, [s1, end) far right (every r <= -R) ----------------
   int j_end = Lb;
@@ -119,8 +118,8 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
   int all0 = 0, all1 = end;
   const int part = p.key_parts > 1 ? (int)blockIdx.y : 0;
   if (p.key_parts > 1) {   // this workgroup's share
-    all0 = (int)((int64_t)end * part / p.key_parts);
-    all1 = (int)((int64_t)end * (part + 1) / p.key_parts);
+    all0 = share_begins(end, part, p.key_parts);
+    all1 = share_begins(end, part + 1, p.key_parts);
   }
   s0 = min(max(s0, all0), all1);
   s1 = max(s0, min(s1, all1));
@@ -167,6 +166,23 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
     }
   };
 
+  // ---- the first step's loads, ahead of everything that can be worked out while they are on their way ------------------------------
+  int dnext[2] = {0, 0};
+  if (n_steps + n_far > 0) {
+    kv_dma(far_step_at(-n_far), n_far & 1);
+    if (n_steps > 0) {
+      int d0[6][2];
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) batch_delta(d0[bt]);
+#pragma unroll
+      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt][0]), "+v"(d0[bt][1]));
+#pragma unroll
+      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
+      dnext[0] = d0[5][0], dnext[1] = d0[5][1];
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
   // ---- per-lane constants ---------------------------------------------------------------------------------------------------------
   const int arow = 31 - li;
   const uint32_t k_lane = (uint32_t)(li * kRow + ((g ^ row_f(li)) * 16)), e_lane = (uint32_t)(arow * kRow + ((g ^ row_f(arow)) * 16));
@@ -208,7 +224,6 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
   float m_run = -INFINITY, l_run = 0.f, row_add = 0.f;
 
   int slot_rd = 4 - wave, slot_dma = 0;
-  int dnext[2] = {0, 0};
   Operand aq[2];   // E_Q's rows of the new block and of the one before, by the step's parity
   Operand qx;      // the query of the far steps at hand, with Q_r's row
   auto side_begins = [&](int side) __attribute__((always_inline)) {   // 0: left of the near steps, delta(R); 1: right of them, delta(-R)
@@ -385,17 +400,8 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
   };
 
   if (n_steps + n_far > 0) {
-    kv_dma(far_step_at(-n_far), n_far & 1);
-    if (n_steps > 0) {
-      int d0[6][2];
 #pragma unroll
-      for (int bt = 0; bt < 6; ++bt) batch_delta(d0[bt]);
-#pragma unroll
-      for (int bt = 0; bt < 6; ++bt) asm volatile("" : "+v"(d0[bt][0]), "+v"(d0[bt][1]));
-#pragma unroll
-      for (int bt = 0; bt < 5; ++bt) batch_dma(d0[bt], bt);
-      dnext[0] = d0[5][0], dnext[1] = d0[5][1];
-    }
+    for (int x = 0; x < 8; ++x) qf.a[x] *= x_scale;   // the soft-max scale, in base 2
     using T0 = std::integral_constant<int, 0>;
     using T1 = std::integral_constant<int, 1>;
     if (n_far > 0) {

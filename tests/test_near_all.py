@@ -121,6 +121,16 @@ def test_far_steps_and_shares(L, H, buckets, most, shared, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,H", [(1, 1), (3, 7), (400001, 12)])   # the last: more workgroups than quick_div's fp32 quotients reach
+def test_every_workgroup_finds_its_place(B, H):
+    """Texts of one token: the output is v."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    q, k, v = [torch.randn(B, 1, H, 64, device="cuda", generator=g, dtype=torch.bfloat16) for _ in range(3)]
+    pk, pq = [torch.randn(H, 64, 64, device="cuda", generator=g, dtype=torch.bfloat16) for _ in range(2)]
+    assert torch.equal(ops.disentangled_attention_fwd(q, k, v, pk, pq, position_buckets=32, max_relative_positions=64), v)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("causal", [False, True], ids=["all", "causal"])
 @pytest.mark.parametrize("L,terms,buckets,most", [(289, (1, 1), 32, 64), (320, (1, 0), 256, 512), (321, (0, 1), 32, 64), (352, (1, 1), 256, 512), (900, (1, 1), 32, 64)])

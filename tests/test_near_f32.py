@@ -83,3 +83,18 @@ def test_scores_that_rise_through_the_far_steps(L, terms, causal, shares, rise):
     # a score of 60 carries 2^-24 of itself from each of some ten sums that are as large: 4e-5 of a probability, and as much of lse
     assert np.abs(out.cpu().numpy() - ref).max() <= 1e-4 * max(1.0, np.abs(ref).max())
     assert np.abs(lse.view(1, L, 2).cpu().numpy() - ref_lse).max() <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,H,padded", [(1, 1, 1, False), (3, 70, 7, True), (700, 3, 5, False), (2800, 129, 12, True)])   # the last: past 2^22 rows of the outputs
+def test_merged_shares_lie_where_one_launch_puts_them(B, L, H, padded):
+    g = torch.Generator(device="cuda").manual_seed(B + L)
+    q, k, v = [torch.randn(B, L, H, 64, device="cuda", generator=g) for _ in range(3)]
+    pk, pq = [torch.randn(H, 64, 64, device="cuda", generator=g) for _ in range(2)]
+    kw = dict(position_buckets=32, max_relative_positions=64, return_lse=True)
+    if padded:
+        kw["seq_len"] = torch.randint(0, L + 1, (B,), device="cuda", generator=g, dtype=torch.int32)
+    (one, one_lse), (shared, shared_lse) = [ops.disentangled_attention_fwd(q, k, v, pk, pq, far_splits=n, **kw) for n in (1, 2)]
+    # sums in another order: a few 2^-24 of outputs whose weights are at most 1, and of log-sum-exps of at most 40
+    assert (shared - one).abs().max() <= 4e-6 * max(1.0, one.abs().max().item()) and (shared_lse - one_lse).nan_to_num(posinf=0, neginf=0).abs().max() <= 1e-5
+    assert torch.equal(shared_lse.isinf(), one_lse.isinf())
