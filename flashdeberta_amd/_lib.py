@@ -47,7 +47,7 @@ class FdbAttnBwdArgs(ctypes.Structure):
 EXPORTS = (
     "fdb_version", "fdb_attn_args_size", "fdb_strerror", "fdb_attn_check", "fdb_attn_fwd", "fdb_attn_fwd_part", "fdb_attn_fwd_noalloc",
     "fdb_attn_bwd", "fdb_attn_bwd_tables", "fdb_attn_bwd_tables_workspace_bytes", "fdb_attn_bwd_chain", "fdb_attn_bwd_args_size",
-    "fdb_attn_workspace_bytes", "fdb_worklist_ints", "fdb_worklist_max_tiles", "fdb_tile_rows", "fdb_build_worklist",
+    "fdb_attn_workspace_bytes", "fdb_worklist_ints", "fdb_worklist_max_tiles", "fdb_needs_worklist", "fdb_tile_rows", "fdb_build_worklist",
     "fdb_delta_lut_radius", "fdb_delta_lut", "fdb_delta_lut_window", "fdb_linear", "fdb_layer_small", "fdb_layer_small_serves", "fdb_gemm", "fdb_gemm_serves", "fdb_gemm_real",
     "fdb_gemm_real_cleared", "fdb_gemm_real_serves", "fdb_join", "fdb_dgrad", "fdb_dgrad_serves", "fdb_wgrad", "fdb_wgrad_workspace_bytes",
     "fdb_column_sums", "fdb_column_sums_workspace_bytes", "fdb_mask_bounds", "fdb_quant_e4m3_per_head", "fdb_quant_e4m3_per_head_pair",
@@ -98,6 +98,8 @@ def _load():
     lib.fdb_worklist_ints.argtypes = [i32, i32]
     lib.fdb_worklist_max_tiles.restype = i32
     lib.fdb_worklist_max_tiles.argtypes = [i32, i32]
+    lib.fdb_needs_worklist.restype = i32
+    lib.fdb_needs_worklist.argtypes = [i32, i32, i32]
     lib.fdb_tile_rows.restype = i32
     lib.fdb_build_worklist.restype = ctypes.c_int
     lib.fdb_build_worklist.argtypes = [vp, i32, i32, vp, vp]

@@ -321,6 +321,15 @@ int32_t fdb_worklist_max_tiles(int32_t total_tokens, int32_t batch) {
   return (int32_t)n;
 }
 
+// Packed calls whose workgroups find their tiles themselves (packed_place): the work-list's launch, 4 us with what it delays, against 0.3 us more at the start of each
+// workgroup, once for every round of them.  us, work-list -> without, sequences of lengths spread evenly over their logarithm, 12 heads, workgroups at most:
+//   4 of 16 to 256      84   15.9 -> 13.4      32 of 32 to 512    936   45.3 -> 44.8     64 of 32 to 512   1848   69.1 -> 69.8 (kept)
+//   8 of 32 to 512     264   28.0 -> 26.4      16 of 32 to 2048  1092  104.0 -> 104.1    32 of 32 to 2048  1992  175.4 -> 176.7 (kept)
+//   16 of 32 to 512    504   33.2 -> 30.7      8 of 2000 to 2048 1608  233.7 -> 233.9    64 of 32 to 2048  3840  305.5 -> 308.4 (kept)
+int32_t fdb_needs_worklist(int32_t total_tokens, int32_t batch, int32_t heads) {
+  return batch > 64 || (int64_t)fdb_worklist_max_tiles(total_tokens, batch) * heads > 4 * fdb_cu_count();
+}
+
 int64_t fdb_worklist_ints(int32_t total_tokens, int32_t batch) {
   return 2 + 2 * (int64_t)fdb_worklist_max_tiles(total_tokens, batch);
 }
@@ -397,7 +406,7 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
   p.out = (char*)a->out;
   p.lse = a->lse;
   p.cu = a->cu_seqlens;
-  p.wl = a->worklist;
+  p.wl = fdb_needs_worklist(a->total_tokens, a->batch, a->heads) ? a->worklist : nullptr;
   p.lut = a->delta_lut;
   p.seq_start = a->cu_seqlens ? nullptr : a->seq_start;
   p.seq_len = a->cu_seqlens ? nullptr : a->seq_len;
@@ -507,7 +516,7 @@ int fdb_attn_fwd_noalloc(const fdb_attn_args* a, void* stream) {
   // what is left holds as many partial results as fit: the call shares less with a smaller remainder
   b.workspace = base + off;
   b.workspace_bytes = FDB_NOALLOC_SCRATCH_BYTES - off;
-  if (b.cu_seqlens) {
+  if (b.cu_seqlens && fdb_needs_worklist(b.total_tokens, b.batch, b.heads)) {
     const int rw = fdb_launch_worklist(b.cu_seqlens, b.batch, b.worklist, fdb_worklist_max_tiles(b.total_tokens, b.batch), stream);
     if (rw != 0) return rw;
   }

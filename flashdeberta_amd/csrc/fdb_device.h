@@ -421,6 +421,57 @@ __device__ __forceinline__ void place_of(int n, const Params& p, int tiles_per_s
   }
 }
 
+// Packed sequences: the query tile with the number `tile`, of the sequences with the most tiles first; false: there are fewer.  Large batches have a work-list
+// that a launch of its own wrote; of small ones, up to 64 sequences, a lane has one, and every wave finds the tile itself: `of`, the largest number of tiles so that the sequences
+// with at least that many have more than `tile` of them, bit by bit, then which of those with just as many.  One load's latency where the work-list's
+// entry and the two ends of the sequence were three, and no launch ahead of the first workgroup (fdb_needs_worklist has the figures).
+template <class Op>
+__device__ __forceinline__ int wave_fold(int x, Op op) {   // of numbers of which 0 changes nothing
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));   // row_shr:1, 2, 4, 8
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));   // row_bcast:15 into rows 1 and 3, :31 into rows 2 and 3
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(x, 63);
+}
+template <class Params>
+__device__ __forceinline__ bool packed_place(const Params& p, int tile, int lane, int& b, int& m0, int& tok0, int& len) {
+  if (p.wl) {
+    if (tile >= p.wl[0]) return false;
+    b = p.wl[2 + 2 * tile];
+    m0 = p.wl[3 + 2 * tile];
+    tok0 = p.cu[b];
+    len = p.cu[b + 1] - tok0;
+    return true;
+  }
+  int first = 0, mine = 0;
+  if (lane < p.B) {
+    first = p.cu[lane];
+    mine = max(p.cu[lane + 1] - first, 0);
+  }
+  const int tiles = (int)(((uint32_t)mine + FDB_BM - 1) / FDB_BM);
+  auto tiles_from = [&](int least) __attribute__((always_inline)) {   // of the sequences with at least that many
+    return wave_fold(tiles >= least ? tiles : 0, [](int x, int y) { return x + y; });
+  };
+  const int most = wave_fold(tiles, [](int x, int y) { return max(x, y); });
+  int of = 0, ahead = 0;   // tiles of the sequences with more than `of`: the last number that was too high is of + 1
+  for (int bit = 31 - __builtin_clz(most | 1); bit >= 0; --bit) {
+    const int x = of | (1 << bit), those = x <= most ? tiles_from(x) : 0;
+    if (those > tile) of = x;
+    else ahead = those;
+  }
+  if (of == 0) return false;
+  const int u = tile - ahead, rank = __builtin_amdgcn_readfirstlane(quick_div(u, of));
+  const uint64_t those = __ballot(tiles == of);
+  const int ahead_of_me = __builtin_amdgcn_mbcnt_hi((uint32_t)(those >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)those, 0u));
+  b = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(tiles == of && ahead_of_me == rank)) - 1);
+  m0 = (u - rank * of) * FDB_BM;
+  tok0 = __builtin_amdgcn_readlane(first, b);
+  len = __builtin_amdgcn_readlane(mine, b);
+  return true;
+}
+
 // The 16-bit products by tiles of 16 x 16 outputs, and where they keep a row of 128 bytes in LDS: slot (row, s) holds chunk s ^ swz16(row), so that
 // sixteen rows' same chunk lies in sixteen bank groups.
 __device__ __forceinline__ f32x4 mma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }

@@ -97,11 +97,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   int m0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
-    if (tile >= p.wl[0]) return;
-    b = p.wl[2 + 2 * tile];
-    m0 = p.wl[3 + 2 * tile];
-    tok0 = p.cu[b];
-    Lb = p.cu[b + 1] - tok0;
+    if (!packed_place(p, tile, lane, b, m0, tok0, Lb)) return;
     qo = ko = vo = oo = 0;
   } else {
     m0 = tile * FDB_BM;
@@ -422,11 +418,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   int m0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
-    if (tile >= p.wl[0]) return;
-    b = p.wl[2 + 2 * tile];
-    m0 = p.wl[3 + 2 * tile];
-    tok0 = p.cu[b];
-    Lb = p.cu[b + 1] - tok0;
+    if (!packed_place(p, tile, lane, b, m0, tok0, Lb)) return;
     qo = ko = vo = oo = 0;
   } else {
     m0 = tile * FDB_BM;

@@ -69,11 +69,7 @@ __global__ __launch_bounds__(256, 1) void fdb_near_f32_kernel(const FdbKParams p
   int m0, Lb;
   int64_t qo, ko, vo, oo;
   if (p.cu) {
-    if (tile >= p.wl[0]) return;
-    b = p.wl[2 + 2 * tile];
-    m0 = p.wl[3 + 2 * tile];
-    tok0 = p.cu[b];
-    Lb = p.cu[b + 1] - tok0;
+    if (!packed_place(p, tile, lane, b, m0, tok0, Lb)) return;
     qo = ko = vo = oo = 0;
   } else {
     m0 = tile * FDB_BM;

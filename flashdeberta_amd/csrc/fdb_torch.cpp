@@ -388,10 +388,10 @@ constexpr int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 void launch_forward(fdb_attn_args& a, const Tensor& on, bool need_lse, const Fwd& o) {
   void* stream = stream_of(on);
   const int64_t lse_bytes = need_lse && !a.lse ? up256((int64_t)a.total_tokens * a.heads * 4) : 0;
-  const int64_t wl_bytes = a.cu_seqlens ? up256(fdb_worklist_ints(a.total_tokens, a.batch) * 4) : 0;
+  const int64_t wl_bytes = a.cu_seqlens && fdb_needs_worklist(a.total_tokens, a.batch, a.heads) ? up256(fdb_worklist_ints(a.total_tokens, a.batch) * 4) : 0;
   // the size depends on whether these buffers are there, not on where
   if (lse_bytes) a.lse = (float*)16;
-  if (wl_bytes) a.worklist = (int32_t*)16;
+  if (a.cu_seqlens) a.worklist = (int32_t*)16;   // (where there is none, this stands for it: nobody reads it)
   int64_t ws_bytes = 0;
   if (o.workspace) {
     const Tensor& w = *o.workspace;
