@@ -126,7 +126,7 @@ __device__ __forceinline__ void bwd_ring(const FdbBwdRingParams& p, const int wg
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
   int b, tile_x, h;
   if constexpr (BY_LENGTH) b = (int)own_sgpr((uint32_t)at->b), tile_x = (int)own_sgpr((uint32_t)at->tile), h = (int)own_sgpr((uint32_t)at->h);
-  else block_map(wg, p.B, p.H, p.tiles, p.groups_together, true, order_of(p, kDQ), b, tile_x, h);
+  else block_map<false>(wg, p.B, p.H, p.tiles, p.groups_together, true, order_of(p, kDQ), b, tile_x, h);
   const int m0 = tile_x * FDB_BM;
   const int tok0 = BY_LENGTH ? (int)own_sgpr((uint32_t)at->tok0) : p.seq_start ? min(max(p.seq_start[b], 0), p.L) : 0;
   const int Lb = BY_LENGTH ? (int)own_sgpr((uint32_t)at->tokens) : p.seq_len ? min(max(p.seq_len[b], 0), p.L - tok0) : p.L;

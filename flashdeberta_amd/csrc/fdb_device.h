@@ -280,11 +280,14 @@ __device__ __forceinline__ int quick_div(int a, int b) {
 }
 // Where the share `part` of `all` steps begins, of `parts` equal ones (at most 8, of at most 2^26 steps).
 __device__ __forceinline__ int share_begins(int all, int part, int parts) { return __builtin_amdgcn_readfirstlane(quick_div(all * part, parts)); }
+// QUICK: not in the backward's roles, whose registers are so full that quick_div's branches spill 31 more of them in dQ's (8 x 4096 947 -> 1073 us; the other role the same).
+template <bool QUICK = true>
 __device__ __forceinline__ void block_place(int n, int batch, int heads, int tiles_per_seq, int most, int order, int& b, int& t, int& h) {   // the fixed layout's; a lane each
   const int groups = batch * heads;
-  const int first = groups <= most ? 0 : quick_div(n, most * tiles_per_seq) * most;
+  auto div = [](int x, int y) __attribute__((always_inline)) { return QUICK ? quick_div(x, y) : x / y; };
+  const int first = QUICK && groups <= most ? 0 : div(n, most * tiles_per_seq) * most;
   const int here = min(groups - first, most), m = n - first * tiles_per_seq;
-  t = quick_div(m, here);
+  t = div(m, here);
   const int i = m - t * here;
   const int grp = first + (i < (here & ~7) ? (n & 7) | (i & ~7) : i);
   if (order == kLastFirst) {
@@ -293,21 +296,22 @@ __device__ __forceinline__ void block_place(int n, int batch, int heads, int til
     if (order == kMiddleFirst) t = tiles_per_seq - 1 - t;
     t = (t & 1) ? tiles_per_seq - 1 - (t >> 1) : (t >> 1);  // 0, T-1, 1, T-2, ...
   }
-  b = quick_div(grp, heads);
+  b = div(grp, heads);
   h = grp - b * heads;
 }
+template <bool QUICK = true>
 __device__ __forceinline__ void block_map(int n, int batch, int heads, int tiles_per_seq, int most, bool fixed, int order, int& b_out, int& t_out,
                                           int& h_out) {
   // Not the caller's variables: the compiler makes one store, to a chosen address, of the two branches' stores, and the numbers then
   // pass through scratch memory before a workgroup's first load.  Forward of 1 x 4096, 16 heads: 119.5 -> 117.9 us.
   int b, t, h;
   if (fixed) {
-    block_place(n, batch, heads, tiles_per_seq, most, order, b, t, h);
+    block_place<QUICK>(n, batch, heads, tiles_per_seq, most, order, b, t, h);
   } else {
     // packed sequences: the work-list holds the tiles longest sequence first; all heads of a tile are
     // dealt before the next tile, so the whole launch runs from long workgroups to short ones
     b = 0;
-    t = quick_div(n, heads);
+    t = QUICK ? quick_div(n, heads) : n / heads;
     h = n - t * heads;
   }
   // the divisions run on vector registers: taken back, or every address that depends on these stays there too (the e4m3 near kernel
