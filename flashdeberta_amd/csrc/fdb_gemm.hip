@@ -3,8 +3,8 @@
 // hipBLASLt does the plain product as fast; what is gained is what follows it.  An encoder layer adds the residual to two of its products
 // and takes the GELU of a third, each a pass of its own over memory that is as long as a tenth of the layer.  Here these happen on the
 // tile that is being written.  [4096 rows, bf16, on the GPU alone, in a replayed graph; product and pass by torch -> here]
-//   768 -> 768 + residual 17.0 -> 9.8 us,  768 -> 3072 + GELU 37.8 -> 27.7,  3072 -> 768 + residual 30.6 -> 26.9;
-// with 1500 rows 11.6 -> 7.3, 22.1 -> 16.2 and 21.7 -> 18.3.
+//   768 -> 768 + residual 17.0 -> 9.0 us,  768 -> 3072 + GELU 37.8 -> 26.3,  3072 -> 768 + residual 30.6 -> 26.4;
+// with 1500 rows 11.6 -> 6.5, 22.1 -> 15.5 and 21.7 -> 16.7.
 //
 // The sums run over the contraction in order, 32 at a time, in one accumulator, and are rounded where torch's separate passes round:
 // the bits are those of torch's product, GELU and addition (where the library does not split the contraction).
