@@ -396,8 +396,12 @@ int fdb_launch_worklist(const int32_t* cu, int32_t batch, int32_t* wl, int32_t m
 // per eight elements of a (token, head) row; padded rows of a fixed-layout batch are left alone.
 //
 // What bounds these two launches is how long one thread takes: a few MB are read and written by threads that live once.  So the place of a row is found with
-// 32-bit numbers instead of three 64-bit divisions a thread, and everything that a thread may read is asked for at once, weights and values of all parts together
-// (1 x 512 in fp32, four parts: with the two 64-bit divisions ahead of the attention launch's first load gone, too, the call takes 34.4 us instead of 36.0).
+// 32-bit numbers instead of three 64-bit divisions a thread, and what a thread reads is asked for together, the weights of all parts and the values of up to four.
+// Not of all eight that the far and near launch may leave: their values and addresses take 234 registers, two waves a SIMD instead of eight, whose second round
+// cost more than one trip to memory.  us of the whole call, 12 heads: a part's values when its turn comes -> all eight ahead -> four
+//   bf16, three shares  1 x 1536  43.9 (two shares) -> 38.1 -> 35.4      e4m3, two shares  2 x 1280  37.7 -> 38.2 -> 36.2
+//   bf16, four shares, 4 heads  1 x 2048  27.0 -> 25.3 -> 24.3          e4m3, two shares  1 x 2048  49.0 -> 50.2 -> 48.4
+//   bf16, near_splits = 4  8 x 2048  282 -> 297 -> 278                  fp32, four parts (the one-kernel mode's merge, which has four at most)  1 x 512  35.1 -> 33.8
 namespace {
 
 // Where a thread's row lies: CPR threads a row, in whole rows.
@@ -439,21 +443,26 @@ __global__ __launch_bounds__(256) void fdb_merge_kernel(const FdbKParams p) {
   const MergeRow r = merge_row<CPR>(p);
   if (r.row >= p.ws_rows * p.H) return;
   char* dst = p.out + ((p.cu ? r.tok * p.o_st : (int64_t)r.b * p.o_sb + (int64_t)r.l * p.o_st) + (int64_t)r.h * p.o_sh) * 2 + r.cc * 16;
-  constexpr int kMax = 2 * FDB_MAX_FAR_PARTS;
+  constexpr int kMax = 2 * FDB_MAX_FAR_PARTS, kGroup = 4;
   const int n_far = p.far_done ? p.far_parts : 0, n = n_far + p.near_parts;
+  // source s: far part s (s < n_far), else near part s - n_far
+  auto slot_of = [&](int s) __attribute__((always_inline)) { return s < n_far ? s - 1 : p.far_parts - 1 + (s - n_far); };
+  u32x4 part[kGroup];
+  auto ask = [&](int first) __attribute__((always_inline)) {
+#pragma unroll
+    for (int x = 0; x < kGroup; ++x) {
+      const int slot = slot_of(first + x);
+      if (first + x < n) part[x] = *(const u32x4*)(slot < 0 ? dst : ws_slot_out(p, slot, RB) + r.row * RB + r.cc * 16);
+    }
+  };
   float w[kMax], m = -INFINITY;
-  u32x4 part[kMax];
 #pragma unroll
   for (int s = 0; s < kMax; ++s) {
+    const int slot = slot_of(s);
     w[s] = -INFINITY;
-    part[s] = u32x4{0, 0, 0, 0};
-    if (s < n) {
-      // source s: far part s (s < n_far), else near part s - n_far
-      const int slot = s < n_far ? s - 1 : p.far_parts - 1 + (s - n_far);
-      w[s] = (slot < 0 ? p.lse : ws_slot_lse(p, slot, RB))[r.row];
-      part[s] = *(const u32x4*)(slot < 0 ? dst : ws_slot_out(p, slot, RB) + r.row * RB + r.cc * 16);
-    }
+    if (s < n) w[s] = (slot < 0 ? p.lse : ws_slot_lse(p, slot, RB))[r.row];
   }
+  ask(0);
   if (!merge_row_is_real(p, r)) return;
 #pragma unroll
   for (int s = 0; s < kMax; ++s) {
@@ -469,13 +478,20 @@ __global__ __launch_bounds__(256) void fdb_merge_kernel(const FdbKParams p) {
   const float inv = denom > 0.f ? 1.f / denom : 0.f;
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int s = 0; s < kMax; ++s)
-    if (s < n && w[s] > 0.f) {
-      const f32x8 x = VT::to_f32(__builtin_bit_cast(typename VT::frag, part[s]));
-      const float f = w[s] * inv;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(x[e], f, acc[e]);
+  for (int first = 0; first < kMax; first += kGroup) {
+    if (first > 0) {
+      if (first >= n) break;
+      ask(first);
     }
+#pragma unroll
+    for (int x = 0; x < kGroup; ++x)
+      if (first + x < n && w[first + x] > 0.f) {
+        const f32x8 y = VT::to_f32(__builtin_bit_cast(typename VT::frag, part[x]));
+        const float f = w[first + x] * inv;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(y[e], f, acc[e]);
+      }
+  }
   VT::store4(dst, acc[0], acc[1], acc[2], acc[3]);
   VT::store4(dst + 8, acc[4], acc[5], acc[6], acc[7]);
   if (r.cc == 0) p.lse[r.row] = denom > 0.f ? (m + __builtin_amdgcn_logf(denom)) * 0.6931471805599453f : -INFINITY;

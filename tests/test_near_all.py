@@ -160,3 +160,21 @@ def test_two_teams(L, terms, buckets, most, causal, dtype):
             assert np.abs(got.float().cpu().numpy() - ref).max() <= 3 * EPS[dtype] * max(1.0, np.abs(ref).max()), (b, m)
             assert np.abs(got_lse.cpu().numpy() - ref_lse).max() <= 2 * EPS[dtype], (b, m)
         at += m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("B,L,H,padded,far,near", [(1, 1, 1, False, 1, 2), (3, 70, 7, True, 1, 4), (700, 3, 5, False, 1, 3), (2, 700, 3, False, 2, 2), (2, 700, 3, True, 3, 2),
+                                                   (2, 700, 3, True, 4, 4), (2800, 129, 12, True, 1, 2)])   # the last: past 2^22 rows of the outputs
+def test_merged_shares_lie_where_one_launch_puts_them(B, L, H, padded, far, near, dtype):
+    """Two to eight partial results of a row."""
+    g = torch.Generator(device="cuda").manual_seed(B + L)
+    q, k, v = [torch.randn(B, L, H, 64, device="cuda", generator=g, dtype=dtype) for _ in range(3)]
+    pk, pq = [torch.randn(H, 64, 64, device="cuda", generator=g, dtype=dtype) for _ in range(2)]
+    kw = dict(position_buckets=32, max_relative_positions=64, return_lse=True)
+    if padded:
+        kw["seq_len"] = torch.randint(0, L + 1, (B,), device="cuda", generator=g, dtype=torch.int32)
+    (one, one_lse), (shared, shared_lse) = [ops.disentangled_attention_fwd(q, k, v, pk, pq, far_splits=f, near_splits=n, **kw) for f, n in ((1, 1), (far, near))]
+    # c2p and the scaled query are rounded alike on both sides; probabilities, against other reference points, partial results and outputs by half an eps each of at most max |v|
+    assert (shared - one).abs().max() <= 2.5 * EPS[dtype] * v.abs().max()
+    assert (shared_lse - one_lse).nan_to_num(posinf=0, neginf=0).abs().max() <= 1e-5 and torch.equal(shared_lse.isinf(), one_lse.isinf())
