@@ -229,6 +229,15 @@ constexpr int min_blocks() {
   return (lds <= 40 * 1024 && QT::SZ < 4) ? 3 : lds <= 80 * 1024 ? 2 : 1;  // fp32 fragments are twice the registers
 }
 
+// Whether the kernel's arguments are read together at its start.  Where they are, they hold scalar registers from there on, and the allocator spills others
+// around the loops: 16 bits at head_dim 128 with p2c alone 24 -> 66 registers, 8 x 1024 with 8 heads 95.0 -> 99.3 us; without position terms 84 -> 92 bytes,
+// 48.9 -> 49.8; the ring mode at head_dim 32 18.45 -> 18.65 (4 x 512, 12 heads).  Two forms gain by what the allocator makes of it: fp32 with both terms, 8 x 700 at
+// head_dim 32 178.6 -> 174.1 (p2c alone 94.5 -> 95.0), and bf16 at head_dim 128 with c2p alone, 8 x 1024 125.3 -> 113.9 (fp16 123.5 -> 125.4).
+template <class QT, int D, bool C2P, bool P2C>
+constexpr bool reads_arguments() {
+  return (QT::SZ == 4 && C2P && P2C) || (std::is_same_v<QT, Bf16Tr> && D == 128 && C2P && !P2C);
+}
+
 template <class QT, class VT, int D, bool FP8, bool C2P, bool P2C, int MODE>
 __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())) void fdb_attn_kernel(const FdbKParams p) {
   using C = Cfg<QT, VT, D>;
@@ -237,7 +246,7 @@ __global__ __launch_bounds__(kThreads, (min_blocks<QT, VT, D, C2P, P2C, MODE>())
   constexpr bool FAR_ONLY = MODE == kFarOnly, RING = MODE == kNearRing;
   static_assert(!RING || (!FP8 && QT::SZ == 2 && (C2P || P2C)), "the ring mode is for the position terms of the 16-bit types");
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  read_arguments(p);
+  if constexpr (reads_arguments<QT, D, C2P, P2C>()) read_arguments(p);
   constexpr bool KV_ALIAS = C::kv_alias(C2P, P2C);
   static_assert(!KV_ALIAS || MODE == kFused, "only the fused mode shares one buffer between K and V");
   char* Ks = smem;

@@ -87,7 +87,6 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_far8_kernel(const FdbKParams 
   constexpr int D = 64, DBLKS = 2;
   using VT = Bf16Tr;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  read_arguments(p);
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, li = lane & 31, g = lane >> 5;
@@ -402,7 +401,7 @@ __global__ __launch_bounds__(kThreads, 3) void fdb_near8_kernel(const FdbKParams
   using VT = Bf16Tr;
   using vfrag = typename VT::frag;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  read_arguments(p);
+  if constexpr (ALL && !C2P) read_arguments(p);
   char* Ks = smem;                    // [2][32][64]: step k reads buffer k & 1
   char* Vs = Ks + 2 * N8::K_BYTES;    // [2][32][128]
   char* EK = Vs + 2 * N8::V_BYTES;    // [160][64] rows K_r[delta(r)]: batch u / 32 of u = r_hi0 - r in slot batch mod 5; E_Q: [192][64], mod 6

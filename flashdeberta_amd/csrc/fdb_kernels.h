@@ -175,7 +175,9 @@ int fdb_launch_chain(const FdbChainParams& p, int dtype, void* stream);
 // Workspace slot `slot`: its output rows and its log-sum-exps (row_bytes = head_dim * element size).
 #if defined(__HIPCC__)
 // A kernel's first instruction: one argument of every 64 bytes that are not read at once anyway.  Left to itself the compiler reads the arguments where they
-// are used, each new 64 bytes of them after a wait for memory of their own.
+// are used, each new 64 bytes of them after a wait for memory of their own.  Not for kernels that have no registers to spare: those of csrc/fdb_attn.hip, where reads_arguments
+// has the figures, and the e4m3 pair (near launch of 3 x 777 28.8 -> 29.2 us, of 2 x 700 25.9 -> 26.3; 64 x 128, whose starts count more, 18.9 -> 18.7),
+// but for its near launch of all tiles with p2c alone (2 x 700 22.6 -> 22.3, 5 x 777 31.2 -> 30.7).
 __device__ __forceinline__ void read_arguments(const FdbKParams& p) { asm volatile("" ::"s"(p.q_sb), "s"(p.o_sb)); }
 
 __device__ __forceinline__ char* ws_slot_out(const FdbKParams& p, int slot, int row_bytes) {
