@@ -144,39 +144,12 @@ int far_parts_wanted(const fdb_attn_args* a) {
   return n > 1 ? n : 1;
 }
 
-// The same for the near launch, which keeps two workgroups on a CU.  Every share repeats the prologue
-// (five batches of table rows) and a merge kernel follows, so a share keeps at least sixteen 32-key
-// steps, or eight when all shares together fill at most half of the slots.  (Measured, 12 heads: one
-// sequence of 1024: 0.056 -> 0.040 ms; one of 512: 0.025 -> 0.022; four of 512 in shares of eight
-// steps would go from 0.025 to 0.028.)  Two shares of twelve steps pay while they leave a fifth of the
-// slots free (two of 777 40.0 -> 38.3 us, two of 900 45.2 -> 43.0; three of 777, 504 shares, would lose 7 %).
-// Two shares with a partial second round (288 to 352 query tiles) are not taken: dealt longest first, the tiles are 3 to 8 %
-// faster unshared there.
-//
-// Three shares of nine steps or more where two make between one and one and a third workgroups a CU, some of which then have two and last as long as two do
-// anywhere (1 x 1152 with 16 heads 40.8 -> 34.9 us, 1 x 1536 48.1 -> 40.1, 1 x 1792 53.8 -> 44.7; 2 x 768, eight steps a share, 33.0 -> 30.1, as two teams take).
 int near_steps(const fdb_attn_args* a) {   // 32-key steps of a query tile in mid-sequence
   // A packed batch has its lengths on the device: the host goes by the mean length and by the most query tiles the
   // token count allows (the kernel divides each query tile's own steps among the shares, whatever they are).
   const int32_t typical = a->cu_seqlens ? a->total_tokens / a->batch : a->max_seqlen;
   const int steps_all = (typical + 31) / 32, steps_near = (FDB_BM + 2 * a->lut_radius + 3 * (FDB_BN - 1)) / 32;
   return steps_all < steps_near ? steps_all : steps_near;
-}
-
-bool two_shares_crowd(int64_t wgs) { return 2 * wgs * 16 > 17 * (int64_t)fdb_cu_count(); }   // 132 tiles on 256 CUs: two shares 36.0 us, three 37.2
-
-int near_parts_wanted(const fdb_attn_args* a) {
-  if (!(a->pos_key || a->pos_query) || !a->lse || !steps32_supported(a->dtype, a->head_dim)) return 1;
-  if (a->near_splits > 0) return a->near_splits;
-  const int64_t wgs = query_tiles(a) * a->heads, slots = 2 * (int64_t)fdb_cu_count();
-  const int steps = near_steps(a);
-  if (!fdb_fp8_pair_supported(a->dtype, a->head_dim) && two_shares_crowd(wgs) && wgs * 3 <= slots && steps / 3 >= 9) return 3;
-  int best = 1;
-  for (int n = 2; n <= FDB_MAX_FAR_PARTS && wgs * n <= slots; ++n) {
-    const int per = steps / n;
-    if (per >= 16 || (n == 2 && per >= 12 && wgs * n * 5 <= slots * 4) || (per >= 8 && wgs * n <= slots / 2)) best = n;
-  }
-  return best;
 }
 
 // Whether a near workgroup of the 16-bit kernel is two teams of four waves, which take half of its steps each and add up in LDS: where every workgroup has a
@@ -188,6 +161,34 @@ int near_parts_wanted(const fdb_attn_args* a) {
 // with shares: 1 x 1024, two of 16 29.9 -> 28.6; 1 x 2048 with 4 heads, four of 16 31.5 -> 30.2; 1 x 512, two of 8 21.9 -> 21.8 (kept).
 bool near_takes_teams(const fdb_attn_args* a, int parts) {
   return !fdb_fp8_pair_supported(a->dtype, a->head_dim) && query_tiles(a) * a->heads * parts <= fdb_cu_count() && near_steps(a) / parts >= 10;
+}
+
+bool two_shares_crowd(int64_t wgs) { return 2 * wgs * 16 > 17 * (int64_t)fdb_cu_count(); }   // 132 tiles on 256 CUs: two shares 36.0 us, three 37.2
+
+// The same for the near launch, which keeps two workgroups on a CU.  Every share repeats the prologue
+// (five batches of table rows) and a merge kernel follows, so a share keeps at least sixteen 32-key
+// steps, or eight when all shares together fill at most half of the slots.  (Measured, 12 heads: one
+// sequence of 1024: 0.056 -> 0.040 ms; one of 512: 0.025 -> 0.022; four of 512 in shares of eight
+// steps would go from 0.025 to 0.028.)  Two shares of twelve steps pay while they leave a fifth of the
+// slots free (two of 777 40.0 -> 38.3 us, two of 900 45.2 -> 43.0; three of 777, 504 shares, would lose 7 %).
+// Two shares with a partial second round (288 to 352 query tiles) are not taken: dealt longest first, the tiles are 3 to 8 %
+// faster unshared there.
+//
+// Three shares of nine steps or more where two make between one and one and a third workgroups a CU, some of which then have two and last as long as two do
+// anywhere (1 x 1152 with 16 heads 40.8 -> 34.9 us, 1 x 1536 48.1 -> 40.1, 1 x 1792 53.8 -> 44.7; 2 x 768, eight steps a share, 33.0 -> 30.1, as two teams take).
+int near_parts_wanted(const fdb_attn_args* a) {
+  if (!(a->pos_key || a->pos_query) || !a->lse || !steps32_supported(a->dtype, a->head_dim)) return 1;
+  if (a->near_splits > 0) return a->near_splits;
+  const int64_t wgs = query_tiles(a) * a->heads, slots = 2 * (int64_t)fdb_cu_count();
+  const int steps = near_steps(a);
+  if (!fdb_fp8_pair_supported(a->dtype, a->head_dim) && two_shares_crowd(wgs) && wgs * 3 <= slots && steps / 3 >= 9) return 3;
+  int best = 1;
+  for (int n = 2; n <= FDB_MAX_FAR_PARTS && wgs * n <= slots; ++n) {
+    const int per = steps / n;
+    if (per >= 16 || (n == 2 && per >= 12 && wgs * n * 5 <= slots * 4) || (per >= 8 && wgs * n <= slots / 2)) best = n;
+  }
+  if (best == 2 && two_shares_crowd(wgs) && near_takes_teams(a, 1)) return 1;   // two teams instead, see there
+  return best;
 }
 
 // Does the call take the far / near pair of launches (otherwise one kernel walks every key tile)?
@@ -438,7 +439,6 @@ int attn_fwd_impl(const fdb_attn_args* a, int launch_mask, void* stream) {
     // as many workgroups per query tile as wanted and as the workspace holds partial results for
     p.far_parts = need_far ? far_parts_wanted(a) : 1;
     p.near_parts = near_parts_wanted(a);
-    if (p.near_parts == 2 && a->near_splits == 0 && two_shares_crowd(grid_x * a->heads) && near_takes_teams(a, 1)) p.near_parts = 1;
     const int64_t ws_slots_have = a->workspace ? a->workspace_bytes / far_part_bytes(a) : 0;
     if (p.near_parts > 1 && ws_slots_have < p.far_parts - 1 + p.near_parts) p.near_parts = 1;
     while (p.far_parts > 1 && ws_slots_have < p.far_parts - 1 + (p.near_parts > 1 ? p.near_parts : 0)) --p.far_parts;

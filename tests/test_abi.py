@@ -137,9 +137,11 @@ def test_far_split_policy_and_workspace_size():
     assert ws(args(1, 4096)) == part(4096, 12)            # 384 query tiles: 2 far shares (1 slot), near unshared
     assert ws(args(1, 4096, heads=16)) == 0               # 512: two shares would need a second round
     assert ws(args(1, 4096, heads=10)) == part(4096, 10)  # 320: 2 far shares; 2 near shares would take 1.25 rounds
-    assert ws(args(1, 4096, heads=8)) == (2 + 2) * part(4096, 8)  # 256: 3 far shares (2 slots) + 2 near shares (2 slots)
+    assert ws(args(1, 4096, heads=8)) == 2 * part(4096, 8)  # 256: 3 far shares (2 slots); near workgroups of two teams, which need none
     assert ws(args(2, 4096)) == 0 and ws(args(8, 4096)) == 0  # the launch fills the slots by itself
-    assert ws(args(1, 2048)) == 2 * part(2048, 12)        # 192: too few far tiles to share, 2 near shares
+    assert ws(args(1, 2048)) == 0                         # 192: too few far tiles to share, two near shares become two teams of one workgroup
+    a = args(1, 2048); a.dtype, a.q_scale, a.k_scale, a.pk_scale, a.pq_scale = _lib.FDB_FP8_E4M3, *[0x1000] * 4
+    assert ws(a) == 2 * part(2048, 12)                    # e4m3 has no teams
     assert ws(args(1, 1024)) == 2 * part(1024, 12)        # 96: 32 steps in two shares of sixteen
     assert ws(args(1, 512)) == 2 * part(512, 12)          # 48, no far tile at all: shares of eight steps, 96 workgroups
     assert ws(args(2, 512)) == 2 * part(2 * 512, 12)      # 96 -> 192
