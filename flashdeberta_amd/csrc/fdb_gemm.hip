@@ -68,6 +68,7 @@ struct GemmShape {   // STAGED: rows of w that are fetched, TN or what makes who
 
 // The rows of a product, tile by tile: all `count` of them as they lie.
 struct AllRows {
+  static constexpr bool BIAS_AHEAD = true;
   int count;
   __device__ __forceinline__ int64_t base(int m0) const { return m0; }
   __device__ __forceinline__ uint32_t from_base(int m0, int row) const { return (uint32_t)(min(m0 + row, count - 1) - m0); }  // past the end: the last one
@@ -104,14 +105,15 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
 #pragma unroll
     for (int j = 0; j < S::FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // What the end of the tile reads is asked for ahead of everything: a trip to memory that nothing covers there (4096 x 768 x 768 + residual 9.4 -> 9.0 us, 1500 rows
-  // 7.0 -> 6.5).  Left as it lies in memory, so that nothing waits for it.
+  // 7.0 -> 6.5).  Left as it lies in memory, so that nothing waits for it.  Not the bias of real rows, whose first loads wait for the lengths as it is: 2304 x 768,
+  // 2346 real rows of 8 x 384 15.1 -> 15.3 us, 5223 of 64 x 128 24.0 -> 24.3 (8225 of 64 x 200, three rounds, 40.1 -> 39.9).
   using four = typename QT::scratch4;
   four bias[S::FN];
 #pragma unroll
   for (int j = 0; j < S::FN; ++j) {
     const int col = n0 + (wn * S::FN + j) * 16 + 4 * kg;
     bias[j] = __builtin_bit_cast(four, u32x2{0, 0});
-    if (EPI != kNarrow && p.bias && col < p.N) bias[j] = *(const four*)(p.bias + (int64_t)col * 2);
+    if (EPI != kNarrow && Rows::BIAS_AHEAD && p.bias && col < p.N) bias[j] = *(const four*)(p.bias + (int64_t)col * 2);
   }
   constexpr int CW = EPI == kNarrow ? 4 : 8, CH = TN / CW, PIECES = TM * CH / (64 * S::NW);   // of the result, a thread
   // The residual where few registers hold it, and not where two workgroups share a CU: the other one covers the trip there (8192 x 768 x 3072 42.1 us, ahead 42.9, not 41.5).
@@ -171,6 +173,7 @@ __device__ __forceinline__ void make_tile(const GemmParams& p, const Rows& rows,
   for (int j = 0; j < S::FN; ++j) {
     const int col = (wn * S::FN + j) * 16 + 4 * kg;
     f32x4 b = __builtin_convertvector(bias[j], f32x4);
+    if (EPI != kNarrow && !Rows::BIAS_AHEAD && p.bias && n0 + col < p.N) b = QT::load4(p.bias + (int64_t)(n0 + col) * 2);
     if (EPI == kNarrow && p.bias && n0 + col < p.N) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) b[e] = (float)((const elem*)p.bias)[n0 + col + e];
@@ -296,6 +299,7 @@ constexpr int kRealTiles = R192::TILES;   // the most of the four
 constexpr int kRealBytes = kRealTiles + 256 * 4;   // and where a tile's rows lie
 static_assert(R64::TILES <= kRealTiles && R128::TILES <= kRealTiles && R256::TILES <= kRealTiles && R256x160::TILES <= kRealTiles && kRealBytes <= 160 * 1024, "LDS budget");
 struct RealRows {
+  static constexpr bool BIAS_AHEAD = false;
   int count;
   const int32_t* at;   // LDS
   __device__ __forceinline__ int64_t base(int) const { return 0; }
