@@ -79,6 +79,29 @@ def test_gelu_of_every_value_is_torchs(dtype):
         assert torch.equal(got[0].isnan(), ref.isnan()) and torch.equal(got.nan_to_num(), ref.nan_to_num().expand(3, -1))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("kinds", ["tiny ordinary", "ordinary large", "zero tiny large", "zero tiny ordinary large", "denormal tiny large", "ordinary large inf", "tiny ordinary nan"])
+def test_gelu_of_unlike_values_side_by_side(kinds, dtype):
+    """Of the values a wave looks at together some are in the table, some halves, some themselves or nothing, some neither: each row another mixture."""
+    every = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(dtype)
+    size, least = every.float().abs(), torch.finfo(dtype).tiny
+    of = {"zero": size == 0, "denormal": (size > 0) & (size < least), "tiny": (size >= least) & (size < 2.0 ** -14 + least), "ordinary": (size > 2.0 ** -14) & (size < 8),
+          "large": (size >= 8) & size.isfinite(), "inf": size.isinf(), "nan": size.isnan()}
+    g = torch.Generator(device="cuda").manual_seed(len(kinds))
+    pick = lambda some, n: some[torch.randint(len(some), (n,), device="cuda", generator=g)]
+    rows = torch.stack([pick(every[of[k]], 8192) for k in kinds.split()])
+    mixed = rows.gather(0, torch.randint(len(rows), (70, 8192), device="cuda", generator=g))
+    if set(kinds.split()) & {"denormal", "inf", "nan"}:   # as the bias, alike in all rows: 0 x inf is none of them
+        x, w, bias = torch.zeros(70, 128, device="cuda", dtype=dtype), torch.zeros(8192, 128, device="cuda", dtype=dtype), mixed[0].contiguous()
+        mixed = bias.expand(70, -1)
+    else:                                                 # y = x . w^T to the bit: x the identity, the columns of w the rows of y
+        x, w, bias = torch.eye(70, 128, device="cuda", dtype=dtype), torch.zeros(8192, 128, device="cuda", dtype=dtype), None
+        w[:, :70] = mixed.t()
+    got, ref = _run(x, w, bias, GELU), F.gelu(mixed + 0)   # (-0 + 0 is 0, as in the sums)
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.nan_to_num(), ref.nan_to_num())
+
+
 def test_where_it_serves():
     serves = _lib.lib.fdb_gemm_serves
     assert not serves(32, 768, 768, RESIDUAL) and serves(33, 768, 768, RESIDUAL) and not serves(64, 768, 100, RESIDUAL) and not serves(64, 772, 768, GELU)
