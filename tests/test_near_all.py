@@ -7,7 +7,9 @@ import pytest
 import torch
 
 from flashdeberta_amd import _lib, ops
+from launches import launches
 from oracle import disentangled_oracle as O
+from test_launches import _forward
 
 EPS = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 
@@ -135,7 +137,8 @@ def test_every_workgroup_finds_its_place(B, H):
 @pytest.mark.parametrize("causal", [False, True], ids=["all", "causal"])
 @pytest.mark.parametrize("L,terms,buckets,most", [(289, (1, 1), 32, 64), (320, (1, 0), 256, 512), (321, (0, 1), 32, 64), (352, (1, 1), 256, 512), (900, (1, 1), 32, 64)])
 def test_two_teams(L, terms, buckets, most, causal, dtype):
-    """Workgroups of two teams at even and odd numbers of steps, far ones among them, in padded rows down to no step for a team or for both, and packed."""
+    """Workgroups of two teams at even and odd numbers of steps, far ones among them, in padded rows down to no step for a team or for both, and the same sequences packed,
+    whose mean length makes two teams at 900 alone."""
     lens = [L, 1, 33, 0, 64, L - 1]
     q, k, v, pk, pq = _inputs(len(lens), L, 2, terms, dtype)
     pk, pq = [None if x is None else x[:, :2 * buckets] for x in (pk, pq)]
@@ -159,6 +162,37 @@ def test_two_teams(L, terms, buckets, most, causal, dtype):
             # scores and probabilities are rounded as in every near launch, see above
             assert np.abs(got.float().cpu().numpy() - ref).max() <= 3 * EPS[dtype] * max(1.0, np.abs(ref).max()), (b, m)
             assert np.abs(got_lse.cpu().numpy() - ref_lse).max() <= 2 * EPS[dtype], (b, m)
+        at += m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("causal", [False, True], ids=["all", "causal"])
+@pytest.mark.parametrize("many", [False, True], ids=["few", "with a work-list"])
+@pytest.mark.parametrize("L,terms,buckets,most", [(352, (1, 1), 256, 512), (353, (1, 0), 32, 64), (353, (0, 1), 256, 512), (384, (1, 1), 32, 64), (380, (0, 1), 32, 64)])
+def test_two_teams_of_packed_sequences(L, terms, buckets, most, many, causal, dtype):
+    """Two teams go by the mean length: 10 to 12 steps here, of sequences down to no token; up to 64 without a work-list, more with one."""
+    lens, H = ([L] * 60 + [1, 33, 0, 64, 129, L - 1], 1) if many else ([L] * 16 + [1, 33, 0, 64, L - 1], 2)
+    np.random.default_rng(L).shuffle(lens)
+    T, i32 = sum(lens), lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    assert _lib.lib.fdb_needs_worklist(T, len(lens), H) == many
+    (rc, made), = launches([_forward(len(lens), L, H, _lib.FDB_BF16, most, total_tokens=T, cu_seqlens=0x1000, worklist=0x1000, causal=int(causal))])
+    assert rc == 0 and [m[2:] for m in made if "near" in m[0]] == [(1, 512)], made   # 512 threads: both teams
+    q, k, v, pk, pq = _inputs(1, T, H, terms, dtype)
+    pk, pq = [None if x is None else x[:, :2 * buckets] for x in (pk, pq)]
+    d = lambda x: None if x is None else x.cuda()
+    out, lse = ops.disentangled_attention_fwd(d(q[0]), d(k[0]), d(v[0]), d(pk), d(pq), cu_seqlens=i32(np.cumsum([0] + lens)), max_seqlen=L, position_buckets=buckets,
+                                              max_relative_positions=most, causal=causal, return_lse=True, workspace=torch.empty(16, dtype=torch.uint8, device="cuda"))
+    n = lambda x: None if x is None else x.float().numpy().astype(np.float64)
+    at = 0
+    for m in lens:
+        if m == 0:
+            continue
+        t = lambda x: n(x[:, at:at + m]).transpose(0, 2, 1, 3)
+        ref, ref_lse = O.disentangled_attention(t(q), t(k), t(v), n(pk), n(pq), buckets, most, causal=causal, return_lse=True)
+        # scores and probabilities are rounded as in every near launch, see above
+        assert np.abs(out[at:at + m].float().cpu().numpy() - ref[0].transpose(1, 0, 2)).max() <= 3 * EPS[dtype] * max(1.0, np.abs(ref).max()), (at, m)
+        assert np.abs(lse.view(-1, H)[at:at + m].cpu().numpy() - ref_lse[0].T).max() <= 2 * EPS[dtype], (at, m)
         at += m
 
 
