@@ -115,7 +115,9 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
   using vfrag = typename VT::frag;
   static_assert(QT::SZ == 2 && VT::SZ == 2, "16-bit element types only");
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
-  read_arguments(p);
+  // Not in fp16 with both terms in one team, whose loop comes out in a slower order for it, as in no other form: 8 x 512 30.8 -> 31.7 us, 2 x 1501 61.8 -> 63.2,
+  // 3 x 2048 114.8 -> 117.4 (64 x 128, nearly all start, 23.0 -> 22.7); bf16, 16 x 512 padded, 40.2 -> 39.7; two teams in fp16, 5 x 512, 20.3 -> 20.1.
+  if constexpr (!(std::is_same_v<QT, F16Tr> && C2P && P2C && TEAMS == 1)) read_arguments(p);
   const int team = TEAMS > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kNThreads) : 0;
   char* smem = smem_all + team * NCfg::lds_bytes(C2P, P2C);
   char* Ks = smem;                      // [2][32][128]: step k reads buffer k & 1
@@ -588,7 +590,7 @@ __global__ __launch_bounds__(kNThreads * TEAMS, 2) void fdb_near_kernel(const Fd
         range_begins(0.f);
       }
       // The rings' rows have been waited for, above or in the first far step.  In bf16 also where no near step follows and nobody uses what this reads:
-      // without a condition of its own the near loop comes out in a better order (3 x 777 30.7 -> 30.1 us, 1 x 1300 31.5 -> 31.3; fp16 31.5 -> 31.6).
+      // without a condition of its own the near loop comes out in a better order (four waves a workgroup: 3 x 777 30.7 -> 30.1 us, 1 x 1300 31.5 -> 31.3; fp16 31.5 -> 31.6).
       if (n_steps > 0 || std::is_same<QT, Bf16Tr>::value) near_begins();
     }
     int k = 0;
