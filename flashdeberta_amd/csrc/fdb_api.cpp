@@ -97,7 +97,8 @@ bool has_far_launch(const fdb_attn_args* a) {
 // more than it costs a far one, three of which do; but the far launch costs 6 to 8 us whatever it does, a first and a last round of its own, and a
 // partial result that is written and read again.  So it goes by the far tiles of the query tile at an end of the sequence, which has the most of them:
 // up to 8 for any batch, and while every query tile has a compute unit to itself, where the launch lasts as long as one tile, up to 6 more than a tile in
-// mid-sequence has near ones.  Replays back to back (60 ms of each, so at the clock that lasts), two launches -> one, us, 12 heads unless stated:
+// mid-sequence has near ones.  Replays back to back (60 ms of each, so at the clock that lasts), two launches -> one of four waves a workgroup (two teams of them make 3 x 777
+// 27.8 in bf16), us, 12 heads unless stated:
 //   far at an end, radius   bf16              e4m3                 alone on a compute unit   bf16             e4m3
 //   3    512  3 x 777       38.8 -> 30.0      38.5 -> 28.9         11  512  1 x 1300         43.4 -> 31.6     41.6 -> 30.3
 //   1    512  64 x 700      356 -> 329        269 -> 243           14  512  1 x 1501         46.9 -> 42.4     44.0 -> 37.7
@@ -154,28 +155,33 @@ int near_steps(const fdb_attn_args* a) {   // 32-key steps of a query tile in mi
 
 // Whether a near workgroup of the 16-bit kernel is two teams of four waves, which take half of its steps each and add up in LDS: where every workgroup has a
 // CU to itself.  A wave alone on its SIMD takes 1.0 us a step; two teams take 1.6 us a step of both, bound like two workgroups of a CU, and need neither
-// workspace nor a merge launch (5 us), so two shares of more than a workgroup a CU become one of two teams.  us, 12 heads unless stated, without -> with (and two shares):
-//   steps  7   4 x 200     17.4 -> 17.8 (kept)    16  5 x 512     25.8 -> 24.2         32  2 x 1024, 16 heads  40.8 -> 36.1 (40.8)
-//   10     7 x 300         20.7 -> 20.0           25  3 x 777     36.0 -> 32.6 (37.7)  40  2 x 1280            45.6 -> 41.3 (45.6)
-//   12     5 x 384         21.8 -> 21.1           24  3 x 768     33.0 -> 30.2 (35.0)  60  1 x 2048            59.3 -> 51.7 (59.1)
-// with shares: 1 x 1024, two of 16 29.9 -> 28.6; 1 x 2048 with 4 heads, four of 16 31.5 -> 30.2; 1 x 512, two of 8 21.9 -> 21.8 (kept).
+// workspace nor a merge launch, so two shares of more than a workgroup a CU become one of two teams.  bf16, replays back to back, 12 heads unless stated, us,
+// one share without -> with teams (and two shares without):
+//   steps 10   7 x 300     16.4 -> 16.1           24  3 x 768     28.1 -> 25.7         32  2 x 1024, 16 heads  35.3 -> 32.0 (36.3)
+//   12         5 x 384     17.2 -> 16.3           25  3 x 777     30.1 -> 27.8         40  2 x 1280            42.3 -> 37.2 (40.9)
+//   16         5 x 512     21.1 -> 20.0           25  2 x 777     29.8 -> 27.5 (30.3)  41  1 x 2048            56.9 -> 47.5 (53.9)
+// with shares: 1 x 1024, two of 16 24.5 -> 23.7; 1 x 2048 with 4 heads, four of 10 25.8 -> 25.1.  Below ten steps the teams' start and their last sums cost what they
+// gain: seven steps, 4 x 200, 2 % slower; 1 x 512, two shares of eight, even.  The e4m3 kernel, three workgroups of which share a CU, has no such form.
 bool near_takes_teams(const fdb_attn_args* a, int parts) {
   return !fdb_fp8_pair_supported(a->dtype, a->head_dim) && query_tiles(a) * a->heads * parts <= fdb_cu_count() && near_steps(a) / parts >= 10;
 }
 
-bool two_shares_crowd(int64_t wgs) { return 2 * wgs * 16 > 17 * (int64_t)fdb_cu_count(); }   // 132 tiles on 256 CUs: two shares 36.0 us, three 37.2
+// Whether two shares are so many workgroups that some CUs have two: 132 tiles on 256 CUs (1 x 1340), two shares 31.4 us in bf16 and 31.7 in fp16, three 31.4 and 32.4.
+bool two_shares_crowd(int64_t wgs) { return 2 * wgs * 16 > 17 * (int64_t)fdb_cu_count(); }
 
 // The same for the near launch, which keeps two workgroups on a CU.  Every share repeats the prologue
 // (five batches of table rows) and a merge kernel follows, so a share keeps at least sixteen 32-key
 // steps, or eight when all shares together fill at most half of the slots.  (Measured, 12 heads: one
 // sequence of 1024: 0.056 -> 0.040 ms; one of 512: 0.025 -> 0.022; four of 512 in shares of eight
 // steps would go from 0.025 to 0.028.)  Two shares of twelve steps pay while they leave a fifth of the
-// slots free (two of 777 40.0 -> 38.3 us, two of 900 45.2 -> 43.0; three of 777, 504 shares, would lose 7 %).
+// slots free: e4m3, 2 x 777 28.5 -> 26.5 us, 2 x 900 32.4 -> 29.3 (three of 777, 504 shares, would lose 7 %).  In 16 bits those are one share of two teams, like
+// every two shares that would crowd the CUs (137 tiles and more), and shares of twelve are left for 129 to 136 tiles.
 // Two shares with a partial second round (288 to 352 query tiles) are not taken: dealt longest first, the tiles are 3 to 8 %
 // faster unshared there.
 //
 // Three shares of nine steps or more where two make between one and one and a third workgroups a CU, some of which then have two and last as long as two do
-// anywhere (1 x 1152 with 16 heads 40.8 -> 34.9 us, 1 x 1536 48.1 -> 40.1, 1 x 1792 53.8 -> 44.7; 2 x 768, eight steps a share, 33.0 -> 30.1, as two teams take).
+// anywhere.  bf16, one share of two teams, or two without -> three: 1 x 1152 with 16 heads 34.1, 36.8 -> 31.1; 1 x 1536 40.7, 42.9 -> 35.4; 1 x 1792 44.1, 48.6 -> 40.3.
+// 16 bits alone: the e4m3 kernel's would gain as well (1 x 1536 37.4 -> 31.5) and are not dealt so.
 int near_parts_wanted(const fdb_attn_args* a) {
   if (!(a->pos_key || a->pos_query) || !a->lse || !steps32_supported(a->dtype, a->head_dim)) return 1;
   if (a->near_splits > 0) return a->near_splits;
@@ -324,9 +330,9 @@ int32_t fdb_worklist_max_tiles(int32_t total_tokens, int32_t batch) {
 
 // Packed calls whose workgroups find their tiles themselves (packed_place): the work-list's launch, 4 us with what it delays, against 0.3 us more at the start of each
 // workgroup, once for every round of them.  us, work-list -> without, sequences of lengths spread evenly over their logarithm, 12 heads, workgroups at most:
-//   4 of 16 to 256      84   15.9 -> 13.4      32 of 32 to 512    936   45.3 -> 44.8     64 of 32 to 512   1848   69.1 -> 69.8 (kept)
-//   8 of 32 to 512     264   28.0 -> 26.4      16 of 32 to 2048  1092  104.0 -> 104.1    32 of 32 to 2048  1992  175.4 -> 176.7 (kept)
-//   16 of 32 to 512    504   33.2 -> 30.7      8 of 2000 to 2048 1608  233.7 -> 233.9    64 of 32 to 2048  3840  305.5 -> 308.4 (kept)
+//   4 of 16 to 256      84   15.9 -> 13.4      32 of 32 to 512    936   45.3 -> 44.8            64 of 32 to 512   1848   69.1 -> 69.8 (kept)
+//   8 of 32 to 512     264   28.0 -> 26.4      16 of 32 to 2048  1092  104.0 -> 104.1 (kept)    32 of 32 to 2048  1992  175.4 -> 176.7 (kept)
+//   16 of 32 to 512    504   33.2 -> 30.7      8 of 2000 to 2048 1608  233.7 -> 233.9 (kept)    64 of 32 to 2048  3840  305.5 -> 308.4 (kept)
 int32_t fdb_needs_worklist(int32_t total_tokens, int32_t batch, int32_t heads) {
   return batch > 64 || (int64_t)fdb_worklist_max_tiles(total_tokens, batch) * heads > 4 * fdb_cu_count();
 }

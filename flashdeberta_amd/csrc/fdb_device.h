@@ -269,8 +269,8 @@ __device__ __forceinline__ float scratch_add_hi<float>(float acc, uint32_t) { re
 // that number (fdb_groups_together): each division here costs every workgroup some 40 instructions before its first load.
 enum { kNatural = 0, kEdgesFirst = 1, kMiddleFirst = 2, kLastFirst = 3 };
 // a / b, a >= 0 and b > 0: by a reciprocal in fp32, whose quotient of numbers under 2^22 is off by at most one.  A third of the instructions of the general one, of which
-// every wave would run three to five, one after the other, ahead of its first load (with the arguments and lengths read together: layer of 32 x 128, padded, 28.6 -> 28.1 us,
-// 1 x 4096 with 16 heads 122.7 -> 120.8).
+// every wave would run three to five, one after the other, ahead of its first load (with the arguments and lengths read together: layer of 32 x 128, padded, 28.6 -> 28.1 us;
+// of long launches it is too little to be seen, 1 x 4096 with 16 heads 119.6 and 119.2).
 __device__ __forceinline__ int quick_div(int a, int b) {
   if (__builtin_expect(a >= (1 << 22), 0)) return (int)((uint32_t)a / (uint32_t)b);
   int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
@@ -278,7 +278,7 @@ __device__ __forceinline__ int quick_div(int a, int b) {
   q += rest >= b ? 1 : rest >> 31;
   return q;
 }
-// Where the share `part` of `all` steps begins, of `parts` equal ones (at most 8, of at most 2^26 steps).
+// Where the share `part` of `all` steps begins, of `parts` equal ones (at most 8 and the one past them, of at most 2^26 steps).
 __device__ __forceinline__ int share_begins(int all, int part, int parts) { return __builtin_amdgcn_readfirstlane(quick_div(all * part, parts)); }
 // QUICK: not in the backward's roles, whose registers are so full that quick_div's branches spill 31 more of them in dQ's (8 x 4096 947 -> 1073 us; the other role the same).
 template <bool QUICK = true>

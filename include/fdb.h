@@ -100,8 +100,8 @@ typedef struct fdb_attn_args {
   void* out;
   float* lse;              /* [B*max_seqlen*H] (fixed) / [T*H] (varlen), token-major, or NULL; rows of padding like those of out */
   const int32_t* cu_seqlens; /* device int32[batch+1] or NULL                                 */
-  int32_t* worklist;       /* device int32[fdb_worklist_ints(...)], filled by fdb_build_worklist; not read, and need not be
-                              filled, where fdb_needs_worklist says so */
+  int32_t* worklist;       /* device int32[fdb_worklist_ints(...)], filled by fdb_build_worklist; never NULL where cu_seqlens is
+                              given (FDB_ERR_WORKLIST), but not read, and need not be filled, where fdb_needs_worklist says 0 */
   const int32_t* seq_start; /* fixed layout only, device int32[batch] or NULL: first real token of each row */
   const int32_t* seq_len;   /* fixed layout only, device int32[batch] or NULL: number of real tokens        */
   const int16_t* delta_lut;  /* device int16[2*lut_radius+1] from fdb_delta_lut, or NULL if no pos term */
@@ -434,7 +434,9 @@ int fdb_wgrad(const void* x0, const void* y0, int32_t rows0, int32_t x_cols0, co
  */
 int fdb_join(const void* const w[3], const void* const b[3], void* w_out, void* b_out, int64_t w_bytes, int64_t b_bytes, void* stream);
 
-/* 0: a packed call of these sizes finds its query tiles without a work-list (small batches of up to 64 sequences). */
+/* 0: a packed call of these sizes finds its query tiles without a work-list (small batches of up to 64 sequences).  The answer is
+ * for the device that is current, by its compute units: ask, fill and launch with the same one current, or fill the list whatever the
+ * answer.  A call that needs a list reads whatever the buffer holds. */
 int32_t fdb_needs_worklist(int32_t total_tokens, int32_t batch, int32_t heads);
 
 /* Enqueue the device-side work-list construction from cu_seqlens. */
